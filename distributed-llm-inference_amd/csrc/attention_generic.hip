@@ -31,6 +31,7 @@
 // nothing that the host made from the step's lengths); a kernel of its own takes these, below.
 //
 // Page layout: K [pages][kv_heads][page_size][head_dim], V [pages][kv_heads][value_dim][page_size].
+#include "attention_f32.h"
 #include "common.h"
 
 struct ScoreChanges {
@@ -683,6 +684,11 @@ extern "C" int dli_attention_generic(const void* q, int64_t q_stride, const void
                                      int tiles, int q_heads, int kv_heads, int head_dim, int page_size,
                                      float scale, int window, int is_bf16, hipStream_t stream) {
   if (head_dim % 16 != 0 || tile_entry == nullptr || v_pages == nullptr) return tiles <= 0 ? DLI_OK : DLI_ERR_ARGUMENT;
+  if (!is_bf16 && tiles > 0 && q_heads > 0 && q_heads <= 65535 && kv_heads > 0 && q_heads % kv_heads == 0 && table_stride > 0 &&
+      window >= 0 && page_size > 0 && attention_f32_takes(q, q_stride, k_pages, v_pages, out, out_stride, head_dim, page_size))
+    return attention_f32((const float*)q, q_stride, (const float*)k_pages, (const float*)v_pages, (float*)out, out_stride, q_start,
+                         kv_len, block_tables, table_stride, tile_entry, tile_q0, tiles, dli_attention_generic_tile_rows(head_dim),
+                         q_heads, kv_heads, head_dim, page_size, scale, window, stream);
   return attention_scored(q, q_stride, k_pages, v_pages, out, out_stride, q_start, kv_len,
                           block_tables, table_stride, tile_entry, tile_q0, tiles, q_heads,
                           kv_heads, head_dim, head_dim, page_size, scale, window, 0, 0, nullptr,

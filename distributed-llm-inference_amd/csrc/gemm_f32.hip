@@ -1,87 +1,308 @@
 // 32-bit matrix product for the true 32-bit path: out[m][n] = sum_k a[m][k] * w[n][k]
-// (+ bias[n]) (+ residual[m][n]). Plain FMA on the vector units, no matrix-core mode, so every
-// product and sum is IEEE single precision. Every output element sums its k in the same fixed
-// order whatever the tile it falls in, so a row's result does not depend on how many other rows
-// are in the batch: runs of GF_RUN consecutive k are summed in ascending order, and the runs'
-// sums are added in ascending order (the rounding error of a long sum then grows with the
-// length of a run plus the number of runs, not with k).
+// (+ bias[n]) (+ residual[m][n]), on the matrix cores' 32-bit form (v_mfma_f32_16x16x4_f32: IEEE
+// single-precision products and sums, no narrower operand anywhere).
+//
+// Every output element sums its k in one order that depends on k alone, whatever the tile it falls
+// in and however many waves share the work, so a row's result does not depend on how many other rows
+// are in the batch: 128 consecutive k make a run, whose sum grows four k at a time; the sums of
+// consecutive runs add up to at most GF_SEGMENTS segments, and the segments' sums are added in
+// ascending order (the rounding error of a long sum then grows with the length of a run plus the
+// number of runs, not with k).
+//
+// What bounds it: for few rows the stream of w, for many the matrix cores (157 TFLOP/s dense in 32-bit; a library product of
+// 8,192^3 reaches 152), in between the launch and the few tiles there are. Measured, us a product m x n x k, before (64 x 64
+// tiles of vector FMAs through LDS) and now:
+//   2 x 3072 x 576      37.6 ->   7.7     498 x 960 x 576     39.2 -> 12.5     512 x 3072 x 2048      152 ->   82
+//   2 x 576 x 1536      95.6 ->   7.6     498 x 3072 x 576    47.2 -> 32.6     512 x 16384 x 2048     491 ->  327
+//   2 x 49152 x 576     60.9 ->  24.6     498 x 576 x 1536     109 -> 22.6     2048 x 16384 x 2048   1827 -> 1280
+//   4 x 128256 x 2048    445 ->   177 (5.9 TB/s)                               2048 x 2048 x 8192     985 ->  655 (105 TFLOP/s)
+// (Reading both operands straight from memory also with many rows, a wave a tile: 44 us at 498 x 3072 x 576, 1,980 at 2048 x
+// 16384 x 2048: neighbouring lanes of a load lie in different rows. Choosing between a loaded value and zero beside the load
+// makes a wave wait for it at once: whole steps load without the choice, or choose when the value goes to LDS.)
 #include "common.h"
 
-#define GF_BM 64
-#define GF_BN 64
-#define GF_BK 16
-#define GF_RUN 256  // a multiple of GF_BK
+#define GF_RUN 128
+#define GF_SEGMENTS 16
 
-__global__ __launch_bounds__(256) void gemm_f32_nt_kernel(
-    const float* __restrict__ a, int64_t lda, const float* __restrict__ w, int64_t ldw,
-    const float* __restrict__ bias, const float* __restrict__ residual, int64_t ldr,
-    float* __restrict__ out, int64_t ldo, int m, int n, int k) {
-  __shared__ float as[GF_BK][GF_BM + 4];
-  __shared__ float ws[GF_BK][GF_BN + 4];
-  const int tid = threadIdx.x;
-  const int tx = tid % 16, ty = tid / 16;
-  const int m0 = blockIdx.y * GF_BM, n0 = blockIdx.x * GF_BN;
-  float acc[4][4] = {};    // the run of k in progress
-  float total[4][4] = {};  // the finished runs
-  const int lrow = tid / 4;          // 0..63: tile row loaded by this thread
-  const int lk = (tid % 4) * 4;      // 0,4,8,12: first of its four k values
-  const bool vec = (k % 4 == 0) && (lda % 4 == 0) && (ldw % 4 == 0) &&
-                   (((uintptr_t)a | (uintptr_t)w) % 16 == 0);
-  for (int k0 = 0; k0 < k; k0 += GF_BK) {
-    float av[4] = {0.f, 0.f, 0.f, 0.f}, wv[4] = {0.f, 0.f, 0.f, 0.f};
-    const int gm = m0 + lrow, gn = n0 + lrow, gk = k0 + lk;
-    if (vec) {
-      if (gm < m && gk < k) *(float4*)av = *(const float4*)(a + (int64_t)gm * lda + gk);
-      if (gn < n && gk < k) *(float4*)wv = *(const float4*)(w + (int64_t)gn * ldw + gk);
-    } else {
+typedef float gf4 __attribute__((ext_vector_type(4)));
+
+struct GfArgs {
+  const float* a;
+  const float* w;
+  const float* bias;
+  const float* residual;
+  float* out;
+  int64_t lda, ldw, ldr, ldo;
+  int m, n, k;
+  int segments, seg_runs;   // the sum's order: `segments` of `seg_runs` runs each (the last may be shorter)
+};
+
+struct Zero { static constexpr int value = 0; };
+struct One { static constexpr int value = 1; };
+
+// The four values of `row` from k = kk on. What lies past the row's end is zero.
+template <bool VEC>
+__device__ __forceinline__ gf4 gf_load(const float* row, int kk, int k) {
+  if constexpr (VEC) {
+    const gf4 v = *reinterpret_cast<const gf4*>(row + min(kk, k - 4));   // (k is a multiple of four: never across the end)
+    return kk < k ? v : gf4{0.f, 0.f, 0.f, 0.f};
+  } else {
+    gf4 v;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (gm < m && gk + i < k) av[i] = a[(int64_t)gm * lda + gk + i];
-        if (gn < n && gk + i < k) wv[i] = w[(int64_t)gn * ldw + gk + i];
+    for (int e = 0; e < 4; ++e) {
+      const float x = row[min(kk + e, k - 1)];
+      v[e] = kk + e < k ? x : 0.f;
+    }
+    return v;
+  }
+}
+
+// Lane (i, g) holds rows 4 g .. + 3 of a tile of 16 x 16, column i.
+__device__ __forceinline__ void gf_store(const GfArgs& p, gf4 sum, int m0, int n0, int i, int g) {
+  const int col = n0 + i;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int row = m0 + 4 * g + e;
+    if (row >= p.m || col >= p.n) continue;
+    float v = sum[e];
+    if (p.bias != nullptr) v += p.bias[col];
+    if (p.residual != nullptr) v += p.residual[(int64_t)row * p.ldr + col];
+    p.out[(int64_t)row * p.ldo + col] = v;
+  }
+}
+
+// Up to 16 rows: KW waves share a tile of 16 x 16 NT and take its segments in turn, each straight from memory: half a run's
+// operands are on their way while the other half is multiplied. (The lanes of a load lie in 16 rows, four neighbours in
+// four of them: as fast as any order where w comes from HBM once, but a quarter of the caches' rate where tiles share it.)
+template <int NT, int KW, bool VEC>
+__global__ __launch_bounds__(64 * KW) void gemm_f32_few_kernel(GfArgs p) {
+  extern __shared__ gf4 gf_sums[];   // [segments][NT][64]
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, i = lane % 16, g = lane / 16;
+  const int n0 = blockIdx.x * 16 * NT;
+  const float* ra = p.a + (int64_t)min(i, p.m - 1) * p.lda;   // (rows past the end: not stored)
+  const float* rw[NT];
+#pragma unroll
+  for (int y = 0; y < NT; ++y) rw[y] = p.w + (int64_t)min(n0 + 16 * y + i, p.n - 1) * p.ldw;
+  gf4 seg[NT], acc[NT], fa[2][4], fw[2][4][NT];
+#pragma unroll
+  for (int y = 0; y < NT; ++y) seg[y] = gf4{0.f, 0.f, 0.f, 0.f};
+
+  const auto load = [&](auto half, int k0) {   // 64 k from k0 on
+    constexpr int b = decltype(half)::value;
+    if (VEC && k0 + GF_RUN / 2 <= p.k) {   // (no choice between the value and zero: it would wait for the load at once)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        fa[b][t] = *reinterpret_cast<const gf4*>(ra + k0 + 4 * g + 16 * t);
+#pragma unroll
+        for (int y = 0; y < NT; ++y) fw[b][t][y] = *reinterpret_cast<const gf4*>(rw[y] + k0 + 4 * g + 16 * t);
+      }
+      return;
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      fa[b][t] = gf_load<VEC>(ra, k0 + 16 * t + 4 * g, p.k);
+#pragma unroll
+      for (int y = 0; y < NT; ++y) fw[b][t][y] = gf_load<VEC>(rw[y], k0 + 16 * t + 4 * g, p.k);
+    }
+  };
+  const auto multiply = [&](auto half) {
+    constexpr int b = decltype(half)::value;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int y = 0; y < NT; ++y) acc[y] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[b][t][s], fw[b][t][y][s], acc[y], 0, 0, 0);
+  };
+
+  const int runs = (p.k + GF_RUN - 1) / GF_RUN;
+  int s = wave, left = 0;
+  if (s < p.segments) {
+    load(Zero{}, s * p.seg_runs * GF_RUN);
+    left = min(p.seg_runs, runs - s * p.seg_runs);
+  }
+  for (int r = s * p.seg_runs; s < p.segments;) {   // run r of segment s, `left` runs of it to go
+#pragma unroll
+    for (int y = 0; y < NT; ++y) acc[y] = gf4{0.f, 0.f, 0.f, 0.f};
+    load(One{}, r * GF_RUN + GF_RUN / 2);
+    multiply(Zero{});
+    const bool last = --left == 0;
+    const int s_next = last ? s + KW : s, r_next = last ? s_next * p.seg_runs : r + 1;
+    if (s_next < p.segments) load(Zero{}, r_next * GF_RUN);
+    multiply(One{});
+#pragma unroll
+    for (int y = 0; y < NT; ++y) {
+      seg[y] += acc[y];
+      if (last) {
+        gf_sums[(s * NT + y) * 64 + lane] = seg[y];
+        seg[y] = gf4{0.f, 0.f, 0.f, 0.f};
       }
     }
-    __syncthreads();
+    if (last && s_next < p.segments) left = min(p.seg_runs, runs - r_next);
+    s = s_next;
+    r = r_next;
+  }
+  __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      as[lk + i][lrow] = av[i];
-      ws[lk + i][lrow] = wv[i];
+  for (int y = 0; y < NT; ++y) {
+    if (y % KW != wave) continue;
+    gf4 sum = gf4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < p.segments; ++c) sum += gf_sums[(c * NT + y) * 64 + lane];
+    gf_store(p, sum, 0, n0 + 16 * y, i, g);
+  }
+}
+
+// More rows: a wave makes a tile of 32 x 32 out of LDS, into which 32 k of its rows come in whole cache lines (rows of 36
+// floats there: the 16 rows of a read lie in banks of their own), the next 32 k in flight meanwhile. KG == 1: WM x WN
+// waves lie side by side and share what they stage. KG > 1 (few tiles, long sums): KG waves share one tile and take
+// its segments in turn, each in a part of LDS of its own, without a barrier.
+#define GF_BK 32
+#define GF_LD 36
+
+template <int WM, int WN, int KG, bool VEC>
+__global__ __launch_bounds__(64 * WM * WN * KG) void gemm_f32_tile_kernel(GfArgs p) {
+  static_assert(KG == 1 || WM * WN == 1, "waves that take segments in turn stage for themselves");
+  constexpr int BM = 32 * WM, BN = 32 * WN, THREADS = 64 * WM * WN, PER = (BM + BN) * (GF_BK / 4) / THREADS;
+  extern __shared__ gf4 gf_sums[];
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, i = lane % 16, g = lane / 16;
+  const int part = KG > 1 ? wave : 0, tid = KG > 1 ? lane : threadIdx.x;
+  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+  const int wm = KG > 1 ? 0 : wave / WN * 32, wn = KG > 1 ? 0 : wave % WN * 32;
+  float* stage = reinterpret_cast<float*>(gf_sums) + part * 2 * (BM + BN) * GF_LD;   // two of them in turn
+
+  const float* src[PER];   // this thread's share of the tile's rows: 16 bytes of each 32 k
+  int dst[PER];
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int c = u * THREADS + tid, row = c / (GF_BK / 4), at = c % (GF_BK / 4) * 4;
+    src[u] = (row < BM ? p.a + (int64_t)min(m0 + row, p.m - 1) * p.lda : p.w + (int64_t)min(n0 + row - BM, p.n - 1) * p.ldw) ;
+    dst[u] = row * GF_LD + at;
+  }
+  const int at = tid % (GF_BK / 4) * 4;   // (THREADS is a multiple of eight: the same place in every row)
+  gf4 flight[PER];
+  const auto fetch = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      if constexpr (VEC) flight[u] = *reinterpret_cast<const gf4*>(src[u] + min(k0 + at, p.k - 4));
+      else flight[u] = gf_load<false>(src[u], k0 + at, p.k);
     }
-    __syncthreads();
+  };
+  const auto put = [&](float* to, int k0) {   // (what lies past the row's end is zero; chosen here, long after the load)
 #pragma unroll
-    for (int kk = 0; kk < GF_BK; ++kk) {
-      const float4 af = *(const float4*)&as[kk][ty * 4];
-      const float4 wf = *(const float4*)&ws[kk][tx * 4];
-      const float ar[4] = {af.x, af.y, af.z, af.w};
-      const float wr[4] = {wf.x, wf.y, wf.z, wf.w};
+    for (int u = 0; u < PER; ++u)
+      *reinterpret_cast<gf4*>(to + dst[u]) = !VEC || k0 + at < p.k ? flight[u] : gf4{0.f, 0.f, 0.f, 0.f};
+  };
+
+  gf4 total[2][2], seg[2][2], acc[2][2];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+  for (int x = 0; x < 2; ++x)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(ar[i], wr[j], acc[i][j]);
+    for (int y = 0; y < 2; ++y) total[x][y] = seg[x][y] = acc[x][y] = gf4{0.f, 0.f, 0.f, 0.f};
+
+  gf4 kept[KG > 1 ? GF_SEGMENTS / KG : 1][2][2];   // KG > 1: the sums of this wave's segments (others' lie between them)
+  int seen = 0;
+  const int seg_k = p.seg_runs * GF_RUN;
+  int s = part, k0 = part * seg_k, buf = 0;
+  if (s < p.segments) {
+    fetch(k0);
+    put(stage, k0);
+  }
+  if constexpr (KG == 1) __syncthreads();
+  while (s < p.segments) {
+    int k_next = k0 + GF_BK, s_next = s;
+    const bool seg_ends = k_next >= p.k || k_next % seg_k == 0;
+    if (seg_ends) {
+      s_next = s + KG;
+      k_next = s_next * seg_k;
     }
-    if ((k0 + GF_BK) % GF_RUN == 0) {
+    if (s_next < p.segments) fetch(k_next);
+    const float* cur = stage + buf * (BM + BN) * GF_LD;
+    const float *ca = cur + (wm + i) * GF_LD + 4 * g, *cw = cur + (BM + wn + i) * GF_LD + 4 * g;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+    for (int t = 0; t < GF_BK / 16; ++t) {
+      gf4 fa[2], fw[2];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          total[i][j] += acc[i][j];
-          acc[i][j] = 0.f;
+      for (int x = 0; x < 2; ++x) {
+        fa[x] = *reinterpret_cast<const gf4*>(ca + 16 * x * GF_LD + 16 * t);
+        fw[x] = *reinterpret_cast<const gf4*>(cw + 16 * x * GF_LD + 16 * t);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+          for (int y = 0; y < 2; ++y) acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[x][e], fw[y][e], acc[x][y], 0, 0, 0);
+    }
+    if (seg_ends || k_next % GF_RUN == 0) {
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) {
+          seg[x][y] += acc[x][y];
+          acc[x][y] = gf4{0.f, 0.f, 0.f, 0.f};
+          if (seg_ends) {
+            if constexpr (KG > 1) {
+#pragma unroll
+              for (int c = 0; c < GF_SEGMENTS / KG; ++c)
+                if (c == seen) kept[c][x][y] = seg[x][y];
+            } else {
+              total[x][y] += seg[x][y];
+            }
+            seg[x][y] = gf4{0.f, 0.f, 0.f, 0.f};
+          }
         }
+      if (seg_ends) ++seen;
     }
+    buf ^= 1;
+    if (s_next < p.segments) put(stage + buf * (BM + BN) * GF_LD, k_next);
+    if constexpr (KG == 1) __syncthreads();
+    k0 = k_next;
+    s = s_next;
+  }
+  if constexpr (KG > 1) {   // the segments' sums go where the staging was: [segments][4][64]
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < GF_SEGMENTS / KG; ++c)
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+          if (wave + c * KG < p.segments) gf_sums[((wave + c * KG) * 4 + 2 * x + y) * 64 + lane] = kept[c][x][y];
+    __syncthreads();
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int gm = m0 + ty * 4 + i;
-    if (gm >= m) continue;
+  for (int x = 0; x < 2; ++x)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int gn = n0 + tx * 4 + j;
-      if (gn >= n) continue;
-      float v = total[i][j] + acc[i][j];
-      if (bias != nullptr) v += bias[gn];
-      if (residual != nullptr) v += residual[(int64_t)gm * ldr + gn];
-      out[(int64_t)gm * ldo + gn] = v;
+    for (int y = 0; y < 2; ++y) {
+      if (KG > 1 && (2 * x + y) % KG != wave) continue;
+      gf4 sum = total[x][y];
+      if constexpr (KG > 1)
+        for (int c = 0; c < p.segments; ++c) sum += gf_sums[(c * 4 + 2 * x + y) * 64 + lane];
+      gf_store(p, sum, m0 + wm + 16 * x, n0 + wn + 16 * y, i, g);
     }
-  }
+}
+
+template <int NT, int KW>
+static int gf_few(const GfArgs& p, bool vec, hipStream_t stream) {
+  const int grid = (p.n + 16 * NT - 1) / (16 * NT);
+  const size_t lds = (size_t)p.segments * NT * 64 * sizeof(gf4);   // at most 32 KiB
+  if (vec) gemm_f32_few_kernel<NT, KW, true><<<grid, 64 * KW, lds, stream>>>(p);
+  else gemm_f32_few_kernel<NT, KW, false><<<grid, 64 * KW, lds, stream>>>(p);
+  return dli_launch_status();
+}
+
+template <int WM, int WN, int KG>
+static int gf_tiles(const GfArgs& p, bool vec, hipStream_t stream) {
+  const dim3 grid((p.n + 32 * WN - 1) / (32 * WN), (p.m + 32 * WM - 1) / (32 * WM));
+  if (grid.y > 65535) return DLI_ERR_ARGUMENT;
+  // (KG of 4 and 8: 72 and 144 KiB, where up to 64 KiB of segments' sums find room afterwards)
+  constexpr size_t lds = (size_t)KG * 2 * 32 * (WM + WN) * GF_LD * sizeof(float);
+  static_assert(KG == 1 || (KG >= 4 && lds >= (size_t)GF_SEGMENTS * 4 * 64 * sizeof(gf4)), "room for the segments' sums");
+  const auto kernel = vec ? gemm_f32_tile_kernel<WM, WN, KG, true> : gemm_f32_tile_kernel<WM, WN, KG, false>;
+  if (lds > 65536 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
+    return DLI_ERR_LAUNCH;
+  kernel<<<grid, 64 * WM * WN * KG, lds, stream>>>(p);
+  return dli_launch_status();
 }
 
 extern "C" int dli_gemm_f32_nt(const float* a, int64_t lda, const float* w, int64_t ldw,
@@ -89,8 +310,23 @@ extern "C" int dli_gemm_f32_nt(const float* a, int64_t lda, const float* w, int6
                                int64_t ldo, int m, int n, int k, hipStream_t stream) {
   if (m <= 0 || n <= 0) return DLI_OK;
   if (k <= 0 || lda < k || ldw < k || ldo < n || (residual != nullptr && ldr < n)) return DLI_ERR_ARGUMENT;
-  const dim3 grid((n + GF_BN - 1) / GF_BN, (m + GF_BM - 1) / GF_BM);
-  if (grid.y > 65535) return DLI_ERR_ARGUMENT;
-  gemm_f32_nt_kernel<<<grid, 256, 0, stream>>>(a, lda, w, ldw, bias, residual, ldr, out, ldo, m, n, k);
-  return dli_launch_status();
+  const int runs = (k + GF_RUN - 1) / GF_RUN;
+  const int seg_runs = (runs + GF_SEGMENTS - 1) / GF_SEGMENTS, segments = (runs + seg_runs - 1) / seg_runs;
+  const GfArgs p = {a, w, bias, residual, out, lda, ldw, ldr, ldo, m, n, k, segments, seg_runs};
+  const bool vec = k % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (((uintptr_t)a | (uintptr_t)w) % 16) == 0;
+  // As many waves as the device has SIMDs, where the sum has segments enough: 498 x 3072 x 576 (1,536 tiles) takes 32.6 us
+  // with four waves a tile and 44 with tiles of 64 x 64 for four waves; 2048 x 16384 x 2048 1,280 us in tiles of 128 x 64.
+  const int64_t simds = 4 * dli_compute_units();
+  if (m <= 16) {
+    const int64_t tiles = (n + 15) / 16;
+    if (segments > 8 && tiles * 8 < 2 * simds) return gf_few<1, 16>(p, vec, stream);
+    if (segments > 4 && tiles * 4 < 2 * simds) return gf_few<1, 8>(p, vec, stream);
+    if (segments >= 2 && tiles < 8 * simds) return gf_few<1, 4>(p, vec, stream);
+    return gf_few<2, 2>(p, vec, stream);
+  }
+  const int64_t tiles = (int64_t)((n + 31) / 32) * ((m + 31) / 32);
+  if (tiles * 4 <= simds && segments > 4) return gf_tiles<1, 1, 8>(p, vec, stream);
+  if (tiles <= 2 * simds && segments >= 2) return gf_tiles<1, 1, 4>(p, vec, stream);
+  if (tiles < 8 * simds) return gf_tiles<2, 2, 1>(p, vec, stream);
+  return gf_tiles<4, 2, 1>(p, vec, stream);
 }

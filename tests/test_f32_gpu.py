@@ -1,0 +1,80 @@
+"""The 32-bit path's product and attention on the matrix cores, at the edges of their tiles, runs and splits."""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from test_kernels_gpu import _paged_case, _tiles, ref_paged_attention
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from dli_amd.kernels import ops as module
+
+    return module
+
+
+# rows: the few-row kernel's end and the tiles' (32, 64, 128); columns: part of a tile, and enough of them for every rule
+# of the dispatch; k: below a load, across a run's half and end, several runs a segment (2,048 is 16 runs, 2,100 two a segment)
+@pytest.mark.parametrize("m", [1, 16, 17, 33, 130])
+@pytest.mark.parametrize("n,k", [(31, 3), (16, 62), (48, 64), (576, 132), (1024, 1536), (700, 1030), (65, 2048), (33, 2100), (40000, 100)])
+def test_gemm_f32_edges(ops, m, n, k):
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, w = (torch.randn(r, k, device="cuda", generator=gen) for r in (m, n))
+    out = torch.full((m, n), 7.0, device="cuda")
+    ops.gemm_f32(a, w, out)
+    ref = a.double() @ w.double().T
+    # each of k products and sums rounds by 2^-24 of a partial sum: runs of 128 terms, then the runs' sums
+    bound = (128 + k / 128 + 2) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)
+    assert ((out.double() - ref).abs() <= bound).all()
+    one = torch.empty(1, n, device="cuda")   # a row alone, through the few-row kernel: the same bits
+    ops.gemm_f32(a[m - 1:], w, one)
+    assert torch.equal(one[0], out[m - 1])
+
+
+def test_gemm_f32_rows_of_wider_matrices(ops):
+    """Strides that allow 16-byte loads and strides that do not; a residual that is the result's own buffer."""
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    for pad in (4, 3):
+        a = torch.randn(70, 200 + pad, device="cuda", generator=gen)[:, :200]
+        w = torch.randn(90, 200 + pad, device="cuda", generator=gen)[:, :200]
+        bias = torch.randn(90, device="cuda", generator=gen)
+        wide = torch.randn(70, 90 + pad, device="cuda", generator=gen)
+        before, out = wide.clone(), wide[:, :90]
+        ops.gemm_f32(a, w, out, bias=bias, residual=out)
+        ref = a.double() @ w.double().T + bias.double() + before[:, :90].double()
+        assert (out.double() - ref).abs().max() < 200 * 2.0 ** -24 * 200 and torch.equal(wide[:, 90:], before[:, 90:])
+
+
+@pytest.mark.parametrize("qh,kvh,d,bs,window", [(9, 3, 64, 16, 0), (4, 4, 64, 48, 0), (6, 2, 128, 16, 0), (4, 2, 64, 16, 37), (2, 1, 128, 32, 150)])
+def test_attention_f32(ops, qh, kvh, d, bs, window):
+    """Single tokens, prompts and portions on a prefix; more blocks than waves and fewer; keys that no request has
+    written (NaN behind every request's last key) stay out."""
+    lens = [(1, 1), (1, 16), (1, 17), (1, 127), (1, 129), (7, 7), (16, 16), (33, 33), (5, 40), (17, 300), (130, 130), (1, 1030)]
+    q, kp, vp, q_start, kv_len, tables = _paged_case(torch.float32, qh, kvh, d, bs, lens, seed=d + bs, poison=True)
+    ref = ref_paged_attention(q, kp, vp, q_start, kv_len, tables, qh, d ** -0.5, window)
+    for e, (_, kv) in enumerate(lens):
+        if kv % bs:
+            page = tables[e][kv // bs]
+            kp[page, :, kv % bs:] = float("nan")
+            vp[page, :, :, kv % bs:] = float("nan")
+    rows = ops.attention_generic_tile_rows(d)
+    te, tq = _tiles(q_start, rows)
+    dev = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    out = torch.full(q.shape, 9.0, device="cuda")
+    ops.attention_generic(q.cuda(), kp.cuda(), vp.cuda(), out, dev(q_start), dev(kv_len), dev(tables), dev(te), dev(tq), qh,
+                          d ** -0.5, window)
+    # scores of d terms, exponentials and sums of up to 1,030 weights: well under 1e-5 of values of about one
+    assert (out.cpu().double() - ref).abs().max() < 1e-5
+    # the last prompt's last row as a single token: the same blocks for the same waves, the same bits
+    e = len(lens) - 2
+    last = q_start[e + 1] - 1
+    alone = torch.empty(1, q.shape[1], device="cuda")
+    ops.attention_generic(q[last:last + 1].cuda(), kp.cuda(), vp.cuda(), alone, dev([0, 1]), dev([kv_len[e]]),
+                          dev([tables[e]]), dev([0]), dev([0]), qh, d ** -0.5, window)
+    assert torch.equal(alone[0], out[last])

@@ -1,0 +1,343 @@
+// Matrix-state recurrences for steps with portions, heads of 64 keys and 64 values: a request's rows are cut into runs that
+// are walked at the same time, all in 32-bit. Token by token a request is one chain of 50 instructions a token on
+// 512 waves that have a SIMD each to themselves (2,048 tokens and 32 heads: 578 us the generalized delta rule, 378 the decayed
+// sums with a bonus, at one instruction every four to five cycles); cut into runs the chip's waves are full. A run's effect
+// on the state before it is linear, S_after = M S_before + E, o_t = o_t(from zero) + S_before^T y_t, so:
+//
+//   walk     every run token by token, from a state of zeros (an entry's first run from the request's own, which makes
+//            its results final): o and E. Where the rule mixes keys (RUNS_DELTA, RUNS_GATED) 64 more columns start from the unit
+//            matrix and take no input: they end as M, and their outputs are y. Where it does not (RUNS_BONUS), M is the
+//            product of the run's decays per key and y_t = r_t times their product before t.
+//   carry    per request and head the states between the runs, one after the other: E_s <- M_s E_(s-1) + E_s on the matrix
+//            cores (v_mfma_f32_16x16x4_f32); the last one is the request's new state.
+//   finish   o_t += E_(s-1)^T y_t on the matrix cores, and in the same pass the per-head norm and gate where the rule has them.
+//
+// walk: a workgroup of four waves takes one (run, head) and 64 columns, values or unit matrix; sixteen lanes (a DPP row) share
+// four columns and hold four keys of each, so that five 16-byte reads of LDS a token serve sixteen columns (with one column
+// a lane, as token by token, LDS is what bounds it). The vectors of sixteen tokens are staged by the workgroup, the next
+// sixteen are on their way meanwhile. What bounds it: vector instructions, some 110 to 130 a token and wave at four cycles each.
+//
+// Measured (one prompt of 2,048 tokens, 32 heads, walk + carry + finish, us): RUNS_DELTA 135 + 15 + 21 against 578 and 17 for
+// the norm, RUNS_BONUS 55 + 8 + 17 against 378 and 17, RUNS_GATED 136 in all against 421. Where the cut lies: ops.scan_runs.
+#include "scan_runs.h"
+
+typedef float rf4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ float runs_row_sum(float x) {   // over the sixteen lanes of a DPP row
+  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0xB1, 0xF, 0xF, false));
+  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x4E, 0xF, 0xF, false));
+  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x141, 0xF, 0xF, false));
+  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x140, 0xF, 0xF, false));
+  return x;
+}
+
+// The scratch of a run: sum over the entries before of ceil(rows / run_rows) is at most their rows / run_rows + their number.
+__device__ __forceinline__ int64_t runs_slot(const RunsArgs& p, int first, int entry, int run) {
+  return (int64_t)(first / p.run_rows + entry + run);
+}
+
+template <int RULE>
+__global__ __launch_bounds__(256) void scan_runs_walk_kernel(RunsArgs p) {
+  constexpr int D = 64, TB = 16;
+  __shared__ rf4 sk[TB * 16], sr[TB * 16], sv[TB * 16], sw[RULE == RUNS_GATED ? 1 : TB * 16], sc[RULE == RUNS_DELTA ? TB * 16 : 1];
+  __shared__ float sg[RULE == RUNS_GATED ? 2 * TB : 1];
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, vloc = lane / 16, part = lane % 16;
+  const int entry = blockIdx.x / p.runs, run = blockIdx.x % p.runs, head = blockIdx.y;
+  const bool unit = blockIdx.z != 0;   // the columns of the unit matrix
+  const int first = p.q_start[entry], row0 = first + run * p.run_rows;
+  const int n = min(p.run_rows, p.q_start[entry + 1] - row0);
+  if (n <= 0 || (unit && run == 0)) return;
+  const int col = wave * 16 + vloc * 4;   // the first of this lane's four columns
+  const int64_t qk_col = (int64_t)(head / p.group) * D, v_col = (int64_t)head * D;
+
+  float s[4][4];   // [key][column]
+  rf4 bonus = {0.f, 0.f, 0.f, 0.f}, decay = {1.f, 1.f, 1.f, 1.f};
+  const bool real = run == 0 && p.positions[first] != 0;
+  const float* st = p.state + (int64_t)p.state_slots[entry] * p.state_stride + (int64_t)head * D * D;   // [value][key]
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    rf4 old = {0.f, 0.f, 0.f, 0.f};
+    if (real) old = *reinterpret_cast<const rf4*>(st + (col + c) * D + part * 4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[i][c] = unit ? (part * 4 + i == col + c ? 1.f : 0.f) : old[i];
+  }
+  if (RULE == RUNS_BONUS) bonus = *reinterpret_cast<const rf4*>(p.bonus + v_col + part * 4);
+
+  // staging: sixteen threads a token, four values each
+  const int bt = tid / 16, bc = tid % 16 * 4;
+  rf4 fk, fr, fv = {0.f, 0.f, 0.f, 0.f}, fw, fa;
+  float fb = 0.f, fg = 0.f;
+  const auto fetch = [&](int t0) {
+    const int64_t row = row0 + min(t0 + bt, n - 1);
+    fk = *reinterpret_cast<const rf4*>(p.k + row * p.k_stride + qk_col + bc);
+    fr = *reinterpret_cast<const rf4*>(p.r + row * p.r_stride + qk_col + bc);
+    if (!unit) fv = *reinterpret_cast<const rf4*>(p.v + row * p.v_stride + v_col + bc);
+    if constexpr (RULE == RUNS_GATED) {
+      fb = p.w[row * p.w_stride + head];
+      fg = p.w[row * p.w_stride + p.heads + head];
+    } else {
+      fw = *reinterpret_cast<const rf4*>(p.w + row * p.w_stride + v_col + bc);
+    }
+    if constexpr (RULE == RUNS_DELTA) fa = *reinterpret_cast<const rf4*>(p.a + row * p.a_stride + v_col + bc);
+  };
+  float* dst = unit ? p.y : p.o;
+  const int64_t dst_stride = unit ? (int64_t)p.heads * D : p.o_stride;
+  const auto step = [&](int t) {
+    const rf4 k = sk[t * 16 + part], r = sr[t * 16 + part], v = sv[t * 16 + wave * 4 + vloc];
+    rf4 o;
+    if constexpr (RULE == RUNS_BONUS) {
+      const rf4 w = sw[t * 16 + part];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        float o0 = 0.f, o1 = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float kv = k[i] * v[c];
+          float& sum = i & 1 ? o1 : o0;
+          sum = fmaf(fmaf(bonus[i], kv, s[i][c]), r[i], sum);
+          s[i][c] = fmaf(w[i], s[i][c], kv);
+        }
+        o[c] = o0 + o1;
+      }
+      if (wave == 0 && vloc == 0 && run > 0)
+        *reinterpret_cast<rf4*>(p.y + (int64_t)(row0 + t) * p.heads * D + v_col + part * 4) = r * decay;
+      decay *= w;
+    } else {
+      rf4 us;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        float u0 = k[0] * s[0][c], u1 = k[1] * s[1][c];
+        u0 = fmaf(k[2], s[2][c], u0);
+        u1 = fmaf(k[3], s[3][c], u1);
+        us[c] = u0 + u1;
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) us[c] = runs_row_sum(us[c]);
+      if constexpr (RULE == RUNS_DELTA) {
+        const rf4 w = sw[t * 16 + part], a = sc[t * 16 + part];
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s[i][c] = fmaf(w[i], s[i][c], fmaf(k[i], v[c], -a[i] * us[c]));
+      } else {
+        const float g = sg[2 * t], bg = sg[2 * t + 1];   // g and beta g; v comes times beta
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const float u = fmaf(-bg, us[c], v[c]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s[i][c] = fmaf(k[i], u, g * s[i][c]);
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        float o0 = r[0] * s[0][c], o1 = r[1] * s[1][c];
+        o0 = fmaf(r[2], s[2][c], o0);
+        o1 = fmaf(r[3], s[3][c], o1);
+        o[c] = o0 + o1;
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) o[c] = runs_row_sum(o[c]);
+    return o;
+  };
+
+  fetch(0);
+  for (int t0 = 0; t0 < n; t0 += TB) {
+    __syncthreads();   // the batch before has been walked
+    if constexpr (RULE == RUNS_DELTA) {
+      const float kn = 1.f / sqrtf(runs_row_sum(fk[0] * fk[0] + fk[1] * fk[1] + (fk[2] * fk[2] + fk[3] * fk[3])) + 1e-6f);
+      sc[tid] = fa * (fk * kn) * kn;   // a u (u^T S) = (a u kn) (k^T S)
+    }
+    sk[tid] = fk;
+    sr[tid] = fr;
+    if constexpr (RULE == RUNS_GATED) {
+      sv[tid] = fv * fb;
+      if (bc == 0) {
+        sg[2 * bt] = fg;
+        sg[2 * bt + 1] = fb * fg;
+      }
+    } else {
+      sv[tid] = fv;
+      sw[tid] = fw;
+    }
+    if (t0 + TB < n) fetch(t0 + TB);   // on their way while this batch is walked
+    __syncthreads();
+    const int nb = min(TB, n - t0);
+    float* od = dst + (int64_t)(row0 + t0) * dst_stride + v_col + col;
+    if (nb == TB) {
+#pragma unroll 4
+      for (int t = 0; t < TB; ++t) {
+        const rf4 o = step(t);
+        if (part == 0) *reinterpret_cast<rf4*>(od + t * dst_stride) = o;
+      }
+    } else {
+      for (int t = 0; t < nb; ++t) {
+        const rf4 o = step(t);
+        if (part == 0) *reinterpret_cast<rf4*>(od + t * dst_stride) = o;
+      }
+    }
+    if constexpr (RULE == RUNS_BONUS) p.y += (int64_t)TB * p.heads * D;   // (the step counts its rows from the batch's first)
+  }
+  const int64_t at = (runs_slot(p, first, entry, run) * p.heads + head) * D;
+  float* end = (unit ? p.moves : p.ends) + at * D;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) *reinterpret_cast<rf4*>(end + (col + c) * D + part * 4) = rf4{s[0][c], s[1][c], s[2][c], s[3][c]};
+  if (RULE == RUNS_BONUS && wave == 0 && vloc == 0) *reinterpret_cast<rf4*>(p.moves + at + part * 4) = decay;
+}
+
+// A workgroup takes sixteen values of one (entry, head) through all its runs. Lane (i, g) of wave w makes keys 16 w + i of
+// values 4 g .. + 3: S^T M^T, S^T out of LDS, M^T and E (the next run's while this one is multiplied) from memory.
+template <int RULE>
+__global__ __launch_bounds__(256) void scan_runs_carry_kernel(RunsArgs p) {
+  constexpr int D = 64, LD = 68;
+  __shared__ __attribute__((aligned(16))) float ss[16 * LD];
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, i = lane % 16, g = lane / 16;
+  const int entry = blockIdx.x, head = blockIdx.y, v0 = blockIdx.z * 16;
+  const int first = p.q_start[entry], len = p.q_start[entry + 1] - first;
+  if (len <= 0) return;
+  const int runs = (len + p.run_rows - 1) / p.run_rows;
+  const int64_t slot = runs_slot(p, first, entry, 0), per_run = (int64_t)p.heads * D * D;
+  float* ends = p.ends + (slot * p.heads + head) * D * D + v0 * D;
+  float* st = p.state + (int64_t)p.state_slots[entry] * p.state_stride + ((int64_t)head * D + v0) * D;
+  const int vr = tid / 16, kc = tid % 16 * 4;   // whole rows of the slice, 16 bytes a thread
+  rf4 s = *reinterpret_cast<const rf4*>(ends + vr * D + kc);
+  if constexpr (RULE == RUNS_BONUS) {
+    const float* moves = p.moves + (slot * p.heads + head) * D + kc;
+    for (int run = 1; run < runs; ++run) {
+      const rf4 m = *reinterpret_cast<const rf4*>(moves + (int64_t)run * p.heads * D);
+      float* e = ends + run * per_run + vr * D + kc;
+      s = m * s + *reinterpret_cast<const rf4*>(e);
+      *reinterpret_cast<rf4*>(e) = s;
+    }
+  } else {
+    *reinterpret_cast<rf4*>(ss + vr * LD + kc) = s;
+    const float* moves = p.moves + (slot * p.heads + head) * D * D + 16 * wave + i;
+    float fm[16], fe[4];
+    const auto fetch = [&](int run) {
+#pragma unroll
+      for (int x = 0; x < 16; ++x) fm[x] = moves[run * per_run + (x / 4 * 16 + 4 * g + x % 4) * D];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) fe[e] = ends[run * per_run + (4 * g + e) * D + 16 * wave + i];
+    };
+    if (runs > 1) fetch(1);
+    for (int run = 1; run < runs; ++run) {
+      __syncthreads();
+      rf4 acc[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const rf4 a = *reinterpret_cast<const rf4*>(ss + i * LD + 16 * t + 4 * g);
+        acc[t] = t == 0 ? rf4{fe[0], fe[1], fe[2], fe[3]} : rf4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], fm[4 * t + e], acc[t], 0, 0, 0);
+      }
+      const rf4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+      if (run + 1 < runs) fetch(run + 1);
+      __syncthreads();   // the old state has been read
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        ss[(4 * g + e) * LD + 16 * wave + i] = sum[e];
+        ends[run * per_run + (4 * g + e) * D + 16 * wave + i] = sum[e];
+      }
+    }
+    __syncthreads();
+    s = *reinterpret_cast<const rf4*>(ss + vr * LD + kc);
+  }
+  *reinterpret_cast<rf4*>(st + vr * D + kc) = s;
+}
+
+// A wave takes sixteen rows of one run and head: lane (i, g) holds values 16 c + 4 g .. + 3 of row i.
+template <typename T, int FINISH>
+__global__ __launch_bounds__(256) void scan_runs_finish_kernel(RunsArgs p) {
+  constexpr int D = 64;
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, i = lane % 16, g = lane / 16;
+  const int entry = blockIdx.x / p.runs, run = blockIdx.x % p.runs, head = blockIdx.y;
+  const int first = p.q_start[entry], row0 = first + run * p.run_rows, t0 = blockIdx.z * 64 + wave * 16;
+  const int n = min(p.run_rows, p.q_start[entry + 1] - row0);
+  if (t0 >= n || (FINISH == RUNS_FINISH_SUM && run == 0)) return;
+  const int64_t row = row0 + min(t0 + i, n - 1), c0 = (int64_t)head * D + 4 * g;
+  rf4 o[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) o[c] = *reinterpret_cast<const rf4*>(p.o + row * p.o_stride + c0 + 16 * c);
+  if (run > 0) {
+    const float* s = p.ends + (runs_slot(p, first, entry, run - 1) * p.heads + head) * D * D + i * D + 4 * g;
+    const float* y = p.y + row * p.heads * D + c0;
+    rf4 fy[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) fy[t] = *reinterpret_cast<const rf4*>(y + 16 * t);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      rf4 fs[4], acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < 4; ++t) fs[t] = *reinterpret_cast<const rf4*>(s + 16 * c * D + 16 * t);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(fs[t][e], fy[t][e], acc, 0, 0, 0);
+      o[c] += acc;
+    }
+  }
+  if constexpr (FINISH == RUNS_FINISH_SUM) {
+    if (t0 + i < n)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) *reinterpret_cast<rf4*>(p.o + row * p.o_stride + c0 + 16 * c) = o[c];
+    return;
+  }
+  float sum = 0.f;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) sum += (o[c][0] * o[c][0] + o[c][1] * o[c][1]) + (o[c][2] * o[c][2] + o[c][3] * o[c][3]);
+  sum += __shfl_xor(sum, 16, DLI_WAVE);
+  sum += __shfl_xor(sum, 32, DLI_WAVE);
+  const float rn = 1.f / sqrtf(sum / (float)D + p.eps);
+  if (t0 + i >= n) return;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const rf4 gp = *reinterpret_cast<const rf4*>(p.gate + row * p.gate_stride + c0 + 16 * c);
+    const rf4 nw = *reinterpret_cast<const rf4*>(p.norm_w + c0 + 16 * c);
+    struct alignas(sizeof(T) * 4) Packed { T v[4]; } packed;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float gate = (FINISH == RUNS_FINISH_SILU ? gp[e] : 1.f) / (1.f + expf(-gp[e]));
+      packed.v[e] = from_f32<T>(o[c][e] * rn * nw[e] * gate);
+    }
+    *reinterpret_cast<Packed*>((T*)p.out + row * p.out_stride + c0 + 16 * c) = packed;
+  }
+}
+
+bool scan_runs_takes(const RunsArgs& p, int rule, int finish, int out_is_bf16) {
+  const auto whole = [](const void* at, size_t bytes) { return (uintptr_t)at % bytes == 0; };
+  const auto rows = [&](const float* at, int64_t stride) { return stride % 4 == 0 && whole(at, 16); };
+  if (p.y == nullptr || p.ends == nullptr || p.moves == nullptr || p.runs < 1 || p.run_rows < 16 || p.run_rows % 16 != 0) return false;
+  if (!rows(p.r, p.r_stride) || !rows(p.k, p.k_stride) || !rows(p.v, p.v_stride) || !rows(p.o, p.o_stride) ||
+      !rows(p.state, p.state_stride) || !whole(p.y, 16) || !whole(p.ends, 16) || !whole(p.moves, 16))
+    return false;
+  if (rule != RUNS_GATED && !rows(p.w, p.w_stride)) return false;
+  if (rule == RUNS_DELTA && !rows(p.a, p.a_stride)) return false;
+  if (rule == RUNS_BONUS && !whole(p.bonus, 16)) return false;
+  return finish == RUNS_FINISH_SUM || (rows(p.gate, p.gate_stride) && whole(p.norm_w, 16) && p.out_stride % 4 == 0 &&
+                                       whole(p.out, out_is_bf16 ? 8 : 16));
+}
+
+int scan_runs(const RunsArgs& p, int rule, int finish, int out_is_bf16, int entries, hipStream_t stream) {
+  const dim3 walk(entries * p.runs, p.heads, rule == RUNS_BONUS || p.runs == 1 ? 1 : 2), carry(entries, p.heads, 4);
+  if (rule == RUNS_DELTA) {
+    scan_runs_walk_kernel<RUNS_DELTA><<<walk, 256, 0, stream>>>(p);
+    scan_runs_carry_kernel<RUNS_DELTA><<<carry, 256, 0, stream>>>(p);
+  } else if (rule == RUNS_BONUS) {
+    scan_runs_walk_kernel<RUNS_BONUS><<<walk, 256, 0, stream>>>(p);
+    scan_runs_carry_kernel<RUNS_BONUS><<<carry, 256, 0, stream>>>(p);
+  } else {
+    scan_runs_walk_kernel<RUNS_GATED><<<walk, 256, 0, stream>>>(p);
+    scan_runs_carry_kernel<RUNS_GATED><<<carry, 256, 0, stream>>>(p);
+  }
+  const dim3 done(entries * p.runs, p.heads, (p.run_rows + 63) / 64);
+  if (finish == RUNS_FINISH_SUM) {
+    if (p.runs > 1) scan_runs_finish_kernel<float, RUNS_FINISH_SUM><<<done, 256, 0, stream>>>(p);
+  } else if (finish == RUNS_FINISH_SIGMOID) {
+    if (out_is_bf16) scan_runs_finish_kernel<bf16_t, RUNS_FINISH_SIGMOID><<<done, 256, 0, stream>>>(p);
+    else scan_runs_finish_kernel<float, RUNS_FINISH_SIGMOID><<<done, 256, 0, stream>>>(p);
+  } else {
+    if (out_is_bf16) scan_runs_finish_kernel<bf16_t, RUNS_FINISH_SILU><<<done, 256, 0, stream>>>(p);
+    else scan_runs_finish_kernel<float, RUNS_FINISH_SILU><<<done, 256, 0, stream>>>(p);
+  }
+  return dli_launch_status();
+}

@@ -120,6 +120,11 @@ class StepContext:
     def max_decode_kv_len(self) -> int:
         return int(self.kv_len_host[:self.num_decode].max()) if self.num_decode else 0
 
+    @property
+    def longest_entry(self) -> int:
+        """The most rows that an entry of the step brings."""
+        return self.step_lists("longest entry", lambda: int(np.diff(self.q_start_host).max()) if self.num_entries else 0)
+
     def entry_rows(self, e: int) -> tuple[int, int]:
         return int(self.q_start_host[e]), int(self.q_start_host[e + 1])
 

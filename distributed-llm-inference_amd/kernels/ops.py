@@ -154,7 +154,8 @@ _SIGNATURES = {
     "dli_recurrent_scan_supports": [_c_int],
     "dli_recurrent_scan": [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr,
                            _c_i64, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr,
-                           _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
+                           _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr,
+                           _c_ptr],
     "dli_rotary_cache": [_c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr,
                          _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, ctypes.c_double, _c_ptr, _c_ptr,
                          _c_float, _c_int, _c_ptr],
@@ -186,7 +187,7 @@ _SIGNATURES = {
     "dli_conv_prepare": [_c_ptr, _c_i64, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr,
                          _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "dli_gated_delta_scan": [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_int,
-                             _c_int, _c_int, _c_int, _c_ptr],
+                             _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
     "dli_poly_norm": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_float, _c_int, _c_ptr],
     "dli_clamped_glu": [_c_ptr, _c_i64, _c_ptr, _c_int, _c_int, _c_int, _c_float, _c_float, _c_float, _c_int, _c_ptr],
     "dli_router_choose": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int,
@@ -1875,15 +1876,49 @@ def recurrent_scan_supports(dim: int) -> bool:
     return bool(library().dli_recurrent_scan_supports(int(dim)))
 
 
+# A step whose longest entry has fewer rows is walked token by token: at 100 rows both ways take the same (34 and 35 us a
+# layer with 16 heads, generalized delta rule), at 300 85 and 39, at 2,048 with 32 heads 581 and 153 (bonus rule 387 and 80,
+# gated rule 421 and 136), 16 prompts of 375 tokens with 32 heads 584 and 229 (394 and 186, 272 and 183).
+RUNS_FROM_ROWS = 128
+RUNS_MIN_ROWS = 64      # rows of a run at least
+# Workgroups of the walk that a step is cut for: four a compute unit, one wave of each a SIMD (32 heads, delta / bonus / gated:
+# 2,048 tokens 164 / 80 / 148 us cut for 512, 153 / 80 / 136 for 1,024, 158 / 79 / 139 for 2,048; 375 tokens a
+# request 229 / 186 / 183 for 1,024 and 370 / 195 / 317 for 2,048: every further run walks the unit columns again).
+RUNS_WORKGROUPS = 1024
+
+
+def scan_runs(entries: int, rows: int, heads: int, longest: int, unit_columns: bool) -> tuple[int, int]:
+    """``(rows a run, runs of the longest entry)`` into which the rows of a matrix-state recurrence with heads of 64
+    are cut, or ``(0, 0)`` for token by token. ``longest``: the most rows that an entry of the step brings, as the
+    host knows it; ``unit_columns``: runs after an entry's first also walk the unit matrix's columns."""
+    if longest < RUNS_FROM_ROWS:
+        return 0, 0
+    alike = max(1, rows // longest)   # entries that long the step amounts to
+    runs = max(1, RUNS_WORKGROUPS // (alike * heads * (2 if unit_columns else 1)))
+    run_rows = max(RUNS_MIN_ROWS, -(-longest // runs))
+    run_rows = -(-run_rows // 16) * 16
+    return run_rows, -(-longest // run_rows)
+
+
+def _runs_scratch(device: torch.device, entries: int, rows: int, heads: int, run_rows: int, unit_columns: bool):
+    """The walk's outputs for the unit columns, and per run and head the end state and what moves the one before."""
+    slots = rows // run_rows + entries
+    return (torch.empty(rows, heads * 64, device=device, dtype=torch.float32),
+            torch.empty(slots, heads, 64, 64, device=device, dtype=torch.float32),
+            torch.empty(slots, heads, 64, 64 if unit_columns else 1, device=device, dtype=torch.float32))
+
+
 def recurrent_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, w: torch.Tensor, g_pre: torch.Tensor,
                    norm_w: torch.Tensor, eps: float, state: torch.Tensor, q_start: torch.Tensor,
                    positions: torch.Tensor, state_slots: torch.Tensor, out: torch.Tensor, heads: int, dim: int,
-                   rule: int, a: Optional[torch.Tensor] = None, bonus: Optional[torch.Tensor] = None) -> None:
+                   rule: int, a: Optional[torch.Tensor] = None, bonus: Optional[torch.Tensor] = None,
+                   longest: int = 0) -> None:
     """A matrix-state recurrence per request and head, with the per-head norm and the gate of its
     output (``csrc/recurrent_scan.hip`` states both rules). ``r, k, v``, the decay ``w``, the gate's
     pre-activation ``g_pre`` and (delta rule) the removal rate ``a`` are float32 ``[n, heads*dim]`` with
     contiguous rows (any row stride); ``state`` is float32 ``[slots, >= heads*dim*dim]``, row
-    ``state_slots[e]`` being entry ``e``'s; ``out [n, heads*dim]`` float32 or bfloat16."""
+    ``state_slots[e]`` being entry ``e``'s; ``out [n, heads*dim]`` float32 or bfloat16. ``longest``: the most
+    rows that an entry brings (0: not known on the host; the rows are then walked token by token)."""
     n, width = out.shape[0], heads * dim
     w_pre, a_pre, a_bias = w, a, None
     for name, t in (("r", r), ("k", k), ("v", v), ("w", w), ("g_pre", g_pre), ("a", a)):
@@ -1909,11 +1944,16 @@ def recurrent_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, w: torch.T
         _require(bonus.numel() == width, "bonus must hold heads*dim values")
     sa = a_pre.stride(0) if a_pre is not None else 0
     o_raw = torch.empty(n, width, device=out.device, dtype=torch.float32)  # the recurrence's output before norm and gate
+    run_rows, runs, scratch = 0, 0, (None, None, None)
+    if dim == 64 and entries > 0:
+        run_rows, runs = scan_runs(entries, n, heads, longest, rule == RULE_DELTA)
+        if run_rows:
+            scratch = _runs_scratch(out.device, entries, n, heads, run_rows, rule == RULE_DELTA)
     _check(library().dli_recurrent_scan(
         _ptr(r), r.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(w_pre), w_pre.stride(0), _ptr(a_pre), sa,
         _ptr(a_bias), _ptr(g_pre), g_pre.stride(0), _ptr(bonus), _ptr(norm_w), float(eps), _ptr(state), state.stride(0),
         _ptr(q_start), _ptr(positions), _ptr(state_slots), _ptr(o_raw), o_raw.stride(0), _ptr(out), out.stride(0), entries,
-        n, heads, dim, int(rule), _is_bf16(out.dtype), _stream()), "recurrent_scan")
+        n, heads, dim, int(rule), _is_bf16(out.dtype), run_rows, runs, *map(_ptr, scratch), _stream()), "recurrent_scan")
 
 
 # ----------------------------------------------------------------------------- rotary keys from 32-bit projections
@@ -2060,10 +2100,11 @@ def conv_prepare(proj: torch.Tensor, b_off: int, a_off: int, conv_w: torch.Tenso
 
 
 def gated_delta_scan(prep: torch.Tensor, state: torch.Tensor, q_start: torch.Tensor, positions: torch.Tensor,
-                     state_slots: torch.Tensor, o: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim: int) -> None:
+                     state_slots: torch.Tensor, o: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim: int,
+                     longest: int = 0) -> None:
     """Per request and head ``S <- g S; u = beta (v - S^T k); S <- S + k u^T; o = S^T q`` over the step's rows
     in order, ``S`` float32 ``[heads][vdim][dim]`` at the start of ``state[slot]`` (zeros at position 0);
-    ``prep`` as :func:`conv_prepare` leaves it; ``o [n, heads*vdim]`` float32."""
+    ``prep`` as :func:`conv_prepare` leaves it; ``o [n, heads*vdim]`` float32; ``longest`` as in :func:`recurrent_scan`."""
     _f32_rows(prep, "prep")
     _f32_rows(o, "o")
     n = prep.shape[0]
@@ -2076,9 +2117,15 @@ def gated_delta_scan(prep: torch.Tensor, state: torch.Tensor, q_start: torch.Ten
         _dense(t, name, torch.int32, 1)
     entries = state_slots.shape[0]
     _require(q_start.shape[0] == entries + 1 and positions.shape[0] == n, "q_start/state_slots/positions disagree")
+    run_rows, runs, scratch = 0, 0, (None, None, None)
+    if dim == vdim == 64 and entries > 0:
+        run_rows, runs = scan_runs(entries, n, heads, longest, True)
+        if run_rows:
+            scratch = _runs_scratch(o.device, entries, n, heads, run_rows, True)
     _check(library().dli_gated_delta_scan(
         _ptr(prep), prep.stride(0), _ptr(state), state.stride(0), _ptr(q_start), _ptr(positions), _ptr(state_slots),
-        _ptr(o), o.stride(0), entries, n, heads, kv_heads, dim, vdim, _stream()), "gated_delta_scan")
+        _ptr(o), o.stride(0), entries, n, heads, kv_heads, dim, vdim, run_rows, runs, *map(_ptr, scratch), _stream()),
+        "gated_delta_scan")
 
 
 HEAD_GATES = {"sigmoid": 0, "silu": 1, "none": 2, "silu_first": 3}

@@ -107,7 +107,7 @@ class GeneralDelta(_MatrixStateMixer):
                         rate=a, rate_bias=self.a_bias)
         out = self.rt.empty(n, c)
         ops.recurrent_scan(r, k, v, w, g, self.norm_w, self.norm_eps, state, ctx.q_start, ctx.positions,
-                           ctx.state_slots, out, self.num_heads, self.head_dim, self.rule, a=a)
+                           ctx.state_slots, out, self.num_heads, self.head_dim, self.rule, a=a, longest=ctx.longest_entry)
         return linear_f32(self.rt, out, self.w_o)
 
 
@@ -158,7 +158,8 @@ class WKV(_MatrixStateMixer):
         ops.lowrank_out(proj[:, 4 * c:4 * c + self.rank], self.w2t, self.w0, w, act="tanh", out_act="double_exp_decay")
         out = self.rt.empty(n, c)
         ops.recurrent_scan(r, k, v, w, g, self.norm_w, self.norm_eps, state[:, h:], ctx.q_start, ctx.positions,
-                           ctx.state_slots, out, self.num_heads, self.head_dim, self.rule, bonus=self.bonus)
+                           ctx.state_slots, out, self.num_heads, self.head_dim, self.rule, bonus=self.bonus,
+                           longest=ctx.longest_entry)
         return linear_f32(self.rt, out, self.w_o)
 
 
@@ -238,7 +239,7 @@ class GatedDelta(Mixer):
                          self.value_dim)
         o = torch.empty(n, self.hv, device=self.rt.device, dtype=torch.float32)
         ops.gated_delta_scan(prep, state, ctx.q_start, ctx.positions, ctx.state_slots, o, H, self.num_kv_heads,
-                             self.head_dim, self.value_dim)
+                             self.head_dim, self.value_dim, longest=ctx.longest_entry)
         out = self.rt.empty(n, self.hv)
         ops.head_norm_gate(o, proj[:, g_off:g_off + self.hv], self.norm_w, self.norm_eps, out, H, self.value_dim, gate="silu")
         return linear_f32(self.rt, out, self.w_o)

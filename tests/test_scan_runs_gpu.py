@@ -1,0 +1,130 @@
+"""Matrix-state recurrences whose rows are cut into runs: against the float64 rules and against the token-by-token kernels,
+at the edges of runs and batches, continuing from states and starting in slots that held rubbish."""
+
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import pytest
+import torch
+
+import plain_makodra as M
+import plain_miberax as P
+
+pytestmark = pytest.mark.gpu
+
+D, EPS = 64, 1e-6
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from dli_amd.kernels import ops as module
+
+    return module
+
+
+def i32(values):
+    return torch.tensor(np.asarray(values), dtype=torch.int32, device="cuda")
+
+
+def cut(monkeypatch, ops, workgroups):
+    monkeypatch.setattr(ops, "RUNS_WORKGROUPS", workgroups)
+    monkeypatch.setattr(ops, "RUNS_FROM_ROWS", 1)   # short entries too
+
+
+# steps: rows that each of three requests brings (0: not in it): runs of 64 and of other multiples of 16, an entry
+# that ends with its run and one row behind it, single tokens beside long portions
+STEPS = [[64, 0, 65], [1, 200, 130], [129, 1, 1], [16, 333, 17], [0, 63, 64]]
+
+
+def test_rule_of_the_cut(ops):
+    assert ops.scan_runs(1, 2048, 32, 2048, True) == (128, 16) and ops.scan_runs(1, 2048, 32, 2048, False) == (64, 32)
+    assert ops.scan_runs(3, 134, 4, 127, True) == (0, 0) and ops.scan_runs(64, 64, 32, 1, False) == (0, 0)
+    for entries, rows, heads, longest in ((1, 128, 2, 128), (7, 900, 32, 333), (40, 1539, 32, 1500), (16, 6000, 64, 375)):
+        run_rows, runs = ops.scan_runs(entries, rows, heads, longest, True)
+        assert run_rows % 16 == 0 and run_rows >= 64 and run_rows * runs >= longest > run_rows * (runs - 1)
+
+
+@pytest.mark.parametrize("workgroups", [1024, 12, 1])   # runs of 64 rows, of 176 and the like, and whole entries
+@pytest.mark.parametrize("rule", ["delta", "bonus"])
+def test_recurrent_scan_in_runs(ops, monkeypatch, rule, workgroups):
+    cut(monkeypatch, ops, workgroups)
+    H = 3
+    c, total = H * D, [sum(s[i] for s in STEPS) for i in range(3)]
+    gen = torch.Generator().manual_seed(3)
+    data = [{n: torch.randn(t, c, generator=gen) for n in "rkvgwa"} for t in total]
+    bonus, norm_w = 0.5 * torch.randn(H, D, generator=gen), 1 + 0.2 * torch.randn(c, generator=gen)
+    for d in data:
+        if rule == "delta":
+            d["w"], d["a"] = torch.exp(-math.exp(-0.5) * torch.sigmoid(d["w"])), torch.sigmoid(d["a"])
+        else:
+            d["w"] = torch.exp(-torch.exp(2.0 * d["w"]))   # (some keys forget at once: decays of zero)
+    refs = []
+    for d, n in zip(data, total):
+        v = {k: t.double().view(n, H, D) for k, t in d.items()}
+        o = (M.delta_rule(v["r"], v["k"], v["v"], v["w"], v["a"]) if rule == "delta" else
+             M.bonus_rule(v["r"], v["k"], v["v"], v["w"], bonus.double()))[0]
+        g = d["g"].double()
+        refs.append(M.rms(o, EPS).reshape(n, c) * norm_w.double() * torch.sigmoid(g) * (1 if rule == "delta" else g))
+    states = {way: torch.full((4, c * D + 4), 9.0, device="cuda") for way in ("runs", "tokens")}
+    got, at = {way: [[], [], []] for way in states}, [0, 0, 0]
+    for step in STEPS:
+        who = sorted((i for i in range(3) if step[i]), key=lambda i: step[i] != 1)   # single tokens first, as the engine does
+        pick = lambda n: torch.cat([data[i][n][at[i]:at[i] + step[i]] for i in who]).cuda()
+        starts = np.cumsum([0] + [step[i] for i in who])
+        args = (i32(starts), i32([p for i in who for p in range(at[i], at[i] + step[i])]), i32([3 - i for i in who]))
+        kw = dict(a=pick("a")) if rule == "delta" else dict(bonus=bonus.cuda())
+        for way, state in states.items():
+            out = torch.empty(starts[-1], c, device="cuda")
+            ops.recurrent_scan(pick("r"), pick("k"), pick("v"), pick("w"), pick("g"), norm_w.cuda(), EPS, state, *args, out, H, D,
+                               ops.RULE_DELTA if rule == "delta" else ops.RULE_BONUS, longest=max(step) if way == "runs" else 0, **kw)
+            for i, a, b in zip(who, starts, starts[1:]):
+                got[way][i].append(out[a:b].cpu().double())
+        at = [a + n for a, n in zip(at, step)]
+    off = {way: max((torch.cat(g) - r).abs().max().item() for g, r in zip(got[way], refs)) for way in got}
+    # a row divided by its root mean square: rounding of 2^-24 times the terms of a few hundred decayed sums, in both ways
+    assert off["runs"] < 2e-4 * max(r.abs().max() for r in refs) and off["runs"] < 3 * off["tokens"] + 1e-5, off
+    assert (states["runs"] - states["tokens"]).abs().max() < 1e-4 * states["tokens"].abs().max()
+    assert (states["runs"][:, c * D:] == 9.0).all() and (states["runs"][0] == 9.0).all()   # nobody else's memory
+
+
+@pytest.mark.parametrize("workgroups", [1024, 12, 1])
+@pytest.mark.parametrize("H,G", [(4, 2), (3, 3)])
+def test_gated_delta_in_runs(ops, monkeypatch, H, G, workgroups):
+    cut(monkeypatch, ops, workgroups)
+    qk, hv, total = G * D, H * D, [sum(s[i] for s in STEPS) for i in range(3)]
+    gen = torch.Generator().manual_seed(4)
+    width = 2 * qk + hv + 2 * H
+    data, refs = [], []
+    for n in total:
+        q, k = (P.unit(torch.randn(n, G, D, generator=gen).double()) for _ in "qk")
+        v, beta = torch.randn(n, H, D, generator=gen).double(), torch.rand(n, H, generator=gen).double()
+        g = torch.exp(-torch.rand(n, H, generator=gen).double() ** 4)
+        prep = torch.cat([t.reshape(n, -1) for t in (q, k, v, beta, g)], 1).float()
+        p = prep.double()
+        q, k, v = p[:, :qk].view(n, G, D), p[:, qk:2 * qk].view(n, G, D), p[:, 2 * qk:2 * qk + hv].view(n, H, D)
+        rep = H // G
+        refs.append(P.gated_delta_rule(q.repeat_interleave(rep, 1), k.repeat_interleave(rep, 1), v, p[:, -2 * H:-H], p[:, -H:]))
+        data.append(prep)
+    wide = -(-width // 4) * 4 + 4   # rows on 16-byte boundaries (else the token-by-token kernel takes them)
+    states = {way: torch.full((4, hv * D + 8), 9.0, device="cuda") for way in ("runs", "tokens")}
+    got, at = {way: [[], [], []] for way in states}, [0, 0, 0]
+    for step in STEPS:
+        who = sorted((i for i in range(3) if step[i]), key=lambda i: step[i] != 1)
+        rows = torch.cat([data[i][at[i]:at[i] + step[i]] for i in who])
+        prep = torch.empty(rows.shape[0], wide, device="cuda")[:, :width]
+        prep.copy_(rows)
+        starts = np.cumsum([0] + [step[i] for i in who])
+        args = (i32(starts), i32([p for i in who for p in range(at[i], at[i] + step[i])]), i32([3 - i for i in who]))
+        for way, state in states.items():
+            o = torch.empty(rows.shape[0], hv, device="cuda")
+            ops.gated_delta_scan(prep, state, *args, o, H, G, D, D, longest=max(step) if way == "runs" else 0)
+            for i, a, b in zip(who, starts, starts[1:]):
+                got[way][i].append(o[a:b].cpu().double())
+        at = [a + n for a, n in zip(at, step)]
+    for way in got:
+        for g, r in zip(got[way], refs):
+            assert (torch.cat(g).view(r.shape) - r).abs().max() < 2e-5 * max(1.0, r.abs().max()), way
+    assert (states["runs"] - states["tokens"]).abs().max() < 2e-5 * states["tokens"].abs().max()
+    assert (states["runs"][:, hv * D:] == 9.0).all() and (states["runs"][0] == 9.0).all()

@@ -1,7 +1,8 @@
 // Attention of grouped heads for the portions of a bfloat16 step, on the matrix cores, keys and values through LDS: a
 // chunked mask, a window that may keep the first positions, a sink (of score 0 or of a score per head), values of another
-// size than keys, value heads shared by several key heads, a sigmoid gate, an unrounded result. (A penalty on the distance,
-// and sizes that this file does not take, are computed by csrc/attention_scored_mfma.hip.)
+// size than keys, value heads shared by several key heads, a sigmoid gate, an unrounded result, a penalty on the distance per
+// query head. (Sizes that this file does not take are computed by csrc/attention_scored_mfma.hip, which reads every head's keys
+// from memory: 2,048 tokens, 32 heads of 64 on 8, sink, gate and penalty: 324 us there, 125 here.)
 //
 // A kv head's query heads read the same keys, so the rows of a tile are (token, query head) pairs: as many whole tokens of an
 // entry as fit 64 rows (one token, 64 heads at a time, where a group is larger); a wave takes 16 of them. The tile's
@@ -36,6 +37,7 @@ struct GroupedArgs {
   float scale; int window, chunk, keep_first, sink;
   const float* sinks;
   const float* gate; int64_t gate_stride;
+  const float *r1, *r2;                        // r1[h] log(1 + r2[h] distance) off the scaled score (both or neither)
 };
 
 // The first position that `pos` sees, kept ones aside.
@@ -45,8 +47,9 @@ __device__ __forceinline__ int ag_low(const GroupedArgs& a, int pos) {
   return lo;
 }
 
-// Keys of up to 32 DC components, values of up to 16 VT.
-template <int DC, int VT>
+// Keys of up to 32 DC components, values of up to 16 VT; PEN: with the penalty on the distance. (Its logarithm, one of the
+// quarter-rate operations, is made beside each exponential; scores are then scaled before they are compared.)
+template <int DC, int VT, bool PEN>
 __global__ __launch_bounds__(256, 2) void attention_grouped_kernel(GroupedArgs a) {
   constexpr float LOG2E = 1.4426950408889634f;
   constexpr int LD = 32 * DC + 8, LV = AG_KEYS + 8;
@@ -84,7 +87,8 @@ __global__ __launch_bounds__(256, 2) void attention_grouped_kernel(GroupedArgs a
       qb[d] = at < D ? *reinterpret_cast<const ag_bf8*>(qr + at) : ag_bf8{};
     }
   }
-  const float scale2 = a.scale * LOG2E;
+  const float scale_q = a.scale * LOG2E, scale2 = PEN ? 1.f : scale_q;
+  const float r1 = PEN ? a.r1[head] : 0.f, r2 = PEN ? a.r2[head] : 0.f;
   const float not_seen = scale2 >= 0.f ? -INFINITY : INFINITY;       // times the scale: minus infinity
   ag_f4 acc[VT];
 #pragma unroll
@@ -166,6 +170,15 @@ __global__ __launch_bounds__(256, 2) void attention_grouped_kernel(GroupedArgs a
           s[sub] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
               *reinterpret_cast<const ag_bf8*>(&kb[(16 * sub + col) * LD + 32 * d + 8 * grp]), qb[d], s[sub], 0, 0, 0);
       // s[sub][i]: key j0 + 16 sub + 4 grp + i against row `col`
+      if constexpr (PEN) {
+#pragma unroll
+        for (int sub = 0; sub < 4; ++sub)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float dist = (float)max(pos - (j0 + 16 * sub + 4 * grp + i), 0);
+            s[sub][i] = fmaf(s[sub][i], scale_q, -r1 * __builtin_amdgcn_logf(fmaf(r2, dist, 1.f)));
+          }
+      }
       if (j0 + AG_KEYS - 1 > w_lo || j0 < w_low_hi) {                // (else every key is seen by every row)
 #pragma unroll
         for (int sub = 0; sub < 4; ++sub)
@@ -243,7 +256,11 @@ __global__ __launch_bounds__(256, 2) void attention_grouped_kernel(GroupedArgs a
 
 template <int DC>
 static int launch_grouped(const GroupedArgs& a, const dim3& grid, hipStream_t stream) {
-#define VCASE(VT) case VT: attention_grouped_kernel<DC, VT><<<grid, 256, 0, stream>>>(a); break;
+#define VCASE(VT)                                                                             \
+  case VT:                                                                                    \
+    if (a.r1 != nullptr) attention_grouped_kernel<DC, VT, true><<<grid, 256, 0, stream>>>(a); \
+    else attention_grouped_kernel<DC, VT, false><<<grid, 256, 0, stream>>>(a);                \
+    break;
   switch ((a.V + 15) / 16) {
     VCASE(1) VCASE(2) VCASE(3) VCASE(4) VCASE(5) VCASE(6)
     case 7: VCASE(8)
@@ -271,11 +288,12 @@ int dli_attention_grouped(const void* q, int64_t q_stride, const void* k_pages, 
                           const int* q_start, const int* kv_len, const int* block_tables, int table_stride, const int* tile_entry,
                           const int* tile_q0, int tiles, int q_heads, int kv_heads, int v_heads, int head_dim, int value_dim,
                           int page_size, float scale, int window, int chunk, int keep_first, int sink, const float* sinks,
-                          const float* gate, int64_t gate_stride, int out_is_f32, hipStream_t stream) {
+                          const float* gate, int64_t gate_stride, const float* r1, const float* r2, int out_is_f32,
+                          hipStream_t stream) {
   if (tiles <= 0) return DLI_OK;
   if (!dli_attention_grouped_supports(head_dim, value_dim, page_size) || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads ||
       v_heads <= 0 || kv_heads % v_heads || kv_heads > 65535 || table_stride <= 0 || window < 0 || chunk < 0 || keep_first < 0 ||
-      tile_entry == nullptr || tile_q0 == nullptr || q_stride % 8 || out_stride % 4 ||
+      (r1 == nullptr) != (r2 == nullptr) || tile_entry == nullptr || tile_q0 == nullptr || q_stride % 8 || out_stride % 4 ||
       ((uintptr_t)q | (uintptr_t)k_pages | (uintptr_t)v_pages | (uintptr_t)out) % 16)
     return DLI_ERR_ARGUMENT;
   GroupedArgs a;
@@ -284,6 +302,7 @@ int dli_attention_grouped(const void* q, int64_t q_stride, const void* k_pages, 
   a.block_tables = block_tables; a.table_stride = table_stride; a.tile_entry = tile_entry; a.tile_q0 = tile_q0; a.q_heads = q_heads;
   a.kv_heads = kv_heads; a.v_heads = v_heads; a.D = head_dim; a.V = value_dim; a.page_size = page_size; a.scale = scale;
   a.window = window; a.chunk = chunk; a.keep_first = keep_first; a.sink = sink; a.sinks = sinks; a.gate = gate; a.gate_stride = gate_stride;
+  a.r1 = r1; a.r2 = r2;
   a.tile_tokens = dli_attention_grouped_tile_tokens(q_heads, kv_heads);
   const int group = q_heads / kv_heads;
   const dim3 grid(tiles, kv_heads, (a.tile_tokens * group + AG_ROWS - 1) / AG_ROWS);

@@ -114,7 +114,7 @@ _SIGNATURES = {
     "dli_attention_grouped_tile_tokens": [_c_int, _c_int],
     "dli_attention_grouped": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int,
                               _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_int, _c_int, _c_ptr,
-                              _c_ptr, _c_i64, _c_int, _c_ptr],
+                              _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_ptr],
     "dli_attention_keyvalue_supports": [_c_int, _c_int],
     "dli_attention_keyvalue_tile_tokens": [_c_int, _c_int],
     "dli_attention_keyvalue_splits": [_c_int, _c_int, _c_int, _c_int],
@@ -1773,9 +1773,10 @@ def attention_grouped_tile_tokens(q_heads: int, kv_heads: int) -> int:
 def attention_grouped(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, out: torch.Tensor,
                       q_start: torch.Tensor, kv_len: torch.Tensor, block_tables: torch.Tensor,
                       tile_entry: torch.Tensor, tile_q0: torch.Tensor, q_heads: int, scale: float, *,
-                      window: int = 0, chunk: int = 0, sink: bool = False, gate: Optional[torch.Tensor] = None,
-                      keep_first: int = 0, sinks: Optional[torch.Tensor] = None) -> None:
-    """:func:`attention_scored` without a penalty on the distance, for the portions of a bfloat16 step, keys and values
+                      window: int = 0, chunk: int = 0, sink: bool = False, r1: Optional[torch.Tensor] = None,
+                      r2: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None, keep_first: int = 0,
+                      sinks: Optional[torch.Tensor] = None) -> None:
+    """:func:`attention_scored` for the portions of a bfloat16 step, keys and values
     passing through LDS once for all query heads of a kv head: tiles of :func:`attention_grouped_tile_tokens` tokens, sizes
     that :func:`attention_grouped_supports` takes."""
     _dense(k_pages, "k_pages", torch.bfloat16, 4)
@@ -1799,9 +1800,11 @@ def attention_grouped(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Ten
     entries = kv_len.shape[0]
     _require(q_start.shape[0] == entries + 1 and block_tables.shape[0] >= entries and tile_entry.shape == tile_q0.shape,
              "q_start/kv_len/block_tables or the tile lists disagree")
-    if sinks is not None:
-        _dense(sinks, "sinks", torch.float32, 1)
-        _require(sinks.shape[0] == q_heads, "sinks must hold one value per query head")
+    _require((r1 is None) == (r2 is None), "r1 and r2 come together")
+    for name, t in (("r1", r1), ("r2", r2), ("sinks", sinks)):
+        if t is not None:
+            _dense(t, name, torch.float32, 1)
+            _require(t.shape[0] == q_heads, f"{name} must hold one value per query head")
     gate_stride = 0
     if gate is not None:
         _f32_rows(gate, "gate")
@@ -1811,7 +1814,7 @@ def attention_grouped(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Ten
         _ptr(q), q.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(out), out.stride(0), _ptr(q_start), _ptr(kv_len), _ptr(block_tables),
         block_tables.stride(0), _ptr(tile_entry), _ptr(tile_q0), tile_entry.shape[0], q_heads, kv_heads, v_heads, head_dim, value_dim,
         page_size, float(scale), int(window), int(chunk), int(keep_first), int(bool(sink)), _ptr(sinks), _ptr(gate), gate_stride,
-        int(out32), _stream()), "attention_grouped")
+        _ptr(r1), _ptr(r2), int(out32), _stream()), "attention_grouped")
 
 
 def attention_keyvalue_supports(head_dim: int, value_dim: int, dtype: torch.dtype) -> bool:

@@ -167,13 +167,17 @@ __global__ __launch_bounds__(256) void rope_kv_write_token_kernel(
   }
 }
 
-// Many tokens, vector form: a workgroup takes ROWS consecutive tokens and moves 16 bytes per
+// Many tokens, vector form: a workgroup takes ROWS consecutive tokens and its share of the heads (blockIdx.y of gridDim.y, the kv
+// heads' count a multiple of it) and moves 16 bytes per
 // access. v goes through LDS so that one thread writes a dimension's ROWS keys as one contiguous
 // run of the transposed page when the tokens' slots are consecutive in one page (a prompt's
 // portion, mostly); otherwise element by element. Workgroups that share a page's runs are placed
 // on the same XCD (workgroup b runs on XCD b % 8), so that a page's cache lines are completed in
 // one L2 instead of being written back in pieces from several.
 // Needs rotary_dim/2, head_dim and row_stride to be multiples of the 16-byte vector.
+// What bounds it: the trips to memory of a workgroup, one after the other, where there are few of them; hence the shares.
+// 755 rows of several requests, 32 heads on 32: 34 us with one share and 13.0 with four (two workgroups a compute unit; 16.7 at
+// one, 11.8 at four, 17.7 at sixteen), 2,048 rows of a prompt, 32 heads on 8: 11.7 -> 7.9 (8.0, 9.4, 12.0), 8,192 rows 18.4.
 template <typename T, int ROWS>
 __global__ __launch_bounds__(256) void rope_kv_write_rows_kernel(
     T* __restrict__ qkv, int64_t row_stride, const int* __restrict__ positions,
@@ -184,7 +188,9 @@ __global__ __launch_bounds__(256) void rope_kv_write_rows_kernel(
   typedef T vec_t __attribute__((ext_vector_type(VEC)));
   extern __shared__ __align__(16) unsigned char rope_lds[];
   __shared__ int slot_s[ROWS];
-  const int half = rotary_dim / 2, rest = head_dim - rotary_dim, v_width = kv_heads * head_dim;
+  const int half = rotary_dim / 2, rest = head_dim - rotary_dim;
+  const int qn = q_heads / gridDim.y, q_first = blockIdx.y * qn, kn = kv_heads / gridDim.y, kv_first = blockIdx.y * kn;
+  const int v_width = kn * head_dim;   // this workgroup's heads
   float* cs = reinterpret_cast<float*>(rope_lds);
   float* sn = cs + ROWS * half;
   T* vs = reinterpret_cast<T*>(sn + ROWS * half);
@@ -200,15 +206,16 @@ __global__ __launch_bounds__(256) void rope_kv_write_rows_kernel(
   // with the same run + half. A thread asks for U chunk pairs at once, the first U before the
   // angles are computed, so that the workgroup is few trips to memory long.
   constexpr int U = 5;
-  const int chunks = half / VEC, rot_heads = q_heads + kv_heads;
+  const int chunks = half / VEC, rot_heads = qn + kn;
   const int total = rows * rot_heads * chunks;
+  const auto head_of = [&](int own) { return own < qn ? q_first + own : q_heads + kv_first + own - qn; };
   vec_t lo[U], hi[U];
   int idx0 = threadIdx.x;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int idx = min(idx0 + u * (int)blockDim.x, total - 1);
     const int r = idx / (rot_heads * chunks), rem = idx - r * rot_heads * chunks;
-    const T* h = base + r * row_stride + (int64_t)(rem / chunks) * head_dim + (rem % chunks) * VEC;
+    const T* h = base + r * row_stride + (int64_t)head_of(rem / chunks) * head_dim + (rem % chunks) * VEC;
     lo[u] = *reinterpret_cast<const vec_t*>(h);
     hi[u] = *reinterpret_cast<const vec_t*>(h + half);
   }
@@ -232,7 +239,7 @@ __global__ __launch_bounds__(256) void rope_kv_write_rows_kernel(
     for (int idx = threadIdx.x; idx < rows * v_chunks; idx += blockDim.x) {
       const int r = idx / v_chunks, c = idx - r * v_chunks;
       *reinterpret_cast<vec_t*>(vs + r * v_width + c * VEC) = *reinterpret_cast<const vec_t*>(
-          base + r * row_stride + (int64_t)(q_heads + kv_heads) * head_dim + c * VEC);
+          base + r * row_stride + (int64_t)(q_heads + kv_heads + kv_first) * head_dim + c * VEC);
     }
   }
   __syncthreads();
@@ -243,7 +250,7 @@ __global__ __launch_bounds__(256) void rope_kv_write_rows_kernel(
       const int idx = idx0 + u * (int)blockDim.x;
       if (idx >= total) break;
       const int r = idx / (rot_heads * chunks), rem = idx - r * rot_heads * chunks;
-      const int head = rem / chunks, j = rem - head * chunks;
+      const int own = rem / chunks, j = rem - own * chunks, head = head_of(own);
       const int slot = slot_s[r];
       if (head >= q_heads && slot < 0) continue;
       vec_t ylo, yhi;
@@ -266,16 +273,16 @@ __global__ __launch_bounds__(256) void rope_kv_write_rows_kernel(
     for (int u = 0; u < U; ++u) {
       const int idx = min(idx0 + u * (int)blockDim.x, total - 1);
       const int r = idx / (rot_heads * chunks), rem = idx - r * rot_heads * chunks;
-      const T* h = base + r * row_stride + (int64_t)(rem / chunks) * head_dim + (rem % chunks) * VEC;
+      const T* h = base + r * row_stride + (int64_t)head_of(rem / chunks) * head_dim + (rem % chunks) * VEC;
       lo[u] = *reinterpret_cast<const vec_t*>(h);
       hi[u] = *reinterpret_cast<const vec_t*>(h + half);
     }
   }
   if (!pages) return;
   // the part of k beyond the rotary dimensions passes through
-  for (int idx = threadIdx.x; idx < rows * kv_heads * rest; idx += blockDim.x) {
-    const int r = idx / (kv_heads * rest), rem = idx - r * kv_heads * rest;
-    const int hk = rem / rest, i = rotary_dim + rem - hk * rest;
+  for (int idx = threadIdx.x; idx < rows * kn * rest; idx += blockDim.x) {
+    const int r = idx / (kn * rest), rem = idx - r * kn * rest;
+    const int own = rem / rest, hk = kv_first + own, i = rotary_dim + rem - own * rest;
     const int slot = slot_s[r];
     if (slot < 0) continue;
     k_pages[(((int64_t)(slot / page_size) * kv_heads + hk) * page_size + slot % page_size) * head_dim + i] =
@@ -291,7 +298,7 @@ __global__ __launch_bounds__(256) void rope_kv_write_rows_kernel(
     const int64_t page = slot0 / page_size;
     const int off = slot0 % page_size;
     for (int c = threadIdx.x; c < v_width; c += blockDim.x) {
-      const int hk = c / head_dim, i = c - hk * head_dim;
+      const int own = c / head_dim, hk = kv_first + own, i = c - own * head_dim;
       T* dst = v_pages + ((page * kv_heads + hk) * head_dim + i) * page_size + off;
 #pragma unroll
       for (int r0 = 0; r0 < ROWS; r0 += VEC) {
@@ -306,7 +313,7 @@ __global__ __launch_bounds__(256) void rope_kv_write_rows_kernel(
       const int r = idx / v_width, c = idx - r * v_width;
       const int slot = slot_s[r];
       if (slot < 0) continue;
-      const int hk = c / head_dim, i = c - hk * head_dim;
+      const int own = c / head_dim, hk = kv_first + own, i = c - own * head_dim;
       v_pages[(((int64_t)(slot / page_size) * kv_heads + hk) * head_dim + i) * page_size + slot % page_size] = vs[idx];
     }
   }
@@ -356,12 +363,15 @@ extern "C" int dli_rope_kv_write(void* qkv, int64_t row_stride, const int* posit
     // the vector form where the sizes are multiples of its 16 bytes and a workgroup's v rows fit LDS
     constexpr int ROWS = 8;
     const int vec = is_bf16 ? 8 : 4, elem = is_bf16 ? 2 : 4;
-    const size_t lds = (size_t)2 * ROWS * half * sizeof(float) + (size_t)ROWS * kv_heads * head_dim * elem;
+    const int groups = (tokens + ROWS - 1) / ROWS;
+    // shares of the heads: as many as the kv heads and q heads allow, up to two workgroups a compute unit in all
+    int shares = 1;
+    while (kv_heads % (2 * shares) == 0 && q_heads % (2 * shares) == 0 && (int64_t)groups * 2 * shares <= 2 * dli_compute_units()) shares *= 2;
+    const size_t lds = (size_t)2 * ROWS * half * sizeof(float) + (size_t)ROWS * (kv_heads / shares) * head_dim * elem;
     if (half > 0 && half % vec == 0 && head_dim % vec == 0 && row_stride % vec == 0 &&
         (uintptr_t)qkv % 16 == 0 && (uintptr_t)k_pages % 16 == 0 && (uintptr_t)v_pages % 16 == 0 &&
         lds <= 48 * 1024) {
-      const int groups = (tokens + ROWS - 1) / ROWS;
-      const int grid = (groups + 15) / 16 * 16;  // the XCD-aware order permutes blocks of 16
+      const dim3 grid((groups + 15) / 16 * 16, shares);  // the XCD-aware order permutes blocks of 16
       if (is_bf16)
         rope_kv_write_rows_kernel<bf16_t, ROWS><<<grid, 256, lds, stream>>>(
             (bf16_t*)qkv, row_stride, positions, inv_freq, rotary_dim, slots, (bf16_t*)k_pages,

@@ -32,6 +32,7 @@
 //
 // Page layout: K [pages][kv_heads][page_size][head_dim], V [pages][kv_heads][value_dim][page_size].
 #include "attention_f32.h"
+#include "attention_singles.h"
 #include "common.h"
 
 struct ScoreChanges {
@@ -585,8 +586,21 @@ static int attention_scored(const void* q, int64_t q_stride, const void* k_pages
     return DLI_ERR_ARGUMENT;
   const ScoreChanges sc = {chunk, sink, r1, r2, value_dim, gate, gate_stride, keep_first, v_heads, out32, sinks};
   if (tile_entry == nullptr) {
-    // every entry is one row: the kernel whose lanes own keys, then value columns
+    // every entry is one row: the matrix cores for bfloat16 pages of their sizes, else the kernel whose lanes own keys, then
+    // value columns
     const int group = q_heads / kv_heads;
+    if (is_bf16 && !kv && attention_singles_takes(q, q_stride, k_pages, v_pages, head_dim, value_dim, page_size)) {
+      if (parts == nullptr || splits < 1) splits = 1;
+      if ((int64_t)tiles * splits > 0x7fffffff) return DLI_ERR_ARGUMENT;
+      const SinglesArgs a = {(const bf16_t*)q, q_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages, (bf16_t*)out, out32, out_stride,
+                             kv_len, block_tables, table_stride, q_heads, kv_heads, v_heads, head_dim, value_dim, page_size, scale,
+                             window, chunk, keep_first, sink, r1, r2, sinks, gate, gate_stride, parts, splits};
+      const int status = attention_singles(a, tiles, stream);
+      if (status != DLI_OK || splits == 1) return status;
+      attention_scored_merge_kernel<bf16_t><<<dim3(tiles, q_heads), value_dim <= 64 ? 64 : 128, 0, stream>>>(
+          parts, splits, q_heads, value_dim, gate, gate_stride, (bf16_t*)out, out_stride, out32);
+      return dli_launch_status();
+    }
 #define DECODE_ARGS                                                                                      \
   q, q_stride, k_pages, v_pages, out, out_stride, kv_len, block_tables, table_stride, tiles, q_heads,   \
       kv_heads, head_dim, page_size, scale, window, sc, parts, splits, stream
@@ -642,14 +656,22 @@ extern "C" int dli_attention_scored(const void* q, int64_t q_stride, const void*
 
 // How many workgroups share the keys of an (entry, group of query heads) in a step of single tokens: as
 // many as bring the launch to about two workgroups a compute unit, sixteen at most. It depends on the
-// heads and the number of entries, never on their lengths. A step of many entries fills the chip by
+// heads and the number of entries (on the matrix cores, on the table's width too), never on their lengths. A step of many entries fills the chip by
 // itself and is not cut (cutting it costs more than it gains).
-extern "C" int dli_attention_scored_splits(int q_heads, int kv_heads, int entries) {
+// `most_keys`: the most keys that an entry can see here; `singles`: whether the matrix cores take the step's pages and sizes.
+extern "C" int dli_attention_scored_splits(int q_heads, int kv_heads, int entries, int64_t most_keys, int singles) {
   if (q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads != 0 || entries <= 0) return 1;
+  if (singles) return attention_singles_splits(q_heads, kv_heads, entries, most_keys);
   const int group = q_heads / kv_heads, gq = group == 1 ? 1 : group <= 4 ? 4 : 8;
   const int64_t workgroups = (int64_t)entries * kv_heads * ((group + gq - 1) / gq);
   const int64_t splits = 512 / workgroups;
   return splits < 1 ? 1 : splits > 16 ? 16 : (int)splits;
+}
+
+extern "C" int dli_attention_singles_takes(const void* q, int64_t q_stride, const void* k_pages, const void* v_pages, int head_dim,
+                                           int value_dim, int page_size) {
+  return v_pages != nullptr && head_dim > 0 && value_dim > 0 && page_size > 0 &&
+         attention_singles_takes(q, q_stride, k_pages, v_pages, head_dim, value_dim, page_size);
 }
 
 // A step of single tokens (every entry one row) with each entry's keys cut over `splits` workgroups:

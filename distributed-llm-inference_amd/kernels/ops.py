@@ -102,7 +102,8 @@ _SIGNATURES = {
     "dli_attention_scored": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr,
                              _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_int, _c_ptr,
                              _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr],
-    "dli_attention_scored_splits": [_c_int, _c_int, _c_int],
+    "dli_attention_scored_splits": [_c_int, _c_int, _c_int, _c_i64, _c_int],
+    "dli_attention_singles_takes": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_int, _c_int],
     "dli_attention_scored_single": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int,
                                     _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_i64,
                                     _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr],
@@ -1684,8 +1685,14 @@ def attention_scored(q: torch.Tensor, k_pages: torch.Tensor, v_pages: Optional[t
         gate_stride = gate.stride(0)
     if tile_entry is None:
         # few (kv head, group of query heads) pairs an entry: an entry's keys are cut over several workgroups
-        # (a number that the heads and the number of entries decide), whose shares a second kernel adds up
-        splits = int(library().dli_attention_scored_splits(q_heads, kv_heads, entries))
+        # (a number that the heads, the number of entries and what they can see at most decide), whose shares a second
+        # kernel adds up
+        singles = dtype == torch.bfloat16 and bool(library().dli_attention_singles_takes(
+            _ptr(q), q.stride(0), _ptr(k_pages), _ptr(v_pages), head_dim, value_dim, page_size))
+        most = block_tables.shape[1] * page_size
+        most = min(most, chunk) if chunk else most
+        most = min(most, window + keep_first) if window else most
+        splits = int(library().dli_attention_scored_splits(q_heads, kv_heads, entries, most, int(singles)))
         if splits > 1:
             parts = torch.empty(entries * q_heads * splits * (value_dim + 2), device=q.device, dtype=torch.float32)
             _check(library().dli_attention_scored_single(

@@ -656,8 +656,8 @@ extern "C" int dli_attention_scored(const void* q, int64_t q_stride, const void*
 
 // How many workgroups share the keys of an (entry, group of query heads) in a step of single tokens: as
 // many as bring the launch to about two workgroups a compute unit, sixteen at most. It depends on the
-// heads and the number of entries (on the matrix cores, on the table's width too), never on their lengths. A step of many entries fills the chip by
-// itself and is not cut (cutting it costs more than it gains).
+// heads and the number of entries (on the matrix cores, on the table's width too), never on their
+// lengths. A step of many entries fills the chip by itself and is not cut (cutting it costs more than it gains).
 // `most_keys`: the most keys that an entry can see here; `singles`: whether the matrix cores take the step's pages and sizes.
 extern "C" int dli_attention_scored_splits(int q_heads, int kv_heads, int entries, int64_t most_keys, int singles) {
   if (q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads != 0 || entries <= 0) return 1;

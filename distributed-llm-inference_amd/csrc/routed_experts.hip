@@ -331,10 +331,10 @@ __global__ __launch_bounds__(256) void expert_down_kernel(ExpertArgs p, const T*
 // workgroup of four waves takes 64 NB features, each wave 16 NB of them for all rows of the tile.
 // v_mfma_f32_16x16x32_bf16 with the weights as the first operand: lane l supplies feature l % 16 of a block and row
 // l % 16 of each block of 16 rows, and the eight k values 8 (l / 16) .. + 7 of a step of 32, read straight from memory (16
-// bytes a lane and operand; the rows of a tile are re-read by the four waves from the cache); the operands of the next DEPTH
-// steps are on their way while a step's products are issued. A lane's results are four neighbouring features of one row.
+// bytes a lane and operand; the rows of a tile are re-read by the four waves from the cache); the operands of the next
+// step are on their way while a step's products are issued. A lane's results are four neighbouring features of one row.
 // Every output sums its k in ascending steps of 32 whatever its tile, so a row's result depends on
-// nothing beside the row. Few rows an expert (MB 1) wait for the weights alone: one block of features a wave, many steps ahead.
+// nothing beside the row.
 #define EXM_BM 64
 #define EXM_FEW 16
 typedef __bf16 exm_bf16x8 __attribute__((ext_vector_type(8)));
@@ -342,7 +342,94 @@ typedef float exm_float4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ exm_bf16x8 exm_load(const bf16_t* p) { return *reinterpret_cast<const exm_bf16x8*>(p); }
 
-template <int MB, int NB, int DEPTH>
+// Few rows an expert: the products wait for the weights alone. Lanes that read 16 rows at once, as the operands ask for them, get
+// a quarter of the cache's rate and 16 pages a load, so the weights pass through LDS: a workgroup takes 32 rows of weights (16
+// gate rows and their 16 up rows, or 32 of the down product) and up to 16 rows of the input, in chunks of 256 k, a half wave a row
+// (512 neighbouring bytes), EXF_AHEAD chunks on their way in registers and two in LDS; two of the four waves issue the products.
+// Piece p (16 bytes) of row r lies at place p ^ (r % 16), so that the 16 rows of an operand lie in different banks. Sums run over
+// k in ascending steps of 32, as in the other kernels, and have the same bits.
+// Us of the up and down product with a wave a block of 16 features, eight steps ahead -> now: 32 experts of 1,024 on 2,048, 2 rows
+// (8 experts, 67 and 34 MB) 38.7 -> 15.1 and 9.1 -> 8.4, 32 rows (260 MB) 68 -> 51; 64 experts of 1,408, 32 rows (704 MB) 157 ->
+// 117 (6.0 TB/s); 8 of 2,048 on 4,096, 1 row (67 MB) 72.5 -> 17.3. Four chunks ahead: the same.
+#define EXF_K 256
+#define EXF_AHEAD 3
+template <bool UP>
+__global__ __launch_bounds__(256) void expert_few_kernel(ExpertArgs p, const bf16_t* __restrict__ x, int64_t x_stride,
+                                                         const bf16_t* __restrict__ w0, const bf16_t* __restrict__ w1,
+                                                         bf16_t* __restrict__ y, float* __restrict__ z, float limit, float alpha,
+                                                         float up_shift) {
+  const int tile = blockIdx.x;
+  if (tile >= p.tile_count[0]) return;
+  __shared__ __attribute__((aligned(16))) bf16_t sm[2][48][EXF_K];
+  __shared__ __attribute__((aligned(16))) float up_sums[64][4];
+  const int e = p.tile_expert[tile], r0 = p.tile_row0[tile], rend = min(p.offsets[e + 1], r0 + 16);
+  const int depth = UP ? p.width : p.ff, features = UP ? p.ff : p.width, n0 = blockIdx.y * (UP ? 16 : 32);
+  const int at_row = threadIdx.x / 32, at = threadIdx.x % 32;
+  const bf16_t* src[6];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {                                                  // (a feature past the end repeats the last)
+    const int f = at_row + 8 * i, n = min(n0 + (UP ? f % 16 : f), features - 1);
+    src[i] = (UP && f >= 16 ? w1 : w0) + ((int64_t)e * features + n) * depth;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {                                                  // (a row past the end repeats the last)
+    const int r = min(r0 + at_row + 8 * i, rend - 1);
+    src[4 + i] = x + (int64_t)(UP ? p.order[r] / p.top : r) * x_stride;
+  }
+  const int lane = threadIdx.x % DLI_WAVE, wave = threadIdx.x / DLI_WAVE, c = lane % 16, g = lane / 16;
+  const int chunks = (depth + EXF_K - 1) / EXF_K;
+  exm_bf16x8 held[EXF_AHEAD][6];
+  auto fetch = [&](int j, int chunk) {                                           // (past the end: pieces that no product takes)
+    const int k0 = min(chunk, chunks - 1) * EXF_K;
+#pragma unroll
+    for (int i = 0; i < 6; ++i) held[j][i] = exm_load(src[i] + min(k0 + 8 * (at ^ ((at_row + 8 * i) % 16)), depth - 8));
+  };
+#pragma unroll
+  for (int j = 0; j < EXF_AHEAD; ++j) fetch(j, j);
+  exm_float4 acc = {0.f, 0.f, 0.f, 0.f};
+  int buffer = 0;
+  for (int chunk0 = 0; chunk0 < chunks; chunk0 += EXF_AHEAD) {
+#pragma unroll
+    for (int j = 0; j < EXF_AHEAD; ++j) {
+      const int chunk = chunk0 + j;
+      if (chunk < chunks) {                                                      // (the same in all threads)
+#pragma unroll
+        for (int i = 0; i < 6; ++i) *reinterpret_cast<exm_bf16x8*>(&sm[buffer][at_row + 8 * i][8 * at]) = held[j][i];
+        fetch(j, chunk + EXF_AHEAD);
+        __syncthreads();
+        if (wave < 2) {
+          const int steps = min(EXF_K, depth - chunk * EXF_K) / 32;
+#pragma unroll
+          for (int s = 0; s < EXF_K / 32; ++s) {
+            if (s < steps) {
+              const int place = 8 * ((4 * s + g) ^ c);
+              acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(exm_load(&sm[buffer][16 * wave + c][place]), exm_load(&sm[buffer][32 + c][place]),
+                                                            acc, 0, 0, 0);
+            }
+          }
+        }
+        buffer ^= 1;
+      }
+    }
+  }
+  // a lane's results are four neighbouring features of row c
+  if (UP) {
+    if (wave == 1) *reinterpret_cast<exm_float4*>(up_sums[lane]) = acc;
+    __syncthreads();
+  }
+  const int r = r0 + c, n = n0 + (UP ? 0 : 16 * wave) + 4 * g;
+  if (wave >= (UP ? 1 : 2) || r >= rend || n >= features) return;               // (features come in fours)
+  if (UP) {
+    const float iw = p.in_weight != nullptr ? p.in_weight[p.order[r]] : 1.f;
+    const exm_float4 up = *reinterpret_cast<const exm_float4*>(up_sums[lane]);
+    for (int i = 0; i < 4; ++i) y[(int64_t)r * p.ff + n + i] = (bf16_t)clamped_glu(iw * acc[i], iw * up[i], limit, alpha, up_shift);
+  } else {
+    const int64_t slot = p.order[r];
+    for (int i = 0; i < 4; ++i) z[slot * p.width + n + i] = acc[i];
+  }
+}
+
+template <int MB, int NB>
 __global__ __launch_bounds__(256) void expert_up_mfma_kernel(ExpertArgs p, const bf16_t* __restrict__ h, int64_t h_stride,
                                                              const bf16_t* __restrict__ w_gate,
                                                              const bf16_t* __restrict__ w_up, bf16_t* __restrict__ y,
@@ -371,34 +458,28 @@ __global__ __launch_bounds__(256) void expert_up_mfma_kernel(ExpertArgs p, const
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) accg[nb][mb] = accu[nb][mb] = exm_float4{0.f, 0.f, 0.f, 0.f};
   const int blocks = (rend - r0 + 15) / 16;                                     // blocks of 16 rows that hold a row
-  exm_bf16x8 a[DEPTH][NB], b[DEPTH][NB], x[DEPTH][MB];
-  auto fetch = [&](int j, int k) {
+  exm_bf16x8 a[NB], b[NB], x[MB];
+  auto fetch = [&](int k) {
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) { a[j][nb] = exm_load(wg[nb] + k); b[j][nb] = exm_load(wu[nb] + k); }
+    for (int nb = 0; nb < NB; ++nb) { a[nb] = exm_load(wg[nb] + k); b[nb] = exm_load(wu[nb] + k); }
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) x[j][mb] = exm_load(xr[mb] + k);             // (unconditional: clamped rows are valid memory)
+    for (int mb = 0; mb < MB; ++mb) x[mb] = exm_load(xr[mb] + k);                // (unconditional: clamped rows are valid memory)
   };
+  fetch(0);
+  for (int k = 0; k < p.width; k += 32) {
+    exm_bf16x8 a0[NB], b0[NB], x0[MB];
 #pragma unroll
-  for (int j = 0; j < DEPTH; ++j) fetch(j, min(32 * j, p.width - 32));
-  for (int k0 = 0; k0 < p.width; k0 += 32 * DEPTH) {
+    for (int nb = 0; nb < NB; ++nb) { a0[nb] = a[nb]; b0[nb] = b[nb]; }
 #pragma unroll
-    for (int j = 0; j < DEPTH; ++j) {
-      const int k = k0 + 32 * j;
-      exm_bf16x8 a0[NB], b0[NB], x0[MB];
+    for (int mb = 0; mb < MB; ++mb) x0[mb] = x[mb];
+    fetch(min(k + 32, p.width - 32));                                           // the last turn asks for its own step again
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) { a0[nb] = a[j][nb]; b0[nb] = b[j][nb]; }
+    for (int mb = 0; mb < MB; ++mb) {
+      if (mb < blocks) {
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) x0[mb] = x[j][mb];
-      if (DEPTH > 1 && k >= p.width) x0[0] = exm_bf16x8{};                       // (past the last step: a product of zero)
-      fetch(j, min(k + 32 * DEPTH, p.width - 32));                              // the last turn asks for its own step again
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        if (MB == 1 || mb < blocks) {
-#pragma unroll
-          for (int nb = 0; nb < NB; ++nb) {
-            accg[nb][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[nb], x0[mb], accg[nb][mb], 0, 0, 0);
-            accu[nb][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b0[nb], x0[mb], accu[nb][mb], 0, 0, 0);
-          }
+        for (int nb = 0; nb < NB; ++nb) {
+          accg[nb][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[nb], x0[mb], accg[nb][mb], 0, 0, 0);
+          accu[nb][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b0[nb], x0[mb], accu[nb][mb], 0, 0, 0);
         }
       }
     }
@@ -419,7 +500,7 @@ __global__ __launch_bounds__(256) void expert_up_mfma_kernel(ExpertArgs p, const
   }
 }
 
-template <int MB, int NB, int DEPTH>
+template <int MB, int NB>
 __global__ __launch_bounds__(256) void expert_down_mfma_kernel(ExpertArgs p, const bf16_t* __restrict__ y,
                                                                const bf16_t* __restrict__ w_down, float* __restrict__ z) {
   const int tile = blockIdx.x;
@@ -439,32 +520,26 @@ __global__ __launch_bounds__(256) void expert_down_mfma_kernel(ExpertArgs p, con
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = exm_float4{0.f, 0.f, 0.f, 0.f};
   const int blocks = (rend - r0 + 15) / 16;
-  exm_bf16x8 a[DEPTH][NB], x[DEPTH][MB];
-  auto fetch = [&](int j, int k) {
+  exm_bf16x8 a[NB], x[MB];
+  auto fetch = [&](int k) {
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) a[j][nb] = exm_load(wd[nb] + k);
+    for (int nb = 0; nb < NB; ++nb) a[nb] = exm_load(wd[nb] + k);
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) x[j][mb] = exm_load(yr[mb] + k);
+    for (int mb = 0; mb < MB; ++mb) x[mb] = exm_load(yr[mb] + k);
   };
+  fetch(0);
+  for (int k = 0; k < p.ff; k += 32) {
+    exm_bf16x8 a0[NB], x0[MB];
 #pragma unroll
-  for (int j = 0; j < DEPTH; ++j) fetch(j, min(32 * j, p.ff - 32));
-  for (int k0 = 0; k0 < p.ff; k0 += 32 * DEPTH) {
+    for (int nb = 0; nb < NB; ++nb) a0[nb] = a[nb];
 #pragma unroll
-    for (int j = 0; j < DEPTH; ++j) {
-      const int k = k0 + 32 * j;
-      exm_bf16x8 a0[NB], x0[MB];
+    for (int mb = 0; mb < MB; ++mb) x0[mb] = x[mb];
+    fetch(min(k + 32, p.ff - 32));
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) a0[nb] = a[j][nb];
+    for (int mb = 0; mb < MB; ++mb)
+      if (mb < blocks)
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) x0[mb] = x[j][mb];
-      if (DEPTH > 1 && k >= p.ff) x0[0] = exm_bf16x8{};
-      fetch(j, min(k + 32 * DEPTH, p.ff - 32));
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-        if (MB == 1 || mb < blocks)
-#pragma unroll
-          for (int nb = 0; nb < NB; ++nb) acc[nb][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[nb], x0[mb], acc[nb][mb], 0, 0, 0);
-    }
+        for (int nb = 0; nb < NB; ++nb) acc[nb][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[nb], x0[mb], acc[nb][mb], 0, 0, 0);
   }
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
@@ -690,11 +765,13 @@ static bool expert_tiled(int64_t slots, int experts, int width, int ff, int is_b
   return is_bf16 && width % 128 == 0 && ff % 64 == 0 && slots >= 48 * (int64_t)experts;
 }
 // Few rows an expert: the kernels that wait for the weights alone.
-static bool expert_few(int64_t slots, int experts) { return slots <= 16 * (int64_t)experts; }
+static bool expert_few(int64_t slots, int experts, int width, int ff) {
+  return slots <= 16 * (int64_t)experts && ff <= 16 * 65535 && width <= 16 * 65535;
+}
 int dli_expert_tile_rows(int64_t slots, int experts, int width, int ff, int is_bf16) {
   if (expert_tiled(slots, experts, width, ff, is_bf16)) return EXL_BM;
   if (!expert_mfma(width, ff, is_bf16)) return EX_BM;
-  return expert_few(slots, experts) ? EXM_FEW : EXM_BM;
+  return expert_few(slots, experts, width, ff) ? EXM_FEW : EXM_BM;
 }
 
 // The experts' part of a mixture for `rows` tokens: sort, up product with activation, down product.
@@ -730,16 +807,19 @@ int dli_expert_products(const int* ids, const void* h, int64_t h_stride, const v
                                                                            nullptr, z, width / 128, 0.f, 0.f, 0.f);
     return dli_launch_status();
   }
-  const int bn = !mfma ? EX_BN : expert_few(slots, experts) ? 64 : 128;
+  if (mfma && expert_few(slots, experts, width, ff)) {
+    expert_few_kernel<true><<<dim3(max_tiles, (ff + 15) / 16), 256, 0, stream>>>(p, (const bf16_t*)h, h_stride, (const bf16_t*)w_gate,
+                                                                                 (const bf16_t*)w_up, (bf16_t*)y, nullptr, limit, alpha, up_shift);
+    expert_few_kernel<false><<<dim3(max_tiles, (width + 31) / 32), 256, 0, stream>>>(p, (const bf16_t*)y, ff, (const bf16_t*)w_down, nullptr,
+                                                                                     nullptr, z, 0.f, 0.f, 0.f);
+    return dli_launch_status();
+  }
+  const int bn = mfma ? 128 : EX_BN;
   const dim3 up_grid(max_tiles, (ff + bn - 1) / bn), down_grid(max_tiles, (width + bn - 1) / bn);
-#define EXM_LAUNCH(MB, NB, DU, DD)                                                                                                 \
-  expert_up_mfma_kernel<MB, NB, DU><<<up_grid, 256, 0, stream>>>(p, (const bf16_t*)h, h_stride, (const bf16_t*)w_gate,             \
-                                                                 (const bf16_t*)w_up, (bf16_t*)y, limit, alpha, up_shift);          \
-  expert_down_mfma_kernel<MB, NB, DD><<<down_grid, 256, 0, stream>>>(p, (const bf16_t*)y, (const bf16_t*)w_down, z)
-  if (mfma && expert_few(slots, experts)) {
-    EXM_LAUNCH(1, 1, 8, 8);
-  } else if (mfma) {
-    EXM_LAUNCH(4, 2, 1, 1);
+  if (mfma) {
+    expert_up_mfma_kernel<4, 2><<<up_grid, 256, 0, stream>>>(p, (const bf16_t*)h, h_stride, (const bf16_t*)w_gate, (const bf16_t*)w_up,
+                                                             (bf16_t*)y, limit, alpha, up_shift);
+    expert_down_mfma_kernel<4, 2><<<down_grid, 256, 0, stream>>>(p, (const bf16_t*)y, (const bf16_t*)w_down, z);
   } else if (is_bf16) {
     expert_up_kernel<bf16_t><<<up_grid, 256, 0, stream>>>(p, (const bf16_t*)h, h_stride, (const bf16_t*)w_gate,
                                                           (const bf16_t*)w_up, (bf16_t*)y, limit, alpha, up_shift);

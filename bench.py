@@ -107,7 +107,7 @@ def decode_run(engine, cfg, batch, context, steps, warmup, decode_steps=1):
     # shortened by that many steps so that no request outgrows `context` while the clock runs.
     budget = engine.scheduler.config.max_num_batched_tokens
     slack = slack_for(batch, context, budget)
-    # (the engine has brought this down to what its runner can do: the 32-bit path decodes one token a step)
+    # (the engine has brought this down to what its runner can do: one token a step where no graph is recorded)
     decode_steps = min(decode_steps, engine.scheduler.config.decode_steps)
     # An engine step may decode several tokens of every request (SchedulerConfig.decode_steps): the
     # clock runs over exactly `steps` decode steps of the model, cut into engine steps of 8, 4, 2 or 1

@@ -135,9 +135,13 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_f32_kernel(
   }
 }
 
+extern "C" int dli_attention_f32_supports(int head_dim, int page_size) {
+  return (head_dim == 64 || head_dim == 128) && page_size > 0 && page_size % 16 == 0;
+}
+
 bool attention_f32_takes(const void* q, int64_t q_stride, const void* k_pages, const void* v_pages, const void* out,
                          int64_t out_stride, int head_dim, int page_size) {
-  return (head_dim == 64 || head_dim == 128) && page_size % 16 == 0 && q_stride % 4 == 0 && out_stride % 4 == 0 &&
+  return dli_attention_f32_supports(head_dim, page_size) && q_stride % 4 == 0 && out_stride % 4 == 0 &&
          (((uintptr_t)q | (uintptr_t)k_pages | (uintptr_t)v_pages | (uintptr_t)out) % 16) == 0;
 }
 

@@ -49,8 +49,8 @@ class StepFunction:
                                  if part is not None and hasattr(part, "decode_plan")}.values())
 
     def enable_decode_graphs(self, max_batch: int, max_model_len: int) -> None:
-        """Replay decode-only steps through HIP graphs (bfloat16 with the matrix-core decode path
-        only; other steps run eagerly)."""
+        """Replay decode-only steps through HIP graphs (where every part of the model can be recorded: attention on the
+        matrix cores, in bfloat16 or 32-bit; other steps run eagerly)."""
         from .decode_graph import DecodeGraphs
 
         self.graphs = DecodeGraphs(self, max_batch=max_batch,

@@ -103,6 +103,7 @@ _SIGNATURES = {
                              _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_int, _c_ptr,
                              _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr],
     "dli_attention_scored_splits": [_c_int, _c_int, _c_int, _c_i64, _c_int],
+    "dli_attention_f32_supports": [_c_int, _c_int],
     "dli_attention_singles_takes": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_int, _c_int],
     "dli_attention_scored_single": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int,
                                     _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_i64,
@@ -1621,6 +1622,11 @@ def qk_unit_cache(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, q_out:
         _ptr(proj), proj.stride(0), q_off, k_off, v_off, _ptr(q_out), _ptr(mix), _ptr(v_first_in), _ptr(v_first_out),
         _ptr(slots), _ptr(k_pages), _ptr(v_pages), n, q_heads, kv_heads, dim, vdim, page_size, float(eps),
         _is_bf16(dtype), _stream()), "qk_unit_cache")
+
+
+def attention_f32_supports(head_dim: int, page_size: int, dtype: torch.dtype) -> bool:
+    """Whether :func:`attention_generic` runs these sizes on the matrix cores' 32-bit form."""
+    return dtype == torch.float32 and bool(library().dli_attention_f32_supports(int(head_dim), int(page_size)))
 
 
 def attention_scored(q: torch.Tensor, k_pages: torch.Tensor, v_pages: Optional[torch.Tensor], out: torch.Tensor,

@@ -144,13 +144,18 @@ class GQAttention(Mixer):
     def cache_spec(self) -> Optional[PagedKVSpec]:
         return None if self.shares_kv else PagedKVSpec(self.num_kv_heads, self.head_dim, self.window)
 
+    captures_32_bit = True   # steps of single tokens can be recorded on the 32-bit path too
+
     def graph_capturable(self, page_size: int) -> bool:
-        # the matrix-core decode path is all kernels on the step's device arrays
-        return (self.rt.is_bf16 and ops.attention_mfma_supports(self.head_dim, page_size, self.rt.dtype)
-                and self.position.graph_capturable(page_size))
+        # the matrix-core decode paths are all kernels on the step's device arrays (the 32-bit one's tile list is the same for
+        # every step of single tokens: entry i, query 0)
+        takes = ops.attention_mfma_supports if self.rt.is_bf16 else ops.attention_f32_supports
+        return takes(self.head_dim, page_size, self.rt.dtype) and self.position.graph_capturable(page_size)
 
     def decode_plan(self, requests: int, max_keys: int) -> Optional[int]:
-        """Into how many runs the decode kernel cuts each request's keys in a recorded step."""
+        """Into how many runs the decode kernel cuts each request's keys in a recorded step (the 32-bit kernel cuts none)."""
+        if not self.rt.is_bf16:
+            return None
         return planned_splits(requests, head_tiles(self.num_heads, self.num_kv_heads), max_keys,
                               ops.compute_units(self.rt.device))
 

@@ -78,3 +78,57 @@ def test_attention_f32(ops, qh, kvh, d, bs, window):
     ops.attention_generic(q[last:last + 1].cuda(), kp.cuda(), vp.cuda(), alone, dev([0, 1]), dev([kv_len[e]]),
                           dev([tables[e]]), dev([0]), dev([0]), qh, d ** -0.5, window)
     assert torch.equal(alone[0], out[last])
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_recorded_steps_have_the_eager_steps_bits(tmp_path, head_dim):
+    """Steps of single tokens on the 32-bit path, replayed from graphs against launched one by one: batches that change (padding
+    rows), other work and synchronisations between the replays, pages that are handed on."""
+    import random
+
+    from dli_amd.engine.core import build_core
+    from dli_amd.trace import TraceSession
+    from dli_amd.weights import write_random_model
+
+    cfg = {"model_type": "llama", "architectures": ["LlamaForCausalLM"], "hidden_size": 192, "intermediate_size": 320,
+           "num_hidden_layers": 2, "num_attention_heads": 3, "num_key_value_heads": 1, "head_dim": head_dim, "vocab_size": 301,
+           "rms_norm_eps": 1e-5, "rope_theta": 10000.0, "max_position_embeddings": 512, "tie_word_embeddings": True}
+    write_random_model(tmp_path, cfg, seed=3, std=0.1)
+
+    def run(graphs):
+        core = build_core(tmp_path, num_pages=40, page_size=16, max_seqs=8, dtype="float32", enable_prefix_caching=False,
+                          watermark=0.0)
+        if graphs:
+            core.step.enable_decode_graphs(8, 640)
+            assert core.step.graphs is not None
+        s, rng, outs = TraceSession(core), random.Random(4), []
+        toks = [[rng.randrange(301) for _ in range(n)] for n in (40, 9, 70, 23, 55)]
+        fed, live, pending = {}, [0, 1, 2], [3, 4]
+        for r in live:
+            outs.append(s.step([{"id": r, "tokens": toks[r][:5], "want": [4]}]).float().cpu())
+            fed[r] = 5
+        while live:
+            chosen = [r for r in live if len(live) == 1 or rng.random() > 0.15]
+            if not chosen:
+                continue
+            entries = [{"id": r, "tokens": [toks[r][fed[r]]], "want": [0]} for r in chosen]
+            for r in chosen:
+                fed[r] += 1
+            end = [r for r in chosen if fed[r] == len(toks[r])]
+            outs.append(s.step(entries, end).float().cpu())
+            torch.cuda.synchronize()
+            for r in end:
+                live.remove(r)
+                if pending:
+                    new = pending.pop(0)
+                    outs.append(s.step([{"id": new, "tokens": toks[new][:6], "want": [5]}]).float().cpu())
+                    fed[new] = 6
+                    live.append(new)
+        return outs, core
+
+    eager, _ = run(False)
+    replayed, core = run(True)
+    assert core.step.graphs.replays > 20 and len(core.step.graphs.captured) >= 2
+    assert len(eager) == len(replayed)
+    for i, (a, b) in enumerate(zip(eager, replayed)):
+        assert torch.equal(a, b), (i, float((a - b).abs().max()))

@@ -534,7 +534,17 @@ def skinny_gemm_plan(rows: int, n: int, k: int, epilogue: int, device: torch.dev
             out_feats = n * (2 if epilogue == SKINNY_SWIGLU else 1)
             few = out_feats <= 16 * _units(device)
             if not (tiled and (rows >= 2 or few)):
-                blocks4 = 1 if few else 0
+                if few and k <= 1024:
+                    # Short rows: eight k-waves share at most eight chunks of 128 k. The tile kernel finishes sooner where
+                    # it sums k in as few steps (us for one row, tiles and blocks in shapes 0 and 1, k 576: 576 features
+                    # with the residual 3.3, 4.1, 4.0, 960 stored 3.8, 4.2, 4.5; k 832: 4.5, 4.4, 4.8), else four waves
+                    # on four quads do, which leave no compute unit a second workgroup (gate and up of 1,536 features,
+                    # k 576: 5.5, 5.2, 7.0; k 320: 4.9, 5.2, 7.0).
+                    if k <= {SKINNY_RESIDUAL: 1024, SKINNY_SWIGLU: 448}.get(epilogue, 640):
+                        return "tiles16", 1, -(-n // 16)
+                    blocks4 = 0
+                else:
+                    blocks4 = 1 if few else 0
     if blocks4 is not None:
         feats = int(library().dli_skinny4_tile_features(blocks4, epilogue))
         return "blocks4", blocks4, -(-n // feats)

@@ -145,7 +145,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
       if constexpr (TILED) {
         // the tile's first block, at this lane's 16 bytes of a 1 KB load
         const int tile = min(tile0 + j, (N - 1) / 16) + a * (up_offset / 16);
-        wrow[j][a] = w + (int64_t)tile * 16 * K + lane * 8;
+        wrow[j][a] = w + (int64_t)tile * 16 * (EPI == EPI_QKV ? (K + 127) / 128 * 128 : K) + lane * 8;
       } else {
         const int n = min((tile0 + j) * 16 + col, N - 1) + a * up_offset;
         wrow[j][a] = w + (int64_t)n * K + grp * 32;
@@ -194,8 +194,9 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
 
   // this wave's share of the k steps of 32
   const int steps = K / 32;
-  const int s_begin = TILED ? 4 * (int)((int64_t)(steps / 4) * ks / KS) : (int)((int64_t)steps * ks / KS);
-  const int s_end = TILED ? 4 * (int)((int64_t)(steps / 4) * (ks + 1) / KS) : (int)((int64_t)steps * (ks + 1) / KS);
+  const int whole = EPI == EPI_QKV ? (steps + 3) / 4 : steps / 4;   // (EPI_QKV: the last block may be filled up with zeros)
+  const int s_begin = TILED ? 4 * (int)((int64_t)whole * ks / KS) : (int)((int64_t)steps * ks / KS);
+  const int s_end = TILED ? 4 * (int)((int64_t)whole * (ks + 1) / KS) : (int)((int64_t)steps * (ks + 1) / KS);
   int s = s_begin;
   // Blocks of 128: lane group g reads k in [32g, 32g + 32). The weights and activations of the
   // next block are asked for before the products of the current one. The two sets of registers
@@ -220,7 +221,10 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) b.x[t][q] = fetch_x<NORM>(xrow[t], norm_w, at * 32 + grp * 32 + q * 8);
+      for (int q = 0; q < 4; ++q) {
+        const int k = at * 32 + grp * 32 + q * 8;   // (past K, where the weights are zeros: the last values again)
+        b.x[t][q] = fetch_x<NORM>(xrow[t], norm_w, EPI == EPI_QKV ? min(k, K - 8) : k);
+      }
   };
   auto multiply = [&](const Block& b) __attribute__((always_inline)) {
 #pragma unroll
@@ -577,7 +581,8 @@ extern "C" int dli_skinny_gemm(const void* x, int64_t ldx, const float* ssq_in, 
 }
 
 // The fused q/k/v projection of a decode step with rotation and cache write inside (EPI_QKV):
-// w_tiled is the [(q_heads + 2*kv_heads) * head_dim, K] matrix in tile order with the q and k
+// w_tiled is the [(q_heads + 2*kv_heads) * head_dim, K] matrix in tile order (K filled up with zeros to whole blocks of 128;
+// the norm's K is a multiple of 32) with the q and k
 // heads' tiles made of rotary pairs (see the top), bias (optional) in the same feature order.
 // q goes to out[row][head*head_dim + dim] (row stride ldo), rotated; rotated k and v go to the
 // pages at slots[row]. angles: [M][2][head_dim/2] float32 cos/sin of the rows' positions.
@@ -588,7 +593,8 @@ extern "C" int dli_skinny_gemm_qkv_rope(const void* x, int64_t ldx, const float*
                                         int q_heads, int kv_heads, int head_dim, int page_size,
                                         int shape, hipStream_t stream) {
   if (M <= 0) return DLI_OK;
-  if (M > 16 || K <= 0 || K % 128 != 0 || ldx % 8 != 0 || ldo % 8 != 0 || shape < 0 || shape > 4 ||
+  // (without the norm a last block of zeros could make a NaN of an infinite activation)
+  if (M > 16 || K <= 0 || K % (norm_w != nullptr ? 32 : 128) != 0 || ldx % 8 != 0 || ldo % 8 != 0 || shape < 0 || shape > 4 ||
       q_heads <= 0 || kv_heads <= 0 || head_dim <= 0 || head_dim % 16 != 0 || page_size <= 0 ||
       out == nullptr || angles == nullptr || slots == nullptr || k_pages == nullptr ||
       v_pages == nullptr || (norm_w != nullptr && (ssq_in == nullptr || ssq_parts <= 0)))

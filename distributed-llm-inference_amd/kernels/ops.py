@@ -1042,10 +1042,10 @@ def skinny_gemm_qkv_rope(x: torch.Tensor, w_tiled: torch.Tensor, q_out: torch.Te
     pages, kv_heads, page_size, head_dim = k_pages.shape
     _require(v_pages.shape == (pages, kv_heads, head_dim, page_size), "v_pages must be [pages, kv_heads, head_dim, page_size]")
     n = (q_heads + 2 * kv_heads) * head_dim
-    _require(0 < m <= 16 and k % 128 == 0 and head_dim % 16 == 0 and q_heads > 0,
-             f"this product takes 1..16 rows, k % 128 == 0 and head_dim % 16 == 0, not {m} x {k}, {head_dim}")
+    _require(0 < m <= 16 and k > 0 and k % (128 if norm_w is None else 32) == 0 and head_dim % 16 == 0 and q_heads > 0,
+             f"this product takes 1..16 rows, k % 32 == 0 (128 without a norm) and head_dim % 16 == 0, not {m} x {k}, {head_dim}")
     _dense(w_tiled, "w_tiled", torch.bfloat16, 1)
-    _require(w_tiled.numel() == n * k and w_tiled.data_ptr() % 16 == 0, "w_tiled must hold [(q + 2 kv) * head_dim, k]")
+    _require(w_tiled.numel() == n * padded_k(k) and w_tiled.data_ptr() % 16 == 0, "w_tiled must hold [(q + 2 kv) * head_dim, k]")
     _require(x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0, "x must be 16-byte aligned")
     _rows(q_out, "q_out", torch.bfloat16)
     _require(q_out.shape[0] == m and q_out.shape[1] >= q_heads * head_dim and q_out.stride(0) % 8 == 0

@@ -29,7 +29,9 @@ from .spec import PartSpec, WeightSpec
 # Decode steps with this many rows rotate and write the cache in the epilogue of the q/k/v
 # product, which reads a copy of the matrix whose tiles hold whole rotary pairs: no rotation
 # kernel runs. (A variant that rotated inside the attention kernel instead, repeating the rotation
-# in every split of the keys, was slower from four rows on and no faster below.)
+# in every split of the keys, was slower from four rows on and no faster below.) Widths that are not
+# whole blocks of 128 read the copy whose last block is filled up with zeros (width 576: the rotation
+# kernel's 2.8 us a layer go, the product takes 0.4 more).
 ROPE_IN_PRODUCT_ROWS = range(1, 17)
 # Decode steps with this many rows leave the merge of the runs of keys to the o projection, whose
 # waves merge the k that they multiply while their first weights are on their way. Every workgroup
@@ -215,7 +217,7 @@ class GQAttention(Mixer):
             self._forward_stream_mid(stream, norm, ctx, cache, grp, following)
             return
         qkv = self.rt.empty(n, (nh + 2 * nkv) * d)
-        if self.w_qkv_rope is not None and n in ROPE_IN_PRODUCT_ROWS and self.hidden_size % 128 == 0:
+        if self.w_qkv_rope is not None and n in ROPE_IN_PRODUCT_ROWS and self.hidden_size % 32 == 0:
             # product, rotation and cache write in one kernel; only q comes back
             angles = self.position.step_angles(ctx, qkv.dtype)
             ops.skinny_gemm_qkv_rope(stream.x, self.w_qkv_rope, qkv, angles, grp.slots, cache.k_pages, cache.v_pages,

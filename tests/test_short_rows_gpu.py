@@ -41,3 +41,14 @@ def test_short_rows(k, n):
         assert parts.shape[0] == ops.skinny_gemm_plan(rows, n, k, ops.SKINNY_RESIDUAL, xd.device)[2]
         total = stream.cpu().double().pow(2).sum(1)
         assert ((parts.sum(0).cpu().double() - total).abs() <= 1e-4 * total).all()
+
+
+@pytest.mark.parametrize("m", [1, 4, 5, 16])
+@pytest.mark.parametrize("qh,kvh,d,k,bs,shape", [(9, 3, 64, 576, 16, None), (2, 1, 16, 32, 16, 0), (15, 5, 64, 960, 16, 4),
+                                                 (4, 4, 32, 1056, 8, 1), (3, 1, 64, 160, 16, 2), (3, 1, 64, 224, 16, 3)])
+def test_the_rotating_product_takes_a_last_block_that_is_not_whole(m, qh, kvh, d, k, bs, shape):
+    import test_kernels_gpu as kernels
+
+    from dli_amd.kernels import ops
+
+    kernels.test_skinny_gemm_qkv_with_rotation_and_cache_write(ops, m, qh, kvh, d, k, bs, shape)

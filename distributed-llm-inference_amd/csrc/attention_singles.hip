@@ -13,8 +13,8 @@
 // kept short (one multiplication finds a tile's page, the penalty is a kernel of its own, results leave by way of LDS: together
 // 7.8 -> 6.7 us a call). On the vector units a lane reads a key's whole row alone and every weight passes through LDS. Us a call,
 // merges with them, before -> now: 4 requests of 32 heads of 64 on 8, 256 keys 15.0 -> 6.7, 1,024 keys 21.8 -> 9.3, 16,384 keys
-// 44.1 -> 29.6; 64 such requests of 1,024 keys 41.5 -> 26.4, of 16,384 keys 581 -> 360 (3.0 TB/s); 8 requests of 16 heads of 128 on
-// 2, 1,024 keys 29.6 -> 12.8.
+// 44.1 -> 29.6 (4.5 TB/s); 64 such requests of 1,024 keys 41.5 -> 26.4, of 16,384 keys 581 -> 360 (6.0 TB/s); 8 requests of 16
+// heads of 128 on 2, 1,024 keys 29.6 -> 12.8.
 #include "attention_singles.h"
 
 typedef short as_s4 __attribute__((ext_vector_type(4)));

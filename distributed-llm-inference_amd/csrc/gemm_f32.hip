@@ -155,7 +155,8 @@ __global__ __launch_bounds__(64 * KW) void gemm_f32_few_kernel(GfArgs p) {
 // More rows: a wave makes a tile of 32 x 32 out of LDS, into which 32 k of its rows come in whole cache lines (rows of 36
 // floats there: the 16 rows of a read lie in banks of their own), the next 32 k in flight meanwhile. KG == 1: WM x WN
 // waves lie side by side and share what they stage. KG > 1 (few tiles, long sums): KG waves share one tile and take
-// its segments in turn, each in a part of LDS of its own, without a barrier.
+// its segments in turn, each in a part of LDS of its own: its lanes hand each other what they stage behind a fence of
+// the wave, without a wait for other waves.
 #define GF_BK 32
 #define GF_LD 36
 
@@ -193,6 +194,17 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_f32_tile_kernel(GfArgs
       *reinterpret_cast<gf4*>(to + dst[u]) = !VEC || k0 + at < p.k ? flight[u] : gf4{0.f, 0.f, 0.f, 0.f};
   };
 
+  // What has been put there is seen by the lanes that read it, and nothing put later overtakes what they read.
+  const auto staged = [&] {
+    if constexpr (KG == 1) {
+      __syncthreads();
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+  };
+
   gf4 total[2][2], seg[2][2], acc[2][2];
 #pragma unroll
   for (int x = 0; x < 2; ++x)
@@ -207,7 +219,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_f32_tile_kernel(GfArgs
     fetch(k0);
     put(stage, k0);
   }
-  if constexpr (KG == 1) __syncthreads();
+  staged();
   while (s < p.segments) {
     int k_next = k0 + GF_BK, s_next = s;
     const bool seg_ends = k_next >= p.k || k_next % seg_k == 0;
@@ -255,7 +267,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_f32_tile_kernel(GfArgs
     }
     buf ^= 1;
     if (s_next < p.segments) put(stage + buf * (BM + BN) * GF_LD, k_next);
-    if constexpr (KG == 1) __syncthreads();
+    staged();
     k0 = k_next;
     s = s_next;
   }
@@ -305,28 +317,55 @@ static int gf_tiles(const GfArgs& p, bool vec, hipStream_t stream) {
   return dli_launch_status();
 }
 
+// Which kernel takes m rows, n columns and `segments` segments: 0 to 3 the few-row kernel, from sixteen waves a tile down to two for
+// two tiles, 4 to 7 the tile kernel, from eight waves a tile of 32 x 32 up to tiles of 128 x 64.
+// As many waves as the device has SIMDs, where the sum has segments enough: 498 x 3072 x 576 (1,536 tiles) takes 32.6 us
+// with four waves a tile and 44 with tiles of 64 x 64 for four waves; 2048 x 16384 x 2048 1,280 us in tiles of 128 x 64.
+static int gf_rule(int m, int n, int segments) {
+  const int64_t simds = 4 * dli_compute_units();
+  if (m <= 16) {
+    const int64_t tiles = (n + 15) / 16;
+    if (segments > 8 && tiles * 8 < 2 * simds) return 0;
+    if (segments > 4 && tiles * 4 < 2 * simds) return 1;
+    return segments >= 2 && tiles < 8 * simds ? 2 : 3;
+  }
+  const int64_t tiles = (int64_t)((n + 31) / 32) * ((m + 31) / 32);
+  if (tiles * 4 <= simds && segments > 4) return 4;
+  if (tiles <= 2 * simds && segments >= 2) return 5;
+  return tiles < 8 * simds ? 6 : 7;
+}
+
+// The order of a sum over k: `segments` of `seg_runs` runs each.
+static void gf_order(int k, int& segments, int& seg_runs) {
+  const int runs = (k + GF_RUN - 1) / GF_RUN;
+  seg_runs = (runs + GF_SEGMENTS - 1) / GF_SEGMENTS;
+  segments = (runs + seg_runs - 1) / seg_runs;
+}
+
+extern "C" int dli_gemm_f32_rule(int m, int n, int k) {
+  if (m <= 0 || n <= 0 || k <= 0) return -1;
+  int segments, seg_runs;
+  gf_order(k, segments, seg_runs);
+  return gf_rule(m, n, segments);
+}
+
 extern "C" int dli_gemm_f32_nt(const float* a, int64_t lda, const float* w, int64_t ldw,
                                const float* bias, const float* residual, int64_t ldr, float* out,
                                int64_t ldo, int m, int n, int k, hipStream_t stream) {
   if (m <= 0 || n <= 0) return DLI_OK;
   if (k <= 0 || lda < k || ldw < k || ldo < n || (residual != nullptr && ldr < n)) return DLI_ERR_ARGUMENT;
-  const int runs = (k + GF_RUN - 1) / GF_RUN;
-  const int seg_runs = (runs + GF_SEGMENTS - 1) / GF_SEGMENTS, segments = (runs + seg_runs - 1) / seg_runs;
+  int segments, seg_runs;
+  gf_order(k, segments, seg_runs);
   const GfArgs p = {a, w, bias, residual, out, lda, ldw, ldr, ldo, m, n, k, segments, seg_runs};
   const bool vec = k % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (((uintptr_t)a | (uintptr_t)w) % 16) == 0;
-  // As many waves as the device has SIMDs, where the sum has segments enough: 498 x 3072 x 576 (1,536 tiles) takes 32.6 us
-  // with four waves a tile and 44 with tiles of 64 x 64 for four waves; 2048 x 16384 x 2048 1,280 us in tiles of 128 x 64.
-  const int64_t simds = 4 * dli_compute_units();
-  if (m <= 16) {
-    const int64_t tiles = (n + 15) / 16;
-    if (segments > 8 && tiles * 8 < 2 * simds) return gf_few<1, 16>(p, vec, stream);
-    if (segments > 4 && tiles * 4 < 2 * simds) return gf_few<1, 8>(p, vec, stream);
-    if (segments >= 2 && tiles < 8 * simds) return gf_few<1, 4>(p, vec, stream);
-    return gf_few<2, 2>(p, vec, stream);
+  switch (gf_rule(m, n, segments)) {
+    case 0: return gf_few<1, 16>(p, vec, stream);
+    case 1: return gf_few<1, 8>(p, vec, stream);
+    case 2: return gf_few<1, 4>(p, vec, stream);
+    case 3: return gf_few<2, 2>(p, vec, stream);
+    case 4: return gf_tiles<1, 1, 8>(p, vec, stream);
+    case 5: return gf_tiles<1, 1, 4>(p, vec, stream);
+    case 6: return gf_tiles<2, 2, 1>(p, vec, stream);
+    default: return gf_tiles<4, 2, 1>(p, vec, stream);
   }
-  const int64_t tiles = (int64_t)((n + 31) / 32) * ((m + 31) / 32);
-  if (tiles * 4 <= simds && segments > 4) return gf_tiles<1, 1, 8>(p, vec, stream);
-  if (tiles <= 2 * simds && segments >= 2) return gf_tiles<1, 1, 4>(p, vec, stream);
-  if (tiles < 8 * simds) return gf_tiles<2, 2, 1>(p, vec, stream);
-  return gf_tiles<4, 2, 1>(p, vec, stream);
 }

@@ -41,6 +41,7 @@ _SIGNATURES = {
     "dli_skinny4_tile_features": [_c_int, _c_int],
     "dli_rope_kv_write": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int,
                           _c_int, _c_int, _c_int, _c_int, _c_ptr],
+    "dli_gemm_f32_rule": [_c_int, _c_int, _c_int],
     "dli_gemm_f32_nt": [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_int,
                         _c_int, _c_int, _c_ptr],
     "dli_sample": [_c_ptr, _c_i64, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
@@ -431,6 +432,12 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, bias: Optional
         ldr = residual.stride(0)
     _check(library().dli_gemm_f32_nt(_ptr(a), a.stride(0), _ptr(w), w.stride(0), _ptr(bias), _ptr(residual),
                                      ldr, _ptr(out), out.stride(0), m, n, k, _stream()), "gemm_f32")
+
+
+def gemm_f32_rule(m: int, n: int, k: int) -> int:
+    """The kernel that :func:`gemm_f32` runs for ``m`` rows and ``n`` columns of depth ``k``: 0 to 3 for up to 16 rows, 4 to 7 in
+    tiles (``csrc/gemm_f32.hip`` says which)."""
+    return int(library().dli_gemm_f32_rule(int(m), int(n), int(k)))
 
 
 SKINNY_STORE, SKINNY_SWIGLU, SKINNY_RESIDUAL, SKINNY_F32 = 0, 1, 2, 3

@@ -19,8 +19,9 @@ def ops():
     return module
 
 
-# rows: the few-row kernel's end and the tiles' (32, 64, 128); columns: part of a tile, and enough of them for every rule
-# of the dispatch; k: below a load, across a run's half and end, several runs a segment (2,048 is 16 runs, 2,100 two a segment)
+# rows: the few-row kernel's end and the tiles' (32, 64, 128); columns: part of a tile, and enough of them for most rules
+# of the dispatch (the test below goes through every one); k: below a load, across a run's half and end, several runs a
+# segment (2,048 is 16 runs, 2,100 two a segment)
 @pytest.mark.parametrize("m", [1, 16, 17, 33, 130])
 @pytest.mark.parametrize("n,k", [(31, 3), (16, 62), (48, 64), (576, 132), (1024, 1536), (700, 1030), (65, 2048), (33, 2100), (40000, 100)])
 def test_gemm_f32_edges(ops, m, n, k):
@@ -35,6 +36,34 @@ def test_gemm_f32_edges(ops, m, n, k):
     one = torch.empty(1, n, device="cuda")   # a row alone, through the few-row kernel: the same bits
     ops.gemm_f32(a[m - 1:], w, one)
     assert torch.equal(one[0], out[m - 1])
+
+
+# (rows, columns, k, kernel): every kernel of the dispatch with as many segments as its waves take several of, k in whole loads and
+# in single values. Few rows with 2 and 4 waves a tile and one segment, 2 to 4, 5 to 8 (8 waves), more (16); tiles of 32 x 32
+# with 8 waves (5, 9 and 16 segments of one, two and five runs) and with 4 (2, 5, 9 and 12 segments), of 64 x 64, of 128 x 64
+RULES = [(2, 960, 576, 1), (16, 3072, 576, 1), (9, 600, 1023, 1), (2, 576, 1536, 0), (5, 90, 9001, 0), (2, 40000, 576, 2),
+         (7, 700, 390, 2), (2, 300, 100, 3), (3, 140000, 300, 3), (100, 100, 576, 4), (498, 192, 1536, 4), (61, 33, 9001, 4),
+         (498, 960, 576, 5), (498, 3072, 576, 5), (498, 576, 1536, 5), (300, 1000, 1101, 5), (130, 65, 132, 5), (333, 9000, 576, 6),
+         (300, 1000, 100, 6), (300, 30000, 132, 7), (390, 33000, 61, 7)]
+
+
+@pytest.mark.parametrize("m,n,k,rule", RULES)
+def test_gemm_f32_every_kernel(ops, m, n, k, rule):
+    """Each kernel against float64, and each of some rows against the row alone: the same bits."""
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:   # (the rule follows the device's compute units)
+        assert ops.gemm_f32_rule(m, n, k) == rule
+        assert {r[3] for r in RULES} == set(range(8))
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, w = (torch.randn(r, k, device="cuda", generator=gen) for r in (m, n))
+    out = torch.full((m, n), 7.0, device="cuda")
+    ops.gemm_f32(a, w, out)
+    # each of k products and sums rounds by 2^-24 of a partial sum: runs of 128 terms, then the runs' sums
+    bound = (128 + k / 128 + 2) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)
+    assert ((out.double() - a.double() @ w.double().T).abs() <= bound).all()
+    for row in {0, m // 2, m - 1}:
+        one = torch.empty(1, n, device="cuda")
+        ops.gemm_f32(a[row:row + 1], w, one)
+        assert torch.equal(one[0], out[row]), row
 
 
 def test_gemm_f32_rows_of_wider_matrices(ops):

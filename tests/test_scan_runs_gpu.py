@@ -38,6 +38,15 @@ def cut(monkeypatch, ops, workgroups):
 STEPS = [[64, 0, 65], [1, 200, 130], [129, 1, 1], [16, 333, 17], [0, 63, 64]]
 
 
+def no_further_off(got, refs):
+    """The runs' distance from the float64 rule against the token-by-token kernel's. Measured with random rows at 8 to 32 heads and
+    300 to 4,096 tokens: 0.99 to 1.02 times as far (2-norm; what a run adds is one more sum of 64 terms a value), 1.05 leaves
+    room for the few heads here."""
+    far = {way: (sum((torch.cat(g) - r).norm() ** 2 for g, r in zip(got[way], refs)) / sum(r.norm() ** 2 for r in refs)).sqrt().item()
+           for way in got}
+    assert far["runs"] <= 1.05 * far["tokens"], far
+
+
 def test_rule_of_the_cut(ops):
     assert ops.scan_runs(1, 2048, 32, 2048, True) == (128, 16) and ops.scan_runs(1, 2048, 32, 2048, False) == (64, 32)
     assert ops.scan_runs(3, 134, 4, 127, True) == (0, 0) and ops.scan_runs(64, 64, 32, 1, False) == (0, 0)
@@ -84,7 +93,8 @@ def test_recurrent_scan_in_runs(ops, monkeypatch, rule, workgroups):
         at = [a + n for a, n in zip(at, step)]
     off = {way: max((torch.cat(g) - r).abs().max().item() for g, r in zip(got[way], refs)) for way in got}
     # a row divided by its root mean square: rounding of 2^-24 times the terms of a few hundred decayed sums, in both ways
-    assert off["runs"] < 2e-4 * max(r.abs().max() for r in refs) and off["runs"] < 3 * off["tokens"] + 1e-5, off
+    assert off["runs"] < 2e-4 * max(r.abs().max() for r in refs), off
+    no_further_off(got, refs)
     assert (states["runs"] - states["tokens"]).abs().max() < 1e-4 * states["tokens"].abs().max()
     assert (states["runs"][:, c * D:] == 9.0).all() and (states["runs"][0] == 9.0).all()   # nobody else's memory
 
@@ -126,5 +136,33 @@ def test_gated_delta_in_runs(ops, monkeypatch, H, G, workgroups):
     for way in got:
         for g, r in zip(got[way], refs):
             assert (torch.cat(g).view(r.shape) - r).abs().max() < 2e-5 * max(1.0, r.abs().max()), way
+    no_further_off(got, [r.reshape(r.shape[0], -1) for r in refs])
     assert (states["runs"] - states["tokens"]).abs().max() < 2e-5 * states["tokens"].abs().max()
     assert (states["runs"][:, hv * D:] == 9.0).all() and (states["runs"][0] == 9.0).all()
+
+
+@pytest.mark.parametrize("rule", ["delta", "bonus"])
+def test_state_after_runs(ops, rule):
+    """The state that sixteen runs of 64 rows leave, with keys that forget slowly and at once: no further from the float64 rule than
+    token by token (measured 0.95 to 1.03 times as far; a run's own part is added last, so that what is left of the state before
+    it does not round at that part's size: added first it was 1.2 to 2 times as far)."""
+    H, n = 4, 1000
+    c, gen = H * D, torch.Generator().manual_seed(5)
+    r, k, v, g, a = (torch.randn(n, c, generator=gen) for _ in range(5))
+    pre = torch.randn(n, c, generator=gen) + 2 * torch.randn(c, generator=gen)
+    bonus, heads = torch.randn(H, D, generator=gen), lambda t: t.double().view(n, H, D)
+    if rule == "delta":
+        w, a = torch.exp(-math.exp(-0.5) * torch.sigmoid(pre)), torch.sigmoid(a)
+        S = M.delta_rule(*map(heads, (r, k, v, w, a)))[1]
+    else:
+        w = torch.exp(-torch.exp(pre - 2))
+        S = M.bonus_rule(*map(heads, (r, k, v, w)), bonus.double())[1]
+    S = S.transpose(1, 2).reshape(-1)
+    far = []
+    for longest in (0, n):
+        state, out = torch.zeros(1, c * D, device="cuda"), torch.empty(n, c, device="cuda")
+        ops.recurrent_scan(r.cuda(), k.cuda(), v.cuda(), w.cuda(), g.cuda(), torch.ones(c, device="cuda"), EPS, state, i32([0, n]),
+                           i32(range(n)), i32([0]), out, H, D, ops.RULE_DELTA if rule == "delta" else ops.RULE_BONUS,
+                           a=a.cuda() if rule == "delta" else None, bonus=None if rule == "delta" else bonus.cuda(), longest=longest)
+        far.append((state[0].cpu().double() - S).norm() / S.norm())
+    assert far[1] <= 1.05 * far[0], far

@@ -25,7 +25,8 @@
 // chain itself reads LDS and registers only. o goes out in 32-bit; a second kernel normalises
 // each head's o and applies the gate (it needs all of a head's columns, which lie in several
 // waves). The sums of a token do not depend on where a step cut the request: the state is the
-// only thing carried, and it is carried exactly.
+// only thing carried, and it is carried exactly. (Heads of 64 in bfloat16 steps with long portions are
+// cut into runs, scan_runs.hip: there the sums depend on the cut, which follows the step's entries.)
 //
 // State slot layout: [heads][D (value)][D (key)] floats at `state + slot * state_stride`.
 // A request whose first row of the step has position 0 starts from a zero state.

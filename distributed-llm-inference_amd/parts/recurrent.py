@@ -30,6 +30,13 @@ def default_rank(hidden_size: int) -> int:
     return max(8, min(64, hidden_size // 16 // 8 * 8))
 
 
+def longest_to_cut(rt: Runtime, ctx: Any) -> int:
+    """The most rows that an entry of the step brings, where a recurrence may cut them into runs (``ops.scan_runs``); 0 on the 32-bit
+    path: the cut follows the step's longest entry, and there a request's rows have the same bits whatever requests share its
+    steps and wherever its own portions were cut. (In bfloat16 the library's products already differ with the step's rows.)"""
+    return ctx.longest_entry if rt.is_bf16 else 0
+
+
 class _MatrixStateMixer(Mixer):
     """What the two rules share: sizes, the state, the decay's low-rank projection and the output."""
 
@@ -107,7 +114,8 @@ class GeneralDelta(_MatrixStateMixer):
                         rate=a, rate_bias=self.a_bias)
         out = self.rt.empty(n, c)
         ops.recurrent_scan(r, k, v, w, g, self.norm_w, self.norm_eps, state, ctx.q_start, ctx.positions,
-                           ctx.state_slots, out, self.num_heads, self.head_dim, self.rule, a=a, longest=ctx.longest_entry)
+                           ctx.state_slots, out, self.num_heads, self.head_dim, self.rule, a=a,
+                           longest=longest_to_cut(self.rt, ctx))
         return linear_f32(self.rt, out, self.w_o)
 
 
@@ -159,7 +167,7 @@ class WKV(_MatrixStateMixer):
         out = self.rt.empty(n, c)
         ops.recurrent_scan(r, k, v, w, g, self.norm_w, self.norm_eps, state[:, h:], ctx.q_start, ctx.positions,
                            ctx.state_slots, out, self.num_heads, self.head_dim, self.rule, bonus=self.bonus,
-                           longest=ctx.longest_entry)
+                           longest=longest_to_cut(self.rt, ctx))
         return linear_f32(self.rt, out, self.w_o)
 
 
@@ -239,7 +247,7 @@ class GatedDelta(Mixer):
                          self.value_dim)
         o = torch.empty(n, self.hv, device=self.rt.device, dtype=torch.float32)
         ops.gated_delta_scan(prep, state, ctx.q_start, ctx.positions, ctx.state_slots, o, H, self.num_kv_heads,
-                             self.head_dim, self.value_dim, longest=ctx.longest_entry)
+                             self.head_dim, self.value_dim, longest=longest_to_cut(self.rt, ctx))
         out = self.rt.empty(n, self.hv)
         ops.head_norm_gate(o, proj[:, g_off:g_off + self.hv], self.norm_w, self.norm_eps, out, H, self.value_dim, gate="silu")
         return linear_f32(self.rt, out, self.w_o)

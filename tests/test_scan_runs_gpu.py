@@ -11,6 +11,8 @@ import torch
 
 import plain_makodra as M
 import plain_miberax as P
+import test_makodra_gpu as TM
+import test_miberax_gpu as TP
 
 pytestmark = pytest.mark.gpu
 
@@ -166,3 +168,44 @@ def test_state_after_runs(ops, rule):
                            a=a.cuda() if rule == "delta" else None, bonus=None if rule == "delta" else bonus.cuda(), longest=longest)
         far.append((state[0].cpu().double() - S).norm() / S.norm())
     assert far[1] <= 1.05 * far[0], far
+
+
+WHOLE = {
+    "makodra": (TM, M, {"architecture": "Makodra", "vocab": 97, "width": 96, "norm": {"eps": 1e-2}, "logit_softcap": 12.0, "layers": [
+        TM.rec("general_delta", 2, 64, 64, rank=12), TM.attn(4, 2, 32, 16, 50, 0.25, True, 0), TM.rec("wkv", 2, 64, 96, rank=8)]}),
+    "miberax": (TP, P, {"architecture": "Miberax", "vocab": 97, "width": 96, "norm": {"eps": 1e-5, "groups": 3}, "layers": [
+        TP.layer(TP.left(4, 2, 32, 16, 24, 0.2, rot=16), TP.right(4, 2, 64, 64, 3), TP.dense(72)),
+        TP.layer(TP.left(2, 2, 48, 48, 70, 0.15, rot=48), TP.right(3, 3, 64, 64, 4), TP.dense(64))]}),
+}
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("name", list(WHOLE))
+def test_whole_models_with_long_portions(ops, monkeypatch, tmp_path, name, dtype):
+    """Prompts of 200 and 300 tokens alone, beside each other and a single token, and cut in portions: against the plain model. In
+    bfloat16 the rows are cut into runs; in 32-bit they are walked in order, so that every way leaves the same bits."""
+    T, plain, cfg = WHOLE[name]
+    W = plain.random_weights(cfg, seed=4)
+    folder = plain.write_folder(tmp_path / name, cfg, W)
+    cuts, rule = [], ops.scan_runs
+    monkeypatch.setattr(ops, "scan_runs", lambda *a, **kw: cuts.append(rule(*a, **kw)) or cuts[-1])
+    toks = {"a": T.prompt(cfg, 200, 1), "b": T.prompt(cfg, 300, 2), "c": T.prompt(cfg, 6, 3)}
+    refs = {i: (T.reference(name, W, cfg, t, dtype) if T is TP else T.reference(W, cfg, t, dtype)) for i, t in toks.items()}
+    entry = lambda i, lo, hi: {"id": i, "tokens": toks[i][lo:hi], "want": list(range(hi - lo))}
+    s = T.session(folder, dtype, pages=60)
+    alone = {i: s.step([entry(i, 0, len(toks[i]))], end=[i]) for i in "ab"}
+    s.step([entry("c", 0, 5)])
+    both = s.step([entry("a", 0, 200), entry("b", 0, 300), entry("c", 5, 6)], end=["a", "b", "c"])
+    ways = {"a": [alone["a"], both[:200]], "b": [alone["b"], both[200:500]]}
+    parts = [s.step([entry("b", 0, 130)]), s.step([entry("a", 0, 40), entry("b", 130, 147)]),
+             s.step([entry("b", 147, 300), entry("a", 40, 200)], end=["a", "b"])]
+    ways["a"].append(torch.cat([parts[1][:40], parts[2][153:]]))
+    ways["b"].append(torch.cat([parts[0], parts[1][40:], parts[2][:153]]))
+    T.close(both[500:], T.rows_of(refs["c"], slice(5, 6)), dtype, "c")
+    for i in "ab":
+        for k, got in enumerate(ways[i]):
+            T.close(got, refs[i], dtype, (i, k))
+            if dtype == "float32":
+                assert torch.equal(got, ways[i][0]), (i, k)
+    assert (len([c for c in cuts if c[0]]) >= 8) == (dtype == "bfloat16"), cuts
+    s.core.manager.check_invariants()

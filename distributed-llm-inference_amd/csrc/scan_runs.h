@@ -22,10 +22,14 @@ struct RunsArgs {
   const int *q_start, *positions, *state_slots;
   float* o; int64_t o_stride;        // [rows][heads * 64]
   void* out; int64_t out_stride;
-  float *y, *ends, *moves;           // scratch: [rows][heads * 64], and per run and head 64 x 64 (moves of RUNS_BONUS: 64)
+  float *y, *ends, *moves;           // scratch: [rows][heads * 64], and per slot and head 64 x 64 (moves of RUNS_BONUS: 64)
   int heads, group, run_rows, runs;  // runs of `run_rows` (a multiple of 16) rows; `runs` of them hold the longest entry
+  int entries, rows, row0;           // entries, whose rows begin at row `row0` (y: at its start) and are `rows` in all
 };
+
+// Slots that hold every run of these entries: the sum of ceil(rows of an entry / run_rows) is no more.
+static inline int scan_runs_slots(int entries, int rows, int run_rows) { return rows / run_rows + entries; }
 
 // Whether these rows can be walked so (16-byte loads and stores).
 bool scan_runs_takes(const RunsArgs& p, int rule, int finish, int out_is_bf16);
-int scan_runs(const RunsArgs& p, int rule, int finish, int out_is_bf16, int entries, hipStream_t stream);
+int scan_runs(const RunsArgs& p, int rule, int finish, int out_is_bf16, hipStream_t stream);

@@ -19,6 +19,8 @@
 //
 // Measured (one prompt of 2,048 tokens, 32 heads, walk + carry + finish, us): RUNS_DELTA 135 + 15 + 21 against 578 and 17 for
 // the norm, RUNS_BONUS 55 + 8 + 17 against 378 and 17, RUNS_GATED 136 in all against 421. Where the cut lies: ops.scan_runs.
+// Beside 255 single tokens, which keep the kernel of steps of single tokens: 245, 168 and 183 us a layer (5,150, 2,880 and 2,610 token
+// by token; 1,048, 1,301 and 818 with every entry cut and the launch as large as the longest entry times the entries).
 // Distance from the rules in 64 bits against token by token (2-norm; 300 to 4,096 tokens, 8 to 32 heads, every row of outputs and
 // the state left): 0.99 to 1.00 times as far RUNS_DELTA, 1.01 to 1.03 RUNS_BONUS, 0.97 to 1.04 RUNS_GATED, 4e-8 to 2e-7 either way.
 #include "scan_runs.h"
@@ -33,9 +35,49 @@ __device__ __forceinline__ float runs_row_sum(float x) {   // over the sixteen l
   return x;
 }
 
-// The scratch of a run: sum over the entries before of ceil(rows / run_rows) is at most their rows / run_rows + their number.
-__device__ __forceinline__ int64_t runs_slot(const RunsArgs& p, int first, int entry, int run) {
-  return (int64_t)(first / p.run_rows + entry + run);
+// Runs lie one behind the other in slots, by entry and place, and a launch has a workgroup a slot and head: as large as the rows
+// are and not as the longest entry times the entries, what is left over at its end (empty workgroups between the others leave
+// the compute units unevenly filled: 360 us instead of 221 for 16 prompts of 375 tokens). A wave looks its run up, 64 entries a trip.
+struct RunsPlace { int entry, run, first, n, row0; };
+__device__ __forceinline__ int runs_of(const RunsArgs& p, int entry) {
+  return entry < p.entries ? (p.q_start[entry + 1] - p.q_start[entry] + p.run_rows - 1) / p.run_rows : 0;
+}
+__device__ __forceinline__ RunsPlace runs_place(const RunsArgs& p, int slot) {
+  const int lane = threadIdx.x % 64;
+  RunsPlace at = {0, slot, 0, 0, 0};
+  if (p.entries > 1) {
+    int before = 0, e0 = 0;
+    for (;; e0 += 64) {
+      if (e0 >= p.entries) return at;   // past the last run
+      const int own = runs_of(p, e0 + lane);
+      int upto = own;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int up = __shfl_up(upto, d, DLI_WAVE);
+        upto += lane >= d ? up : 0;
+      }
+      const uint64_t behind = __ballot(before + upto > slot);
+      if (behind != 0) {
+        const int l = __ffsll((unsigned long long)behind) - 1;
+        at.entry = e0 + l;
+        at.run = __builtin_amdgcn_readfirstlane(slot - before - __shfl(upto - own, l, DLI_WAVE));
+        break;
+      }
+      before += __builtin_amdgcn_readfirstlane(__shfl(upto, 63, DLI_WAVE));
+    }
+  }
+  at.first = p.q_start[at.entry];
+  at.row0 = at.first + at.run * p.run_rows;
+  at.n = min(p.run_rows, p.q_start[at.entry + 1] - at.row0);
+  return at;
+}
+// The slot of an entry's first run.
+__device__ __forceinline__ int runs_before(const RunsArgs& p, int entry) {
+  int sum = 0;
+  for (int e = threadIdx.x % 64; e < entry; e += 64) sum += runs_of(p, e);
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor(sum, d, DLI_WAVE);
+  return __builtin_amdgcn_readfirstlane(sum);
 }
 
 template <int RULE>
@@ -44,10 +86,9 @@ __global__ __launch_bounds__(256) void scan_runs_walk_kernel(RunsArgs p) {
   __shared__ rf4 sk[TB * 16], sr[TB * 16], sv[TB * 16], sw[RULE == RUNS_GATED ? 1 : TB * 16], sc[RULE == RUNS_DELTA ? TB * 16 : 1];
   __shared__ float sg[RULE == RUNS_GATED ? 2 * TB : 1];
   const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, vloc = lane / 16, part = lane % 16;
-  const int entry = blockIdx.x / p.runs, run = blockIdx.x % p.runs, head = blockIdx.y;
+  const RunsPlace place = runs_place(p, blockIdx.y);
+  const int entry = place.entry, run = place.run, first = place.first, row0 = place.row0, n = place.n, head = blockIdx.x;
   const bool unit = blockIdx.z != 0;   // the columns of the unit matrix
-  const int first = p.q_start[entry], row0 = first + run * p.run_rows;
-  const int n = min(p.run_rows, p.q_start[entry + 1] - row0);
   if (n <= 0 || (unit && run == 0)) return;
   const int col = wave * 16 + vloc * 4;   // the first of this lane's four columns
   const int64_t qk_col = (int64_t)(head / p.group) * D, v_col = (int64_t)head * D;
@@ -82,8 +123,8 @@ __global__ __launch_bounds__(256) void scan_runs_walk_kernel(RunsArgs p) {
     }
     if constexpr (RULE == RUNS_DELTA) fa = *reinterpret_cast<const rf4*>(p.a + row * p.a_stride + v_col + bc);
   };
-  float* dst = unit ? p.y : p.o;
   const int64_t dst_stride = unit ? (int64_t)p.heads * D : p.o_stride;
+  float* dst = unit ? p.y + (row0 - p.row0) * dst_stride : p.o + row0 * dst_stride;
   const auto step = [&](int t) {
     const rf4 k = sk[t * 16 + part], r = sr[t * 16 + part], v = sv[t * 16 + wave * 4 + vloc];
     rf4 o;
@@ -102,7 +143,7 @@ __global__ __launch_bounds__(256) void scan_runs_walk_kernel(RunsArgs p) {
         o[c] = o0 + o1;
       }
       if (wave == 0 && vloc == 0 && run > 0)
-        *reinterpret_cast<rf4*>(p.y + (int64_t)(row0 + t) * p.heads * D + v_col + part * 4) = r * decay;
+        *reinterpret_cast<rf4*>(p.y + (int64_t)(row0 - p.row0 + t) * p.heads * D + v_col + part * 4) = r * decay;
       decay *= w;
     } else {
       rf4 us;
@@ -165,7 +206,7 @@ __global__ __launch_bounds__(256) void scan_runs_walk_kernel(RunsArgs p) {
     if (t0 + TB < n) fetch(t0 + TB);   // on their way while this batch is walked
     __syncthreads();
     const int nb = min(TB, n - t0);
-    float* od = dst + (int64_t)(row0 + t0) * dst_stride + v_col + col;
+    float* od = dst + t0 * dst_stride + v_col + col;
     if (nb == TB) {
 #pragma unroll 4
       for (int t = 0; t < TB; ++t) {
@@ -180,7 +221,7 @@ __global__ __launch_bounds__(256) void scan_runs_walk_kernel(RunsArgs p) {
     }
     if constexpr (RULE == RUNS_BONUS) p.y += (int64_t)TB * p.heads * D;   // (the step counts its rows from the batch's first)
   }
-  const int64_t at = (runs_slot(p, first, entry, run) * p.heads + head) * D;
+  const int64_t at = ((int64_t)blockIdx.y * p.heads + head) * D;
   float* end = (unit ? p.moves : p.ends) + at * D;
 #pragma unroll
   for (int c = 0; c < 4; ++c) *reinterpret_cast<rf4*>(end + (col + c) * D + part * 4) = rf4{s[0][c], s[1][c], s[2][c], s[3][c]};
@@ -198,7 +239,7 @@ __global__ __launch_bounds__(256) void scan_runs_carry_kernel(RunsArgs p) {
   const int first = p.q_start[entry], len = p.q_start[entry + 1] - first;
   if (len <= 0) return;
   const int runs = (len + p.run_rows - 1) / p.run_rows;
-  const int64_t slot = runs_slot(p, first, entry, 0), per_run = (int64_t)p.heads * D * D;
+  const int64_t slot = runs_before(p, entry), per_run = (int64_t)p.heads * D * D;
   float* ends = p.ends + (slot * p.heads + head) * D * D + v0 * D;
   float* st = p.state + (int64_t)p.state_slots[entry] * p.state_stride + ((int64_t)head * D + v0) * D;
   const int vr = tid / 16, kc = tid % 16 * 4;   // whole rows of the slice, 16 bytes a thread
@@ -253,17 +294,16 @@ template <typename T, int FINISH>
 __global__ __launch_bounds__(256) void scan_runs_finish_kernel(RunsArgs p) {
   constexpr int D = 64;
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, i = lane % 16, g = lane / 16;
-  const int entry = blockIdx.x / p.runs, run = blockIdx.x % p.runs, head = blockIdx.y;
-  const int first = p.q_start[entry], row0 = first + run * p.run_rows, t0 = blockIdx.z * 64 + wave * 16;
-  const int n = min(p.run_rows, p.q_start[entry + 1] - row0);
+  const RunsPlace place = runs_place(p, blockIdx.y);
+  const int run = place.run, row0 = place.row0, n = place.n, head = blockIdx.x, t0 = blockIdx.z * 64 + wave * 16;
   if (t0 >= n || (FINISH == RUNS_FINISH_SUM && run == 0)) return;
   const int64_t row = row0 + min(t0 + i, n - 1), c0 = (int64_t)head * D + 4 * g;
   rf4 o[4];
 #pragma unroll
   for (int c = 0; c < 4; ++c) o[c] = *reinterpret_cast<const rf4*>(p.o + row * p.o_stride + c0 + 16 * c);
   if (run > 0) {
-    const float* s = p.ends + (runs_slot(p, first, entry, run - 1) * p.heads + head) * D * D + i * D + 4 * g;
-    const float* y = p.y + row * p.heads * D + c0;
+    const float* s = p.ends + ((int64_t)(blockIdx.y - 1) * p.heads + head) * D * D + i * D + 4 * g;
+    const float* y = p.y + (row - p.row0) * p.heads * D + c0;
     rf4 fy[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) fy[t] = *reinterpret_cast<const rf4*>(y + 16 * t);
@@ -311,7 +351,7 @@ __global__ __launch_bounds__(256) void scan_runs_finish_kernel(RunsArgs p) {
 bool scan_runs_takes(const RunsArgs& p, int rule, int finish, int out_is_bf16) {
   const auto whole = [](const void* at, size_t bytes) { return (uintptr_t)at % bytes == 0; };
   const auto rows = [&](const float* at, int64_t stride) { return stride % 4 == 0 && whole(at, 16); };
-  if (p.y == nullptr || p.ends == nullptr || p.moves == nullptr || p.runs < 1 || p.run_rows < 16 || p.run_rows % 16 != 0) return false;
+  if (p.y == nullptr || p.ends == nullptr || p.moves == nullptr || p.entries < 1 || p.rows < p.entries || p.runs < 1 || p.run_rows < 16 || p.run_rows % 16 != 0) return false;
   if (!rows(p.r, p.r_stride) || !rows(p.k, p.k_stride) || !rows(p.v, p.v_stride) || !rows(p.o, p.o_stride) ||
       !rows(p.state, p.state_stride) || !whole(p.y, 16) || !whole(p.ends, 16) || !whole(p.moves, 16))
     return false;
@@ -322,8 +362,10 @@ bool scan_runs_takes(const RunsArgs& p, int rule, int finish, int out_is_bf16) {
                                        whole(p.out, out_is_bf16 ? 8 : 16));
 }
 
-int scan_runs(const RunsArgs& p, int rule, int finish, int out_is_bf16, int entries, hipStream_t stream) {
-  const dim3 walk(entries * p.runs, p.heads, rule == RUNS_BONUS || p.runs == 1 ? 1 : 2), carry(entries, p.heads, 4);
+int scan_runs(const RunsArgs& p, int rule, int finish, int out_is_bf16, hipStream_t stream) {
+  const int slots = scan_runs_slots(p.entries, p.rows, p.run_rows);
+  if (slots > 65535) return DLI_ERR_ARGUMENT;
+  const dim3 walk(p.heads, slots, rule == RUNS_BONUS || p.runs == 1 ? 1 : 2), carry(p.entries, p.heads, 4);
   if (rule == RUNS_DELTA) {
     scan_runs_walk_kernel<RUNS_DELTA><<<walk, 256, 0, stream>>>(p);
     scan_runs_carry_kernel<RUNS_DELTA><<<carry, 256, 0, stream>>>(p);
@@ -334,7 +376,7 @@ int scan_runs(const RunsArgs& p, int rule, int finish, int out_is_bf16, int entr
     scan_runs_walk_kernel<RUNS_GATED><<<walk, 256, 0, stream>>>(p);
     scan_runs_carry_kernel<RUNS_GATED><<<carry, 256, 0, stream>>>(p);
   }
-  const dim3 done(entries * p.runs, p.heads, (p.run_rows + 63) / 64);
+  const dim3 done(p.heads, slots, (p.run_rows + 63) / 64);
   if (finish == RUNS_FINISH_SUM) {
     if (p.runs > 1) scan_runs_finish_kernel<float, RUNS_FINISH_SUM><<<done, 256, 0, stream>>>(p);
   } else if (finish == RUNS_FINISH_SIGMOID) {

@@ -157,8 +157,8 @@ _SIGNATURES = {
     "dli_recurrent_scan_supports": [_c_int],
     "dli_recurrent_scan": [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr,
                            _c_i64, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr,
-                           _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr,
-                           _c_ptr],
+                           _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr,
+                           _c_ptr, _c_ptr],
     "dli_rotary_cache": [_c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr,
                          _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, ctypes.c_double, _c_ptr, _c_ptr,
                          _c_float, _c_int, _c_ptr],
@@ -190,7 +190,7 @@ _SIGNATURES = {
     "dli_conv_prepare": [_c_ptr, _c_i64, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr,
                          _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "dli_gated_delta_scan": [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_int,
-                             _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
+                             _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
     "dli_poly_norm": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_float, _c_int, _c_ptr],
     "dli_clamped_glu": [_c_ptr, _c_i64, _c_ptr, _c_int, _c_int, _c_int, _c_float, _c_float, _c_float, _c_int, _c_ptr],
     "dli_router_choose": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int,
@@ -1920,23 +1920,36 @@ RUNS_MIN_ROWS = 64      # rows of a run at least
 RUNS_WORKGROUPS = 1024
 
 
+# Ends and moves of a step at most, a pair for every run and head (32 KB): half a gigabyte. A step of more entries than that walks
+# its rows token by token.
+RUNS_MOST_SCRATCH = 16384
+
+
 def scan_runs(entries: int, rows: int, heads: int, longest: int, unit_columns: bool) -> tuple[int, int]:
     """``(rows a run, runs of the longest entry)`` into which the rows of a matrix-state recurrence with heads of 64
-    are cut, or ``(0, 0)`` for token by token. ``longest``: the most rows that an entry of the step brings, as the
-    host knows it; ``unit_columns``: runs after an entry's first also walk the unit matrix's columns."""
+    are cut, or ``(0, 0)`` for token by token. ``entries``, ``rows``: those that bring portions, single tokens aside; ``longest``:
+    the most rows that one of them brings, as the host knows it; ``unit_columns``: runs after an entry's first also walk
+    the unit matrix's columns."""
     if longest < RUNS_FROM_ROWS:
         return 0, 0
     alike = max(1, rows // longest)   # entries that long the step amounts to
     runs = max(1, RUNS_WORKGROUPS // (alike * heads * (2 if unit_columns else 1)))
     run_rows = max(RUNS_MIN_ROWS, -(-longest // runs))
     run_rows = -(-run_rows // 16) * 16
+    if (rows // run_rows + entries) * heads > RUNS_MOST_SCRATCH:
+        return 0, 0
     return run_rows, -(-longest // run_rows)
 
 
-def _runs_scratch(device: torch.device, entries: int, rows: int, heads: int, run_rows: int, unit_columns: bool):
-    """The walk's outputs for the unit columns, and per run and head the end state and what moves the one before."""
-    slots = rows // run_rows + entries
-    return (torch.empty(rows, heads * 64, device=device, dtype=torch.float32),
+def _cut(device: torch.device, entries: int, rows: int, heads: int, longest: int, singles: int, unit_columns: bool) -> tuple:
+    """What the scans' entry points are told about runs: single-row entries that lead, rows a run, runs of the longest entry, and
+    the scratch: the walk's outputs for the unit columns, and per run and head the end state and what moves the one before."""
+    portions, rows = entries - singles, rows - singles
+    run_rows, runs = scan_runs(portions, rows, heads, longest, unit_columns) if portions > 0 else (0, 0)
+    if not run_rows:
+        return 0, 0, 0, None, None, None
+    slots = rows // run_rows + portions
+    return (singles, run_rows, runs, torch.empty(rows, heads * 64, device=device, dtype=torch.float32),
             torch.empty(slots, heads, 64, 64, device=device, dtype=torch.float32),
             torch.empty(slots, heads, 64, 64 if unit_columns else 1, device=device, dtype=torch.float32))
 
@@ -1945,13 +1958,15 @@ def recurrent_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, w: torch.T
                    norm_w: torch.Tensor, eps: float, state: torch.Tensor, q_start: torch.Tensor,
                    positions: torch.Tensor, state_slots: torch.Tensor, out: torch.Tensor, heads: int, dim: int,
                    rule: int, a: Optional[torch.Tensor] = None, bonus: Optional[torch.Tensor] = None,
-                   longest: int = 0) -> None:
+                   longest: int = 0, singles: int = 0) -> None:
     """A matrix-state recurrence per request and head, with the per-head norm and the gate of its
     output (``csrc/recurrent_scan.hip`` states both rules). ``r, k, v``, the decay ``w``, the gate's
     pre-activation ``g_pre`` and (delta rule) the removal rate ``a`` are float32 ``[n, heads*dim]`` with
     contiguous rows (any row stride); ``state`` is float32 ``[slots, >= heads*dim*dim]``, row
     ``state_slots[e]`` being entry ``e``'s; ``out [n, heads*dim]`` float32 or bfloat16. ``longest``: the most
-    rows that an entry brings (0: not known on the host; the rows are then walked token by token)."""
+    rows that an entry brings (0: not known on the host; the rows are then walked token by token). ``singles``: how many
+    leading entries the host knows to bring one row each; where the others are cut into runs, these keep the kernel of steps
+    of single tokens."""
     n, width = out.shape[0], heads * dim
     w_pre, a_pre, a_bias = w, a, None
     for name, t in (("r", r), ("k", k), ("v", v), ("w", w), ("g_pre", g_pre), ("a", a)):
@@ -1977,16 +1992,12 @@ def recurrent_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, w: torch.T
         _require(bonus.numel() == width, "bonus must hold heads*dim values")
     sa = a_pre.stride(0) if a_pre is not None else 0
     o_raw = torch.empty(n, width, device=out.device, dtype=torch.float32)  # the recurrence's output before norm and gate
-    run_rows, runs, scratch = 0, 0, (None, None, None)
-    if dim == 64 and entries > 0:
-        run_rows, runs = scan_runs(entries, n, heads, longest, rule == RULE_DELTA)
-        if run_rows:
-            scratch = _runs_scratch(out.device, entries, n, heads, run_rows, rule == RULE_DELTA)
+    cut = _cut(out.device, entries, n, heads, longest if dim == 64 else 0, singles, rule == RULE_DELTA)
     _check(library().dli_recurrent_scan(
         _ptr(r), r.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(w_pre), w_pre.stride(0), _ptr(a_pre), sa,
         _ptr(a_bias), _ptr(g_pre), g_pre.stride(0), _ptr(bonus), _ptr(norm_w), float(eps), _ptr(state), state.stride(0),
         _ptr(q_start), _ptr(positions), _ptr(state_slots), _ptr(o_raw), o_raw.stride(0), _ptr(out), out.stride(0), entries,
-        n, heads, dim, int(rule), _is_bf16(out.dtype), run_rows, runs, *map(_ptr, scratch), _stream()), "recurrent_scan")
+        n, heads, dim, int(rule), _is_bf16(out.dtype), *cut[:3], *map(_ptr, cut[3:]), _stream()), "recurrent_scan")
 
 
 # ----------------------------------------------------------------------------- rotary keys from 32-bit projections
@@ -2134,10 +2145,11 @@ def conv_prepare(proj: torch.Tensor, b_off: int, a_off: int, conv_w: torch.Tenso
 
 def gated_delta_scan(prep: torch.Tensor, state: torch.Tensor, q_start: torch.Tensor, positions: torch.Tensor,
                      state_slots: torch.Tensor, o: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim: int,
-                     longest: int = 0) -> None:
+                     longest: int = 0, singles: int = 0) -> None:
     """Per request and head ``S <- g S; u = beta (v - S^T k); S <- S + k u^T; o = S^T q`` over the step's rows
     in order, ``S`` float32 ``[heads][vdim][dim]`` at the start of ``state[slot]`` (zeros at position 0);
-    ``prep`` as :func:`conv_prepare` leaves it; ``o [n, heads*vdim]`` float32; ``longest`` as in :func:`recurrent_scan`."""
+    ``prep`` as :func:`conv_prepare` leaves it; ``o [n, heads*vdim]`` float32; ``longest`` and ``singles`` as in
+    :func:`recurrent_scan`."""
     _f32_rows(prep, "prep")
     _f32_rows(o, "o")
     n = prep.shape[0]
@@ -2150,14 +2162,10 @@ def gated_delta_scan(prep: torch.Tensor, state: torch.Tensor, q_start: torch.Ten
         _dense(t, name, torch.int32, 1)
     entries = state_slots.shape[0]
     _require(q_start.shape[0] == entries + 1 and positions.shape[0] == n, "q_start/state_slots/positions disagree")
-    run_rows, runs, scratch = 0, 0, (None, None, None)
-    if dim == vdim == 64 and entries > 0:
-        run_rows, runs = scan_runs(entries, n, heads, longest, True)
-        if run_rows:
-            scratch = _runs_scratch(o.device, entries, n, heads, run_rows, True)
+    cut = _cut(o.device, entries, n, heads, longest if dim == vdim == 64 else 0, singles, True)
     _check(library().dli_gated_delta_scan(
         _ptr(prep), prep.stride(0), _ptr(state), state.stride(0), _ptr(q_start), _ptr(positions), _ptr(state_slots),
-        _ptr(o), o.stride(0), entries, n, heads, kv_heads, dim, vdim, run_rows, runs, *map(_ptr, scratch), _stream()),
+        _ptr(o), o.stride(0), entries, n, heads, kv_heads, dim, vdim, *cut[:3], *map(_ptr, cut[3:]), _stream()),
         "gated_delta_scan")
 
 

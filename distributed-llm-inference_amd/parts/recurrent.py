@@ -115,7 +115,7 @@ class GeneralDelta(_MatrixStateMixer):
         out = self.rt.empty(n, c)
         ops.recurrent_scan(r, k, v, w, g, self.norm_w, self.norm_eps, state, ctx.q_start, ctx.positions,
                            ctx.state_slots, out, self.num_heads, self.head_dim, self.rule, a=a,
-                           longest=longest_to_cut(self.rt, ctx))
+                           longest=longest_to_cut(self.rt, ctx), singles=ctx.num_decode)
         return linear_f32(self.rt, out, self.w_o)
 
 
@@ -167,7 +167,7 @@ class WKV(_MatrixStateMixer):
         out = self.rt.empty(n, c)
         ops.recurrent_scan(r, k, v, w, g, self.norm_w, self.norm_eps, state[:, h:], ctx.q_start, ctx.positions,
                            ctx.state_slots, out, self.num_heads, self.head_dim, self.rule, bonus=self.bonus,
-                           longest=longest_to_cut(self.rt, ctx))
+                           longest=longest_to_cut(self.rt, ctx), singles=ctx.num_decode)
         return linear_f32(self.rt, out, self.w_o)
 
 
@@ -247,7 +247,7 @@ class GatedDelta(Mixer):
                          self.value_dim)
         o = torch.empty(n, self.hv, device=self.rt.device, dtype=torch.float32)
         ops.gated_delta_scan(prep, state, ctx.q_start, ctx.positions, ctx.state_slots, o, H, self.num_kv_heads,
-                             self.head_dim, self.value_dim, longest=longest_to_cut(self.rt, ctx))
+                             self.head_dim, self.value_dim, longest=longest_to_cut(self.rt, ctx), singles=ctx.num_decode)
         out = self.rt.empty(n, self.hv)
         ops.head_norm_gate(o, proj[:, g_off:g_off + self.hv], self.norm_w, self.norm_eps, out, H, self.value_dim, gate="silu")
         return linear_f32(self.rt, out, self.w_o)

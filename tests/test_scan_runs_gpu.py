@@ -170,6 +170,51 @@ def test_state_after_runs(ops, rule):
     assert far[1] <= 1.05 * far[0], far
 
 
+def test_scratch_follows_the_portions(ops):
+    """A step's single tokens take no scratch; a step with more entries that bring portions than the scratch may hold is not cut."""
+    cut = ops._cut(torch.device("cpu"), 258, 2555, 4, 1500, 255, True)   # 255 single tokens, portions of 1,500, 400 and 400 rows
+    run_rows, slots = cut[1], 2300 // cut[1] + 3
+    assert cut[0] == 255 and cut[3].shape == (2300, 256) and cut[4].shape == cut[5].shape == (slots, 4, 64, 64)
+    assert ops.scan_runs(480, 4000, 32, 2048, True)[0] and not ops.scan_runs(520, 4000, 32, 2048, True)[0]
+    assert not ops._cut(torch.device("cpu"), 5, 5, 4, 1, 5, True)[1]
+
+
+@pytest.mark.parametrize("rule", ["delta", "bonus", "gated"])
+@pytest.mark.parametrize("lens,singles", [([1, 1, 1, 200, 2, 70, 129], 3), ([1] * 70 + [5, 300], 70), ([3] * 40 + [150], 0), ([1, 128], 1)])
+def test_single_tokens_beside_portions(ops, rule, lens, singles):
+    """The leading single tokens have the bits that a step of single tokens gives them, the portions those of a step without them;
+    nobody else's state is written. (Entries of many lengths: slots of the launch that hold no run.)"""
+    H, n, E = 2, sum(lens), len(lens)
+    c, gen = H * D, torch.Generator(device="cuda").manual_seed(n)
+    rnd = lambda *shape: torch.randn(*shape, device="cuda", generator=gen)
+    r, k, v, g, a, w = (rnd(n, c) for _ in range(6))
+    a, w = torch.sigmoid(a), torch.exp(-math.exp(-0.5) * torch.sigmoid(w))
+    bonus, norm_w, state0 = rnd(H, D), rnd(c), rnd(E + 2, c * D)
+    prep = torch.cat([0.1 * rnd(n, 2 * c), rnd(n, c), torch.rand(n, 2 * H, device="cuda", generator=gen)], 1)
+    starts = np.cumsum([0] + lens)
+    positions = np.concatenate([np.arange(m) + (7 if i % 3 else 0) for i, m in enumerate(lens)])
+
+    def run(lo, hi, longest, lead):
+        rows, state = slice(starts[lo], starts[hi]), state0.clone()
+        args = (i32(starts[lo:hi + 1] - starts[lo]), i32(positions[rows]), i32(range(E - 1, -1, -1)[lo:hi]))
+        out = torch.full((starts[hi] - starts[lo], c), 9.0, device="cuda")
+        if rule == "gated":
+            ops.gated_delta_scan(prep[rows], state, *args, out, H, H, D, D, longest=longest, singles=lead)
+        else:
+            ops.recurrent_scan(r[rows], k[rows], v[rows], w[rows], g[rows], norm_w, EPS, state, *args, out, H, D,
+                               ops.RULE_DELTA if rule == "delta" else ops.RULE_BONUS, a=a[rows] if rule == "delta" else None,
+                               bonus=None if rule == "delta" else bonus, longest=longest, singles=lead)
+        return out, state
+
+    out, state = run(0, E, max(lens), singles)
+    portions, portion_state = run(singles, E, max(lens), 0)
+    assert torch.equal(out[starts[singles]:], portions)
+    assert torch.equal(state[:E - singles], portion_state[:E - singles]) and torch.equal(state[E:], state0[E:])
+    if singles:
+        alone, alone_state = run(0, singles, 0, 0)
+        assert torch.equal(out[:starts[singles]], alone) and torch.equal(state[E - singles:E], alone_state[E - singles:E])
+
+
 WHOLE = {
     "makodra": (TM, M, {"architecture": "Makodra", "vocab": 97, "width": 96, "norm": {"eps": 1e-2}, "logit_softcap": 12.0, "layers": [
         TM.rec("general_delta", 2, 64, 64, rank=12), TM.attn(4, 2, 32, 16, 50, 0.25, True, 0), TM.rec("wkv", 2, 64, 96, rank=8)]}),

@@ -1909,31 +1909,46 @@ def recurrent_scan_supports(dim: int) -> bool:
     return bool(library().dli_recurrent_scan_supports(int(dim)))
 
 
-# A step whose longest entry has fewer rows is walked token by token: at 100 rows both ways take the same (34 and 35 us a
-# layer with 16 heads, generalized delta rule), at 300 85 and 39, at 2,048 with 32 heads 581 and 153 (bonus rule 387 and 80,
-# gated rule 421 and 136), 16 prompts of 375 tokens with 32 heads 584 and 229 (394 and 186, 272 and 183).
+# A step whose longest entry has fewer rows is walked token by token: at 128 rows of one entry both ways take the same (41 to 45 and
+# 36 us a layer, generalized delta rule with 8 to 32 heads; 29 and 32 the bonus rule), at 300 with 32 heads 90 and 48, at 2,048
+# 584 and 150 (bonus rule 388 and 80, gated rule 422 and 137).
 RUNS_FROM_ROWS = 128
 RUNS_MIN_ROWS = 64      # rows of a run at least
 # Workgroups of the walk that a step is cut for: four a compute unit, one wave of each a SIMD (32 heads, delta / bonus / gated:
-# 2,048 tokens 164 / 80 / 148 us cut for 512, 153 / 80 / 136 for 1,024, 158 / 79 / 139 for 2,048; 375 tokens a
-# request 229 / 186 / 183 for 1,024 and 370 / 195 / 317 for 2,048: every further run walks the unit columns again).
+# 2,048 tokens 166 / 77 / 143 us in runs of 64 rows, 150 / 77 / 137 of 128, 157 / 98 / 147 of 256).
 RUNS_WORKGROUPS = 1024
-
-
+# From this many heads on that are walked side by side, entries as long as the longest counted, an entry is one run where every
+# further run would walk the unit columns again: 12 prompts of 400 tokens with 16 heads (192) 160 us instead of 169 in runs of 208
+# (generalized delta rule), 16 of 375 with 16 heads (256) 153 instead of 201, 4 of 1,024 with 64 heads (256) 396 and 510.
+RUNS_ONE_FROM = 192
 # Ends and moves of a step at most, a pair for every run and head (32 KB): half a gigabyte. A step of more entries than that walks
 # its rows token by token.
 RUNS_MOST_SCRATCH = 16384
 
 
-def scan_runs(entries: int, rows: int, heads: int, longest: int, unit_columns: bool) -> tuple[int, int]:
+def scan_runs(entries: int, rows: int, heads: int, longest: int, unit_columns: bool, gated: bool = False) -> tuple[int, int]:
     """``(rows a run, runs of the longest entry)`` into which the rows of a matrix-state recurrence with heads of 64
     are cut, or ``(0, 0)`` for token by token. ``entries``, ``rows``: those that bring portions, single tokens aside; ``longest``:
     the most rows that one of them brings, as the host knows it; ``unit_columns``: runs after an entry's first also walk
-    the unit matrix's columns."""
-    if longest < RUNS_FROM_ROWS:
+    the unit matrix's columns; ``gated``: the rule whose decay is one value a head."""
+    from_rows, side_by_side = RUNS_FROM_ROWS, 0
+    if longest > 0:
+        alike = max(1, rows // longest)   # entries that long the step amounts to
+        side_by_side = alike * heads
+    if gated and side_by_side < 336:
+        # token by token this rule is the fastest of the three, and the heads of several entries fill the device as they are.
+        # Rows of the longest entry from which runs take less: 150 with 8 to 32 heads side by side (160 rows: 34 us and 34; of two
+        # entries 34 and 36), 200 with 64 (4 entries of 16 heads, 192 rows 45 and 47, 256 rows 57 and 49), 380 with 96, 700 with
+        # 128 (8 of 16 heads, 200 rows 54 and 73, 700 rows 172 and 180), never with 192 (12 of 16 heads, 400 rows 120 and 139)
+        # and 288 (12 of 24 heads 168 and 188). With more, one run an entry is faster (16 of 375 rows with 32 heads 273 and 183).
+        from_rows += 24 + (20 if entries > 1 else 0) + side_by_side ** 3 // 3800
+    elif side_by_side <= 64 and (entries > 1 or not unit_columns):
+        from_rows += 16   # (2 entries of 128 rows with 32 heads, generalized delta rule: 44.5 and 47.6)
+    if longest < from_rows:
         return 0, 0
-    alike = max(1, rows // longest)   # entries that long the step amounts to
-    runs = max(1, RUNS_WORKGROUPS // (alike * heads * (2 if unit_columns else 1)))
+    runs = max(1, RUNS_WORKGROUPS // (side_by_side * (2 if unit_columns else 1)))
+    if unit_columns and side_by_side >= RUNS_ONE_FROM:
+        runs = 1
     run_rows = max(RUNS_MIN_ROWS, -(-longest // runs))
     run_rows = -(-run_rows // 16) * 16
     if (rows // run_rows + entries) * heads > RUNS_MOST_SCRATCH:
@@ -1941,11 +1956,12 @@ def scan_runs(entries: int, rows: int, heads: int, longest: int, unit_columns: b
     return run_rows, -(-longest // run_rows)
 
 
-def _cut(device: torch.device, entries: int, rows: int, heads: int, longest: int, singles: int, unit_columns: bool) -> tuple:
+def _cut(device: torch.device, entries: int, rows: int, heads: int, longest: int, singles: int, unit_columns: bool,
+         gated: bool = False) -> tuple:
     """What the scans' entry points are told about runs: single-row entries that lead, rows a run, runs of the longest entry, and
     the scratch: the walk's outputs for the unit columns, and per run and head the end state and what moves the one before."""
     portions, rows = entries - singles, rows - singles
-    run_rows, runs = scan_runs(portions, rows, heads, longest, unit_columns) if portions > 0 else (0, 0)
+    run_rows, runs = scan_runs(portions, rows, heads, longest, unit_columns, gated) if portions > 0 else (0, 0)
     if not run_rows:
         return 0, 0, 0, None, None, None
     slots = rows // run_rows + portions
@@ -2162,7 +2178,7 @@ def gated_delta_scan(prep: torch.Tensor, state: torch.Tensor, q_start: torch.Ten
         _dense(t, name, torch.int32, 1)
     entries = state_slots.shape[0]
     _require(q_start.shape[0] == entries + 1 and positions.shape[0] == n, "q_start/state_slots/positions disagree")
-    cut = _cut(o.device, entries, n, heads, longest if dim == vdim == 64 else 0, singles, True)
+    cut = _cut(o.device, entries, n, heads, longest if dim == vdim == 64 else 0, singles, True, gated=True)
     _check(library().dli_gated_delta_scan(
         _ptr(prep), prep.stride(0), _ptr(state), state.stride(0), _ptr(q_start), _ptr(positions), _ptr(state_slots),
         _ptr(o), o.stride(0), entries, n, heads, kv_heads, dim, vdim, *cut[:3], *map(_ptr, cut[3:]), _stream()),

@@ -57,6 +57,18 @@ def test_rule_of_the_cut(ops):
         assert run_rows % 16 == 0 and run_rows >= 64 and run_rows * runs >= longest > run_rows * (runs - 1)
 
 
+def test_rule_where_heads_fill_the_device(ops):
+    """Where entries' heads fill the device token by token the gated rule is walked so, and from many heads on an entry is one run;
+    a short prompt of the rules that are fast token by token is not cut. (Times of both ways beside ``ops.scan_runs``.)"""
+    whole = lambda longest: (-(-longest // 16) * 16, 1)
+    for entries, heads, longest, want in ((1, 16, 128, (0, 0)), (1, 32, 160, (64, 3)), (8, 16, 200, (0, 0)), (4, 32, 512, (0, 0)),
+                                          (12, 16, 400, (0, 0)), (16, 16, 375, (0, 0)), (12, 24, 400, (0, 0)), (16, 32, 375, whole(375)),
+                                          (4, 16, 256, (64, 4)), (1, 32, 2048, (128, 16)), (4, 32, 1024, (256, 4))):
+        assert ops.scan_runs(entries, entries * longest, heads, longest, True, gated=True) == want, (entries, heads, longest)
+    assert ops.scan_runs(1, 128, 32, 128, False) == (0, 0) and ops.scan_runs(4, 576, 16, 144, False) == (64, 3)
+    assert ops.scan_runs(12, 4800, 16, 400, True) == whole(400) and ops.scan_runs(4, 2048, 32, 512, True) == (128, 4)
+
+
 @pytest.mark.parametrize("workgroups", [1024, 12, 1])   # runs of 64 rows, of 176 and the like, and whole entries
 @pytest.mark.parametrize("rule", ["delta", "bonus"])
 def test_recurrent_scan_in_runs(ops, monkeypatch, rule, workgroups):
@@ -252,5 +264,5 @@ def test_whole_models_with_long_portions(ops, monkeypatch, tmp_path, name, dtype
             T.close(got, refs[i], dtype, (i, k))
             if dtype == "float32":
                 assert torch.equal(got, ways[i][0]), (i, k)
-    assert (len([c for c in cuts if c[0]]) >= 8) == (dtype == "bfloat16"), cuts
+    assert (len([c for c in cuts if c[0]]) >= 6) == (dtype == "bfloat16"), cuts
     s.core.manager.check_invariants()

@@ -576,19 +576,18 @@ int dli_gated_delta_scan(const float* prep, int64_t stride, float* state, int64_
   p.prep = prep; p.stride = stride; p.state = state; p.state_stride = state_stride; p.q_start = q_start;
   p.positions = positions; p.state_slots = state_slots; p.o = o; p.o_stride = o_stride; p.heads = heads;
   p.kv_heads = kv_heads; p.vdim = vdim;
-  if (run_rows > 0 && dim == 64 && vdim == 64) {
+  if (run_rows > 0) {
     // the rows of the entries behind the first `singles`, which bring one row each and keep the kernel of steps of single
     // tokens, in runs that are walked side by side (the caller's choice and scratch)
-    if (singles < 0 || singles >= entries) return DLI_ERR_ARGUMENT;
+    if (dim != 64 || vdim != 64 || singles < 0 || singles >= entries) return DLI_ERR_ARGUMENT;
     const int64_t qk = (int64_t)kv_heads * dim;
     const RunsArgs q = {prep, prep + qk, prep + 2 * qk, prep + 2 * qk + (int64_t)heads * vdim, nullptr, nullptr, nullptr, nullptr,
                         stride, stride, stride, stride, 0, 0, 0.f, state, state_stride, q_start + singles, positions,
                         state_slots + singles, o, o_stride, nullptr, 0, y, ends, moves, heads, heads / kv_heads, run_rows, runs,
                         entries - singles, rows - singles, singles};
-    if (scan_runs_takes(q, RUNS_GATED, RUNS_FINISH_SUM, 0)) {
-      if (singles > 0) gated_delta_scan_kernel<4, 1><<<dim3(singles, heads, vdim / 4), 64, 0, stream>>>(p);
-      return scan_runs(q, RUNS_GATED, RUNS_FINISH_SUM, 0, stream);
-    }
+    if (!scan_runs_takes(q, RUNS_GATED, RUNS_FINISH_SUM, 0)) return DLI_ERR_ARGUMENT;
+    if (singles > 0) gated_delta_scan_kernel<4, 1><<<dim3(singles, heads, vdim / 4), 64, 0, stream>>>(p);
+    return scan_runs(q, RUNS_GATED, RUNS_FINISH_SUM, 0, stream);
   }
   const bool single = rows == entries;
   const dim3 grid(entries, heads, (vdim + 3) / 4);

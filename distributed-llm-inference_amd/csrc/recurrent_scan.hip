@@ -404,22 +404,21 @@ extern "C" int dli_recurrent_scan(const float* r, int64_t r_stride, const float*
   p.o_raw = o_raw; p.o_stride = o_stride;
   p.heads = heads;
   if (o_raw == nullptr || o_stride < (int64_t)heads * dim) return DLI_ERR_ARGUMENT;
-  if (run_rows > 0 && dim == 64) {
+  if (run_rows > 0) {
     // the rows of the entries behind the first `singles`, which bring one row each and keep the kernel of steps of single
     // tokens, in runs that are walked side by side (the caller's choice and scratch)
-    if (singles < 0 || singles >= entries) return DLI_ERR_ARGUMENT;
+    if (dim != 64 || singles < 0 || singles >= entries) return DLI_ERR_ARGUMENT;
     const RunsArgs q = {r, k, v, w_pre, a_pre, g_pre, bonus, norm_w, r_stride, k_stride, v_stride, w_stride, a_stride, g_stride, eps,
                         state, state_stride, q_start + singles, positions, state_slots + singles, o_raw, o_stride, out, out_stride,
                         y, ends, moves, heads, 1, run_rows, runs, entries - singles, rows - singles, singles};
     const int walk = rule == RULE_DELTA ? RUNS_DELTA : RUNS_BONUS, finish = rule == RULE_DELTA ? RUNS_FINISH_SIGMOID : RUNS_FINISH_SILU;
-    if (scan_runs_takes(q, walk, finish, out_is_bf16)) {
-      if (singles > 0) {
-        const int status = rule == RULE_DELTA ? launch_scan<RULE_DELTA>(p, singles, singles, dim, out_is_bf16, stream)
-                                              : launch_scan<RULE_BONUS>(p, singles, singles, dim, out_is_bf16, stream);
-        if (status != DLI_OK) return status;
-      }
-      return scan_runs(q, walk, finish, out_is_bf16, stream);
+    if (a_bias != nullptr || !scan_runs_takes(q, walk, finish, out_is_bf16)) return DLI_ERR_ARGUMENT;
+    if (singles > 0) {
+      const int status = rule == RULE_DELTA ? launch_scan<RULE_DELTA>(p, singles, singles, dim, out_is_bf16, stream)
+                                            : launch_scan<RULE_BONUS>(p, singles, singles, dim, out_is_bf16, stream);
+      if (status != DLI_OK) return status;
     }
+    return scan_runs(q, walk, finish, out_is_bf16, stream);
   }
   return rule == RULE_DELTA ? launch_scan<RULE_DELTA>(p, entries, rows, dim, out_is_bf16, stream)
                             : launch_scan<RULE_BONUS>(p, entries, rows, dim, out_is_bf16, stream);

@@ -30,6 +30,6 @@ struct RunsArgs {
 // Slots that hold every run of these entries: the sum of ceil(rows of an entry / run_rows) is no more.
 static inline int scan_runs_slots(int entries, int rows, int run_rows) { return rows / run_rows + entries; }
 
-// Whether these rows can be walked so (16-byte loads and stores).
+// Whether these rows can be walked so (16-byte loads and stores; the caller asks before it makes the scratch).
 bool scan_runs_takes(const RunsArgs& p, int rule, int finish, int out_is_bf16);
 int scan_runs(const RunsArgs& p, int rule, int finish, int out_is_bf16, hipStream_t stream);

@@ -1956,6 +1956,11 @@ def scan_runs(entries: int, rows: int, heads: int, longest: int, unit_columns: b
     return run_rows, -(-longest // run_rows)
 
 
+def _whole(*tensors: torch.Tensor) -> bool:
+    """Whether all rows of these float32 matrices (and vectors) begin on 16-byte boundaries, as the runs' loads ask."""
+    return all(t.data_ptr() % 16 == 0 and (t.dim() < 2 or t.stride(0) % 4 == 0) for t in tensors)
+
+
 def _cut(device: torch.device, entries: int, rows: int, heads: int, longest: int, singles: int, unit_columns: bool,
          gated: bool = False) -> tuple:
     """What the scans' entry points are told about runs: single-row entries that lead, rows a run, runs of the longest entry, and
@@ -2008,7 +2013,9 @@ def recurrent_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, w: torch.T
         _require(bonus.numel() == width, "bonus must hold heads*dim values")
     sa = a_pre.stride(0) if a_pre is not None else 0
     o_raw = torch.empty(n, width, device=out.device, dtype=torch.float32)  # the recurrence's output before norm and gate
-    cut = _cut(out.device, entries, n, heads, longest if dim == 64 else 0, singles, rule == RULE_DELTA)
+    takes = (dim == 64 and _whole(r, k, v, w, g_pre, norm_w, state, *(t for t in (a, bonus) if t is not None))
+             and out.stride(0) % 4 == 0 and out.data_ptr() % (4 * out.element_size()) == 0)
+    cut = _cut(out.device, entries, n, heads, longest if takes else 0, singles, rule == RULE_DELTA)
     _check(library().dli_recurrent_scan(
         _ptr(r), r.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(w_pre), w_pre.stride(0), _ptr(a_pre), sa,
         _ptr(a_bias), _ptr(g_pre), g_pre.stride(0), _ptr(bonus), _ptr(norm_w), float(eps), _ptr(state), state.stride(0),
@@ -2142,7 +2149,7 @@ def conv_prepare(proj: torch.Tensor, b_off: int, a_off: int, conv_w: torch.Tenso
     for name, t in (("a_log", a_log), ("dt_bias", dt_bias)):
         _dense(t, name, torch.float32, 1)
         _require(t.shape[0] == heads, f"{name} must hold a value per head")
-    _dense(out, "out", torch.float32, 2)
+    _f32_rows(out, "out")
     n = proj.shape[0]
     _require(out.shape == (n, channels + 2 * heads), "out must be [n, channels + 2 heads]")
     _require(state.is_cuda and state.dtype == torch.float32 and state.dim() == 2 and state.stride(1) == 1
@@ -2178,7 +2185,8 @@ def gated_delta_scan(prep: torch.Tensor, state: torch.Tensor, q_start: torch.Ten
         _dense(t, name, torch.int32, 1)
     entries = state_slots.shape[0]
     _require(q_start.shape[0] == entries + 1 and positions.shape[0] == n, "q_start/state_slots/positions disagree")
-    cut = _cut(o.device, entries, n, heads, longest if dim == vdim == 64 else 0, singles, True, gated=True)
+    takes = dim == vdim == 64 and _whole(prep, state, o)
+    cut = _cut(o.device, entries, n, heads, longest if takes else 0, singles, True, gated=True)
     _check(library().dli_gated_delta_scan(
         _ptr(prep), prep.stride(0), _ptr(state), state.stride(0), _ptr(q_start), _ptr(positions), _ptr(state_slots),
         _ptr(o), o.stride(0), entries, n, heads, kv_heads, dim, vdim, *cut[:3], *map(_ptr, cut[3:]), _stream()),

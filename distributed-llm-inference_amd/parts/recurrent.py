@@ -95,7 +95,8 @@ class GeneralDelta(_MatrixStateMixer):
 
     def load_weights(self, tensors: Mapping[str, torch.Tensor]) -> None:
         # one product for everything that reads h: r, k, v, g, a, and the first half of the decay's
-        self.w_in = torch.cat([tensors[n] for n in ("r", "k", "v", "g", "a", "w1")], dim=0).contiguous()
+        # (rows of whole 16 bytes, whatever the rank)
+        self.w_in = stack_rows([tensors[n] for n in ("r", "k", "v", "g", "a", "w1")], 4)
         self.rank = tensors["w1"].shape[0]
         self.a_bias = tensors["a.b"]
         self._load_shared(tensors)
@@ -241,7 +242,8 @@ class GatedDelta(Mixer):
             proj = linear_f32(self.rt, as_operand(self.rt, x, ctx), self.w_in)
         g_off = self.channels
         b_off, a_off = g_off + self.hv, g_off + self.hv + H
-        prep = torch.empty(n, self.channels + 2 * H, device=self.rt.device, dtype=torch.float32)
+        width = self.channels + 2 * H
+        prep = torch.empty(n, -(-width // 4) * 4, device=self.rt.device, dtype=torch.float32)[:, :width]   # rows of whole 16 bytes
         ops.conv_prepare(proj, b_off, a_off, self.conv_w, self.a_log, self.dt_bias, state, self.state_floats,
                          ctx.q_start, ctx.positions, ctx.state_slots, prep, H, self.num_kv_heads, self.head_dim,
                          self.value_dim)

@@ -83,14 +83,10 @@ class DecodeGraphs:
         self.enabled = self._supported()
 
     def _supported(self) -> bool:
-        """Graphs are recorded for models all of whose parts can be recorded; on the 32-bit path, where all that keep a
-        cache say so for that type too (``captures_32_bit``). A 32-bit step of few rows is launches more than work:
-        two prompts and four tokens of each at the 135M sizes 14.4 ms launched one by one, 9.3 with the steps replayed."""
+        """Graphs are recorded for models all of whose parts can be recorded. (A 32-bit step of few rows is launches more than
+        work: two prompts and four tokens of each at the 135M sizes 14.4 ms launched one by one, 9.3 with the steps replayed.)"""
         model = self.step_fn.model
-        if self.rt.dtype != torch.bfloat16 and not all(
-                getattr(part, "captures_32_bit", False) for part in model.cache_owners() if part is not None):
-            return False
-        return model.graph_capturable(self.step_fn.store.page_size)
+        return (self.rt.is_bf16 or model.captures_32_bit) and model.graph_capturable(self.step_fn.store.page_size)
 
     def can_run(self, entries: Sequence[StepEntry], steps: int = 1) -> bool:
         if not self.enabled or not entries or len(entries) > self.max_batch:

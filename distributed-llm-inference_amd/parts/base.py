@@ -180,6 +180,9 @@ class Part:
         parts say True (``Model.graph_capturable``); otherwise its decode steps run eagerly."""
         return False
 
+    # Whether that promise also holds for 32-bit steps (they are launched part by part unless every part of the model says so).
+    captures_32_bit = False
+
     def streams(self, ctx: Any) -> bool:
         """Whether this part can run ``ctx``'s step on a :class:`DecodeStream` (its
         ``forward_stream``). Parts that do not implement the fused form return False, and the

@@ -22,6 +22,8 @@ class PreNormBlock(Block):
     def __init__(self, runtime: Runtime) -> None:
         super().__init__(runtime)
 
+    captures_32_bit = True
+
     def graph_capturable(self, page_size: int) -> bool:
         return True  # kernels on device arrays only
 

@@ -36,6 +36,8 @@ class TokenEmbedding(Embedding):
     def sub_parts(self) -> dict:
         return {"norm": self.norm} if self.norm is not None else {}
 
+    captures_32_bit = True
+
     def graph_capturable(self, page_size: int) -> bool:
         return True  # kernels on device arrays only
 

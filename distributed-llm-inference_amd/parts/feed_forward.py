@@ -52,6 +52,8 @@ class GatedMLP(FeedForward):
         self.w_gate_up = self.b_gate_up = self.w_down = self.b_down = None
         self.w_gate_up_tiled = self.w_down_tiled = None
 
+    captures_32_bit = True
+
     def graph_capturable(self, page_size: int) -> bool:
         return True  # kernels on device arrays only
 

@@ -25,6 +25,8 @@ class LinearHead(Head):
         self.weight: Optional[torch.Tensor] = None
         self.weight_tiled: Optional[torch.Tensor] = None
 
+    captures_32_bit = True
+
     def graph_capturable(self, page_size: int) -> bool:
         return True  # kernels on device arrays only
 

@@ -137,6 +137,11 @@ class Model:
             parts.extend(layer.parts.values())
         return all(p.graph_capturable(page_size) for p in parts)
 
+    @property
+    def captures_32_bit(self) -> bool:
+        """Whether that also holds for 32-bit steps: every part, and every part that one owns, says so."""
+        return all(p.captures_32_bit for p in self._all_parts())
+
     def bind_caches(self, layer_caches: Sequence[Any]) -> BoundCaches:
         """Per schedule entry, the cache it uses: its own, or a read-only view of another's."""
         out = BoundCaches()

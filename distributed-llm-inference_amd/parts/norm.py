@@ -25,6 +25,8 @@ class RMSNorm(Norm):
         self.weight_scale = float(weight_scale)
         self.weight: torch.Tensor | None = None
 
+    captures_32_bit = True
+
     def graph_capturable(self, page_size: int) -> bool:
         return True  # kernels on device arrays only
 

@@ -64,6 +64,8 @@ class Rotary(PositionEncoding):
             original_max_position_embeddings)
         self._table: Optional[torch.Tensor] = None
 
+    captures_32_bit = True
+
     def graph_capturable(self, page_size: int) -> bool:
         return True  # kernels on device arrays only
 
@@ -88,6 +90,8 @@ class NoPosition(PositionEncoding):
 
     def __init__(self, runtime: Runtime) -> None:
         super().__init__(runtime)
+
+    captures_32_bit = True
 
     def graph_capturable(self, page_size: int) -> bool:
         return True  # kernels on device arrays only

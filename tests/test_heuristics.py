@@ -174,3 +174,51 @@ def test_which_recorded_shape_stands_in_for_one_that_is_not_recorded():
     assert choice(want, 3, [(8, plans_a, 64, True, 2), (8, plans_a, 64, False, 1)]) is None
     assert choice(want, 3, [(4 * decode_graph.STAND_IN_ROWS, plans_a, 64, True, 1)]) is not None
     assert choice(want, 3, [(4 * decode_graph.STAND_IN_ROWS + 16, plans_a, 64, True, 1)]) is None
+
+
+def test_32_bit_steps_are_recorded_only_where_every_part_says_so():
+    """A model without any cache, a part that borrows one, a feed-forward or a block that promises nothing for 32-bit steps: these are
+    launched part by part, as a part's promise for recorded steps was once given for bfloat16 alone."""
+    from types import SimpleNamespace
+
+    import torch
+
+    import dli_amd.architectures  # noqa: F401
+    from dli_amd.config.registry import resolve_architecture
+    from dli_amd.engine.decode_graph import DecodeGraphs
+    from dli_amd.parts import Runtime
+    from dli_amd.parts.model import Model
+
+    raw = {"architectures": ["LlamaForCausalLM"], "model_type": "llama", "vocab_size": 31, "hidden_size": 64, "intermediate_size": 64,
+           "num_hidden_layers": 2, "num_attention_heads": 1, "num_key_value_heads": 1, "head_dim": 64, "rms_norm_eps": 1e-5,
+           "rope_theta": 1e4, "max_position_embeddings": 64, "tie_word_embeddings": True}
+    arch = resolve_architecture(raw)
+    spec = arch.build_spec(arch.parse_config(raw))
+
+    def recorded(dtype, change=lambda model: None):
+        rt = Runtime(torch.device("cpu"), dtype)
+        model = Model(spec, rt)
+        change(model)
+        graphs = DecodeGraphs.__new__(DecodeGraphs)
+        graphs.rt, graphs.step_fn = rt, SimpleNamespace(model=model, store=SimpleNamespace(page_size=16))
+        return graphs._supported()
+
+    class Promises:   # recorded in bfloat16; nothing said of 32-bit
+        captures_32_bit, cache_spec = False, staticmethod(lambda: None)
+        graph_capturable = staticmethod(lambda page_size: True)
+        sub_parts = staticmethod(dict)
+
+    def without_cache(model):
+        for layer in model.layers:
+            layer.parts["mixer"] = Promises()
+
+    def borrowing(model):
+        model.layers[1].parts["mixer"] = Promises()
+
+    def other_feed_forward(model):
+        model.layers[0].parts["feed_forward"] = Promises()
+
+    assert recorded(torch.float32) and recorded(torch.bfloat16)
+    for change in (without_cache, borrowing, other_feed_forward):
+        assert not recorded(torch.float32, change), change
+        assert recorded(torch.bfloat16, change), change

@@ -6,7 +6,8 @@
 // turn, each with an online softmax of its own, merged through LDS. S = K Q^T and O^T = V^T P^T (v_mfma_f32_16x16x16_bf16): lane
 // (col, grp) holds the scores of head `col` with keys 4 grp .. + 3, which are the operand of the second product as they stand.
 // A weight is not rounded: it goes into the second product as the three bfloat16 values that add up to its 24 bits, three
-// products for one (there is little else for the matrix cores to do here).
+// products for one (there is little else for the matrix cores to do here). Its bits are cut into three, none of them negative and,
+// where the rest is none, 2^-32 of the weight instead: an infinite value then stays infinite and makes no NaN of its own.
 //
 // What bounds it: the chain of trips to memory (table entry, keys and values) of a wave's pairs of tiles, of which two are on
 // their way at a time, and fetching its own instructions: every launch finds the instruction cache cold, so the code is
@@ -24,7 +25,6 @@ __device__ __forceinline__ float as_column_max(float v) {   // over the four lan
   v = fmaxf(v, __shfl_xor(v, 16, DLI_WAVE));
   return fmaxf(v, __shfl_xor(v, 32, DLI_WAVE));
 }
-__device__ __forceinline__ short as_bits(bf16_t x) { return *reinterpret_cast<const short*>(&x); }
 
 template <int DCH, int VCH, bool PEN>   // keys of up to 16 DCH components, values of up to 16 VCH; with r1 and r2
 __global__ __launch_bounds__(256) void attention_singles_kernel(SinglesArgs a) {
@@ -129,12 +129,14 @@ __global__ __launch_bounds__(256) void attention_singles_kernel(SinglesArgs a) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float p = __builtin_amdgcn_exp2f(s[u][i] - m_safe);
-        const bf16_t hi = (bf16_t)p;
-        const float rest = p - (float)hi;
-        const bf16_t mid = (bf16_t)rest;
-        part[0][i] = as_bits(hi);
-        part[1][i] = as_bits(mid);
-        part[2][i] = as_bits((bf16_t)(rest - (float)mid));
+        const float least = p * 0x1p-32f;
+        float part_of = p;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const unsigned bits = __builtin_bit_cast(unsigned, part_of) & 0xffff0000u;
+          part[k][i] = (short)(bits >> 16);
+          part_of = fmaxf(part_of - __builtin_bit_cast(float, bits), least);
+        }
         l += p;
       }
 #pragma unroll

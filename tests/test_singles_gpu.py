@@ -95,6 +95,24 @@ def test_single_tokens(ops, H, G, D, V, extra):
             print(H, D, V, case.keys(), out32, worst)
 
 
+@pytest.mark.parametrize("n", [1, 40, 700])
+def test_infinite_values(ops, n):
+    """A value that is infinite makes its component of the result infinite with its sign, as one sum over the weights does, and
+    leaves the other components alone; a weight of exactly one is among them (a single key)."""
+    H, G, D, ps = 4, 2, 32, 16
+    gen = torch.Generator().manual_seed(n)
+    q = torch.randn(1, H * D, dtype=F, generator=gen).bfloat16().double()
+    k, v = (torch.randn(n, G, D, dtype=F, generator=gen).bfloat16().double() for _ in range(2))
+    v[n // 2, 0, 3], v[n // 3, 1, 7], v[n - 1, 1, 7], v[0, 1, 30] = float("inf"), float("-inf"), float("-inf"), float("inf")
+    kp, vp, table = paged(k, v, ps, torch.bfloat16)
+    got = run(ops, q, kp, vp, [table], [n], H, True, None, 0, scale=D ** -0.5)[0]
+    s = torch.einsum("hgd,nhd->hgn", q.view(G, H // G, D), k) * D ** -0.5
+    ref = torch.einsum("hgn,nhv->hgv", s.softmax(2), v).reshape(H * D)
+    assert not ref.isnan().any() and ref.isinf().sum() == 6
+    assert torch.equal(got.isinf(), ref.isinf()) and torch.equal(got[ref.isinf()], ref[ref.isinf()])
+    assert (got - ref)[ref.isfinite()].abs().max() < 1.5e-5
+
+
 def test_splits_and_replays(ops):
     """Few requests over a wide table: the keys are cut, and a captured step gives the same again for other lengths."""
     gen = torch.Generator().manual_seed(5)

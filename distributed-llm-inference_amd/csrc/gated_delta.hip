@@ -55,27 +55,30 @@ struct PrepArgs {
 };
 
 // The convolution of channel c at `row`, which lies at position pos of its request, whose step starts at row `first`, and silu. An
-// input lies among the step's rows or the kept inputs, or before the sequence (zero; another input is read in its place). Four taps
-// are asked for together: no load hangs on a condition.
+// input lies among the step's rows or the kept inputs, or before the sequence (zero; another input is read in its place). The taps
+// are asked for together (TAPS of them, or where that is 0 four at a time): no load hangs on a condition. Oldest input first.
+template <int TAPS>
 __device__ __forceinline__ float conv_silu(const PrepArgs& p, const float* kept, int channels, int row, int first, int pos, int c) {
-  const float* w = p.conv_w + (int64_t)c * p.taps;
+  constexpr int AT_ONCE = TAPS > 0 ? TAPS : 4;
+  const int taps = TAPS > 0 ? TAPS : p.taps;
+  const float* w = p.conv_w + (int64_t)c * taps;
   float acc = 0.f;
-  if (row - (p.taps - 1) >= first) {                            // (most rows of a portion)
-    const float* x = p.proj + (int64_t)(row - (p.taps - 1)) * p.stride + c;
+  if (row - (taps - 1) >= first) {                              // (most rows of a portion)
+    const float* x = p.proj + (int64_t)(row - (taps - 1)) * p.stride + c;
 #pragma unroll 4
-    for (int t = 0; t < p.taps; ++t) acc = fmaf(w[t], x[(int64_t)t * p.stride], acc);
+    for (int t = 0; t < taps; ++t) acc = fmaf(w[t], x[(int64_t)t * p.stride], acc);
   } else {
-    for (int t0 = 0; t0 < p.taps; t0 += 4) {                    // tap t: the input taps - 1 - t places back, oldest first
-      float in[4], wt[4];
+    for (int t0 = 0; t0 < taps; t0 += AT_ONCE) {                // tap t: the input taps - 1 - t places back
+      float in[AT_ONCE], wt[AT_ONCE];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int t = min(t0 + k, p.taps - 1), back = min(p.taps - 1 - t, pos), src = row - back;
-        in[k] = *(src >= first ? p.proj + (int64_t)src * p.stride + c : kept + (int64_t)(p.taps - 1 - (first - src)) * channels + c);
+      for (int k = 0; k < AT_ONCE; ++k) {
+        const int t = min(t0 + k, taps - 1), back = min(taps - 1 - t, pos), src = row - back;
+        in[k] = *(src >= first ? p.proj + (int64_t)src * p.stride + c : kept + (int64_t)(taps - 1 - (first - src)) * channels + c);
         wt[k] = w[t];
       }
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (t0 + k < p.taps) acc = fmaf(wt[k], p.taps - 1 - (t0 + k) <= pos ? in[k] : 0.f, acc);
+      for (int k = 0; k < AT_ONCE; ++k)
+        if (t0 + k < taps) acc = fmaf(wt[k], taps - 1 - (t0 + k) <= pos ? in[k] : 0.f, acc);
     }
   }
   return acc / (1.f + expf(-acc));
@@ -94,6 +97,7 @@ __device__ __forceinline__ float conv_unit_scale(const PrepArgs& p, int unit, fl
   return (1.f / sqrtf(wave_sum(ss) + 1e-6f)) * (unit < p.kv_heads ? 1.f / sqrtf((float)p.dim) : 1.f);
 }
 // One row of a unit of q, k or v.
+template <int TAPS>
 __device__ __forceinline__ void conv_prepare_row(const PrepArgs& p, int row, int unit) {
   const int lane = threadIdx.x, qk = p.kv_heads * p.dim, channels = 2 * qk + p.heads * p.vdim;
   float* out = p.out + (int64_t)row * p.out_stride;
@@ -102,13 +106,13 @@ __device__ __forceinline__ void conv_prepare_row(const PrepArgs& p, int row, int
   const float* kept = p.kept + (int64_t)p.state_slots[e] * p.state_stride;
   if (unit >= 2 * p.kv_heads) {
     const int c = 2 * qk + (unit - 2 * p.kv_heads) * 64 + lane;
-    if (c < channels) out[c] = conv_silu(p, kept, channels, row, first, pos, c);
+    if (c < channels) out[c] = conv_silu<TAPS>(p, kept, channels, row, first, pos, c);
     return;
   }
   const int c0 = unit * p.dim;                                  // q heads, then k heads
   float ss = 0.f;
   for (int c = lane; c < p.dim; c += DLI_WAVE) {
-    const float y = conv_silu(p, kept, channels, row, first, pos, c0 + c);
+    const float y = conv_silu<TAPS>(p, kept, channels, row, first, pos, c0 + c);
     out[c0 + c] = y;
     ss += y * y;
   }
@@ -117,9 +121,10 @@ __device__ __forceinline__ void conv_prepare_row(const PrepArgs& p, int row, int
 }
 
 // A wave a (row, unit): steps of few rows.
+template <int TAPS>
 __global__ __launch_bounds__(64) void conv_prepare_kernel(PrepArgs p) {
   const int row = blockIdx.x, unit = blockIdx.y;
-  if (unit + 1 < (int)gridDim.y) { conv_prepare_row(p, row, unit); return; }
+  if (unit + 1 < (int)gridDim.y) { conv_prepare_row<TAPS>(p, row, unit); return; }
   const int channels = 2 * p.kv_heads * p.dim + p.heads * p.vdim;
   for (int h = threadIdx.x; h < p.heads; h += DLI_WAVE)
     conv_prepare_gates(p, row, h, p.out + (int64_t)row * p.out_stride + channels + h);
@@ -127,13 +132,24 @@ __global__ __launch_bounds__(64) void conv_prepare_kernel(PrepArgs p) {
 
 // A wave PREP_RUN neighbouring rows of a unit, up to PREP_TAPS taps: a channel's inputs are read once for all rows that they reach
 // where the run lies in one entry with its inputs among the step's rows; other runs take the rows one by one, in the same order of
-// sums. Us a call, 3,072 channels and 32 heads, a wave a row -> now: 2,990 rows of 4 requests 54 -> 28, 1,030 of 3 23 -> 18. Not
-// below 1,024 rows (256 rows of 4 requests 8.5 and 13.6) nor with under 64 rows a request (1,030 of 32 25.1 and 25.9).
+// sums. Us a call, 3,072 channels and 32 heads, a wave a row -> now: 2,990 rows of 4 requests 53 -> 26, 1,100 of one 23.5 -> 16. It
+// takes enough waves to make up for a wave's eight rows one after the other, the more the fewer taps a row has: with heads of 64
+// and four taps 3,328 waves 13.4 -> 12.4 us and 2,444 11.5 -> 12.6, with two taps and heads of 32 6,144 16.5 -> 16.0 and 4,500
+// 13.3 -> 14.5; heads above 64, whose lanes store before they scale, three taps, heads of 128: 12,375 41.8 -> 34.5, 8,448 30.8 ->
+// 33.7. Not below 1,024 rows (256 rows of 4 requests 8.5 and 13.6) nor with under 64 rows a request (1,030 of 32 25.1 and 25.9).
 #define PREP_RUN 8
 #define PREP_TAPS 4
 #define PREP_FROM_ROWS 1024
+static bool conv_prepare_in_runs(int rows, int entries, int units, int dim, int taps) {
+  const int64_t waves = (int64_t)((rows + PREP_RUN - 1) / PREP_RUN) * units;
+  return rows >= PREP_FROM_ROWS && rows / 64 >= entries && taps <= PREP_TAPS && waves * taps >= (dim <= DLI_WAVE ? 16000 : 29000);
+}
 __global__ __launch_bounds__(64) void conv_prepare_run_kernel(PrepArgs p, int rows) {
-  const int row0 = blockIdx.x * PREP_RUN, unit = blockIdx.y, lane = threadIdx.x, last = min(row0 + PREP_RUN, rows);
+  // (of several entries the runs are turned by the unit: those that take their rows one by one lie where entries begin, often at
+  // multiples of eight runs, and would all fall to one XCD: 16 requests of 128 rows, 32 heads, 40.6 us, so 24.3)
+  const int unit = blockIdx.y, turn = p.entries > 1 ? (blockIdx.x + blockIdx.y) % gridDim.x : blockIdx.x;
+  const int row0 = turn * PREP_RUN, lane = threadIdx.x;
+  const int last = min(row0 + PREP_RUN, rows);
   const int qk = p.kv_heads * p.dim, channels = 2 * qk + p.heads * p.vdim;
   if (unit + 1 == (int)gridDim.y) {
     for (int i = lane; i < (last - row0) * p.heads; i += DLI_WAVE) {
@@ -144,7 +160,7 @@ __global__ __launch_bounds__(64) void conv_prepare_run_kernel(PrepArgs p, int ro
   }
   const int e = gd_entry_of_row(p.q_start, p.entries, row0);
   if (row0 - (PREP_TAPS - 1) < p.q_start[e] || row0 + PREP_RUN > p.q_start[e + 1]) {
-    for (int row = row0; row < last; ++row) conv_prepare_row(p, row, unit);
+    for (int row = row0; row < last; ++row) conv_prepare_row<0>(p, row, unit);
     return;
   }
   const auto convolve = [&](int c, float (&y)[PREP_RUN]) {
@@ -484,6 +500,11 @@ extern "C" {
 
 int dli_gated_delta_max_taps() { return GD_MAX_TAPS; }
 
+// Whether a step's rows are convolved PREP_RUN at a time.
+int dli_conv_prepare_in_runs(int rows, int entries, int heads, int kv_heads, int dim, int vdim, int taps) {
+  return rows > 0 && entries > 0 && conv_prepare_in_runs(rows, entries, 2 * kv_heads + (int)(((int64_t)heads * vdim + 63) / 64) + 1, dim, taps);
+}
+
 int dli_conv_prepare(const float* proj, int64_t stride, int b_off, int a_off, const float* conv_w, const float* a_log,
                      const float* dt_bias, float* state, int64_t state_stride, int64_t kept_offset, const int* q_start,
                      const int* positions, const int* state_slots, float* out, int64_t out_stride, int entries, int rows,
@@ -501,10 +522,14 @@ int dli_conv_prepare(const float* proj, int64_t stride, int b_off, int a_off, co
   p.heads = heads; p.kv_heads = kv_heads; p.dim = dim; p.vdim = vdim; p.taps = taps;
   const int units = 2 * kv_heads + (int)(((int64_t)heads * vdim + 63) / 64) + 1;
   if (units > 65535) return DLI_ERR_ARGUMENT;
-  if (rows >= PREP_FROM_ROWS && rows / 64 >= entries && taps <= PREP_TAPS)
+  if (conv_prepare_in_runs(rows, entries, units, dim, taps))
     conv_prepare_run_kernel<<<dim3((rows + PREP_RUN - 1) / PREP_RUN, units), 64, 0, stream>>>(p, rows);
+  else if (taps == 3)   // (numbers that four does not divide: known ones are asked for together)
+    conv_prepare_kernel<3><<<dim3(rows, units), 64, 0, stream>>>(p);
+  else if (taps == 2)
+    conv_prepare_kernel<2><<<dim3(rows, units), 64, 0, stream>>>(p);
   else
-    conv_prepare_kernel<<<dim3(rows, units), 64, 0, stream>>>(p);
+    conv_prepare_kernel<0><<<dim3(rows, units), 64, 0, stream>>>(p);
   if (dli_launch_status() != DLI_OK) return DLI_ERR_LAUNCH;
   if (taps > 1) {
     const dim3 grid(entries, (unsigned)((channels + 255) / 256));

@@ -46,10 +46,13 @@ def test_norms_at_the_edges_of_what_is_held(ops, width):
     assert float((out.double() - want).abs().max()) < 2e-5 * max(1.0, width ** 0.5 / 10)   # cubes: results of up to sqrt(width)
 
 
-@pytest.mark.parametrize("dim,vdim,taps", [(64, 64, 4), (128, 48, 3), (40, 100, 1), (16, 130, 2)])
-def test_runs_of_rows_convolve_alike(ops, dim, vdim, taps):
+@pytest.mark.parametrize("dim,vdim,taps,heads,kv_heads", [(64, 64, 4, 32, 2), (128, 48, 3, 96, 4), (40, 100, 1, 80, 2), (16, 130, 2, 28, 4),
+                                                          (64, 64, 4, 4, 2), (128, 48, 3, 4, 2)])
+def test_runs_of_rows_convolve_alike(ops, dim, vdim, taps, heads, kv_heads):
     """A step of many rows gives the bits of the wave a row (chosen when there are many requests: empty ones are added)."""
-    heads, kv_heads, lengths, starts = 4, 2, [1, 7, 530, 3, 491], [0, 9, 0, 1, 2]
+    lengths, starts = [1, 7, 530, 3, 491], [0, 9, 0, 1, 2]
+    in_runs = lambda entries: bool(ops.library().dli_conv_prepare_in_runs(sum(lengths), entries, heads, kv_heads, dim, vdim, taps))
+    assert in_runs(5) == (heads > 4) and not in_runs(45)
     rows, channels = sum(lengths), 2 * kv_heads * dim + heads * vdim
     gen = torch.Generator(device="cuda").manual_seed(dim)
     draw = lambda *s: torch.randn(*s, device="cuda", generator=gen)

@@ -275,10 +275,17 @@ __device__ __forceinline__ float lowrank_activated(float y, int out_act) {
 
 // Sixteen rows a workgroup: a thread makes four neighbouring features of four rows, so that the weights, which a workgroup a row
 // reads again for every row, come once for sixteen (the same four sums a value, so the same bits). What bounds it: two
-// exponentials and two divisions a value on the vector units. 2,048 features, rank 64, with rates, us: 2,048 rows 53.7 a row a
-// workgroup and 30.4 here, 512 rows 14.8 and 16.2, 64 rows 4.6 and 14.7 (a thread's sixteen values take that long alone).
+// exponentials and two divisions a value on the vector units, and under some hundred workgroups a thread's sixteen values one
+// after the other (11 us at rank 8, 16 at 64, 36 at 256, whatever the rows). lowrank_takes_rows says where it is ahead (us, a
+// row a workgroup and this, with rates: 2,048 rows of 2,048 features, rank 64, 51 and 30; 1,000 of 4,096 51 and 31; 1,536
+// of 1,024 21.2 and 19.0; 1,000 of 1,024 15.3 and 18.1; 768 of 512 7.6 and 16.2; rank 8: 2,048 of 2,048 20.8 and 19.5, 2,048 of
+// 1,024 12.0 and 14.2; rank 256: 768 of 1,024 37.9 and 36.7; rank 512: 768 of 4,096 237 and 105).
 #define LOWRANK_ROWS 16
-#define LOWRANK_FROM_ROWS 768
+// The crossover lies at 3.1, 2.3, 1.7, 1.2 and 0.8 million values for ranks of 8, 32, 64, 128 and 256.
+static bool lowrank_takes_rows(int rows, int features, int rank) {
+  return rows >= 16 * LOWRANK_ROWS && rank % 4 == 0 && rank <= 512 && features % 4 == 0 &&
+         (int64_t)rows * features * ((rank < 224 ? rank : 224) + 64) >= (int64_t)216 << 20;
+}
 __global__ __launch_bounds__(256) void lowrank_out_rows_kernel(LowrankArgs p) {
   typedef float f4 __attribute__((ext_vector_type(4)));
   extern __shared__ __attribute__((aligned(16))) float ts[];   // [LOWRANK_ROWS][rank]
@@ -340,6 +347,11 @@ __global__ __launch_bounds__(256) void lowrank_out_rows_kernel(LowrankArgs p) {
   }
 }
 
+// A row a workgroup, a feature a thread. AHEAD: sixteen weights on their way at a time, where the workgroups are few (up to
+// LOWRANK_AHEAD_GROUPS: one row of 2,048 features, rank 64, 4.1 us four at a time and 3.2 so; 300 rows of 1,024, rank 128, 7.9 and
+// 9.4: there the device's waves are ahead enough for each other).
+#define LOWRANK_AHEAD_GROUPS 768
+template <bool AHEAD>
 __global__ void lowrank_out_kernel(const float* __restrict__ t, int64_t t_stride, const float* __restrict__ w2t,
                                    const float* __restrict__ bias, float* __restrict__ out, int features, int rank,
                                    int act, int out_act, float* __restrict__ rate, int64_t rate_stride,
@@ -355,7 +367,8 @@ __global__ void lowrank_out_kernel(const float* __restrict__ t, int64_t t_stride
   if (c >= features) return;
   float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;          // four sums: the weights' loads do not wait for each other
   int j = 0;
-  for (; j + 16 <= rank; j += 16) {                      // (sixteen of them on their way; four at a time: 4.1 us at rank 64, 3.2 so)
+  if constexpr (AHEAD)
+  for (; j + 16 <= rank; j += 16) {
     float w[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) w[e] = w2t[(int64_t)(j + e) * features + c];
@@ -935,18 +948,27 @@ int dli_lowrank_out(const float* t, int64_t t_stride, const float* w2t, const fl
       (rate != nullptr && rate_stride < features))
     return DLI_ERR_ARGUMENT;
   const auto whole = [](const void* at) { return (uintptr_t)at % 16 == 0; };
-  // (with fewer rows the workgroups of a row are what fills the device; 16-byte accesses throughout)
-  if (rows >= LOWRANK_FROM_ROWS && rank % 4 == 0 && rank <= 512 && features % 4 == 0 && whole(w2t) && whole(out) &&
+  // (16-byte accesses throughout)
+  if (lowrank_takes_rows(rows, features, rank) && whole(w2t) && whole(out) &&
       (rate == nullptr || (rate_stride % 4 == 0 && whole(rate)))) {
     const LowrankArgs p = {t, w2t, bias, out, rows, features, rank, act, out_act, t_stride, rate, rate_stride, rate_bias};
     lowrank_out_rows_kernel<<<dim3((rows + LOWRANK_ROWS - 1) / LOWRANK_ROWS, (features + 255) / 256), 256,
                               LOWRANK_ROWS * rank * sizeof(float), stream>>>(p);
     return dli_launch_status();
   }
-  lowrank_out_kernel<<<dim3(rows, (features + 255) / 256), 256, rank * sizeof(float), stream>>>(t, t_stride, w2t, bias, out,
-                                                                                                features, rank, act, out_act,
-                                                                                                rate, rate_stride, rate_bias);
+  const dim3 grid(rows, (features + 255) / 256);
+  if (rank >= 16 && (int64_t)grid.x * grid.y <= LOWRANK_AHEAD_GROUPS)
+    lowrank_out_kernel<true><<<grid, 256, rank * sizeof(float), stream>>>(t, t_stride, w2t, bias, out, features, rank, act, out_act,
+                                                                          rate, rate_stride, rate_bias);
+  else
+    lowrank_out_kernel<false><<<grid, 256, rank * sizeof(float), stream>>>(t, t_stride, w2t, bias, out, features, rank, act, out_act,
+                                                                           rate, rate_stride, rate_bias);
   return dli_launch_status();
+}
+
+// Whether so many rows are made sixteen a workgroup.
+int dli_lowrank_takes_rows(int rows, int features, int rank) {
+  return rows > 0 && features > 0 && rank > 0 && lowrank_takes_rows(rows, features, rank);
 }
 
 int dli_qk_unit_cache(const float* proj, int64_t stride, int q_off, int k_off, int v_off, void* q_out,

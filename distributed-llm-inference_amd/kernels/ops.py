@@ -150,6 +150,7 @@ _SIGNATURES = {
                           _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr],
     "dli_token_shift": [_c_ptr, _c_ptr, _c_int, _c_ptr, _c_i64, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int,
                         _c_int, _c_ptr],
+    "dli_lowrank_takes_rows": [_c_int, _c_int, _c_int],
     "dli_lowrank_out": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_i64,
                         _c_ptr, _c_ptr],
     "dli_qk_unit_cache": [_c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,

@@ -47,9 +47,14 @@ def test_grouped_attention_with_a_penalty(ops, H, G, D, V, ps, scale):
                 assert (out.cpu().double() - want).abs().max() < 3e-2, (case, first, out32)
 
 
-@pytest.mark.parametrize("rows", [767, 768, 769, 1000])
-@pytest.mark.parametrize("features,rank", [(4, 4), (260, 8), (1024, 64), (96, 512)])
+@pytest.mark.parametrize("rows,features,rank", [(rows, *sizes) for rows in (767, 768, 769, 1000)
+                                                for sizes in ((4, 4), (260, 8), (1024, 64), (96, 512))]
+                         + [(1009, 4100, 4), (2050, 1604, 8), (770, 2308, 64), (257, 4612, 128), (1023, 772, 512), (300, 100, 128),
+                            (300, 1028, 100), (7, 33, 21)])
 def test_lowrank_rows_have_the_single_rows_bits(ops, rows, features, rank):
+    """Rows made sixteen a workgroup, rows of few and of many workgroups of their own: the bits of a row alone."""
+    assert bool(ops.library().dli_lowrank_takes_rows(rows, features, rank)) == (
+        (rows, features, rank) in ((1009, 4100, 4), (2050, 1604, 8), (770, 2308, 64), (257, 4612, 128), (1023, 772, 512)))
     gen = torch.Generator(device="cuda").manual_seed(rows + features)
     t = torch.randn(rows, rank + 3, device="cuda", generator=gen)[:, :rank]
     w2t, bias = torch.randn(rank, features, device="cuda", generator=gen), torch.randn(features, device="cuda", generator=gen)

@@ -578,29 +578,31 @@ __global__ __launch_bounds__(256) void rotary_cache_kernel(const float* __restri
 // asked for together, with their weights, and held for the second pass (longer rows read the rest twice). Sums run in the same
 // order as one value after the other. Us a call of 2,048 values, 4 and 3,000 rows, one value after the other -> now: group_norm of
 // 4 parts 3.1 -> 2.5 and 22.4 -> 16.6, branch_norm_mean of 2 4.6 -> 4.0 and 20.1 -> 16.7, rms_norm_pair 3.1 -> 2.5 and 14.3 -> 11.0.
+// HELD of them: one where a row has no more, which the other loads would only delay (3,000 rows of 64, two branches, 5.2 and 5.7 us),
+// none where the second reading is most of the work (rms_norm_pair of 12,000 values 8.2 and 9.1).
 #define NORM_HELD 4
 
 // x [rows][width] float32 (with delta: x += delta first, stored); each of `groups` equal consecutive
 // parts of the row is divided by its own root mean square; out(T) = w * that. A workgroup a (row, part).
-template <typename T>
+template <typename T, int HELD>
 __global__ void group_norm_kernel(float* __restrict__ x, const float* __restrict__ delta, int64_t delta_stride,
                                   const float* __restrict__ weight, T* __restrict__ out, int width, int groups, float eps) {
   __shared__ float scratch[16];
   const int64_t row = blockIdx.x;
-  const int part = width / groups, first = blockIdx.y * part, end = first + part, tail = first + threadIdx.x + NORM_HELD * blockDim.x;
+  const int part = width / groups, first = blockIdx.y * part, end = first + part, tail = first + threadIdx.x + HELD * blockDim.x;
   float* xr = x + row * width;
-  float held[NORM_HELD], w[NORM_HELD], d[NORM_HELD];
+  float held[HELD > 0 ? HELD : 1], w[HELD > 0 ? HELD : 1], d[HELD > 0 ? HELD : 1];
 #pragma unroll
-  for (int k = 0; k < NORM_HELD; ++k) held[k] = xr[min((int)(first + threadIdx.x + k * blockDim.x), end - 1)];
+  for (int k = 0; k < HELD; ++k) held[k] = xr[min((int)(first + threadIdx.x + k * blockDim.x), end - 1)];
   if (delta != nullptr) {
 #pragma unroll
-    for (int k = 0; k < NORM_HELD; ++k) d[k] = delta[row * delta_stride + min((int)(first + threadIdx.x + k * blockDim.x), end - 1)];
+    for (int k = 0; k < HELD; ++k) d[k] = delta[row * delta_stride + min((int)(first + threadIdx.x + k * blockDim.x), end - 1)];
   }
 #pragma unroll
-  for (int k = 0; k < NORM_HELD; ++k) w[k] = weight[min((int)(first + threadIdx.x + k * blockDim.x), end - 1)];
+  for (int k = 0; k < HELD; ++k) w[k] = weight[min((int)(first + threadIdx.x + k * blockDim.x), end - 1)];
   float ss = 0.f;
 #pragma unroll
-  for (int k = 0; k < NORM_HELD; ++k) {
+  for (int k = 0; k < HELD; ++k) {
     const int i = first + threadIdx.x + k * blockDim.x;
     if (i < end) {
       if (delta != nullptr) {
@@ -620,7 +622,7 @@ __global__ void group_norm_kernel(float* __restrict__ x, const float* __restrict
   }
   const float r = 1.f / sqrtf(block_sum(ss, scratch) / (float)part + eps);
 #pragma unroll
-  for (int k = 0; k < NORM_HELD; ++k) {
+  for (int k = 0; k < HELD; ++k) {
     const int i = first + threadIdx.x + k * blockDim.x;
     if (i < end) out[row * width + i] = from_f32<T>(w[k] * (held[k] * r));
   }
@@ -635,16 +637,16 @@ struct BranchArgs {
 
 // (the branches' sums of squares are made side by side and meet in one exchange through LDS; COUNT is a
 // template parameter so that no load hangs on a condition)
-template <int COUNT>
+template <int COUNT, int HELD>
 __global__ void branch_norm_mean_kernel(BranchArgs b, float* __restrict__ out, int width, float eps) {
   __shared__ float scratch[COUNT][16];
   const int64_t row = blockIdx.x;
   const int lane = threadIdx.x % DLI_WAVE, wave = threadIdx.x / DLI_WAVE, waves = blockDim.x / DLI_WAVE;
-  float ss[COUNT], held[COUNT][NORM_HELD], wt[COUNT][NORM_HELD];
+  float ss[COUNT], held[COUNT][HELD], wt[COUNT][HELD];
 #pragma unroll
   for (int j = 0; j < COUNT; ++j)
 #pragma unroll
-    for (int k = 0; k < NORM_HELD; ++k) {
+    for (int k = 0; k < HELD; ++k) {
       const int i = min((int)(threadIdx.x + k * blockDim.x), width - 1);
       held[j][k] = b.y[j][row * b.stride[j] + i];
       wt[j][k] = b.weight[j][i];
@@ -653,10 +655,10 @@ __global__ void branch_norm_mean_kernel(BranchArgs b, float* __restrict__ out, i
   for (int j = 0; j < COUNT; ++j) {
     ss[j] = 0.f;
 #pragma unroll
-    for (int k = 0; k < NORM_HELD; ++k)
+    for (int k = 0; k < HELD; ++k)
       if ((int)(threadIdx.x + k * blockDim.x) < width) ss[j] += held[j][k] * held[j][k];
   }
-  const int tail = threadIdx.x + NORM_HELD * blockDim.x;
+  const int tail = threadIdx.x + HELD * blockDim.x;
   for (int i = tail; i < width; i += blockDim.x)
 #pragma unroll
     for (int j = 0; j < COUNT; ++j) {
@@ -678,7 +680,7 @@ __global__ void branch_norm_mean_kernel(BranchArgs b, float* __restrict__ out, i
   }
   const float share = 1.f / (float)COUNT;
 #pragma unroll
-  for (int k = 0; k < NORM_HELD; ++k) {
+  for (int k = 0; k < HELD; ++k) {
     const int i = threadIdx.x + k * blockDim.x;
     float sum = 0.f;
 #pragma unroll
@@ -736,28 +738,28 @@ __global__ void scale_f32_kernel(float* __restrict__ y, int64_t n, float scale) 
 
 // Two norms of the same float32 row with one pass over its statistics: out1 = w1 * x * r, out2 = w2 * x * r,
 // r = 1 / sqrt(mean(x^2) + eps) (a mixer and a feed-forward that read the same stream behind norms of their own).
-template <typename T>
+template <typename T, int HELD>
 __global__ void rms_norm_pair_kernel(const float* __restrict__ x, const float* __restrict__ w1, const float* __restrict__ w2,
                                      T* __restrict__ out1, T* __restrict__ out2, int width, float eps) {
   __shared__ float scratch[16];
   const int64_t row = blockIdx.x;
   const float* xr = x + row * width;
-  const int tail = threadIdx.x + NORM_HELD * blockDim.x;
-  float held[NORM_HELD], w[2][NORM_HELD], ss = 0.f;
+  const int tail = threadIdx.x + HELD * blockDim.x;
+  float held[HELD > 0 ? HELD : 1], w[2][HELD > 0 ? HELD : 1], ss = 0.f;
 #pragma unroll
-  for (int k = 0; k < NORM_HELD; ++k) {
+  for (int k = 0; k < HELD; ++k) {
     const int i = min((int)(threadIdx.x + k * blockDim.x), width - 1);
     held[k] = xr[i];
     w[0][k] = w1[i];
     w[1][k] = w2[i];
   }
 #pragma unroll
-  for (int k = 0; k < NORM_HELD; ++k)
+  for (int k = 0; k < HELD; ++k)
     if ((int)(threadIdx.x + k * blockDim.x) < width) ss += held[k] * held[k];
   for (int i = tail; i < width; i += blockDim.x) ss += xr[i] * xr[i];
   const float r = 1.f / sqrtf(block_sum(ss, scratch) / (float)width + eps);
 #pragma unroll
-  for (int k = 0; k < NORM_HELD; ++k) {
+  for (int k = 0; k < HELD; ++k) {
     const int i = threadIdx.x + k * blockDim.x;
     const float v = held[k] * r;
     if (i < width) {
@@ -1026,10 +1028,12 @@ int dli_group_norm(float* x, const float* delta, int64_t delta_stride, const flo
   if (groups > 65535) return DLI_ERR_ARGUMENT;
   const int part = width / groups, threads = part >= 2048 ? 512 : part >= 512 ? 256 : part >= 128 ? 128 : 64;
   const dim3 grid(rows, groups);
-  if (is_bf16)
-    group_norm_kernel<bf16_t><<<grid, threads, 0, stream>>>(x, delta, delta_stride, weight, (bf16_t*)out, width, groups, eps);
-  else
-    group_norm_kernel<float><<<grid, threads, 0, stream>>>(x, delta, delta_stride, weight, (float*)out, width, groups, eps);
+#define GROUP(T)                                                                                                                  \
+  if (part <= 2 * NORM_HELD * threads)                                                                                            \
+    group_norm_kernel<T, NORM_HELD><<<grid, threads, 0, stream>>>(x, delta, delta_stride, weight, (T*)out, width, groups, eps);    \
+  else group_norm_kernel<T, 0><<<grid, threads, 0, stream>>>(x, delta, delta_stride, weight, (T*)out, width, groups, eps)
+  if (is_bf16) { GROUP(bf16_t); } else { GROUP(float); }
+#undef GROUP
   return dli_launch_status();
 }
 
@@ -1044,12 +1048,16 @@ int dli_branch_norm_mean(const float* const* y, const int64_t* strides, const fl
     if (y[s] == nullptr || weights[s] == nullptr || strides[s] < width) return DLI_ERR_ARGUMENT;
     b.y[j] = y[s]; b.stride[j] = strides[s]; b.weight[j] = weights[s];
   }
+#define BRANCH(COUNT)                                                                                \
+  if (width <= 256) branch_norm_mean_kernel<COUNT, 1><<<rows, 256, 0, stream>>>(b, out, width, eps); \
+  else branch_norm_mean_kernel<COUNT, NORM_HELD><<<rows, 256, 0, stream>>>(b, out, width, eps)
   switch (count) {
-    case 1: branch_norm_mean_kernel<1><<<rows, 256, 0, stream>>>(b, out, width, eps); break;
-    case 2: branch_norm_mean_kernel<2><<<rows, 256, 0, stream>>>(b, out, width, eps); break;
-    case 3: branch_norm_mean_kernel<3><<<rows, 256, 0, stream>>>(b, out, width, eps); break;
-    default: branch_norm_mean_kernel<4><<<rows, 256, 0, stream>>>(b, out, width, eps);
+    case 1: BRANCH(1); break;
+    case 2: BRANCH(2); break;
+    case 3: BRANCH(3); break;
+    default: BRANCH(4);
   }
+#undef BRANCH
   return dli_launch_status();
 }
 
@@ -1102,10 +1110,13 @@ int dli_rms_norm_pair(const float* x, const float* w1, const float* w2, void* ou
   if (rows <= 0) return DLI_OK;
   if (width <= 0) return DLI_ERR_ARGUMENT;
   const int threads = width >= 2048 ? 512 : 256;
-  if (is_bf16)
-    rms_norm_pair_kernel<bf16_t><<<rows, threads, 0, stream>>>(x, w1, w2, (bf16_t*)out1, (bf16_t*)out2, width, eps);
-  else
-    rms_norm_pair_kernel<float><<<rows, threads, 0, stream>>>(x, w1, w2, (float*)out1, (float*)out2, width, eps);
+#define PAIR(T)                                                                                                                          \
+  if (width <= threads) rms_norm_pair_kernel<T, 1><<<rows, threads, 0, stream>>>(x, w1, w2, (T*)out1, (T*)out2, width, eps);              \
+  else if (width <= 2 * NORM_HELD * threads)                                                                                             \
+    rms_norm_pair_kernel<T, NORM_HELD><<<rows, threads, 0, stream>>>(x, w1, w2, (T*)out1, (T*)out2, width, eps);                          \
+  else rms_norm_pair_kernel<T, 0><<<rows, threads, 0, stream>>>(x, w1, w2, (T*)out1, (T*)out2, width, eps)
+  if (is_bf16) { PAIR(bf16_t); } else { PAIR(float); }
+#undef PAIR
   return dli_launch_status();
 }
 

@@ -132,9 +132,10 @@ class RoutedExperts(FeedForward):
         shared = gate = None
         if self.shared_size:
             act = self.rt.empty(n, self.shared_size)
-            if few_rows_take(self.rt, x, self.ws_gate_up):
+            if few_rows_take(self.rt, x, self.ws_gate_up) and not (n > 8 and x.shape[1] >= 4096 and self.shared_size >= 2048):
                 # a few rows: the product that streams the weights, the activation inside (2 rows of 2,048 to twice 2,048: the
-                # library's product and the activation's kernel 11.5 + 4.7 us, this one 7.1)
+                # library's product and the activation's kernel 14.5 us, this one 7.8; 8 rows of 4,096 to twice 2,048 19.2 and 14.3,
+                # but 16 rows 18.8 and 20.9)
                 ops.skinny_gemm(x, self.ws_gate_up, epilogue=ops.SKINNY_SWIGLU, out=act,
                                 clamped=(self.shared_limit, self.alpha, self.up_shift))
             else:

@@ -46,3 +46,29 @@ def test_few_rows_have_the_many_rows_bits(ops, width, ff, weighted):
     want = torch.einsum("rf,rwf->rw", y, w_down.double()[pick])
     # a few of the intermediate's values round to bfloat16 the other way, by 2^-8 of up to about eight, times weights of ff^-0.5
     assert (many.double() - want).abs().max() < 2 ** -8 * 8 * 4 * ff ** -0.5 + 1e-5
+
+
+@pytest.mark.parametrize("rows,k,ff", [(1, 32, 8), (4, 96, 24), (5, 1024, 304), (16, 2048, 40), (8, 4096, 2048), (16, 4096, 2048), (17, 64, 24)])
+def test_shared_expert(rows, k, ff):
+    """A mixture whose shared expert is all there is: the streaming product with the activation inside, and the library's product with
+    the activation behind it (more than 16 rows, or many of wide weights), against 64-bit arithmetic."""
+    from dli_amd.parts import Runtime
+    from dli_amd.parts.experts import RoutedExperts
+
+    gen, rt = torch.Generator().manual_seed(rows + k), Runtime(torch.device("cuda"), torch.bfloat16)
+    part = RoutedExperts(rt, hidden_size=k, experts=0, top=1, expert_size=0, limit=7.0, identity=1, shared_size=ff, shared_limit=1.5,
+                         shared_gate=False, up_shift=0.5, correction=False)
+    draw = lambda *s: torch.randn(*s, generator=gen).mul_(s[-1] ** -0.5).bfloat16()
+    t = {"shared.gate": draw(ff, k), "shared.up": draw(ff, k), "shared.down": draw(k, ff), "router": draw(1, k)}
+    missing = set(part.weight_specs()) - set(t)
+    assert not missing, missing
+    part.load_weights({n: w.cuda() for n, w in t.items() if n in part.weight_specs()})
+    x = draw(rows, k).mul_(k ** 0.5 * 2)
+    got = part.forward(x.cuda(), None).float().cpu().double()
+    xd, d = x.double(), {n: w.double() for n, w in t.items()}
+    gate, up = xd @ d["shared.gate"].T, xd @ d["shared.up"].T
+    gate, up = gate.bfloat16().double().clamp(max=1.5), up.bfloat16().double().clamp(-1.5, 1.5)
+    want = (gate * torch.sigmoid(part.alpha * gate) * (up + 0.5)).bfloat16().double() @ d["shared.down"].T + xd
+    # gate, up and their product round to 2^-9 of up to three, some the other way (2^-8), summed with weights of ff^-0.5; the
+    # identity expert's row is the input, the sums stay 32-bit
+    assert (got - want).abs().max() < 2 ** -8 * 3 * 4

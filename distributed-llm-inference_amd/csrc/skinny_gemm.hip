@@ -14,7 +14,8 @@
 //   t[tile][block][q][g][c][8] = w[16*tile + c][128*block + 32*g + 8*q + (0..7)],
 // so that the 16 features x 128 k of one tile and block are 4 KB of consecutive memory in the
 // order in which the lanes take them (lane = 16*g + c) and every load of a wave is 1 KB of
-// consecutive bytes. Needs K % 128 == 0 and whole tiles (N % 16 == 0, gate and up parts included).
+// consecutive bytes. Needs K % 128 == 0 and whole tiles (N % 16 == 0, gate and up parts included); EPI_QKV behind a
+// norm also takes K % 32 == 0, the last block filled up with zeros.
 //
 // Fused in (template switches):
 //   NORM     xhat = cast(norm_w[k] * cast(x[m][k] * rs[m])), rs[m] = rsqrt(sum_k x^2 / K + eps),

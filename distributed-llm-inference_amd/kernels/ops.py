@@ -486,7 +486,8 @@ def tile_weights(w: torch.Tensor, whole_blocks: bool = True) -> torch.Tensor:
     kernel's lanes read it: ``t[tile][block][q][g][c][8] = w[16*tile + c][128*block + 32*g + 8*q + ...]``,
     so that each load of a wave is 1 KB of consecutive memory. Same number of elements, flat.
     ``whole_blocks=False`` takes any k % 8 == 0 and fills the last block of 128 with zeros (the copy
-    then has ``n * padded_k(k)`` elements; only :func:`mid_gemm` reads such a copy)."""
+    then has ``n * padded_k(k)`` elements; :func:`mid_gemm` reads such a copy, and :func:`skinny_gemm_qkv_rope` its own in the
+    same blocks)."""
     _dense(w, "w", torch.bfloat16, 2)
     n, k = w.shape
     if k % 128 != 0 and not whole_blocks:
@@ -545,10 +546,12 @@ def skinny_gemm_plan(rows: int, n: int, k: int, epilogue: int, device: torch.dev
             if not (tiled and (rows >= 2 or few)):
                 if few and k <= 1024:
                     # Short rows: eight k-waves share at most eight chunks of 128 k. The tile kernel finishes sooner where
-                    # it sums k in as few steps (us for one row, tiles and blocks in shapes 0 and 1, k 576: 576 features
-                    # with the residual 3.3, 4.1, 4.0, 960 stored 3.8, 4.2, 4.5; k 832: 4.5, 4.4, 4.8), else four waves
-                    # on four quads do, which leave no compute unit a second workgroup (gate and up of 1,536 features,
-                    # k 576: 5.5, 5.2, 7.0; k 320: 4.9, 5.2, 7.0).
+                    # it sums k in as few steps, else four waves on four quads do, which leave no compute unit a second
+                    # workgroup. Us of tiles, blocks in shape 0 and in shape 1, mean over 64 to 4,096 features and one to
+                    # four rows: stored or 32-bit, k 64 3.4, 4.4, 5.1; 576 4.6, 4.8, 5.5; 640 4.7, 4.8, 5.4; 704 4.8, 4.8,
+                    # 5.5; 1,024 5.7, 4.9, 5.5. Gated, k 64 4.4, 5.1, 6.0; 384 5.3, 5.4, 6.1; 448 5.4, 5.4, 6.2; 576 6.0,
+                    # 5.5, 6.2. With the residual, k 64 3.4, 3.9, 4.1; 576 4.5, 5.1, 5.0; 896 5.0, 5.2, 5.3; 1,024 4.7, 5.2,
+                    # 5.5. Of 960 products none was slower than blocks in shape 1, and none more than 2% behind the best.
                     if k <= {SKINNY_RESIDUAL: 1024, SKINNY_SWIGLU: 448}.get(epilogue, 640):
                         return "tiles16", 1, -(-n // 16)
                     blocks4 = 0
@@ -604,7 +607,7 @@ def skinny_gemm(x: torch.Tensor, w: torch.Tensor, *, epilogue: int, out: Optiona
         _dense(bias, "bias", torch.bfloat16, 1)
         _require(bias.shape[0] == w.shape[0], "bias length differs from rows of w")
     if k % 128 != 0:
-        w_tiled = None   # a copy in whole blocks with a zero-filled last one: the 17-to-64-row kernel's alone
+        w_tiled = None   # a copy in whole blocks with a zero-filled last one: this kernel does not read it
     if shape is not None:
         _require(shape in (0, 1, 2, 3, 4), "shape must be 0..4")
         kernel, a, n_parts = "tiles16", shape, -(-n // 16)

@@ -67,7 +67,7 @@ def decode_copy(rt: Runtime, weight: Optional[torch.Tensor], epilogue: int) -> O
     if not (ops.tiled_weights_help(weight.shape[0], weight.shape[1], epilogue, weight.device)
             or ops.mid_tiles_help(weight.shape[0], weight.shape[1], epilogue)):
         return None
-    # (rows that are no whole blocks of 128: zero-filled to whole blocks, for the 17-to-64-row kernel alone)
+    # (rows that are no whole blocks of 128: zero-filled to whole blocks, which the 17-to-64-row kernel reads)
     return ops.tile_weights(weight, whole_blocks=False)
 
 

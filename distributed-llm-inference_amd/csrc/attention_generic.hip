@@ -656,9 +656,11 @@ extern "C" int dli_attention_scored(const void* q, int64_t q_stride, const void*
 
 // How many workgroups share the keys of an (entry, group of query heads) in a step of single tokens: as
 // many as bring the launch to about two workgroups a compute unit, sixteen at most. It depends on the
-// heads and the number of entries (on the matrix cores, on the table's width too), never on their
-// lengths. A step of many entries fills the chip by itself and is not cut (cutting it costs more than it gains).
-// `most_keys`: the most keys that an entry can see here; `singles`: whether the matrix cores take the step's pages and sizes.
+// heads and the number of entries; on the matrix cores also on `most_keys`, the most that an entry can see here: what
+// a window or chunk leaves of the table's width, which is as wide as the step's longest request asks (in a
+// recorded step, as its shape's). There a request's sums may run in another order when a longer one shares
+// its step. A step of many entries fills the chip by itself and is not cut (cutting it costs more than it gains).
+// `singles`: whether the matrix cores take the step's pages and sizes.
 extern "C" int dli_attention_scored_splits(int q_heads, int kv_heads, int entries, int64_t most_keys, int singles) {
   if (q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads != 0 || entries <= 0) return 1;
   if (singles) return attention_singles_splits(q_heads, kv_heads, entries, most_keys);

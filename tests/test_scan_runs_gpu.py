@@ -192,10 +192,12 @@ def test_scratch_follows_the_portions(ops):
 
 
 @pytest.mark.parametrize("rule", ["delta", "bonus", "gated"])
-@pytest.mark.parametrize("lens,singles", [([1, 1, 1, 200, 2, 70, 129], 3), ([1] * 70 + [5, 300], 70), ([3] * 40 + [150], 0), ([1, 128], 1)])
+@pytest.mark.parametrize("lens,singles", [([1, 1, 1, 200, 2, 70, 129], 3), ([1] * 70 + [5, 300], 70), ([3] * 40 + [150], 0), ([1, 128], 1),
+                                          ([3, 0, 5] * 45 + [300, 2] + [4] * 20, 0), ([1] * 3 + [2] * 63 + [200], 3)])
 def test_single_tokens_beside_portions(ops, rule, lens, singles):
-    """The leading single tokens have the bits that a step of single tokens gives them, the portions those of a step without them;
-    nobody else's state is written. (Entries of many lengths: slots of the launch that hold no run.)"""
+    """The leading single tokens have the bits that a step of single tokens gives them, the portions those of a step without them,
+    near those of token by token; nobody else's state is written. (Entries of many lengths, none among them, and more than a wave
+    looks up at once: slots of the launch that hold no run.)"""
     H, n, E = 2, sum(lens), len(lens)
     c, gen = H * D, torch.Generator(device="cuda").manual_seed(n)
     rnd = lambda *shape: torch.randn(*shape, device="cuda", generator=gen)
@@ -219,6 +221,9 @@ def test_single_tokens_beside_portions(ops, rule, lens, singles):
         return out, state
 
     out, state = run(0, E, max(lens), singles)
+    by_token, token_state = run(0, E, 0, 0)
+    # (an output is divided by its root mean square: a head whose outputs are small there carries the roundings on)
+    assert (out - by_token).abs().max() < 2e-4 * by_token.abs().max() and (state - token_state).abs().max() < 2e-5 * token_state.abs().max()
     portions, portion_state = run(singles, E, max(lens), 0)
     assert torch.equal(out[starts[singles]:], portions)
     assert torch.equal(state[:E - singles], portion_state[:E - singles]) and torch.equal(state[E:], state0[E:])

@@ -9,7 +9,7 @@ stream; nothing here computes with torch.
 from __future__ import annotations
 
 import ctypes
-from typing import Optional, Sequence
+from typing import Callable, Optional, Sequence
 
 import torch
 
@@ -1966,14 +1966,20 @@ def _whole(*tensors: torch.Tensor) -> bool:
     return all(t.data_ptr() % 16 == 0 and (t.dim() < 2 or t.stride(0) % 4 == 0) for t in tensors)
 
 
+NO_CUT = (0, 0, 0, None, None, None)
+
+
 def _cut(device: torch.device, entries: int, rows: int, heads: int, longest: int, singles: int, unit_columns: bool,
-         gated: bool = False) -> tuple:
+         gated: bool = False, takes: Callable[[], bool] = lambda: True) -> tuple:
     """What the scans' entry points are told about runs: single-row entries that lead, rows a run, runs of the longest entry, and
-    the scratch: the walk's outputs for the unit columns, and per run and head the end state and what moves the one before."""
+    the scratch: the walk's outputs for the unit columns, and per run and head the end state and what moves the one before.
+    ``takes``: whether the rows can be cut at all, asked last (short steps wait for the host)."""
     portions, rows = entries - singles, rows - singles
-    run_rows, runs = scan_runs(portions, rows, heads, longest, unit_columns, gated) if portions > 0 else (0, 0)
-    if not run_rows:
-        return 0, 0, 0, None, None, None
+    if longest < RUNS_FROM_ROWS or portions <= 0:
+        return NO_CUT
+    run_rows, runs = scan_runs(portions, rows, heads, longest, unit_columns, gated)
+    if not run_rows or not takes():
+        return NO_CUT
     slots = rows // run_rows + portions
     return (singles, run_rows, runs, torch.empty(rows, heads * 64, device=device, dtype=torch.float32),
             torch.empty(slots, heads, 64, 64, device=device, dtype=torch.float32),
@@ -2018,9 +2024,9 @@ def recurrent_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, w: torch.T
         _require(bonus.numel() == width, "bonus must hold heads*dim values")
     sa = a_pre.stride(0) if a_pre is not None else 0
     o_raw = torch.empty(n, width, device=out.device, dtype=torch.float32)  # the recurrence's output before norm and gate
-    takes = (dim == 64 and _whole(r, k, v, w, g_pre, norm_w, state, *(t for t in (a, bonus) if t is not None))
-             and out.stride(0) % 4 == 0 and out.data_ptr() % (4 * out.element_size()) == 0)
-    cut = _cut(out.device, entries, n, heads, longest if takes else 0, singles, rule == RULE_DELTA)
+    cut = _cut(out.device, entries, n, heads, longest if dim == 64 else 0, singles, rule == RULE_DELTA, takes=lambda: (
+        _whole(r, k, v, w, g_pre, norm_w, state, *(t for t in (a, bonus) if t is not None))
+        and out.stride(0) % 4 == 0 and out.data_ptr() % (4 * out.element_size()) == 0))
     _check(library().dli_recurrent_scan(
         _ptr(r), r.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(w_pre), w_pre.stride(0), _ptr(a_pre), sa,
         _ptr(a_bias), _ptr(g_pre), g_pre.stride(0), _ptr(bonus), _ptr(norm_w), float(eps), _ptr(state), state.stride(0),
@@ -2190,8 +2196,8 @@ def gated_delta_scan(prep: torch.Tensor, state: torch.Tensor, q_start: torch.Ten
         _dense(t, name, torch.int32, 1)
     entries = state_slots.shape[0]
     _require(q_start.shape[0] == entries + 1 and positions.shape[0] == n, "q_start/state_slots/positions disagree")
-    takes = dim == vdim == 64 and _whole(prep, state, o)
-    cut = _cut(o.device, entries, n, heads, longest if takes else 0, singles, True, gated=True)
+    cut = _cut(o.device, entries, n, heads, longest if dim == vdim == 64 else 0, singles, True, gated=True,
+               takes=lambda: _whole(prep, state, o))
     _check(library().dli_gated_delta_scan(
         _ptr(prep), prep.stride(0), _ptr(state), state.stride(0), _ptr(q_start), _ptr(positions), _ptr(state_slots),
         _ptr(o), o.stride(0), entries, n, heads, kv_heads, dim, vdim, *cut[:3], *map(_ptr, cut[3:]), _stream()),

@@ -140,7 +140,7 @@ __global__ __launch_bounds__(256) void attention_singles_kernel(SinglesArgs a) {
         l += p;
       }
 #pragma unroll
-      for (int k = 0; k < 3; ++k)
+      for (int k = 2; k >= 0; --k)   // the smallest first
 #pragma unroll
         for (int c = 0; c < VCH; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(t.v[u][c], part[k], acc[c], 0, 0, 0);
     }

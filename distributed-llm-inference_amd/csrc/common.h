@@ -62,6 +62,29 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// Exchanges between lanes without a trip through LDS (all lanes of the wave take part).
+template <int SHIFT>
+__device__ __forceinline__ float row_ror(float v) {  // rotated by SHIFT within each row of sixteen lanes
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + SHIFT, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float quad_sum(float v) {  // over the lanes l, l^1, l^2, l^3
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xb1, 0xf, 0xf, true));
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4e, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float quad_pairs(float v) {  // over the lanes l, l^2
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4e, 0xf, 0xf, true));
+}
+// a[l] + a[l^32] in the lower half of the lanes, b[l] + b[l^32] in the upper
+__device__ __forceinline__ float add_halves(float a, float b) {
+  const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+// a[l] + a[l^16] in the rows of sixteen lanes 0 and 2, b[l] + b[l^16] in the rows 1 and 3
+__device__ __forceinline__ float add_rows(float a, float b) {
+  const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+
 // Sum over a block of up to 1024 threads; every thread gets the result. `scratch` holds 16 floats.
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
   const int lane = threadIdx.x % DLI_WAVE, wave = threadIdx.x / DLI_WAVE;

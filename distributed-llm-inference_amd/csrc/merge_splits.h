@@ -57,51 +57,65 @@ __device__ __forceinline__ void device_store2(__amdgpu_buffer_rsrc_t r, unsigned
 }
 
 // part_o [.. slots][head_dim], part_ml [.. slots][2]; `base`: the first of the S slots of this
-// (request, head); d: the first of the four dims. All loads are asked for before the first is used.
+// (request, head); d: the first of the four dims. All loads are asked for before the first is used
+// (`ask`), so that the caller may ask for other things before it has them added up (`merged`).
 // SAME_LAUNCH: the partial results were stored by other workgroups of this launch (each array
 // under 4 GB).
 template <bool SAME_LAUNCH = false>
-__device__ __forceinline__ merge_float4 merged_quad(const float* part_o, const float* part_ml, int64_t base, int S,
-                                                    int head_dim, int d) {
+struct MergeQuad {
   merge_float2 ml[MERGE_SPLITS];
   merge_float4 po[MERGE_SPLITS];
+
+  __device__ __forceinline__ void ask(const float* part_o, const float* part_ml, int64_t base, int S, int head_dim, int d) {
 #pragma unroll
-  for (int j = 0; j < MERGE_SPLITS; ++j) {
-    ml[j] = merge_float2{-INFINITY, 0.f};
-    po[j] = merge_float4{0.f, 0.f, 0.f, 0.f};
-    if (j < S) {
-      const float* ml_at = part_ml + (base + j) * 2;
-      const float* po_at = part_o + (base + j) * head_dim + d;
-      if constexpr (SAME_LAUNCH) {
-        ml[j] = device_load2(device_scope_buffer(part_ml), (unsigned)((base + j) * 2 * 4));
-        po[j] = device_load4(device_scope_buffer(part_o), (unsigned)(((base + j) * head_dim + d) * 4));
-      } else {
-        ml[j] = *reinterpret_cast<const merge_float2*>(ml_at);
-        po[j] = *reinterpret_cast<const merge_float4*>(po_at);
+    for (int j = 0; j < MERGE_SPLITS; ++j) {
+      ml[j] = merge_float2{-INFINITY, 0.f};
+      po[j] = merge_float4{0.f, 0.f, 0.f, 0.f};
+      if (j < S) {
+        const float* ml_at = part_ml + (base + j) * 2;
+        const float* po_at = part_o + (base + j) * head_dim + d;
+        if constexpr (SAME_LAUNCH) {
+          ml[j] = device_load2(device_scope_buffer(part_ml), (unsigned)((base + j) * 2 * 4));
+          po[j] = device_load4(device_scope_buffer(part_o), (unsigned)(((base + j) * head_dim + d) * 4));
+        } else {
+          ml[j] = *reinterpret_cast<const merge_float2*>(ml_at);
+          po[j] = *reinterpret_cast<const merge_float4*>(po_at);
+        }
       }
     }
   }
-  float m_all = -INFINITY;
+
+  __device__ __forceinline__ merge_float4 merged(int S) const {
+    float m_all = -INFINITY;
 #pragma unroll
-  for (int j = 0; j < MERGE_SPLITS; ++j) m_all = fmaxf(m_all, ml[j][0]);
-  const float m_safe = m_all == -INFINITY ? 0.f : m_all;
-  float wgt[MERGE_SPLITS], t[MERGE_SPLITS];
+    for (int j = 0; j < MERGE_SPLITS; ++j) m_all = fmaxf(m_all, ml[j][0]);
+    const float m_safe = m_all == -INFINITY ? 0.f : m_all;
+    float wgt[MERGE_SPLITS], t[MERGE_SPLITS];
 #pragma unroll
-  for (int j = 0; j < MERGE_SPLITS; ++j) {
-    wgt[j] = j < S ? __builtin_amdgcn_exp2f(ml[j][0] - m_safe) : 0.f;
-    t[j] = __fmul_rn(ml[j][1], wgt[j]);
+    for (int j = 0; j < MERGE_SPLITS; ++j) {
+      wgt[j] = j < S ? __builtin_amdgcn_exp2f(ml[j][0] - m_safe) : 0.f;
+      t[j] = __fmul_rn(ml[j][1], wgt[j]);
+    }
+#pragma unroll
+    for (int h = MERGE_SPLITS / 2; h > 0; h >>= 1)
+#pragma unroll
+      for (int j = 0; j < h; ++j) t[j] = __fadd_rn(t[j], t[j + h]);
+    const float inv = t[0] > 0.f ? 1.f / t[0] : 0.f;
+    merge_float4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < MERGE_SPLITS; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] = __fmaf_rn(po[j][i], wgt[j], acc[i]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = __fmul_rn(acc[i], inv);
+    return acc;
   }
-#pragma unroll
-  for (int h = MERGE_SPLITS / 2; h > 0; h >>= 1)
-#pragma unroll
-    for (int j = 0; j < h; ++j) t[j] = __fadd_rn(t[j], t[j + h]);
-  const float inv = t[0] > 0.f ? 1.f / t[0] : 0.f;
-  merge_float4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int j = 0; j < MERGE_SPLITS; ++j)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = __fmaf_rn(po[j][i], wgt[j], acc[i]);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) acc[i] = __fmul_rn(acc[i], inv);
-  return acc;
+};
+
+template <bool SAME_LAUNCH = false>
+__device__ __forceinline__ merge_float4 merged_quad(const float* part_o, const float* part_ml, int64_t base, int S,
+                                                    int head_dim, int d) {
+  MergeQuad<SAME_LAUNCH> parts;
+  parts.ask(part_o, part_ml, base, S, head_dim, d);
+  return parts.merged(S);
 }

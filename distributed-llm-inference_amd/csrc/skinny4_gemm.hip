@@ -10,8 +10,13 @@
 // features (a "quad") and columns four activation rows: lane l loads the 16 bytes at k = chunk*128
 // + 8*(l/4) of its feature's weight row, so that sixteen neighbouring lanes read four rows times 64
 // contiguous bytes, and does two products (k halves) per quad and group of four activation rows.
-// The blocks' partial sums are added at the end: lanes l, l^16, l^32, l^48 by lane swaps, the rest
-// and the waves' shares of k through LDS, always in the same order.
+// The blocks' partial sums are added at the end, in registers (add_blocks: two lane swaps and two
+// rotations for four sums at a time), the waves' shares of k through LDS, always in the same order.
+// What follows the last product is a chain that nothing hides, so it is kept short: one LDS value
+// per wave and output, all read before the first is added, one output a thread. (With four values a
+// lane by way of LDS and up to 64 reads of a few threads one after the other, the chain took 1.0 to
+// 1.2 us of a kernel of 3.5 to 12, now 0.3: gate and up at the 135M sizes 3.5 -> 2.6 us from start to
+// end, down at the 1B sizes 7.9 -> 6.4, one row)
 //
 // A workgroup has KS waves that split k among themselves and owns FQ quads of features. Few
 // quads and many waves suit products with few features (every compute unit still gets a
@@ -50,6 +55,22 @@ __device__ __forceinline__ float4v mfma4(short4v a, short4v b, float4v c) {
   return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(a, b, c, 0, 0, 0);
 }
 
+// Sums over the sixteen blocks (the lanes that share l % 4), all in registers. add_blocks(float4v)
+// takes four sums at once: a swap of lane halves leaves one register with two of them, a swap of
+// neighbouring rows one with all four (row j of sixteen lanes: element 0, 2, 1, 3), then the row's
+// four blocks by rotations.
+__device__ __forceinline__ float add_blocks(float4v v) {
+  float s = add_rows(add_halves(v[0], v[1]), add_halves(v[2], v[3]));
+  s += row_ror<8>(s);
+  return s + row_ror<4>(s);
+}
+__device__ __forceinline__ float add_blocks(float v) {  // one sum, the same in all blocks
+  float s = add_halves(v, v);
+  s = add_rows(s, s);
+  s += row_ror<8>(s);
+  return s + row_ror<4>(s);
+}
+
 template <int KS, int FQ, int MG, int EPI, bool NORM, bool XL, int DEPTH>
 __global__ __launch_bounds__(KS * 64) void skinny4_kernel(
     const bf16_t* __restrict__ x, int64_t ldx, const float* __restrict__ ssq_in, int ssq_parts,
@@ -59,8 +80,9 @@ __global__ __launch_bounds__(KS * 64) void skinny4_kernel(
     int up_offset, GluForm glu) {
   constexpr int PAIRS = FQ * MG;                        // (quad, row group) accumulators per lane
   constexpr int OQ = EPI == EPI_SWIGLU ? FQ / 2 : FQ;   // quads of output features per tile
-  __shared__ float4v red[KS][PAIRS][16];
-  __shared__ float4v fin[PAIRS][4];
+  constexpr int OUTS = OQ * MG * 16;                    // outputs of the tile, at most one a thread
+  static_assert(OUTS <= KS * 64, "one output a thread");
+  __shared__ float red[KS][PAIRS * 16];                 // [pair][row][feature of the quad]
   __shared__ float sqs[OQ][MG][4];
   extern __shared__ __attribute__((aligned(16))) bf16_t xs[];  // XL: xhat, rows of XPAD(K) values
 
@@ -69,26 +91,27 @@ __global__ __launch_bounds__(KS * 64) void skinny4_kernel(
   const int tile = blockIdx.x;
   const int n_tile = tile * 4 * OQ;  // first output feature of the tile
 
-  // EPI_RESIDUAL: the stream values that this thread will add to at the end are asked for now, so
-  // that the epilogue does not wait for a trip to memory of its own (same thread, same places)
-  union Pack4 {
-    short4v v;
-    bf16_t e[4];
-  } old;
-  old.v = short4v{0, 0, 0, 0};
-  if (EPI == EPI_RESIDUAL) {
-    const int t0 = threadIdx.x, p0 = t0 / 4, f0 = p0 / MG;
-    const int m0 = 4 * (p0 % MG) + t0 % 4, nb0 = n_tile + 4 * f0;
-    if (t0 < 4 * PAIRS && f0 < OQ && m0 < M && nb0 < N) {
-      const bf16_t* sp = stream + (int64_t)m0 * lds_ + nb0;
-      if (nb0 + 3 < N && lds_ % 4 == 0) {
-        old.v = *reinterpret_cast<const short4v*>(sp);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) old.e[i] = nb0 + i < N ? sp[i] : (bf16_t)0.f;
-      }
-    }
-  }
+  // Thread t < OUTS ends with one output: pair t / 16 (quad f = pair / MG, row group pair % MG), row
+  // t / 4 % 4 of the group, feature t % 4 of the quad. What it will add to the sum (bias, the
+  // stream's value) is asked for now, so that the end does not wait for a trip to memory of its own;
+  // no load hangs on a condition (a place outside reads the nearest inside, a missing bias a
+  // resource without bytes: zeros).
+  const int out_pair = min((int)threadIdx.x, OUTS - 1) / 16;
+  const int out_f = out_pair / MG, out_g = out_pair % MG;
+  const int out_m = 4 * out_g + threadIdx.x / 4 % 4;
+  const int out_n = n_tile + 4 * out_f + threadIdx.x % 4;
+  const bool owner = (int)threadIdx.x < OUTS && out_m < M && out_n < N;
+  union Half {
+    unsigned short raw;
+    bf16_t v;
+  } old, b0, b1;
+  old.raw = 0;
+  if (EPI == EPI_RESIDUAL) old.v = stream[(int64_t)min(out_m, M - 1) * lds_ + min(out_n, N - 1)];
+  const __amdgpu_buffer_rsrc_t bres = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)bias, 0, bias != nullptr ? (unsigned)(N + (EPI == EPI_SWIGLU ? up_offset : 0)) * 2u : 0u, 0x00020000);
+  b0.raw = __builtin_amdgcn_raw_buffer_load_b16(bres, min(out_n, N - 1) * 2, 0, 0);
+  b1.raw = 0;
+  if (EPI == EPI_SWIGLU) b1.raw = __builtin_amdgcn_raw_buffer_load_b16(bres, (min(out_n, N - 1) + up_offset) * 2, 0, 0);
 
   // weight rows of this lane, one per quad (clamped at the matrix's end: computed and dropped)
   const bf16_t* wrow[FQ];
@@ -190,12 +213,20 @@ __global__ __launch_bounds__(KS * 64) void skinny4_kernel(
   }
   fetch_first();
   __builtin_amdgcn_sched_barrier(0);
+  __shared__ float rsum[NORM ? KS : 1][MG][4];
+  auto row_scale = [&](int m) __attribute__((always_inline)) {  // from the waves' sums, in wave order
+    float part[KS], sum = 0.f;
+#pragma unroll
+    for (int wv = 0; wv < KS; ++wv) part[wv] = rsum[wv][m / 4][m % 4];
+#pragma unroll
+    for (int wv = 0; wv < KS; ++wv) sum += part[wv];
+    return rsqrtf(sum / (float)K + eps);
+  };
   if constexpr (NORM) {
     // rs[m] from the parts of sum x^2. The parts are dealt out to all blocks of all waves (block
     // q of 16*KS takes the parts q, q + 16*KS, ...), eight loads at a time so that they share one
     // trip to memory; a wave adds its blocks, the waves' sums meet in LDS and are added in wave
     // order.
-    __shared__ float rsum[KS][MG][4];
 #pragma unroll
     for (int g = 0; g < MG; ++g) {
       const int m = min(4 * g + r, M - 1);
@@ -212,37 +243,21 @@ __global__ __launch_bounds__(KS * 64) void skinny4_kernel(
 #pragma unroll
         for (int u = 0; u < 8; ++u) sum += v[u];
       }
-      sum += __shfl_xor(sum, 4, 64);
-      sum += __shfl_xor(sum, 8, 64);
-      sum += __shfl_xor(sum, 16, 64);
-      sum += __shfl_xor(sum, 32, 64);
+      sum = add_blocks(sum);
       if (blk == 0) rsum[ks][g][r] = sum;
     }
     __syncthreads();
 #pragma unroll
-    for (int g = 0; g < MG; ++g) {
-      float sum = 0.f;
-#pragma unroll
-      for (int wv = 0; wv < KS; ++wv) sum += rsum[wv][g][r];
-      rs[g] = rsqrtf(sum / (float)K + eps);
-    }
+    for (int g = 0; g < MG; ++g) rs[g] = row_scale(4 * g + r);
   }
 
   if constexpr (XL) {
     // thread t stages the 8 values at k = 8*(t % (chunks*16)) of row t / (chunks*16), and so on
-    __shared__ float rs_row[4 * MG];
-    if constexpr (NORM) {
-      if (ks == 0 && blk == 0) {
-#pragma unroll
-        for (int g = 0; g < MG; ++g) rs_row[4 * g + r] = rs[g];
-      }
-      __syncthreads();
-    }
     auto stage = [&](int idx, Frag16 v, float4v g0, float4v g1) __attribute__((always_inline)) {
       const int m = idx / per_row, k = (idx - m * per_row) * 8;
       if (k < K) {
         if constexpr (NORM) {
-          const float rsm = rs_row[m];
+          const float rsm = row_scale(m);
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
             const float normed = (float)(bf16_t)((float)v.e[i] * rsm);
@@ -307,100 +322,53 @@ __global__ __launch_bounds__(KS * 64) void skinny4_kernel(
       if (c + d < c1) multiply(st[d], c + d);  // the last group (what was loaded past the end is not waited for)
   }
 
-  // blocks l/4 that differ in their upper two bits are added by lane swaps, the remaining four
-  // blocks and the waves through LDS
+  // the sixteen blocks' sums: row j of sixteen lanes is left with feature FEATURE[j] of the quad
 #pragma unroll
   for (int f = 0; f < FQ; ++f)
 #pragma unroll
-    for (int g = 0; g < MG; ++g)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float v = acc[f][g][i];
-        v += __shfl_xor(v, 32, 64);
-        v += __shfl_xor(v, 16, 64);
-        acc[f][g][i] = v;
-      }
-  if (lane < 16) {
-#pragma unroll
-    for (int f = 0; f < FQ; ++f)
-#pragma unroll
-      for (int g = 0; g < MG; ++g) red[ks][f * MG + g][lane] = acc[f][g];
-  }
+    for (int g = 0; g < MG; ++g) {
+      const float v = add_blocks(acc[f][g]);
+      const int feature = (lane / 32) | (lane / 16 % 2) * 2;
+      if (blk % 4 == 0) red[ks][(f * MG + g) * 16 + r * 4 + feature] = v;
+    }
   __syncthreads();
-  // thread t < 4*PAIRS owns the four features of quad f = p / MG for activation row m = 4g + rr
   const int t = threadIdx.x;
-  const bool owner = t < 4 * PAIRS;
-  const int p = t / 4, rr = t % 4;
-  float4v total = {0.f, 0.f, 0.f, 0.f};
-  if (owner) {
+  float part[KS], up_part[KS], y = 0.f, y_up = 0.f;
+  const int at = min(t, OUTS - 1);
 #pragma unroll
-    for (int k = 0; k < KS; ++k)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) total += red[k][p][4 * b + rr];
+  for (int k = 0; k < KS; ++k) {
+    part[k] = red[k][at];
+    if (EPI == EPI_SWIGLU) up_part[k] = red[k][at + OUTS];
   }
-  if (EPI == EPI_SWIGLU) {
-    if (owner) fin[p][rr] = total;
-    __syncthreads();
+#pragma unroll
+  for (int k = 0; k < KS; ++k) {
+    y += part[k];
+    if (EPI == EPI_SWIGLU) y_up += up_part[k];
   }
-  const int f = p / MG, g = p % MG;
-  const int m = 4 * g + rr;
-  const int nb = n_tile + 4 * f;
-  float sq = 0.f;
-  if (owner && f < OQ && m < M && nb < N) {
-    const bool whole = nb + 3 < N;
-    float y[2][4];
-#pragma unroll
-    for (int a = 0; a < (EPI == EPI_SWIGLU ? 2 : 1); ++a) {
-      const float4v src = EPI == EPI_SWIGLU ? fin[(f + a * OQ) * MG + g][rr] : total;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        y[a][i] = src[i] + (bias != nullptr && nb + i < N ? (float)bias[nb + i + a * up_offset] : 0.f);
-    }
-    if (EPI == EPI_F32) {
-      float* op = reinterpret_cast<float*>(out) + (int64_t)m * ldo + nb;
-      if (whole && ldo % 4 == 0) {
-        *reinterpret_cast<float4v*>(op) = float4v{y[0][0], y[0][1], y[0][2], y[0][3]};
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (nb + i < N) op[i] = y[0][i];
-      }
-    } else {
-      bf16_t* op = EPI == EPI_RESIDUAL ? stream + (int64_t)m * lds_ + nb
-                                       : reinterpret_cast<bf16_t*>(out) + (int64_t)m * ldo + nb;
-      const bool vec = whole && (EPI == EPI_RESIDUAL ? lds_ : ldo) % 4 == 0;
-      Pack4 res;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (EPI == EPI_STORE) {
-          res.e[i] = (bf16_t)y[0][i];
-        } else if (EPI == EPI_SWIGLU) {
-          const float gt = (float)(bf16_t)y[0][i], up = (float)(bf16_t)y[1][i];
-          res.e[i] = glu_bf16(gt, up, glu);
-        } else {  // EPI_RESIDUAL: the sum in 32-bit, rounded to the stream's type
-          res.e[i] = (bf16_t)((float)old.e[i] + (float)(bf16_t)y[0][i]);
-          if (nb + i < N) sq += (float)res.e[i] * (float)res.e[i];
-        }
-      }
-      if (vec) {
-        *reinterpret_cast<short4v*>(op) = res.v;
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (nb + i < N) op[i] = res.e[i];
-      }
-    }
+  if (bias != nullptr) {
+    y += (float)b0.v;
+    if (EPI == EPI_SWIGLU) y_up += (float)b1.v;
   }
   if (EPI == EPI_RESIDUAL) {
-    // the tile's part of the row's sum of squares: the quads' shares, added in quad order
-    if (owner) sqs[f][g][rr] = sq;
+    // the sum in 32-bit, rounded to the stream's type
+    const bf16_t res = (bf16_t)((float)old.v + (float)(bf16_t)y);
+    float sq = owner ? (float)res * (float)res : 0.f;
+    if (owner) stream[(int64_t)out_m * lds_ + out_n] = res;
+    // the tile's part of the row's sum of squares: a quad's features by lane exchanges, the quads in order
+    sq = quad_sum(sq);
+    if (t < OUTS && t % 4 == 0) sqs[out_f][out_g][t / 4 % 4] = sq;
     __syncthreads();
-    if (owner && f == 0 && m < M) {
+    if (t < 4 * MG && t < M) {
       float s = 0.f;
 #pragma unroll
-      for (int q = 0; q < OQ; ++q) s += sqs[q][g][rr];
-      ssq_out[(int64_t)tile * M + m] = s;
+      for (int q = 0; q < OQ; ++q) s += sqs[q][t / 4][t % 4];
+      ssq_out[(int64_t)tile * M + t] = s;
     }
+  } else if (owner) {
+    const int64_t place = (int64_t)out_m * ldo + out_n;
+    if (EPI == EPI_F32) reinterpret_cast<float*>(out)[place] = y;
+    else if (EPI == EPI_STORE) reinterpret_cast<bf16_t*>(out)[place] = (bf16_t)y;
+    else reinterpret_cast<bf16_t*>(out)[place] = glu_bf16((float)(bf16_t)y, (float)(bf16_t)y_up, glu);
   }
 }
 

@@ -126,11 +126,17 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
     int up_offset, QkvRope qr, MergedIn mi, GluForm glu) {
   static_assert(EPI != EPI_QKV || (TILED && MT == 1), "the q/k/v epilogue reads tiled weights, at most 16 rows");
   static_assert(!MERGED || (TILED && MT == 1 && NS == 1 && !NORM), "merged activations: tiled weights, one row tile");
+  static_assert(KS * NS * 64 >= 256, "a thread for each output of a tile");
   // MERGED: each wave's run of k for up to MERGE_ROWS rows
   __shared__ __align__(16) bf16_t xs[MERGED ? KS : 1][MERGED ? MERGE_ROWS : 1][MERGED ? MERGE_RANGE : 8];
   constexpr int NA = EPI == EPI_SWIGLU ? 2 : 1;  // weight row sets per tile (gate and up)
-  constexpr int KR = KS > 1 ? KS - 1 : 1;
-  __shared__ float red[KR][NS][NT][NA][MT][4][64];  // k-split waves 1.. hand their tiles to wave 0
+  // What follows the last product is a chain that nothing hides, so it is kept short. With one row
+  // tile and one group of waves (SHORT) all waves leave their parts in LDS and thread t makes
+  // output t of each tile: element t % 4 of lane t / 4 of the product's result, that is row
+  // t / 4 % 16 and feature 4 (t / 64) + t % 4. Otherwise k-split waves 1.. hand their parts to wave 0.
+  constexpr bool SHORT = MT == 1 && NS == 1;
+  constexpr int KR = SHORT ? KS : (KS > 1 ? KS - 1 : 1);
+  __shared__ float4v red[KR][NS][NT][NA][MT][64];
 
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
   const int ks = wave % KS, ns = wave / KS;
@@ -157,24 +163,68 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
     return reinterpret_cast<const bf16x8*>(TILED ? base + (s / 4) * 2048 + q * 512 : base + s * 32 + q * 8);
   };
 
-  // EPI_RESIDUAL: the stream values that this lane will add to at the end (lane holds
-  // y[m = 16t + col][n = 16*tile + 4*grp + i]) are asked for now, so that the epilogue does not
-  // wait for a trip to memory of its own
-  bf16_t old_s[EPI == EPI_RESIDUAL ? NT : 1][EPI == EPI_RESIDUAL ? MT : 1][4];
+  // What the end adds to the product (the stream's values, the bias, and for q/k/v the rows' slots,
+  // cosines and sines) is asked for now, so that the end does not wait for a trip to memory of its
+  // own. In every wave and for every element (an element past the edge reads the edge's and is not
+  // stored; a missing bias is a resource without bytes, which reads zeros): a load under a
+  // condition is waited for on the spot, one trip to memory after the other, and leaves the count
+  // of loads on their way unknown to everything behind it.
+  constexpr int EL = SHORT ? 1 : 4;  // a thread's (SHORT) or lane's elements of a tile
+  const int e_row = SHORT ? threadIdx.x / 4 % 16 : col;
+  const int e_grp = SHORT ? threadIdx.x / 64 % 4 : grp, e_i = SHORT ? threadIdx.x % 4 : 0;
+  const int e_n = 4 * e_grp + e_i;   // first of them within the tile
+  bf16_t old_s[EPI == EPI_RESIDUAL ? NT : 1][EPI == EPI_RESIDUAL ? MT : 1][EL];
   if constexpr (EPI == EPI_RESIDUAL) {
-    // In every wave and for every element (only the first k-split wave uses them; an element past
-    // the edge reads the edge's and is not stored): a load under a condition is waited for on
-    // the spot, one trip to memory after the other, and leaves the count of loads on their way
-    // unknown to everything behind it.
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int t = 0; t < MT; ++t)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int n = (tile0 + j) * 16 + 4 * grp + i, m = t * 16 + col;
+        for (int i = 0; i < EL; ++i) {
+          const int n = (tile0 + j) * 16 + e_n + i, m = t * 16 + e_row;
           old_s[j][t][i] = stream[(int64_t)min(m, M - 1) * lds_ + min(n, N - 1)];
         }
+  }
+  const __amdgpu_buffer_rsrc_t bres = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)bias, 0, bias != nullptr ? (unsigned)(N + (NA - 1) * up_offset) * 2u : 0u, 0x00020000);
+  auto bias_at = [&](int n) __attribute__((always_inline)) {
+    union {
+      unsigned short raw;
+      bf16_t v;
+    } b;
+    b.raw = __builtin_amdgcn_raw_buffer_load_b16(bres, n * 2, 0, 0);
+    return b.v;
+  };
+  // (SHORT q/k/v: a thread adds up its element's rotary partner too, eight features on)
+  constexpr int BA = SHORT && EPI == EPI_QKV ? 2 : NA;
+  bf16_t b_at[NT][BA][EL];
+  auto load_bias = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int a = 0; a < BA; ++a)
+#pragma unroll
+        for (int i = 0; i < EL; ++i) {
+          const int n = (tile0 + j) * 16 + (BA > NA && a == 1 ? (e_n ^ 8) + i : e_n + i);
+          b_at[j][a][i] = bias_at(min(n, N - 1) + (BA > NA ? 0 : a * up_offset));
+        }
+  };
+  if constexpr (MT == 1) load_bias();  // (several row tiles: at the end, the registers are taken)
+  int slot_at = -1;
+  float cs_at[EPI == EPI_QKV ? NT : 1][EL], sn_at[EPI == EPI_QKV ? NT : 1][EL];
+  if constexpr (EPI == EPI_QKV) {
+    const int half = qr.head_dim / 2, mm = min(e_row, M - 1);
+    slot_at = qr.slots[mm];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int t_in = min(tile0 + j, (N - 1) / 16) % (qr.head_dim / 16);
+      const float* at = qr.angles + (int64_t)mm * 2 * half + 8 * t_in + 4 * (e_grp & 1) + e_i;  // the rotary pairs
+#pragma unroll
+      for (int i = 0; i < EL; ++i) {
+        cs_at[j][i] = at[i];
+        sn_at[j][i] = at[half + i];
+      }
+    }
   }
 
   const bf16_t* xrow[MT];
@@ -242,6 +292,13 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
   };
   int blocks = (s_end - s) / 4;
   Block b0, b1;
+  // The second block sets out with the first: what is waited for before the first product (the
+  // sums of squares, the merge) then hides both trips. (A wave of one block reads that again.)
+  auto fetch_second = [&]() __attribute__((always_inline)) {
+    const int at = blocks > 1 ? s + 4 : (blocks > 0 ? s : 0);
+    fetch_rows(b1, at);
+    fetch_weights(b1, at);
+  };
   if constexpr (NORM) {
     // rs[m] from the parts of sum x^2 that the producer of x left. The parts are dealt out to
     // all lane groups of all waves (group q of W*4 takes the parts q, q + 4W, ...), eight loads
@@ -268,6 +325,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
     if (TILED || blocks > 0) {
       fetch_rows(b0, blocks > 0 ? s : 0);
       fetch_weights(b0, blocks > 0 ? s : 0);
+      if constexpr (MT == 1) fetch_second();
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -298,21 +356,35 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
       for (int wv = 0; wv < W; ++wv) sum += rsum[wv][t][col];
       rs[t] = rsqrtf(sum / (float)K + eps);
     }
-  } else {
+  } else if constexpr (!MERGED) {
     if (blocks > 0) fetch_weights(b0, s);
   }
   if constexpr (MERGED) {
-    // The wave's run of k, four values a lane and turn, merged as attention_merge_kernel does.
-    const int kb0 = s_begin * 32, quads = (s_end - s_begin) * 8;
+    // The wave's run of k, four values a lane and turn, merged as attention_merge_kernel does. The
+    // first turn's partial results are asked for before the first two blocks of weights (loads
+    // come back in their order), which are on their way while the merge is made.
+    const int kb0 = s_begin * 32, quads = (s_end - s_begin) * 8, items = M * quads;
     const int D = mi.head_dim, S = mi.splits;
-    for (int item = lane; item < M * quads; item += 64) {
-      const int row = item / quads, idx = (item - row * quads) * 4;
-      const int k = kb0 + idx, head = k / D, d = k - head * D;
-      const int64_t base = ((int64_t)row * mi.heads + head) * S;
-      const float4v merged = merged_quad(mi.part_o, mi.part_ml, base, S, D, d);
-      bf16_t* dst = &xs[ks][row][idx];
+    MergeQuad<> parts;
+    auto ask = [&](int item) __attribute__((always_inline)) {
+      const int row = item / quads, k = kb0 + (item - row * quads) * 4, head = k / D;
+      parts.ask(mi.part_o, mi.part_ml, ((int64_t)row * mi.heads + head) * S, S, D, k - head * D);
+    };
+    if (items > 0) ask(min(lane, items - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    if (blocks > 0) fetch_weights(b0, s);
+    if (blocks > 1) fetch_weights(b1, s + 4);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int item0 = 0; item0 < items; item0 += 64) {
+      const int item = item0 + lane;
+      if (item0 > 0) ask(min(item, items - 1));
+      const float4v merged = parts.merged(S);
+      if (item < items) {
+        const int row = item / quads;
+        bf16_t* dst = &xs[ks][row][(item - row * quads) * 4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) dst[i] = (bf16_t)merged[i];
+        for (int i = 0; i < 4; ++i) dst[i] = (bf16_t)merged[i];
+      }
     }
     __syncthreads();
 #pragma unroll
@@ -320,6 +392,11 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
   }
   if constexpr (!NORM) {
     if (blocks > 0) fetch_rows(b0, s);
+    if constexpr (MERGED) {
+      if (blocks > 1) fetch_rows(b1, s + 4);
+    } else if constexpr (MT == 1) {
+      if (blocks > 0) fetch_second();
+    }
   }
   if constexpr (MT > 1) {
     // several row tiles: one body for every turn (the registers do not hold two whole blocks)
@@ -333,26 +410,28 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
       if (more) b0 = b1;
     }
   } else if (blocks > 0) {
-    while (blocks >= 3) {
-      fetch_rows(b1, s + 4);
-      fetch_weights(b1, s + 4);
-      __builtin_amdgcn_sched_barrier(0);  // all of the next block's loads leave before the products
+    while (blocks >= 4) {
+      multiply(b0);
+      fetch_rows(b0, s + 8);
+      fetch_weights(b0, s + 8);
+      __builtin_amdgcn_sched_barrier(0);  // all of a block's loads leave before the other's products
+      multiply(b1);
+      fetch_rows(b1, s + 12);
+      fetch_weights(b1, s + 12);
+      __builtin_amdgcn_sched_barrier(0);
+      s += 8;
+      blocks -= 2;
+    }
+    if (blocks == 3) {
       multiply(b0);
       fetch_rows(b0, s + 8);
       fetch_weights(b0, s + 8);
       __builtin_amdgcn_sched_barrier(0);
       multiply(b1);
-      s += 8;
-      blocks -= 2;
-    }
-    if (blocks == 2) {
-      fetch_rows(b1, s + 4);
-      fetch_weights(b1, s + 4);
-      __builtin_amdgcn_sched_barrier(0);
       multiply(b0);
-      multiply(b1);
     } else {
       multiply(b0);
+      if (blocks == 2) multiply(b1);
     }
     s = s_begin + (s_end - s_begin) / 4 * 4;
   }
@@ -369,37 +448,119 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
     }
   }
 
+  if constexpr (SHORT) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int a = 0; a < NA; ++a) red[ks][0][j][a][0][lane] = acc[j][a][0];
+    __syncthreads();
+    // this thread's elements: the waves' parts, all read before the first is added, in wave order
+    const int m = e_row;
+    const bool here = (int)threadIdx.x < 256 && m < M;
+    float y[NT][BA];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      float part[BA][KS];
+#pragma unroll
+      for (int a = 0; a < BA; ++a) {
+        const float* src = reinterpret_cast<const float*>(&red[0][0][j][BA > NA ? 0 : a][0][0]) +
+                           (BA > NA && a == 1 ? (threadIdx.x % 256) ^ 128 : threadIdx.x % 256);
+#pragma unroll
+        for (int wv = 0; wv < KS; ++wv) part[a][wv] = src[wv * (NT * NA * 256)];
+      }
+#pragma unroll
+      for (int a = 0; a < BA; ++a) {
+        float sum = part[a][0];
+#pragma unroll
+        for (int wv = 1; wv < KS; ++wv) sum += part[a][wv];
+        if (bias != nullptr) sum += (float)b_at[j][a][0];  // (past the last feature: dropped)
+        y[j][a] = sum;
+      }
+    }
+    __shared__ float sqs[EPI == EPI_RESIDUAL ? NT : 1][4][16];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int tile = tile0 + j, n = tile * 16 + e_n;
+      if (EPI == EPI_QKV) {
+        if (!here || tile * 16 >= N) continue;
+        const int d = qr.head_dim, half = d / 2;
+        const int head = tile * 16 / d, t_in = (tile * 16 - head * d) / 16;
+        const float v = (float)(bf16_t)y[j][0], partner = (float)(bf16_t)y[j][BA - 1];
+        const int jt = EPI == EPI_QKV ? j : 0;
+        if (head < qr.q_heads + qr.kv_heads) {  // rotary
+          const float cs = cs_at[jt][0], sn = sn_at[jt][0];
+          const bf16_t r = e_grp < 2 ? (bf16_t)(v * cs - partner * sn) : (bf16_t)(v * cs + partner * sn);
+          const int dim = (e_grp < 2 ? 0 : half) + 8 * t_in + 4 * (e_grp & 1) + e_i;
+          if (head < qr.q_heads) {
+            reinterpret_cast<bf16_t*>(out)[(int64_t)m * ldo + head * d + dim] = r;
+          } else if (slot_at >= 0) {
+            const int64_t page = slot_at / qr.page_size;
+            const int off = slot_at - (int)page * qr.page_size;
+            qr.k_pages[((page * qr.kv_heads + (head - qr.q_heads)) * qr.page_size + off) * d + dim] = r;
+          }
+        } else if (slot_at >= 0) {
+          const int64_t page = slot_at / qr.page_size;
+          const int off = slot_at - (int)page * qr.page_size;
+          const int hv = head - qr.q_heads - qr.kv_heads;
+          qr.v_pages[((page * qr.kv_heads + hv) * d + 16 * t_in + e_n) * qr.page_size + off] = (bf16_t)v;
+        }
+      } else if (EPI == EPI_RESIDUAL) {
+        const bf16_t summed = (bf16_t)((float)old_s[EPI == EPI_RESIDUAL ? j : 0][0][0] + (float)(bf16_t)y[j][0]);
+        const bool in = here && n < N;
+        if (in) stream[(int64_t)m * lds_ + n] = summed;
+        const float sq = quad_sum(in ? (float)summed * (float)summed : 0.f);
+        if ((int)threadIdx.x < 256 && e_i == 0) sqs[j][e_grp][m] = sq;
+      } else if (here && n < N) {
+        const int64_t place = (int64_t)m * ldo + n;
+        if (EPI == EPI_STORE) reinterpret_cast<bf16_t*>(out)[place] = (bf16_t)y[j][0];
+        else if (EPI == EPI_F32) reinterpret_cast<float*>(out)[place] = y[j][0];
+        else reinterpret_cast<bf16_t*>(out)[place] = glu_bf16((float)(bf16_t)y[j][0], (float)(bf16_t)y[j][NA - 1], glu);
+      }
+    }
+    if (EPI == EPI_RESIDUAL) {
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        if ((int)threadIdx.x < M && (tile0 + j) * 16 < N)
+          ssq_out[(int64_t)(tile0 + j) * M + threadIdx.x] =
+              (sqs[j][0][threadIdx.x] + sqs[j][1][threadIdx.x]) + (sqs[j][2][threadIdx.x] + sqs[j][3][threadIdx.x]);
+    }
+    return;
+  }
+
   // k-split wave 0 of each group adds the other waves' partial tiles to its own, in wave order
-  if (KS > 1) {
+  if constexpr (!SHORT && KS > 1) {
     if (ks != 0) {
 #pragma unroll
       for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int a = 0; a < NA; ++a)
 #pragma unroll
-          for (int t = 0; t < MT; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) red[ks - 1][ns][j][a][t][i][lane] = acc[j][a][t][i];
+          for (int t = 0; t < MT; ++t) red[ks - 1][ns][j][a][t][lane] = acc[j][a][t];
     }
     __syncthreads();
-    if (ks == 0) {
+    if (ks == 0) {  // all of a tile's parts are read before the first is added
 #pragma unroll
       for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int a = 0; a < NA; ++a)
+        for (int t = 0; t < MT; ++t) {
+          float4v part[NA][KR];
 #pragma unroll
-          for (int t = 0; t < MT; ++t)
+          for (int a = 0; a < NA; ++a)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              float v = acc[j][a][t][i];
-              for (int wv = 0; wv < KS - 1; ++wv) v += red[wv][ns][j][a][t][i][lane];
-              acc[j][a][t][i] = v;
-            }
+            for (int wv = 0; wv < KS - 1; ++wv) part[a][wv] = red[wv][ns][j][a][t][lane];
+#pragma unroll
+          for (int a = 0; a < NA; ++a)
+#pragma unroll
+            for (int wv = 0; wv < KS - 1; ++wv) acc[j][a][t] += part[a][wv];
+        }
     }
   }
 
   // lane holds y[m = 16t + col][n = 16*tile + 4*grp + i]
+  if constexpr (!SHORT) {
   if (ks == 0) {
+  if constexpr (MT > 1) load_bias();
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     const int tile = tile0 + j;
@@ -414,15 +575,14 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           y[a][i] = acc[j][a][t][i];
-          if (bias != nullptr && nb + i < N) y[a][i] += (float)bias[nb + i + a * up_offset];
+          if (bias != nullptr) y[a][i] += (float)b_at[j][a][i];  // (past the last feature: dropped)
         }
       if constexpr (EPI == EPI_QKV) {
         // all lanes take part in the exchange of partners; rows beyond M hold zeros
         const int d = qr.head_dim, half = d / 2;
         const int head = tile * 16 / d, t_in = (tile * 16 - head * d) / 16;
         const bool rotary = head < qr.q_heads + qr.kv_heads;
-        const int mm = min(m, M - 1);
-        const int slot = qr.slots[mm];
+        const int slot = slot_at, jt = EPI == EPI_QKV ? j : 0;
         float v[4], partner[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -431,12 +591,10 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
         }
         if (rotary) {
           const int j = 8 * t_in + 4 * (grp & 1);  // first of this lane's four rotary pairs
-          const float4v cs = *reinterpret_cast<const float4v*>(qr.angles + ((int64_t)mm * 2 + 0) * half + j);
-          const float4v sn = *reinterpret_cast<const float4v*>(qr.angles + ((int64_t)mm * 2 + 1) * half + j);
           bf16_t r[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            r[i] = grp < 2 ? (bf16_t)(v[i] * cs[i] - partner[i] * sn[i]) : (bf16_t)(v[i] * cs[i] + partner[i] * sn[i]);
+            r[i] = grp < 2 ? (bf16_t)(v[i] * cs_at[jt][i] - partner[i] * sn_at[jt][i]) : (bf16_t)(v[i] * cs_at[jt][i] + partner[i] * sn_at[jt][i]);
           const int dim = (grp < 2 ? 0 : half) + j;
           bf16_t* dst = nullptr;
           if (head < qr.q_heads) {
@@ -489,6 +647,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
     }
   }
   }
+  }
 }
 
 // Embedding rows with the sum of squares of each (one part), for the first layer's norm.
@@ -514,10 +673,323 @@ __global__ void embedding_ssq_kernel(const bf16_t* __restrict__ table, const int
 #define SK_ARGS \
   x, ldx, ssq_in, ssq_parts, norm_w, eps, w, bias, out, ldo, stream_buf, lds_, ssq_out, M, N, K, up_offset, qr, glu, stream
 
+// The products that open the two halves of a decode layer (q/k/v with rotation and cache write, gate and up), with the
+// row norm inside: at most 16 rows, weights in tile order, k split over the KS waves of a workgroup,
+// which owns NT tiles. What bounds such a launch beside its weights is the time until they are asked
+// for and the vector cache, which accepts 64 bytes a cycle and compute unit:
+//  - The workgroup normalises the rows once, into LDS, and its waves read their fragments from there.
+//    (Read from memory by every wave, a block's fragments are 12 KB, 16 bytes of x and 32 of norm
+//    weights a lane and product, beside 4 KB of weights a tile.)
+//  - Sums of squares, rows, norm weights and the first SETS blocks of weights are asked for in this order before
+//    anything is waited for (loads come back in their order), with few instructions on the way:
+//    through buffer resources, which count what lies past their end as zeros, so that no load needs a condition
+//    or a bound of its own. What only the end needs is asked for last.
+// MR: rows whose pieces are asked for at the start (further rows afterwards).
+// In decode steps of one row from start to end of the launch (135M and 1B sizes): q/k/v 2.7 -> 1.7 us and 4.6 -> 2.5.
+struct NormedArgs {
+  const bf16_t* x;
+  const float* ssq_in;
+  const float* norm_w;
+  const bf16_t* w;
+  const bf16_t* bias;
+  bf16_t* out;
+  int64_t ldo;
+  int ldx, ssq_parts, M, N, K, up_offset;
+  float eps;
+  QkvRope qr;
+  GluForm glu;
+};
+
+// Values per row of the normalised rows in LDS: whole blocks, and 16 bytes more, so that the sixteen
+// rows that a fragment reads lie in different banks.
+__host__ __device__ constexpr int normed_row(int K) { return (K + 127) / 128 * 128 + 8; }
+
+template <int KS, int NT, int EPI, int SETS, int MR>
+__global__ __launch_bounds__(KS * 64) void normed_tiles_kernel(NormedArgs p) {
+  static_assert(EPI == EPI_SWIGLU || EPI == EPI_QKV, "the products behind a norm");
+  constexpr int NA = EPI == EPI_SWIGLU ? 2 : 1;  // weight row sets per tile (gate and up)
+  constexpr int BA = 2;                          // sums a thread makes per tile: gate and up, or a feature and its rotary partner
+  constexpr int PARTS = MR == 1 ? 2 : MR;         // loads of 64 parts of the sums of squares a wave asks for at the start
+  constexpr int PRE = KS == 4 ? 3 : 2;           // pieces of 256 values of the rows likewise
+  constexpr unsigned OUTSIDE = 0x80000000u;      // an offset past the end of every resource here
+  typedef short short4v __attribute__((ext_vector_type(4)));
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  __shared__ float red[KS][NT][NA][256];
+  __shared__ float rsum[KS][16];
+  extern __shared__ __attribute__((aligned(16))) bf16_t xs[];  // rows of normed_row(K) values
+
+  const int lane = threadIdx.x % 64, ks = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int col = lane % 16, grp = lane / 16;
+  const int tile0 = blockIdx.x * NT, tiles = p.N / 16;
+  const int M = p.M, K = p.K, row = normed_row(K);
+
+  // The parts of sum x^2 that the producer of x left, [part][row]. Where the rows are a power of two
+  // (decode graphs) a wave takes 64 of them in a row, lane l for row l % M; else the lane group grp takes
+  // part 4 ks + grp, and every 4 KS-th behind it, for row l % 16.
+  const __amdgpu_buffer_rsrc_t sres = __builtin_amdgcn_make_buffer_rsrc((void*)p.ssq_in, 0, (unsigned)(p.ssq_parts * M * 4), 0x00020000);
+  const bool even = (M & (M - 1)) == 0;
+  const int s_at = even ? threadIdx.x * 4 : ((4 * ks + grp) * M + min(col, M - 1)) * 4;
+  const int s_step = even ? 256 * KS : 16 * KS * M, s_end = p.ssq_parts * M * 4;
+  float first[PARTS];
+#pragma unroll
+  for (int u = 0; u < PARTS; ++u) first[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(sres, s_at + u * s_step, 0, 0));
+  // rows: wave ks takes the pieces ks, ks + KS, ... of 256 values, four a lane
+  const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, (unsigned)(((M - 1) * p.ldx + K) * 2), 0x00020000);
+  const __amdgpu_buffer_rsrc_t gres = __builtin_amdgcn_make_buffer_rsrc((void*)p.norm_w, 0, (unsigned)(K * 4), 0x00020000);
+  union Four {
+    u32x2 raw;
+    bf16_t e[4];
+  };
+  union Gain {
+    u32x4 raw;
+    float e[4];
+  };
+  Four piece[PRE][MR];
+  Gain gain[PRE];
+  auto ask_gain = [&](Gain& g, int j) __attribute__((always_inline)) {
+    g.raw = __builtin_amdgcn_raw_buffer_load_b128(gres, ((ks + j * KS) * 256 + lane * 4) * 4, 0, 0);
+  };
+  auto ask_rows = [&](Four (&v)[MR], int j, int m0) __attribute__((always_inline)) {
+    const int k = (ks + j * KS) * 256 + lane * 4;
+    const unsigned at = k < K ? (unsigned)(k * 2) : OUTSIDE;
+#pragma unroll
+    for (int u = 0; u < MR; ++u) v[u].raw = __builtin_amdgcn_raw_buffer_load_b64(xres, at + (unsigned)((m0 + u) * p.ldx * 2), 0, 0);
+  };
+#pragma unroll
+  for (int j = 0; j < PRE; ++j) {
+    ask_gain(gain[j], j);
+    ask_rows(piece[j], j, 0);
+  }
+  // weights: this wave's share of the blocks of 128 k
+  const int whole = (K + 127) / 128, c0 = whole * ks / KS, blocks = whole * (ks + 1) / KS - c0;
+  const bf16_t* wrow[NT][NA];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+      wrow[j][a] = p.w + ((int64_t)min(tile0 + j, tiles - 1) + a * (p.up_offset / 16)) * 16 * (whole * 128) + c0 * 2048;
+  struct Set {
+    bf16x8 a[NT][NA][4];
+  } sets[SETS];
+  auto fetch = [&](Set& b, int c) __attribute__((always_inline)) {
+    const int at = max(min(c, blocks - 1), 0) * 2048;  // (a wave without a block: one that is there, for nothing)
+    const int from = blocks > 0 ? at : -c0 * 2048;
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) b.a[j][a][q] = *reinterpret_cast<const bf16x8*>(wrow[j][a] + from + q * 512 + lane * 8);
+  };
+#pragma unroll
+  for (int d = 0; d < SETS; ++d) fetch(sets[d], d);
+  __builtin_amdgcn_sched_barrier(0);
+  // What the end adds. Thread t makes output t of each tile: element t % 4 of lane t / 4 of the
+  // product's result, that is row t / 4 % 16 and feature 4 (t / 64) + t % 4.
+  const int o_m = threadIdx.x / 4 % 16, o_grp = threadIdx.x / 64 % 4, o_n = 4 * o_grp + threadIdx.x % 4;
+  const __amdgpu_buffer_rsrc_t bres = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)p.bias, 0, p.bias != nullptr ? (unsigned)(p.N + (NA - 1) * p.up_offset) * 2u : 0u, 0x00020000);
+  union Half {
+    unsigned short raw;
+    bf16_t v;
+  } b_at[NT][BA];
+  float cs_at[NT], sn_at[NT];
+  int slot = -1;
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const int n = (tile0 + j) * 16;
+    b_at[j][0].raw = __builtin_amdgcn_raw_buffer_load_b16(bres, (n + o_n) * 2, 0, 0);
+    b_at[j][1].raw = __builtin_amdgcn_raw_buffer_load_b16(bres, (EPI == EPI_SWIGLU ? n + o_n + p.up_offset : n + (o_n ^ 8)) * 2, 0, 0);
+  }
+  if constexpr (EPI == EPI_QKV) {
+    const int half = p.qr.head_dim / 2, m = min(o_m, M - 1);
+    slot = p.qr.slots[m];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int t_in = min(tile0 + j, tiles - 1) % (p.qr.head_dim / 16);
+      const float* at = p.qr.angles + (int64_t)m * 2 * half + 8 * t_in + (o_n & 7);  // the rotary pair
+      cs_at[j] = at[0];
+      sn_at[j] = at[half];
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  // 1 / rms of row `col`: the lane's parts, the wave's lanes of a row, the waves in order
+  float sum = 0.f;
+#pragma unroll
+  for (int u = 0; u < PARTS; ++u) sum += first[u];
+  for (int at = PARTS * s_step; at < s_end; at += s_step) sum += __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(sres, s_at + at, 0, 0));
+  sum = add_halves(sum, sum);
+  sum = add_rows(sum, sum);
+  if (even) {
+    if (M <= 8) sum += row_ror<8>(sum);
+    if (M <= 4) sum += row_ror<4>(sum);
+    if (M == 1) sum = quad_sum(sum);
+    else if (M == 2) sum = quad_pairs(sum);
+  }
+  if (lane < M) rsum[ks][lane] = sum;
+  __syncthreads();
+  float part[KS], total = 0.f;
+#pragma unroll
+  for (int wv = 0; wv < KS; ++wv) part[wv] = rsum[wv][min(col, M - 1)];
+#pragma unroll
+  for (int wv = 0; wv < KS; ++wv) total += part[wv];
+  const float rs = rsqrtf(total / (float)K + p.eps);
+  auto put_rows = [&](const Four (&v)[MR], const Gain& g, int j, int m0) __attribute__((always_inline)) {
+    const int k = (ks + j * KS) * 256 + lane * 4;
+#pragma unroll
+    for (int u = 0; u < MR; ++u)
+      if (m0 + u < M) {
+        const float rsm = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rs), m0 + u));
+        Four h;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {  // (past K values and weights are zeros)
+          const float normed = (float)(bf16_t)((float)v[u].e[i] * rsm);
+          h.e[i] = (bf16_t)(g.e[i] * normed);
+        }
+        if (k < whole * 128) *reinterpret_cast<u32x2*>(xs + (m0 + u) * row + k) = h.raw;
+      }
+  };
+#pragma unroll
+  for (int j = 0; j < PRE; ++j)
+    if ((ks + j * KS) * 256 < whole * 128) put_rows(piece[j], gain[j], j, 0);
+  // what did not fit the start: further rows, further pieces of long rows
+  for (int j = 0; (ks + j * KS) * 256 < whole * 128; ++j)
+    for (int m0 = j < PRE ? MR : 0; m0 < M; m0 += MR) {
+      Four v[MR];
+      Gain g;
+      ask_gain(g, j);
+      ask_rows(v, j, m0);
+      put_rows(v, g, j, m0);
+    }
+  __syncthreads();
+
+  float4v acc[NT][NA];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int a = 0; a < NA; ++a) acc[j][a] = float4v{0.f, 0.f, 0.f, 0.f};
+  const bf16_t* frag = xs + min(col, M - 1) * row + c0 * 128 + grp * 32;
+  auto multiply = [&](const Set& b, int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const bf16x8 bf = *reinterpret_cast<const bf16x8*>(frag + c * 128 + q * 8);
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int a = 0; a < NA; ++a) acc[j][a] = mfma32(b.a[j][a][q], bf, acc[j][a]);
+    }
+  };
+  int c = 0;
+  for (; c + 2 * SETS <= blocks; c += SETS) {
+#pragma unroll
+    for (int d = 0; d < SETS; ++d) {
+      multiply(sets[d], c + d);
+      fetch(sets[d], c + d + SETS);
+      __builtin_amdgcn_sched_barrier(0);  // the loads leave before the next block's products
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < SETS; ++d) {
+    if (c + d < blocks) multiply(sets[d], c + d);
+    if (c + d + SETS < blocks) fetch(sets[d], c + d + SETS);
+  }
+#pragma unroll
+  for (int d = 0; d < SETS; ++d)
+    if (c + d + SETS < blocks) multiply(sets[d], c + d + SETS);
+
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int a = 0; a < NA; ++a) *reinterpret_cast<float4v*>(&red[ks][j][a][lane * 4]) = acc[j][a];
+  __syncthreads();
+  if (KS > 4 && ks >= 4) return;  // 256 outputs a tile
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    float part_y[BA][KS], y[BA];
+#pragma unroll
+    for (int wv = 0; wv < KS; ++wv) {
+      part_y[0][wv] = red[wv][j][0][threadIdx.x];
+      part_y[1][wv] = EPI == EPI_SWIGLU ? red[wv][j][NA - 1][threadIdx.x] : red[wv][j][0][threadIdx.x ^ 128];
+    }
+#pragma unroll
+    for (int a = 0; a < BA; ++a) {
+      y[a] = part_y[a][0];
+#pragma unroll
+      for (int wv = 1; wv < KS; ++wv) y[a] += part_y[a][wv];
+      if (p.bias != nullptr) y[a] += (float)b_at[j][a].v;
+    }
+    const int tile = tile0 + j;
+    if (o_m >= M || tile >= tiles) continue;
+    if constexpr (EPI == EPI_SWIGLU) {
+      p.out[(int64_t)o_m * p.ldo + tile * 16 + o_n] = glu_bf16((float)(bf16_t)y[0], (float)(bf16_t)y[1], p.glu);
+    } else {
+      const int d = p.qr.head_dim, half = d / 2;
+      const int head = tile * 16 / d, t_in = (tile * 16 - head * d) / 16;
+      const float v = (float)(bf16_t)y[0], partner = (float)(bf16_t)y[1];
+      const int64_t page = slot / p.qr.page_size;
+      const int off = slot - (int)page * p.qr.page_size;
+      if (head < p.qr.q_heads + p.qr.kv_heads) {  // rotary
+        const bf16_t r = o_grp < 2 ? (bf16_t)(v * cs_at[j] - partner * sn_at[j]) : (bf16_t)(v * cs_at[j] + partner * sn_at[j]);
+        const int dim = (o_grp < 2 ? 0 : half) + 8 * t_in + (o_n & 7);
+        if (head < p.qr.q_heads) p.out[(int64_t)o_m * p.ldo + head * d + dim] = r;
+        else if (slot >= 0) p.qr.k_pages[((page * p.qr.kv_heads + (head - p.qr.q_heads)) * p.qr.page_size + off) * d + dim] = r;
+      } else if (slot >= 0) {
+        const int hv = head - p.qr.q_heads - p.qr.kv_heads;
+        p.qr.v_pages[((page * p.qr.kv_heads + hv) * d + 16 * t_in + o_n) * p.qr.page_size + off] = (bf16_t)v;
+      }
+    }
+  }
+}
+
+// More than 40 KB of LDS beside the kernel's own has to be allowed; whether the runtime refused (it
+// then holds an error, which the launch's status reports).
+static bool lds_refused(const void* kernel, size_t lds) {
+  return lds > 40 * 1024 &&
+         hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024) != hipSuccess;
+}
+
+// Whether normed_tiles_kernel takes the product: its rows leave room in LDS for two workgroups on a
+// compute unit, and lie within what its 31-bit offsets reach. Four blocks of weights on their way where every
+// wave has three or more, else two; a gated pair of two tiles takes the registers of two.
+template <int KS, int NT, int EPI>
+static bool launch_normed_tiles(SK_PARAMS) {
+  constexpr int PER = NT * (EPI == EPI_SWIGLU ? 2 : 1);
+  const size_t lds = (size_t)M * normed_row(K) * 2;
+  if (lds + (size_t)KS * PER * 1024 + 1024 > 80 * 1024 || N % 16 != 0 || ldx > INT32_MAX / 64 || ssq_parts > INT32_MAX / 256 ||
+      (int64_t)N + up_offset > INT32_MAX / 4)
+    return false;
+  const NormedArgs args{(const bf16_t*)x, ssq_in, norm_w, (const bf16_t*)w, (const bf16_t*)bias, (bf16_t*)out, ldo, (int)ldx,
+                        ssq_parts, M, N, K, up_offset, eps, qr, glu};
+  const int groups = (N / 16 + NT - 1) / NT;
+#define NORMED_LAUNCH(SETS_, MR_)                                                        \
+  {                                                                                      \
+    const auto kernel = normed_tiles_kernel<KS, NT, EPI, SETS_, MR_>;                     \
+    if (!lds_refused((const void*)kernel, lds)) kernel<<<groups, KS * 64, lds, stream>>>(args); \
+  }
+  if constexpr (PER <= 2) {
+    if ((K + 127) / 128 / KS >= 3) {
+      if (M == 1) NORMED_LAUNCH(4, 1)
+      else if (M <= 4) NORMED_LAUNCH(4, 4)
+      else NORMED_LAUNCH(4, 8)
+      return true;
+    }
+  }
+  if (M == 1) NORMED_LAUNCH(2, 1)
+  else if (M <= 4) NORMED_LAUNCH(2, 4)
+  else NORMED_LAUNCH(2, 8)
+#undef NORMED_LAUNCH
+  return true;
+}
+
 template <int KS, int NS, int NT, int MT, int EPI, bool NORM, bool TILED>
 static void launch_skinny(SK_PARAMS) {
   const int tiles = (N + 15) / 16;
   const int groups = (tiles + NS * NT - 1) / (NS * NT);
+  if constexpr (NORM && TILED && MT == 1 && NS == 1 && (EPI == EPI_SWIGLU || EPI == EPI_QKV)) {
+    if (launch_normed_tiles<KS, NT, EPI>(SK_ARGS)) return;
+  }
   skinny_gemm_kernel<KS, NS, NT, MT, EPI, NORM, TILED><<<groups, KS * NS * 64, 0, stream>>>(
       (const bf16_t*)x, ldx, ssq_in, ssq_parts, norm_w, eps, (const bf16_t*)w, (const bf16_t*)bias,
       out, ldo, (bf16_t*)stream_buf, lds_, ssq_out, M, N, K, up_offset, qr, MergedIn{}, glu);

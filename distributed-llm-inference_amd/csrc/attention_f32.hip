@@ -28,12 +28,12 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_f32_kernel(
     const float* __restrict__ q, int64_t q_stride, const float* __restrict__ k_pages, const float* __restrict__ v_pages,
     float* __restrict__ out, int64_t out_stride, const int* __restrict__ q_start, const int* __restrict__ kv_len,
     const int* __restrict__ block_tables, int table_stride, const int* __restrict__ tile_entry, const int* __restrict__ tile_q0,
-    int per_tile, int q_heads, int kv_heads, int page_size, float scale, int window) {
+    int per_tile, int group, int kv_heads, int page_size, PageOf page_of_tile, float scale, int window) {
   constexpr int D = 16 * DT;
   __shared__ af4 accs[AF_WAVES][DT][64];
   __shared__ float ms[AF_WAVES][16], ls[AF_WAVES][16];
-  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, i = lane % 16, g = lane / 16;
-  const int tile = blockIdx.x / per_tile, entry = tile_entry[tile], head = blockIdx.y, kvh = head / (q_heads / kv_heads);
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), i = lane % 16, g = lane / 16;
+  const int tile = blockIdx.x / per_tile, entry = tile_entry[tile], head = blockIdx.y, kvh = head / group;
   const int q0 = tile_q0[tile] + blockIdx.x % per_tile * 16;
   const int tok0 = q_start[entry], q_len = q_start[entry + 1] - tok0;
   if (q0 >= q_len) return;   // (the list's tiles are 16 * per_tile queries high)
@@ -52,22 +52,36 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_f32_kernel(
   const int b_end = (first_pos + rows + 15) / 16;   // blocks that some query sees
   int b = window > 0 ? max(0, first_pos - window + 1) / 16 : 0;
   b += (wave - b % AF_WAVES + AF_WAVES) % AF_WAVES;
+  // Block b's page is looked up two turns ahead and its keys are asked for one turn ahead, on the scalar unit where they are
+  // the same for all lanes: a turn then waits for no table entry. (A block past the last reads the last one's page.)
+  const int b_last = max(b_end - 1, 0);
+  struct Where {
+    int64_t page;   // (a page that a window has passed: any page, its keys are not seen)
+    int off;        // the block's first key in it
+  };
+  const auto look_up = [&](int block) {
+    const unsigned t = (unsigned)min(block, b_last), page = page_of_tile.page(t);
+    return Where{(int64_t)max(table[page], 0) * kv_heads + kvh, (int)(t - page * page_of_tile.tiles) * 16};
+  };
   af4 fk[DT];
-  const auto page_of = [&](int block) -> int64_t {   // (a page that a window has passed: any page, its keys are not seen)
-    return (int64_t)max(table[block * 16 / page_size], 0) * kv_heads + kvh;
-  };
-  const auto load_keys = [&](int block) {
-    const float* kr = k_pages + (page_of(block) * page_size + block * 16 % page_size + i) * D + 4 * g;
+  const auto load_keys = [&](const Where& at) {
+    const float* kr = k_pages + (at.page * page_size + at.off) * D;
 #pragma unroll
-    for (int t = 0; t < DT; ++t) fk[t] = *reinterpret_cast<const af4*>(kr + 16 * t);
+    for (int t = 0; t < DT; ++t) fk[t] = *reinterpret_cast<const af4*>(kr + i * D + 4 * g + 16 * t);
   };
-  if (b < b_end) load_keys(b);
+  Where here{0, 0}, next{0, 0};
+  if (b < b_end) {
+    here = look_up(b);
+    next = look_up(b + AF_WAVES);
+    load_keys(here);
+  }
   for (; b < b_end; b += AF_WAVES) {
     const int j0 = b * 16 + 4 * g;
     af4 fv[DT];
-    const float* vr = v_pages + (page_of(b) * D + i) * page_size + b * 16 % page_size + 4 * g;
+    const float* vr = v_pages + here.page * D * page_size + here.off;
 #pragma unroll
-    for (int t = 0; t < DT; ++t) fv[t] = *reinterpret_cast<const af4*>(vr + (int64_t)16 * t * page_size);
+    for (int t = 0; t < DT; ++t) fv[t] = *reinterpret_cast<const af4*>(vr + (i + 16 * t) * page_size + 4 * g);
+    const Where after = look_up(b + 2 * AF_WAVES);
     // two sums side by side: a chain of products waits for itself
     af4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -77,7 +91,9 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_f32_kernel(
         s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(fk[t][e], fq[t][e], s0, 0, 0, 0);
         s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(fk[t + 1][e], fq[t + 1][e], s1, 0, 0, 0);
       }
-    if (b + AF_WAVES < b_end) load_keys(b + AF_WAVES);
+    if (b + AF_WAVES < b_end) load_keys(next);
+    here = next;
+    next = after;
     af4 s = s0 + s1;
     float top = -INFINITY;
 #pragma unroll
@@ -121,19 +137,26 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_f32_kernel(
   for (int t = 0; t < DT; ++t) accs[wave][t][lane] = acc[t];
   __syncthreads();
   if (wave >= DT) return;
-  float top = -INFINITY, total = 0.f, w[AF_WAVES];
+  float top = -INFINITY, total = 0.f, w[AF_WAVES], m_c[AF_WAVES], l_c[AF_WAVES];
 #pragma unroll
-  for (int c = 0; c < AF_WAVES; ++c) top = fmaxf(top, ms[c][i]);
+  for (int c = 0; c < AF_WAVES; ++c) {   // (all read before the first is used)
+    m_c[c] = ms[c][i];
+    l_c[c] = ls[c][i];
+  }
+#pragma unroll
+  for (int c = 0; c < AF_WAVES; ++c) top = fmaxf(top, m_c[c]);
 #pragma unroll
   for (int c = 0; c < AF_WAVES; ++c) {
-    w[c] = ms[c][i] > -INFINITY ? expf(ms[c][i] - top) : 0.f;
-    total += ls[c][i] * w[c];
+    w[c] = m_c[c] > -INFINITY ? expf(m_c[c] - top) : 0.f;
+    total += l_c[c] * w[c];
   }
   const float inv = total > 0.f ? 1.f / total : 0.f;
   for (int t = wave; t < DT; t += AF_WAVES) {
-    af4 sum = {0.f, 0.f, 0.f, 0.f};
+    af4 sum = {0.f, 0.f, 0.f, 0.f}, part[AF_WAVES];
 #pragma unroll
-    for (int c = 0; c < AF_WAVES; ++c) sum += accs[c][t][lane] * w[c];
+    for (int c = 0; c < AF_WAVES; ++c) part[c] = accs[c][t][lane];
+#pragma unroll
+    for (int c = 0; c < AF_WAVES; ++c) sum += part[c] * w[c];
     if (i < rows)
       *reinterpret_cast<af4*>(out + (int64_t)(tok0 + q0 + i) * out_stride + (int64_t)head * D + 16 * t + 4 * g) = sum * inv;
   }
@@ -157,7 +180,7 @@ int attention_f32(const float* q, int64_t q_stride, const float* k_pages, const 
   const dim3 grid(tiles * per_tile, q_heads);
 #define AF_LAUNCH(DT)                                                                                               \
   attention_f32_kernel<DT><<<grid, 64 * AF_WAVES, 0, stream>>>(q, q_stride, k_pages, v_pages, out, out_stride, q_start, kv_len, \
-      block_tables, table_stride, tile_entry, tile_q0, per_tile, q_heads, kv_heads, page_size, scale, window)
+      block_tables, table_stride, tile_entry, tile_q0, per_tile, q_heads / kv_heads, kv_heads, page_size, page_of_tile(page_size), scale, window)
   if (head_dim == 64) AF_LAUNCH(4);
   else AF_LAUNCH(8);
 #undef AF_LAUNCH

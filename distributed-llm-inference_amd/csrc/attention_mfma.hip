@@ -171,24 +171,22 @@ __device__ __forceinline__ void blank_v(short4v (&vreg)[DCH], int grp, int t, in
 }
 
 // ------------------------------------------------------------------------------------ decode
-// grid (splits, kv_heads * head_tiles, requests); 256 threads. Request e's single query is row e.
+// grid (splits, kv_heads * head_tiles, requests); NW waves, which share out a run's tiles of 16 keys. Request e's single query is row e.
 // part_o, part_ml and arrivals without __restrict__: the workgroup that merges reads what other
 // workgroups of the launch stored.
-template <int DCH>
-__global__ __launch_bounds__(256) void attention_decode_kernel(
+template <int DCH, int NW>
+__global__ __launch_bounds__(NW * 64) void attention_decode_kernel(
     const bf16_t* __restrict__ q, int64_t q_stride, const bf16_t* __restrict__ k_pages,
     const bf16_t* __restrict__ v_pages, bf16_t* __restrict__ out, int64_t out_stride,
     float* part_o, float* part_ml, const int* __restrict__ kv_len,
-    const int* __restrict__ block_tables, int table_stride, int q_heads, int kv_heads, int page_size,
-    float scale_log2e, int window, int splits, unsigned* arrivals) {
+    const int* __restrict__ block_tables, int table_stride, int q_heads, int kv_heads, int group,
+    int head_tiles, int page_size, PageOf page_of, float scale_log2e, int window, int splits, unsigned* arrivals) {
   constexpr int D = DCH * 16;
-  __shared__ float sm_o[3][D][16];
-  __shared__ float sm_m[3][16], sm_l[3][16];
+  extern __shared__ float4v sm_o[];  // [wave][chunk of 16 dims][lane group][query head of the group]
+  __shared__ float sm_m[NW][16], sm_l[NW][16];
 
   const int split = blockIdx.x, e = blockIdx.z;
-  const int group = q_heads / kv_heads;
-  const int head_tiles = (group + 15) / 16;
-  const int kvh = blockIdx.y / head_tiles, ht = blockIdx.y % head_tiles;
+  const int kvh = head_tiles == 1 ? blockIdx.y : blockIdx.y / head_tiles, ht = blockIdx.y - kvh * head_tiles;
   const int lane = threadIdx.x % DLI_WAVE;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / DLI_WAVE);  // known to be the same in all lanes
   const int col = lane % 16, grp = lane / 16;
@@ -215,7 +213,7 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(
 
   ColumnTile<DCH> st;
   st.init();
-  // A wave takes every fourth tile of 16 keys, UN tiles (a group) at a time. A group costs a chain
+  // A wave takes every NW-th tile of 16 keys, UN tiles (a group) at a time. A group costs a chain
   // of two trips to memory (its block-table entries, then its keys and values), so the chain is
   // taken apart: while group g is multiplied, the keys and values of group g+1 are on their way
   // (two sets of registers take turns) and the table entries of group g+2 have been asked for.
@@ -223,7 +221,8 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(
   // is skipped by the arithmetic; values of keys past the end are blanked when they are used),
   // so at every wait the number of younger loads is known and only the group's own are waited for.
   constexpr int UN = 1, NG = 4;  // tiles of a group, groups on their way
-  constexpr int STEP = 64 * UN;  // keys between a wave's groups
+  constexpr int STRIDE = 16 * NW;     // keys between a wave's tiles
+  constexpr int STEP = STRIDE * UN;   // and its groups
   struct Group {
     short4v k[UN][DCH], v[UN][DCH];
   };
@@ -237,9 +236,9 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(
     auto look_up = [&](Where& w, int tg) __attribute__((always_inline)) {
 #pragma unroll
       for (int u = 0; u < UN; ++u) {
-        const int t = min(tg + 64 * u, t_last);
-        w.page[u] = table[t / page_size];
-        w.off[u] = t % page_size;
+        const unsigned tile = (unsigned)min(tg + STRIDE * u, t_last) / 16, page = page_of.page(tile);
+        w.page[u] = table[page];
+        w.off[u] = (tile - page * page_of.tiles) * 16;
       }
     };
     auto fetch = [&](Group& g, const Where& w) __attribute__((always_inline)) {
@@ -252,7 +251,7 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(
     auto attend = [&](const Group& g, int tg) __attribute__((always_inline)) {
 #pragma unroll
       for (int u = 0; u < UN; ++u) {
-        const int t = tg + 64 * u;
+        const int t = tg + STRIDE * u;
         if (t < k1) {
           const bool need_mask = t + 16 > k1 || t < first_visible;
           short4v v[DCH];  // a copy: the group's registers are written by loads only
@@ -288,45 +287,53 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(
     for (int d = 0; d < NG; ++d) attend(sets[d], tg + d * STEP);  // the last round
   }
 
-  // merge the four waves' states in wave 0
-  if (wave > 0) {
-    if (grp == 0) {
-      sm_m[wave - 1][col] = st.m;
-      sm_l[wave - 1][col] = st.l;
-    }
-#pragma unroll
-    for (int c = 0; c < DCH; ++c)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) sm_o[wave - 1][c * 16 + 4 * grp + i][col] = st.o[c][i];
+  // Merge the waves' states: every wave leaves its own in LDS (the columns that are heads), then takes the chunks
+  // wave, wave + NW, ... of sixteen dims from all of them. (Merged by one wave from values read one by one, this took
+  // 0.9 us of a launch of 6.4 at 512 keys; now 0.3.)
+  const int cols = min(16, group), per_chunk = 4 * cols;
+  if (grp == 0) {
+    sm_m[wave][col] = st.m;
+    sm_l[wave][col] = st.l;
   }
+  const int at = grp * cols + min(col, cols - 1);
+#pragma unroll
+  for (int c = 0; c < DCH; ++c)
+    if (col < cols) sm_o[(wave * DCH + c) * per_chunk + at] = st.o[c];
   __syncthreads();
-  if (wave != 0) return;
-  float m_all = st.m;
+  float m_w[NW], l_w[NW];
 #pragma unroll
-  for (int w = 0; w < 3; ++w) m_all = fmaxf(m_all, sm_m[w][col]);
+  for (int w = 0; w < NW; ++w) {
+    m_w[w] = sm_m[w][col];
+    l_w[w] = sm_l[w][col];
+  }
+  constexpr int CW = (DCH + NW - 1) / NW;  // chunks a wave merges
+  float4v o_w[CW][NW];
+#pragma unroll
+  for (int i = 0; i < CW; ++i)
+#pragma unroll
+    for (int w = 0; w < NW; ++w) o_w[i][w] = sm_o[(w * DCH + min(wave + NW * i, DCH - 1)) * per_chunk + at];
+  float m_all = m_w[0];
+#pragma unroll
+  for (int w = 1; w < NW; ++w) m_all = max2(m_all, m_w[w]);
   const float m_safe = m_all == -INFINITY ? 0.f : m_all;
-  float scale_own = fast_exp2(st.m - m_safe);
-  float l_all = st.l * scale_own;
+  float l_all = 0.f;
 #pragma unroll
-  for (int c = 0; c < DCH; ++c) st.o[c] *= scale_own;
+  for (int w = 0; w < NW; ++w) {
+    const float sw = fast_exp2(m_w[w] - m_safe);
+    l_all += l_w[w] * sw;
 #pragma unroll
-  for (int w = 0; w < 3; ++w) {
-    const float sw = fast_exp2(sm_m[w][col] - m_safe);
-    l_all += sm_l[w][col] * sw;
-#pragma unroll
-    for (int c = 0; c < DCH; ++c)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) st.o[c][i] += sm_o[w][c * 16 + 4 * grp + i][col] * sw;
+    for (int i = 0; i < CW; ++i) o_w[i][0] = w == 0 ? o_w[i][0] * sw : o_w[i][0] + o_w[i][w] * sw;
   }
   if (splits == 1) {
     if (!valid) return;
     const float inv = l_all > 0.f ? 1.f / l_all : 0.f;
     bf16_t* op = out + (int64_t)e * out_stride + (int64_t)head * D + 4 * grp;
 #pragma unroll
-    for (int c = 0; c < DCH; ++c) {
-      const short4v packed = {bf16_bits(st.o[c][0] * inv), bf16_bits(st.o[c][1] * inv),
-                              bf16_bits(st.o[c][2] * inv), bf16_bits(st.o[c][3] * inv)};
-      *reinterpret_cast<short4v*>(op + c * 16) = packed;
+    for (int i = 0; i < CW; ++i) {
+      const int c = wave + NW * i;
+      const float4v y = o_w[i][0] * inv;
+      const short4v packed = {bf16_bits(y[0]), bf16_bits(y[1]), bf16_bits(y[2]), bf16_bits(y[3])};
+      if (c < DCH) *reinterpret_cast<short4v*>(op + c * 16) = packed;
     }
     return;
   }
@@ -335,8 +342,11 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(
     const int64_t slot = ((int64_t)e * q_heads + head) * splits + split;
     float* po = part_o + slot * D + 4 * grp;
 #pragma unroll
-    for (int c = 0; c < DCH; ++c) *reinterpret_cast<float4v*>(po + c * 16) = st.o[c];
-    if (grp == 0) {
+    for (int i = 0; i < CW; ++i) {
+      const int c = wave + NW * i;
+      if (c < DCH) *reinterpret_cast<float4v*>(po + c * 16) = o_w[i][0];
+    }
+    if (wave == 0 && grp == 0) {
       part_ml[slot * 2] = m_all;
       part_ml[slot * 2 + 1] = l_all;
     }
@@ -354,12 +364,17 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(
     const int64_t slot = ((int64_t)e * q_heads + head) * splits + split;
     const __amdgpu_buffer_rsrc_t po = device_scope_buffer(part_o);
 #pragma unroll
-    for (int c = 0; c < DCH; ++c) device_store4(po, (unsigned)((slot * D + 4 * grp + c * 16) * 4), st.o[c]);
-    if (grp == 0) device_store2(device_scope_buffer(part_ml), (unsigned)(slot * 2 * 4), merge_float2{m_all, l_all});
+    for (int i = 0; i < CW; ++i) {
+      const int c = wave + NW * i;
+      if (c < DCH) device_store4(po, (unsigned)((slot * D + 4 * grp + c * 16) * 4), o_w[i][0]);
+    }
+    if (wave == 0 && grp == 0) device_store2(device_scope_buffer(part_ml), (unsigned)(slot * 2 * 4), merge_float2{m_all, l_all});
   }
-  // every store of this wave has been acknowledged before the count goes up ...
+  // every store of every wave has been acknowledged before the count goes up ...
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (wave != 0) return;
   unsigned* counter = arrivals + (int64_t)e * gridDim.y + blockIdx.y;
   unsigned before = 0;
   if (lane == 0) before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1102,17 +1117,25 @@ static int attention_decode(const void* q, int64_t q_stride, const void* k_pages
       (splits > 1 && (part_o == nullptr || part_ml == nullptr)) || q_stride % 4 != 0 ||
       out_stride % 4 != 0)
     return DLI_ERR_ARGUMENT;
-  const int head_tiles = (q_heads / kv_heads + 15) / 16;
+  const int group = q_heads / kv_heads, head_tiles = (group + 15) / 16;
   const dim3 grid(splits, kv_heads * head_tiles, requests);
   // with counters the last workgroup of each (request, kv head, head tile) merges
   const bool self_merging = merge && arrivals != nullptr && splits >= 2 && splits <= MERGE_SPLITS;
   unsigned* counters = self_merging ? arrivals : nullptr;
-#define DECODE_CASE(N)                                                                            \
-  case N:                                                                                         \
-    attention_decode_kernel<N><<<grid, 256, 0, stream>>>(                                         \
+  // Eight waves where every workgroup has a compute unit to itself: few keys then need no second run, whose merge costs more than
+  // it saves (planned_splits has the figures); with more workgroups four, of which several share a unit. The waves' states
+  // have to fit LDS.
+  const size_t lds = (size_t)4 * (head_dim / 16) * 4 * (group < 16 ? group : 16) * sizeof(float4v);  // of four waves
+  const bool eight = (int64_t)splits * kv_heads * head_tiles * requests <= dli_compute_units() && 2 * lds <= 48 * 1024;
+#define DECODE_LAUNCH(N, NW)                                                                      \
+    attention_decode_kernel<N, NW><<<grid, NW * 64, lds * (NW / 4), stream>>>(                     \
         (const bf16_t*)q, q_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages, (bf16_t*)out, \
-        out_stride, part_o, part_ml, kv_len, block_tables, table_stride, q_heads, kv_heads,       \
-        page_size, scale * LOG2E, window, splits, counters);                                      \
+        out_stride, part_o, part_ml, kv_len, block_tables, table_stride, q_heads, kv_heads, group, \
+        head_tiles, page_size, page_of_tile(page_size), scale * LOG2E, window, splits, counters)
+#define DECODE_CASE(N)                     \
+  case N:                                  \
+    if (eight) DECODE_LAUNCH(N, 8);        \
+    else DECODE_LAUNCH(N, 4);              \
     break;
   switch (head_dim / 16) {
     DECODE_CASE(1) DECODE_CASE(2) DECODE_CASE(3) DECODE_CASE(4)
@@ -1120,6 +1143,7 @@ static int attention_decode(const void* q, int64_t q_stride, const void* k_pages
     default: return DLI_ERR_ARGUMENT;
   }
 #undef DECODE_CASE
+#undef DECODE_LAUNCH
   if (dli_launch_status() != DLI_OK) return DLI_ERR_LAUNCH;
   if (splits > 1 && merge && !self_merging) {
     const int pairs = requests * q_heads;

@@ -98,6 +98,19 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
   return total;
 }
 
+// Page of a tile of sixteen keys, page size in tiles. A quotient by a number that the compiler does not know costs some
+// twenty instructions, eight cycles each where one waits for the other, and an attention kernel's waves need several of them
+// before their first keys are asked for: so the host hands over 2^32 / tiles, rounded up, whose product's upper
+// half is the quotient for every tile below 2^32 / tiles.
+struct PageOf {
+  unsigned tiles, reciprocal;
+  __device__ __forceinline__ unsigned page(unsigned tile) const { return tiles == 1 ? tile : __umulhi(tile, reciprocal); }
+};
+static inline PageOf page_of_tile(int page_size) {
+  const unsigned tiles = (unsigned)page_size / 16;
+  return PageOf{tiles, tiles > 1 ? (unsigned)((0x100000000ull + tiles - 1) / tiles) : 0u};
+}
+
 static inline int dli_launch_status() {
   return hipGetLastError() == hipSuccess ? DLI_OK : DLI_ERR_LAUNCH;
 }

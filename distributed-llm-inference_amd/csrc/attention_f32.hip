@@ -102,8 +102,7 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_f32_kernel(
       s[e] = seen ? s[e] : -INFINITY;
       top = fmaxf(top, s[e]);
     }
-    top = fmaxf(top, __shfl_xor(top, 16, DLI_WAVE));
-    top = fmaxf(top, __shfl_xor(top, 32, DLI_WAVE));
+    top = max_across32(max_across16(top));
     const float m_new = fmaxf(m, top);
     float alpha = 1.f;
     af4 p = {0.f, 0.f, 0.f, 0.f};
@@ -127,8 +126,7 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_f32_kernel(
 #pragma unroll
       for (int t = 0; t < DT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(fv[t][e], p[e], acc[t], 0, 0, 0);
   }
-  l += __shfl_xor(l, 16, DLI_WAVE);
-  l += __shfl_xor(l, 32, DLI_WAVE);
+  l = add_across32(add_across16(l));
   if (g == 0) {
     ms[wave][i] = m;
     ls[wave][i] = l;

@@ -594,7 +594,8 @@ static int attention_scored(const void* q, int64_t q_stride, const void* k_pages
       if ((int64_t)tiles * splits > 0x7fffffff) return DLI_ERR_ARGUMENT;
       const SinglesArgs a = {(const bf16_t*)q, q_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages, (bf16_t*)out, out32, out_stride,
                              kv_len, block_tables, table_stride, q_heads, kv_heads, v_heads, head_dim, value_dim, page_size, scale,
-                             window, chunk, keep_first, sink, r1, r2, sinks, gate, gate_stride, parts, splits};
+                             window, chunk, keep_first, sink, r1, r2, sinks, gate, gate_stride, parts, splits,
+                             group, (group + 15) / 16, page_of_tile(page_size)};
       const int status = attention_singles(a, tiles, stream);
       if (status != DLI_OK || splits == 1) return status;
       attention_scored_merge_kernel<bf16_t><<<dim3(tiles, q_heads), value_dim <= 64 ? 64 : 128, 0, stream>>>(

@@ -168,8 +168,7 @@ __global__ __launch_bounds__(256, DC <= 12 ? 2 : 1) void attention_keyvalue_kern
 #pragma unroll
         for (int i = 0; i < 4; ++i) mx = scale2 >= 0.f ? fmaxf(mx, s[sub][i]) : fminf(mx, s[sub][i]);
       mx *= scale2;
-      mx = fmaxf(mx, __shfl_xor(mx, 16, DLI_WAVE));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, DLI_WAVE));
+      mx = max_across32(max_across16(mx));
       const float m_new = fmaxf(m_run, mx);
       const float m_safe = m_new > -INFINITY ? m_new : 0.f;            // (nothing seen yet: every weight is exp2(-inf))
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_safe);
@@ -239,8 +238,7 @@ __global__ __launch_bounds__(256, DC <= 12 ? 2 : 1) void attention_keyvalue_kern
       }
     }
   }
-  float l = l_run + __shfl_xor(l_run, 16, DLI_WAVE);
-  l += __shfl_xor(l, 32, DLI_WAVE);
+  const float l = add_across32(add_across16(l_run));
   if (!live) return;
   // acc[v][i] is value 16 v + 4 grp + i of this lane's row
   if (a.splits > 1) {

@@ -108,8 +108,7 @@ __global__ __launch_bounds__(256) void attention_scored_mfma_kernel(ScoredArgs a
         s[sub][i] = x;
         mx = fmaxf(mx, x);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, DLI_WAVE));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, DLI_WAVE));
+    mx = max_across32(max_across16(mx));
     const float m_new = fmaxf(m_run, mx);
     const bool any = m_new > -INFINITY;
     const float alpha = any ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.f;
@@ -139,8 +138,7 @@ __global__ __launch_bounds__(256) void attention_scored_mfma_kernel(ScoredArgs a
                                                           pb[sub], acc[t], 0, 0, 0);
     }
   }
-  float l = l_run + __shfl_xor(l_run, 16, DLI_WAVE);
-  l += __shfl_xor(l, 32, DLI_WAVE);
+  const float l = add_across32(add_across16(l_run));
   if (!q_live) return;
   const float inv = l > 0.f ? 1.f / l : 0.f;
   // acc[t][i] is value 16 t + 4 grp + i of query `col`: four neighbours in the output row

@@ -12,6 +12,7 @@ struct SinglesArgs {
   float scale; int window, chunk, keep_first, sink;
   const float *r1, *r2, *sinks, *gate; int64_t gate_stride;
   float* parts; int splits;                    // splits > 1: [entries][q_heads][splits][V + 2], to be merged
+  int group, head_tiles; PageOf page_of;       // q_heads / kv_heads, its tiles of 16, the page of a tile of 16 keys
 };
 
 bool attention_singles_takes(const void* q, int64_t q_stride, const void* k_pages, const void* v_pages, int head_dim, int value_dim,

@@ -22,8 +22,7 @@ typedef short as_s4 __attribute__((ext_vector_type(4)));
 typedef float as_f4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float as_column_max(float v) {   // over the four lanes that share a column
-  v = fmaxf(v, __shfl_xor(v, 16, DLI_WAVE));
-  return fmaxf(v, __shfl_xor(v, 32, DLI_WAVE));
+  return max_across32(max_across16(v));
 }
 
 template <int DCH, int VCH, bool PEN>   // keys of up to 16 DCH components, values of up to 16 VCH; with r1 and r2
@@ -32,9 +31,12 @@ __global__ __launch_bounds__(256) void attention_singles_kernel(SinglesArgs a) {
   __shared__ __attribute__((aligned(16))) float sm_o[4][16][16 * VCH + 4];
   __shared__ float sm_m[4][16], sm_l[4][16];
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), col = lane % 16, grp = lane / 16;
-  const int entry = blockIdx.x / a.splits, split = blockIdx.x % a.splits;
-  const int group = a.q_heads / a.kv_heads, head_tiles = (group + 15) / 16;
-  const int kvh = blockIdx.y / head_tiles, vh = kvh % a.v_heads, in_group = blockIdx.y % head_tiles * 16 + col;
+  // (quotients by numbers that the compiler does not know cost some twenty instructions each before the first key is asked for:
+  // the host makes them, and what is one in most calls is not divided by)
+  const int entry = a.splits == 1 ? blockIdx.x : blockIdx.x / a.splits, split = blockIdx.x - entry * a.splits;
+  const int group = a.group, head_tiles = a.head_tiles;
+  const int kvh = head_tiles == 1 ? blockIdx.y : blockIdx.y / head_tiles, head_tile = blockIdx.y - kvh * head_tiles;
+  const int vh = a.v_heads == a.kv_heads ? kvh : kvh % a.v_heads, in_group = head_tile * 16 + col;
   const bool valid = in_group < group;
   const int head = kvh * group + min(in_group, group - 1), nd = a.D / 16, nv = a.V / 16, ps = a.page_size;
   const int pos = a.kv_len[entry] - 1;
@@ -57,7 +59,7 @@ __global__ __launch_bounds__(256) void attention_singles_kernel(SinglesArgs a) {
 #pragma unroll
   for (int c = 0; c < VCH; ++c) acc[c] = as_f4{0.f, 0.f, 0.f, 0.f};
 
-  const int j_lo = a.chunk > 0 ? max(pos, 0) / a.chunk * a.chunk : 0;            // nothing before it is seen
+  const int j_lo = a.chunk > 0 && pos >= a.chunk ? pos / a.chunk * a.chunk : 0;   // nothing before it is seen
   const int j_begin = a.window > 0 ? max(j_lo, pos - a.window + 1) : j_lo;
   const int keep = a.window > 0 ? a.keep_first : 0;                              // keys below it are seen from any distance
   // the tiles that hold something visible: those of the kept keys that lie before the window's, then the window's
@@ -68,15 +70,14 @@ __global__ __launch_bounds__(256) void attention_singles_kernel(SinglesArgs a) {
   const auto first_key = [&](int b) { return (b < n_keep ? j_lo / 16 + b : t_win + b - n_keep) * 16; };
   struct Pair { as_s4 k[2][DCH], v[2][VCH]; };
   struct Place { int page[2], off[2]; };
-  const unsigned page_tiles = ps / 16, magic = (0x80000000u + page_tiles - 1) / page_tiles;   // (exact: up to 16 tiles a page)
   const unsigned lane_k = col * a.D + 4 * grp, lane_v = col * ps + 4 * grp;
   const auto look = [&](int b) {   // (a page that a window has passed: any page, its keys are not seen)
     Place at;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const int tile = first_key(min(b + u, n_all - 1)) / 16, nth = (int)(((uint64_t)(unsigned)tile * magic) >> 31);
+      const int tile = first_key(min(b + u, n_all - 1)) / 16, nth = (int)a.page_of.page((unsigned)tile);
       at.page[u] = __builtin_amdgcn_readfirstlane(max(table[min(nth, a.table_stride - 1)], 0));
-      at.off[u] = (tile - nth * (int)page_tiles) * 16;
+      at.off[u] = (tile - nth * (int)a.page_of.tiles) * 16;
     }
     return at;
   };
@@ -162,8 +163,7 @@ __global__ __launch_bounds__(256) void attention_singles_kernel(SinglesArgs a) {
       p1 = look(b + 5 * stride);
     }
   }
-  l += __shfl_xor(l, 16, DLI_WAVE);
-  l += __shfl_xor(l, 32, DLI_WAVE);
+  l = add_across32(add_across16(l));
   if (grp == 0) {
     sm_m[wave][col] = m;
     sm_l[wave][col] = l;
@@ -172,9 +172,9 @@ __global__ __launch_bounds__(256) void attention_singles_kernel(SinglesArgs a) {
   for (int c = 0; c < VCH; ++c) *reinterpret_cast<as_f4*>(&sm_o[wave][col][16 * c + 4 * grp]) = acc[c];
   __syncthreads();
   // four neighbouring values of a head a thread
-  const int quads = a.V / 4, heads = min(16, group - blockIdx.y % head_tiles * 16);
+  const int quads = a.V / 4, heads = min(16, group - head_tile * 16);
   for (int idx = threadIdx.x; idx < heads * quads; idx += 256) {
-    const int h = idx / quads, v0 = idx % quads * 4, out_head = kvh * group + blockIdx.y % head_tiles * 16 + h;
+    const int h = idx / quads, v0 = idx % quads * 4, out_head = kvh * group + head_tile * 16 + h;
     float top = sm_m[0][h], sum = 0.f;
 #pragma unroll
     for (int w = 1; w < 4; ++w) top = fmaxf(top, sm_m[w][h]);
@@ -240,7 +240,7 @@ static void launch_singles(const SinglesArgs& a, const dim3& grid, hipStream_t s
 }
 
 int attention_singles(const SinglesArgs& a, int entries, hipStream_t stream) {
-  const dim3 grid(entries * a.splits, a.kv_heads * ((a.q_heads / a.kv_heads + 15) / 16));
+  const dim3 grid(entries * a.splits, a.kv_heads * a.head_tiles);
   if (grid.y > 65535) return DLI_ERR_ARGUMENT;
   if (a.D <= 32) launch_singles<2>(a, grid, stream);
   else if (a.D <= 64) launch_singles<4>(a, grid, stream);

@@ -51,17 +51,6 @@ __device__ __forceinline__ bf16_t glu_bf16(float gate, float up, const GluForm& 
   return (bf16_t)((float)(bf16_t)silu<bf16_t>(gate) * up);
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int m = DLI_WAVE / 2; m > 0; m >>= 1) v += __shfl_xor(v, m, DLI_WAVE);
-  return v;
-}
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int m = DLI_WAVE / 2; m > 0; m >>= 1) v = fmaxf(v, __shfl_xor(v, m, DLI_WAVE));
-  return v;
-}
-
 // Exchanges between lanes without a trip through LDS (all lanes of the wave take part).
 template <int SHIFT>
 __device__ __forceinline__ float row_ror(float v) {  // rotated by SHIFT within each row of sixteen lanes
@@ -83,6 +72,40 @@ __device__ __forceinline__ float add_halves(float a, float b) {
 __device__ __forceinline__ float add_rows(float a, float b) {
   const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
   return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+
+// v[l] + v[l^32] and v[l] + v[l^16] in every lane, and the larger of the two
+__device__ __forceinline__ float add_across32(float v) { return add_halves(v, v); }
+__device__ __forceinline__ float add_across16(float v) { return add_rows(v, v); }
+__device__ __forceinline__ float max_across32(float v) {
+  const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(s[0]), __uint_as_float(s[1]));
+}
+__device__ __forceinline__ float max_across16(float v) {
+  const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(s[0]), __uint_as_float(s[1]));
+}
+template <int MASK>
+__device__ __forceinline__ float quad_xor(float v) {  // the value of lane l ^ MASK, MASK 1 or 2
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), MASK == 1 ? 0xb1 : 0x4e, 0xf, 0xf, true));
+}
+
+// Sum and maximum over the wave, the same in every lane, by exchanges with the lanes l ^ 32, 16, 8, 4, 2, 1 in this order (once the
+// first three are done a value repeats every eight lanes, and a rotation by four is the exchange with l ^ 4). All in registers: six
+// exchanges through LDS, one after the other, take 0.3 us.
+__device__ __forceinline__ float wave_sum(float v) {
+  v = add_across16(add_across32(v));
+  v += row_ror<8>(v);
+  v += row_ror<4>(v);
+  v += quad_xor<2>(v);
+  return v + quad_xor<1>(v);
+}
+__device__ __forceinline__ float wave_max(float v) {
+  v = max_across16(max_across32(v));
+  v = fmaxf(v, row_ror<8>(v));
+  v = fmaxf(v, row_ror<4>(v));
+  v = fmaxf(v, quad_xor<2>(v));
+  return fmaxf(v, quad_xor<1>(v));
 }
 
 // Sum over a block of up to 1024 threads; every thread gets the result. `scratch` holds 16 floats.

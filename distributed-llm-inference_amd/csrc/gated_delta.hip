@@ -438,8 +438,7 @@ __global__ __launch_bounds__(64) void gated_delta_scan_kernel(GdArgs p) {
     for (int t = lane >> 2; t < TB; t += 16) {
       float kq = 0.f;
       for (int c = (lane & 3) * (D / 4); c < ((lane & 3) + 1) * (D / 4); ++c) kq = fmaf(sk[t * D + c], sq[t * D + c], kq);
-      kq += __shfl_xor(kq, 1, DLI_WAVE);
-      kq += __shfl_xor(kq, 2, DLI_WAVE);
+      kq = quad_sum(kq);
       if ((lane & 3) == 0) skq[t] = kq;
     }
     __syncthreads();

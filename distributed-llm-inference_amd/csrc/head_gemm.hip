@@ -61,8 +61,7 @@ __global__ __launch_bounds__(HEAD_KS * 64) void head_gemm_kernel(
 #pragma unroll
       for (int u = 0; u < 8; ++u) sum += v[u];
     }
-    sum += __shfl_xor(sum, 16, 64);
-    sum += __shfl_xor(sum, 32, 64);
+    sum = add_across32(add_across16(sum));
     if (grp == 0) rsum[ks][col] = sum;
     __syncthreads();
     float total = 0.f;

@@ -161,8 +161,7 @@ __global__ __launch_bounds__(64) void recurrent_scan_kernel(ScanArgs p) {
       for (int t = lane >> 2; t < TB; t += 16) {
         float kk = 0.f;
         for (int c = (lane & 3) * (D / 4); c < ((lane & 3) + 1) * (D / 4); ++c) kk = fmaf(sk[t * D + c], sk[t * D + c], kk);
-        kk += __shfl_xor(kk, 1, DLI_WAVE);
-        kk += __shfl_xor(kk, 2, DLI_WAVE);
+        kk = quad_sum(kk);
         if ((lane & 3) == 0) skn[t] = 1.f / sqrtf(kk + 1e-6f);
       }
       __syncthreads();

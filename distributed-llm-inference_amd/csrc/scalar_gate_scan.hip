@@ -379,10 +379,8 @@ __global__ __launch_bounds__(256) void scalar_gate_chunk_kernel(SgArgs p, const 
         float sum = 0.f, qn = 0.f;
         for (int s_ = 16 * lk; s_ < 16 * lk + 16; ++s_) sum += s_ <= t ? sP[t * PS + s_] : 0.f;
         for (int d = lk * (D / 4); d < (lk + 1) * (D / 4); ++d) qn = fmaf(sQ[t * DS + d], sN[d], qn);
-        sum += __shfl_xor(sum, 16, DLI_WAVE);
-        sum += __shfl_xor(sum, 32, DLI_WAVE);
-        qn += __shfl_xor(qn, 16, DLI_WAVE);
-        qn += __shfl_xor(qn, 32, DLI_WAVE);
+        sum = add_across32(add_across16(sum));
+        qn = add_across32(add_across16(qn));
         if (lk == 0 && t < nb)
           p.den[(int64_t)(row0 + t0 + t) * p.heads + head] = fmaxf(fabsf(fmaf(expf((float)sA[t]), qn, sum)), sFl[t]) + 1e-6f;
       }

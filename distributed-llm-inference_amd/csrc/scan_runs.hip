@@ -330,8 +330,7 @@ __global__ __launch_bounds__(256) void scan_runs_finish_kernel(RunsArgs p) {
   float sum = 0.f;
 #pragma unroll
   for (int c = 0; c < 4; ++c) sum += (o[c][0] * o[c][0] + o[c][1] * o[c][1]) + (o[c][2] * o[c][2] + o[c][3] * o[c][3]);
-  sum += __shfl_xor(sum, 16, DLI_WAVE);
-  sum += __shfl_xor(sum, 32, DLI_WAVE);
+  sum = add_across32(add_across16(sum));
   const float rn = 1.f / sqrtf(sum / (float)D + p.eps);
   if (t0 + i >= n) return;
 #pragma unroll

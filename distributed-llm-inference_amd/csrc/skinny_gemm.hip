@@ -344,8 +344,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
 #pragma unroll
         for (int u = 0; u < 8; ++u) sum += v[u];
       }
-      sum += __shfl_xor(sum, 16, 64);
-      sum += __shfl_xor(sum, 32, 64);
+      sum = add_across32(add_across16(sum));
       if (grp == 0) rsum[wave][t][col] = sum;
     }
     __syncthreads();
@@ -640,8 +639,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
         }
       }
       if (EPI == EPI_RESIDUAL) {
-        sq += __shfl_xor(sq, 16, 64);
-        sq += __shfl_xor(sq, 32, 64);
+        sq = add_across32(add_across16(sq));
         if (grp == 0 && m < M) ssq_out[(int64_t)tile * M + m] = sq;
       }
     }

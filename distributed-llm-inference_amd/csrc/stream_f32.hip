@@ -39,17 +39,26 @@ template <typename T>
 __global__ void embed_sinusoid_kernel(const T* __restrict__ table, const int* __restrict__ ids,
                                       const int* __restrict__ positions, const float* __restrict__ inv_freq,
                                       float* __restrict__ out, bf16_t* __restrict__ rounded, int width, float scale) {
+  // A thread a pair of values, which share an angle: its sine and cosine cost more than all else here (a row of few is
+  // dealt over gridDim.y workgroups: one of 2,048 values by one workgroup, a value at a time, took 12 us, now 3)
   const int64_t row = blockIdx.x;
   const T* src = table + (int64_t)ids[row] * width;
   const float p = (float)positions[row];
-  for (int i = threadIdx.x; i < width; i += blockDim.x) {
-    float sum = to_f32(src[i]) * scale;
+  for (int i = 2 * (blockIdx.y * blockDim.x + threadIdx.x); i < width; i += 2 * gridDim.y * blockDim.x) {
+    const bool both = i + 1 < width;
+    float s0 = to_f32(src[i]) * scale, s1 = both ? to_f32(src[i + 1]) * scale : 0.f;
     if (inv_freq != nullptr) {   // (nullptr: the token's row alone)
-      const float angle = p * inv_freq[i >> 1];
-      sum += (i & 1) ? cosf(angle) : sinf(angle);
+      float sn, cs;
+      sincosf(p * inv_freq[i >> 1], &sn, &cs);
+      s0 += sn;
+      s1 += cs;
     }
-    out[row * width + i] = sum;
-    if (rounded != nullptr) rounded[row * width + i] = (bf16_t)sum;
+    out[row * width + i] = s0;
+    if (both) out[row * width + i + 1] = s1;
+    if (rounded != nullptr) {
+      rounded[row * width + i] = (bf16_t)s0;
+      if (both) rounded[row * width + i + 1] = (bf16_t)s1;
+    }
   }
 }
 
@@ -415,7 +424,8 @@ __global__ void qk_unit_cache_kernel(const float* __restrict__ proj, int64_t str
   const int slot = slots[row];
   const int64_t page = slot >= 0 ? slot / page_size : 0;
   const int off = slot >= 0 ? slot % page_size : 0;
-  for (int h = wave; h < q_heads + kv_heads; h += waves) {
+  // (a row of a step with few rows is shared by gridDim.y workgroups: 40 heads of one row in turn on four waves took 11 us, now 3)
+  for (int h = blockIdx.y * waves + wave; h < q_heads + kv_heads; h += gridDim.y * waves) {
     const bool is_q = h < q_heads;
     const float* src = is_q ? pr + q_off + (int64_t)h * dim : pr + k_off + (int64_t)(h - q_heads) * dim;
     float ss = 0.f;
@@ -429,7 +439,7 @@ __global__ void qk_unit_cache_kernel(const float* __restrict__ proj, int64_t str
     }
   }
   const float lam = lambda != nullptr ? lambda[0] : 0.f;
-  for (int i = threadIdx.x; i < kv_heads * vdim; i += blockDim.x) {
+  for (int i = blockIdx.y * blockDim.x + threadIdx.x; i < kv_heads * vdim; i += gridDim.y * blockDim.x) {
     float v = pr[v_off + i];
     if (lambda != nullptr) v = (1.f - lam) * v + lam * v_first_in[row * kv_heads * vdim + i];
     if (v_first_out != nullptr) v_first_out[row * kv_heads * vdim + i] = v;
@@ -493,57 +503,95 @@ __global__ __launch_bounds__(256) void rotary_cache_kernel(const float* __restri
   const int off = slot >= 0 ? slot % page_size : 0;
   const int half = rot_dims / 2;
   const bool in_lds = half <= ROTARY_LDS_PAIRS;
+  // (a row of a step with few rows is shared by gridDim.y workgroups)
+  const int at0 = (blockIdx.y * blockDim.x + threadIdx.x) * E, stride0 = gridDim.y * blockDim.x * E;
+  const int elements = (q_heads + kv_heads) * dim;
+  // an element's column of proj, its partner's (the same where it has none) and whether it is its pair's first
+  struct Source { int h, c, at, partner; bool first; };
+  auto source_of = [&](int i) {
+    Source s;
+    s.h = i / dim;
+    s.c = i - s.h * dim;
+    s.at = (s.h < q_heads ? q_off + s.h * dim : k_off + (s.h - q_heads) * dim) + s.c;
+    s.partner = s.at;
+    s.first = true;
+    if (s.c < rot_dims) {
+      if (!interleaved) { s.first = s.c < half; s.partner = s.first ? s.at + half : s.at - half; }
+      else if (E == 1) { s.first = (s.c & 1) == 0; s.partner = s.first ? s.at + 1 : s.at - 1; }
+    }
+    return s;
+  };
+  // this thread's first elements are asked for before the angles are made and the sums meet
+  Source src = source_of(min(at0, elements - E));
+  RotaryElements<E> own = rotary_load<E>(pr + src.at), other = rotary_load<E>(pr + src.partner);
   if (in_lds)
     for (int i = threadIdx.x; i < half; i += blockDim.x) rotary_cos_sin(p, inv_freq[i], &cs_[i], &sn_[i]);
   float rq = 1.f, rk = 1.f;
   if (NORM) {
-    auto rms = [&](int off, int size) {
+    // both sums of a wave, then one exchange between the waves for both
+    auto squares = [&](int off, int size) {   // (HELD rounds asked for together)
+      constexpr int HELD = 2;
       float ss = 0.f;
-      for (int i = threadIdx.x * E; i < size; i += blockDim.x * E) {
-        const RotaryElements<E> x = rotary_load<E>(pr + off + i);
+      for (int i0 = threadIdx.x * E; i0 < size; i0 += HELD * 256 * E) {
+        RotaryElements<E> x[HELD], b[HELD];
 #pragma unroll
-        for (int j = 0; j < E; ++j) {
-          const float v = x.v[j] + (bias != nullptr ? bias[off + i + j] : 0.f);
-          ss += v * v;
+        for (int k = 0; k < HELD; ++k) {
+          const int i = min(i0 + k * 256 * E, size - E);
+          x[k] = rotary_load<E>(pr + off + i);
+#pragma unroll
+          for (int j = 0; j < E; ++j) b[k].v[j] = bias != nullptr ? bias[off + i + j] : 0.f;
         }
+#pragma unroll
+        for (int k = 0; k < HELD; ++k)
+          if (i0 + k * 256 * E < size)
+#pragma unroll
+            for (int j = 0; j < E; ++j) {
+              const float v = x[k].v[j] + b[k].v[j];
+              ss += v * v;
+            }
       }
-      return 1.f / sqrtf(block_sum(ss, scratch) / (float)size + eps);
+      return wave_sum(ss);
     };
-    rq = rms(q_off, q_heads * dim);
-    if (kv_heads > 0) rk = rms(k_off, kv_heads * dim);
+    const float q_sum = squares(q_off, q_heads * dim), k_sum = squares(k_off, kv_heads * dim);
+    if (threadIdx.x % DLI_WAVE == 0) {
+      scratch[threadIdx.x / DLI_WAVE] = q_sum;
+      scratch[8 + threadIdx.x / DLI_WAVE] = k_sum;
+    }
   }
   __syncthreads();
-  // (a row of a step with few rows is shared by gridDim.y workgroups)
-  const int at0 = (blockIdx.y * blockDim.x + threadIdx.x) * E, stride0 = gridDim.y * blockDim.x * E;
-  for (int i = at0; i < (q_heads + kv_heads) * dim; i += stride0) {
-    const int h = i / dim, c = i - h * dim;
-    const bool is_q = h < q_heads;
-    const int64_t at = is_q ? q_off + (int64_t)h * dim : k_off + (int64_t)(h - q_heads) * dim;
-    const float* src = pr + at;
-    const float* bs = bias != nullptr ? bias + at : nullptr;
-    const float r = is_q ? rq : rk;
-    const float* nw = NORM ? (is_q ? q_norm + (int64_t)h * dim : k_norm + (int64_t)(h - q_heads) * dim) : nullptr;
-    auto read = [&](int from) {
-      RotaryElements<E> x = rotary_load<E>(src + from);
-      if (bs != nullptr) {
+  if (NORM) {
+    float tq = 0.f, tk = 0.f;
 #pragma unroll
-        for (int j = 0; j < E; ++j) x.v[j] += bs[from + j];
+    for (int w = 0; w < 256 / DLI_WAVE; ++w) {
+      tq += scratch[w];
+      tk += scratch[8 + w];
+    }
+    rq = 1.f / sqrtf(tq / (float)(q_heads * dim) + eps);
+    if (kv_heads > 0) rk = 1.f / sqrtf(tk / (float)(kv_heads * dim) + eps);
+  }
+  for (int i = at0; i < elements; i += stride0) {
+    const int h = src.h, c = src.c;
+    const bool is_q = h < q_heads, first = src.first;
+    const float r = is_q ? rq : rk;
+    const float* nw = NORM ? (is_q ? q_norm - q_off : k_norm - k_off) : nullptr;   // (a column of proj is its index)
+    auto finish = [&](RotaryElements<E>& x, int at) {
+      if (bias != nullptr) {
+#pragma unroll
+        for (int j = 0; j < E; ++j) x.v[j] += bias[at + j];
       }
       if (NORM) {
 #pragma unroll
-        for (int j = 0; j < E; ++j) x.v[j] = x.v[j] * r * nw[from + j];
+        for (int j = 0; j < E; ++j) x.v[j] = x.v[j] * r * nw[at + j];
       }
-      return x;
     };
-    RotaryElements<E> y = read(c);
+    RotaryElements<E> y = own;
+    finish(y, src.at);
     if (c < rot_dims) {
-      RotaryElements<E> other;
-      bool first = true;
-      if (!interleaved) { first = c < half; other = read(first ? c + half : c - half); }
-      else if (E == 1) { first = (c & 1) == 0; other = read(c ^ 1); }
-      else {
+      if (interleaved && E > 1) {
 #pragma unroll
         for (int j = 0; j < E; ++j) other.v[j] = y.v[j ^ 1];
+      } else {
+        finish(other, src.partner);
       }
 #pragma unroll
       for (int j = 0; j < E; ++j) {
@@ -561,6 +609,11 @@ __global__ __launch_bounds__(256) void rotary_cache_kernel(const float* __restri
       rotary_store<T, E>(q_out + (row * q_heads + h) * dim + c, y.v);
     } else if (slot >= 0) {
       rotary_store<T, E>(k_pages + ((page * kv_heads + (h - q_heads)) * page_size + off) * dim + c, y.v);
+    }
+    if (i + stride0 < elements) {
+      src = source_of(i + stride0);
+      own = rotary_load<E>(pr + src.at);
+      other = rotary_load<E>(pr + src.partner);
     }
   }
   if (slot >= 0)
@@ -850,12 +903,13 @@ int dli_embed_sinusoid(const void* table, const int* ids, const int* positions, 
                        void* rounded_bf16, int rows, int width, float scale, int is_bf16, hipStream_t stream) {
   if (rows <= 0) return DLI_OK;
   if (width <= 0) return DLI_ERR_ARGUMENT;
-  const int threads = width >= 1024 ? 256 : 128;
+  const int threads = width >= 1024 ? 256 : 128, shares = (width + 2 * threads - 1) / (2 * threads);
+  const dim3 grid(rows, rows >= 128 ? 1 : (unsigned)(shares < 16 ? shares : 16));
   if (is_bf16)
-    embed_sinusoid_kernel<bf16_t><<<rows, threads, 0, stream>>>((const bf16_t*)table, ids, positions, inv_freq, out,
+    embed_sinusoid_kernel<bf16_t><<<grid, threads, 0, stream>>>((const bf16_t*)table, ids, positions, inv_freq, out,
                                                                 (bf16_t*)rounded_bf16, width, scale);
   else
-    embed_sinusoid_kernel<float><<<rows, threads, 0, stream>>>((const float*)table, ids, positions, inv_freq, out,
+    embed_sinusoid_kernel<float><<<grid, threads, 0, stream>>>((const float*)table, ids, positions, inv_freq, out,
                                                                (bf16_t*)rounded_bf16, width, scale);
   return dli_launch_status();
 }
@@ -981,12 +1035,14 @@ int dli_qk_unit_cache(const float* proj, int64_t stride, int q_off, int k_off, i
   if (q_heads <= 0 || kv_heads <= 0 || dim <= 0 || vdim <= 0 || page_size <= 0 ||
       (lambda != nullptr && v_first_in == nullptr))
     return DLI_ERR_ARGUMENT;
+  const int shares = (q_heads + kv_heads + 3) / 4;
+  const dim3 grid(rows, rows >= 128 ? 1 : (unsigned)(shares < 32 ? shares : 32));
   if (is_bf16)
-    qk_unit_cache_kernel<bf16_t><<<rows, 256, 0, stream>>>(proj, stride, q_off, k_off, v_off, (bf16_t*)q_out, lambda,
+    qk_unit_cache_kernel<bf16_t><<<grid, 256, 0, stream>>>(proj, stride, q_off, k_off, v_off, (bf16_t*)q_out, lambda,
                                                            v_first_in, v_first_out, slots, (bf16_t*)k_pages,
                                                            (bf16_t*)v_pages, q_heads, kv_heads, dim, vdim, page_size, eps);
   else
-    qk_unit_cache_kernel<float><<<rows, 256, 0, stream>>>(proj, stride, q_off, k_off, v_off, (float*)q_out, lambda,
+    qk_unit_cache_kernel<float><<<grid, 256, 0, stream>>>(proj, stride, q_off, k_off, v_off, (float*)q_out, lambda,
                                                           v_first_in, v_first_out, slots, (float*)k_pages,
                                                           (float*)v_pages, q_heads, kv_heads, dim, vdim, page_size, eps);
   return dli_launch_status();

@@ -89,8 +89,8 @@ __global__ void rms_norm_vec_kernel(const T* x, const T* __restrict__ delta,
       }
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const float f = to_f32((T)v[i]);
-        ss += f * f;
+        const float f = to_f32((T)v[i]);   // (fused, in this order, in the 32-bit products that make the norm themselves too)
+        ss = fmaf(f, f, ss);
       }
     }
     const float r = rsqrtf(block_sum(ss, scratch) / (float)width + eps);
@@ -114,7 +114,7 @@ __global__ void rms_norm_vec_kernel(const T* x, const T* __restrict__ delta,
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const float f = to_f32((T)v[i]);
-      ss += f * f;
+      ss = fmaf(f, f, ss);
     }
   }
   const float r = rsqrtf(block_sum(ss, scratch) / (float)width + eps);

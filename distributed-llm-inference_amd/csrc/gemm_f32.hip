@@ -37,6 +37,22 @@ struct GfArgs {
   int segments, seg_runs;   // the sum's order: `segments` of `seg_runs` runs each (the last may be shorter)
 };
 
+// What a few-row product of the recorded decode steps takes in besides: the norm before it, and what follows it.
+#define GF_PLAIN 0
+#define GF_GLU 1    // silu(gate) * up: the first half of w's rows are gates, the second ups
+#define GF_ROPE 2   // q, k and v heads: q and k rotated (the pairs i, i + head_dim / 2), k and v written at their slots
+struct GfAround {
+  const float* norm_w;
+  float eps;
+  int norm_waves;   // waves of the norm's own kernel, whose order of sums this one keeps
+  const int* positions;
+  const float* inv_freq;
+  const int* slots;
+  float* k_pages;
+  float* v_pages;
+  int q_heads, kv_heads, head_dim, page_size;
+};
+
 struct Zero { static constexpr int value = 0; };
 struct One { static constexpr int value = 1; };
 
@@ -74,16 +90,38 @@ __device__ __forceinline__ void gf_store(const GfArgs& p, gf4 sum, int m0, int n
 // Up to 16 rows: KW waves share a tile of 16 x 16 NT and take its segments in turn, each straight from memory: half a run's
 // operands are on their way while the other half is multiplied. (The lanes of a load lie in 16 rows, four neighbours in
 // four of them: as fast as any order where w comes from HBM once, but a quarter of the caches' rate where tiles share it.)
-template <int NT, int KW, bool VEC>
-__global__ __launch_bounds__(64 * KW) void gemm_f32_few_kernel(GfArgs p) {
+//
+// FORM GF_GLU and GF_ROPE: the rows are normalised on their way to the matrix cores and the sums go on where they are, so that a
+// decode step's norms, activations and rotations are no kernels of their own (each 2.8 to 3.9 us of a step of two rows, which
+// this one's 5 to 6 outlasts by less than one; two prompts of 333 and 178 tokens and four steps at the 135M sizes:
+// 9.00 -> 8.06 ms a pass). A tile's sixteen columns are then eight of one half and the eight that they are paired with, a rotation
+// by eight lanes away. The norm's sum of squares and its products are those of its own kernel, bit for bit: a wave takes a row,
+// after the first weights are asked for.
+template <int NT, int KW, bool VEC, int FORM = GF_PLAIN>
+__global__ __launch_bounds__(64 * KW) void gemm_f32_few_kernel(GfArgs p, GfAround x) {
+  static_assert(FORM == GF_PLAIN || (NT == 1 && VEC), "one tile of whole vectors");
   extern __shared__ gf4 gf_sums[];   // [segments][NT][64]
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, i = lane % 16, g = lane / 16;
-  const int n0 = blockIdx.x * 16 * NT;
+  __shared__ float rstd[16];
+  int n0 = blockIdx.x * 16 * NT;
   const float* ra = p.a + (int64_t)min(i, p.m - 1) * p.lda;   // (rows past the end: not stored)
   const float* rw[NT];
 #pragma unroll
   for (int y = 0; y < NT; ++y) rw[y] = p.w + (int64_t)min(n0 + 16 * y + i, p.n - 1) * p.ldw;
-  gf4 seg[NT], acc[NT], fa[2][4], fw[2][4][NT];
+  int feature = n0 + i, head = 0;   // this lane's row of w
+  bool rotates = false;
+  if constexpr (FORM == GF_GLU) {
+    n0 = blockIdx.x * 8;
+    feature = (i < 8 ? 0 : p.n / 2) + min(n0 + i % 8, p.n / 2 - 1);
+  }
+  if constexpr (FORM == GF_ROPE) {
+    const int tiles = x.head_dim / 16, t = blockIdx.x % tiles;
+    head = blockIdx.x / tiles;
+    rotates = head < x.q_heads + x.kv_heads;
+    feature = head * x.head_dim + (rotates ? 8 * t + i % 8 + (i < 8 ? 0 : x.head_dim / 2) : 16 * t + i);
+  }
+  if constexpr (FORM != GF_PLAIN) rw[0] = p.w + (int64_t)feature * p.ldw;
+  gf4 seg[NT], acc[NT], fa[2][4], fw[2][4][NT], fn[2][FORM != GF_PLAIN ? 4 : 1];
 #pragma unroll
   for (int y = 0; y < NT; ++y) seg[y] = gf4{0.f, 0.f, 0.f, 0.f};
 
@@ -93,6 +131,7 @@ __global__ __launch_bounds__(64 * KW) void gemm_f32_few_kernel(GfArgs p) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         fa[b][t] = *reinterpret_cast<const gf4*>(ra + k0 + 4 * g + 16 * t);
+        if constexpr (FORM != GF_PLAIN) fn[b][t] = *reinterpret_cast<const gf4*>(x.norm_w + k0 + 4 * g + 16 * t);
 #pragma unroll
         for (int y = 0; y < NT; ++y) fw[b][t][y] = *reinterpret_cast<const gf4*>(rw[y] + k0 + 4 * g + 16 * t);
       }
@@ -101,12 +140,17 @@ __global__ __launch_bounds__(64 * KW) void gemm_f32_few_kernel(GfArgs p) {
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       fa[b][t] = gf_load<VEC>(ra, k0 + 16 * t + 4 * g, p.k);
+      if constexpr (FORM != GF_PLAIN) fn[b][t] = gf_load<VEC>(x.norm_w, k0 + 16 * t + 4 * g, p.k);
 #pragma unroll
       for (int y = 0; y < NT; ++y) fw[b][t][y] = gf_load<VEC>(rw[y], k0 + 16 * t + 4 * g, p.k);
     }
   };
+  float r = 1.f;
   const auto multiply = [&](auto half) {
     constexpr int b = decltype(half)::value;
+    if constexpr (FORM != GF_PLAIN)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) fa[b][t] = fn[b][t] * (fa[b][t] * r);
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -121,13 +165,51 @@ __global__ __launch_bounds__(64 * KW) void gemm_f32_few_kernel(GfArgs p) {
     load(Zero{}, s * p.seg_runs * GF_RUN);
     left = min(p.seg_runs, runs - s * p.seg_runs);
   }
-  for (int r = s * p.seg_runs; s < p.segments;) {   // run r of segment s, `left` runs of it to go
+  gf4 c = {1.f, 1.f, 1.f, 1.f}, sn = {0.f, 0.f, 0.f, 0.f};
+  int slot[4] = {-1, -1, -1, -1};
+  if constexpr (FORM != GF_PLAIN) {
+    for (int row = wave; row < p.m; row += KW) {
+      const float* xr = p.a + (int64_t)row * p.lda;
+      float ss = 0.f;
+      for (int j = 0; j < x.norm_waves; ++j) {
+        float part = 0.f;
+        for (int at = (64 * j + lane) * 8; at < p.k; at += 512 * x.norm_waves) {
+          const gf4 lo = *reinterpret_cast<const gf4*>(xr + at), hi = *reinterpret_cast<const gf4*>(xr + at + 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) part = fmaf(lo[e], lo[e], part);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) part = fmaf(hi[e], hi[e], part);
+        }
+        ss += wave_sum(part);
+      }
+      if (lane == 0) rstd[row] = rsqrtf(ss / (float)p.k + x.eps);
+    }
+    if constexpr (FORM == GF_ROPE) {
+      if (wave == 0) {   // the wave that ends the tile
+        const float freq = rotates ? x.inv_freq[feature % x.head_dim % (x.head_dim / 2)] : 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (4 * g + e >= p.m) continue;
+          slot[e] = x.slots[4 * g + e];
+          if (rotates) {
+            float sine, cosine;
+            sincosf((float)x.positions[4 * g + e] * freq, &sine, &cosine);
+            c[e] = cosine;
+            sn[e] = i < 8 ? -sine : sine;
+          }
+        }
+      }
+    }
+    __syncthreads();
+    r = rstd[min(i, p.m - 1)];
+  }
+  for (int u = s * p.seg_runs; s < p.segments;) {   // run u of segment s, `left` runs of it to go
 #pragma unroll
     for (int y = 0; y < NT; ++y) acc[y] = gf4{0.f, 0.f, 0.f, 0.f};
-    load(One{}, r * GF_RUN + GF_RUN / 2);
+    load(One{}, u * GF_RUN + GF_RUN / 2);
     multiply(Zero{});
     const bool last = --left == 0;
-    const int s_next = last ? s + KW : s, r_next = last ? s_next * p.seg_runs : r + 1;
+    const int s_next = last ? s + KW : s, r_next = last ? s_next * p.seg_runs : u + 1;
     if (s_next < p.segments) load(Zero{}, r_next * GF_RUN);
     multiply(One{});
 #pragma unroll
@@ -140,7 +222,7 @@ __global__ __launch_bounds__(64 * KW) void gemm_f32_few_kernel(GfArgs p) {
     }
     if (last && s_next < p.segments) left = min(p.seg_runs, runs - r_next);
     s = s_next;
-    r = r_next;
+    u = r_next;
   }
   __syncthreads();
 #pragma unroll
@@ -148,7 +230,33 @@ __global__ __launch_bounds__(64 * KW) void gemm_f32_few_kernel(GfArgs p) {
     if (y % KW != wave) continue;
     gf4 sum = gf4{0.f, 0.f, 0.f, 0.f};
     for (int c = 0; c < p.segments; ++c) sum += gf_sums[(c * NT + y) * 64 + lane];
-    gf_store(p, sum, 0, n0 + 16 * y, i, g);
+    if constexpr (FORM == GF_PLAIN) {
+      gf_store(p, sum, 0, n0 + 16 * y, i, g);
+      continue;
+    }
+    if (p.bias != nullptr) sum += p.bias[feature];
+    gf4 other;   // the tile's other half (all lanes take part)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) other[e] = row_ror<8>(sum[e]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int row = 4 * g + e;
+      if (row >= p.m) continue;
+      if constexpr (FORM == GF_GLU) {
+        if (i < 8 && n0 + i < p.n / 2) p.out[(int64_t)row * p.ldo + n0 + i] = silu<float>(sum[e]) * other[e];
+      } else {
+        const float v = rotates ? sum[e] * c[e] + other[e] * sn[e] : sum[e];
+        const int d = feature - head * x.head_dim;
+        if (head < x.q_heads) {
+          p.out[(int64_t)row * p.ldo + feature] = v;
+        } else if (slot[e] >= 0) {
+          const int64_t page = slot[e] / x.page_size;
+          const int off = slot[e] % x.page_size;
+          if (rotates) x.k_pages[((page * x.kv_heads + head - x.q_heads) * x.page_size + off) * x.head_dim + d] = v;
+          else x.v_pages[((page * x.kv_heads + head - x.q_heads - x.kv_heads) * x.head_dim + d) * x.page_size + off] = v;
+        }
+      }
+    }
   }
 }
 
@@ -298,8 +406,19 @@ template <int NT, int KW>
 static int gf_few(const GfArgs& p, bool vec, hipStream_t stream) {
   const int grid = (p.n + 16 * NT - 1) / (16 * NT);
   const size_t lds = (size_t)p.segments * NT * 64 * sizeof(gf4);   // at most 32 KiB
-  if (vec) gemm_f32_few_kernel<NT, KW, true><<<grid, 64 * KW, lds, stream>>>(p);
-  else gemm_f32_few_kernel<NT, KW, false><<<grid, 64 * KW, lds, stream>>>(p);
+  if (vec) gemm_f32_few_kernel<NT, KW, true><<<grid, 64 * KW, lds, stream>>>(p, GfAround{});
+  else gemm_f32_few_kernel<NT, KW, false><<<grid, 64 * KW, lds, stream>>>(p, GfAround{});
+  return dli_launch_status();
+}
+
+template <int FORM>
+static int gf_few_around(const GfArgs& p, const GfAround& x, int rule, int grid, hipStream_t stream) {
+  const size_t lds = (size_t)p.segments * 64 * sizeof(gf4);
+  switch (rule) {
+    case 0: gemm_f32_few_kernel<1, 16, true, FORM><<<grid, 64 * 16, lds, stream>>>(p, x); break;
+    case 1: gemm_f32_few_kernel<1, 8, true, FORM><<<grid, 64 * 8, lds, stream>>>(p, x); break;
+    default: gemm_f32_few_kernel<1, 4, true, FORM><<<grid, 64 * 4, lds, stream>>>(p, x);
+  }
   return dli_launch_status();
 }
 
@@ -368,4 +487,31 @@ extern "C" int dli_gemm_f32_nt(const float* a, int64_t lda, const float* w, int6
     case 6: return gf_tiles<2, 2, 1>(p, vec, stream);
     default: return gf_tiles<4, 2, 1>(p, vec, stream);
   }
+}
+
+// The few-row products of a decode step behind a norm: act = silu(gate) * up of rms_norm(x) (positions null; w: the gates' rows,
+// then the ups'), or q, k and v of it, rotated and written (q to `out`). Up to 16 rows, k a multiple of eight, heads of
+// whole tiles, x, w and norm_w of whole vectors: what else there is takes the kernels one by one.
+extern "C" int dli_gemm_f32_normed(const float* x, int64_t ldx, const float* w, const float* bias, const float* norm_w, float eps,
+                                   float* out, int64_t ldo, int m, int n, int k, const int* positions, const float* inv_freq,
+                                   const int* slots, float* k_pages, float* v_pages, int q_heads, int kv_heads, int head_dim,
+                                   int page_size, hipStream_t stream) {
+  if (m <= 0) return DLI_OK;
+  if (m > 16 || n <= 0 || k <= 0 || k % 8 != 0 || ldx < k || ldx % 4 != 0 ||
+      (((uintptr_t)x | (uintptr_t)w | (uintptr_t)norm_w) % 16) != 0)
+    return DLI_ERR_ARGUMENT;
+  int segments, seg_runs;
+  gf_order(k, segments, seg_runs);
+  const GfArgs p = {x, w, bias, nullptr, out, ldx, k, 0, ldo, m, n, k, segments, seg_runs};
+  const int threads = k / 8 >= 256 ? 256 : (k / 8 >= 128 ? 128 : 64);   // (as dli_rms_norm's)
+  const GfAround around = {norm_w, eps, threads / 64, positions, inv_freq, slots, k_pages, v_pages, q_heads, kv_heads, head_dim, page_size};
+  const int rule = gf_rule(m, n, segments);
+  if (positions == nullptr) {
+    if (n % 2 != 0 || ldo < n / 2) return DLI_ERR_ARGUMENT;
+    return gf_few_around<GF_GLU>(p, around, rule, (n / 2 + 7) / 8, stream);
+  }
+  if (inv_freq == nullptr || slots == nullptr || k_pages == nullptr || v_pages == nullptr || q_heads <= 0 || kv_heads <= 0 ||
+      head_dim <= 0 || head_dim % 16 != 0 || page_size <= 0 || n != (q_heads + 2 * kv_heads) * head_dim || ldo < q_heads * head_dim)
+    return DLI_ERR_ARGUMENT;
+  return gf_few_around<GF_ROPE>(p, around, rule, n / 16, stream);
 }

@@ -42,6 +42,8 @@ _SIGNATURES = {
     "dli_rope_kv_write": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int,
                           _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "dli_gemm_f32_rule": [_c_int, _c_int, _c_int],
+    "dli_gemm_f32_normed": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_ptr, _c_ptr,
+                            _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "dli_gemm_f32_nt": [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_int,
                         _c_int, _c_int, _c_ptr],
     "dli_sample": [_c_ptr, _c_i64, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
@@ -434,6 +436,60 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, bias: Optional
         ldr = residual.stride(0)
     _check(library().dli_gemm_f32_nt(_ptr(a), a.stride(0), _ptr(w), w.stride(0), _ptr(bias), _ptr(residual),
                                      ldr, _ptr(out), out.stride(0), m, n, k, _stream()), "gemm_f32")
+
+
+def gemm_f32_normed_supports(rows: int, w: torch.Tensor) -> bool:
+    """Whether :func:`gemm_f32_swiglu` and :func:`gemm_f32_qkv_rope` take so many rows and this matrix: up to 16 rows, whole
+    vectors. (The norm's weight begins at a whole vector too.)"""
+    return 0 < rows <= 16 and w.dtype == torch.float32 and w.is_contiguous() and w.shape[1] % 8 == 0 and w.data_ptr() % 16 == 0
+
+
+def _normed_operands(x, w, bias, norm_w) -> None:
+    _rows(x, "x", torch.float32)
+    _dense(w, "w", torch.float32, 2)
+    _dense(norm_w, "norm_w", torch.float32, 1)
+    _require(x.shape[1] == w.shape[1] == norm_w.shape[0], "x, w and norm_w differ in inner size")
+    _require(gemm_f32_normed_supports(x.shape[0], w) and x.stride(0) % 4 == 0 and (x.data_ptr() | norm_w.data_ptr()) % 16 == 0,
+             "up to 16 rows of whole vectors")
+    if bias is not None:
+        _dense(bias, "bias", torch.float32, 1)
+        _require(bias.shape[0] == w.shape[0], "bias length differs from rows of w")
+
+
+def gemm_f32_swiglu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, norm_w: torch.Tensor, eps: float,
+                    bias: Optional[torch.Tensor] = None) -> None:
+    """``out = silu(gate) * up`` of the up to 16 rows ``rms_norm(x)``, in IEEE single precision; ``w``: the gates' rows, then the
+    ups'. The same bits as :func:`rms_norm`, :func:`gemm_f32` and :func:`silu_mul` one after the other."""
+    _normed_operands(x, w, bias, norm_w)
+    _rows(out, "out", torch.float32)
+    m, k = x.shape
+    _require(w.shape[0] % 2 == 0 and out.shape == (m, w.shape[0] // 2), "out must be [rows of x, half the rows of w]")
+    _check(library().dli_gemm_f32_normed(_ptr(x), x.stride(0), _ptr(w), _ptr(bias), _ptr(norm_w), eps, _ptr(out), out.stride(0), m,
+                                         w.shape[0], k, None, None, None, None, None, 0, 0, 0, 0, _stream()), "gemm_f32_swiglu")
+
+
+def gemm_f32_qkv_rope(x: torch.Tensor, w: torch.Tensor, q_out: torch.Tensor, norm_w: torch.Tensor, eps: float,
+                      positions: torch.Tensor, inv_freq: torch.Tensor, slots: torch.Tensor, k_pages: torch.Tensor,
+                      v_pages: torch.Tensor, bias: Optional[torch.Tensor] = None) -> None:
+    """``rms_norm(x) @ w.T (+ bias)`` of up to 16 rows as q, k and v heads: q rotated to ``q_out``, k rotated and v as they are
+    to the tokens' slots (as :func:`rope_kv_write`; the rotation covers whole heads)."""
+    _normed_operands(x, w, bias, norm_w)
+    _rows(q_out, "q_out", torch.float32)
+    _dense(k_pages, "k_pages", torch.float32, 4)
+    _dense(v_pages, "v_pages", torch.float32, 4)
+    _dense(positions, "positions", torch.int32, 1)
+    _dense(slots, "slots", torch.int32, 1)
+    _dense(inv_freq, "inv_freq", torch.float32, 1)
+    m, k = x.shape
+    pages, kv_heads, page_size, d = k_pages.shape
+    q_heads = w.shape[0] // d - 2 * kv_heads
+    _require(d % 16 == 0 and q_heads > 0 and w.shape[0] == (q_heads + 2 * kv_heads) * d, "w must hold q, k and v heads")
+    _require(v_pages.shape == (pages, kv_heads, d, page_size), "v_pages must be [pages, kv_heads, head_dim, page_size]")
+    _require(q_out.shape == (m, q_heads * d) and positions.shape[0] == m and slots.shape[0] == m, "q_out, positions and slots go by rows of x")
+    _require(inv_freq.shape[0] * 2 == d, "inv_freq must hold head_dim/2 frequencies")
+    _check(library().dli_gemm_f32_normed(_ptr(x), x.stride(0), _ptr(w), _ptr(bias), _ptr(norm_w), eps, _ptr(q_out), q_out.stride(0),
+                                         m, w.shape[0], k, _ptr(positions), _ptr(inv_freq), _ptr(slots), _ptr(k_pages),
+                                         _ptr(v_pages), q_heads, kv_heads, d, page_size, _stream()), "gemm_f32_qkv_rope")
 
 
 def gemm_f32_rule(m: int, n: int, k: int) -> int:

@@ -192,6 +192,10 @@ class GQAttention(Mixer):
     #    the two projections' kernels
     def streams(self, ctx: Any) -> bool:
         nh, d, n = self.num_heads, self.head_dim, ctx.num_tokens
+        if not self.rt.is_bf16:
+            table = self.position.rotary_table()
+            return (not self.shares_kv and table is not None and table.dim == d and ctx.num_decode == ctx.num_entries
+                    and ops.gemm_f32_normed_supports(n, self.w_qkv))
         if not (self.rt.is_bf16 and ctx.num_decode == ctx.num_entries and self.hidden_size % 8 == 0
                 and ops.attention_mfma_supports(d, ctx.page_size, self.rt.dtype)):
             return False
@@ -213,6 +217,13 @@ class GQAttention(Mixer):
         grp = ctx.groups[cache.group]
         n = stream.x.shape[0]
         norm_w, eps = norm.fused_params()
+        if not self.rt.is_bf16:
+            q, out = self.rt.empty(n, nh * d), self.rt.empty(n, nh * d)
+            ops.gemm_f32_qkv_rope(stream.x, self.w_qkv, q, norm_w, eps, ctx.positions, self.position.rotary_table().inv_freq,
+                                  grp.slots, cache.k_pages, cache.v_pages, bias=self.b_qkv)
+            paged_attention(q, cache.k_pages, cache.v_pages, out, ctx, grp, nh, self.scale, self.window)
+            ops.gemm_f32(out, self.w_o, stream.x, bias=self.b_o, residual=stream.x)
+            return
         if n > FEW_ROWS:
             self._forward_stream_mid(stream, norm, ctx, cache, grp, following)
             return

@@ -104,10 +104,11 @@ class DecodeStream:
     """The residual stream of a step with few rows, in the form the fused decode kernels pass on:
     ``x [rows, hidden]`` already holds every residual sum, and ``ssq [parts, rows]`` holds each
     row's sum of squares in parts, as the kernel that last wrote ``x`` left them (the next
-    RMSNorm is computed from them inside the product kernel that consumes ``x``)."""
+    RMSNorm is computed from them inside the product kernel that consumes ``x``; None in 32-bit, where that
+    kernel makes the sums itself)."""
 
     x: torch.Tensor
-    ssq: torch.Tensor
+    ssq: Optional[torch.Tensor]
     # The rows of ``x`` already normalised by ``normed_for`` (a norm's weight address and eps),
     # where the kernel that last wrote ``x`` was told which norm follows and applied it too.
     normed: Optional[torch.Tensor] = None

@@ -61,7 +61,8 @@ class PreNormBlock(Block):
     def streams(self, ctx: Any, parts: Mapping[str, Part]) -> bool:
         if "feed_forward" not in parts:
             return False
-        fused_norms = all(hasattr(parts[r], "fused_params") for r in ("mixer_norm", "feed_forward_norm"))
+        fused_norms = all(hasattr(parts[r], "fused_params") and (self.rt.is_bf16 or parts[r].fused_params()[0].data_ptr() % 16 == 0)
+                          for r in ("mixer_norm", "feed_forward_norm"))   # (the 32-bit products read whole vectors)
         return fused_norms and parts["mixer"].streams(ctx) and parts["feed_forward"].streams(ctx)
 
     def first_norm(self, parts: Mapping[str, Part]) -> Optional[Part]:

@@ -66,11 +66,14 @@ class TokenEmbedding(Embedding):
         return out if self.norm is None else self.norm.forward_f32(out)
 
     def streams(self, ctx) -> bool:
-        return self.rt.is_bf16 and not self.float32_rows  # the fused decode kernels keep a stream of the runtime's type
+        return not self.float32_rows  # the fused decode kernels keep a stream of the runtime's type
 
     def forward_stream(self, ids: torch.Tensor) -> DecodeStream:
         n = ids.shape[0]
         out = self.rt.empty(n, self.hidden_size)
+        if not self.rt.is_bf16:   # (the 32-bit products sum the squares themselves)
+            ops.embedding(self.table(), ids, out)
+            return DecodeStream(out, None)
         ssq = torch.empty(1, n, device=self.rt.device, dtype=torch.float32)
         ops.embedding_ssq(self.table(), ids, out, ssq)
         return DecodeStream(out, ssq)

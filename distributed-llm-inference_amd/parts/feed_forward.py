@@ -126,8 +126,10 @@ class GatedMLP(FeedForward):
 
     def streams(self, ctx: Any) -> bool:
         n = ctx.num_tokens
-        if self.activation != "silu" or self.float32_out or not (self.rt.is_bf16 and self.hidden_size % 8 == 0):
+        if self.activation != "silu" or self.float32_out or self.hidden_size % 8:
             return False
+        if not self.rt.is_bf16:
+            return ops.gemm_f32_normed_supports(n, self.w_gate_up)
         if n > self.FEW_ROWS:
             return (self.w_gate_up_tiled is not None and self.w_down_tiled is not None
                     and ops.mid_gemm_supports(n, self.hidden_size, self.rt.dtype)
@@ -141,6 +143,11 @@ class GatedMLP(FeedForward):
         the residual sum applies it as well, so that the next product reads normalised rows."""
         n = stream.x.shape[0]
         norm_w, eps = norm.fused_params()
+        if not self.rt.is_bf16:
+            act = self.rt.empty(n, self.intermediate_size)
+            ops.gemm_f32_swiglu(stream.x, self.w_gate_up, act, norm_w, eps, bias=self.b_gate_up)
+            ops.gemm_f32(act, self.w_down, stream.x, bias=self.b_down, residual=stream.x)
+            return
         if n > self.FEW_ROWS:
             ready = stream.normed_by(norm)
             if ready is not None:

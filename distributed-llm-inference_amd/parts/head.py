@@ -75,14 +75,14 @@ class LinearHead(Head):
         return out
 
     def streams(self, ctx) -> bool:
-        return self.softcap == 0 and self.scale == 1.0 and self.rt.is_bf16 and (ctx.num_tokens > self.FEW_ROWS
+        return self.softcap == 0 and self.scale == 1.0 and (not self.rt.is_bf16 or ctx.num_tokens > self.FEW_ROWS
                                     or ops.skinny_gemm_supports(ctx.num_tokens, self.hidden_size, self.rt.dtype))
 
     def forward_stream(self, stream: DecodeStream, norm: Norm, argmax: Optional[ArgmaxStage] = None) -> torch.Tensor:
         """Logits of every row of the stream, the final norm computed inside the product (with
         more than a few rows: the norm kernel, then the library product). ``argmax``: where the
         kernel that makes the logits may leave the first stage of every row's argmax."""
-        if stream.x.shape[0] > self.FEW_ROWS:
+        if stream.x.shape[0] > self.FEW_ROWS or not self.rt.is_bf16:
             ready = stream.normed_by(norm)  # the last residual sum's kernel may have normalised already
             return self.forward(ready if ready is not None else norm.forward(stream.x))
         norm_w, eps = norm.fused_params()

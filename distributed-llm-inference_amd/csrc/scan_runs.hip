@@ -15,10 +15,12 @@
 // walk: a workgroup of four waves takes one (run, head) and 64 columns, values or unit matrix; sixteen lanes (a DPP row) share
 // four columns and hold four keys of each, so that five 16-byte reads of LDS a token serve sixteen columns (with one column
 // a lane, as token by token, LDS is what bounds it). The vectors of sixteen tokens are staged by the workgroup, the next
-// sixteen are on their way meanwhile. What bounds it: vector instructions, some 110 to 130 a token and wave at four cycles each.
+// sixteen are on their way meanwhile. What bounds it: vector instructions, some 75 to 110 a token and wave at four cycles each (110 to 130
+// while a sum over the lanes took each column by itself: the walk of one prompt of 2,048 tokens 133 -> 108 us RUNS_DELTA, 54 -> 49
+// RUNS_BONUS, of four prompts, 2,990 tokens, 168 -> 125 RUNS_GATED, and as far from 64 bits or less).
 //
-// Measured (one prompt of 2,048 tokens, 32 heads, walk + carry + finish, us): RUNS_DELTA 135 + 15 + 21 against 578 and 17 for
-// the norm, RUNS_BONUS 55 + 8 + 17 against 378 and 17, RUNS_GATED 136 in all against 421. Where the cut lies: ops.scan_runs.
+// Measured (one prompt of 2,048 tokens, 32 heads, walk + carry + finish, us): RUNS_DELTA 108 + 15 + 21 against 578 and 17 for
+// the norm, RUNS_BONUS 49 + 8 + 17 against 378 and 17, RUNS_GATED 136 in all (before the sums were made together) against 421. Where the cut lies: ops.scan_runs.
 // Beside 255 single tokens, which keep the kernel of steps of single tokens: 245, 168 and 183 us a layer (5,150, 2,880 and 2,610 token
 // by token; 1,048, 1,301 and 818 with every entry cut and the launch as large as the longest entry times the entries).
 // Distance from the rules in 64 bits against token by token (2-norm; 300 to 4,096 tokens, 8 to 32 heads, every row of outputs and
@@ -34,6 +36,15 @@ __device__ __forceinline__ float runs_row_sum(float x) {   // over the sixteen l
   x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x140, 0xF, 0xF, false));
   return x;
 }
+
+// Four sums over the sixteen lanes of a DPP row, each where it is wanted: the lanes of quad b hold column (b + j) % 4 in register j, so
+// column b's other parts lie 4 j lanes back, and three rotated additions bring them together; two more sum the quad. Column
+// by column it is four additions each, sixteen in all.
+__device__ __forceinline__ float runs_own_sum(const rf4& x) {
+  return quad_sum(((x[0] + row_ror<8>(x[2])) + (row_ror<4>(x[1]) + row_ror<12>(x[3]))));
+}
+// Every quad's own value to the registers of its column.
+__device__ __forceinline__ rf4 runs_to_columns(float own) { return rf4{own, row_ror<12>(own), row_ror<8>(own), row_ror<4>(own)}; }
 
 // Runs lie one behind the other in slots, by entry and place, and a launch has a workgroup a slot and head: as large as the rows
 // are and not as the longest entry times the entries, what is left over at its end (empty workgroups between the others leave
@@ -90,7 +101,10 @@ __global__ __launch_bounds__(256) void scan_runs_walk_kernel(RunsArgs p) {
   const int entry = place.entry, run = place.run, first = place.first, row0 = place.row0, n = place.n, head = blockIdx.x;
   const bool unit = blockIdx.z != 0;   // the columns of the unit matrix
   if (n <= 0 || (unit && run == 0)) return;
-  const int col = wave * 16 + vloc * 4;   // the first of this lane's four columns
+  const int col = wave * 16 + vloc * 4, quad = part / 4;   // the first of these sixteen lanes' four columns; the one whose sums are this lane's
+  int column[4];   // of s's registers (runs_own_sum)
+#pragma unroll
+  for (int c = 0; c < 4; ++c) column[c] = col + (quad + c) % 4;
   const int64_t qk_col = (int64_t)(head / p.group) * D, v_col = (int64_t)head * D;
 
   float s[4][4];   // [key][column]
@@ -100,9 +114,9 @@ __global__ __launch_bounds__(256) void scan_runs_walk_kernel(RunsArgs p) {
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     rf4 old = {0.f, 0.f, 0.f, 0.f};
-    if (real) old = *reinterpret_cast<const rf4*>(st + (col + c) * D + part * 4);
+    if (real) old = *reinterpret_cast<const rf4*>(st + column[c] * D + part * 4);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) s[i][c] = unit ? (part * 4 + i == col + c ? 1.f : 0.f) : old[i];
+    for (int i = 0; i < 4; ++i) s[i][c] = unit ? (part * 4 + i == column[c] ? 1.f : 0.f) : old[i];
   }
   if (RULE == RUNS_BONUS) bonus = *reinterpret_cast<const rf4*>(p.bonus + v_col + part * 4);
 
@@ -126,10 +140,11 @@ __global__ __launch_bounds__(256) void scan_runs_walk_kernel(RunsArgs p) {
   const int64_t dst_stride = unit ? (int64_t)p.heads * D : p.o_stride;
   float* dst = unit ? p.y + (row0 - p.row0) * dst_stride : p.o + row0 * dst_stride;
   const auto step = [&](int t) {
-    const rf4 k = sk[t * 16 + part], r = sr[t * 16 + part], v = sv[t * 16 + wave * 4 + vloc];
+    const rf4 k = sk[t * 16 + part], r = sr[t * 16 + part];
+    const float v_own = reinterpret_cast<const float*>(sv)[t * 64 + col + quad];
     rf4 o;
     if constexpr (RULE == RUNS_BONUS) {
-      const rf4 w = sw[t * 16 + part];
+      const rf4 w = sw[t * 16 + part], v = runs_to_columns(v_own);
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         float o0 = 0.f, o1 = 0.f;
@@ -149,39 +164,30 @@ __global__ __launch_bounds__(256) void scan_runs_walk_kernel(RunsArgs p) {
       rf4 us;
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        float u0 = k[0] * s[0][c], u1 = k[1] * s[1][c];
-        u0 = fmaf(k[2], s[2][c], u0);
-        u1 = fmaf(k[3], s[3][c], u1);
-        us[c] = u0 + u1;
+        us[c] = fmaf(k[3], s[3][c], fmaf(k[2], s[2][c], fmaf(k[1], s[1][c], k[0] * s[0][c])));
       }
-#pragma unroll
-      for (int c = 0; c < 4; ++c) us[c] = runs_row_sum(us[c]);
+      const float us_own = runs_own_sum(us);
       if constexpr (RULE == RUNS_DELTA) {
-        const rf4 w = sw[t * 16 + part], a = sc[t * 16 + part];
+        const rf4 w = sw[t * 16 + part], a = sc[t * 16 + part], v = runs_to_columns(v_own);
+        us = runs_to_columns(us_own);
 #pragma unroll
         for (int c = 0; c < 4; ++c)
 #pragma unroll
           for (int i = 0; i < 4; ++i) s[i][c] = fmaf(w[i], s[i][c], fmaf(k[i], v[c], -a[i] * us[c]));
       } else {
         const float g = sg[2 * t], bg = sg[2 * t + 1];   // g and beta g; v comes times beta
+        const rf4 u = runs_to_columns(fmaf(-bg, us_own, v_own));
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const float u = fmaf(-bg, us[c], v[c]);
+        for (int c = 0; c < 4; ++c)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) s[i][c] = fmaf(k[i], u, g * s[i][c]);
-        }
+          for (int i = 0; i < 4; ++i) s[i][c] = fmaf(k[i], u[c], g * s[i][c]);
       }
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        float o0 = r[0] * s[0][c], o1 = r[1] * s[1][c];
-        o0 = fmaf(r[2], s[2][c], o0);
-        o1 = fmaf(r[3], s[3][c], o1);
-        o[c] = o0 + o1;
+        o[c] = fmaf(r[3], s[3][c], fmaf(r[2], s[2][c], fmaf(r[1], s[1][c], r[0] * s[0][c])));
       }
     }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) o[c] = runs_row_sum(o[c]);
-    return o;
+    return runs_own_sum(o);
   };
 
   fetch(0);
@@ -206,17 +212,17 @@ __global__ __launch_bounds__(256) void scan_runs_walk_kernel(RunsArgs p) {
     if (t0 + TB < n) fetch(t0 + TB);   // on their way while this batch is walked
     __syncthreads();
     const int nb = min(TB, n - t0);
-    float* od = dst + t0 * dst_stride + v_col + col;
+    float* od = dst + t0 * dst_stride + v_col + col + quad;
     if (nb == TB) {
 #pragma unroll 4
       for (int t = 0; t < TB; ++t) {
-        const rf4 o = step(t);
-        if (part == 0) *reinterpret_cast<rf4*>(od + t * dst_stride) = o;
+        const float o = step(t);
+        if (part % 4 == 0) od[t * dst_stride] = o;
       }
     } else {
       for (int t = 0; t < nb; ++t) {
-        const rf4 o = step(t);
-        if (part == 0) *reinterpret_cast<rf4*>(od + t * dst_stride) = o;
+        const float o = step(t);
+        if (part % 4 == 0) od[t * dst_stride] = o;
       }
     }
     if constexpr (RULE == RUNS_BONUS) p.y += (int64_t)TB * p.heads * D;   // (the step counts its rows from the batch's first)
@@ -224,7 +230,7 @@ __global__ __launch_bounds__(256) void scan_runs_walk_kernel(RunsArgs p) {
   const int64_t at = ((int64_t)blockIdx.y * p.heads + head) * D;
   float* end = (unit ? p.moves : p.ends) + at * D;
 #pragma unroll
-  for (int c = 0; c < 4; ++c) *reinterpret_cast<rf4*>(end + (col + c) * D + part * 4) = rf4{s[0][c], s[1][c], s[2][c], s[3][c]};
+  for (int c = 0; c < 4; ++c) *reinterpret_cast<rf4*>(end + column[c] * D + part * 4) = rf4{s[0][c], s[1][c], s[2][c], s[3][c]};
   if (RULE == RUNS_BONUS && wave == 0 && vloc == 0) *reinterpret_cast<rf4*>(p.moves + at + part * 4) = decay;
 }
 

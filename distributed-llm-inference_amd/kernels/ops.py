@@ -203,6 +203,8 @@ _SIGNATURES = {
     "dli_expert_products": [_c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int,
                             _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_float, _c_float, _c_int,
                             _c_ptr],
+    "dli_expert_combine_stream": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
+                                  _c_float, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "dli_expert_combine": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_int, _c_int,
                            _c_int, _c_int, _c_int, _c_ptr],
 }
@@ -2419,6 +2421,51 @@ def expert_combine(ids: torch.Tensor, weights: Optional[torch.Tensor], z: Option
     _check(library().dli_expert_combine(_ptr(ids), _ptr(weights), _ptr(z), _ptr(h), h.stride(0), _ptr(shared_gate), g_stride,
                                         _ptr(shared), s_stride, _ptr(out), n, top, int(experts), width, _is_bf16(h.dtype),
                                         _stream()), "expert_combine")
+
+
+def expert_combine_stream_supports(x: torch.Tensor, a: torch.Tensor, z: Optional[torch.Tensor], shared: Optional[torch.Tensor]) -> bool:
+    """Whether :func:`expert_combine_stream` takes these: rows of whole vectors, results of experts among them."""
+    return (z is not None and x.shape[1] % 4 == 0 and all(t.data_ptr() % 16 == 0 for t in (x, a, z))
+            and (shared is None or (shared.data_ptr() % 16 == 0 and shared.stride(0) % 4 == 0)))
+
+
+def expert_combine_stream(ids: torch.Tensor, weights: Optional[torch.Tensor], z: torch.Tensor, h: torch.Tensor, experts: int,
+                          x: torch.Tensor, a: torch.Tensor, shared: Optional[torch.Tensor] = None,
+                          shared_gate: Optional[torch.Tensor] = None, w1: Optional[torch.Tensor] = None,
+                          w2: Optional[torch.Tensor] = None, eps: float = 0.0, out1: Optional[torch.Tensor] = None,
+                          out2: Optional[torch.Tensor] = None) -> None:
+    """``x += a + out`` with ``out`` as :func:`expert_combine` makes it, and in the same kernel two norms of the new ``x`` as
+    :func:`rms_norm_pair` (``w1`` ``None``: none). ``x, a`` float32 ``[n, width]``."""
+    _dense(ids, "ids", torch.int32, 2)
+    n, top = ids.shape
+    if weights is not None:
+        _dense(weights, "weights", torch.float32, 2)
+    _rows(h, "h", h.dtype)
+    for name, t in (("x", x), ("a", a), ("z", z)):
+        _dense(t, name, torch.float32, 2)
+    width = x.shape[1]
+    _require((weights is None or weights.shape == (n, top)) and h.shape == x.shape == a.shape == (n, width) and z.shape == (n * top, width),
+             "ids, weights, z, h, x and a disagree")
+    s_stride = g_stride = 0
+    if shared is not None:
+        _f32_rows(shared, "shared")
+        _require(shared.shape == (n, width), "shared must be [n, width]")
+        s_stride = shared.stride(0)
+    if shared_gate is not None:
+        _require(shared is not None and shared_gate.is_cuda and shared_gate.dtype == torch.float32
+                 and shared_gate.dim() == 2 and shared_gate.shape == (n, 1), "shared_gate must be float32 [n, 1] beside shared")
+        g_stride = shared_gate.stride(0)
+    if w1 is not None:
+        for name, w in (("w1", w1), ("w2", w2)):
+            _dense(w, name, torch.float32, 1)
+            _require(w.shape[0] == width, f"{name} must hold a value per column")
+        for name, t in (("out1", out1), ("out2", out2)):
+            _dense(t, name, h.dtype, 2)
+            _require(t.shape == x.shape, f"{name} differs from x in shape")
+    _check(library().dli_expert_combine_stream(
+        _ptr(ids), _ptr(weights), _ptr(z), _ptr(h), h.stride(0), _ptr(shared_gate), g_stride, _ptr(shared), s_stride, _ptr(x), _ptr(a),
+        _ptr(w1), _ptr(w2), float(eps), _ptr(out1), _ptr(out2), n, top, int(experts), width, _is_bf16(h.dtype), _stream()),
+        "expert_combine_stream")
 
 
 # ----------------------------------------------------------------------------- short convolutions, the selective scan

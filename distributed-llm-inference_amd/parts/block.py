@@ -177,6 +177,26 @@ class PostNormBlock(Block):
         return x, None
 
 
+class NormPair:
+    """Two plain RMS norms that agree on eps and read the same rows: what a :class:`ParallelNormsBlock` meets the stream with."""
+
+    def __init__(self, one: Part, two: Part) -> None:
+        self.one, self.two = one, two
+
+    @staticmethod
+    def of(one: Part, two: Part) -> Optional["NormPair"]:
+        fused = [getattr(n, "fused_params", None) for n in (one, two)]
+        return NormPair(one, two) if all(fused) and fused[0]()[1] == fused[1]()[1] else None
+
+    def pair_params(self) -> tuple:
+        (w1, eps), (w2, _) = self.one.fused_params(), self.two.fused_params()
+        return w1, w2, eps
+
+    def stream_key(self) -> tuple:
+        w1, w2, eps = self.pair_params()
+        return ("pair", w1.data_ptr(), w2.data_ptr(), float(eps))
+
+
 @register_part("block", "parallel_norms")
 class ParallelNormsBlock(Block):
     """Mixer and feed-forward side by side, each behind a norm of its own, both reading the same stream:
@@ -184,6 +204,7 @@ class ParallelNormsBlock(Block):
     its norm may be absent. ``x`` is float32 in both runtimes; the norms round once, to the type that the
     products read; the two results are added to each other and then into the stream, in 32-bit."""
 
+    asks_following = True
     roles = ("mixer_norm", "mixer")   # and, unless the layer has no feed-forward, "feed_forward_norm" and "feed_forward"
 
     def __init__(self, runtime: Runtime) -> None:
@@ -191,6 +212,9 @@ class ParallelNormsBlock(Block):
 
     def graph_capturable(self, page_size: int) -> bool:
         return True  # kernels on device arrays only
+
+    def first_norm(self, parts: Mapping[str, Part]) -> Optional[Any]:
+        return NormPair.of(parts["mixer_norm"], parts["feed_forward_norm"]) if "feed_forward" in parts else parts["mixer_norm"]
 
     def forward(self, x: torch.Tensor, delta: Optional[torch.Tensor], ctx: Any, cache: Any,
                 parts: Mapping[str, Part]) -> tuple[torch.Tensor, Optional[torch.Tensor]]:
@@ -200,20 +224,33 @@ class ParallelNormsBlock(Block):
             raise RuntimeError("the parallel_norms block keeps a float32 residual stream")
         if delta is not None:
             ops.add(x, delta, x)
+            NormedStream.offer(ctx, x, None, None)
         if "feed_forward" not in parts:
-            ops.add(x, _as_f32(parts["mixer"].forward(parts["mixer_norm"].forward(x), ctx, cache)), x)
+            h = NormedStream.take(ctx, x, parts["mixer_norm"])
+            ops.add(x, _as_f32(parts["mixer"].forward(parts["mixer_norm"].forward(x) if h is None else h, ctx, cache)), x)
+            NormedStream.offer(ctx, x, None, None)
             return x, None
-        n1, n2 = parts["mixer_norm"], parts["feed_forward_norm"]
-        pair = [getattr(n, "fused_params", None) for n in (n1, n2)]
-        if all(pair) and pair[0]()[1] == pair[1]()[1]:
+        n1, n2, ff = parts["mixer_norm"], parts["feed_forward_norm"], parts["feed_forward"]
+        pair = NormPair.of(n1, n2)
+        ready = NormedStream.take(ctx, x, pair) if pair is not None else None
+        if ready is not None:
+            h1, h2 = ready   # (made by the kernel that wrote the stream)
+        elif pair is not None:
             # plain RMS norms that agree on eps: one pass over the rows' statistics for both
             h1, h2 = self.rt.empty(*x.shape), self.rt.empty(*x.shape)
-            ops.rms_norm_pair(x, pair[0]()[0], pair[1]()[0], pair[0]()[1], h1, h2)
+            w1, w2, eps = pair.pair_params()
+            ops.rms_norm_pair(x, w1, w2, eps, h1, h2)
         else:
             h1, h2 = n1.forward(x), n2.forward(x)
         y = _as_f32(parts["mixer"].forward(h1, ctx, cache))
-        f = _as_f32(parts["feed_forward"].forward(h2, ctx))
-        ops.add_pair_into_stream(x, y, f)
+        if hasattr(ff, "forward_into_stream"):
+            following = NormedStream.following(ctx)
+            following = following if hasattr(following, "pair_params") else None
+            rows = ff.forward_into_stream(h2, ctx, x, y, following)
+            NormedStream.offer(ctx, x, following, rows)
+            return x, None
+        ops.add_pair_into_stream(x, y, _as_f32(ff.forward(h2, ctx)))
+        NormedStream.offer(ctx, x, None, None)
         return x, None
 
 

@@ -28,7 +28,7 @@ one kernel adds everything up in 32-bit. The expert matrices are stacked ``[expe
 
 from __future__ import annotations
 
-from typing import Any, Mapping
+from typing import Any, Mapping, Optional
 
 import torch
 
@@ -114,7 +114,8 @@ class RoutedExperts(FeedForward):
             self.ws_gate_up = torch.cat([tensors["shared.gate"], tensors["shared.up"]], dim=0).contiguous()
             self.ws_down = tensors["shared.down"]
 
-    def forward(self, x: torch.Tensor, ctx: Any) -> torch.Tensor:
+    def _results(self, x: torch.Tensor, ctx: Any) -> tuple:
+        """The choices with their weights (None: ones), their results, and the shared expert's with its gate."""
         n, dev = x.shape[0], self.rt.device
         ids = torch.empty(n, self.top, device=dev, dtype=torch.int32)
         weights = torch.empty(n, self.top, device=dev, dtype=torch.float32)
@@ -143,6 +144,28 @@ class RoutedExperts(FeedForward):
             shared = linear_f32(self.rt, act, self.ws_down)
             if self.shared_gate:
                 gate = logits[:, self.total:self.total + 1]
-        out = torch.empty(n, self.hidden_size, device=dev, dtype=torch.float32)
-        ops.expert_combine(ids, None if self.weight_input else weights, z, x, self.experts, out, shared=shared, shared_gate=gate)
+        return ids, None if self.weight_input else weights, z, shared, gate
+
+    def _combined(self, x: torch.Tensor, results: tuple) -> torch.Tensor:
+        ids, weights, z, shared, gate = results
+        out = torch.empty(x.shape[0], self.hidden_size, device=self.rt.device, dtype=torch.float32)
+        ops.expert_combine(ids, weights, z, x, self.experts, out, shared=shared, shared_gate=gate)
         return out
+
+    def forward(self, x: torch.Tensor, ctx: Any) -> torch.Tensor:
+        return self._combined(x, self._results(x, ctx))
+
+    def forward_into_stream(self, x: torch.Tensor, ctx: Any, stream: torch.Tensor, other: torch.Tensor, following: Any) -> Optional[tuple]:
+        """``stream += other + self.forward(x)`` (float32), in the kernel that combines the experts where it can, and with it the
+        pair of norms ``following`` that the stream meets next, whose rows are returned (None: not made)."""
+        results = self._results(x, ctx)
+        ids, weights, z, shared, gate = results
+        if not ops.expert_combine_stream_supports(stream, other, z, shared):
+            ops.add_pair_into_stream(stream, other, self._combined(x, results))
+            return None
+        w1, w2, eps = following.pair_params() if following is not None else (None, None, 0.0)
+        rows = None
+        if w1 is not None and (w1.data_ptr() | w2.data_ptr()) % 16 == 0:
+            rows = (self.rt.empty(*stream.shape), self.rt.empty(*stream.shape))
+        ops.expert_combine_stream(ids, weights, z, x, self.experts, stream, other, shared, gate, *((w1, w2, eps, *rows) if rows else ()))
+        return rows

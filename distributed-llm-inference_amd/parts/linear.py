@@ -10,7 +10,7 @@ takes on the GPU when a step has a few hundred tokens.
 
 from __future__ import annotations
 
-from typing import Optional
+from typing import Any, Optional
 
 import torch
 
@@ -122,7 +122,17 @@ class NormedStream:
     the stream was told which norm follows: kept on the step's context for whoever applies that norm next, and
     dropped by whoever changes the stream."""
 
-    KEY = "normed stream"
+    KEY, NEXT = "normed stream", "following norm"
+
+    @staticmethod
+    def follow(ctx, norm: Any) -> None:
+        """What the stream meets after the block that runs next (``Block.asks_following``)."""
+        if hasattr(ctx, "_memo"):
+            ctx._memo[NormedStream.NEXT] = norm
+
+    @staticmethod
+    def following(ctx) -> Any:
+        return getattr(ctx, "_memo", {}).pop(NormedStream.NEXT, None)
 
     @staticmethod
     def offer(ctx, x: torch.Tensor, norm: Optional[Norm], rows: Optional[torch.Tensor]) -> None:

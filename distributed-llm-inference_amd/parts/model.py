@@ -219,6 +219,8 @@ class Model:
                              else self.final_norm if getattr(ctx, "all_rows_wanted", False) else None)
                     x, delta = layer.block.forward(x, delta, ctx, cache, layer.parts, following=after)
                 else:
+                    if layer.block.asks_following:
+                        NormedStream.follow(ctx, order[i + 1].block.first_norm(order[i + 1].parts) if i + 1 < len(order) else None)
                     x, delta = layer.block.forward(x, delta, ctx, cache, layer.parts)
         k = ctx.logit_rows.shape[0]
         if k == 0:

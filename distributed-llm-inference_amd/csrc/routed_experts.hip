@@ -214,7 +214,14 @@ __device__ __forceinline__ int sum_before(int v) {   // over the lanes before th
   }
   return s - v;
 }
-__global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict__ ids, int slots, int experts,
+// With a table (TableChoice) the kernel looks the choices up itself and writes them and their weights: a kernel of its own for that took
+// 4.3 us a layer of a step of two rows, this one takes 4.7 without it and 4.6 with it (9,216 slots, nine a thread: some 15 more, so not there).
+struct TableChoice { const int* table; const int* token_ids; int vocab, top; float* weights; };
+__device__ __forceinline__ int table_choice(const int* table, const int* token_ids, int vocab, int top, int i) {
+  const int t = i / top, tok = min(max(token_ids[t], 0), vocab - 1);
+  return table[(int64_t)tok * top + i - t * top];
+}
+__global__ __launch_bounds__(1024) void expert_sort_kernel(int* ids, TableChoice choice, int slots, int experts,
                                                            int* __restrict__ offsets, int* __restrict__ order,
                                                            int* __restrict__ tile_expert, int* __restrict__ tile_row0,
                                                            int* __restrict__ tile_count, int max_tiles, int tile_rows) {
@@ -224,16 +231,25 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict
   const int lane = threadIdx.x % DLI_WAVE, wave = threadIdx.x / DLI_WAVE;
   for (int e = threadIdx.x; e < experts; e += 1024) counts[e] = 0;
   __syncthreads();
+  int own = -1;   // the first slot's choice (the others are read once more)
   for (int i = threadIdx.x; i < slots; i += 1024) {
-    const int e = ids[i];
+    int e;
+    if (choice.table != nullptr) {
+      e = table_choice(choice.table, choice.token_ids, choice.vocab, choice.top, i);
+      ids[i] = e;
+      choice.weights[i] = 1.f / (float)choice.top;
+    } else {
+      e = ids[i];
+    }
+    if (i == (int)threadIdx.x) own = e;
     if (e >= 0 && e < experts) atomicAdd(&counts[e], 1);
   }
   __syncthreads();
   int at = 0, tiles = 0;                                        // of the experts before these 1024
   for (int e0 = 0; e0 < experts; e0 += 1024) {
-    const int e = e0 + threadIdx.x, rows = e < experts ? counts[e] : 0, own = (rows + tile_rows - 1) / tile_rows;
-    int row = sum_before(rows), tile = sum_before(own);
-    if (lane == DLI_WAVE - 1) { rows_of[wave] = row + rows; tiles_of[wave] = tile + own; }
+    const int e = e0 + threadIdx.x, rows = e < experts ? counts[e] : 0, parts = (rows + tile_rows - 1) / tile_rows;
+    int row = sum_before(rows), tile = sum_before(parts);
+    if (lane == DLI_WAVE - 1) { rows_of[wave] = row + rows; tiles_of[wave] = tile + parts; }
     __syncthreads();
     row += at;
     tile += tiles;
@@ -246,7 +262,7 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict
     if (e < experts) {
       offsets[e] = row;
       cursor[e] = row;
-      for (int k = 0; k < own && tile + k < max_tiles; ++k) {
+      for (int k = 0; k < parts && tile + k < max_tiles; ++k) {
         tile_expert[tile + k] = e;
         tile_row0[tile + k] = row + k * tile_rows;
       }
@@ -258,7 +274,7 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict
     tile_count[0] = min(tiles, max_tiles);
   }
   for (int i = threadIdx.x; i < slots; i += 1024) {
-    const int e = ids[i];
+    const int e = i == (int)threadIdx.x ? own : ids[i];
     if (e >= 0 && e < experts) order[atomicAdd(&cursor[e], 1)] = i;
   }
 }
@@ -852,9 +868,7 @@ __global__ void table_choose_kernel(const int* __restrict__ table, const int* __
                                     int vocab, int* __restrict__ ids, float* __restrict__ weights) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n * top) return;
-  const int t = i / top, j = i - t * top;
-  const int tok = min(max(token_ids[t], 0), vocab - 1);
-  ids[i] = table[(int64_t)tok * top + j];
+  ids[i] = table_choice(table, token_ids, vocab, top, i);
   weights[i] = 1.f / (float)top;
 }
 
@@ -915,24 +929,39 @@ int dli_expert_tile_rows(int64_t slots, int experts, int width, int ff, int is_b
   return expert_few(slots, experts, width, ff) ? EXM_FEW : EXM_BM;
 }
 
+int dli_table_choose(const int* table, const int* token_ids, int n, int top, int vocab, int* ids, float* weights,
+                     hipStream_t stream) {
+  if (n <= 0) return DLI_OK;
+  if (top <= 0 || vocab <= 0 || (int64_t)n * top > 0x7fffffff) return DLI_ERR_ARGUMENT;
+  table_choose_kernel<<<(n * top + 255) / 256, 256, 0, stream>>>(table, token_ids, n, top, vocab, ids, weights);
+  return dli_launch_status();
+}
+
 // The experts' part of a mixture for `rows` tokens: sort, up product with activation, down product.
 // ids [rows][top]; scratch: offsets [experts + 1], order [rows * top], tile_expert and tile_row0 [max_tiles],
 // tile_count [1] (int32), y [rows * top][ff] (T), z [rows * top][width] (float32). in_weight [rows][top] (may be nullptr):
 // what each slot's expert input is multiplied by.
-int dli_expert_products(const int* ids, const void* h, int64_t h_stride, const void* w_gate, const void* w_up,
+// table [vocab][top] (may be nullptr): ids and weights [rows][top] are written here, the row of each token's id with weights of 1 / top.
+int dli_expert_products(int* ids, const int* table, const int* token_ids, int vocab, float* weights, const void* h, int64_t h_stride,
+                        const void* w_gate, const void* w_up,
                         const void* w_down, int* offsets, int* order, int* tile_expert, int* tile_row0, int* tile_count,
                         int max_tiles, void* y, float* z, const float* in_weight, int rows, int top, int experts, int width,
                         int ff, float limit, float alpha, float up_shift, int is_bf16, hipStream_t stream) {
   if (rows <= 0) return DLI_OK;
   const int64_t slots = (int64_t)rows * top;
   if (top < 1 || experts < 1 || experts > 4096 || width <= 0 || ff <= 0 || h_stride < width || slots > (1 << 30) ||
-      max_tiles < 1 || max_tiles > 65535 * 16)
+      max_tiles < 1 || max_tiles > 65535 * 16 || (table != nullptr && (token_ids == nullptr || vocab < 1 || weights == nullptr)))
     return DLI_ERR_ARGUMENT;
   const bool mfma = expert_mfma(width, ff, is_bf16);
   if (mfma && ((h_stride % 8) || ((uintptr_t)h % 16) || ((uintptr_t)w_gate % 16) || ((uintptr_t)w_up % 16) ||
                ((uintptr_t)w_down % 16) || ((uintptr_t)y % 16)))
     return DLI_ERR_ARGUMENT;
-  expert_sort_kernel<<<1, 1024, 2 * experts * sizeof(int), stream>>>(ids, (int)slots, experts, offsets, order, tile_expert,
+  TableChoice choice = {table, token_ids, vocab, top, weights};
+  if (table != nullptr && slots > 1024) {   // (several a thread: one workgroup's trips to memory, one after the other)
+    if (dli_table_choose(table, token_ids, rows, top, vocab, ids, weights, stream) != DLI_OK) return DLI_ERR_LAUNCH;
+    choice.table = nullptr;
+  }
+  expert_sort_kernel<<<1, 1024, 2 * experts * sizeof(int), stream>>>(ids, choice, (int)slots, experts, offsets, order, tile_expert,
                                                                      tile_row0, tile_count, max_tiles,
                                                                      dli_expert_tile_rows(slots, experts, width, ff, is_bf16));
   if (dli_launch_status() != DLI_OK) return DLI_ERR_LAUNCH;
@@ -1008,12 +1037,5 @@ int dli_expert_combine(const int* ids, const float* weights, const float* z, con
   return dli_launch_status();
 }
 
-int dli_table_choose(const int* table, const int* token_ids, int n, int top, int vocab, int* ids, float* weights,
-                     hipStream_t stream) {
-  if (n <= 0) return DLI_OK;
-  if (top <= 0 || vocab <= 0 || (int64_t)n * top > 0x7fffffff) return DLI_ERR_ARGUMENT;
-  table_choose_kernel<<<(n * top + 255) / 256, 256, 0, stream>>>(table, token_ids, n, top, vocab, ids, weights);
-  return dli_launch_status();
-}
 
 }  // extern "C"

@@ -200,7 +200,7 @@ _SIGNATURES = {
     "dli_router_choose": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int,
                           _c_ptr, _c_ptr, _c_ptr],
     "dli_expert_tile_rows": [_c_i64, _c_int, _c_int, _c_int, _c_int],
-    "dli_expert_products": [_c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int,
+    "dli_expert_products": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int,
                             _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_float, _c_float, _c_int,
                             _c_ptr],
     "dli_expert_combine_stream": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
@@ -2356,15 +2356,25 @@ def router_choose(logits: torch.Tensor, total: int, correction: Optional[torch.T
 
 def expert_products(ids: torch.Tensor, h: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
                     limit: float, alpha: float, up_shift: float = 1.0,
-                    in_weights: Optional[torch.Tensor] = None) -> torch.Tensor:
+                    in_weights: Optional[torch.Tensor] = None,
+                    choose: Optional[tuple[torch.Tensor, torch.Tensor, torch.Tensor]] = None) -> torch.Tensor:
     """The chosen experts' results for every (token, choice): ``z [n * top, width]`` float32, row
     ``t * top + j`` holding ``w_down[e] clamped_glu(w_gate[e] h_t, w_up[e] h_t)`` for ``e = ids[t, j]`` (rows of
     ids at or above the number of experts are left unwritten). ``w_gate, w_up [experts, ff, width]``,
     ``w_down [experts, width, ff]`` of ``h``'s type. ``in_weights`` (float32 ``[n, top]``): what each choice's input ``h_t`` is
     multiplied by (the products being linear, their 32-bit sums are). Nothing here waits for the device: the rows are
-    sorted by expert and cut into tiles on the device."""
+    sorted by expert and cut into tiles on the device. ``choose`` ``(table, token_ids, weights)``: the kernel that sorts also
+    writes ``ids`` and ``weights``, as :func:`table_choose`."""
     _dense(ids, "ids", torch.int32, 2)
     n, top = ids.shape
+    table = token_ids = weights = None
+    if choose is not None:
+        table, token_ids, weights = choose
+        _dense(table, "table", torch.int32, 2)
+        _dense(token_ids, "token_ids", torch.int32, 1)
+        _dense(weights, "weights", torch.float32, 2)
+        _require(table.shape[0] > 0 and table.shape[1] == top and token_ids.shape[0] == n and weights.shape == (n, top),
+                 "table must hold a row of choices a token id, weights be [n, top]")
     _rows(h, "h", h.dtype)
     for name, w in (("w_gate", w_gate), ("w_up", w_up), ("w_down", w_down)):
         _dense(w, name, h.dtype, 3)
@@ -2384,7 +2394,8 @@ def expert_products(ids: torch.Tensor, h: torch.Tensor, w_gate: torch.Tensor, w_
     y = torch.empty(slots, ff, device=h.device, dtype=h.dtype)
     z = torch.empty(slots, width, device=h.device, dtype=torch.float32)
     _check(library().dli_expert_products(
-        _ptr(ids), _ptr(h), h.stride(0), _ptr(w_gate), _ptr(w_up), _ptr(w_down), _ptr(offsets), _ptr(order),
+        _ptr(ids), _ptr(table), _ptr(token_ids), 0 if table is None else table.shape[0], _ptr(weights), _ptr(h), h.stride(0),
+        _ptr(w_gate), _ptr(w_up), _ptr(w_down), _ptr(offsets), _ptr(order),
         _ptr(tile_expert), _ptr(tile_row0), _ptr(tile_count), max_tiles, _ptr(y), _ptr(z), _ptr(in_weights), n, top, experts, width, ff,
         float(limit), float(alpha), float(up_shift), _is_bf16(h.dtype), _stream()), "expert_products")
     return z

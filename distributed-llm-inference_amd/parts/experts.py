@@ -119,9 +119,10 @@ class RoutedExperts(FeedForward):
         n, dev = x.shape[0], self.rt.device
         ids = torch.empty(n, self.top, device=dev, dtype=torch.int32)
         weights = torch.empty(n, self.top, device=dev, dtype=torch.float32)
+        choose = None
         if self.routing == "table":
             logits = None
-            ops.table_choose(self.table, ctx.token_ids, ids, weights)
+            choose = (self.table, ctx.token_ids, weights)   # (by the kernel that sorts the choices)
         else:
             logits = linear_f32(self.rt, x, self.w_router)
             ops.router_choose(logits, self.total, self.correction, self.groups, self.groups_kept, self.top, self.scale, ids,
@@ -129,7 +130,9 @@ class RoutedExperts(FeedForward):
         z = None
         if self.experts:
             z = ops.expert_products(ids, x, self.w_gate, self.w_up, self.w_down, self.limit, self.alpha, self.up_shift,
-                                    in_weights=weights if self.weight_input else None)
+                                    in_weights=weights if self.weight_input else None, choose=choose)
+        elif choose is not None:
+            ops.table_choose(self.table, ctx.token_ids, ids, weights)
         shared = gate = None
         if self.shared_size:
             act = self.rt.empty(n, self.shared_size)

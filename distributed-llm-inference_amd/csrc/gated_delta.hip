@@ -49,6 +49,7 @@ struct PrepArgs {
   const float* conv_w;                     // [channels][taps], the last column the current token's
   const float* a_log; const float* dt_bias;  // [heads]
   const float* kept; int64_t state_stride; // the requests' kept inputs: state + offset, [taps-1][channels] a slot
+  float* keep;                             // the same where every entry is one row: its wave also writes the new ones (else nullptr)
   const int* q_start; const int* positions; const int* state_slots;
   float* out; int64_t out_stride;          // [rows][channels + 2 heads]: q | k | v | beta | g
   int entries, heads, kv_heads, dim, vdim, taps;
@@ -57,8 +58,11 @@ struct PrepArgs {
 // The convolution of channel c at `row`, which lies at position pos of its request, whose step starts at row `first`, and silu. An
 // input lies among the step's rows or the kept inputs, or before the sequence (zero; another input is read in its place). The taps
 // are asked for together (TAPS of them, or where that is 0 four at a time): no load hangs on a condition. Oldest input first.
+// keep: an entry's only row also leaves the inputs that the next one needs, one place further back, so that a step of single tokens needs
+// no kernel for that after this one (4.8 us of a step of four requests): tap t's input, from place t, goes to place t - 1, which
+// has been read.
 template <int TAPS>
-__device__ __forceinline__ float conv_silu(const PrepArgs& p, const float* kept, int channels, int row, int first, int pos, int c) {
+__device__ __forceinline__ float conv_silu(const PrepArgs& p, const float* kept, float* keep, int channels, int row, int first, int pos, int c) {
   constexpr int AT_ONCE = TAPS > 0 ? TAPS : 4;
   const int taps = TAPS > 0 ? TAPS : p.taps;
   const float* w = p.conv_w + (int64_t)c * taps;
@@ -77,8 +81,11 @@ __device__ __forceinline__ float conv_silu(const PrepArgs& p, const float* kept,
         wt[k] = w[t];
       }
 #pragma unroll
-      for (int k = 0; k < AT_ONCE; ++k)
-        if (t0 + k < taps) acc = fmaf(wt[k], taps - 1 - (t0 + k) <= pos ? in[k] : 0.f, acc);
+      for (int k = 0; k < AT_ONCE; ++k) {
+        const float x = taps - 1 - (t0 + k) <= pos ? in[k] : 0.f;
+        if (t0 + k < taps) acc = fmaf(wt[k], x, acc);
+        if (keep != nullptr && t0 + k >= 1 && t0 + k < taps) keep[(int64_t)(t0 + k - 1) * channels + c] = x;
+      }
     }
   }
   return acc / (1.f + expf(-acc));
@@ -104,15 +111,16 @@ __device__ __forceinline__ void conv_prepare_row(const PrepArgs& p, int row, int
   const int e = gd_entry_of_row(p.q_start, p.entries, row);
   const int first = p.q_start[e], pos = p.positions[row];
   const float* kept = p.kept + (int64_t)p.state_slots[e] * p.state_stride;
+  float* keep = p.keep != nullptr ? p.keep + (int64_t)p.state_slots[e] * p.state_stride : nullptr;
   if (unit >= 2 * p.kv_heads) {
     const int c = 2 * qk + (unit - 2 * p.kv_heads) * 64 + lane;
-    if (c < channels) out[c] = conv_silu<TAPS>(p, kept, channels, row, first, pos, c);
+    if (c < channels) out[c] = conv_silu<TAPS>(p, kept, keep, channels, row, first, pos, c);
     return;
   }
   const int c0 = unit * p.dim;                                  // q heads, then k heads
   float ss = 0.f;
   for (int c = lane; c < p.dim; c += DLI_WAVE) {
-    const float y = conv_silu<TAPS>(p, kept, channels, row, first, pos, c0 + c);
+    const float y = conv_silu<TAPS>(p, kept, keep, channels, row, first, pos, c0 + c);
     out[c0 + c] = y;
     ss += y * y;
   }
@@ -212,7 +220,8 @@ __global__ __launch_bounds__(64) void conv_prepare_run_kernel(PrepArgs p, int ro
 }
 
 // A thread a channel: it reads what it needs of the old kept inputs before it writes the new ones,
-// and no other thread touches its channel. (Runs after conv_prepare of the same step.)
+// and no other thread touches its channel. (Runs after conv_prepare of the same step, which reads what this overwrites for all rows
+// of an entry, unless every entry is one row.)
 #define GD_MAX_TAPS 16
 __global__ void conv_keep_kernel(const float* __restrict__ proj, int64_t stride, float* kept_base, int64_t state_stride,
                                  const int* __restrict__ q_start, const int* __restrict__ positions,
@@ -507,8 +516,9 @@ int dli_conv_prepare_in_runs(int rows, int entries, int heads, int kv_heads, int
 int dli_conv_prepare(const float* proj, int64_t stride, int b_off, int a_off, const float* conv_w, const float* a_log,
                      const float* dt_bias, float* state, int64_t state_stride, int64_t kept_offset, const int* q_start,
                      const int* positions, const int* state_slots, float* out, int64_t out_stride, int entries, int rows,
-                     int heads, int kv_heads, int dim, int vdim, int taps, hipStream_t stream) {
+                     int heads, int kv_heads, int dim, int vdim, int taps, int singles, hipStream_t stream) {
   if (rows <= 0 || entries <= 0) return DLI_OK;
+  if (singles && rows != entries) return DLI_ERR_ARGUMENT;
   const int64_t channels = 2 * (int64_t)kv_heads * dim + (int64_t)heads * vdim;
   if (heads <= 0 || kv_heads <= 0 || heads % kv_heads || dim <= 0 || vdim <= 0 || taps < 1 || taps > GD_MAX_TAPS ||
       stride < channels || out_stride < channels + 2 * heads || b_off < channels || a_off < channels ||
@@ -516,7 +526,7 @@ int dli_conv_prepare(const float* proj, int64_t stride, int b_off, int a_off, co
     return DLI_ERR_ARGUMENT;
   PrepArgs p;
   p.proj = proj; p.stride = stride; p.b_off = b_off; p.a_off = a_off; p.conv_w = conv_w; p.a_log = a_log;
-  p.dt_bias = dt_bias; p.kept = state + kept_offset; p.state_stride = state_stride; p.q_start = q_start;
+  p.dt_bias = dt_bias; p.kept = state + kept_offset; p.keep = singles ? state + kept_offset : nullptr; p.state_stride = state_stride; p.q_start = q_start;
   p.positions = positions; p.state_slots = state_slots; p.out = out; p.out_stride = out_stride; p.entries = entries;
   p.heads = heads; p.kv_heads = kv_heads; p.dim = dim; p.vdim = vdim; p.taps = taps;
   const int units = 2 * kv_heads + (int)(((int64_t)heads * vdim + 63) / 64) + 1;
@@ -530,7 +540,7 @@ int dli_conv_prepare(const float* proj, int64_t stride, int b_off, int a_off, co
   else
     conv_prepare_kernel<0><<<dim3(rows, units), 64, 0, stream>>>(p);
   if (dli_launch_status() != DLI_OK) return DLI_ERR_LAUNCH;
-  if (taps > 1) {
+  if (taps > 1 && !singles) {
     const dim3 grid(entries, (unsigned)((channels + 255) / 256));
     conv_keep_kernel<<<grid, 256, 0, stream>>>(proj, stride, state + kept_offset, state_stride, q_start, positions,
                                                state_slots, (int)channels, taps, nullptr);

@@ -192,7 +192,7 @@ _SIGNATURES = {
     "dli_gated_delta_max_taps": [],
     "dli_conv_prepare_in_runs": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
     "dli_conv_prepare": [_c_ptr, _c_i64, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr,
-                         _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
+                         _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "dli_gated_delta_scan": [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_int,
                              _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
     "dli_poly_norm": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_float, _c_int, _c_ptr],
@@ -2203,13 +2203,13 @@ def gated_delta_max_taps() -> int:
 def conv_prepare(proj: torch.Tensor, b_off: int, a_off: int, conv_w: torch.Tensor, a_log: torch.Tensor,
                  dt_bias: torch.Tensor, state: torch.Tensor, kept_offset: int, q_start: torch.Tensor,
                  positions: torch.Tensor, state_slots: torch.Tensor, out: torch.Tensor, heads: int, kv_heads: int,
-                 dim: int, vdim: int) -> None:
+                 dim: int, vdim: int, singles: bool = False) -> None:
     """What the gated delta rule reads, from a step's float32 projections ``proj [n, >=]`` (columns: q and
     k, ``kv_heads x dim`` each, then v, ``heads x vdim``; beta's and the decay's pre-activations at ``b_off``
     and ``a_off``): the short causal convolution per channel (``conv_w [channels, taps]``, the inputs before
     the step's first row from ``state[slot, kept_offset:]``, which then receives the step's last
     ``taps - 1`` inputs), silu, unit q and k per head (q times ``dim^-1/2``), ``beta = sigmoid(b)``,
-    ``g = exp(-exp(a_log) softplus(a + dt_bias))``; ``out [n, channels + 2 heads]`` float32."""
+    ``g = exp(-exp(a_log) softplus(a + dt_bias))``; ``out [n, channels + 2 heads]`` float32. ``singles``: every entry is one row."""
     _f32_rows(proj, "proj")
     _dense(conv_w, "conv_w", torch.float32, 2)
     channels, taps = conv_w.shape
@@ -2227,12 +2227,13 @@ def conv_prepare(proj: torch.Tensor, b_off: int, a_off: int, conv_w: torch.Tenso
         _dense(t, name, torch.int32, 1)
     entries = state_slots.shape[0]
     _require(q_start.shape[0] == entries + 1 and positions.shape[0] == n, "q_start/state_slots/positions disagree")
+    _require(not singles or n == entries, "single tokens: a row an entry")
     _require(channels <= b_off and b_off + heads <= proj.shape[1] and channels <= a_off and a_off + heads <= proj.shape[1],
              "beta's or the decay's columns lie outside proj")
     _check(library().dli_conv_prepare(
         _ptr(proj), proj.stride(0), int(b_off), int(a_off), _ptr(conv_w), _ptr(a_log), _ptr(dt_bias), _ptr(state),
         state.stride(0), int(kept_offset), _ptr(q_start), _ptr(positions), _ptr(state_slots), _ptr(out), out.stride(0),
-        entries, n, heads, kv_heads, dim, vdim, taps, _stream()), "conv_prepare")
+        entries, n, heads, kv_heads, dim, vdim, taps, int(bool(singles)), _stream()), "conv_prepare")
 
 
 def gated_delta_scan(prep: torch.Tensor, state: torch.Tensor, q_start: torch.Tensor, positions: torch.Tensor,

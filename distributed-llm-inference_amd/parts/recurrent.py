@@ -246,7 +246,7 @@ class GatedDelta(Mixer):
         prep = torch.empty(n, -(-width // 4) * 4, device=self.rt.device, dtype=torch.float32)[:, :width]   # rows of whole 16 bytes
         ops.conv_prepare(proj, b_off, a_off, self.conv_w, self.a_log, self.dt_bias, state, self.state_floats,
                          ctx.q_start, ctx.positions, ctx.state_slots, prep, H, self.num_kv_heads, self.head_dim,
-                         self.value_dim)
+                         self.value_dim, singles=ctx.num_decode == ctx.num_entries)
         o = torch.empty(n, self.hv, device=self.rt.device, dtype=torch.float32)
         ops.gated_delta_scan(prep, state, ctx.q_start, ctx.positions, ctx.state_slots, o, H, self.num_kv_heads,
                              self.head_dim, self.value_dim, longest=longest_to_cut(self.rt, ctx), singles=ctx.num_decode)

@@ -215,7 +215,7 @@ __device__ __forceinline__ int sum_before(int v) {   // over the lanes before th
   return s - v;
 }
 // With a table (TableChoice) the kernel looks the choices up itself and writes them and their weights: a kernel of its own for that took
-// 4.3 us a layer of a step of two rows, this one takes 4.7 without it and 4.6 with it (9,216 slots, nine a thread: some 15 more, so not there).
+// 4.3 us a layer of a step of two rows, this one takes 4.7 without it and 4.6 with it (9,216 slots, nine a thread: about as much longer as it saves, so not there).
 struct TableChoice { const int* table; const int* token_ids; int vocab, top; float* weights; };
 __device__ __forceinline__ int table_choice(const int* table, const int* token_ids, int vocab, int top, int i) {
   const int t = i / top, tok = min(max(token_ids[t], 0), vocab - 1);

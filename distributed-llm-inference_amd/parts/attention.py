@@ -190,6 +190,8 @@ class GQAttention(Mixer):
 
     # -- decode steps with few rows: the norm before and the residual sum after are fused into
     #    the two projections' kernels
+    streams_32_bit = True
+
     def streams(self, ctx: Any) -> bool:
         nh, d, n = self.num_heads, self.head_dim, ctx.num_tokens
         if not self.rt.is_bf16:

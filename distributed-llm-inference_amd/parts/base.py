@@ -131,10 +131,30 @@ def norm_key(norm: Any) -> Optional[tuple]:
     norm itself answers (``stream_key()``)."""
     if norm is not None and hasattr(norm, "stream_key"):
         return norm.stream_key()
-    if norm is None or not hasattr(norm, "fused_params"):
+    if norm is None or fused_form(norm, "fused_params") is None:
         return None
     w, eps = norm.fused_params()
     return (w.data_ptr(), float(eps))
+
+
+def fused_form(part: Any, name: str, *plain: str) -> Any:
+    """The attribute ``name`` of a part that stands for what its methods ``plain`` (none given: ``forward``) compute, such as a method
+    that does the same inside a neighbour's kernel; or ``None`` where the part has none, or has one that may compute something
+    else: a class below the one that defines it, or the object itself, defines one of ``plain`` anew. (A part that derives from
+    a built-in one and changes its ``forward`` inherits the fused forms; it must not be run as its parent.)"""
+    for scope in (vars(part), *map(vars, type(part).__mro__)):
+        if name in scope:
+            return getattr(part, name)
+        if any(p in scope for p in plain or ("forward",)):
+            return None
+    return None
+
+
+def takes_stream(part: Any, *plain: str) -> bool:
+    """Whether ``part.forward_stream`` may run in the place of its methods ``plain`` (:func:`fused_form`), in 32-bit only where the
+    class that defines it, or one below, says that it takes such a stream (``streams_32_bit``)."""
+    return (fused_form(part, "forward_stream", *plain) is not None
+            and (part.rt.is_bf16 or bool(fused_form(part, "streams_32_bit", "forward_stream"))))
 
 
 class Part:
@@ -187,8 +207,12 @@ class Part:
     def streams(self, ctx: Any) -> bool:
         """Whether this part can run ``ctx``'s step on a :class:`DecodeStream` (its
         ``forward_stream``). Parts that do not implement the fused form return False, and the
-        model then runs the step through the plain ``forward`` methods."""
+        model then runs the step through the plain ``forward`` methods. It is asked only of a part whose
+        ``forward_stream`` stands for its ``forward`` (:func:`takes_stream`)."""
         return False
+
+    # Whether ``forward_stream`` also takes the stream of a 32-bit step, whose ``ssq`` is None.
+    streams_32_bit = False
 
 
 class Embedding(Part):

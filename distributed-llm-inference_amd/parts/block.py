@@ -10,7 +10,7 @@ from typing import Any, Mapping, Optional
 
 import torch
 
-from .base import Block, DecodeStream, Part, Runtime
+from .base import Block, DecodeStream, Part, Runtime, fused_form, takes_stream
 from .linear import NormedStream, as_operand
 from .registry import register_part
 
@@ -61,9 +61,13 @@ class PreNormBlock(Block):
     def streams(self, ctx: Any, parts: Mapping[str, Part]) -> bool:
         if "feed_forward" not in parts:
             return False
-        fused_norms = all(hasattr(parts[r], "fused_params") and (self.rt.is_bf16 or parts[r].fused_params()[0].data_ptr() % 16 == 0)
-                          for r in ("mixer_norm", "feed_forward_norm"))   # (the 32-bit products read whole vectors)
-        return fused_norms and parts["mixer"].streams(ctx) and parts["feed_forward"].streams(ctx)
+        for role in ("mixer_norm", "feed_forward_norm"):
+            fused = fused_form(parts[role], "fused_params")
+            if fused is None or not (self.rt.is_bf16 or fused()[0].data_ptr() % 16 == 0):   # (the 32-bit products read whole vectors)
+                return False
+        return all(takes_stream(parts[role]) and parts[role].streams(ctx) for role in ("mixer", "feed_forward"))
+
+    streams_32_bit = True
 
     def first_norm(self, parts: Mapping[str, Part]) -> Optional[Part]:
         return parts["mixer_norm"]
@@ -185,7 +189,7 @@ class NormPair:
 
     @staticmethod
     def of(one: Part, two: Part) -> Optional["NormPair"]:
-        fused = [getattr(n, "fused_params", None) for n in (one, two)]
+        fused = [fused_form(n, "fused_params") for n in (one, two)]
         return NormPair(one, two) if all(fused) and fused[0]()[1] == fused[1]()[1] else None
 
     def pair_params(self) -> tuple:
@@ -243,7 +247,7 @@ class ParallelNormsBlock(Block):
         else:
             h1, h2 = n1.forward(x), n2.forward(x)
         y = _as_f32(parts["mixer"].forward(h1, ctx, cache))
-        if hasattr(ff, "forward_into_stream"):
+        if fused_form(ff, "forward_into_stream") is not None:
             following = NormedStream.following(ctx)
             following = following if hasattr(following, "pair_params") else None
             rows = ff.forward_into_stream(h2, ctx, x, y, following)
@@ -311,7 +315,7 @@ class ParallelScaledBlock(Block):
             h = parts["norm"].forward(x)
         y = _as_f32(parts["mixer"].forward(h, ctx, cache))
         f = _as_f32(parts["feed_forward"].forward(h, ctx)) if "feed_forward" in parts else None
-        fused = following is not None and hasattr(following, "tanh_params")
+        fused = following is not None and fused_form(following, "tanh_params") is not None
         out = self.rt.empty(*x.shape) if fused else None
         ops.tanh_norm_stream(x, a=y, b=f, a_scale=self.scales.get("mixer"),
                              b_scale=self.scales.get("feed_forward") if f is not None else None, constant=self.constant,
@@ -341,7 +345,8 @@ class SandwichNormsBlock(Block):
 
     def _add(self, x: torch.Tensor, y: torch.Tensor, out_norm: Part, following: Optional[Part], ctx: Any) -> None:
         """``x += out_norm(y)``; the rows normalised by ``following`` are left on the context where one kernel makes both."""
-        if following is not None and hasattr(out_norm, "add_normed_then") and hasattr(following, "fused_params"):
+        if (following is not None and fused_form(out_norm, "add_normed_then", "add_normed") is not None
+                and fused_form(following, "fused_params") is not None):
             NormedStream.offer(ctx, x, following, out_norm.add_normed_then(x, _as_f32(y), following))
         else:
             out_norm.add_normed(x, y, ctx)

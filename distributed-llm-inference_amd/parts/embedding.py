@@ -65,6 +65,8 @@ class TokenEmbedding(Embedding):
         ops.embed_sinusoid(self.table(), ctx.token_ids, ctx.positions, None, out, scale=self.scale)
         return out if self.norm is None else self.norm.forward_f32(out)
 
+    streams_32_bit = True
+
     def streams(self, ctx) -> bool:
         return not self.float32_rows  # the fused decode kernels keep a stream of the runtime's type
 

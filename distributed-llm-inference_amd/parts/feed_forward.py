@@ -124,6 +124,8 @@ class GatedMLP(FeedForward):
 
     FEW_ROWS = 16  # the few-row product kernels; 17 to 64 rows take the one that shares activations
 
+    streams_32_bit = True
+
     def streams(self, ctx: Any) -> bool:
         n = ctx.num_tokens
         if self.activation != "silu" or self.float32_out or self.hidden_size % 8:

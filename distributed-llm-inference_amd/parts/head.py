@@ -74,6 +74,8 @@ class LinearHead(Head):
         ops.to_float(logits, out)
         return out
 
+    streams_32_bit = True
+
     def streams(self, ctx) -> bool:
         return self.softcap == 0 and self.scale == 1.0 and (not self.rt.is_bf16 or ctx.num_tokens > self.FEW_ROWS
                                     or ops.skinny_gemm_supports(ctx.num_tokens, self.hidden_size, self.rt.dtype))

@@ -15,7 +15,7 @@ from typing import Any, Optional
 import torch
 
 from ..kernels import ops
-from .base import DecodeStream, Norm, Runtime, norm_key
+from .base import DecodeStream, Norm, Runtime, fused_form, norm_key
 
 
 def linear(rt: Runtime, x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
@@ -84,7 +84,7 @@ def finish_residual(rt: Runtime, stream: DecodeStream, partial: torch.Tensor, bi
     """The residual sum of a product that left partial sums, and with it the norm that follows
     where that is known, the rows are many enough for it to pay and narrow enough for one
     workgroup each."""
-    fused = following.fused_params() if following is not None and hasattr(following, "fused_params") else None
+    fused = following.fused_params() if following is not None and fused_form(following, "fused_params") is not None else None
     rows, width = stream.x.shape
     if (fused is not None and rows >= NORM_WITH_THE_SUM_FROM_ROWS and width <= ops.MID_NORMED_WIDTH
             and fused[0].shape[0] == width):

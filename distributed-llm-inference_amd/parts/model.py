@@ -15,7 +15,7 @@ from typing import Any, Mapping, Optional, Sequence
 import torch
 
 from ..kernels import ops
-from .base import Part, Runtime
+from .base import Part, Runtime, fused_form, takes_stream
 from .linear import NormedStream
 from .registry import build_part
 from .spec import ModelSpec, WeightSpec
@@ -163,9 +163,17 @@ class Model:
         # the plain kernels issued from the loop in C (2.1 against 1.7 ms for 64 tokens at the 1B sizes).
         if not 0 < ctx.num_tokens <= self.STREAM_ROWS or ctx.num_decode != ctx.num_entries:
             return False
-        if not (self.embedding.streams(ctx) and self.head.streams(ctx) and hasattr(self.final_norm, "fused_params")):
+        if not (takes_stream(self.embedding, "forward", "forward_step") and self.embedding.streams(ctx)
+                and takes_stream(self.head) and self.head.streams(ctx) and fused_form(self.final_norm, "fused_params") is not None):
             return False
-        return all(hasattr(l.block, "forward_stream") and l.block.streams(ctx, l.parts) for l in self.layers)
+        return all(takes_stream(l.block) and l.block.streams(ctx, l.parts) for l in self.layers)
+
+    @staticmethod
+    def _first_norm(layer: BuiltLayer) -> Optional[Part]:
+        """The norm that a layer meets the stream with, for the block before it. (A block that derives from another and arranges
+        its parts anew does not meet it with the other's.)"""
+        first = fused_form(layer.block, "first_norm")
+        return first(layer.parts) if first is not None else None
 
     def _forward_stream(self, ctx: Any, caches: Sequence[Any]) -> torch.Tensor:
         stream = self.embedding.forward_stream(ctx.token_ids)
@@ -215,12 +223,12 @@ class Model:
             for i, (layer, cache) in enumerate(zip(order, caches)):
                 if layer.block.takes_following:
                     # (the final norm reads the wanted rows: it follows where those are all rows, in order)
-                    after = (order[i + 1].block.first_norm(order[i + 1].parts) if i + 1 < len(order)
+                    after = (self._first_norm(order[i + 1]) if i + 1 < len(order)
                              else self.final_norm if getattr(ctx, "all_rows_wanted", False) else None)
                     x, delta = layer.block.forward(x, delta, ctx, cache, layer.parts, following=after)
                 else:
                     if layer.block.asks_following:
-                        NormedStream.follow(ctx, order[i + 1].block.first_norm(order[i + 1].parts) if i + 1 < len(order) else None)
+                        NormedStream.follow(ctx, self._first_norm(order[i + 1]) if i + 1 < len(order) else None)
                     x, delta = layer.block.forward(x, delta, ctx, cache, layer.parts)
         k = ctx.logit_rows.shape[0]
         if k == 0:

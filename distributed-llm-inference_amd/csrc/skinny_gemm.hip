@@ -133,8 +133,10 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
   // What follows the last product is a chain that nothing hides, so it is kept short. With one row
   // tile and one group of waves (SHORT) all waves leave their parts in LDS and thread t makes
   // output t of each tile: element t % 4 of lane t / 4 of the product's result, that is row
-  // t / 4 % 16 and feature 4 (t / 64) + t % 4. Otherwise k-split waves 1.. hand their parts to wave 0.
-  constexpr bool SHORT = MT == 1 && NS == 1;
+  // t / 4 % 16 and feature 4 (t / 64) + t % 4. Otherwise k-split waves 1.. hand their parts to wave 0. So do q, k and v,
+  // which wave 0 stores four values at a time (a value a thread, 2 and 8 rows: 6.9 us for 6.4 and 6.8 for 6.7 at the 1B sizes,
+  // 10.4 for 9.0 and 9.9 for 9.0 at the 1.7B sizes, 13.3 for 11.9 and 12.6 for 11.7 at the 3B sizes).
+  constexpr bool SHORT = MT == 1 && NS == 1 && EPI != EPI_QKV;
   constexpr int KR = SHORT ? KS : (KS > 1 ? KS - 1 : 1);
   __shared__ float4v red[KR][NS][NT][NA][MT][64];
 
@@ -163,9 +165,8 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
     return reinterpret_cast<const bf16x8*>(TILED ? base + (s / 4) * 2048 + q * 512 : base + s * 32 + q * 8);
   };
 
-  // What the end adds to the product (the stream's values, the bias, and for q/k/v the rows' slots,
-  // cosines and sines) is asked for now, so that the end does not wait for a trip to memory of its
-  // own. In every wave and for every element (an element past the edge reads the edge's and is not
+  // What the end adds to the product (the stream's values, the bias) is asked for now, so that the end does not wait for a
+  // trip to memory of its own. In every wave and for every element (an element past the edge reads the edge's and is not
   // stored; a missing bias is a resource without bytes, which reads zeros): a load under a
   // condition is waited for on the spot, one trip to memory after the other, and leaves the count
   // of loads on their way unknown to everything behind it.
@@ -195,37 +196,18 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
     b.raw = __builtin_amdgcn_raw_buffer_load_b16(bres, n * 2, 0, 0);
     return b.v;
   };
-  // (SHORT q/k/v: a thread adds up its element's rotary partner too, eight features on)
-  constexpr int BA = SHORT && EPI == EPI_QKV ? 2 : NA;
-  bf16_t b_at[NT][BA][EL];
+  bf16_t b_at[NT][NA][EL];
   auto load_bias = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
-      for (int a = 0; a < BA; ++a)
+      for (int a = 0; a < NA; ++a)
 #pragma unroll
-        for (int i = 0; i < EL; ++i) {
-          const int n = (tile0 + j) * 16 + (BA > NA && a == 1 ? (e_n ^ 8) + i : e_n + i);
-          b_at[j][a][i] = bias_at(min(n, N - 1) + (BA > NA ? 0 : a * up_offset));
-        }
+        for (int i = 0; i < EL; ++i) b_at[j][a][i] = bias_at(min((tile0 + j) * 16 + e_n + i, N - 1) + a * up_offset);
   };
-  if constexpr (MT == 1) load_bias();  // (several row tiles: at the end, the registers are taken)
-  int slot_at = -1;
-  float cs_at[EPI == EPI_QKV ? NT : 1][EL], sn_at[EPI == EPI_QKV ? NT : 1][EL];
-  if constexpr (EPI == EPI_QKV) {
-    const int half = qr.head_dim / 2, mm = min(e_row, M - 1);
-    slot_at = qr.slots[mm];
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      const int t_in = min(tile0 + j, (N - 1) / 16) % (qr.head_dim / 16);
-      const float* at = qr.angles + (int64_t)mm * 2 * half + 8 * t_in + 4 * (e_grp & 1) + e_i;  // the rotary pairs
-#pragma unroll
-      for (int i = 0; i < EL; ++i) {
-        cs_at[j][i] = at[i];
-        sn_at[j][i] = at[half + i];
-      }
-    }
-  }
+  // (several row tiles: at the end, the registers are taken; q/k/v: there as well, with what the rotation needs)
+  constexpr bool EARLY = MT == 1 && EPI != EPI_QKV;
+  if constexpr (EARLY) load_bias();
 
   const bf16_t* xrow[MT];
   float rs[MT];
@@ -292,13 +274,6 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
   };
   int blocks = (s_end - s) / 4;
   Block b0, b1;
-  // The second block sets out with the first: what is waited for before the first product (the
-  // sums of squares, the merge) then hides both trips. (A wave of one block reads that again.)
-  auto fetch_second = [&]() __attribute__((always_inline)) {
-    const int at = blocks > 1 ? s + 4 : (blocks > 0 ? s : 0);
-    fetch_rows(b1, at);
-    fetch_weights(b1, at);
-  };
   if constexpr (NORM) {
     // rs[m] from the parts of sum x^2 that the producer of x left. The parts are dealt out to
     // all lane groups of all waves (group q of W*4 takes the parts q, q + 4W, ...), eight loads
@@ -325,7 +300,6 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
     if (TILED || blocks > 0) {
       fetch_rows(b0, blocks > 0 ? s : 0);
       fetch_weights(b0, blocks > 0 ? s : 0);
-      if constexpr (MT == 1) fetch_second();
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -391,11 +365,6 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
   }
   if constexpr (!NORM) {
     if (blocks > 0) fetch_rows(b0, s);
-    if constexpr (MERGED) {
-      if (blocks > 1) fetch_rows(b1, s + 4);
-    } else if constexpr (MT == 1) {
-      if (blocks > 0) fetch_second();
-    }
   }
   if constexpr (MT > 1) {
     // several row tiles: one body for every turn (the registers do not hold two whole blocks)
@@ -408,7 +377,16 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
       multiply(b0);
       if (more) b0 = b1;
     }
-  } else if (blocks > 0) {
+  } else if (blocks == 1) {
+    multiply(b0);
+    s += 4;
+  } else if (blocks > 1) {
+    // (The second block is asked for here and not with the first, in front of the sums of squares: a wave of one block has
+    // none, and its rows and norm weights stand in the vector cache's way. Gate and up, 8 and 16 rows, asked for there and
+    // here: 6.6 and 5.2 us, 6.8 and 5.3 at the 135M sizes, 15.7 and 15.8, 16.4 and 16.9 at the 1B sizes.)
+    fetch_rows(b1, s + 4);
+    if constexpr (!MERGED) fetch_weights(b1, s + 4);
+    __builtin_amdgcn_sched_barrier(0);
     while (blocks >= 4) {
       multiply(b0);
       fetch_rows(b0, s + 8);
@@ -430,7 +408,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
       multiply(b0);
     } else {
       multiply(b0);
-      if (blocks == 2) multiply(b1);
+      multiply(b1);
     }
     s = s_begin + (s_end - s_begin) / 4 * 4;
   }
@@ -456,19 +434,18 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
     // this thread's elements: the waves' parts, all read before the first is added, in wave order
     const int m = e_row;
     const bool here = (int)threadIdx.x < 256 && m < M;
-    float y[NT][BA];
+    float y[NT][NA];
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-      float part[BA][KS];
+      float part[NA][KS];
 #pragma unroll
-      for (int a = 0; a < BA; ++a) {
-        const float* src = reinterpret_cast<const float*>(&red[0][0][j][BA > NA ? 0 : a][0][0]) +
-                           (BA > NA && a == 1 ? (threadIdx.x % 256) ^ 128 : threadIdx.x % 256);
+      for (int a = 0; a < NA; ++a) {
+        const float* src = reinterpret_cast<const float*>(&red[0][0][j][a][0][0]) + threadIdx.x % 256;
 #pragma unroll
         for (int wv = 0; wv < KS; ++wv) part[a][wv] = src[wv * (NT * NA * 256)];
       }
 #pragma unroll
-      for (int a = 0; a < BA; ++a) {
+      for (int a = 0; a < NA; ++a) {
         float sum = part[a][0];
 #pragma unroll
         for (int wv = 1; wv < KS; ++wv) sum += part[a][wv];
@@ -480,30 +457,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       const int tile = tile0 + j, n = tile * 16 + e_n;
-      if (EPI == EPI_QKV) {
-        if (!here || tile * 16 >= N) continue;
-        const int d = qr.head_dim, half = d / 2;
-        const int head = tile * 16 / d, t_in = (tile * 16 - head * d) / 16;
-        const float v = (float)(bf16_t)y[j][0], partner = (float)(bf16_t)y[j][BA - 1];
-        const int jt = EPI == EPI_QKV ? j : 0;
-        if (head < qr.q_heads + qr.kv_heads) {  // rotary
-          const float cs = cs_at[jt][0], sn = sn_at[jt][0];
-          const bf16_t r = e_grp < 2 ? (bf16_t)(v * cs - partner * sn) : (bf16_t)(v * cs + partner * sn);
-          const int dim = (e_grp < 2 ? 0 : half) + 8 * t_in + 4 * (e_grp & 1) + e_i;
-          if (head < qr.q_heads) {
-            reinterpret_cast<bf16_t*>(out)[(int64_t)m * ldo + head * d + dim] = r;
-          } else if (slot_at >= 0) {
-            const int64_t page = slot_at / qr.page_size;
-            const int off = slot_at - (int)page * qr.page_size;
-            qr.k_pages[((page * qr.kv_heads + (head - qr.q_heads)) * qr.page_size + off) * d + dim] = r;
-          }
-        } else if (slot_at >= 0) {
-          const int64_t page = slot_at / qr.page_size;
-          const int off = slot_at - (int)page * qr.page_size;
-          const int hv = head - qr.q_heads - qr.kv_heads;
-          qr.v_pages[((page * qr.kv_heads + hv) * d + 16 * t_in + e_n) * qr.page_size + off] = (bf16_t)v;
-        }
-      } else if (EPI == EPI_RESIDUAL) {
+      if (EPI == EPI_RESIDUAL) {
         const bf16_t summed = (bf16_t)((float)old_s[EPI == EPI_RESIDUAL ? j : 0][0][0] + (float)(bf16_t)y[j][0]);
         const bool in = here && n < N;
         if (in) stream[(int64_t)m * lds_ + n] = summed;
@@ -559,7 +513,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
   // lane holds y[m = 16t + col][n = 16*tile + 4*grp + i]
   if constexpr (!SHORT) {
   if (ks == 0) {
-  if constexpr (MT > 1) load_bias();
+  if constexpr (!EARLY) load_bias();
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     const int tile = tile0 + j;
@@ -581,7 +535,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
         const int d = qr.head_dim, half = d / 2;
         const int head = tile * 16 / d, t_in = (tile * 16 - head * d) / 16;
         const bool rotary = head < qr.q_heads + qr.kv_heads;
-        const int slot = slot_at, jt = EPI == EPI_QKV ? j : 0;
+        const int mm = min(m, M - 1), slot = qr.slots[mm];
         float v[4], partner[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -590,10 +544,12 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
         }
         if (rotary) {
           const int j = 8 * t_in + 4 * (grp & 1);  // first of this lane's four rotary pairs
+          const float4v cs = *reinterpret_cast<const float4v*>(qr.angles + ((int64_t)mm * 2 + 0) * half + j);
+          const float4v sn = *reinterpret_cast<const float4v*>(qr.angles + ((int64_t)mm * 2 + 1) * half + j);
           bf16_t r[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            r[i] = grp < 2 ? (bf16_t)(v[i] * cs_at[jt][i] - partner[i] * sn_at[jt][i]) : (bf16_t)(v[i] * cs_at[jt][i] + partner[i] * sn_at[jt][i]);
+            r[i] = grp < 2 ? (bf16_t)(v[i] * cs[i] - partner[i] * sn[i]) : (bf16_t)(v[i] * cs[i] + partner[i] * sn[i]);
           const int dim = (grp < 2 ? 0 : half) + j;
           bf16_t* dst = nullptr;
           if (head < qr.q_heads) {
@@ -672,7 +628,7 @@ __global__ void embedding_ssq_kernel(const bf16_t* __restrict__ table, const int
   x, ldx, ssq_in, ssq_parts, norm_w, eps, w, bias, out, ldo, stream_buf, lds_, ssq_out, M, N, K, up_offset, qr, glu, stream
 
 // The products that open the two halves of a decode layer (q/k/v with rotation and cache write, gate and up), with the
-// row norm inside: at most 16 rows, weights in tile order, k split over the KS waves of a workgroup,
+// row norm inside: at most four rows, weights in tile order, k split over the KS waves of a workgroup,
 // which owns NT tiles. What bounds such a launch beside its weights is the time until they are asked
 // for and the vector cache, which accepts 64 bytes a cycle and compute unit:
 //  - The workgroup normalises the rows once, into LDS, and its waves read their fragments from there.
@@ -682,7 +638,7 @@ __global__ void embedding_ssq_kernel(const bf16_t* __restrict__ table, const int
 //    anything is waited for (loads come back in their order), with few instructions on the way:
 //    through buffer resources, which count what lies past their end as zeros, so that no load needs a condition
 //    or a bound of its own. What only the end needs is asked for last.
-// MR: rows whose pieces are asked for at the start (further rows afterwards).
+// MR: one row, or up to four.
 // In decode steps of one row from start to end of the launch (135M and 1B sizes): q/k/v 2.7 -> 1.7 us and 4.6 -> 2.5.
 struct NormedArgs {
   const bf16_t* x;
@@ -707,7 +663,7 @@ __global__ __launch_bounds__(KS * 64) void normed_tiles_kernel(NormedArgs p) {
   static_assert(EPI == EPI_SWIGLU || EPI == EPI_QKV, "the products behind a norm");
   constexpr int NA = EPI == EPI_SWIGLU ? 2 : 1;  // weight row sets per tile (gate and up)
   constexpr int BA = 2;                          // sums a thread makes per tile: gate and up, or a feature and its rotary partner
-  constexpr int PARTS = MR == 1 ? 2 : MR;         // loads of 64 parts of the sums of squares a wave asks for at the start
+  constexpr int PARTS = MR == 1 ? 2 : MR;        // loads of 64 parts of the sums of squares a wave asks for at the start
   constexpr int PRE = KS == 4 ? 3 : 2;           // pieces of 256 values of the rows likewise
   constexpr unsigned OUTSIDE = 0x80000000u;      // an offset past the end of every resource here
   typedef short short4v __attribute__((ext_vector_type(4)));
@@ -748,16 +704,16 @@ __global__ __launch_bounds__(KS * 64) void normed_tiles_kernel(NormedArgs p) {
   auto ask_gain = [&](Gain& g, int j) __attribute__((always_inline)) {
     g.raw = __builtin_amdgcn_raw_buffer_load_b128(gres, ((ks + j * KS) * 256 + lane * 4) * 4, 0, 0);
   };
-  auto ask_rows = [&](Four (&v)[MR], int j, int m0) __attribute__((always_inline)) {
+  auto ask_rows = [&](Four (&v)[MR], int j) __attribute__((always_inline)) {   // (a row past the last lies past the resource's end)
     const int k = (ks + j * KS) * 256 + lane * 4;
     const unsigned at = k < K ? (unsigned)(k * 2) : OUTSIDE;
 #pragma unroll
-    for (int u = 0; u < MR; ++u) v[u].raw = __builtin_amdgcn_raw_buffer_load_b64(xres, at + (unsigned)((m0 + u) * p.ldx * 2), 0, 0);
+    for (int u = 0; u < MR; ++u) v[u].raw = __builtin_amdgcn_raw_buffer_load_b64(xres, at + (unsigned)(u * p.ldx * 2), 0, 0);
   };
 #pragma unroll
   for (int j = 0; j < PRE; ++j) {
     ask_gain(gain[j], j);
-    ask_rows(piece[j], j, 0);
+    ask_rows(piece[j], j);
   }
   // weights: this wave's share of the blocks of 128 k
   const int whole = (K + 127) / 128, c0 = whole * ks / KS, blocks = whole * (ks + 1) / KS - c0;
@@ -821,8 +777,8 @@ __global__ __launch_bounds__(KS * 64) void normed_tiles_kernel(NormedArgs p) {
   sum = add_halves(sum, sum);
   sum = add_rows(sum, sum);
   if (even) {
-    if (M <= 8) sum += row_ror<8>(sum);
-    if (M <= 4) sum += row_ror<4>(sum);
+    sum += row_ror<8>(sum);
+    sum += row_ror<4>(sum);
     if (M == 1) sum = quad_sum(sum);
     else if (M == 2) sum = quad_pairs(sum);
   }
@@ -834,33 +790,31 @@ __global__ __launch_bounds__(KS * 64) void normed_tiles_kernel(NormedArgs p) {
 #pragma unroll
   for (int wv = 0; wv < KS; ++wv) total += part[wv];
   const float rs = rsqrtf(total / (float)K + p.eps);
-  auto put_rows = [&](const Four (&v)[MR], const Gain& g, int j, int m0) __attribute__((always_inline)) {
+  auto put_rows = [&](const Four (&v)[MR], const Gain& g, int j) __attribute__((always_inline)) {
     const int k = (ks + j * KS) * 256 + lane * 4;
 #pragma unroll
     for (int u = 0; u < MR; ++u)
-      if (m0 + u < M) {
-        const float rsm = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rs), m0 + u));
+      if (u < M) {
+        const float rsm = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rs), u));
         Four h;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {  // (past K values and weights are zeros)
           const float normed = (float)(bf16_t)((float)v[u].e[i] * rsm);
           h.e[i] = (bf16_t)(g.e[i] * normed);
         }
-        if (k < whole * 128) *reinterpret_cast<u32x2*>(xs + (m0 + u) * row + k) = h.raw;
+        if (k < whole * 128) *reinterpret_cast<u32x2*>(xs + u * row + k) = h.raw;
       }
   };
 #pragma unroll
   for (int j = 0; j < PRE; ++j)
-    if ((ks + j * KS) * 256 < whole * 128) put_rows(piece[j], gain[j], j, 0);
-  // what did not fit the start: further rows, further pieces of long rows
-  for (int j = 0; (ks + j * KS) * 256 < whole * 128; ++j)
-    for (int m0 = j < PRE ? MR : 0; m0 < M; m0 += MR) {
-      Four v[MR];
-      Gain g;
-      ask_gain(g, j);
-      ask_rows(v, j, m0);
-      put_rows(v, g, j, m0);
-    }
+    if ((ks + j * KS) * 256 < whole * 128) put_rows(piece[j], gain[j], j);
+  for (int j = PRE; (ks + j * KS) * 256 < whole * 128; ++j) {   // further pieces of long rows
+    Four v[MR];
+    Gain g;
+    ask_gain(g, j);
+    ask_rows(v, j);
+    put_rows(v, g, j);
+  }
   __syncthreads();
 
   float4v acc[NT][NA];
@@ -948,15 +902,31 @@ static bool lds_refused(const void* kernel, size_t lds) {
          hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024) != hipSuccess;
 }
 
-// Whether normed_tiles_kernel takes the product: its rows leave room in LDS for two workgroups on a
-// compute unit, and lie within what its 31-bit offsets reach. Four blocks of weights on their way where every
-// wave has three or more, else two; a gated pair of two tiles takes the registers of two.
+// Whether normed_tiles_kernel takes the product. Its workgroups each normalise all rows before their first product, which with
+// more rows costs more than the shared reads save, and the lanes' sums of squares go by rows that are a power of two. Cold, us with
+// skinny_gemm_kernel and with this one at 1, 2, 3, 4, 8 and 16 rows:
+//   q/k/v    135M sizes  4.1 3.9  4.2 4.5  4.2 4.3  4.2 4.4  4.3 5.1  4.4 6.2      1B    6.4 5.3  6.4 5.8  6.5 5.8  6.5 5.8  6.7 6.8  7.2 8.1
+//            1.7B        8.9 8.7  9.0 9.1  9.0 9.7  9.1 9.2  9.0 9.8  9.9 12.1     3B    11.8 9.8  11.9 10.4  12.0 11.8  11.3 10.3  11.7 11.6
+//            width 1,536, 24 heads on 24     6.9 7.1  6.9 7.6  6.9 7.6  7.0 7.5  7.3 8.5  8.0 10.6
+//   gate/up  1B          -  15.4 14.8  15.3 16.0  15.3 15.0  15.8 16.4  16.9 19.0  3B    -  22.1 21.0  21.4 22.5  21.5 20.4  21.7 21.5
+//            width 1,024, 4,096 wide         -  6.5 6.7  6.0 6.6  6.1 6.8  6.2 6.5  6.4 7.6
+// So: one row, but not a short one whose tiles are more than the compute units; two and four rows of 2,048 values and more; three
+// such where the tiles are no more than the units (a gated product's half are as many: never).
+extern "C" int dli_normed_tiles_ahead(int M, int N, int K, int gated, int units) {
+  const bool few = (N + 15) / 16 <= units, deep = K >= 2048;
+  if (M == 1) return few || deep;
+  return deep && (M == 2 || M == 4 || (M == 3 && few && !gated));
+}
+
+// Besides, its rows have to leave room in LDS for two workgroups on a compute unit, and to lie within what its 31-bit offsets
+// reach. Four blocks of weights on their way where every wave has three or more, else two; a gated pair of two tiles takes the
+// registers of two.
 template <int KS, int NT, int EPI>
 static bool launch_normed_tiles(SK_PARAMS) {
   constexpr int PER = NT * (EPI == EPI_SWIGLU ? 2 : 1);
   const size_t lds = (size_t)M * normed_row(K) * 2;
-  if (lds + (size_t)KS * PER * 1024 + 1024 > 80 * 1024 || N % 16 != 0 || ldx > INT32_MAX / 64 || ssq_parts > INT32_MAX / 256 ||
-      (int64_t)N + up_offset > INT32_MAX / 4)
+  if (!dli_normed_tiles_ahead(M, N, K, EPI == EPI_SWIGLU, dli_compute_units()) || lds + (size_t)KS * PER * 1024 + 1024 > 80 * 1024 || N % 16 != 0 ||
+      ldx > INT32_MAX / 64 || ssq_parts > INT32_MAX / 256 || (int64_t)N + up_offset > INT32_MAX / 4)
     return false;
   const NormedArgs args{(const bf16_t*)x, ssq_in, norm_w, (const bf16_t*)w, (const bf16_t*)bias, (bf16_t*)out, ldo, (int)ldx,
                         ssq_parts, M, N, K, up_offset, eps, qr, glu};
@@ -969,14 +939,12 @@ static bool launch_normed_tiles(SK_PARAMS) {
   if constexpr (PER <= 2) {
     if ((K + 127) / 128 / KS >= 3) {
       if (M == 1) NORMED_LAUNCH(4, 1)
-      else if (M <= 4) NORMED_LAUNCH(4, 4)
-      else NORMED_LAUNCH(4, 8)
+      else NORMED_LAUNCH(4, 4)
       return true;
     }
   }
   if (M == 1) NORMED_LAUNCH(2, 1)
-  else if (M <= 4) NORMED_LAUNCH(2, 4)
-  else NORMED_LAUNCH(2, 8)
+  else NORMED_LAUNCH(2, 4)
 #undef NORMED_LAUNCH
   return true;
 }

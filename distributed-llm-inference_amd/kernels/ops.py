@@ -41,6 +41,7 @@ _SIGNATURES = {
     "dli_skinny4_tile_features": [_c_int, _c_int],
     "dli_rope_kv_write": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int,
                           _c_int, _c_int, _c_int, _c_int, _c_ptr],
+    "dli_normed_tiles_ahead": [_c_int, _c_int, _c_int, _c_int, _c_int],
     "dli_gemm_f32_rule": [_c_int, _c_int, _c_int],
     "dli_gemm_f32_normed": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_ptr, _c_ptr,
                             _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr],
@@ -1092,6 +1093,12 @@ def tile_weights_qkv_rope(w: torch.Tensor, q_heads: int, kv_heads: int, head_dim
     _require(w.shape[0] == (q_heads + 2 * kv_heads) * head_dim, "w must hold the q, k and v heads")
     order = qkv_rope_feature_order(q_heads, kv_heads, head_dim).to(w.device)
     return tile_weights(w[order].contiguous(), whole_blocks=False)
+
+
+def normed_tiles_ahead(rows: int, n: int, k: int, gated: bool, units: int) -> bool:
+    """Whether a few-row product behind a norm (q/k/v with the rotation, or ``gated``; ``n`` features, of one half where gated)
+    runs the kernel that normalises the rows once a workgroup (where that takes the sizes at all), and not the general one."""
+    return bool(library().dli_normed_tiles_ahead(rows, n, k, int(gated), units))
 
 
 def skinny_gemm_qkv_rope(x: torch.Tensor, w_tiled: torch.Tensor, q_out: torch.Tensor, angles: torch.Tensor,

@@ -197,7 +197,7 @@ class GQAttention(Mixer):
         if not self.rt.is_bf16:
             table = self.position.rotary_table()
             return (not self.shares_kv and table is not None and table.dim == d and ctx.num_decode == ctx.num_entries
-                    and ops.gemm_f32_normed_supports(n, self.w_qkv))
+                    and ops.gemm_f32_normed_supports(n, self.w_qkv) and ops.gemm_f32_normed_ahead(n, *self.w_qkv.shape))
         if not (self.rt.is_bf16 and ctx.num_decode == ctx.num_entries and self.hidden_size % 8 == 0
                 and ops.attention_mfma_supports(d, ctx.page_size, self.rt.dtype)):
             return False

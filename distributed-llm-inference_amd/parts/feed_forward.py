@@ -131,7 +131,7 @@ class GatedMLP(FeedForward):
         if self.activation != "silu" or self.float32_out or self.hidden_size % 8:
             return False
         if not self.rt.is_bf16:
-            return ops.gemm_f32_normed_supports(n, self.w_gate_up)
+            return ops.gemm_f32_normed_supports(n, self.w_gate_up) and ops.gemm_f32_normed_ahead(n, *self.w_gate_up.shape)
         if n > self.FEW_ROWS:
             return (self.w_gate_up_tiled is not None and self.w_down_tiled is not None
                     and ops.mid_gemm_supports(n, self.hidden_size, self.rt.dtype)

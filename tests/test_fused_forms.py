@@ -92,6 +92,15 @@ def test_a_pre_norm_block_asks_for_the_parts_own_arithmetic(changed):
     assert block.streams(ctx, parts) == (changed is None)
 
 
+@pytest.mark.parametrize("role", ["mixer", "feed_forward"])
+def test_a_32_bit_step_is_fused_where_that_is_ahead(role):
+    block, parts = _pre_norm(ROLES)
+    matrix = {"mixer": "w_qkv", "feed_forward": "w_gate_up"}[role]
+    setattr(parts[role], matrix, torch.zeros(8256, 64))   # more columns than three rows and more are normalised for again
+    ctx = lambda n: SimpleNamespace(num_tokens=n, num_decode=n, num_entries=n, page_size=16)
+    assert block.streams(ctx(2), parts) and not block.streams(ctx(3), parts)
+
+
 @pytest.mark.parametrize("changed", [False, True])
 def test_a_parallel_block_adds_what_its_feed_forward_computes(changed, monkeypatch):
     """On the CPU, with plain additions in the kernels' place: ones from the experts, halved by a class of one's own."""

@@ -121,6 +121,13 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
   return total;
 }
 
+// A component of a rotated pair: `own` turned by the angle's cosine and sine, the sine with the pair's sign (negative for the first
+// component). The one product is rounded, the other goes into the sum unrounded, written out so that every kernel that
+// rotates 32-bit values gives the same bits: a request's keys do not depend on which of them a step takes.
+__device__ __forceinline__ float rotated(float own, float other, float cosine, float signed_sine) {
+  return fmaf(own, cosine, other * signed_sine);
+}
+
 // Page of a tile of sixteen keys, page size in tiles. A quotient by a number that the compiler does not know costs some
 // twenty instructions, eight cycles each where one waits for the other, and an attention kernel's waves need several of them
 // before their first keys are asked for: so the host hands over 2^32 / tiles, rounded up, whose product's upper

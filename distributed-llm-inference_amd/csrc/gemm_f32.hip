@@ -245,7 +245,7 @@ __global__ __launch_bounds__(64 * KW) void gemm_f32_few_kernel(GfArgs p, GfAroun
       if constexpr (FORM == GF_GLU) {
         if (i < 8 && n0 + i < p.n / 2) p.out[(int64_t)row * p.ldo + n0 + i] = silu<float>(sum[e]) * other[e];
       } else {
-        const float v = rotates ? sum[e] * c[e] + other[e] * sn[e] : sum[e];
+        const float v = rotates ? rotated(sum[e], other[e], c[e], sn[e]) : sum[e];
         const int d = feature - head * x.head_dim;
         if (head < x.q_heads) {
           p.out[(int64_t)row * p.ldo + feature] = v;

@@ -81,8 +81,8 @@ __global__ __launch_bounds__(256) void rope_kv_write_kernel(
   const int off = slot >= 0 ? slot % page_size : 0;
   while (true) {
     if (it.kind == 0) {
-      const T y1 = from_f32<T>(it.x1 * cs[it.i] - it.x2 * sn[it.i]);
-      const T y2 = from_f32<T>(it.x2 * cs[it.i] + it.x1 * sn[it.i]);
+      const T y1 = from_f32<T>(rotated(it.x1, it.x2, cs[it.i], -sn[it.i]));
+      const T y2 = from_f32<T>(rotated(it.x2, it.x1, cs[it.i], sn[it.i]));
       if (it.head < q_heads) {
         T* h = row + (int64_t)it.head * head_dim;
         h[it.i] = y1;
@@ -140,8 +140,8 @@ __global__ __launch_bounds__(256) void rope_kv_write_token_kernel(
       const int head = idx / half, i = idx - head * half;
       T* h = row + (int64_t)head * head_dim;
       const float x1 = to_f32(h[i]), x2 = to_f32(h[i + half]);
-      const T y1 = from_f32<T>(x1 * cs[i] - x2 * sn[i]);
-      const T y2 = from_f32<T>(x2 * cs[i] + x1 * sn[i]);
+      const T y1 = from_f32<T>(rotated(x1, x2, cs[i], -sn[i]));
+      const T y2 = from_f32<T>(rotated(x2, x1, cs[i], sn[i]));
       if (head < q_heads) {
         h[i] = y1;
         h[i + half] = y2;
@@ -261,8 +261,8 @@ __global__ __launch_bounds__(256) void rope_kv_write_rows_kernel(
       for (int e = 0; e < VEC; ++e) {
         const float c = cs[r * half + j * VEC + e], sv = sn[r * half + j * VEC + e];
         const float x1 = to_f32(lo[u][e]), x2 = to_f32(hi[u][e]);
-        ylo[e] = from_f32<T>(x1 * c - x2 * sv);
-        yhi[e] = from_f32<T>(x2 * c + x1 * sv);
+        ylo[e] = from_f32<T>(rotated(x1, x2, c, -sv));
+        yhi[e] = from_f32<T>(rotated(x2, x1, c, sv));
       }
       T* dst = base + r * row_stride + (int64_t)head * head_dim + j * VEC;
       if (head >= q_heads)

@@ -1,5 +1,5 @@
 """The 32-bit few-row products behind a norm: bit for bit what the norm, product and activation kernels give one after the
-other; rotated q and k as far from 64 bits as rounding of angle, product and sum allows."""
+other, and so for rotated q and k."""
 
 import pytest
 import torch
@@ -49,8 +49,5 @@ def test_qkv_behind_a_norm_rotated(ops, m, heads, kv, d, k, page, bias):
     ops.gemm_f32(normed, w, qkv, bias=b)
     ops.rope_kv_write(qkv, positions, inv_freq, d, slots, pages[0], pages[2], heads, kv, d)
     ops.gemm_f32_qkv_rope(x, w, q, norm_w, 1e-5, positions, inv_freq, slots, pages[1], pages[3], bias=b)
-    # the two products and the sum of a rotation may be contracted the one way or the other: one rounding of a product, 2^-24
-    # of a value whose partner is up to six times its size
-    for got, want in ((q, qkv[:, :heads * d]), (pages[1], pages[0])):
-        assert (got - want).abs().max().item() <= 2 ** -23 * 8 * want.abs().max().item()
+    assert torch.equal(q, qkv[:, :heads * d]) and torch.equal(pages[1], pages[0])
     assert torch.equal(pages[3], pages[2])

@@ -1104,6 +1104,18 @@ extern "C" int dli_attention_prefill_tile_rows(int head_dim, int q_heads, int kv
   return hw == 0 ? PF_TILE_ROWS : (4 / hw) * 32;
 }
 
+// LDS of the states of four waves of a decode workgroup.
+static size_t decode_states(int group, int head_dim) {
+  return (size_t)4 * (head_dim / 16) * 4 * (group < 16 ? group : 16) * sizeof(float4v);
+}
+
+// Waves of a decode workgroup, `group` query heads a kv head: eight where every workgroup has a compute unit to itself (few keys then
+// need no second run, whose merge costs more than it saves: one_run_keys in parts/attention_kernels.py has the figures), with more workgroups four, of
+// which several share a unit. The waves' states have to fit 48 KB of LDS: heads of 128 in groups of up to twelve, of 112 up to 13.
+extern "C" int dli_attention_decode_waves(int64_t workgroups, int group, int head_dim, int units) {
+  return workgroups <= units && 2 * decode_states(group, head_dim) <= 48 * 1024 ? 8 : 4;
+}
+
 // merge: whether the partial results of more than one run of keys are merged into `out` here, or
 // left in part_o / part_ml for the kernel that reads them next.
 static int attention_decode(const void* q, int64_t q_stride, const void* k_pages, const void* v_pages,
@@ -1122,11 +1134,8 @@ static int attention_decode(const void* q, int64_t q_stride, const void* k_pages
   // with counters the last workgroup of each (request, kv head, head tile) merges
   const bool self_merging = merge && arrivals != nullptr && splits >= 2 && splits <= MERGE_SPLITS;
   unsigned* counters = self_merging ? arrivals : nullptr;
-  // Eight waves where every workgroup has a compute unit to itself: few keys then need no second run, whose merge costs more than
-  // it saves (planned_splits has the figures); with more workgroups four, of which several share a unit. The waves' states
-  // have to fit LDS.
-  const size_t lds = (size_t)4 * (head_dim / 16) * 4 * (group < 16 ? group : 16) * sizeof(float4v);  // of four waves
-  const bool eight = (int64_t)splits * kv_heads * head_tiles * requests <= dli_compute_units() && 2 * lds <= 48 * 1024;
+  const size_t lds = decode_states(group, head_dim);
+  const bool eight = dli_attention_decode_waves((int64_t)splits * kv_heads * head_tiles * requests, group, head_dim, dli_compute_units()) == 8;
 #define DECODE_LAUNCH(N, NW)                                                                      \
     attention_decode_kernel<N, NW><<<grid, NW * 64, lds * (NW / 4), stream>>>(                     \
         (const bf16_t*)q, q_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages, (bf16_t*)out, \

@@ -84,6 +84,7 @@ _SIGNATURES = {
     "dli_embedding_ssq": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr],
     "dli_attention_generic_tile_rows": [_c_int],
     "dli_attention_mfma_supports": [_c_int, _c_int],
+    "dli_attention_decode_waves": [_c_i64, _c_int, _c_int, _c_int],
     "dli_attention_prefill_tile_rows": [_c_int, _c_int, _c_int],
     "dli_attention_decode_bf16": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
                                   _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_ptr],
@@ -1260,6 +1261,12 @@ def _check_paged(q, k_pages, v_pages, out, q_heads):
              f"the matrix-core attention takes head_dim 16..128 in steps of 16 and pages of a multiple of 16, "
              f"not head_dim {head_dim}, page size {page_size}")
     return kv_heads, page_size, head_dim
+
+
+def attention_decode_waves(workgroups: int, group: int, head_dim: int, units: int) -> int:
+    """How many waves a workgroup of :func:`attention_decode` has in a launch of so many on so many compute units, ``group`` query
+    heads a kv head."""
+    return int(library().dli_attention_decode_waves(workgroups, group, head_dim, units))
 
 
 def attention_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, out: Optional[torch.Tensor],

@@ -20,7 +20,7 @@ from typing import Any, Mapping, Optional
 import torch
 
 from ..kernels import ops
-from .attention_kernels import decode_attention_unmerged, head_tiles, paged_attention, planned_splits
+from .attention_kernels import decode_attention_unmerged, paged_attention, planned_splits
 from .base import DecodeStream, Mixer, Norm, PagedKVSpec, Part, Runtime
 from .linear import decode_copy, finish_residual, linear
 from .registry import build_part, register_part
@@ -158,7 +158,7 @@ class GQAttention(Mixer):
         """Into how many runs the decode kernel cuts each request's keys in a recorded step (the 32-bit kernel cuts none)."""
         if not self.rt.is_bf16:
             return None
-        return planned_splits(requests, head_tiles(self.num_heads, self.num_kv_heads), max_keys,
+        return planned_splits(requests, self.num_heads, self.num_kv_heads, self.head_dim, max_keys,
                               ops.compute_units(self.rt.device))
 
     # -- step

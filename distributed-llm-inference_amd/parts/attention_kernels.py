@@ -7,6 +7,7 @@ decode kernel and portions to the tiled prefill kernel.
 
 from __future__ import annotations
 
+import functools
 from typing import Any, Callable, Optional
 
 import numpy as np
@@ -25,7 +26,7 @@ MIN_KEYS_PER_SPLIT = 256
 FEW_SPLITS = 16          # the limit up to 8K keys
 KEYS_PER_EXTRA_SPLIT = 512
 MAX_SPLITS = 64
-ONE_RUN_KEYS = 576
+ONE_RUN_KEYS, ONE_RUN_KEYS_WIDE, ONE_RUN_KEYS_ALONE = 576, 544, 528   # heads up to 64; wider; wider, one request
 
 
 def choose_splits(requests: int, kv_head_tiles: int, max_keys: int, units: int = 256) -> int:
@@ -39,15 +40,32 @@ def choose_splits(requests: int, kv_head_tiles: int, max_keys: int, units: int =
     return max(1, min(want, most, limit))
 
 
-def planned_splits(requests: int, kv_head_tiles: int, max_keys: int, units: int = 256) -> int:
+@functools.lru_cache(maxsize=256)
+def one_run_keys(requests: int, q_heads: int, kv_heads: int, head_dim: int, units: int = 256) -> int:
+    """Up to how many keys one run serves a recorded step better than two, where every workgroup has a compute unit to itself. It
+    then has eight waves, which walk up to 512 keys in one round of what they have on their way; what follows costs more the
+    wider the heads are, and the second run's merge is cheaper for a single request, whose o projection makes it. Passes of 8 steps,
+    two runs and one, ms: 135M sizes, 1 request, 520 keys 5.91 and 5.60, 568 5.90 and 5.87, 600 5.92 and 5.94; 1B sizes, 8 requests,
+    568 7.04 and 6.96, 600 7.01 and 7.04. Heads of 128: 24 on 8, 8 requests, 520 5.53 and 5.43, 552 5.53 and 5.56; 16 on 2, 8
+    requests, 552 4.60 and 4.48, 1 request, 536 3.70 and 3.75. Heads of 96: 16 on 8, 8 requests, 552 3.98 and 3.97, 568 3.98 and
+    4.02, 1 request, 536 3.31 and 3.35. Groups whose states do not fit (heads of 128, 16 on one) have four waves: 1 request, 520
+    3.53 and 3.63; 2 requests, 584 4.28 and 3.95; 16 requests, 584 5.54 and 5.24."""
+    workgroups = requests * head_tiles(q_heads, kv_heads)
+    if workgroups > units:
+        return 0
+    alone = requests == 1
+    if ops.attention_decode_waves(workgroups, q_heads // kv_heads, head_dim, units) == 4:
+        return 0 if alone else ONE_RUN_KEYS
+    return ONE_RUN_KEYS if head_dim <= 64 else ONE_RUN_KEYS_ALONE if alone else ONE_RUN_KEYS_WIDE
+
+
+def planned_splits(requests: int, q_heads: int, kv_heads: int, head_dim: int, max_keys: int, units: int = 256) -> int:
     """:func:`choose_splits` rounded up to a power of two: the coarse form of the rule, for steps
     that are recorded once and replayed for a range of lengths (each distinct answer is a
-    recording of its own). Up to :data:`ONE_RUN_KEYS` keys one run where every workgroup has a compute unit to
-    itself (it then has eight waves): four or five tiles of keys a wave cost less than the merge of two runs (512 keys, a pass
-    of 8 steps at the 135M sizes: 5.54 ms against 5.78, at the 1B sizes with 8 requests 6.80 against 6.95; with 768
-    keys and 8 requests at the 360M sizes 9.01 against 8.80 in two runs)."""
-    if max_keys <= ONE_RUN_KEYS and requests * kv_head_tiles <= units:
+    recording of its own). Up to :func:`one_run_keys` keys one run."""
+    if max_keys <= ONE_RUN_KEYS and max_keys <= one_run_keys(requests, q_heads, kv_heads, head_dim, units):
         return 1
+    kv_head_tiles = head_tiles(q_heads, kv_heads)
     splits, coarse = choose_splits(requests, kv_head_tiles, max_keys, units), 1
     while coarse < splits:
         coarse *= 2

@@ -348,6 +348,20 @@ extern "C" int dli_rope_angles(const int* positions, const float* inv_freq, floa
   return dli_launch_status();
 }
 
+// How many shares of the heads the vector form's workgroups take, or 0 where a workgroup's v rows do not fit LDS: up to 48 KB,
+// and a vector a row more, by which the rows are apart (22 kv heads of 128 and 46 of 64 fill the 48 KB: 4,096 rows 34 and 36 us, in the
+// other form 88 and 95).
+#define ROPE_ROWS 8
+extern "C" int dli_rope_kv_shares(int tokens, int rotary_dim, int q_heads, int kv_heads, int head_dim, int is_bf16, int units) {
+  const int vec = is_bf16 ? 8 : 4, elem = is_bf16 ? 2 : 4;
+  const int groups = (tokens + ROPE_ROWS - 1) / ROPE_ROWS;
+  // as many as the kv heads and q heads allow, up to two workgroups a compute unit in all
+  int shares = 1;
+  while (kv_heads % (2 * shares) == 0 && q_heads % (2 * shares) == 0 && (int64_t)groups * 2 * shares <= 2 * units) shares *= 2;
+  const int64_t v_bytes = (int64_t)ROPE_ROWS * (kv_heads / shares) * head_dim * elem, angles = (int64_t)ROPE_ROWS * rotary_dim * sizeof(float);
+  return angles + v_bytes <= 48 * 1024 && rotary_dim / 2 % vec == 0 && head_dim % vec == 0 ? shares : 0;
+}
+
 extern "C" int dli_rope_kv_write(void* qkv, int64_t row_stride, const int* positions,
                                  const float* inv_freq, int rotary_dim, const int* slots,
                                  void* k_pages, void* v_pages, int tokens, int q_heads, int kv_heads,
@@ -366,16 +380,13 @@ extern "C" int dli_rope_kv_write(void* qkv, int64_t row_stride, const int* posit
   // a prompt: 11.7 against 7.1)
   if (tokens > 512) {
     // the vector form where the sizes are multiples of its 16 bytes and a workgroup's v rows fit LDS
-    constexpr int ROWS = 8;
+    constexpr int ROWS = ROPE_ROWS;
     const int vec = is_bf16 ? 8 : 4, elem = is_bf16 ? 2 : 4;
     const int groups = (tokens + ROWS - 1) / ROWS;
-    // shares of the heads: as many as the kv heads and q heads allow, up to two workgroups a compute unit in all
-    int shares = 1;
-    while (kv_heads % (2 * shares) == 0 && q_heads % (2 * shares) == 0 && (int64_t)groups * 2 * shares <= 2 * dli_compute_units()) shares *= 2;
-    const size_t lds = (size_t)2 * ROWS * half * sizeof(float) + (size_t)ROWS * ((kv_heads / shares) * head_dim + vec) * elem;
-    if (half > 0 && half % vec == 0 && head_dim % vec == 0 && row_stride % vec == 0 &&
-        (uintptr_t)qkv % 16 == 0 && (uintptr_t)k_pages % 16 == 0 && (uintptr_t)v_pages % 16 == 0 &&
-        lds <= 48 * 1024) {
+    const int shares = dli_rope_kv_shares(tokens, rotary_dim, q_heads, kv_heads, head_dim, is_bf16, dli_compute_units());
+    if (shares > 0 && half > 0 && row_stride % vec == 0 &&
+        (uintptr_t)qkv % 16 == 0 && (uintptr_t)k_pages % 16 == 0 && (uintptr_t)v_pages % 16 == 0) {
+      const size_t lds = (size_t)2 * ROWS * half * sizeof(float) + (size_t)ROWS * ((kv_heads / shares) * head_dim + vec) * elem;
       const dim3 grid((groups + 15) / 16 * 16, shares);  // the XCD-aware order permutes blocks of 16
       if (is_bf16)
         rope_kv_write_rows_kernel<bf16_t, ROWS><<<grid, 256, lds, stream>>>(

@@ -39,6 +39,7 @@ _SIGNATURES = {
                          _c_i64, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float,
                          _c_float, _c_float, _c_ptr],
     "dli_skinny4_tile_features": [_c_int, _c_int],
+    "dli_rope_kv_shares": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
     "dli_rope_kv_write": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int,
                           _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "dli_normed_tiles_ahead": [_c_int, _c_int, _c_int, _c_int, _c_int],
@@ -381,6 +382,12 @@ def copy_pages(pool: torch.Tensor, src: torch.Tensor, dst: torch.Tensor) -> None
 
 
 # ----------------------------------------------------------------------------- position + cache write
+
+def rope_kv_shares(tokens: int, rotary_dim: int, q_heads: int, kv_heads: int, head_dim: int, dtype: torch.dtype, units: int) -> int:
+    """Over how many workgroups :func:`rope_kv_write` deals the heads of eight rows in its vector form (steps of more than 512
+    rows), or 0 where it does not take these sizes."""
+    return int(library().dli_rope_kv_shares(tokens, rotary_dim, q_heads, kv_heads, head_dim, _is_bf16(dtype), units))
+
 
 def rope_kv_write(qkv: torch.Tensor, positions: torch.Tensor, inv_freq: Optional[torch.Tensor],
                   rotary_dim: int, slots: Optional[torch.Tensor], k_pages: Optional[torch.Tensor],

@@ -106,3 +106,15 @@ def test_waves_of_a_decode_workgroup():
             assert ops.attention_decode_waves(256, group, d, 256) == (8 if fits else 4)
             assert ops.attention_decode_waves(257, group, d, 256) == 4
     assert ops.attention_decode_waves(1, 12, 128, 256) == 8 and ops.attention_decode_waves(1, 13, 128, 256) == 4
+
+
+@pytest.mark.parametrize("kv,d,dtype", [(22, 128, "bfloat16"), (46, 64, "bfloat16"), (11, 128, "float32"), (23, 64, "float32")])
+def test_rotated_rows_that_just_fit(kv, d, dtype):
+    """Eight rows of v beside their angles fill 48 KB of LDS; one kv head more does not fit."""
+    import torch
+
+    from dli_amd.kernels import ops
+
+    shares = lambda heads: ops.rope_kv_shares(4096, d, heads, heads, d, getattr(torch, dtype), 256)
+    assert 8 * d * 4 + 8 * kv * d * getattr(torch, dtype).itemsize == 48 * 1024
+    assert shares(kv) == 1 and shares(kv - 1) == 1 and shares(kv + 1 + kv % 2) == 0

@@ -38,3 +38,8 @@ def test_rope_kv_write_in_shares_of_heads(ops, qh, kvh, d, rd, n, offset):
         results.append((rows[:, :qh * d], kp, vp))
     for one, other in zip(*results):
         assert torch.equal(one, other)
+
+
+@pytest.mark.parametrize("heads,d", [(22, 128), (46, 64)])
+def test_rows_whose_v_fills_the_lds(ops, heads, d):
+    test_rope_kv_write_in_shares_of_heads(ops, heads, heads, d, d, 2100, 3)

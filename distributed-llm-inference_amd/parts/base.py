@@ -325,7 +325,7 @@ class Block(Part):
     # Whether ``forward`` takes a keyword ``following``: the norm that the stream meets after this block
     # (the next block's ``first_norm``, the final norm, or None), for a block whose last kernel can apply it.
     takes_following: bool = False
-    # Whether it asks the step's context for that norm instead (``NormedStream.following``).
+    # Whether it asks the step's context (``NormedStream.following``) for what the stream meets after it (``meets``).
     asks_following: bool = False
 
     def forward(self, x: torch.Tensor, delta: Optional[torch.Tensor], ctx: Any, cache: Any,
@@ -351,6 +351,11 @@ class Block(Part):
         """The norm that this arrangement applies to the stream before anything else, if there is
         one: the block before it may apply it in the kernel that writes the stream (the fused
         decode path passes it on as ``following``)."""
+        return None
+
+    def meets(self, parts: Mapping[str, Part]) -> Any:
+        """For a block before it that asks (``asks_following``): what this arrangement meets the stream with where that is no
+        single norm, such as two norms of the same rows."""
         return None
 
 

@@ -217,8 +217,11 @@ class ParallelNormsBlock(Block):
     def graph_capturable(self, page_size: int) -> bool:
         return True  # kernels on device arrays only
 
-    def first_norm(self, parts: Mapping[str, Part]) -> Optional[Any]:
-        return NormPair.of(parts["mixer_norm"], parts["feed_forward_norm"]) if "feed_forward" in parts else parts["mixer_norm"]
+    def first_norm(self, parts: Mapping[str, Part]) -> Optional[Part]:
+        return None if "feed_forward" in parts else parts["mixer_norm"]
+
+    def meets(self, parts: Mapping[str, Part]) -> Any:
+        return NormPair.of(parts["mixer_norm"], parts["feed_forward_norm"]) if "feed_forward" in parts else None
 
     def forward(self, x: torch.Tensor, delta: Optional[torch.Tensor], ctx: Any, cache: Any,
                 parts: Mapping[str, Part]) -> tuple[torch.Tensor, Optional[torch.Tensor]]:

@@ -169,11 +169,11 @@ class Model:
         return all(takes_stream(l.block) and l.block.streams(ctx, l.parts) for l in self.layers)
 
     @staticmethod
-    def _first_norm(layer: BuiltLayer) -> Optional[Part]:
-        """The norm that a layer meets the stream with, for the block before it. (A block that derives from another and arranges
-        its parts anew does not meet it with the other's.)"""
-        first = fused_form(layer.block, "first_norm")
-        return first(layer.parts) if first is not None else None
+    def _met_with(layer: BuiltLayer, how: str) -> Any:
+        """``first_norm`` or ``meets`` of a layer's block, for the block before it. (A block that derives from another and arranges
+        its parts anew does not meet the stream with the other's norm.)"""
+        ask = fused_form(layer.block, how)
+        return ask(layer.parts) if ask is not None else None
 
     def _forward_stream(self, ctx: Any, caches: Sequence[Any]) -> torch.Tensor:
         stream = self.embedding.forward_stream(ctx.token_ids)
@@ -223,12 +223,12 @@ class Model:
             for i, (layer, cache) in enumerate(zip(order, caches)):
                 if layer.block.takes_following:
                     # (the final norm reads the wanted rows: it follows where those are all rows, in order)
-                    after = (self._first_norm(order[i + 1]) if i + 1 < len(order)
+                    after = (self._met_with(order[i + 1], "first_norm") if i + 1 < len(order)
                              else self.final_norm if getattr(ctx, "all_rows_wanted", False) else None)
                     x, delta = layer.block.forward(x, delta, ctx, cache, layer.parts, following=after)
                 else:
                     if layer.block.asks_following:
-                        NormedStream.follow(ctx, self._first_norm(order[i + 1]) if i + 1 < len(order) else None)
+                        NormedStream.follow(ctx, self._met_with(order[i + 1], "meets") if i + 1 < len(order) else None)
                     x, delta = layer.block.forward(x, delta, ctx, cache, layer.parts)
         k = ctx.logit_rows.shape[0]
         if k == 0:

@@ -218,3 +218,21 @@ def test_experts_of_ones_own_beside_a_mixer(dtype, tmp_path, monkeypatch):
     want = _decoded(load_model(folder, dtype=dtype), [list(range(3, 40)), list(range(50, 61))], 3)
     assert all(torch.equal(g, w) for g, w in zip(got, want))
     assert not any(torch.allclose(g, p, atol=1e-3) for g, p in zip(got, plain))
+
+
+def test_a_block_of_ones_own_is_told_of_norms_only():
+    """A block that takes ``following`` may apply whatever it is handed: a norm, or nothing where the next block meets the stream with
+    two; that pair goes to the blocks that know it."""
+    from dli_amd.parts.base import Norm
+    from dli_amd.parts.model import BuiltLayer, Model
+
+    rt = Runtime(torch.device("cpu"), torch.float32)
+    norms = {"mixer_norm": RMSNorm(rt, width=8, eps=1e-5), "feed_forward_norm": RMSNorm(rt, width=8, eps=1e-5)}
+    for n in norms.values():
+        n.weight = torch.ones(8)
+    both = BuiltLayer(ParallelNormsBlock(rt), {**norms, "mixer": None, "feed_forward": None})
+    alone = BuiltLayer(ParallelNormsBlock(rt), {"mixer_norm": norms["mixer_norm"], "mixer": None})
+    changed = BuiltLayer(_halved(ParallelNormsBlock)(rt), both.parts)
+    assert Model._met_with(both, "first_norm") is None and isinstance(Model._met_with(both, "meets"), NormPair)
+    assert isinstance(Model._met_with(alone, "first_norm"), Norm) and Model._met_with(alone, "meets") is None
+    assert Model._met_with(changed, "first_norm") is None and Model._met_with(changed, "meets") is None

@@ -1104,6 +1104,15 @@ extern "C" int dli_attention_prefill_tile_rows(int head_dim, int q_heads, int kv
   return hw == 0 ? PF_TILE_ROWS : (4 / hw) * 32;
 }
 
+// What the host hands to the attention kernels to find a tile's page by.
+extern "C" int dli_page_of_tile(int page_size, unsigned* tiles, unsigned* reciprocal) {
+  if (page_size < 16 || page_size % 16 != 0) return DLI_ERR_ARGUMENT;
+  const PageOf p = page_of_tile(page_size);
+  *tiles = p.tiles;
+  *reciprocal = p.reciprocal;
+  return DLI_OK;
+}
+
 // LDS of the states of four waves of a decode workgroup.
 static size_t decode_states(int group, int head_dim) {
   return (size_t)4 * (head_dim / 16) * 4 * (group < 16 ? group : 16) * sizeof(float4v);

@@ -85,6 +85,7 @@ _SIGNATURES = {
     "dli_embedding_ssq": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr],
     "dli_attention_generic_tile_rows": [_c_int],
     "dli_attention_mfma_supports": [_c_int, _c_int],
+    "dli_page_of_tile": [_c_int, _c_ptr, _c_ptr],
     "dli_attention_decode_waves": [_c_i64, _c_int, _c_int, _c_int],
     "dli_attention_prefill_tile_rows": [_c_int, _c_int, _c_int],
     "dli_attention_decode_bf16": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
@@ -1268,6 +1269,13 @@ def _check_paged(q, k_pages, v_pages, out, q_heads):
              f"the matrix-core attention takes head_dim 16..128 in steps of 16 and pages of a multiple of 16, "
              f"not head_dim {head_dim}, page size {page_size}")
     return kv_heads, page_size, head_dim
+
+
+def page_of_tile(page_size: int) -> tuple[int, int]:
+    """Tiles of sixteen keys in a page and the reciprocal by which the attention kernels find a tile's page."""
+    tiles, reciprocal = ctypes.c_uint(), ctypes.c_uint()
+    _check(library().dli_page_of_tile(page_size, ctypes.addressof(tiles), ctypes.addressof(reciprocal)), "page_of_tile")
+    return tiles.value, reciprocal.value
 
 
 def attention_decode_waves(workgroups: int, group: int, head_dim: int, units: int) -> int:

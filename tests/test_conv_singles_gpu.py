@@ -30,6 +30,10 @@ def test_kept_inputs_of_single_tokens(taps, heads, kv_heads, dim, vdim):
         results.append((*outs, kept))
     assert all(torch.equal(one, other) for one, other in zip(*results))
     assert torch.equal(results[1][-1][[4, 7]], state[[4, 7]])   # nobody else's memory
-    with pytest.raises(Exception):
-        ops.conv_prepare(steps[0], channels, channels + heads, conv_w, a_log, dt_bias, state, 11, q_start[:4], positions, slots[:3],
-                         outs[0], heads, kv_heads, dim, vdim, singles=True)
+    # entries of several rows: only the flag makes them wrong, whose waves would write what others of their entry still read
+    several = torch.tensor([0, 3, 4, 7], dtype=torch.int32, device="cuda")
+    call = lambda singles: ops.conv_prepare(steps[0], channels, channels + heads, conv_w, a_log, dt_bias, state, 11, several, positions,
+                                            slots[:3].contiguous(), outs[0], heads, kv_heads, dim, vdim, singles=singles)
+    call(False)
+    with pytest.raises(ops.KernelArgumentError, match="single tokens"):
+        call(True)

@@ -44,10 +44,39 @@ def test_pages_of_the_32_bit_attention(page):
     f32.test_attention_f32(ops, 4, 2, 128, page, 45)
 
 
+@gpu
+@pytest.mark.parametrize("page", [48, 112, 1040])
+def test_pages_of_a_long_context(page):
+    """Tiles of far larger numbers than a short context has, in both attentions of single tokens."""
+    import test_kernels_gpu as kernels
+    from kernel_refs import ref_paged_attention
+
+    from dli_amd.kernels import ops
+
+    dev = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    lens = [(1, 70003), (1, 65537)]
+    q, kp, vp, q_start, kv_len, tables = kernels._paged_case(torch.bfloat16, 2, 1, 64, page, lens, seed=page)
+    ref = ref_paged_attention(q, kp, vp, q_start, kv_len, tables, 2, 0.5, 0)
+    out = torch.empty(q.shape, dtype=torch.bfloat16, device="cuda")
+    ops.attention_decode(q.cuda(), kp.cuda(), vp.cuda(), out, dev(kv_len), dev(tables), 2, 0.5)
+    assert (out.cpu().double() - ref).abs().max() < kernels.tol(torch.bfloat16)
+    q, kp, vp = q.float(), kp.float(), vp.float()
+    ref = ref_paged_attention(q, kp, vp, q_start, kv_len, tables, 2, 0.5, 0)
+    out = torch.empty(q.shape, device="cuda")
+    ops.attention_generic(q.cuda(), kp.cuda(), vp.cuda(), out, dev(q_start), dev(kv_len), dev(tables), dev([0, 1]), dev([0, 0]), 2, 0.5)
+    assert (out.cpu().double() - ref).abs().max() < 2e-5
+
+
 def test_a_tile_is_in_the_page_that_division_names():
-    """The rule of csrc/common.h, PageOf, in whole numbers: exact for every tile below 2^32 / tiles (checked at multiples of tiles)."""
-    for tiles in [*range(2, 130), 255, 256, 1000, 4097]:
-        reciprocal = ((1 << 32) + tiles - 1) // tiles
+    """What the host hands over (csrc/common.h, page_of_tile): the upper half of the product with the reciprocal is the quotient for every
+    tile below 2^32 / tiles (checked about multiples of the page's tiles)."""
+    from dli_amd.kernels import ops
+
+    for tiles in [*range(1, 130), 255, 256, 1000, 4097]:
+        held, reciprocal = ops.page_of_tile(16 * tiles)
+        assert held == tiles
+        if tiles == 1:   # (a page a tile: no product)
+            continue
         top = (1 << 32) // tiles - 1
         for q in (1, 2, 3, 1000, top // tiles - 1, top // tiles):
             for tile in (q * tiles - 1, q * tiles, q * tiles + 1):

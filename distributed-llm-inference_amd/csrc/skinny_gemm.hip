@@ -117,7 +117,8 @@ __device__ __forceinline__ bf16x8 finish_x(const XFrag<NORM>& f, float rs) {
 // KS waves split k, NS groups of waves split the workgroup's tiles, each wave owns NT tiles:
 // a workgroup computes NS*NT tiles of 16 features with KS*NS waves. The activation fragments are
 // loaded once per block of k and reused for the wave's NT tiles.
-template <int KS, int NS, int NT, int MT, int EPI, bool NORM, bool TILED, bool MERGED = false>
+// AHEAD: up to four rows, no wave has a single block of k (two_blocks_or_none), and the second sets out with the first.
+template <int KS, int NS, int NT, int MT, int EPI, bool NORM, bool TILED, bool AHEAD, bool MERGED = false>
 __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
     const bf16_t* __restrict__ x, int64_t ldx, const float* __restrict__ ssq_in, int ssq_parts,
     const float* __restrict__ norm_w, float eps, const bf16_t* __restrict__ w,
@@ -126,6 +127,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
     int up_offset, QkvRope qr, MergedIn mi, GluForm glu) {
   static_assert(EPI != EPI_QKV || (TILED && MT == 1), "the q/k/v epilogue reads tiled weights, at most 16 rows");
   static_assert(!MERGED || (TILED && MT == 1 && NS == 1 && !NORM), "merged activations: tiled weights, one row tile");
+  static_assert(!AHEAD || (MT == 1 && !NORM && !MERGED), "one row tile, no sums of squares to wait for");
   static_assert(KS * NS * 64 >= 256, "a thread for each output of a tile");
   // MERGED: each wave's run of k for up to MERGE_ROWS rows
   __shared__ __align__(16) bf16_t xs[MERGED ? KS : 1][MERGED ? MERGE_ROWS : 1][MERGED ? MERGE_RANGE : 8];
@@ -365,6 +367,10 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
   }
   if constexpr (!NORM) {
     if (blocks > 0) fetch_rows(b0, s);
+    if (MERGED ? blocks > 1 : AHEAD && blocks > 0) {
+      fetch_rows(b1, s + 4);
+      if constexpr (!MERGED) fetch_weights(b1, s + 4);
+    }
   }
   if constexpr (MT > 1) {
     // several row tiles: one body for every turn (the registers do not hold two whole blocks)
@@ -377,38 +383,69 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
       multiply(b0);
       if (more) b0 = b1;
     }
-  } else if (blocks == 1) {
+  } else if (NORM && blocks == 1) {
     multiply(b0);
     s += 4;
-  } else if (blocks > 1) {
-    // (The second block is asked for here and not with the first, in front of the sums of squares: a wave of one block has
-    // none, and its rows and norm weights stand in the vector cache's way. Gate and up, 8 and 16 rows, asked for there and
-    // here: 6.6 and 5.2 us, 6.8 and 5.3 at the 135M sizes, 15.7 and 15.8, 16.4 and 16.9 at the 1B sizes.)
-    fetch_rows(b1, s + 4);
-    if constexpr (!MERGED) fetch_weights(b1, s + 4);
-    __builtin_amdgcn_sched_barrier(0);
-    while (blocks >= 4) {
-      multiply(b0);
-      fetch_rows(b0, s + 8);
-      fetch_weights(b0, s + 8);
-      __builtin_amdgcn_sched_barrier(0);  // all of a block's loads leave before the other's products
-      multiply(b1);
-      fetch_rows(b1, s + 12);
-      fetch_weights(b1, s + 12);
-      __builtin_amdgcn_sched_barrier(0);
-      s += 8;
-      blocks -= 2;
-    }
-    if (blocks == 3) {
-      multiply(b0);
-      fetch_rows(b0, s + 8);
-      fetch_weights(b0, s + 8);
-      __builtin_amdgcn_sched_barrier(0);
-      multiply(b1);
-      multiply(b0);
+  } else if (blocks > 0) {
+    // Where the second block is asked for, us with the first, and after what is waited for before the first product:
+    //  - A wave of one block would read it twice: o, 8 rows, 3.8 and 3.2 at the 135M sizes, 1 row 4.2 and 3.7 at the 360M sizes.
+    //  - With two and more and few rows it pays: o, 1 row, 4.4 and 4.6 at the 1B sizes, 5.6 and 6.0 at the 3B sizes.
+    //  - With more rows not, and there a block is best asked for right before the other's products, not after them: down, 16
+    //    rows, 17.5 and 16.6 at the 3B sizes; 32-bit sums of 8,192 features of 2,048, 16 rows, 12.2 and 11.4.
+    //  - In front of sums of squares it stands, with rows and norm weights, in the vector cache's way: gate and up, 8 and 16
+    //    rows, 6.6 and 5.2, 6.8 and 5.3 at the 135M sizes. Right after the other's products is best there: 16 rows, 15.9 at
+    //    the 1B sizes, 16.9 before them.
+    if constexpr (NORM || AHEAD || MERGED) {
+      if constexpr (NORM) {
+        fetch_rows(b1, s + 4);
+        fetch_weights(b1, s + 4);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      while (blocks >= 4) {
+        multiply(b0);
+        fetch_rows(b0, s + 8);
+        fetch_weights(b0, s + 8);
+        __builtin_amdgcn_sched_barrier(0);  // all of a block's loads leave before the other's products
+        multiply(b1);
+        fetch_rows(b1, s + 12);
+        fetch_weights(b1, s + 12);
+        __builtin_amdgcn_sched_barrier(0);
+        s += 8;
+        blocks -= 2;
+      }
+      if (blocks == 3) {
+        multiply(b0);
+        fetch_rows(b0, s + 8);
+        fetch_weights(b0, s + 8);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(b1);
+        multiply(b0);
+      } else {
+        multiply(b0);
+        if (!MERGED || blocks == 2) multiply(b1);
+      }
     } else {
-      multiply(b0);
-      multiply(b1);
+      while (blocks >= 3) {
+        fetch_rows(b1, s + 4);
+        fetch_weights(b1, s + 4);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(b0);
+        fetch_rows(b0, s + 8);
+        fetch_weights(b0, s + 8);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(b1);
+        s += 8;
+        blocks -= 2;
+      }
+      if (blocks == 2) {
+        fetch_rows(b1, s + 4);
+        fetch_weights(b1, s + 4);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(b0);
+        multiply(b1);
+      } else {
+        multiply(b0);
+      }
     }
     s = s_begin + (s_end - s_begin) / 4 * 4;
   }
@@ -949,6 +986,14 @@ static bool launch_normed_tiles(SK_PARAMS) {
   return true;
 }
 
+// Whether each of KS waves that share K has at least two blocks of 128, or none has any (whole blocks are dealt out in tile
+// order, else steps of 32).
+static bool two_blocks_or_none(int K, int KS, bool tiled) {
+  const int least = tiled ? K / 128 / KS : K / 32 / KS / 4;
+  const int most = tiled ? (K / 128 + KS - 1) / KS : (K / 32 + KS - 1) / KS / 4;
+  return least >= 2 || most == 0;
+}
+
 template <int KS, int NS, int NT, int MT, int EPI, bool NORM, bool TILED>
 static void launch_skinny(SK_PARAMS) {
   const int tiles = (N + 15) / 16;
@@ -956,9 +1001,18 @@ static void launch_skinny(SK_PARAMS) {
   if constexpr (NORM && TILED && MT == 1 && NS == 1 && (EPI == EPI_SWIGLU || EPI == EPI_QKV)) {
     if (launch_normed_tiles<KS, NT, EPI>(SK_ARGS)) return;
   }
-  skinny_gemm_kernel<KS, NS, NT, MT, EPI, NORM, TILED><<<groups, KS * NS * 64, 0, stream>>>(
-      (const bf16_t*)x, ldx, ssq_in, ssq_parts, norm_w, eps, (const bf16_t*)w, (const bf16_t*)bias,
-      out, ldo, (bf16_t*)stream_buf, lds_, ssq_out, M, N, K, up_offset, qr, MergedIn{}, glu);
+#define SK_LAUNCH(AHEAD_)                                                                                          \
+  skinny_gemm_kernel<KS, NS, NT, MT, EPI, NORM, TILED, AHEAD_><<<groups, KS * NS * 64, 0, stream>>>(                \
+      (const bf16_t*)x, ldx, ssq_in, ssq_parts, norm_w, eps, (const bf16_t*)w, (const bf16_t*)bias,               \
+      out, ldo, (bf16_t*)stream_buf, lds_, ssq_out, M, N, K, up_offset, qr, MergedIn{}, glu)
+  if constexpr (MT == 1 && !NORM && EPI != EPI_QKV) {
+    if (M <= 4 && two_blocks_or_none(K, KS, TILED)) {
+      SK_LAUNCH(true);
+      return;
+    }
+  }
+  SK_LAUNCH(false);
+#undef SK_LAUNCH
 }
 
 // shapes of the workgroup: 0: 4 k-waves x 1 tile (few tiles, short k); 1: 8 k-waves x 1 tile (few
@@ -1068,7 +1122,7 @@ extern "C" int dli_skinny_gemm_merged(const float* part_o, const float* part_ml,
   const MergedIn mi{part_o, part_ml, splits, heads, head_dim};
   const int groups = N / 16;
 #define MERGED_LAUNCH(KS)                                                                          \
-  skinny_gemm_kernel<KS, 1, 1, 1, EPI_RESIDUAL, false, true, true><<<groups, KS * 64, 0, stream>>>( \
+  skinny_gemm_kernel<KS, 1, 1, 1, EPI_RESIDUAL, false, true, false, true><<<groups, KS * 64, 0, stream>>>( \
       nullptr, 0, nullptr, 0, nullptr, 0.f, (const bf16_t*)w_tiled, (const bf16_t*)bias, nullptr, 0, \
       (bf16_t*)stream_buf, lds_, ssq_out, M, N, K, 0, QkvRope{}, mi, GluForm{})
   if (shape == 0) MERGED_LAUNCH(4);

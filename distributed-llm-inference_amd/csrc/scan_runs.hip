@@ -20,7 +20,7 @@
 // RUNS_BONUS, of four prompts, 2,990 tokens, 168 -> 125 RUNS_GATED, and as far from 64 bits or less).
 //
 // Measured (one prompt of 2,048 tokens, 32 heads, walk + carry + finish, us): RUNS_DELTA 108 + 15 + 21 against 578 and 17 for
-// the norm, RUNS_BONUS 49 + 8 + 17 against 378 and 17, RUNS_GATED 136 in all (before the sums were made together) against 421. Where the cut lies: ops.scan_runs.
+// the norm, RUNS_BONUS 49 + 8 + 17 against 378 and 17, RUNS_GATED 117 in all against 410. Where the cut lies: ops.scan_runs.
 // Beside 255 single tokens, which keep the kernel of steps of single tokens: 245, 168 and 183 us a layer (5,150, 2,880 and 2,610 token
 // by token; 1,048, 1,301 and 818 with every entry cut and the launch as large as the longest entry times the entries).
 // Distance from the rules in 64 bits against token by token (2-norm; 300 to 4,096 tokens, 8 to 32 heads, every row of outputs and

@@ -14,9 +14,9 @@
 // rotations for four sums at a time), the waves' shares of k through LDS, always in the same order.
 // What follows the last product is a chain that nothing hides, so it is kept short: one LDS value
 // per wave and output, all read before the first is added, one output a thread. (With four values a
-// lane by way of LDS and up to 64 reads of a few threads one after the other, the chain took 1.0 to
-// 1.2 us of a kernel of 3.5 to 12, now 0.3: gate and up at the 135M sizes 3.5 -> 2.6 us from start to
-// end, down at the 1B sizes 7.9 -> 6.4, one row)
+// lane by way of LDS and up to 64 reads of a few threads one after the other, the chain was about a
+// microsecond longer: gate and up at the 135M sizes 5.4 -> 4.2 us, down at the 1B sizes 9.7 -> 8.7,
+// one row, cold weights, launches one after the other in a replayed graph)
 //
 // A workgroup has KS waves that split k among themselves and owns FQ quads of features. Few
 // quads and many waves suit products with few features (every compute unit still gets a

@@ -56,6 +56,10 @@ template <int SHIFT>
 __device__ __forceinline__ float row_ror(float v) {  // rotated by SHIFT within each row of sixteen lanes
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + SHIFT, 0xf, 0xf, true));
 }
+template <int SHIFT>
+__device__ __forceinline__ float row_shl(float v) {  // the value SHIFT lanes further on in the row of sixteen, 0 past its end
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x100 + SHIFT, 0xf, 0xf, true));
+}
 __device__ __forceinline__ float quad_sum(float v) {  // over the lanes l, l^1, l^2, l^3
   v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xb1, 0xf, 0xf, true));
   return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4e, 0xf, 0xf, true));

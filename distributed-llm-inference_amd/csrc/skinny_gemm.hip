@@ -696,12 +696,12 @@ struct NormedArgs {
 // rows that a fragment reads lie in different banks.
 __host__ __device__ constexpr int normed_row(int K) { return (K + 127) / 128 * 128 + 8; }
 
-template <int KS, int NT, int EPI, int SETS, int MR>
+template <int KS, int NT, int EPI, int SETS, int MR, bool IN_TURN>
 __global__ __launch_bounds__(KS * 64) void normed_tiles_kernel(NormedArgs p) {
   static_assert(EPI == EPI_SWIGLU || EPI == EPI_QKV, "the products behind a norm");
   constexpr int NA = EPI == EPI_SWIGLU ? 2 : 1;  // weight row sets per tile (gate and up)
   constexpr int BA = 2;                          // sums a thread makes per tile: gate and up, or a feature and its rotary partner
-  constexpr int PARTS = MR == 1 ? 2 : MR;        // loads of 64 parts of the sums of squares a wave asks for at the start
+  constexpr int PARTS = IN_TURN ? 1 : MR == 1 ? 2 : MR;  // loads of 64 parts of the sums of squares a wave asks for at the start
   constexpr int PRE = KS == 4 ? 3 : 2;           // pieces of 256 values of the rows likewise
   constexpr unsigned OUTSIDE = 0x80000000u;      // an offset past the end of every resource here
   typedef short short4v __attribute__((ext_vector_type(4)));
@@ -719,9 +719,11 @@ __global__ __launch_bounds__(KS * 64) void normed_tiles_kernel(NormedArgs p) {
   // The parts of sum x^2 that the producer of x left, [part][row]. Where the rows are a power of two
   // (decode graphs) a wave takes 64 of them in a row, lane l for row l % M; else the lane group grp takes
   // part 4 ks + grp, and every 4 KS-th behind it, for row l % 16.
+  // IN_TURN (one row): the lane group's parts likewise, one a lane, added in their order as the general kernel adds them. More rows
+  // of such a product take that kernel, and a request's row then has the same bits whether others share the step or not.
   const __amdgpu_buffer_rsrc_t sres = __builtin_amdgcn_make_buffer_rsrc((void*)p.ssq_in, 0, (unsigned)(p.ssq_parts * M * 4), 0x00020000);
   const bool even = (M & (M - 1)) == 0;
-  const int s_at = even ? threadIdx.x * 4 : ((4 * ks + grp) * M + min(col, M - 1)) * 4;
+  const int s_at = IN_TURN ? (4 * ks + grp + col * 4 * KS) * 4 : even ? threadIdx.x * 4 : ((4 * ks + grp) * M + min(col, M - 1)) * 4;
   const int s_step = even ? 256 * KS : 16 * KS * M, s_end = p.ssq_parts * M * 4;
   float first[PARTS];
 #pragma unroll
@@ -809,16 +811,28 @@ __global__ __launch_bounds__(KS * 64) void normed_tiles_kernel(NormedArgs p) {
 
   // 1 / rms of row `col`: the lane's parts, the wave's lanes of a row, the waves in order
   float sum = 0.f;
+  auto add_parts = [&](float v) __attribute__((always_inline)) {
+    sum += v;
+    if constexpr (IN_TURN) {   // (zeros behind the last part; no branch, which would wait for the weights as well)
+      sum += row_shl<1>(v); sum += row_shl<2>(v); sum += row_shl<3>(v); sum += row_shl<4>(v); sum += row_shl<5>(v);
+      sum += row_shl<6>(v); sum += row_shl<7>(v); sum += row_shl<8>(v); sum += row_shl<9>(v); sum += row_shl<10>(v);
+      sum += row_shl<11>(v); sum += row_shl<12>(v); sum += row_shl<13>(v); sum += row_shl<14>(v); sum += row_shl<15>(v);
+    }
+  };
 #pragma unroll
-  for (int u = 0; u < PARTS; ++u) sum += first[u];
-  for (int at = PARTS * s_step; at < s_end; at += s_step) sum += __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(sres, s_at + at, 0, 0));
-  sum = add_halves(sum, sum);
-  sum = add_rows(sum, sum);
-  if (even) {
-    sum += row_ror<8>(sum);
-    sum += row_ror<4>(sum);
-    if (M == 1) sum = quad_sum(sum);
-    else if (M == 2) sum = quad_pairs(sum);
+  for (int u = 0; u < PARTS; ++u) add_parts(first[u]);
+  for (int at = PARTS * s_step; at < s_end; at += s_step) add_parts(__uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(sres, s_at + at, 0, 0)));
+  if constexpr (IN_TURN) {
+    sum = add_across32(add_across16(sum));
+  } else {
+    sum = add_halves(sum, sum);
+    sum = add_rows(sum, sum);
+    if (even) {
+      sum += row_ror<8>(sum);
+      sum += row_ror<4>(sum);
+      if (M == 1) sum = quad_sum(sum);
+      else if (M == 2) sum = quad_pairs(sum);
+    }
   }
   if (lane < M) rsum[ks][lane] = sum;
   __syncthreads();
@@ -969,20 +983,25 @@ static bool launch_normed_tiles(SK_PARAMS) {
   const NormedArgs args{(const bf16_t*)x, ssq_in, norm_w, (const bf16_t*)w, (const bf16_t*)bias, (bf16_t*)out, ldo, (int)ldx,
                         ssq_parts, M, N, K, up_offset, eps, qr, glu};
   const int groups = (N / 16 + NT - 1) / NT;
-#define NORMED_LAUNCH(SETS_, MR_)                                                        \
+  // A single row where more rows take the general kernel: its sums in that kernel's order (a step of the 135M sizes 0.2% longer, of
+  // the 1B sizes, where two and four rows take this one as well, 0.6% without need).
+  const bool alone = M == 1 && !dli_normed_tiles_ahead(2, N, K, EPI == EPI_SWIGLU, dli_compute_units());
+#define NORMED_LAUNCH(SETS_, MR_, IN_TURN_)                                              \
   {                                                                                      \
-    const auto kernel = normed_tiles_kernel<KS, NT, EPI, SETS_, MR_>;                     \
+    const auto kernel = normed_tiles_kernel<KS, NT, EPI, SETS_, MR_, IN_TURN_>;           \
     if (!lds_refused((const void*)kernel, lds)) kernel<<<groups, KS * 64, lds, stream>>>(args); \
   }
   if constexpr (PER <= 2) {
     if ((K + 127) / 128 / KS >= 3) {
-      if (M == 1) NORMED_LAUNCH(4, 1)
-      else NORMED_LAUNCH(4, 4)
+      if (alone) NORMED_LAUNCH(4, 1, true)
+      else if (M == 1) NORMED_LAUNCH(4, 1, false)
+      else NORMED_LAUNCH(4, 4, false)
       return true;
     }
   }
-  if (M == 1) NORMED_LAUNCH(2, 1)
-  else NORMED_LAUNCH(2, 4)
+  if (alone) NORMED_LAUNCH(2, 1, true)
+  else if (M == 1) NORMED_LAUNCH(2, 1, false)
+  else NORMED_LAUNCH(2, 4, false)
 #undef NORMED_LAUNCH
   return true;
 }

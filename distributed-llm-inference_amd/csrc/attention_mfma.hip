@@ -171,187 +171,243 @@ __device__ __forceinline__ void blank_v(short4v (&vreg)[DCH], int grp, int t, in
 }
 
 // ------------------------------------------------------------------------------------ decode
-// grid (splits, kv_heads * head_tiles, requests); NW waves, which share out a run's tiles of 16 keys. Request e's single query is row e.
-// part_o, part_ml and arrivals without __restrict__: the workgroup that merges reads what other
-// workgroups of the launch stored.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_pair __attribute__((aligned(8)));  // rows may begin at any multiple of 8 bytes
+
+__device__ __forceinline__ float4v mfma32(u32x4 a, u32x4 b, float4v c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// grid (splits, kv_heads * head_tiles, requests); NW waves, which share out the keys in pairs of tiles of sixteen: pair i belongs to
+// wave i mod NW of the run i / NW mod splits. (So a wave knows its first pairs without the number of keys, and looks their pages up
+// while that number is on its way.) Request e's single query is row e.
+//
+// What bounds the launch is, with few keys, the chain launch, number of keys and pages, keys and values, states of the waves;
+// with many, the bytes. In between lies the rate at which a compute unit's vector cache takes loads, 64 bytes a cycle, a wave's
+// load of 8 bytes a lane about as long as one of 16: every load here is 16 bytes a lane and covers whole runs of 64 (8 bytes and
+// single tiles before; one request of 4,096 keys at the 1B sizes in 16 runs 6.3 us, now 4.7; 8 requests in 8 runs 17.6 and 15.9; 64
+// requests of 640 to 4,096 keys 69.9 and 67). A pair is one product of depth 32 for the values, whose
+// operand A gives lane group g the eight keys 8g.. of the pair: both tiles' rows of a dim, 512 bytes each of one page. So that
+// P^T comes out in the same order, the pair's keys are dealt to the two products K Q^T as 8 (row / 4) + 4 u + row % 4.
+// What a wave needs for its first loads comes first, as arguments of its own; the rest when those are on their way.
+struct DecodeArgs {
+  const bf16_t* q;
+  int64_t q_stride;
+  const bf16_t* k_pages;
+  const bf16_t* v_pages;
+  bf16_t* out;
+  int64_t out_stride;
+  float* part_o;   // (the workgroup that merges reads what other workgroups of the launch stored here)
+  float* part_ml;
+  unsigned* arrivals;
+  int group, page_size;
+  float scale_log2e;
+};
+
+// table_width: entries of a request's row of the table, at least one.
 template <int DCH, int NW>
 __global__ __launch_bounds__(NW * 64) void attention_decode_kernel(
-    const bf16_t* __restrict__ q, int64_t q_stride, const bf16_t* __restrict__ k_pages,
-    const bf16_t* __restrict__ v_pages, bf16_t* __restrict__ out, int64_t out_stride,
-    float* part_o, float* part_ml, const int* __restrict__ kv_len,
-    const int* __restrict__ block_tables, int table_stride, int q_heads, int kv_heads, int group,
-    int head_tiles, int page_size, PageOf page_of, float scale_log2e, int window, int splits, unsigned* arrivals) {
+    const int* __restrict__ kv_len, const int* __restrict__ block_tables, int table_width, int window, int splits,
+    unsigned page_tiles, unsigned page_reciprocal, unsigned head_tiles, unsigned head_reciprocal, int kv_heads, DecodeArgs p) {
   constexpr int D = DCH * 16;
-  extern __shared__ float4v sm_o[];  // [wave][chunk of 16 dims][lane group][query head of the group]
-  __shared__ float sm_m[NW][16], sm_l[NW][16];
-
+  constexpr int KC = DCH / 2, TAIL = DCH % 2;  // dims in products of depth 32, and sixteen more in one of depth 16
+  const PageOf page_of{page_tiles, page_reciprocal}, kv_head_of{head_tiles, head_reciprocal};
   const int split = blockIdx.x, e = blockIdx.z;
-  const int kvh = head_tiles == 1 ? blockIdx.y : blockIdx.y / head_tiles, ht = blockIdx.y - kvh * head_tiles;
+  extern __shared__ float4v sm_o[];  // [wave][chunk of 16 dims][lane group][query head of the group]
+  __shared__ float4v sm_ml[16][NW / 2];  // [column][two waves' maximum and sum]
+
   const int lane = threadIdx.x % DLI_WAVE;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / DLI_WAVE);  // known to be the same in all lanes
+  const int n_keys = kv_len[e];
+  const int* table = block_tables + (int64_t)e * table_width;
+  const unsigned pair0 = split * NW + wave, stride = splits * NW;      // this wave's first pair, and from one to the next
+
+  // Where a pair's tiles lie, the run of keys beginning with `tile0`. Past the last key the table may hold anything: such an
+  // entry is not used.
+  unsigned tile0 = 0;
+  struct Where {
+    int page[2], off[2];
+  };
+  auto tile_of = [&](unsigned pair, int u) __attribute__((always_inline)) { return tile0 + 2 * pair + u; };
+  auto look_up = [&](Where& w, unsigned pair) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const unsigned tile = tile_of(pair, u), entry = page_of.page(tile);
+      w.page[u] = table[min(entry, (unsigned)table_width - 1)];
+      w.off[u] = (int)(tile - entry * page_of.tiles) * 16;
+    }
+  };
+  // A pair costs a chain of two trips to memory (its table entries, then its keys and values), so the chain is taken apart: while one
+  // pair is multiplied, the keys and values of the next are on their way (two sets of registers take turns) and the entries of the
+  // one behind it have been asked for. (Two, three and four sets, the last two for fewer waves on a compute unit, steps of: 1B sizes,
+  // 64 requests of up to 4,096 keys 18.91, 19.06 and 19.09 ms, 8 requests 8.02, 8.21 and 8.14; 360M sizes, 59 requests of 4,443
+  // keys 29.35, 29.35 and 29.74.)
+  constexpr int NG = 2;
+  Where where[NG];
+  look_up(where[0], pair0);
+  // (one trip for the number of keys, the first pair's pages and the arguments: left to itself the compiler asks for each where it
+  // is used)
+  asm volatile("" ::"s"(n_keys), "s"(where[0].page[0]), "s"(where[0].page[1]), "s"(p.q), "s"(p.q_stride), "s"(p.k_pages),
+               "s"(p.v_pages), "s"(p.group), "s"(p.page_size), "s"(p.arrivals), "s"(p.scale_log2e));
+  int first_visible = 0;
+  if (window > 0) {  // the run begins where the number of keys says
+    first_visible = max(0, n_keys - window);
+    tile0 = (unsigned)first_visible / 16;
+    look_up(where[0], pair0);
+  }
+
+  const int kvh = kv_head_of.page(blockIdx.y), ht = blockIdx.y - kvh * head_tiles;
   const int col = lane % 16, grp = lane / 16;
+  const int group = p.group, page_size = p.page_size;
+  unsigned* arrivals = p.arrivals;
   const int head_in_group = ht * 16 + col;
   const bool valid = head_in_group < group;
   const int head = kvh * group + head_in_group;
-
-  const int n_keys = kv_len[e];
-  const int first_visible = window > 0 ? max(0, n_keys - window) : 0;
-  const int begin = first_visible / 16 * 16;
-  const int chunk = (((n_keys - begin + splits - 1) / splits) + 15) / 16 * 16;
-  const int k0 = begin + split * chunk;
-  const int k1 = min(n_keys, k0 + chunk);
-  const int* table = block_tables + (int64_t)e * table_stride;
-
-  short4v qreg[DCH];
+  u32x4 qreg[KC > 0 ? KC : 1];
+  short4v qtail = {0, 0, 0, 0};
+  {
+    // (a column without a head: the group's first head again, whose result is dropped)
+    const bf16_t* qp = p.q + (int64_t)e * p.q_stride + (int64_t)(valid ? head : kvh * group) * D;
 #pragma unroll
-  for (int c = 0; c < DCH; ++c) qreg[c] = short4v{0, 0, 0, 0};
-  if (valid) {
-    const bf16_t* qp = q + (int64_t)e * q_stride + (int64_t)head * D + grp * (D / 4);
-#pragma unroll
-    for (int c = 0; c < DCH; ++c) qreg[c] = *reinterpret_cast<const short4v*>(qp + c * 4);
+    for (int c = 0; c < KC; ++c) qreg[c] = *reinterpret_cast<const u32x4_pair*>(qp + c * 32 + grp * 8);
+    if (TAIL) qtail = *reinterpret_cast<const short4v*>(qp + KC * 32 + grp * 4);
   }
 
   ColumnTile<DCH> st;
-  st.init();
-  // A wave takes every NW-th tile of 16 keys, UN tiles (a group) at a time. A group costs a chain
-  // of two trips to memory (its block-table entries, then its keys and values), so the chain is
-  // taken apart: while group g is multiplied, the keys and values of group g+1 are on their way
-  // (two sets of registers take turns) and the table entries of group g+2 have been asked for.
-  // No load hangs on a condition (a tile past the run's end reads the run's last tile again and
-  // is skipped by the arithmetic; values of keys past the end are blanked when they are used),
-  // so at every wait the number of younger loads is known and only the group's own are waited for.
-  constexpr int UN = 1, NG = 4;  // tiles of a group, groups on their way
-  constexpr int STRIDE = 16 * NW;     // keys between a wave's tiles
-  constexpr int STEP = STRIDE * UN;   // and its groups
-  struct Group {
-    short4v k[UN][DCH], v[UN][DCH];
+  st.init();  // (st.l: the sum over this lane's keys; the lanes of a column are added up at the end)
+  struct Pair {
+    u32x4 k[2][KC > 0 ? KC : 1], v[DCH];
+    short4v k_tail[2];
   };
-  struct Where {
-    int64_t page[UN];
-    int off[UN];
-  };
-  const int t_first = k0 + wave * 16;
-  if (t_first < k1) {
-    const int t_last = (k1 - 1) / 16 * 16;  // the run's last tile
-    auto look_up = [&](Where& w, int tg) __attribute__((always_inline)) {
+  const unsigned last_tile = (unsigned)(n_keys - 1) / 16;
+  auto has = [&](unsigned pair) __attribute__((always_inline)) { return (int)tile_of(pair, 0) * 16 < n_keys; };
+  if (has(pair0)) {
+    const int safe = where[0].page[0];  // a page that is there
+    const unsigned head_page = (unsigned)page_size * D;  // values of a page and kv head
+    const int k_row = (col >> 2 & 1) * 8 + (col & 3);   // and 4 u
+    const bool k_second = col >= 8, v_second = grp >= 2;
+    // No load hangs on a condition (a tile past the end reads a page that is there and is masked by the arithmetic, values of
+    // keys past the end are blanked when they are used), so at every wait the number of younger loads is
+    // known and only the pair's own are waited for.
+    auto fetch = [&](Pair& g, const Where& w, unsigned pair) __attribute__((always_inline)) {
+      uint64_t at[2];
+      int off[2];
 #pragma unroll
-      for (int u = 0; u < UN; ++u) {
-        const unsigned tile = (unsigned)min(tg + STRIDE * u, t_last) / 16, page = page_of.page(tile);
-        w.page[u] = table[page];
-        w.off[u] = (tile - page * page_of.tiles) * 16;
+      for (int u = 0; u < 2; ++u) {
+        const bool there = tile_of(pair, u) <= last_tile;
+        at[u] = (uint64_t)(unsigned)((there ? w.page[u] : safe) * kv_heads + kvh) * head_page;
+        off[u] = there ? w.off[u] : 0;
       }
-    };
-    auto fetch = [&](Group& g, const Where& w) __attribute__((always_inline)) {
+      const bf16_t* kp = p.k_pages + (k_second ? at[1] : at[0]) + ((k_second ? off[1] : off[0]) + k_row) * D + grp * 8;
+      const bf16_t* vp = p.v_pages + (v_second ? at[1] : at[0]) + (col * page_size + (v_second ? off[1] : off[0]) + 8 * (grp & 1));
 #pragma unroll
-      for (int u = 0; u < UN; ++u) {
-        load_k<DCH>(g.k[u], k_pages, w.page[u], kv_heads, kvh, page_size, w.off[u], col, grp);
-        load_v<DCH>(g.v[u], v_pages, w.page[u], kv_heads, kvh, page_size, w.off[u], col, grp);
+      for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int c = 0; c < KC; ++c) g.k[u][c] = *reinterpret_cast<const u32x4_pair*>(kp + 4 * u * D + c * 32);
+        if (TAIL) g.k_tail[u] = *reinterpret_cast<const short4v*>(kp + 4 * u * D + KC * 32 - grp * 4);
       }
+#pragma unroll
+      for (int c = 0; c < DCH; ++c) g.v[c] = *reinterpret_cast<const u32x4_pair*>(vp + c * 16 * page_size);
     };
-    auto attend = [&](const Group& g, int tg) __attribute__((always_inline)) {
+    auto attend = [&](const Pair& g, unsigned pair) __attribute__((always_inline)) {
+      if (!has(pair)) return;
+      const int t = (int)tile_of(pair, 0) * 16;
+      float sv[8];  // keys t + 8 grp + i
 #pragma unroll
-      for (int u = 0; u < UN; ++u) {
-        const int t = tg + STRIDE * u;
-        if (t < k1) {
-          const bool need_mask = t + 16 > k1 || t < first_visible;
-          short4v v[DCH];  // a copy: the group's registers are written by loads only
+      for (int u = 0; u < 2; ++u) {
+        float4v s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int c = 0; c < DCH; ++c) v[c] = g.v[u][c];
-          blank_v<DCH>(v, grp, t, k1);
-          attend_tile<DCH>(st, g.k[u], qreg, v, t, grp, k1 - 1, first_visible, scale_log2e, need_mask);
+        for (int c = 0; c < KC; ++c) s = mfma32(g.k[u][c], qreg[c], s);
+        // (a sum of its own: a product of one depth that adds to the result of one of the other depth, right behind it, has read
+        // that result before it was there)
+        if (TAIL) {
+          const float4v tail = mfma16(g.k_tail[u], qtail, float4v{0.f, 0.f, 0.f, 0.f});
+          s = KC > 0 ? s + tail : tail;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sv[4 * u + i] = s[i] * p.scale_log2e;
+      }
+      const int here = t + 8 * grp;
+      u32x4 v[DCH];  // a copy: the set's registers are written by loads only
+#pragma unroll
+      for (int c = 0; c < DCH; ++c) v[c] = g.v[c];
+      if (t + 32 > n_keys || t < first_visible) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (here + i >= n_keys || here + i < first_visible) sv[i] = -INFINITY;
+        // a zero probability must not multiply whatever a not yet written slot holds
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const unsigned keep = (here + 2 * j < n_keys ? 0xffffu : 0u) | (here + 2 * j + 1 < n_keys ? 0xffff0000u : 0u);
+#pragma unroll
+          for (int c = 0; c < DCH; ++c) v[c][j] &= keep;
         }
       }
-    };
-    // NG sets of registers take turns; set d holds group g = d (mod NG), and where[d] the place of
-    // the group that it loads next
-    Group sets[NG];
-    Where where[NG];
+      const float m_new = max2(st.m, column_max(max2(max3(max3(sv[0], sv[1], sv[2]), sv[3], sv[4]), max3(sv[5], sv[6], sv[7]))));
+      const float m_safe = m_new == -INFINITY ? 0.f : m_new;
+      const float alpha = fast_exp2(st.m - m_safe);
+      float pr[8], sum = 0.f;
 #pragma unroll
-    for (int d = 0; d < NG; ++d) look_up(where[d], t_first + d * STEP);
-#pragma unroll
-    for (int d = 0; d < NG; ++d) {
-      fetch(sets[d], where[d]);
-      look_up(where[d], t_first + (d + NG) * STEP);
-    }
-    int tg = t_first;
-    for (; tg + NG * STEP < k1; tg += NG * STEP) {  // rounds that have a group behind them
-#pragma unroll
-      for (int d = 0; d < NG; ++d) {
-        attend(sets[d], tg + d * STEP);
-        fetch(sets[d], where[d]);
-        look_up(where[d], tg + (d + 2 * NG) * STEP);
-        __builtin_amdgcn_sched_barrier(0);  // the loads leave before the next group's arithmetic
+      for (int i = 0; i < 8; ++i) {
+        pr[i] = fast_exp2(sv[i] - m_safe);
+        sum += pr[i];
       }
-    }
+      st.l = st.l * alpha + sum;
+      st.m = m_new;
+      bf16x8 pb;
 #pragma unroll
-    for (int d = 0; d < NG; ++d) attend(sets[d], tg + d * STEP);  // the last round
+      for (int i = 0; i < 8; ++i) pb[i] = (bf16_t)pr[i];
+      if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {  // the running maximum rose somewhere
+#pragma unroll
+        for (int c = 0; c < DCH; ++c) st.o[c] *= alpha;
+      }
+#pragma unroll
+      for (int c = 0; c < DCH; ++c) st.o[c] = mfma32(v[c], __builtin_bit_cast(u32x4, pb), st.o[c]);
+    };
+    Pair sets[NG];
+    if (!has(pair0 + stride)) {
+      // One pair: nothing else is asked for. (A set that is not needed, loaded all the same, would take the vector cache as long as
+      // one that is.)
+      fetch(sets[0], where[0], pair0);
+      attend(sets[0], pair0);
+    } else {
+      // set d holds the pairs d, d + NG, ... of this wave, and where[d] the place of the one that it loads next
+#pragma unroll
+      for (int d = 1; d < NG; ++d) look_up(where[d], pair0 + d * stride);
+#pragma unroll
+      for (int d = 0; d < NG; ++d) fetch(sets[d], where[d], pair0 + d * stride);
+#pragma unroll
+      for (int d = 0; d < NG; ++d) look_up(where[d], pair0 + (d + NG) * stride);
+      unsigned pair = pair0;
+      for (; has(pair + NG * stride); pair += NG * stride) {  // rounds that have a pair behind them
+#pragma unroll
+        for (int d = 0; d < NG; ++d) {
+          attend(sets[d], pair + d * stride);
+          fetch(sets[d], where[d], pair + (d + NG) * stride);
+          look_up(where[d], pair + (d + 2 * NG) * stride);
+          __builtin_amdgcn_sched_barrier(0);  // the loads leave before the next pair's arithmetic
+        }
+      }
+#pragma unroll
+      for (int d = 0; d < NG; ++d) attend(sets[d], pair + d * stride);  // the last round
+    }
+    st.l = column_sum(st.l);
   }
 
-  // Merge the waves' states: every wave leaves its own in LDS (the columns that are heads), then takes the chunks
-  // wave, wave + NW, ... of sixteen dims from all of them. (Merged by one wave from values read one by one, this took
-  // 0.9 us of a launch of 6.4 at 512 keys; now 0.3.)
-  const int cols = min(16, group), per_chunk = 4 * cols;
-  if (grp == 0) {
-    sm_m[wave][col] = st.m;
-    sm_l[wave][col] = st.l;
-  }
-  const int at = grp * cols + min(col, cols - 1);
+  // Merge the waves' states: every wave leaves its own in LDS (the columns that are heads), as [chunk of sixteen dims][lane group]
+  // [column]; thread i then makes the i-th four dims from all of them. (One wave does it for up to four heads of 64. Dealt to all waves
+  // by chunks, lanes without a head reading along, the reads alone took LDS 768 cycles of a launch of 12,000.)
+  const int cols = min(16, group), per_state = DCH * 4 * cols;
+  const float by_cols = (1.f + 1.f / 4096.f) / (float)cols;  // item / cols: right for every item below 512 and up to 16 columns
+  if (grp == 0) reinterpret_cast<float2*>(sm_ml[col])[wave] = float2{st.m, st.l};
 #pragma unroll
   for (int c = 0; c < DCH; ++c)
-    if (col < cols) sm_o[(wave * DCH + c) * per_chunk + at] = st.o[c];
+    if (col < cols) sm_o[wave * per_state + (c * 4 + grp) * cols + col] = st.o[c];
   __syncthreads();
-  float m_w[NW], l_w[NW];
-#pragma unroll
-  for (int w = 0; w < NW; ++w) {
-    m_w[w] = sm_m[w][col];
-    l_w[w] = sm_l[w][col];
-  }
-  constexpr int CW = (DCH + NW - 1) / NW;  // chunks a wave merges
-  float4v o_w[CW][NW];
-#pragma unroll
-  for (int i = 0; i < CW; ++i)
-#pragma unroll
-    for (int w = 0; w < NW; ++w) o_w[i][w] = sm_o[(w * DCH + min(wave + NW * i, DCH - 1)) * per_chunk + at];
-  float m_all = m_w[0];
-#pragma unroll
-  for (int w = 1; w < NW; ++w) m_all = max2(m_all, m_w[w]);
-  const float m_safe = m_all == -INFINITY ? 0.f : m_all;
-  float l_all = 0.f;
-#pragma unroll
-  for (int w = 0; w < NW; ++w) {
-    const float sw = fast_exp2(m_w[w] - m_safe);
-    l_all += l_w[w] * sw;
-#pragma unroll
-    for (int i = 0; i < CW; ++i) o_w[i][0] = w == 0 ? o_w[i][0] * sw : o_w[i][0] + o_w[i][w] * sw;
-  }
-  if (splits == 1) {
-    if (!valid) return;
-    const float inv = l_all > 0.f ? 1.f / l_all : 0.f;
-    bf16_t* op = out + (int64_t)e * out_stride + (int64_t)head * D + 4 * grp;
-#pragma unroll
-    for (int i = 0; i < CW; ++i) {
-      const int c = wave + NW * i;
-      const float4v y = o_w[i][0] * inv;
-      const short4v packed = {bf16_bits(y[0]), bf16_bits(y[1]), bf16_bits(y[2]), bf16_bits(y[3])};
-      if (c < DCH) *reinterpret_cast<short4v*>(op + c * 16) = packed;
-    }
-    return;
-  }
-  if (arrivals == nullptr) {  // attention_merge_kernel follows
-    if (!valid) return;
-    const int64_t slot = ((int64_t)e * q_heads + head) * splits + split;
-    float* po = part_o + slot * D + 4 * grp;
-#pragma unroll
-    for (int i = 0; i < CW; ++i) {
-      const int c = wave + NW * i;
-      if (c < DCH) *reinterpret_cast<float4v*>(po + c * 16) = o_w[i][0];
-    }
-    if (wave == 0 && grp == 0) {
-      part_ml[slot * 2] = m_all;
-      part_ml[slot * 2 + 1] = l_all;
-    }
-    return;
-  }
+  const int q_heads = kv_heads * group;
+  float* part_o = p.part_o;
+  float* part_ml = p.part_ml;
   // The workgroup that finishes last of those that share (request, kv head, head tile) merges their
   // results, which saves the launch of a kernel that is one trip to memory long. Each workgroup
   // stores its partial results at the device's scope (through the caches that only a part of the
@@ -360,16 +416,45 @@ __global__ __launch_bounds__(NW * 64) void attention_decode_kernel(
   // launch. (Ordinary stores and loads with a release and an acquire fence of the device's scope
   // on the way give the same result, but those fences write back and empty the whole level-2
   // cache under the workgroups that still stream keys: 40 us instead of 16 for the launch.)
-  if (valid) {
-    const int64_t slot = ((int64_t)e * q_heads + head) * splits + split;
-    const __amdgpu_buffer_rsrc_t po = device_scope_buffer(part_o);
+#pragma unroll 1
+  for (int first = wave * DLI_WAVE; first < per_state; first += NW * DLI_WAVE) {
+    const int item = min(first + lane, per_state - 1), quad = (int)(item * by_cols), own = item - quad * cols;
+    const bool mine = first + lane < per_state && ht * 16 + own < group;
+    const int own_head = kvh * group + ht * 16 + own, dim = 4 * quad;
+    float4v ml[NW / 2], o_w[NW];
 #pragma unroll
-    for (int i = 0; i < CW; ++i) {
-      const int c = wave + NW * i;
-      if (c < DCH) device_store4(po, (unsigned)((slot * D + 4 * grp + c * 16) * 4), o_w[i][0]);
+    for (int w = 0; w < NW / 2; ++w) ml[w] = sm_ml[own][w];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) o_w[w] = sm_o[w * per_state + item];
+    float m_all = ml[0][0];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) m_all = max2(m_all, ml[w / 2][w % 2 * 2]);
+    const float m_safe = m_all == -INFINITY ? 0.f : m_all;
+    float l_all = 0.f;
+    float4v o_all = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float sw = fast_exp2(ml[w / 2][w % 2 * 2] - m_safe);
+      l_all += ml[w / 2][w % 2 * 2 + 1] * sw;
+      o_all = o_all + o_w[w] * sw;
     }
-    if (wave == 0 && grp == 0) device_store2(device_scope_buffer(part_ml), (unsigned)(slot * 2 * 4), merge_float2{m_all, l_all});
+    if (!mine) continue;
+    if (splits == 1) {
+      const float4v y = o_all * (l_all > 0.f ? 1.f / l_all : 0.f);
+      const short4v packed = {bf16_bits(y[0]), bf16_bits(y[1]), bf16_bits(y[2]), bf16_bits(y[3])};
+      *reinterpret_cast<short4v*>(p.out + (int64_t)e * p.out_stride + (int64_t)own_head * D + dim) = packed;
+      continue;
+    }
+    const int64_t slot = ((int64_t)e * q_heads + own_head) * splits + split;
+    if (arrivals == nullptr) {  // attention_merge_kernel, or the product that merges, follows
+      *reinterpret_cast<float4v*>(part_o + slot * D + dim) = o_all;
+      if (quad == 0) *reinterpret_cast<float2*>(part_ml + slot * 2) = float2{m_all, l_all};
+    } else {
+      device_store4(device_scope_buffer(part_o), (unsigned)((slot * D + dim) * 4), o_all);
+      if (quad == 0) device_store2(device_scope_buffer(part_ml), (unsigned)(slot * 2 * 4), merge_float2{m_all, l_all});
+    }
   }
+  if (splits == 1 || arrivals == nullptr) return;
   // every store of every wave has been acknowledged before the count goes up ...
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_s_waitcnt(0);
@@ -391,7 +476,7 @@ __global__ __launch_bounds__(NW * 64) void attention_decode_kernel(
     const int64_t base = ((int64_t)e * q_heads + merged_head) * splits;
     const float4v y = merged_quad<true>(part_o, part_ml, base, splits, D, d);
     const short4v packed = {bf16_bits(y[0]), bf16_bits(y[1]), bf16_bits(y[2]), bf16_bits(y[3])};
-    *reinterpret_cast<short4v*>(out + (int64_t)e * out_stride + (int64_t)merged_head * D + d) = packed;
+    *reinterpret_cast<short4v*>(p.out + (int64_t)e * p.out_stride + (int64_t)merged_head * D + d) = packed;
   }
 }
 
@@ -1145,11 +1230,16 @@ static int attention_decode(const void* q, int64_t q_stride, const void* k_pages
   unsigned* counters = self_merging ? arrivals : nullptr;
   const size_t lds = decode_states(group, head_dim);
   const bool eight = dli_attention_decode_waves((int64_t)splits * kv_heads * head_tiles * requests, group, head_dim, dli_compute_units()) == 8;
+  const DecodeArgs args{(const bf16_t*)q, q_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages, (bf16_t*)out, out_stride, part_o,
+                        part_ml, counters, group, page_size, scale * LOG2E};
+  const PageOf page_of = page_of_tile(page_size), kv_head_of = page_of_tile(16 * head_tiles);
+  // (a table without entries, whose requests hold no keys: something that can be read, and is not used)
+  const int* tables = table_stride > 0 ? block_tables : kv_len;
+  const int table_width = table_stride > 0 ? table_stride : 1;
 #define DECODE_LAUNCH(N, NW)                                                                      \
-    attention_decode_kernel<N, NW><<<grid, NW * 64, lds * (NW / 4), stream>>>(                     \
-        (const bf16_t*)q, q_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages, (bf16_t*)out, \
-        out_stride, part_o, part_ml, kv_len, block_tables, table_stride, q_heads, kv_heads, group, \
-        head_tiles, page_size, page_of_tile(page_size), scale * LOG2E, window, splits, counters)
+    attention_decode_kernel<N, NW><<<grid, NW * 64, lds * (NW / 4), stream>>>(kv_len, tables, table_width, window, splits, page_of.tiles, \
+                                                                     page_of.reciprocal, kv_head_of.tiles, kv_head_of.reciprocal,  \
+                                                                     kv_heads, args)
 #define DECODE_CASE(N)                     \
   case N:                                  \
     if (eight) DECODE_LAUNCH(N, 8);        \

@@ -138,7 +138,8 @@ __device__ __forceinline__ float rotated(float own, float other, float cosine, f
 // half is the quotient for every tile below 2^32 / tiles.
 struct PageOf {
   unsigned tiles, reciprocal;
-  __device__ __forceinline__ unsigned page(unsigned tile) const { return tiles == 1 ? tile : __umulhi(tile, reciprocal); }
+  // (pages of one tile: reciprocal 0 and the tile itself; no branch, which would part the loads that wait for their pages)
+  __device__ __forceinline__ unsigned page(unsigned tile) const { return __umulhi(tile, reciprocal) + (tiles == 1 ? tile : 0u); }
 };
 static inline PageOf page_of_tile(int page_size) {
   const unsigned tiles = (unsigned)page_size / 16;

@@ -1317,7 +1317,7 @@ def attention_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tens
     if not merge:
         _check(library().dli_attention_decode_partial_bf16(
             _ptr(q), q.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(part_o), _ptr(part_ml), _ptr(kv_len),
-            _ptr(block_tables), block_tables.stride(0), rows, q_heads, kv_heads, head_dim, page_size, float(scale),
+            _ptr(block_tables), block_tables.shape[1], rows, q_heads, kv_heads, head_dim, page_size, float(scale),
             int(window), int(splits), _stream()), "attention_decode")
         return
     if arrivals is not None and splits > 1:
@@ -1326,12 +1326,12 @@ def attention_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tens
                  "one arrival counter per request, kv head and tile of 16 heads")
         _check(library().dli_attention_decode_self_merging_bf16(
             _ptr(q), q.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(out), out.stride(0), _ptr(part_o), _ptr(part_ml),
-            _ptr(arrivals), _ptr(kv_len), _ptr(block_tables), block_tables.stride(0), rows, q_heads, kv_heads,
+            _ptr(arrivals), _ptr(kv_len), _ptr(block_tables), block_tables.shape[1], rows, q_heads, kv_heads,
             head_dim, page_size, float(scale), int(window), int(splits), _stream()), "attention_decode")
         return
     _check(library().dli_attention_decode_bf16(
         _ptr(q), q.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(out), out.stride(0), _ptr(part_o), _ptr(part_ml),
-        _ptr(kv_len), _ptr(block_tables), block_tables.stride(0), rows, q_heads, kv_heads, head_dim, page_size,
+        _ptr(kv_len), _ptr(block_tables), block_tables.shape[1], rows, q_heads, kv_heads, head_dim, page_size,
         float(scale), int(window), int(splits), _stream()), "attention_decode")
 
 
@@ -1354,7 +1354,7 @@ def attention_decode_static(q: torch.Tensor, k_pages: torch.Tensor, v_pages: tor
     _require(1 <= splits <= 65535 and rows <= 65535, "splits and requests must fit the grid")
     status = library().dli_attention_decode_bf16_static(
         _ptr(q), q.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(out), out.stride(0), _ptr(kv_len),
-        _ptr(block_tables), block_tables.stride(0), rows, q_heads, kv_heads, head_dim, page_size, float(scale),
+        _ptr(block_tables), block_tables.shape[1], rows, q_heads, kv_heads, head_dim, page_size, float(scale),
         int(window), int(splits), _stream())
     if status == -3:
         raise KernelArgumentError(

@@ -1,0 +1,63 @@
+"""Decode attention in pairs of key tiles."""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from kernel_refs import ref_paged_attention
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from dli_amd.kernels import ops as o
+
+    o.library()
+    return o
+
+
+def _pool(shape, gen, offset):
+    """Values in a buffer that begins `offset` elements behind an allocation."""
+    n = math.prod(shape)
+    flat = torch.empty(n + offset, dtype=torch.bfloat16, device="cuda")
+    flat[offset:] = torch.randn(n, generator=gen).bfloat16().cuda()
+    return flat[offset:].view(shape)
+
+
+# a wave's first and second pair of tiles (32 keys), its rounds of two to four pairs, the last tile's edges
+@pytest.mark.parametrize("keys", [1, 16, 17, 31, 32, 33, 48, 255, 256, 257, 511, 513, 1024, 1025, 2600])
+@pytest.mark.parametrize("qh,kvh,d,bs,splits,window", [(9, 3, 64, 16, 1, 0), (8, 2, 32, 32, 2, 0), (6, 2, 128, 16, 3, 700), (5, 5, 48, 16, 1, 20)])
+def test_pairs_of_tiles_at_their_edges(ops, keys, qh, kvh, d, bs, splits, window):
+    """One request whose table holds its pages and nothing more, pages that begin 8 bytes behind a multiple of 16, slots past the last
+    key not a number; the same bits beside other requests. Probabilities and results are rounded to bfloat16 (2^-9 each), values
+    are below 4.5: 1.8e-2."""
+    gen = torch.Generator().manual_seed(keys + d)
+    pages = -(-keys // bs)
+    kp, vp = _pool((pages + 2, kvh, bs, d), gen, 4), _pool((pages + 2, kvh, d, bs), gen, 4)
+    table = torch.randperm(pages + 2, generator=gen)[:pages].int()
+    rest = pages * bs - keys
+    if rest:
+        kp[int(table[-1]), :, bs - rest:] = float("nan")
+        vp[int(table[-1]), :, :, bs - rest:] = float("nan")
+    q = torch.randn(2, qh * d, generator=gen).bfloat16().cuda()
+    scale = 1.0 / math.sqrt(d)
+    dev = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+
+    def run(rows, kv_len, tables):
+        po = torch.full((rows * qh * splits * d,), float("nan"), device="cuda")
+        ml = torch.full((rows * qh * splits * 2,), float("nan"), device="cuda")
+        out = torch.full((rows, qh * d), 9.0, dtype=torch.bfloat16, device="cuda")
+        ops.attention_decode(q[:rows], kp, vp, out, dev(kv_len), tables, qh, scale, window, splits, po, ml)
+        return out
+
+    one = table[None].cuda()
+    got = run(1, [keys], one)
+    want = ref_paged_attention(q[:1].cpu(), kp.cpu().nan_to_num(), vp.cpu().nan_to_num(), [0, 1], [keys], one.tolist(), qh, scale, window)
+    assert (got.cpu().double() - want).abs().max().item() < 1.8e-2
+    wide = torch.cat([one.repeat(2, 1), torch.zeros(2, 3, dtype=torch.int32, device="cuda")], 1).contiguous()
+    both = run(2, [keys, 0], wide)
+    assert torch.equal(both[:1], got) and not both[1].any()

@@ -61,26 +61,23 @@ __device__ __forceinline__ void device_store2(__amdgpu_buffer_rsrc_t r, unsigned
 // (`ask`), so that the caller may ask for other things before it has them added up (`merged`).
 // SAME_LAUNCH: the partial results were stored by other workgroups of this launch (each array
 // under 4 GB).
-template <bool SAME_LAUNCH = false>
+// MOST: 2, 4, 8 or 16, no fewer than the S runs. (The kernels take the least: written out for sixteen runs the sums of two are 700
+// cycles of a chain that nothing hides. What is added for runs that are not there are zeros, so the bits do not depend on it.)
+template <int MOST, bool SAME_LAUNCH = false>
 struct MergeQuad {
-  merge_float2 ml[MERGE_SPLITS];
-  merge_float4 po[MERGE_SPLITS];
+  merge_float2 ml[MOST];
+  merge_float4 po[MOST];
 
   __device__ __forceinline__ void ask(const float* part_o, const float* part_ml, int64_t base, int S, int head_dim, int d) {
 #pragma unroll
-    for (int j = 0; j < MERGE_SPLITS; ++j) {
-      ml[j] = merge_float2{-INFINITY, 0.f};
-      po[j] = merge_float4{0.f, 0.f, 0.f, 0.f};
-      if (j < S) {
-        const float* ml_at = part_ml + (base + j) * 2;
-        const float* po_at = part_o + (base + j) * head_dim + d;
-        if constexpr (SAME_LAUNCH) {
-          ml[j] = device_load2(device_scope_buffer(part_ml), (unsigned)((base + j) * 2 * 4));
-          po[j] = device_load4(device_scope_buffer(part_o), (unsigned)(((base + j) * head_dim + d) * 4));
-        } else {
-          ml[j] = *reinterpret_cast<const merge_float2*>(ml_at);
-          po[j] = *reinterpret_cast<const merge_float4*>(po_at);
-        }
+    for (int j = 0; j < MOST; ++j) {
+      const int64_t slot = base + min(j, S - 1);  // (a run that is not there: the last again, which counts as nothing)
+      if constexpr (SAME_LAUNCH) {
+        ml[j] = device_load2(device_scope_buffer(part_ml), (unsigned)(slot * 2 * 4));
+        po[j] = device_load4(device_scope_buffer(part_o), (unsigned)((slot * head_dim + d) * 4));
+      } else {
+        ml[j] = *reinterpret_cast<const merge_float2*>(part_ml + slot * 2);
+        po[j] = *reinterpret_cast<const merge_float4*>(part_o + slot * head_dim + d);
       }
     }
   }
@@ -88,24 +85,24 @@ struct MergeQuad {
   __device__ __forceinline__ merge_float4 merged(int S) const {
     float m_all = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < MERGE_SPLITS; ++j) m_all = fmaxf(m_all, ml[j][0]);
+    for (int j = 0; j < MOST; ++j) m_all = fmaxf(m_all, ml[j][0]);
     const float m_safe = m_all == -INFINITY ? 0.f : m_all;
-    float wgt[MERGE_SPLITS], t[MERGE_SPLITS];
+    float wgt[MOST], t[MOST];
 #pragma unroll
-    for (int j = 0; j < MERGE_SPLITS; ++j) {
+    for (int j = 0; j < MOST; ++j) {
       wgt[j] = j < S ? __builtin_amdgcn_exp2f(ml[j][0] - m_safe) : 0.f;
-      t[j] = __fmul_rn(ml[j][1], wgt[j]);
+      t[j] = j < S ? __fmul_rn(ml[j][1], wgt[j]) : 0.f;
     }
 #pragma unroll
-    for (int h = MERGE_SPLITS / 2; h > 0; h >>= 1)
+    for (int h = MOST / 2; h > 0; h >>= 1)
 #pragma unroll
       for (int j = 0; j < h; ++j) t[j] = __fadd_rn(t[j], t[j + h]);
     const float inv = t[0] > 0.f ? 1.f / t[0] : 0.f;
     merge_float4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int j = 0; j < MERGE_SPLITS; ++j)
+    for (int j = 0; j < MOST; ++j)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = __fmaf_rn(po[j][i], wgt[j], acc[i]);
+      for (int i = 0; i < 4; ++i) acc[i] = j < S ? __fmaf_rn(po[j][i], wgt[j], acc[i]) : acc[i];
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i] = __fmul_rn(acc[i], inv);
     return acc;
@@ -115,7 +112,12 @@ struct MergeQuad {
 template <bool SAME_LAUNCH = false>
 __device__ __forceinline__ merge_float4 merged_quad(const float* part_o, const float* part_ml, int64_t base, int S,
                                                     int head_dim, int d) {
-  MergeQuad<SAME_LAUNCH> parts;
-  parts.ask(part_o, part_ml, base, S, head_dim, d);
-  return parts.merged(S);
+  auto merge = [&](auto parts) __attribute__((always_inline)) {
+    parts.ask(part_o, part_ml, base, S, head_dim, d);
+    return parts.merged(S);
+  };
+  if (S <= 2) return merge(MergeQuad<2, SAME_LAUNCH>());
+  if (S <= 4) return merge(MergeQuad<4, SAME_LAUNCH>());
+  if (S <= 8) return merge(MergeQuad<8, SAME_LAUNCH>());
+  return merge(MergeQuad<16, SAME_LAUNCH>());
 }

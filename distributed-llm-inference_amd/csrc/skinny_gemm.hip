@@ -15,7 +15,7 @@
 // so that the 16 features x 128 k of one tile and block are 4 KB of consecutive memory in the
 // order in which the lanes take them (lane = 16*g + c) and every load of a wave is 1 KB of
 // consecutive bytes. Needs K % 128 == 0 and whole tiles (N % 16 == 0, gate and up parts included); EPI_QKV behind a
-// norm also takes K % 32 == 0, the last block filled up with zeros.
+// norm and MERGED also take K % 32 == 0, the last block filled up with zeros.
 //
 // Fused in (template switches):
 //   NORM     xhat = cast(norm_w[k] * cast(x[m][k] * rs[m])), rs[m] = rsqrt(sum_k x^2 / K + eps),
@@ -118,13 +118,15 @@ __device__ __forceinline__ bf16x8 finish_x(const XFrag<NORM>& f, float rs) {
 // a workgroup computes NS*NT tiles of 16 features with KS*NS waves. The activation fragments are
 // loaded once per block of k and reused for the wave's NT tiles.
 // AHEAD: up to four rows, no wave has a single block of k (two_blocks_or_none), and the second sets out with the first.
-template <int KS, int NS, int NT, int MT, int EPI, bool NORM, bool TILED, bool AHEAD, bool MERGED = false>
+// RUNS: 0, or (MERGED) 2, 4, 8 or 16, no fewer than the runs of keys that are merged.
+template <int KS, int NS, int NT, int MT, int EPI, bool NORM, bool TILED, bool AHEAD, int RUNS = 0>
 __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
     const bf16_t* __restrict__ x, int64_t ldx, const float* __restrict__ ssq_in, int ssq_parts,
     const float* __restrict__ norm_w, float eps, const bf16_t* __restrict__ w,
     const bf16_t* __restrict__ bias, void* __restrict__ out, int64_t ldo,
     bf16_t* __restrict__ stream, int64_t lds_, float* __restrict__ ssq_out, int M, int N, int K,
     int up_offset, QkvRope qr, MergedIn mi, GluForm glu) {
+  constexpr bool MERGED = RUNS != 0;
   static_assert(EPI != EPI_QKV || (TILED && MT == 1), "the q/k/v epilogue reads tiled weights, at most 16 rows");
   static_assert(!MERGED || (TILED && MT == 1 && NS == 1 && !NORM), "merged activations: tiled weights, one row tile");
   static_assert(!AHEAD || (MT == 1 && !NORM && !MERGED), "one row tile, no sums of squares to wait for");
@@ -132,6 +134,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
   // MERGED: each wave's run of k for up to MERGE_ROWS rows
   __shared__ __align__(16) bf16_t xs[MERGED ? KS : 1][MERGED ? MERGE_ROWS : 1][MERGED ? MERGE_RANGE : 8];
   constexpr int NA = EPI == EPI_SWIGLU ? 2 : 1;  // weight row sets per tile (gate and up)
+  constexpr bool PADDED = EPI == EPI_QKV || MERGED;  // the weights' last block of 128 k may be filled up with zeros
   // What follows the last product is a chain that nothing hides, so it is kept short. With one row
   // tile and one group of waves (SHORT) all waves leave their parts in LDS and thread t makes
   // output t of each tile: element t % 4 of lane t / 4 of the product's result, that is row
@@ -156,7 +159,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
       if constexpr (TILED) {
         // the tile's first block, at this lane's 16 bytes of a 1 KB load
         const int tile = min(tile0 + j, (N - 1) / 16) + a * (up_offset / 16);
-        wrow[j][a] = w + (int64_t)tile * 16 * (EPI == EPI_QKV ? (K + 127) / 128 * 128 : K) + lane * 8;
+        wrow[j][a] = w + (int64_t)tile * 16 * (PADDED ? (K + 127) / 128 * 128 : K) + lane * 8;
       } else {
         const int n = min((tile0 + j) * 16 + col, N - 1) + a * up_offset;
         wrow[j][a] = w + (int64_t)n * K + grp * 32;
@@ -229,7 +232,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
 
   // this wave's share of the k steps of 32
   const int steps = K / 32;
-  const int whole = EPI == EPI_QKV ? (steps + 3) / 4 : steps / 4;   // (EPI_QKV: the last block may be filled up with zeros)
+  const int whole = PADDED ? (steps + 3) / 4 : steps / 4;
   const int s_begin = TILED ? 4 * (int)((int64_t)whole * ks / KS) : (int)((int64_t)steps * ks / KS);
   const int s_end = TILED ? 4 * (int)((int64_t)whole * (ks + 1) / KS) : (int)((int64_t)steps * (ks + 1) / KS);
   int s = s_begin;
@@ -340,9 +343,9 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
     // come back in their order), which are on their way while the merge is made.
     const int kb0 = s_begin * 32, quads = (s_end - s_begin) * 8, items = M * quads;
     const int D = mi.head_dim, S = mi.splits;
-    MergeQuad<> parts;
+    MergeQuad<MERGED ? RUNS : 2> parts;
     auto ask = [&](int item) __attribute__((always_inline)) {
-      const int row = item / quads, k = kb0 + (item - row * quads) * 4, head = k / D;
+      const int row = item / quads, k = min(kb0 + (item - row * quads) * 4, K - 4), head = k / D;   // (past K: zeros, below)
       parts.ask(mi.part_o, mi.part_ml, ((int64_t)row * mi.heads + head) * S, S, D, k - head * D);
     };
     if (items > 0) ask(min(lane, items - 1));
@@ -358,7 +361,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
         const int row = item / quads;
         bf16_t* dst = &xs[ks][row][(item - row * quads) * 4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) dst[i] = (bf16_t)merged[i];
+        for (int i = 0; i < 4; ++i) dst[i] = (bf16_t)(kb0 + (item - row * quads) * 4 < K ? merged[i] : 0.f);
       }
     }
     __syncthreads();
@@ -1127,26 +1130,35 @@ extern "C" int dli_skinny_gemm_qkv_rope(const void* x, int64_t ldx, const float*
 // The o projection of a decode step of at most MERGE_ROWS rows, fed with the split-key partial
 // results of the attention instead of its merged output (MERGED above): stream += merge(...) @ w^T
 // (+ bias), and the parts of the rows' sums of squares. w_tiled [N, K] in tile order with
-// K = heads * head_dim; splits 2..MERGE_SPLITS; shape 0 or 1 (4 or 8 waves split k).
+// K = heads * head_dim, filled up with zeros to whole blocks of 128; splits 2..MERGE_SPLITS; shape 0 or 1 (4 or 8 waves split k).
 extern "C" int dli_skinny_gemm_merged(const float* part_o, const float* part_ml, int splits, int heads,
                                       int head_dim, const void* w_tiled, const void* bias, void* stream_buf,
                                       int64_t lds_, float* ssq_out, int M, int N, int shape, hipStream_t stream) {
   if (M <= 0 || N <= 0) return DLI_OK;
   const int64_t K64 = (int64_t)heads * head_dim;
   if (M > MERGE_ROWS || splits < 2 || splits > MERGE_SPLITS || heads <= 0 || head_dim <= 0 || head_dim % 4 != 0 ||
-      K64 % 128 != 0 || K64 > (1 << 20) || N % 16 != 0 || (shape != 0 && shape != 1) || part_o == nullptr ||
+      K64 % 32 != 0 || K64 > (1 << 20) || N % 16 != 0 || (shape != 0 && shape != 1) || part_o == nullptr ||
       part_ml == nullptr || w_tiled == nullptr || stream_buf == nullptr || ssq_out == nullptr)
     return DLI_ERR_ARGUMENT;
   const int K = (int)K64, ks = shape == 0 ? 4 : 8;
-  if (((K / 128 + ks - 1) / ks) * 128 > MERGE_RANGE) return DLI_ERR_ARGUMENT;
+  if ((((K + 127) / 128 + ks - 1) / ks) * 128 > MERGE_RANGE) return DLI_ERR_ARGUMENT;
   const MergedIn mi{part_o, part_ml, splits, heads, head_dim};
   const int groups = N / 16;
-#define MERGED_LAUNCH(KS)                                                                          \
-  skinny_gemm_kernel<KS, 1, 1, 1, EPI_RESIDUAL, false, true, false, true><<<groups, KS * 64, 0, stream>>>( \
+#define MERGED_LAUNCH(KS, RUNS)                                                                    \
+  skinny_gemm_kernel<KS, 1, 1, 1, EPI_RESIDUAL, false, true, false, RUNS><<<groups, KS * 64, 0, stream>>>( \
       nullptr, 0, nullptr, 0, nullptr, 0.f, (const bf16_t*)w_tiled, (const bf16_t*)bias, nullptr, 0, \
       (bf16_t*)stream_buf, lds_, ssq_out, M, N, K, 0, QkvRope{}, mi, GluForm{})
-  if (shape == 0) MERGED_LAUNCH(4);
-  else MERGED_LAUNCH(8);
+#define MERGED_RUNS(KS)                       \
+  if (splits <= 2) MERGED_LAUNCH(KS, 2);      \
+  else if (splits <= 4) MERGED_LAUNCH(KS, 4); \
+  else if (splits <= 8) MERGED_LAUNCH(KS, 8); \
+  else MERGED_LAUNCH(KS, 16)
+  if (shape == 0) {
+    MERGED_RUNS(4);
+  } else {
+    MERGED_RUNS(8);
+  }
+#undef MERGED_RUNS
 #undef MERGED_LAUNCH
   return dli_launch_status();
 }

@@ -795,20 +795,20 @@ def skinny_gemm_merged_supports(rows: int, n: int, heads: int, head_dim: int, sp
     """Whether :func:`skinny_gemm_merged` takes this o projection: few rows, few runs of keys, a
     product that the 16x16-tile kernel runs with k split over the waves of a workgroup."""
     k = heads * head_dim
-    if not (0 < rows <= MERGED_ROWS and 2 <= splits <= MERGED_SPLITS and head_dim % 4 == 0 and k % 128 == 0
-            and n % 16 == 0):
+    if not (0 < rows <= MERGED_ROWS and 2 <= splits <= MERGED_SPLITS and head_dim % 4 == 0 and n % 16 == 0
+            and (k % 128 == 0 or (k % 32 == 0 and k > 512))):
         return False
     return _merged_shape(rows, n, k, device) is not None
 
 
 def _merged_shape(rows: int, n: int, k: int, device: torch.device) -> Optional[int]:
     """The workgroup shape (0: four k-waves, 1: eight) with which the merging o projection runs:
-    that of the plain product with the residual sum, so that both add in the same order, or None
-    if that one runs on another kernel or a wave's run of k does not fit the merge's buffer."""
-    kernel, shape, _ = skinny_gemm_plan(rows, n, k, SKINNY_RESIDUAL, device, tiled=True)
+    that of the plain product with the residual sum, so that both add in the same order (where k is whole blocks of 128; else that
+    one reads the weights row by row), or None if that one runs on another kernel or a wave's run of k does not fit the merge's buffer."""
+    kernel, shape, _ = skinny_gemm_plan(rows, n, k, SKINNY_RESIDUAL, device, tiled=k % 128 == 0)
     if kernel != "tiles16" or shape not in (0, 1):
         return None
-    return shape if -(-(k // 128) // (4 if shape == 0 else 8)) * 128 <= _MERGED_RANGE else None
+    return shape if -(-(padded_k(k) // 128) // (4 if shape == 0 else 8)) * 128 <= _MERGED_RANGE else None
 
 
 def skinny_gemm_merged(part_o: torch.Tensor, part_ml: torch.Tensor, splits: int, heads: int, head_dim: int,
@@ -831,11 +831,11 @@ def skinny_gemm_merged(part_o: torch.Tensor, part_ml: torch.Tensor, splits: int,
              "partial-result buffers are too small")
     _require(part_o.data_ptr() % 16 == 0 and part_ml.data_ptr() % 8 == 0, "partial results must be 16-byte aligned")
     _dense(w_tiled, "w_tiled", torch.bfloat16, 1)
-    _require(w_tiled.numel() == n * k and w_tiled.data_ptr() % 16 == 0, "w_tiled must hold [n, heads*head_dim] in tile order")
+    _require(w_tiled.numel() == n * padded_k(k) and w_tiled.data_ptr() % 16 == 0, "w_tiled must hold [n, heads*head_dim] in tile order")
     if bias is not None:
         _dense(bias, "bias", torch.bfloat16, 1)
         _require(bias.shape[0] == n, "bias length differs from rows of w")
-    _, _, n_parts = skinny_gemm_plan(m, n, k, SKINNY_RESIDUAL, stream.device, tiled=True)
+    n_parts = n // 16
     shape = _merged_shape(m, n, k, stream.device)
     if ssq_out is None:
         ssq_out = torch.empty(n_parts, m, device=stream.device, dtype=torch.float32)

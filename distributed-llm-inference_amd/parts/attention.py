@@ -20,7 +20,7 @@ from typing import Any, Mapping, Optional
 import torch
 
 from ..kernels import ops
-from .attention_kernels import decode_attention_unmerged, paged_attention, planned_splits
+from .attention_kernels import decode_attention_unmerged, paged_attention, planned_splits, runs_for_the_product
 from .base import DecodeStream, Mixer, Norm, PagedKVSpec, Part, Runtime
 from .linear import decode_copy, finish_residual, linear
 from .registry import build_part, register_part
@@ -158,8 +158,12 @@ class GQAttention(Mixer):
         """Into how many runs the decode kernel cuts each request's keys in a recorded step (the 32-bit kernel cuts none)."""
         if not self.rt.is_bf16:
             return None
-        return planned_splits(requests, self.num_heads, self.num_kv_heads, self.head_dim, max_keys,
-                              ops.compute_units(self.rt.device))
+        units = ops.compute_units(self.rt.device)
+        if requests <= MERGE_IN_PRODUCT_ROWS and self.w_o_tiled is not None:
+            runs = runs_for_the_product(self.num_heads, self.num_kv_heads, max_keys, units)
+            if runs == 1 or ops.skinny_gemm_merged_supports(requests, self.hidden_size, self.num_heads, self.head_dim, runs, self.rt.device):
+                return runs
+        return planned_splits(requests, self.num_heads, self.num_kv_heads, self.head_dim, max_keys, units)
 
     # -- step
     def forward(self, x: torch.Tensor, ctx: Any, cache: Any) -> torch.Tensor:

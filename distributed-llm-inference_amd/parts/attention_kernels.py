@@ -72,6 +72,20 @@ def planned_splits(requests: int, q_heads: int, kv_heads: int, head_dim: int, ma
     return coarse
 
 
+def runs_for_the_product(q_heads: int, kv_heads: int, max_keys: int, units: int = 256) -> int:
+    """Runs of keys in a recorded step of one request whose o projection merges them: about 256 keys each, which eight waves have on
+    their way at once, in powers of two; no more workgroups than compute units, since every run is 16 KB and more that each
+    workgroup of the product reads. Passes of eight steps, ms, with 1, 2, 4, ... runs: 135M sizes, 304 keys 4.91 and 4.92, 400 5.19
+    and 5.05, 520 5.30, 4.95 and 5.00, 640 5.56, 5.17 and 5.02, 1,000 (from 2 on) 5.38, 5.02 and 5.09, 2,000 (from 4 on) 5.47, 5.17
+    and 5.55; 1B sizes, 2,000 (from 4 on) 5.78 and 5.64, with 16 5.78, 8,000 (from 16 on) 6.07, 5.99 and 6.14; 1.7B sizes, 4,000 (from
+    4 on) 9.08, 8.87 and 9.11; 3B sizes, 520 13.80, 13.50 and 13.16, 2,000 (from 4 on) 13.76, 13.60 and 14.25."""
+    want, runs = max(1, (max_keys + 128) // 256), 1
+    most = min(MAX_SPLITS, units // head_tiles(q_heads, kv_heads))
+    while runs < want and 2 * runs <= most:
+        runs *= 2
+    return runs
+
+
 # A launch of fewer workgroups than this per compute unit is as long as its longest workgroup, and
 # cutting the keys of its longest tiles into runs, each a workgroup, shortens that (one prompt of
 # 2,048 tokens at the 1B sizes: 43 -> 33 us a layer); with more, the workgroups queue anyway and

@@ -1,4 +1,4 @@
-"""Decode attention in pairs of key tiles."""
+"""Decode attention in pairs of key tiles, and the o projection that merges its runs where the width is no whole blocks of 128."""
 
 from __future__ import annotations
 
@@ -61,3 +61,30 @@ def test_pairs_of_tiles_at_their_edges(ops, keys, qh, kvh, d, bs, splits, window
     wide = torch.cat([one.repeat(2, 1), torch.zeros(2, 3, dtype=torch.int32, device="cuda")], 1).contiguous()
     both = run(2, [keys, 0], wide)
     assert torch.equal(both[:1], got) and not both[1].any()
+
+
+@pytest.mark.parametrize("qh,kvh,d,n", [(9, 3, 64, 576), (15, 5, 64, 960), (17, 1, 32, 272)])
+@pytest.mark.parametrize("splits", [2, 3, 8, 9, 16])
+def test_merging_o_projection_of_odd_widths(ops, qh, kvh, d, n, splits):
+    """Widths that end inside a block of 128: the weights' copy is filled up with zeros, whatever the rows hold there. Against the
+    products of the merged attention in 64 bits: 32-bit sums of bfloat16 products, the sum rounded once, then the stream's (2^-8)."""
+    rows, bs, k = 2, 16, qh * d
+    assert k % 128 and ops.skinny_gemm_merged_supports(rows, n, qh, d, splits, torch.device("cuda", 0))
+    gen = torch.Generator().manual_seed(n + splits)
+    lens = [700, 33]
+    width = -(-lens[0] // bs)
+    kp, vp = _pool((2 * width, kvh, bs, d), gen, 0), _pool((2 * width, kvh, d, bs), gen, 0)
+    tables = torch.randperm(2 * width, generator=gen).view(2, width).int().cuda()
+    q = torch.randn(rows, k, generator=gen).bfloat16().cuda()
+    kv_len = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    w = (torch.randn(n, k, generator=gen) / math.sqrt(k)).bfloat16().cuda()
+    base, bias = torch.randn(rows, n, generator=gen).bfloat16().cuda(), torch.randn(n, generator=gen).bfloat16().cuda()
+    po = torch.full((rows * qh * splits * d,), float("nan"), device="cuda")
+    ml = torch.full((rows * qh * splits * 2,), float("nan"), device="cuda")
+    out = torch.empty_like(q)
+    ops.attention_decode(q, kp, vp, out, kv_len, tables, qh, 0.125, 0, splits, po, ml)
+    got = base.clone()
+    ssq = ops.skinny_gemm_merged(po, ml, splits, qh, d, ops.tile_weights(w, whole_blocks=False), got, bias=bias)
+    want = base.cpu().double() + out.cpu().double() @ w.cpu().double().T + bias.cpu().double()
+    assert ((got.cpu().double() - want).abs() <= 2.0 ** -8 * (want.abs() + base.cpu().double().abs() + 4.0)).all()
+    assert torch.allclose(ssq.sum(0).cpu(), (got.float() ** 2).sum(1).cpu(), rtol=1e-5)

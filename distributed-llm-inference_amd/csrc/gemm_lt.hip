@@ -7,6 +7,7 @@
 // that a call costs a few microseconds on the host instead of the tens that a framework's
 // dispatch takes: an eager step of a few hundred tokens issues 65 products and is bound by the
 // host otherwise. The bias is added inside the product (one rounding, as in the reference).
+// Products whose result is about one tile a compute unit take a kernel of this project instead (tile_gemm.hip).
 #include <hipblaslt/hipblaslt.h>
 
 #include <map>
@@ -14,6 +15,7 @@
 #include <tuple>
 
 #include "common.h"
+#include "tile_gemm.h"
 
 namespace {
 
@@ -84,6 +86,8 @@ int gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bia
          bool out_f32, hipStream_t stream) {
   if (rows <= 0 || feats <= 0) return DLI_OK;
   if (k <= 0 || ldx < k || ldw < k || ldo < feats || workspace_bytes < 0) return DLI_ERR_ARGUMENT;
+  if (tile_gemm_takes(x, ldx, w, ldw, out, ldo, rows, feats, k, out_f32))
+    return tile_gemm(x, ldx, w, ldw, bias, out, ldo, rows, feats, k, out_f32, stream);
   std::lock_guard<std::mutex> lock(g_mutex);
   hipblasLtHandle_t handle = handle_for(device);
   if (handle == nullptr) return DLI_ERR_LAUNCH;

@@ -41,6 +41,10 @@ struct GfArgs {
 #define GF_PLAIN 0
 #define GF_GLU 1    // silu(gate) * up: the first half of w's rows are gates, the second ups
 #define GF_ROPE 2   // q, k and v heads: q and k rotated (the pairs i, i + head_dim / 2), k and v written at their slots
+// How it reads w: word by word, 16 bytes a lane, or 16 bytes a lane by way of LDS (whole halves of runs).
+#define GF_WORDS 0
+#define GF_WIDE 1
+#define GF_STAGED 2
 struct GfAround {
   const float* norm_w;
   float eps;
@@ -73,6 +77,27 @@ __device__ __forceinline__ gf4 gf_load(const float* row, int kk, int k) {
   }
 }
 
+// 16 bytes a lane from its own address into LDS, the wave's lanes one behind the other, without passing registers.
+// (the host's pass over the source does not know this builtin, and would drop every kernel that names it)
+__device__ __forceinline__ void gf_to_lds(const float* from, gf4* to) {
+#ifdef __HIP_DEVICE_COMPILE__
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from, (__attribute__((address_space(3))) void*)to, 16, 0, 0);
+#endif
+}
+// Waits until at most N of the wave's loads are outstanding.
+template <int N>
+__device__ __forceinline__ void gf_wait() {
+  static_assert(N >= 0 && N < 64, "6 bits");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+  asm volatile("" ::: "memory");
+}
+
+// Waits for the wave's reads of LDS.
+__device__ __forceinline__ void gf_wait_lds() {
+  __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));
+  asm volatile("" ::: "memory");
+}
+
 // Lane (i, g) holds rows 4 g .. + 3 of a tile of 16 x 16, column i.
 __device__ __forceinline__ void gf_store(const GfArgs& p, gf4 sum, int m0, int n0, int i, int g) {
   const int col = n0 + i;
@@ -88,53 +113,75 @@ __device__ __forceinline__ void gf_store(const GfArgs& p, gf4 sum, int m0, int n
 }
 
 // Up to 16 rows: KW waves share a tile of 16 x 16 NT and take its segments in turn, each straight from memory: half a run's
-// operands are on their way while the other half is multiplied. (The lanes of a load lie in 16 rows, four neighbours in
-// four of them: as fast as any order where w comes from HBM once, but a quarter of the caches' rate where tiles share it.)
+// operands are on their way while the other half is multiplied. The lanes that multiply lie in 16 rows, four neighbours in four
+// of them: a load so laid out passes the compute unit's loads at a quarter of their rate, and few tiles mean few units.
+// READ == GF_STAGED (k of whole half runs, a tile of sixteen columns) therefore brings w into LDS, four neighbours in 64 bytes of
+// one row, and reads it from there; both halves of a wave's first run are asked for at once. us, weights from memory, two rows,
+// before and now: 576 x 576 4.5 3.3, 576 x 1,536 6.7 5.7, 2,048 x 8,192 24.2 20.6, 49,152 x 576 26.8 21.6, 100,000 x 1,024 77.6 75.1;
+// 16 rows: 576 x 576 5.4 4.0, 2,048 x 8,192 34.0 28.0.
 //
 // FORM GF_GLU and GF_ROPE: the rows are normalised on their way to the matrix cores and the sums go on where they are, so that a
 // decode step's norms, activations and rotations are no kernels of their own (each 2.8 to 3.9 us of a step of two rows, which
 // this one's 5 to 6 outlasts by less than one; two prompts of 333 and 178 tokens and four steps at the 135M sizes:
-// 9.00 -> 8.06 ms a pass). A tile's sixteen columns are then eight of one half and the eight that they are paired with, a rotation
-// by eight lanes away. The norm's sum of squares and its products are those of its own kernel, bit for bit: a wave takes a row,
-// after the first weights are asked for.
-template <int NT, int KW, bool VEC, int FORM = GF_PLAIN>
+// 9.00 -> 8.06 ms a pass, and 7.38 with w through LDS and what the norm and the rotation read asked for ahead of it: q, k and v
+// of two rows at these sizes 6.8 -> 5.0 us, gate and up 6.9 -> 5.5). A tile's sixteen columns are then eight of one half and the
+// eight that they are paired with, a rotation by eight lanes away. The norm's sum of squares and its products are those of
+// its own kernel, bit for bit: a wave takes a row, while the first weights are on their way.
+template <int NT, int KW, int READ, int FORM = GF_PLAIN>
 __global__ __launch_bounds__(64 * KW) void gemm_f32_few_kernel(GfArgs p, GfAround x) {
-  static_assert(FORM == GF_PLAIN || (NT == 1 && VEC), "one tile of whole vectors");
-  extern __shared__ gf4 gf_sums[];   // [segments][NT][64]
-  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, i = lane % 16, g = lane / 16;
+  constexpr bool VEC = READ != GF_WORDS, STAGED = READ == GF_STAGED;
+  static_assert((FORM == GF_PLAIN || VEC) && (NT == 1 || (FORM == GF_PLAIN && !STAGED)), "one tile of whole vectors");
+  constexpr int LOADS = FORM == GF_PLAIN ? 8 : 12;   // a wave's loads for half a run
+  extern __shared__ gf4 gf_sums[];   // [segments][NT][64], then, STAGED, [KW][2][4][64]
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), i = lane % 16, g = lane / 16;
   __shared__ float rstd[16];
   int n0 = blockIdx.x * 16 * NT;
   const float* ra = p.a + (int64_t)min(i, p.m - 1) * p.lda;   // (rows past the end: not stored)
+  int head = 0;
+  bool rotates = false;
+  if constexpr (FORM == GF_GLU) n0 = blockIdx.x * 8;
+  if constexpr (FORM == GF_ROPE) {
+    head = blockIdx.x / (x.head_dim / 16);
+    rotates = head < x.q_heads + x.kv_heads;
+  }
+  const auto row_of_w = [&](int at) {   // of the tile's row `at`
+    if constexpr (FORM == GF_GLU) return (at < 8 ? 0 : p.n / 2) + min(n0 + at % 8, p.n / 2 - 1);
+    if constexpr (FORM == GF_ROPE) {
+      const int t = blockIdx.x % (x.head_dim / 16);
+      return head * x.head_dim + (rotates ? 8 * t + at % 8 + (at < 8 ? 0 : x.head_dim / 2) : 16 * t + at);
+    }
+    return min(n0 + at, p.n - 1);
+  };
+  const int feature = row_of_w(i);   // this lane's row of w (the first of NT)
   const float* rw[NT];
 #pragma unroll
-  for (int y = 0; y < NT; ++y) rw[y] = p.w + (int64_t)min(n0 + 16 * y + i, p.n - 1) * p.ldw;
-  int feature = n0 + i, head = 0;   // this lane's row of w
-  bool rotates = false;
-  if constexpr (FORM == GF_GLU) {
-    n0 = blockIdx.x * 8;
-    feature = (i < 8 ? 0 : p.n / 2) + min(n0 + i % 8, p.n / 2 - 1);
-  }
-  if constexpr (FORM == GF_ROPE) {
-    const int tiles = x.head_dim / 16, t = blockIdx.x % tiles;
-    head = blockIdx.x / tiles;
-    rotates = head < x.q_heads + x.kv_heads;
-    feature = head * x.head_dim + (rotates ? 8 * t + i % 8 + (i < 8 ? 0 : x.head_dim / 2) : 16 * t + i);
-  }
-  if constexpr (FORM != GF_PLAIN) rw[0] = p.w + (int64_t)feature * p.ldw;
+  for (int y = 0; y < NT; ++y) rw[y] = p.w + (int64_t)row_of_w(16 * y + i) * p.ldw;
+  // STAGED: what the lane brings, chunk lane % 4 ^ row / 4 of row lane / 4, and where its own chunk g of row i then lies: a load's
+  // four neighbours in one line, a read's sixteen lanes in banks of their own
+  gf4* const stage = gf_sums + p.segments * NT * 64 + wave * 512;
+  const float* const brings = p.w + (int64_t)row_of_w(lane / 4) * p.ldw + (lane % 4 ^ lane / 16) * 4;
+  const int own = 4 * i + (g ^ i / 4);
   gf4 seg[NT], acc[NT], fa[2][4], fw[2][4][NT], fn[2][FORM != GF_PLAIN ? 4 : 1];
 #pragma unroll
   for (int y = 0; y < NT; ++y) seg[y] = gf4{0.f, 0.f, 0.f, 0.f};
 
   const auto load = [&](auto half, int k0) {   // 64 k from k0 on
     constexpr int b = decltype(half)::value;
-    if (VEC && k0 + GF_RUN / 2 <= p.k) {   // (no choice between the value and zero: it would wait for the load at once)
+    if (STAGED || (VEC && k0 + GF_RUN / 2 <= p.k)) {   // (no choice between the value and zero: it would wait for the load at once)
+      if constexpr (STAGED) {
+        k0 = min(k0, p.k - GF_RUN / 2);   // (behind the last half run: not used)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) gf_to_lds(brings + k0 + 16 * t, stage + (4 * b + t) * 64);
+      }
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         fa[b][t] = *reinterpret_cast<const gf4*>(ra + k0 + 4 * g + 16 * t);
         if constexpr (FORM != GF_PLAIN) fn[b][t] = *reinterpret_cast<const gf4*>(x.norm_w + k0 + 4 * g + 16 * t);
+        if constexpr (!STAGED)
 #pragma unroll
-        for (int y = 0; y < NT; ++y) fw[b][t][y] = *reinterpret_cast<const gf4*>(rw[y] + k0 + 4 * g + 16 * t);
+          for (int y = 0; y < NT; ++y) fw[b][t][y] = *reinterpret_cast<const gf4*>(rw[y] + k0 + 4 * g + 16 * t);
       }
+      if constexpr (STAGED) asm volatile("" ::: "memory");   // (loads are counted: none moves into another half's)
       return;
     }
 #pragma unroll
@@ -146,8 +193,14 @@ __global__ __launch_bounds__(64 * KW) void gemm_f32_few_kernel(GfArgs p, GfAroun
     }
   };
   float r = 1.f;
-  const auto multiply = [&](auto half) {
+  // `behind`: the other half's loads were asked for behind this one's
+  const auto multiply = [&](auto half, auto behind) {
     constexpr int b = decltype(half)::value;
+    if constexpr (STAGED) {
+      gf_wait<decltype(behind)::value ? LOADS : 0>();
+#pragma unroll
+      for (int t = 0; t < 4; ++t) fw[b][t][0] = stage[(4 * b + t) * 64 + own];
+    }
     if constexpr (FORM != GF_PLAIN)
 #pragma unroll
       for (int t = 0; t < 4; ++t) fa[b][t] = fn[b][t] * (fa[b][t] * r);
@@ -159,59 +212,107 @@ __global__ __launch_bounds__(64 * KW) void gemm_f32_few_kernel(GfArgs p, GfAroun
         for (int y = 0; y < NT; ++y) acc[y] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[b][t][s], fw[b][t][y][s], acc[y], 0, 0, 0);
   };
 
+  // What the norm and the rotation read is asked for before the weights, and so is there long before them: loads come back in
+  // their order. (Of the wave's first row, up to 1,024 values.)
+  gf4 row_in[4];
+  float freq = 0.f;
+  int at_position[4], at_slot[4];
+  if constexpr (FORM != GF_PLAIN) {
+    if (wave < p.m) {
+      const float* xr = p.a + (int64_t)wave * p.lda;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int at = min(512 * q + 8 * lane, p.k - 8);
+        row_in[2 * q] = *reinterpret_cast<const gf4*>(xr + at);
+        row_in[2 * q + 1] = *reinterpret_cast<const gf4*>(xr + at + 4);
+      }
+    }
+    if constexpr (FORM == GF_ROPE) {
+      if (wave == 0) {   // the wave that ends the tile
+        freq = x.inv_freq[feature % x.head_dim % (x.head_dim / 2)];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          at_position[e] = x.positions[min(4 * g + e, p.m - 1)];
+          at_slot[e] = x.slots[min(4 * g + e, p.m - 1)];
+        }
+      }
+    }
+    asm volatile("" ::: "memory");
+  }
   const int runs = (p.k + GF_RUN - 1) / GF_RUN;
   int s = wave, left = 0;
-  if (s < p.segments) {
-    load(Zero{}, s * p.seg_runs * GF_RUN);
-    left = min(p.seg_runs, runs - s * p.seg_runs);
-  }
   gf4 c = {1.f, 1.f, 1.f, 1.f}, sn = {0.f, 0.f, 0.f, 0.f};
   int slot[4] = {-1, -1, -1, -1};
-  if constexpr (FORM != GF_PLAIN) {
-    for (int row = wave; row < p.m; row += KW) {
+  const auto prepare = [&](auto behind) {   // the rows' factors to LDS, this lane's rotations
+    if constexpr (STAGED) gf_wait<decltype(behind)::value ? 2 * LOADS : 0>();
+    const auto squares = [](gf4 lo, gf4 hi, float part) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) part = fmaf(lo[e], lo[e], part);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) part = fmaf(hi[e], hi[e], part);
+      return part;
+    };
+    const auto factor = [&](int row, float ss) {
+      if (lane == 0) rstd[row] = rsqrtf(ss / (float)p.k + x.eps);
+    };
+    int row = wave;
+    if (row < p.m && p.k <= 1024) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) asm volatile("" : "+v"(row_in[q]));   // (not used before the weights are asked for)
+      float ss = 0.f, part = 8 * lane < p.k ? squares(row_in[0], row_in[1], 0.f) : 0.f;
+      if (x.norm_waves == 2) {
+        ss = wave_sum(part);
+        part = 0.f;
+      }
+      if (512 + 8 * lane < p.k) part = squares(row_in[2], row_in[3], part);
+      factor(row, ss + wave_sum(part));
+      row += KW;
+    }
+    for (; row < p.m; row += KW) {
       const float* xr = p.a + (int64_t)row * p.lda;
       float ss = 0.f;
       for (int j = 0; j < x.norm_waves; ++j) {
         float part = 0.f;
-        for (int at = (64 * j + lane) * 8; at < p.k; at += 512 * x.norm_waves) {
-          const gf4 lo = *reinterpret_cast<const gf4*>(xr + at), hi = *reinterpret_cast<const gf4*>(xr + at + 4);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) part = fmaf(lo[e], lo[e], part);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) part = fmaf(hi[e], hi[e], part);
-        }
+        for (int at = (64 * j + lane) * 8; at < p.k; at += 512 * x.norm_waves)
+          part = squares(*reinterpret_cast<const gf4*>(xr + at), *reinterpret_cast<const gf4*>(xr + at + 4), part);
         ss += wave_sum(part);
       }
-      if (lane == 0) rstd[row] = rsqrtf(ss / (float)p.k + x.eps);
+      factor(row, ss);
     }
     if constexpr (FORM == GF_ROPE) {
-      if (wave == 0) {   // the wave that ends the tile
-        const float freq = rotates ? x.inv_freq[feature % x.head_dim % (x.head_dim / 2)] : 0.f;
+      if (wave == 0) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
+          asm volatile("" : "+v"(at_position[e]), "+v"(at_slot[e]));
           if (4 * g + e >= p.m) continue;
-          slot[e] = x.slots[4 * g + e];
+          slot[e] = at_slot[e];
           if (rotates) {
             float sine, cosine;
-            sincosf((float)x.positions[4 * g + e] * freq, &sine, &cosine);
+            sincosf((float)at_position[e] * freq, &sine, &cosine);
             c[e] = cosine;
             sn[e] = i < 8 ? -sine : sine;
           }
         }
       }
     }
+  };
+  if (s < p.segments) {
+    load(Zero{}, s * p.seg_runs * GF_RUN);
+    if constexpr (STAGED) load(One{}, s * p.seg_runs * GF_RUN + GF_RUN / 2);
+    left = min(p.seg_runs, runs - s * p.seg_runs);
+    if constexpr (FORM != GF_PLAIN) prepare(One{});   // (written out for both sides: how many loads are behind the row's is known then)
+  } else if constexpr (FORM != GF_PLAIN) {
+    prepare(Zero{});
+  }
+  if constexpr (FORM != GF_PLAIN) {
     __syncthreads();
     r = rstd[min(i, p.m - 1)];
   }
-  for (int u = s * p.seg_runs; s < p.segments;) {   // run u of segment s, `left` runs of it to go
+  const auto begin = [&] {
 #pragma unroll
     for (int y = 0; y < NT; ++y) acc[y] = gf4{0.f, 0.f, 0.f, 0.f};
-    load(One{}, u * GF_RUN + GF_RUN / 2);
-    multiply(Zero{});
-    const bool last = --left == 0;
-    const int s_next = last ? s + KW : s, r_next = last ? s_next * p.seg_runs : u + 1;
-    if (s_next < p.segments) load(Zero{}, r_next * GF_RUN);
-    multiply(One{});
+  };
+  const auto end = [&](bool last) {   // of a run, the last of its segment
 #pragma unroll
     for (int y = 0; y < NT; ++y) {
       seg[y] += acc[y];
@@ -220,9 +321,31 @@ __global__ __launch_bounds__(64 * KW) void gemm_f32_few_kernel(GfArgs p, GfAroun
         seg[y] = gf4{0.f, 0.f, 0.f, 0.f};
       }
     }
-    if (last && s_next < p.segments) left = min(p.seg_runs, runs - r_next);
-    s = s_next;
-    u = r_next;
+  };
+  if (s < p.segments) {
+    for (int u = s * p.seg_runs;;) {   // run u of segment s, `left` runs of it to go; its first half is on its way (STAGED: both)
+      const bool last = --left == 0;
+      const int s_next = last ? s + KW : s, r_next = last ? s_next * p.seg_runs : u + 1;
+      begin();
+      if constexpr (!STAGED) load(One{}, u * GF_RUN + GF_RUN / 2);
+      multiply(Zero{}, One{});
+      if (s_next >= p.segments) {
+        if (u * GF_RUN + GF_RUN / 2 < p.k) multiply(One{}, Zero{});   // (the sum's last run may have one half)
+        end(last);
+        break;
+      }
+      if constexpr (STAGED) gf_wait_lds();   // what is read here has been read
+      load(Zero{}, r_next * GF_RUN);
+      multiply(One{}, One{});
+      if constexpr (STAGED) {
+        gf_wait_lds();
+        load(One{}, r_next * GF_RUN + GF_RUN / 2);
+      }
+      end(last);
+      if (last) left = min(p.seg_runs, runs - r_next);
+      s = s_next;
+      u = r_next;
+    }
   }
   __syncthreads();
 #pragma unroll
@@ -402,24 +525,37 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_f32_tile_kernel(GfArgs
     }
 }
 
+template <int NT, int KW, int READ, int FORM>
+static int gf_few_launch(const GfArgs& p, const GfAround& x, int grid, hipStream_t stream) {
+  // (sums: at most 16 KiB a tile; what a wave stages: 8)
+  const size_t lds = (size_t)p.segments * NT * 64 * sizeof(gf4) + (READ == GF_STAGED ? KW * 8192 : 0);
+  const auto kernel = gemm_f32_few_kernel<NT, KW, READ, FORM>;
+  if (lds > 65536 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, KW * 8192 + 16 * 1024) != hipSuccess)
+    return DLI_ERR_LAUNCH;
+  kernel<<<grid, 64 * KW, lds, stream>>>(p, x);
+  return dli_launch_status();
+}
+
 template <int NT, int KW>
 static int gf_few(const GfArgs& p, bool vec, hipStream_t stream) {
   const int grid = (p.n + 16 * NT - 1) / (16 * NT);
-  const size_t lds = (size_t)p.segments * NT * 64 * sizeof(gf4);   // at most 32 KiB
-  if (vec) gemm_f32_few_kernel<NT, KW, true><<<grid, 64 * KW, lds, stream>>>(p, GfAround{});
-  else gemm_f32_few_kernel<NT, KW, false><<<grid, 64 * KW, lds, stream>>>(p, GfAround{});
-  return dli_launch_status();
+  if constexpr (NT == 1)
+    if (vec && p.k % (GF_RUN / 2) == 0) return gf_few_launch<1, KW, GF_STAGED, GF_PLAIN>(p, GfAround{}, grid, stream);
+  return vec ? gf_few_launch<NT, KW, GF_WIDE, GF_PLAIN>(p, GfAround{}, grid, stream) : gf_few_launch<NT, KW, GF_WORDS, GF_PLAIN>(p, GfAround{}, grid, stream);
+}
+
+template <int KW, int FORM>
+static int gf_few_form(const GfArgs& p, const GfAround& x, int grid, hipStream_t stream) {
+  return p.k % (GF_RUN / 2) == 0 ? gf_few_launch<1, KW, GF_STAGED, FORM>(p, x, grid, stream) : gf_few_launch<1, KW, GF_WIDE, FORM>(p, x, grid, stream);
 }
 
 template <int FORM>
 static int gf_few_around(const GfArgs& p, const GfAround& x, int rule, int grid, hipStream_t stream) {
-  const size_t lds = (size_t)p.segments * 64 * sizeof(gf4);
   switch (rule) {
-    case 0: gemm_f32_few_kernel<1, 16, true, FORM><<<grid, 64 * 16, lds, stream>>>(p, x); break;
-    case 1: gemm_f32_few_kernel<1, 8, true, FORM><<<grid, 64 * 8, lds, stream>>>(p, x); break;
-    default: gemm_f32_few_kernel<1, 4, true, FORM><<<grid, 64 * 4, lds, stream>>>(p, x);
+    case 0: return gf_few_form<16, FORM>(p, x, grid, stream);
+    case 1: return gf_few_form<8, FORM>(p, x, grid, stream);
+    default: return gf_few_form<4, FORM>(p, x, grid, stream);
   }
-  return dli_launch_status();
 }
 
 template <int WM, int WN, int KG>

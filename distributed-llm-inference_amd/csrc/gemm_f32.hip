@@ -12,10 +12,10 @@
 // What bounds it: for few rows the stream of w, for many the matrix cores (157 TFLOP/s dense in 32-bit; a library product of
 // 8,192^3 reaches 152), in between the launch and the few tiles there are. Measured, us a product m x n x k, before (64 x 64
 // tiles of vector FMAs through LDS) and now:
-//   2 x 3072 x 576      37.6 ->   7.7     498 x 960 x 576     39.2 -> 12.5     512 x 3072 x 2048      152 ->   82
-//   2 x 576 x 1536      95.6 ->   7.6     498 x 3072 x 576    47.2 -> 32.6     512 x 16384 x 2048     491 ->  327
-//   2 x 49152 x 576     60.9 ->  24.6     498 x 576 x 1536     109 -> 22.6     2048 x 16384 x 2048   1827 -> 1280
-//   4 x 128256 x 2048    445 ->   177 (5.9 TB/s)                               2048 x 2048 x 8192     985 ->  655 (105 TFLOP/s)
+//   2 x 3072 x 576      37.6 ->   5.6     498 x 960 x 576     39.2 -> 12.5     512 x 3072 x 2048      152 ->   79
+//   2 x 576 x 1536      95.6 ->   5.7     498 x 3072 x 576    47.2 -> 28.5     512 x 16384 x 2048     491 ->  290
+//   2 x 49152 x 576     60.9 ->  21.6     498 x 576 x 1536     109 -> 22.6     2048 x 16384 x 2048   1827 -> 1128 (122 TFLOP/s)
+//   4 x 128256 x 2048    445 ->   177 (5.9 TB/s)                               2048 x 2048 x 8192     985 ->  606 (113 TFLOP/s)
 // (Reading both operands straight from memory also with many rows, a wave a tile: 44 us at 498 x 3072 x 576, 1,980 at 2048 x
 // 16384 x 2048: neighbouring lanes of a load lie in different rows. Choosing between a loaded value and zero beside the load
 // makes a wave wait for it at once: whole steps load without the choice, or choose when the value goes to LDS.)
@@ -525,6 +525,87 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void gemm_f32_tile_kernel(GfArgs
     }
 }
 
+// The same with k in whole GF_BK: loads write LDS without passing registers, STAGES - 1 blocks of k ahead, and a block has one
+// barrier. The kernel above waits for each block's loads; here most of the time is the matrix cores'.
+// us before and now: 1,500 x 3,072 x 576 73.5 61.7, 511 x 16,384 x 2,048 331 290, 2,048 x 16,384 x 2,048 1,290 1,128, 2,048 x 2,048 x
+// 8,192 662 606, and for tiles of 32 x 32 with four waves each 511 x 3,072 x 576 36.6 28.5, 1,000 x 960 x 2,560 77.5 59.7. (Three
+// stages are ahead of four where units have several tiles, 1,500 x 3,072 x 576 67.0 with four; four where they have one.)
+// The eight chunks of a row lie at chunk ^ gf_turn(row): a load's lanes in whole lines, a read's sixteen lanes in banks of their own.
+__device__ __forceinline__ int gf_turn(int row) { return (row ^ (row >> 3 & 1)) & 7; }
+
+template <int WM, int WN, int STAGES>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_f32_ahead_kernel(GfArgs p) {
+  constexpr int BM = 32 * WM, BN = 32 * WN, WAVES = WM * WN, STAGE = (BM + BN) * 8, LOADS = (BM + BN) / 8 / WAVES;
+  static_assert(LOADS * 8 * WAVES == BM + BN, "whole loads");
+  extern __shared__ gf4 gf_sums[];
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), i = lane % 16, g = lane / 16;
+  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN, wm = wave / WN * 32, wn = wave % WN * 32;
+  const float* src[LOADS];   // this lane's share of a block: 16 bytes of eight rows
+#pragma unroll
+  for (int u = 0; u < LOADS; ++u) {
+    const int row = 8 * (u * WAVES + wave) + lane / 8;
+    src[u] = (row < BM ? p.a + (int64_t)min(m0 + row, p.m - 1) * p.lda : p.w + (int64_t)min(n0 + row - BM, p.n - 1) * p.ldw) +
+             4 * (lane % 8 ^ gf_turn(row));
+  }
+  const auto load = [&](int block) {
+#pragma unroll
+    for (int u = 0; u < LOADS; ++u) gf_to_lds(src[u] + block * GF_BK, gf_sums + block % STAGES * STAGE + (u * WAVES + wave) * 64);
+  };
+  const int blocks = p.k / GF_BK, seg_blocks = p.seg_runs * (GF_RUN / GF_BK);
+#pragma unroll
+  for (int b = 0; b < STAGES - 1; ++b)
+    if (b < blocks) load(b);
+  gf4 total[2][2], seg[2][2], acc[2][2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y) total[x][y] = seg[x][y] = acc[x][y] = gf4{0.f, 0.f, 0.f, 0.f};
+  const int turn = gf_turn(i);
+  for (int b = 0; b < blocks; ++b) {
+    gf_wait_lds();   // what was read of the stage that is loaded next
+    if (b + STAGES - 2 < blocks) gf_wait<(STAGES - 2) * LOADS>();
+    else gf_wait<0>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (b + STAGES - 1 < blocks) load(b + STAGES - 1);
+    const gf4 *ca = gf_sums + b % STAGES * STAGE + (wm + i) * 8, *cw = gf_sums + b % STAGES * STAGE + (BM + wn + i) * 8;
+    gf4 fa[GF_BK / 16][2], fw[GF_BK / 16][2];
+#pragma unroll
+    for (int t = 0; t < GF_BK / 16; ++t)
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        fa[t][x] = ca[16 * x * 8 + (4 * t + g ^ turn)];
+        fw[t][x] = cw[16 * x * 8 + (4 * t + g ^ turn)];
+      }
+#pragma unroll
+    for (int t = 0; t < GF_BK / 16; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+          for (int y = 0; y < 2; ++y) acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[t][x][e], fw[t][y][e], acc[x][y], 0, 0, 0);
+    const bool last = b + 1 == blocks;
+    if (!last && (b + 1) % (GF_RUN / GF_BK) != 0) continue;
+    const bool seg_ends = last || (b + 1) % seg_blocks == 0;
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y) {
+        seg[x][y] += acc[x][y];
+        acc[x][y] = gf4{0.f, 0.f, 0.f, 0.f};
+        if (seg_ends) {
+          total[x][y] += seg[x][y];
+          seg[x][y] = gf4{0.f, 0.f, 0.f, 0.f};
+        }
+      }
+  }
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y) gf_store(p, total[x][y], m0 + wm + 16 * x, n0 + wn + 16 * y, i, g);
+}
+
 template <int NT, int KW, int READ, int FORM>
 static int gf_few_launch(const GfArgs& p, const GfAround& x, int grid, hipStream_t stream) {
   // (sums: at most 16 KiB a tile; what a wave stages: 8)
@@ -572,10 +653,23 @@ static int gf_tiles(const GfArgs& p, bool vec, hipStream_t stream) {
   return dli_launch_status();
 }
 
+template <int WM, int WN, int STAGES>
+static int gf_ahead(const GfArgs& p, hipStream_t stream) {
+  const dim3 grid((p.n + 32 * WN - 1) / (32 * WN), (p.m + 32 * WM - 1) / (32 * WM));
+  if (grid.y > 65535) return DLI_ERR_ARGUMENT;
+  constexpr size_t lds = (size_t)STAGES * 32 * (WM + WN) * GF_BK * sizeof(float);
+  const auto kernel = gemm_f32_ahead_kernel<WM, WN, STAGES>;
+  if (lds > 65536 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+    return DLI_ERR_LAUNCH;
+  kernel<<<grid, 64 * WM * WN, lds, stream>>>(p);
+  return dli_launch_status();
+}
+
 // Which kernel takes m rows, n columns and `segments` segments: 0 to 3 the few-row kernel, from sixteen waves a tile down to two for
 // two tiles, 4 to 7 the tile kernel, from eight waves a tile of 32 x 32 up to tiles of 128 x 64.
 // As many waves as the device has SIMDs, where the sum has segments enough: 498 x 3072 x 576 (1,536 tiles) takes 32.6 us
-// with four waves a tile and 44 with tiles of 64 x 64 for four waves; 2048 x 16384 x 2048 1,280 us in tiles of 128 x 64.
+// with four waves a tile and 44 with tiles of 64 x 64 for four waves (28.5 where those have loads ahead); 2048 x 16384 x 2048
+// 1,280 us in tiles of 128 x 64 (1,128).
 static int gf_rule(int m, int n, int segments) {
   const int64_t simds = 4 * dli_compute_units();
   if (m <= 16) {
@@ -588,6 +682,15 @@ static int gf_rule(int m, int n, int segments) {
   if (tiles * 4 <= simds && segments > 4) return 4;
   if (tiles <= 2 * simds && segments >= 2) return 5;
   return tiles < 8 * simds ? 6 : 7;
+}
+
+// Where the rule names four waves a tile of 32 x 32: whether tiles of 64 x 64 with loads ahead take less. They do where most units
+// have such a tile, and with sums of up to 1,024, whose segments four waves share badly, from half of them on: us with four waves a
+// tile and with loads ahead, k of 576, 960 and 2,048: 192 x 2,800 (132 tiles of 64 x 64) 21.0 17.6, 26.7 25.8, 48.0 48.6;
+// 500 x 1,536 (192) 23.1 17.6, 27.4 25.6, 46.7 48.1; 700 x 1,280 (220) 23.4 17.4, 31.5 25.4, 57.1 48.6; 100 x 3,072 (96) 13.7 16.9.
+static bool gf_few_waves_ahead(int m, int n, int k) {
+  const int64_t tiles = (int64_t)((n + 63) / 64) * ((m + 63) / 64), units = dli_compute_units();
+  return k <= 1024 ? 2 * tiles > units : 4 * tiles > 3 * units;
 }
 
 // The order of a sum over k: `segments` of `seg_runs` runs each.
@@ -613,15 +716,16 @@ extern "C" int dli_gemm_f32_nt(const float* a, int64_t lda, const float* w, int6
   gf_order(k, segments, seg_runs);
   const GfArgs p = {a, w, bias, residual, out, lda, ldw, ldr, ldo, m, n, k, segments, seg_runs};
   const bool vec = k % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (((uintptr_t)a | (uintptr_t)w) % 16) == 0;
+  const bool ahead = vec && k % GF_BK == 0;
   switch (gf_rule(m, n, segments)) {
     case 0: return gf_few<1, 16>(p, vec, stream);
     case 1: return gf_few<1, 8>(p, vec, stream);
     case 2: return gf_few<1, 4>(p, vec, stream);
     case 3: return gf_few<2, 2>(p, vec, stream);
     case 4: return gf_tiles<1, 1, 8>(p, vec, stream);
-    case 5: return gf_tiles<1, 1, 4>(p, vec, stream);
-    case 6: return gf_tiles<2, 2, 1>(p, vec, stream);
-    default: return gf_tiles<4, 2, 1>(p, vec, stream);
+    case 5: return ahead && gf_few_waves_ahead(m, n, k) ? gf_ahead<2, 2, 4>(p, stream) : gf_tiles<1, 1, 4>(p, vec, stream);
+    case 6: return ahead ? gf_ahead<2, 2, 3>(p, stream) : gf_tiles<2, 2, 1>(p, vec, stream);
+    default: return ahead ? gf_ahead<4, 2, 3>(p, stream) : gf_tiles<4, 2, 1>(p, vec, stream);
   }
 }
 

@@ -42,3 +42,22 @@ def test_norm_ahead_of_the_weights(m, inter, k):
     ops.silu_mul(both, want)
     ops.gemm_f32_swiglu(x, w, got[:m], norm_w, 1e-5, bias=bias)
     assert torch.equal(got[:m], want) and (got[m] == 7).all()
+
+
+# rows and columns: parts of tiles of 64 x 64 and 128 x 64, one and several a unit; k: fewer blocks than stages, as many, a segment of
+# several runs with a rest
+@pytest.mark.parametrize("m,n,k", [(17, 40000, 32), (130, 20000, 64), (300, 9001, 96), (65, 17000, 128), (511, 3072, 576), (193, 2800, 1024),
+                                   (960, 960, 2080), (1000, 1030, 4192), (700, 8200, 160)])
+def test_tiles_with_loads_ahead(m, n, k):
+    from dli_amd.kernels import ops
+
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, w = torch.randn(m, k, device="cuda", generator=g), torch.randn(n, k, device="cuda", generator=g)
+    bias, whole = torch.randn(n, device="cuda", generator=g), torch.full((m + 2, n), 7.0, device="cuda")
+    odd = torch.empty(n, k + 1, device="cuda")[:, :k].copy_(w)   # rows that begin at no whole load: tiles without
+    want = torch.empty(m, n, device="cuda")
+    ops.gemm_f32(a, w, whole[1:-1], bias=bias)
+    ops.gemm_f32(a, odd, want, bias=bias)
+    assert torch.equal(whole[1:-1], want) and (whole[0] == 7).all() and (whole[-1] == 7).all()
+    bound = (128 + k / 128 + 3) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T + bias.double().abs())
+    assert ((want.double() - a.double() @ w.double().T - bias.double()).abs() <= bound).all()

@@ -461,9 +461,10 @@ def gemm_f32_normed_ahead(rows: int, n: int, k: int) -> bool:
     """Whether :func:`gemm_f32_swiglu` (``n``: gates and ups) and :func:`gemm_f32_qkv_rope` are ahead of norm, product and what follows
     it one after the other. Each of their workgroups normalises all rows, so they lose with many columns and rows, and with
     rows of more than 1,024 values, whose sums are cut among more waves. A pass of eight steps of a model of twelve layers,
-    apart and fused, ms: width 512 with 8,192 columns 4.39 and 3.92 at 2 rows, 5.55 and 5.42 at 16; 1,024 with 8,192 5.21 and
-    4.66, 6.55 and 6.49; 1,024 with 16,384 7.25 and 7.15 at 2 rows, 7.61 and 7.65 at 4, 8.19 and 8.43 at 6; 1,088 with 5,888
-    5.37 and 5.68 at 2 rows; 2,048 with 16,384 8.36 and 9.20 at one row, 11.55 and 13.29 at 16."""
+    apart and fused, ms (before the weights of both passed through LDS): width 512 with 8,192 columns 4.39 and 3.92 at 2 rows, 5.55
+    and 5.42 at 16; 1,024 with 8,192 5.21 and 4.66, 6.55 and 6.49; 1,024 with 16,384 7.25 and 7.15 at 2 rows, 7.61 and 7.65 at 4,
+    8.19 and 8.43 at 6; 1,088 with 5,888 5.37 and 5.68 at 2 rows; 2,048 with 16,384 8.36 and 9.20 at one row, 11.55 and 13.29 at
+    16."""
     return k <= 1024 and (n <= 8192 or (n <= 16384 and rows <= 2))
 
 

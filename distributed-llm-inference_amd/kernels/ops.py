@@ -1066,7 +1066,7 @@ def prenorm_blocks(x: torch.Tensor, blocks, count: int, step) -> bool:
 
 def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, bias: Optional[torch.Tensor] = None) -> bool:
     """``out = x @ w.T (+ bias)`` for bfloat16 matrices with contiguous rows through the vendor
-    library, 32-bit accumulation, the bias added before the one rounding (``out`` float32: the
+    library (a result of about one tile of 128 x 128 a compute unit: ``csrc/tile_gemm.hip``), 32-bit accumulation, the bias added before the one rounding (``out`` float32: the
     sums as they are, unrounded). The library's choice
     of kernel is looked up once per shape. Returns False where the library has no kernel for the
     shape (nothing was computed then)."""

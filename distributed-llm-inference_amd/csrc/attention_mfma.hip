@@ -319,8 +319,8 @@ __global__ __launch_bounds__(NW * 64) void attention_decode_kernel(
         float4v s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int c = 0; c < KC; ++c) s = mfma32(g.k[u][c], qreg[c], s);
-        // (a sum of its own: a product of one depth that adds to the result of one of the other depth, right behind it, has read
-        // that result before it was there)
+        // (A sum of its own: a product of one depth that adds to the result of one of the other depth, right behind it, has read
+        // that result before it was there. The compiler puts no wait between the two, so none adds to the other's anywhere.)
         if (TAIL) {
           const float4v tail = mfma16(g.k_tail[u], qtail, float4v{0.f, 0.f, 0.f, 0.f});
           s = KC > 0 ? s + tail : tail;
@@ -637,6 +637,12 @@ __global__ __launch_bounds__(256) void attention_prefill_kernel(
 // both halves of the tile, so the half's page is chosen lane by lane.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
+__device__ __forceinline__ bf16x8 four_and_zeros(const bf16_t* from) {
+  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+  const bf16x4 v = *reinterpret_cast<const bf16x4*>(from);
+  return bf16x8{v[0], v[1], v[2], v[3], 0, 0, 0, 0};
+}
+
 __device__ __forceinline__ float4v mfma32(bf16x8 a, bf16x8 b, float4v c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
@@ -739,7 +745,10 @@ void attention_prefill_shared_kernel(
   const int* table = block_tables + (int64_t)e * table_stride;
 
   bf16x8 qreg[2][DK];
-  short4v qtail[2];   // dims 32 DK + 4 grp .. + 3 (ODD)
+  // ODD: dims 32 DK + 4 grp .. + 3 and four zeros, in a product as deep as the others. (One of depth 16 may not add to their sums, as
+  // in the decode kernel. us of 4,096 tokens, 16 heads on 4, so, with sums of its own, and with it added to theirs, which only
+  // the compiler's order kept apart: heads of 48 85.0, 88.0 and 83.2, of 112 118.7, 122.6 and 116.7.)
+  bf16x8 qtail[2];
   ColumnTile<DCH> st[2];
   // beside st[j].m: the value subtracted in the exponent (m, or 0 while m is -inf), and the raw
   // score above which m has to rise
@@ -756,12 +765,12 @@ void attention_prefill_shared_kernel(
     pos[j] = qi < q_len ? first_pos + qi : -1;
 #pragma unroll
     for (int c = 0; c < DK; ++c) qreg[j][c] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    qtail[j] = short4v{0, 0, 0, 0};
+    qtail[j] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
     if (qi < q_len) {
       const bf16_t* qp = q + (int64_t)(tok0 + qi) * q_stride + (int64_t)head * D + grp * 8;
 #pragma unroll
       for (int c = 0; c < DK; ++c) qreg[j][c] = *reinterpret_cast<const bf16x8*>(qp + c * 32);
-      if constexpr (ODD) qtail[j] = *reinterpret_cast<const short4v*>(qp - grp * 8 + 32 * DK + grp * 4);
+      if constexpr (ODD) qtail[j] = four_and_zeros(qp - grp * 8 + 32 * DK + grp * 4);
     }
   }
   // this wave's span, the same in all its lanes and said so: what is decided from it per tile
@@ -939,10 +948,10 @@ void attention_prefill_shared_kernel(
         kf0[c] = *reinterpret_cast<const bf16x8*>(ks + k_at[0][c]);
         kf1[c] = *reinterpret_cast<const bf16x8*>(ks + k_at[1][c]);
       }
-      short4v kt0 = short4v{0, 0, 0, 0}, kt1 = short4v{0, 0, 0, 0};
+      bf16x8 kt0, kt1;
       if constexpr (ODD) {
-        kt0 = *reinterpret_cast<const short4v*>(ks + k_tail_at[0]);
-        kt1 = *reinterpret_cast<const short4v*>(ks + k_tail_at[1]);
+        kt0 = four_and_zeros(ks + k_tail_at[0]);
+        kt1 = four_and_zeros(ks + k_tail_at[1]);
       }
 #pragma unroll
       for (int c = 0; c < DCH; ++c) {
@@ -965,8 +974,8 @@ void attention_prefill_shared_kernel(
       if constexpr (ODD) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          sa[j] = mfma16(kt0, qtail[j], sa[j]);
-          sb[j] = mfma16(kt1, qtail[j], sb[j]);
+          sa[j] = mfma32(kt0, qtail[j], sa[j]);
+          sb[j] = mfma32(kt1, qtail[j], sb[j]);
         }
       }
       float sv[2][8];

@@ -1,0 +1,75 @@
+"""The built kernels' instructions: what the matrix cores' results ask of the instructions behind them (no GPU).
+
+The cores' results are not interlocked. The compiler keeps their distances where it knows both instructions, and not all of them.
+"""
+
+from __future__ import annotations
+
+import re
+import shutil
+import subprocess
+from typing import NamedTuple, Optional
+
+import pytest
+
+OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+
+
+class Instruction(NamedTuple):
+    kernel: str
+    op: str
+    operands: list[str]
+
+
+def _registers(operand: str) -> Optional[tuple[int, int]]:
+    m = re.match(r"-?\|?v\[?(\d+)(?::(\d+))?\]?", operand)
+    return (int(m.group(1)), int(m.group(2) or m.group(1))) if m else None
+
+
+def _overlap(a: Optional[tuple[int, int]], b: Optional[tuple[int, int]]) -> bool:
+    return a is not None and b is not None and a[0] <= b[1] and b[0] <= a[1]
+
+
+@pytest.fixture(scope="module")
+def listing(tmp_path_factory):
+    """The instructions of the kernels that use the matrix cores, in their order."""
+    if shutil.which(OBJDUMP) is None:
+        pytest.skip("needs the ROCm toolchain's disassembler")
+    from dli_amd.kernels import build
+
+    folder = tmp_path_factory.mktemp("listing")
+    shutil.copy(build.find_library() or build.build(), folder / "lib.so")
+    subprocess.run([OBJDUMP, "--offloading", "lib.so"], cwd=folder, check=True, capture_output=True)
+    instructions = []
+    for code in sorted(folder.glob("lib.so.*amdgcn*")):
+        text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", code.name], cwd=folder, check=True, capture_output=True, text=True).stdout
+        for block in text.split("\n\n"):
+            if "v_mfma" not in block:
+                continue
+            kernel, *lines = block.strip().splitlines()[-block.strip().count("//") - 1:]
+            for line in lines:
+                op, _, rest = line.split("//")[0].strip().partition(" ")
+                instructions.append(Instruction(kernel, op, [o.split(" ")[0] for o in rest.strip().split(", ")]))
+    assert sum(i.op.startswith("v_mfma") for i in instructions) > 1000
+    return instructions
+
+
+def test_no_product_adds_to_one_of_another_depth(listing):
+    """A product that takes the sum of a product of another depth right behind it has read that sum before it was there, and the
+    compiler inserts no wait: nothing may depend on what happens to stand between the two."""
+    found, sums, kernel = set(), {}, ""
+    for i in listing:
+        if i.kernel != kernel:
+            sums, kernel = {}, i.kernel
+        if not i.op.startswith("v_mfma"):
+            written = _registers(i.operands[0]) if i.op.startswith(("v_", "ds_read", "buffer_load", "global_load")) else None
+            if written is not None:
+                sums = {r: op for r, op in sums.items() if not _overlap(r, written)}
+            continue
+        taken, written = _registers(i.operands[3]), _registers(i.operands[0])
+        if taken is not None and sums.get(taken, i.op) != i.op:
+            found.add((i.kernel, i.op, sums[taken]))
+        sums = {r: op for r, op in sums.items() if not _overlap(r, written)}
+        if written is not None:
+            sums[written] = i.op
+    assert not found

@@ -43,20 +43,12 @@ __device__ __forceinline__ short bf16_bits(float x) {
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // Maximum as one instruction. fmaxf() asks for a quieted NaN, which costs a second instruction per
-// operand that the compiler cannot prove canonical (every matrix-core result); scores are never
-// NaN here (masked ones are -inf), and the instruction itself orders -inf and finite values as
-// fmaxf does. The prefill kernel is bound by the vector unit's instruction count: 65 -> 59 us a
-// layer at 2,048 tokens of the 1B sizes.
-__device__ __forceinline__ float max2(float a, float b) {
-  float r;
-  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
-}
-__device__ __forceinline__ float max3(float a, float b, float c) {
-  float r;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
+// operand that the compiler cannot prove canonical (every matrix-core result). The prefill kernel is
+// bound by the vector unit's instruction count: 65 -> 59 us a layer at 2,048 tokens of the 1B sizes.
+// (Not in inline asm: the compiler does not know what that reads, and keeps no distance between it
+// and the product whose result it takes.)
+__device__ __forceinline__ float max2(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+__device__ __forceinline__ float max3(float a, float b, float c) { return max2(max2(a, b), c); }
 
 // Reductions over the four lanes l, l^16, l^32, l^48 (the lane groups that share a column) with
 // the gfx950 lane-swap instructions: after v_permlane32_swap of two copies of v, one copy holds

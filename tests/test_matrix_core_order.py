@@ -17,6 +17,7 @@ OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
 
 class Instruction(NamedTuple):
     kernel: str
+    address: int
     op: str
     operands: list[str]
 
@@ -46,10 +47,13 @@ def listing(tmp_path_factory):
         for block in text.split("\n\n"):
             if "v_mfma" not in block:
                 continue
-            kernel, *lines = block.strip().splitlines()[-block.strip().count("//") - 1:]
-            for line in lines:
-                op, _, rest = line.split("//")[0].strip().partition(" ")
-                instructions.append(Instruction(kernel, op, [o.split(" ")[0] for o in rest.strip().split(", ")]))
+            kernel = re.search(r"<(.*)>:", block).group(1) + code.name
+            for line in block.splitlines():
+                instruction, _, place = line.partition("//")
+                op, _, rest = instruction.strip().partition(" ")
+                if place:
+                    operands = [o.split(" ")[0] for o in rest.strip().split(", ")]
+                    instructions.append(Instruction(kernel, int(place.split(":")[0], 16), op, operands))
     assert sum(i.op.startswith("v_mfma") for i in instructions) > 1000
     return instructions
 
@@ -72,4 +76,37 @@ def test_no_product_adds_to_one_of_another_depth(listing):
         sums = {r: op for r, op in sums.items() if not _overlap(r, written)}
         if written is not None:
             sums[written] = i.op
+    assert not found
+
+
+def test_vector_instructions_wait_for_a_products_result(listing):
+    """A vector instruction that reads the result of a 16x16x16 or 16x16x32 product stands at least seven wait states (an
+    instruction each, s_nop n another n) behind it on every way there, branches taken included."""
+    apart = 7
+    at = {(i.kernel, i.address): n for n, i in enumerate(listing)}
+    found = set()
+    for n, product in enumerate(listing):
+        if not product.op.startswith(("v_mfma_f32_16x16x16_bf16", "v_mfma_f32_16x16x32_bf16")):
+            continue
+        result, ways, seen = _registers(product.operands[0]), [(n + 1, 0)], {}
+        while ways:
+            j, states = ways.pop()
+            if j >= len(listing) or states >= apart or seen.get(j, apart) <= states:
+                continue
+            seen[j] = states
+            i = listing[j]
+            if i.op.startswith("v_mfma"):
+                if _overlap(_registers(i.operands[0]), result):
+                    continue   # (another product's result from here on)
+            elif i.op.startswith("v_") and any(_overlap(_registers(o), result) for o in i.operands[1:]):
+                found.add((i.kernel, i.op, states))
+                continue
+            if i.op in ("s_endpgm", "s_setpc_b64"):
+                continue
+            if i.op.startswith("s_cbranch") or i.op == "s_branch":
+                words = int(i.operands[0])
+                ways.append((at[i.kernel, i.address + 4 + 4 * (words - 65536 if words > 32767 else words)], states + 1))
+                if i.op == "s_branch":
+                    continue
+            ways.append((j + 1, states + 1 + (int(i.operands[0]) if i.op == "s_nop" else 0)))
     assert not found

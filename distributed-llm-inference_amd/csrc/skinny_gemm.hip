@@ -15,7 +15,7 @@
 // so that the 16 features x 128 k of one tile and block are 4 KB of consecutive memory in the
 // order in which the lanes take them (lane = 16*g + c) and every load of a wave is 1 KB of
 // consecutive bytes. Needs K % 128 == 0 and whole tiles (N % 16 == 0, gate and up parts included); EPI_QKV behind a
-// norm and MERGED also take K % 32 == 0, the last block filled up with zeros.
+// norm also takes K % 32 == 0, the last block filled up with zeros.
 //
 // Fused in (template switches):
 //   NORM     xhat = cast(norm_w[k] * cast(x[m][k] * rs[m])), rs[m] = rsqrt(sum_k x^2 / K + eps),
@@ -40,7 +40,8 @@
 //            arithmetic in the same order as attention_merge_kernel, so that the o projection of a
 //            step of one to four rows needs no merge kernel before it. Each wave merges the run of
 //            k that it multiplies (all loads of a lane in flight at once) and hands it to its
-//            lanes through LDS. TILED, EPI_RESIDUAL, at most 16 runs.
+//            lanes through LDS. EPI_RESIDUAL, at most 16 runs. TILED, or row by row where K is no whole blocks of 128, as
+//            the product of several rows reads those: a row alone in its step is summed as among others.
 #include "common.h"
 #include "merge_splits.h"
 
@@ -128,13 +129,13 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
     int up_offset, QkvRope qr, MergedIn mi, GluForm glu) {
   constexpr bool MERGED = RUNS != 0;
   static_assert(EPI != EPI_QKV || (TILED && MT == 1), "the q/k/v epilogue reads tiled weights, at most 16 rows");
-  static_assert(!MERGED || (TILED && MT == 1 && NS == 1 && !NORM), "merged activations: tiled weights, one row tile");
+  static_assert(!MERGED || (MT == 1 && NS == 1 && NT == 1 && !NORM), "merged activations: one tile of rows and of features");
   static_assert(!AHEAD || (MT == 1 && !NORM && !MERGED), "one row tile, no sums of squares to wait for");
   static_assert(KS * NS * 64 >= 256, "a thread for each output of a tile");
   // MERGED: each wave's run of k for up to MERGE_ROWS rows
   __shared__ __align__(16) bf16_t xs[MERGED ? KS : 1][MERGED ? MERGE_ROWS : 1][MERGED ? MERGE_RANGE : 8];
   constexpr int NA = EPI == EPI_SWIGLU ? 2 : 1;  // weight row sets per tile (gate and up)
-  constexpr bool PADDED = EPI == EPI_QKV || MERGED;  // the weights' last block of 128 k may be filled up with zeros
+  constexpr bool PADDED = EPI == EPI_QKV;        // the weights' last block of 128 k may be filled up with zeros
   // What follows the last product is a chain that nothing hides, so it is kept short. With one row
   // tile and one group of waves (SHORT) all waves leave their parts in LDS and thread t makes
   // output t of each tile: element t % 4 of lane t / 4 of the product's result, that is row
@@ -279,6 +280,11 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
   };
   int blocks = (s_end - s) / 4;
   Block b0, b1;
+  // single steps behind the last block (row by row): lane group g reads k in [8g, 8g + 8)
+  auto w_single_at = [&](const bf16_t* base, int s) __attribute__((always_inline)) {
+    return reinterpret_cast<const bf16x8*>(base - grp * 32 + s * 32 + grp * 8);
+  };
+  bf16x8 w_single[MERGED && !TILED ? 3 : 1];   // MERGED: asked for ahead of the merge, like the blocks
   if constexpr (NORM) {
     // rs[m] from the parts of sum x^2 that the producer of x left. The parts are dealt out to
     // all lane groups of all waves (group q of W*4 takes the parts q, q + 4W, ...), eight loads
@@ -345,13 +351,17 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
     const int D = mi.head_dim, S = mi.splits;
     MergeQuad<MERGED ? RUNS : 2> parts;
     auto ask = [&](int item) __attribute__((always_inline)) {
-      const int row = item / quads, k = min(kb0 + (item - row * quads) * 4, K - 4), head = k / D;   // (past K: zeros, below)
+      const int row = item / quads, k = kb0 + (item - row * quads) * 4, head = k / D;
       parts.ask(mi.part_o, mi.part_ml, ((int64_t)row * mi.heads + head) * S, S, D, k - head * D);
     };
     if (items > 0) ask(min(lane, items - 1));
     __builtin_amdgcn_sched_barrier(0);
     if (blocks > 0) fetch_weights(b0, s);
     if (blocks > 1) fetch_weights(b1, s + 4);
+    if constexpr (!TILED) {
+#pragma unroll
+      for (int u = 0; u < 3; ++u) w_single[u] = *w_single_at(wrow[0][0], min(s + 4 * blocks + u, steps - 1));
+    }
     __builtin_amdgcn_sched_barrier(0);
     for (int item0 = 0; item0 < items; item0 += 64) {
       const int item = item0 + lane;
@@ -361,7 +371,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
         const int row = item / quads;
         bf16_t* dst = &xs[ks][row][(item - row * quads) * 4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) dst[i] = (bf16_t)(kb0 + (item - row * quads) * 4 < K ? merged[i] : 0.f);
+        for (int i = 0; i < 4; ++i) dst[i] = (bf16_t)merged[i];
       }
     }
     __syncthreads();
@@ -452,7 +462,13 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
     }
     s = s_begin + (s_end - s_begin) / 4 * 4;
   }
-  for (; !TILED && s < s_end; ++s) {  // single steps: lane group g reads k in [8g, 8g + 8)
+  if constexpr (MERGED && !TILED) {
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+      if (s + u < s_end) acc[0][0][0] = mfma32(w_single[u], fetch_x<false>(xrow[0], nullptr, (s + u) * 32 + grp * 8).v, acc[0][0][0]);
+    s = s_end;
+  }
+  for (; !TILED && s < s_end; ++s) {  // single steps
     const int kb = s * 32 + grp * 8;
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
@@ -461,7 +477,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
       for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int a = 0; a < NA; ++a)
-          acc[j][a][t] = mfma32(*reinterpret_cast<const bf16x8*>(wrow[j][a] - grp * 32 + kb), bf, acc[j][a][t]);
+          acc[j][a][t] = mfma32(*w_single_at(wrow[j][a], s), bf, acc[j][a][t]);
     }
   }
 
@@ -1129,34 +1145,41 @@ extern "C" int dli_skinny_gemm_qkv_rope(const void* x, int64_t ldx, const float*
 
 // The o projection of a decode step of at most MERGE_ROWS rows, fed with the split-key partial
 // results of the attention instead of its merged output (MERGED above): stream += merge(...) @ w^T
-// (+ bias), and the parts of the rows' sums of squares. w_tiled [N, K] in tile order with
-// K = heads * head_dim, filled up with zeros to whole blocks of 128; splits 2..MERGE_SPLITS; shape 0 or 1 (4 or 8 waves split k).
+// (+ bias), and the parts of the rows' sums of squares. w [N, K], K = heads * head_dim, in tile order where K is whole blocks of
+// 128, else row by row; splits 2..MERGE_SPLITS; shape 0 or 1 (4 or 8 waves split k).
 extern "C" int dli_skinny_gemm_merged(const float* part_o, const float* part_ml, int splits, int heads,
-                                      int head_dim, const void* w_tiled, const void* bias, void* stream_buf,
+                                      int head_dim, const void* w, const void* bias, void* stream_buf,
                                       int64_t lds_, float* ssq_out, int M, int N, int shape, hipStream_t stream) {
   if (M <= 0 || N <= 0) return DLI_OK;
   const int64_t K64 = (int64_t)heads * head_dim;
   if (M > MERGE_ROWS || splits < 2 || splits > MERGE_SPLITS || heads <= 0 || head_dim <= 0 || head_dim % 4 != 0 ||
       K64 % 32 != 0 || K64 > (1 << 20) || N % 16 != 0 || (shape != 0 && shape != 1) || part_o == nullptr ||
-      part_ml == nullptr || w_tiled == nullptr || stream_buf == nullptr || ssq_out == nullptr)
+      part_ml == nullptr || w == nullptr || stream_buf == nullptr || ssq_out == nullptr)
     return DLI_ERR_ARGUMENT;
   const int K = (int)K64, ks = shape == 0 ? 4 : 8;
-  if ((((K + 127) / 128 + ks - 1) / ks) * 128 > MERGE_RANGE) return DLI_ERR_ARGUMENT;
+  const bool tiled = K % 128 == 0;
+  if ((tiled ? ((K / 128 + ks - 1) / ks) * 128 : ((K / 32 + ks - 1) / ks) * 32) > MERGE_RANGE) return DLI_ERR_ARGUMENT;
   const MergedIn mi{part_o, part_ml, splits, heads, head_dim};
   const int groups = N / 16;
-#define MERGED_LAUNCH(KS, RUNS)                                                                    \
-  skinny_gemm_kernel<KS, 1, 1, 1, EPI_RESIDUAL, false, true, false, RUNS><<<groups, KS * 64, 0, stream>>>( \
-      nullptr, 0, nullptr, 0, nullptr, 0.f, (const bf16_t*)w_tiled, (const bf16_t*)bias, nullptr, 0, \
+#define MERGED_LAUNCH(KS, TILED, RUNS)                                                             \
+  skinny_gemm_kernel<KS, 1, 1, 1, EPI_RESIDUAL, false, TILED, false, RUNS><<<groups, KS * 64, 0, stream>>>( \
+      nullptr, 0, nullptr, 0, nullptr, 0.f, (const bf16_t*)w, (const bf16_t*)bias, nullptr, 0,     \
       (bf16_t*)stream_buf, lds_, ssq_out, M, N, K, 0, QkvRope{}, mi, GluForm{})
-#define MERGED_RUNS(KS)                       \
-  if (splits <= 2) MERGED_LAUNCH(KS, 2);      \
-  else if (splits <= 4) MERGED_LAUNCH(KS, 4); \
-  else if (splits <= 8) MERGED_LAUNCH(KS, 8); \
-  else MERGED_LAUNCH(KS, 16)
-  if (shape == 0) {
-    MERGED_RUNS(4);
+#define MERGED_RUNS(KS, TILED)                       \
+  if (splits <= 2) MERGED_LAUNCH(KS, TILED, 2);      \
+  else if (splits <= 4) MERGED_LAUNCH(KS, TILED, 4); \
+  else if (splits <= 8) MERGED_LAUNCH(KS, TILED, 8); \
+  else MERGED_LAUNCH(KS, TILED, 16)
+  if (tiled) {
+    if (shape == 0) {
+      MERGED_RUNS(4, true);
+    } else {
+      MERGED_RUNS(8, true);
+    }
+  } else if (shape == 0) {
+    MERGED_RUNS(4, false);
   } else {
-    MERGED_RUNS(8);
+    MERGED_RUNS(8, false);
   }
 #undef MERGED_RUNS
 #undef MERGED_LAUNCH

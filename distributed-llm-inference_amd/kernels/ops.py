@@ -795,7 +795,10 @@ MERGED_ROWS, MERGED_SPLITS, _MERGED_RANGE = 4, 16, 512  # csrc/skinny_gemm.hip: 
 def skinny_gemm_merged_supports(rows: int, n: int, heads: int, head_dim: int, splits: int,
                                 device: torch.device) -> bool:
     """Whether :func:`skinny_gemm_merged` takes this o projection: few rows, few runs of keys, a
-    product that the 16x16-tile kernel runs with k split over the waves of a workgroup."""
+    product that the 16x16-tile kernel runs with k split over the waves of a workgroup. Up to 512, k in whole blocks
+    of 128 only: below, the launches around it hide a merge kernel about as well (passes of eight steps, 24 layers, ms, without and
+    with it: width 192, 450 keys 3.53 and 3.58, 4,000 3.86 and 4.15; 320, 3.90 and 3.92, 4.22 and 4.39; 448, 7.39 and 7.50, 8.80 and
+    8.76; 480, 3.38 and 3.46, 4.12 and 3.96)."""
     k = heads * head_dim
     if not (0 < rows <= MERGED_ROWS and 2 <= splits <= MERGED_SPLITS and head_dim % 4 == 0 and n % 16 == 0
             and (k % 128 == 0 or (k % 32 == 0 and k > 512))):
@@ -805,21 +808,24 @@ def skinny_gemm_merged_supports(rows: int, n: int, heads: int, head_dim: int, sp
 
 def _merged_shape(rows: int, n: int, k: int, device: torch.device) -> Optional[int]:
     """The workgroup shape (0: four k-waves, 1: eight) with which the merging o projection runs:
-    that of the plain product with the residual sum, so that both add in the same order (where k is whole blocks of 128; else that
-    one reads the weights row by row), or None if that one runs on another kernel or a wave's run of k does not fit the merge's buffer."""
+    that of the plain product with the residual sum, so that both add in the same order, or None
+    if that one runs on another kernel or a wave's run of k does not fit the merge's buffer."""
     kernel, shape, _ = skinny_gemm_plan(rows, n, k, SKINNY_RESIDUAL, device, tiled=k % 128 == 0)
     if kernel != "tiles16" or shape not in (0, 1):
         return None
-    return shape if -(-(padded_k(k) // 128) // (4 if shape == 0 else 8)) * 128 <= _MERGED_RANGE else None
+    least = 128 if k % 128 == 0 else 32   # waves share out whole blocks of tiles, or steps of rows
+    return shape if -(-(k // least) // (4 if shape == 0 else 8)) * least <= _MERGED_RANGE else None
 
 
 def skinny_gemm_merged(part_o: torch.Tensor, part_ml: torch.Tensor, splits: int, heads: int, head_dim: int,
-                       w_tiled: torch.Tensor, stream: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                       w: torch.Tensor, stream: torch.Tensor, bias: Optional[torch.Tensor] = None,
                        ssq_out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``stream += merge(part_o, part_ml) @ w.T (+ bias)`` for at most four rows: the o projection
     of a decode step fed with the partial results that :func:`attention_decode` leaves with
     ``merge=False`` (``part_o [rows, heads, splits, head_dim]``, ``part_ml [rows, heads, splits, 2]``),
-    merged inside the product's kernel with the arithmetic of the merge kernel. Returns the parts
+    merged inside the product's kernel with the arithmetic of the merge kernel. ``w``: in tile order
+    (:func:`tile_weights`) where ``heads * head_dim`` is whole blocks of 128, else ``[n, heads * head_dim]`` as it is, as
+    :func:`skinny_gemm` reads them: the same bits as the merge kernel and that product. Returns the parts
     of the rows' sums of squares like the residual epilogue of :func:`skinny_gemm`."""
     _rows(stream, "stream", torch.bfloat16)
     m, n = stream.shape
@@ -832,8 +838,9 @@ def skinny_gemm_merged(part_o: torch.Tensor, part_ml: torch.Tensor, splits: int,
     _require(part_o.numel() >= m * heads * splits * head_dim and part_ml.numel() >= m * heads * splits * 2,
              "partial-result buffers are too small")
     _require(part_o.data_ptr() % 16 == 0 and part_ml.data_ptr() % 8 == 0, "partial results must be 16-byte aligned")
-    _dense(w_tiled, "w_tiled", torch.bfloat16, 1)
-    _require(w_tiled.numel() == n * padded_k(k) and w_tiled.data_ptr() % 16 == 0, "w_tiled must hold [n, heads*head_dim] in tile order")
+    _dense(w, "w", torch.bfloat16, 1 if k % 128 == 0 else 2)
+    _require(w.numel() == n * k and (k % 128 == 0 or w.shape[1] == k) and w.data_ptr() % 16 == 0,
+             "w must hold [n, heads*head_dim], in tile order where that is whole blocks of 128")
     if bias is not None:
         _dense(bias, "bias", torch.bfloat16, 1)
         _require(bias.shape[0] == n, "bias length differs from rows of w")
@@ -845,7 +852,7 @@ def skinny_gemm_merged(part_o: torch.Tensor, part_ml: torch.Tensor, splits: int,
     _require(ssq_out.shape == (n_parts, m), f"ssq_out must be [{n_parts}, rows] for this product")
     _require(stream.data_ptr() % 8 == 0, "stream must be 8-byte aligned")
     _check(library().dli_skinny_gemm_merged(
-        _ptr(part_o), _ptr(part_ml), int(splits), int(heads), int(head_dim), _ptr(w_tiled), _ptr(bias), _ptr(stream),
+        _ptr(part_o), _ptr(part_ml), int(splits), int(heads), int(head_dim), _ptr(w), _ptr(bias), _ptr(stream),
         stream.stride(0), _ptr(ssq_out), m, n, shape, _stream()), "skinny_gemm_merged")
     return ssq_out
 

@@ -261,8 +261,8 @@ class GQAttention(Mixer):
                 planned=ctx.decode_plans.get(id(self)))
             if left is not None:
                 splits, part_o, part_ml = left
-                stream.wrote(ops.skinny_gemm_merged(part_o, part_ml, splits, nh, d, self.w_o_tiled, stream.x,
-                                                    bias=self.b_o))
+                w_o = self.w_o_tiled if nh * d % 128 == 0 else self.w_o
+                stream.wrote(ops.skinny_gemm_merged(part_o, part_ml, splits, nh, d, w_o, stream.x, bias=self.b_o))
                 return
         out = self.rt.empty(n, nh * d)
         paged_attention(qkv[:, :nh * d], cache.k_pages, cache.v_pages, out, ctx, grp, nh, self.scale, self.window,

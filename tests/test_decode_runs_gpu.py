@@ -63,18 +63,20 @@ def test_pairs_of_tiles_at_their_edges(ops, keys, qh, kvh, d, bs, splits, window
     assert torch.equal(both[:1], got) and not both[1].any()
 
 
-@pytest.mark.parametrize("qh,kvh,d,n", [(9, 3, 64, 576), (15, 5, 64, 960), (17, 1, 32, 272)])
+# k of 18, 30, 17 and 31 steps of 32: waves of single steps only, of a block and none to three steps behind it
+@pytest.mark.parametrize("qh,kvh,d,n", [(9, 3, 64, 576), (15, 5, 64, 960), (17, 1, 32, 272), (31, 1, 32, 64)])
 @pytest.mark.parametrize("splits", [2, 3, 8, 9, 16])
-def test_merging_o_projection_of_odd_widths(ops, qh, kvh, d, n, splits):
-    """Widths that end inside a block of 128: the weights' copy is filled up with zeros, whatever the rows hold there. Against the
-    products of the merged attention in 64 bits: 32-bit sums of bfloat16 products, the sum rounded once, then the stream's (2^-8)."""
-    rows, bs, k = 2, 16, qh * d
+@pytest.mark.parametrize("rows", [1, 2, 4])
+def test_merging_o_projection_of_odd_widths(ops, qh, kvh, d, n, splits, rows):
+    """Widths that end inside a block of 128: the bits of the merge kernel and the product that several rows take, and so a row
+    alone in its step those of one among others."""
+    bs, k = 16, qh * d
     assert k % 128 and ops.skinny_gemm_merged_supports(rows, n, qh, d, splits, torch.device("cuda", 0))
     gen = torch.Generator().manual_seed(n + splits)
-    lens = [700, 33]
+    lens = [700, 33, 1, 260][:rows]
     width = -(-lens[0] // bs)
-    kp, vp = _pool((2 * width, kvh, bs, d), gen, 0), _pool((2 * width, kvh, d, bs), gen, 0)
-    tables = torch.randperm(2 * width, generator=gen).view(2, width).int().cuda()
+    kp, vp = _pool((4 * width, kvh, bs, d), gen, 0), _pool((4 * width, kvh, d, bs), gen, 0)
+    tables = torch.randperm(4 * width, generator=gen).view(4, width)[:rows].int().cuda()
     q = torch.randn(rows, k, generator=gen).bfloat16().cuda()
     kv_len = torch.tensor(lens, dtype=torch.int32, device="cuda")
     w = (torch.randn(n, k, generator=gen) / math.sqrt(k)).bfloat16().cuda()
@@ -83,8 +85,11 @@ def test_merging_o_projection_of_odd_widths(ops, qh, kvh, d, n, splits):
     ml = torch.full((rows * qh * splits * 2,), float("nan"), device="cuda")
     out = torch.empty_like(q)
     ops.attention_decode(q, kp, vp, out, kv_len, tables, qh, 0.125, 0, splits, po, ml)
-    got = base.clone()
-    ssq = ops.skinny_gemm_merged(po, ml, splits, qh, d, ops.tile_weights(w, whole_blocks=False), got, bias=bias)
-    want = base.cpu().double() + out.cpu().double() @ w.cpu().double().T + bias.cpu().double()
-    assert ((got.cpu().double() - want).abs() <= 2.0 ** -8 * (want.abs() + base.cpu().double().abs() + 4.0)).all()
-    assert torch.allclose(ssq.sum(0).cpu(), (got.float() ** 2).sum(1).cpu(), rtol=1e-5)
+    got, want = base.clone(), base.clone()
+    ssq = ops.skinny_gemm_merged(po, ml, splits, qh, d, w, got, bias=bias)
+    ssq_want = ops.skinny_gemm(out, w, epilogue=ops.SKINNY_RESIDUAL, stream=want, bias=bias)
+    assert torch.equal(got, want) and torch.equal(ssq, ssq_want)
+    # product and bias rounded once, then their sum with the stream: half of the last of eight bits each, and the 32-bit sums
+    y, old = out.cpu().double() @ w.cpu().double().T + bias.cpu().double(), base.cpu().double()
+    sums = k * 2.0 ** -23 * (out.cpu().double().abs() @ w.cpu().double().abs().T + bias.cpu().double().abs())
+    assert ((got.cpu().double() - old - y).abs() <= 2.0 ** -8 * (y.abs() + (y + old).abs()) * 1.01 + sums).all()

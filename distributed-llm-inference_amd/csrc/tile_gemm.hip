@@ -188,9 +188,18 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_kernel(TileArgs p) {
 //   k 2,048: 984 x 2,304 23.1 20.4, 2,008 x 1,152 (144) 21.0 19.8, 1,500 x 2,048 (192) 21.8 20.8, 2,048 x 2,048 24.2 21.6
 //   k 3,072: 984 x 2,304 28.3 29.5, 984 x 3,072 (192) 30.7 29.9, 2,008 x 1,536 (192) 27.4 28.5, 1,100 x 3,072 (216) 32.3 30.2
 //   k 8,192: 984 x 2,304 61.9 65.4, 1,464 x 2,048 (192) 58.3 64.8, 1,100 x 3,072 (216) 71.8 68.2, 2,048 x 2,048 74.3 67.2
+// Where the last tile of rows is half empty or emptier, tiles of 64 rows may fill a single round as well, and the library has those.
+// It is ahead with them from a k of 2,048 on:
+//   k 1,024: 136 x 8,320 13.1 11.8, 260 x 6,144 13.0 11.8   k 1,984: 136 x 8,320 21.2 18.9, 288 x 6,400 21.3 19.1, 530 x 3,456 20.2 18.6
+//   k 2,048: 136 x 8,320 16.9 19.8, 288 x 6,400 17.4 20.1, 530 x 3,456 16.5 19.3; 352 x 6,144 (288 tiles of 64 rows) 24.5 21.0,
+//     129 x 16,384 (384) 28.4 25.5, 256 x 16,384 (512) 29.0 24.8   k 3,072: 129 x 16,384 31.6 31.1, 256 x 16,384 40.9 35.9
+// and, where up to 64 rows leave half of every tile empty, from above 1,024 on:
+//   k 1,024: 17 x 17,000 14.0 12.1, 64 x 25,000 15.6 14.0   k 1,280: 13.6 14.8, 17.5 17.6   k 1,792: 17.0 18.3, 21.5 21.2
+//   k 2,560: 20 x 27,000 28.8 30.9, 64 x 32,000 34.3 35.9   k 4,096: 50.2 50.4, 62.9 63.8
 extern "C" int dli_tile_gemm_takes(int64_t rows, int64_t feats, int64_t k, int units) {
   if (rows <= 0 || feats <= 0 || feats % 8 != 0 || k % 64 != 0 || k < 64 * STAGES) return 0;
-  const int64_t tiles = ((rows + TILE - 1) / TILE) * ((feats + TILE - 1) / TILE);
+  const int64_t across = (feats + TILE - 1) / TILE, tiles = (rows + TILE - 1) / TILE * across;
+  if ((rows + 63) / 64 * across <= units && (rows <= 64 ? k > 1024 : k >= 2048)) return 0;
   return (k <= 2048 ? 2 * tiles > units : 5 * tiles > 4 * units) && tiles <= units;
 }
 

@@ -161,7 +161,7 @@ class GQAttention(Mixer):
         units = ops.compute_units(self.rt.device)
         if requests <= MERGE_IN_PRODUCT_ROWS and self.w_o_tiled is not None:
             runs = runs_for_the_product(self.num_heads, self.num_kv_heads, max_keys, units)
-            if runs == 1 or ops.skinny_gemm_merged_supports(requests, self.hidden_size, self.num_heads, self.head_dim, runs, self.rt.device):
+            if runs == 1 or runs and ops.skinny_gemm_merged_supports(requests, self.hidden_size, self.num_heads, self.head_dim, runs, self.rt.device):
                 return runs
         return planned_splits(requests, self.num_heads, self.num_kv_heads, self.head_dim, max_keys, units)
 

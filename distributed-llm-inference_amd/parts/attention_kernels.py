@@ -44,12 +44,15 @@ def choose_splits(requests: int, kv_head_tiles: int, max_keys: int, units: int =
 def one_run_keys(requests: int, q_heads: int, kv_heads: int, head_dim: int, units: int = 256) -> int:
     """Up to how many keys one run serves a recorded step better than two, where every workgroup has a compute unit to itself. It
     then has eight waves, which walk up to 512 keys in one round of what they have on their way; what follows costs more the
-    wider the heads are, and the second run's merge is cheaper for a single request, whose o projection makes it. Passes of 8 steps,
-    two runs and one, ms: 135M sizes, 1 request, 520 keys 5.91 and 5.60, 568 5.90 and 5.87, 600 5.92 and 5.94; 1B sizes, 8 requests,
-    568 7.04 and 6.96, 600 7.01 and 7.04. Heads of 128: 24 on 8, 8 requests, 520 5.53 and 5.43, 552 5.53 and 5.56; 16 on 2, 8
-    requests, 552 4.60 and 4.48, 1 request, 536 3.70 and 3.75. Heads of 96: 16 on 8, 8 requests, 552 3.98 and 3.97, 568 3.98 and
-    4.02, 1 request, 536 3.31 and 3.35. Groups whose states do not fit (heads of 128, 16 on one) have four waves: 1 request, 520
-    3.53 and 3.63; 2 requests, 584 4.28 and 3.95; 16 requests, 584 5.54 and 5.24."""
+    wider the heads are. Passes of 8 steps, two runs and one, ms: 1B sizes, 8 requests, 520 keys 6.52 and 6.48, 568 6.52 and 6.51, 632
+    6.54 and 6.58; 135M sizes, 16 requests, 520 6.51 and 6.46, 568 6.55 and 6.55, 600 6.59 and 6.63. Heads of 128: 24 on 8, 4
+    requests, 552 14.1 and 14.1; 16 on 2, 8 requests, 536 4.39 and 4.36, 552 4.42 and 4.42. Heads of 96: 16 on 8, 8 requests, 536 3.48
+    and 3.49, 552 3.49 and 3.52. Groups whose states do not fit (heads of 128, 16 on one) have four waves: 2 requests, 568 4.21 and
+    4.02; 16 requests, 552 5.17 and 4.95.
+
+    One request asks here only where its o projection does not merge the runs (:func:`runs_for_the_product` answers else), with a
+    merge in the attention's launch: 135M sizes, 520 5.24 and 5.18, 568 5.23 and 5.24; 24 on 8 of 128, 520 13.1 and 13.7; 16 on
+    2, 536 3.81 and 3.84; 16 on one, 552 4.02 and 3.80."""
     workgroups = requests * head_tiles(q_heads, kv_heads)
     if workgroups > units:
         return 0
@@ -72,18 +75,23 @@ def planned_splits(requests: int, q_heads: int, kv_heads: int, head_dim: int, ma
     return coarse
 
 
-def runs_for_the_product(q_heads: int, kv_heads: int, max_keys: int, units: int = 256) -> int:
+def runs_for_the_product(q_heads: int, kv_heads: int, max_keys: int, units: int = 256) -> Optional[int]:
     """Runs of keys in a recorded step of one request whose o projection merges them: about 256 keys each, which eight waves have on
-    their way at once, in powers of two; no more workgroups than compute units, since every run is 16 KB and more that each
-    workgroup of the product reads. Passes of eight steps, ms, with 1, 2, 4, ... runs: 135M sizes, 304 keys 4.91 and 4.92, 400 5.19
-    and 5.05, 520 5.30, 4.95 and 5.00, 640 5.56, 5.17 and 5.02, 1,000 (from 2 on) 5.38, 5.02 and 5.09, 2,000 (from 4 on) 5.47, 5.17
-    and 5.55; 1B sizes, 2,000 (from 4 on) 5.78 and 5.64, with 16 5.78, 8,000 (from 16 on) 6.07, 5.99 and 6.14; 1.7B sizes, 4,000 (from
-    4 on) 9.08, 8.87 and 9.11; 3B sizes, 520 13.80, 13.50 and 13.16, 2,000 (from 4 on) 13.76, 13.60 and 14.25."""
+    their way at once, in powers of two; no more workgroups than compute units, since a run is ``q_heads * (4 * head_dim + 8)`` bytes
+    (2.4 KB at the 135M sizes, 12.5 at the 3B sizes) that each workgroup of the product reads. None where that makes more runs than the
+    product merges: :func:`planned_splits` decides then. Passes of eight steps, ms, with 1, 2, 4, ... runs: 135M sizes, 312
+    keys 4.90 and 4.97, 408 5.08 and 4.88, 520 5.18, 4.96 and 5.01, 648 5.53, 5.14 and 5.04, 1,008 (from 2 on) 5.29, 5.06 and 5.23, 2,008
+    (from 4 on) 5.41, 5.23 and 5.55; 1B sizes, 520 5.61 and 5.54, 2,008 (from 4 on) 5.78 and 5.64, with 16 5.78; 1.7B sizes, 4,008 (from 4
+    on) 9.01, 8.86 and 9.06, 32,008 (from 8 on) 15.9 and 16.4; 3B sizes, 520 13.4, 13.1 and 13.2, 2,008 (from 4 on) 13.8, 13.6 and 14.1.
+
+    So a request alone may have its keys in other runs than the same request among others, and the last bit of a rounding
+    differ (as it may between steps of 8 and of 64 requests, whose runs differ too): what a row's sums do not depend on is the
+    other rows of a product."""
     want, runs = max(1, (max_keys + 128) // 256), 1
-    most = min(MAX_SPLITS, units // head_tiles(q_heads, kv_heads))
+    most = units // head_tiles(q_heads, kv_heads)
     while runs < want and 2 * runs <= most:
         runs *= 2
-    return runs
+    return runs if runs <= ops.MERGED_SPLITS else None
 
 
 # A launch of fewer workgroups than this per compute unit is as long as its longest workgroup, and

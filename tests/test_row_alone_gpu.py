@@ -39,3 +39,24 @@ def test_a_row_alone_is_summed_as_among_others(ops, k, parts):
                                      ssq_in=ssq[:, :rows].contiguous())
             got[rows] = q[0], kp[0, :, 0].clone(), vp[0, :, :, 0].clone()
         assert all(torch.equal(a, b) for a, b in zip(got[1], got[3]))
+
+
+# parts: one trip, and more than a workgroup asks for at once (64 a wave of four or eight)
+@pytest.mark.parametrize("k,parts", [(256, 16), (640, 40), (1024, 64), (1024, 520), (1920, 600)])
+@pytest.mark.parametrize("n", [16, 512, 1536])
+def test_a_gated_row_alone_is_summed_as_among_others(ops, n, k, parts):
+    """The same for the gated product."""
+    gen = torch.Generator().manual_seed(n + k)
+    w = (torch.randn(2 * n, k, generator=gen) / math.sqrt(k)).bfloat16().cuda()
+    tiled, norm_w = ops.tile_weights(w), (1 + 0.1 * torch.randn(k, generator=gen)).cuda()
+    assert all(ops.skinny_gemm_plan(rows, n, k, ops.SKINNY_SWIGLU, w.device, tiled=True)[0] == "tiles16" for rows in (1, 3))
+    for _ in range(40):
+        x = torch.randn(3, k, generator=gen).bfloat16().cuda()
+        ssq = (torch.rand(parts, 3, generator=gen) * k / parts * 2).cuda()
+        got = {}
+        for rows in (1, 3):
+            out = torch.empty(rows, n, dtype=torch.bfloat16, device="cuda")
+            ops.skinny_gemm(x[:rows], w, w_tiled=tiled, epilogue=ops.SKINNY_SWIGLU, out=out, norm_w=norm_w, eps=1e-5,
+                            ssq_in=ssq[:, :rows].contiguous())
+            got[rows] = out[0]
+        assert torch.equal(got[1], got[3])

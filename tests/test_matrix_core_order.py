@@ -110,3 +110,21 @@ def test_vector_instructions_wait_for_a_products_result(listing):
                     continue
             ways.append((j + 1, states + 1 + (int(i.operands[0]) if i.op == "s_nop" else 0)))
     assert not found
+
+
+def test_a_merge_of_runs_asks_for_all_of_them_at_once(listing):
+    """The decode attention's workgroup that merges eight or sixteen runs has what all of them left on its way before it waits for
+    the first: a load of four sums and one of two statistics each (of which the compiler takes a pair or two as one)."""
+    most, asked = {}, 0
+    for i in listing:
+        kernel = re.search(r"attention_decode_kernelILi(\d+)ELi(\d+)ELi(\d+)E", i.kernel)
+        if kernel is None:
+            continue
+        kernel = tuple(map(int, kernel.groups()))
+        if i.op.startswith("buffer_load"):
+            asked += 1
+        elif i.op == "s_waitcnt" and any(o.startswith("vmcnt") for o in i.operands):
+            most[kernel], asked = max(most.get(kernel, 0), asked), 0
+    # (sixteenths of a head, waves, runs): heads of up to 48 have a copy for eight runs
+    assert set(most) == {(d, w, r) for d in range(1, 9) for w in (4, 8) for r in ((8, 16) if d <= 3 else (16,))}
+    assert all(n >= 2 * r - 2 for (_, _, r), n in most.items()), most

@@ -684,13 +684,21 @@ static int gf_rule(int m, int n, int segments) {
   return tiles < 8 * simds ? 6 : 7;
 }
 
-// Where the rule names four waves a tile of 32 x 32: whether tiles of 64 x 64 with loads ahead take less. They do where most units
-// have such a tile, and with sums of up to 1,024, whose segments four waves share badly, from half of them on: us with four waves a
-// tile and with loads ahead, k of 576, 960 and 2,048: 192 x 2,800 (132 tiles of 64 x 64) 21.0 17.6, 26.7 25.8, 48.0 48.6;
-// 500 x 1,536 (192) 23.1 17.6, 27.4 25.6, 46.7 48.1; 700 x 1,280 (220) 23.4 17.4, 31.5 25.4, 57.1 48.6; 100 x 3,072 (96) 13.7 16.9.
-static bool gf_few_waves_ahead(int m, int n, int k) {
-  const int64_t tiles = (int64_t)((n + 63) / 64) * ((m + 63) / 64), units = dli_compute_units();
-  return k <= 1024 ? 2 * tiles > units : 4 * tiles > 3 * units;
+// Where the rule names four waves a tile of 32 x 32: whether tiles of 64 x 64 with loads ahead take less, by how many of either a
+// compute unit gets. (Rows that half fill their last tile of 64, and tiles just past a round, make many of them.) us with four
+// waves a tile and with loads ahead, m x n, tiles of either on the busiest unit:
+//   k 576    24 x 12,198  2 1  13.8 16.8   192 x 2,800  3 1  21.0 17.6   556 x 1,826  5 2  29.2 25.7   1,004 x 1,378  6 2  34.0 26.5
+//   k 960    1,265 x 302  2 1  17.8 25.3   192 x 2,800  3 1  26.7 25.8   556 x 1,826  5 2  39.0 39.8   1,004 x 1,378  6 2  45.9 40.6
+//   k 2,048  28 x 14,961  2 1  33.4 48.3   192 x 2,800  3 1  48.0 48.6   700 x 1,280  4 1  57.1 48.6   556 x 1,826    5 2  74.6 79.8
+//            1,004 x 1,378  6 2  84.4 78.7   93 x 10,291  4 2  63.0 80.4   757 x 2,716  8 3  118 122
+extern "C" int dli_gemm_f32_few_waves_ahead(int m, int n, int k, int units) {
+  const auto on_a_unit = [&](int side) {
+    const int64_t tiles = (int64_t)((n + side - 1) / side) * ((m + side - 1) / side);
+    return (tiles + units - 1) / units;
+  };
+  const int64_t small = on_a_unit(32), large = on_a_unit(64);
+  if (k < 960 || (k <= 1024 && large == 1)) return small > 2 * large;
+  return small >= (large == 1 ? 4 : 3 * large);
 }
 
 // The order of a sum over k: `segments` of `seg_runs` runs each.
@@ -723,7 +731,7 @@ extern "C" int dli_gemm_f32_nt(const float* a, int64_t lda, const float* w, int6
     case 2: return gf_few<1, 4>(p, vec, stream);
     case 3: return gf_few<2, 2>(p, vec, stream);
     case 4: return gf_tiles<1, 1, 8>(p, vec, stream);
-    case 5: return ahead && gf_few_waves_ahead(m, n, k) ? gf_ahead<2, 2, 4>(p, stream) : gf_tiles<1, 1, 4>(p, vec, stream);
+    case 5: return ahead && dli_gemm_f32_few_waves_ahead(m, n, k, dli_compute_units()) ? gf_ahead<2, 2, 4>(p, stream) : gf_tiles<1, 1, 4>(p, vec, stream);
     case 6: return ahead ? gf_ahead<2, 2, 3>(p, stream) : gf_tiles<2, 2, 1>(p, vec, stream);
     default: return ahead ? gf_ahead<4, 2, 3>(p, stream) : gf_tiles<4, 2, 1>(p, vec, stream);
   }

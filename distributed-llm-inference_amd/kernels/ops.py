@@ -80,6 +80,7 @@ _SIGNATURES = {
                       _c_int, _c_ptr],
     "dli_gemm_bf16_f32": [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_i64, _c_i64, _c_ptr, _c_i64,
                       _c_int, _c_ptr],
+    "dli_gemm_f32_few_waves_ahead": [_c_int, _c_int, _c_int, _c_int],
     "dli_tile_gemm_takes": [_c_i64, _c_i64, _c_i64, _c_int],
     "dli_gemm_bf16_usable": [_c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_i64, _c_int],
     "dli_prenorm_blocks_bf16": [_c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr],

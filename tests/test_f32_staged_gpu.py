@@ -47,7 +47,7 @@ def test_norm_ahead_of_the_weights(m, inter, k):
 # rows and columns: parts of tiles of 64 x 64 and 128 x 64, one and several a unit; k: fewer blocks than stages, as many, a segment of
 # several runs with a rest
 @pytest.mark.parametrize("m,n,k", [(17, 40000, 32), (130, 20000, 64), (300, 9001, 96), (65, 17000, 128), (511, 3072, 576), (193, 2800, 1024),
-                                   (960, 960, 2080), (1000, 1030, 4192), (700, 8200, 160)])
+                                   (960, 960, 2080), (1000, 1400, 4192), (700, 8200, 160)])
 def test_tiles_with_loads_ahead(m, n, k):
     from dli_amd.kernels import ops
 

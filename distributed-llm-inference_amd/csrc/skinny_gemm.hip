@@ -40,8 +40,11 @@
 //            arithmetic in the same order as attention_merge_kernel, so that the o projection of a
 //            step of one to four rows needs no merge kernel before it. Each wave merges the run of
 //            k that it multiplies (all loads of a lane in flight at once) and hands it to its
-//            lanes through LDS. EPI_RESIDUAL, at most 16 runs. TILED, or row by row where K is no whole blocks of 128, as
-//            the product of several rows reads those: a row alone in its step is summed as among others.
+//            lanes through LDS. EPI_RESIDUAL, at most 16 runs. TILED, or, where K is no whole blocks of 128, in chunks:
+//              t[tile][chunk][c][8] = w[16*tile + c][8*chunk + (0..7)],
+//            of which a wave can take any steps of 32 k in whole lines. k is then split and summed as the product of several rows,
+//            which reads such weights row by row, does it: a row alone in its step has the same bits as among others. (Row by
+//            row here too, whose loads touch a line a lane: 135M sizes 5.05 ms a pass of eight steps, 360M sizes 6.46.)
 #include "common.h"
 #include "merge_splits.h"
 
@@ -136,6 +139,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
   __shared__ __align__(16) bf16_t xs[MERGED ? KS : 1][MERGED ? MERGE_ROWS : 1][MERGED ? MERGE_RANGE : 8];
   constexpr int NA = EPI == EPI_SWIGLU ? 2 : 1;  // weight row sets per tile (gate and up)
   constexpr bool PADDED = EPI == EPI_QKV;        // the weights' last block of 128 k may be filled up with zeros
+  constexpr bool CHUNKS = MERGED && !TILED;      // weights in chunks of eight k, sixteen rows' chunks one behind the other
   // What follows the last product is a chain that nothing hides, so it is kept short. With one row
   // tile and one group of waves (SHORT) all waves leave their parts in LDS and thread t makes
   // output t of each tile: element t % 4 of lane t / 4 of the product's result, that is row
@@ -161,6 +165,8 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
         // the tile's first block, at this lane's 16 bytes of a 1 KB load
         const int tile = min(tile0 + j, (N - 1) / 16) + a * (up_offset / 16);
         wrow[j][a] = w + (int64_t)tile * 16 * (PADDED ? (K + 127) / 128 * 128 : K) + lane * 8;
+      } else if constexpr (CHUNKS) {
+        wrow[j][a] = w + (int64_t)min(tile0 + j, (N - 1) / 16) * 16 * K + col * 8;
       } else {
         const int n = min((tile0 + j) * 16 + col, N - 1) + a * up_offset;
         wrow[j][a] = w + (int64_t)n * K + grp * 32;
@@ -168,6 +174,7 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
     }
   // where a lane finds its eight k values of product q in the block that starts at step s
   auto w_at = [&](const bf16_t* base, int s, int q) __attribute__((always_inline)) {
+    if (CHUNKS) return reinterpret_cast<const bf16x8*>(base + (4 * (s + grp) + q) * 128);
     return reinterpret_cast<const bf16x8*>(TILED ? base + (s / 4) * 2048 + q * 512 : base + s * 32 + q * 8);
   };
 
@@ -280,9 +287,9 @@ __global__ __launch_bounds__(KS * NS * 64) void skinny_gemm_kernel(
   };
   int blocks = (s_end - s) / 4;
   Block b0, b1;
-  // single steps behind the last block (row by row): lane group g reads k in [8g, 8g + 8)
+  // single steps behind the last block (not TILED): lane group g reads k in [8g, 8g + 8)
   auto w_single_at = [&](const bf16_t* base, int s) __attribute__((always_inline)) {
-    return reinterpret_cast<const bf16x8*>(base - grp * 32 + s * 32 + grp * 8);
+    return reinterpret_cast<const bf16x8*>(CHUNKS ? base + (4 * s + grp) * 128 : base - grp * 32 + s * 32 + grp * 8);
   };
   bf16x8 w_single[MERGED && !TILED ? 3 : 1];   // MERGED: asked for ahead of the merge, like the blocks
   if constexpr (NORM) {
@@ -739,7 +746,7 @@ __global__ __launch_bounds__(KS * 64) void normed_tiles_kernel(NormedArgs p) {
   // (decode graphs) a wave takes 64 of them in a row, lane l for row l % M; else the lane group grp takes
   // part 4 ks + grp, and every 4 KS-th behind it, for row l % 16.
   // IN_TURN (one row): the lane group's parts likewise, one a lane, added in their order as the general kernel adds them. More rows
-  // of such a product take that kernel, and a request's row then has the same bits whether others share the step or not.
+  // of such a product take that kernel, and a row then has the same bits whether others share the product or not.
   const __amdgpu_buffer_rsrc_t sres = __builtin_amdgcn_make_buffer_rsrc((void*)p.ssq_in, 0, (unsigned)(p.ssq_parts * M * 4), 0x00020000);
   const bool even = (M & (M - 1)) == 0;
   const int s_at = IN_TURN ? (4 * ks + grp + col * 4 * KS) * 4 : even ? threadIdx.x * 4 : ((4 * ks + grp) * M + min(col, M - 1)) * 4;
@@ -1146,7 +1153,7 @@ extern "C" int dli_skinny_gemm_qkv_rope(const void* x, int64_t ldx, const float*
 // The o projection of a decode step of at most MERGE_ROWS rows, fed with the split-key partial
 // results of the attention instead of its merged output (MERGED above): stream += merge(...) @ w^T
 // (+ bias), and the parts of the rows' sums of squares. w [N, K], K = heads * head_dim, in tile order where K is whole blocks of
-// 128, else row by row; splits 2..MERGE_SPLITS; shape 0 or 1 (4 or 8 waves split k).
+// 128, else in chunks; splits 2..MERGE_SPLITS; shape 0 or 1 (4 or 8 waves split k).
 extern "C" int dli_skinny_gemm_merged(const float* part_o, const float* part_ml, int splits, int heads,
                                       int head_dim, const void* w, const void* bias, void* stream_buf,
                                       int64_t lds_, float* ssq_out, int M, int N, int shape, hipStream_t stream) {

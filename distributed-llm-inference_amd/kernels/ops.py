@@ -580,6 +580,15 @@ def tile_weights(w: torch.Tensor, whole_blocks: bool = True) -> torch.Tensor:
     return t.permute(0, 2, 4, 3, 1, 5).contiguous().view(-1)
 
 
+def tile_weights_in_chunks(w: torch.Tensor) -> torch.Tensor:
+    """``w [n, k]`` (bfloat16, n % 16 == 0, k % 8 == 0) as ``t[tile][chunk][c][8] = w[16*tile + c][8*chunk + ...]``, flat: what
+    :func:`skinny_gemm_merged` reads where k is no whole blocks of 128."""
+    _dense(w, "w", torch.bfloat16, 2)
+    n, k = w.shape
+    _require(n % 16 == 0 and k % 8 == 0, "chunks need n % 16 == 0 and k % 8 == 0")
+    return w.view(n // 16, 16, k // 8, 8).permute(0, 2, 1, 3).contiguous().view(-1)
+
+
 def padded_k(k: int) -> int:
     """``k`` rounded up to whole blocks of 128."""
     return -(-k // 128) * 128
@@ -798,8 +807,8 @@ def skinny_gemm_merged_supports(rows: int, n: int, heads: int, head_dim: int, sp
     """Whether :func:`skinny_gemm_merged` takes this o projection: few rows, few runs of keys, a
     product that the 16x16-tile kernel runs with k split over the waves of a workgroup. Up to 512, k in whole blocks
     of 128 only: below, the launches around it hide a merge kernel about as well (passes of eight steps, 24 layers, ms, without and
-    with it: width 192, 450 keys 3.53 and 3.58, 4,000 3.86 and 4.15; 320, 3.90 and 3.92, 4.22 and 4.39; 448, 7.39 and 7.50, 8.80 and
-    8.76; 480, 3.38 and 3.46, 4.12 and 3.96)."""
+    with it: width 192, 450 keys 3.58 and 3.55, 4,000 3.86 and 4.08; 320, 3.90 and 3.84, 4.18 and 4.31; 448, 7.40 and 7.52, 8.77 and
+    8.75; 480, 3.37 and 3.49, 3.82 and 3.86)."""
     k = heads * head_dim
     if not (0 < rows <= MERGED_ROWS and 2 <= splits <= MERGED_SPLITS and head_dim % 4 == 0 and n % 16 == 0
             and (k % 128 == 0 or (k % 32 == 0 and k > 512))):
@@ -825,8 +834,8 @@ def skinny_gemm_merged(part_o: torch.Tensor, part_ml: torch.Tensor, splits: int,
     of a decode step fed with the partial results that :func:`attention_decode` leaves with
     ``merge=False`` (``part_o [rows, heads, splits, head_dim]``, ``part_ml [rows, heads, splits, 2]``),
     merged inside the product's kernel with the arithmetic of the merge kernel. ``w``: in tile order
-    (:func:`tile_weights`) where ``heads * head_dim`` is whole blocks of 128, else ``[n, heads * head_dim]`` as it is, as
-    :func:`skinny_gemm` reads them: the same bits as the merge kernel and that product. Returns the parts
+    (:func:`tile_weights`) where ``heads * head_dim`` is whole blocks of 128, else in chunks (:func:`tile_weights_in_chunks`): the
+    same bits as the merge kernel and the residual product of :func:`skinny_gemm`. Returns the parts
     of the rows' sums of squares like the residual epilogue of :func:`skinny_gemm`."""
     _rows(stream, "stream", torch.bfloat16)
     m, n = stream.shape
@@ -839,9 +848,8 @@ def skinny_gemm_merged(part_o: torch.Tensor, part_ml: torch.Tensor, splits: int,
     _require(part_o.numel() >= m * heads * splits * head_dim and part_ml.numel() >= m * heads * splits * 2,
              "partial-result buffers are too small")
     _require(part_o.data_ptr() % 16 == 0 and part_ml.data_ptr() % 8 == 0, "partial results must be 16-byte aligned")
-    _dense(w, "w", torch.bfloat16, 1 if k % 128 == 0 else 2)
-    _require(w.numel() == n * k and (k % 128 == 0 or w.shape[1] == k) and w.data_ptr() % 16 == 0,
-             "w must hold [n, heads*head_dim], in tile order where that is whole blocks of 128")
+    _dense(w, "w", torch.bfloat16, 1)
+    _require(w.numel() == n * k and w.data_ptr() % 16 == 0, "w must hold [n, heads*head_dim] in tile order or chunks")
     if bias is not None:
         _dense(bias, "bias", torch.bfloat16, 1)
         _require(bias.shape[0] == n, "bias length differs from rows of w")

@@ -62,6 +62,7 @@ class GQAttention(Mixer):
         self.position = build_part("position", position or PartSpec("none"), runtime)
         self.w_qkv = self.b_qkv = self.w_o = self.b_o = None
         self.w_qkv_tiled = self.w_o_tiled = None
+        self.w_o_merging = None   # as the product that merges the runs of keys reads it
         self.w_qkv_rope = self.b_qkv_rope = None  # tile order with rotary pairs, for the product that rotates
         self._arrivals: Optional[torch.Tensor] = None
 
@@ -105,6 +106,10 @@ class GQAttention(Mixer):
     def finalize(self) -> None:
         self.w_qkv_tiled = decode_copy(self.rt, self.w_qkv, ops.SKINNY_STORE)
         self.w_o_tiled = decode_copy(self.rt, self.w_o, ops.SKINNY_RESIDUAL)
+        self.w_o_merging = self.w_o_tiled
+        if self.w_o_tiled is not None and self.w_o.shape[1] % 128 != 0:
+            takes = ops.skinny_gemm_merged_supports(1, self.hidden_size, self.num_heads, self.head_dim, 2, self.w_o.device)
+            self.w_o_merging = ops.tile_weights_in_chunks(self.w_o) if takes else None
         table = self.position.rotary_table()
         if table is not None and table.pairing != "half":
             raise ops.KernelArgumentError(
@@ -159,7 +164,7 @@ class GQAttention(Mixer):
         if not self.rt.is_bf16:
             return None
         units = ops.compute_units(self.rt.device)
-        if requests <= MERGE_IN_PRODUCT_ROWS and self.w_o_tiled is not None:
+        if requests <= MERGE_IN_PRODUCT_ROWS and self.w_o_merging is not None:
             runs = runs_for_the_product(self.num_heads, self.num_kv_heads, max_keys, units)
             if runs == 1 or runs and ops.skinny_gemm_merged_supports(requests, self.hidden_size, self.num_heads, self.head_dim, runs, self.rt.device):
                 return runs
@@ -252,7 +257,7 @@ class GQAttention(Mixer):
                 inv_freq, rotary_dim = table.inv_freq, table.dim
             ops.rope_kv_write(qkv, ctx.positions, inv_freq, rotary_dim, grp.slots if nkv else None,
                               cache.k_pages if nkv else None, cache.v_pages if nkv else None, nh, nkv, d)
-        if n <= MERGE_IN_PRODUCT_ROWS and self.w_o_tiled is not None:
+        if n <= MERGE_IN_PRODUCT_ROWS and self.w_o_merging is not None:
             # the o projection merges the runs of keys itself while its first
             # weights are on their way, and no merge kernel runs between the two
             left = decode_attention_unmerged(
@@ -261,8 +266,7 @@ class GQAttention(Mixer):
                 planned=ctx.decode_plans.get(id(self)))
             if left is not None:
                 splits, part_o, part_ml = left
-                w_o = self.w_o_tiled if nh * d % 128 == 0 else self.w_o
-                stream.wrote(ops.skinny_gemm_merged(part_o, part_ml, splits, nh, d, w_o, stream.x, bias=self.b_o))
+                stream.wrote(ops.skinny_gemm_merged(part_o, part_ml, splits, nh, d, self.w_o_merging, stream.x, bias=self.b_o))
                 return
         out = self.rt.empty(n, nh * d)
         paged_attention(qkv[:, :nh * d], cache.k_pages, cache.v_pages, out, ctx, grp, nh, self.scale, self.window,

@@ -80,8 +80,8 @@ def runs_for_the_product(q_heads: int, kv_heads: int, max_keys: int, units: int 
     their way at once, in powers of two; no more workgroups than compute units, since a run is ``q_heads * (4 * head_dim + 8)`` bytes
     (2.4 KB at the 135M sizes, 12.5 at the 3B sizes) that each workgroup of the product reads. None where that makes more runs than the
     product merges: :func:`planned_splits` decides then. Passes of eight steps, ms, with 1, 2, 4, ... runs: 135M sizes, 312
-    keys 4.90 and 4.97, 408 5.08 and 4.88, 520 5.18, 4.96 and 5.01, 648 5.53, 5.14 and 5.04, 1,008 (from 2 on) 5.29, 5.06 and 5.23, 2,008
-    (from 4 on) 5.41, 5.23 and 5.55; 1B sizes, 520 5.61 and 5.54, 2,008 (from 4 on) 5.78 and 5.64, with 16 5.78; 1.7B sizes, 4,008 (from 4
+    keys 4.88 and 4.87, 408 5.09 and 4.85, 520 5.17, 4.91 and 4.95, 648 5.53, 5.11 and 4.98, 1,008 (from 2 on) 5.27, 5.05 and 5.11, 2,008
+    (from 4 on) 5.39, 5.19 and 5.46; 1B sizes, 520 5.61 and 5.54, 2,008 (from 4 on) 5.78 and 5.64, with 16 5.78; 1.7B sizes, 4,008 (from 4
     on) 9.01, 8.86 and 9.06, 32,008 (from 8 on) 15.9 and 16.4; 3B sizes, 520 13.4, 13.1 and 13.2, 2,008 (from 4 on) 13.8, 13.6 and 14.1.
 
     So a request alone may have its keys in other runs than the same request among others, and the last bit of a rounding

@@ -9,10 +9,10 @@ import torch
 
 # ms, a pass of eight steps: (query heads, kv heads, head size, width): keys at the pass's end: runs: time
 TIMES = {
-    (9, 3, 64, 576): {312: {1: 4.90, 2: 4.97}, 408: {1: 5.08, 2: 4.88}, 520: {1: 5.18, 2: 4.96, 4: 5.01}, 648: {1: 5.53, 2: 5.14, 4: 5.04},
-                      808: {2: 5.21, 4: 5.04}, 1008: {2: 5.29, 4: 5.06, 8: 5.23}, 1512: {4: 5.41, 8: 5.24}, 2008: {4: 5.41, 8: 5.23, 16: 5.55},
-                      4008: {8: 5.64, 16: 5.67}, 8008: {16: 6.17}},
-    (15, 5, 64, 960): {520: {1: 6.63, 2: 6.41}, 1008: {2: 6.76, 4: 6.50}},
+    (9, 3, 64, 576): {312: {1: 4.88, 2: 4.87}, 408: {1: 5.09, 2: 4.85}, 520: {1: 5.17, 2: 4.91, 4: 4.95}, 648: {1: 5.53, 2: 5.11, 4: 4.98},
+                      808: {2: 5.20, 4: 4.99}, 1008: {2: 5.27, 4: 5.05, 8: 5.11}, 1512: {4: 5.35, 8: 5.18}, 2008: {4: 5.39, 8: 5.19, 16: 5.46},
+                      4008: {8: 5.76, 16: 5.54}, 8008: {16: 5.93}},
+    (15, 5, 64, 960): {520: {1: 6.63, 2: 6.29}, 1008: {2: 6.67, 4: 6.38}},
     (32, 8, 64, 2048): {312: {1: 5.47, 2: 5.59}, 408: {1: 5.60, 2: 5.51}, 520: {1: 5.61, 2: 5.54}, 1008: {2: 5.76, 4: 5.57},
                         2008: {4: 5.78, 8: 5.64}, 8008: {16: 6.05}},
     (32, 32, 64, 2048): {520: {1: 8.17, 2: 8.03}, 1008: {2: 8.30, 4: 8.10}, 2008: {4: 8.42, 8: 8.40}, 4008: {4: 9.01, 8: 8.86, 16: 9.06},
@@ -34,7 +34,7 @@ def plan(monkeypatch):
         layer = object.__new__(GQAttention)
         layer.rt = SimpleNamespace(is_bf16=True, device=torch.device("cuda", 0))
         layer.num_heads, layer.num_kv_heads, layer.head_dim, layer.hidden_size = q_heads, kv_heads, head_dim, width
-        layer.w_o_tiled = torch.empty(0) if merges else None
+        layer.w_o_merging = torch.empty(0) if merges else None
         return layer.decode_plan(requests, keys)
 
     return answer

@@ -86,7 +86,7 @@ def test_merging_o_projection_of_odd_widths(ops, qh, kvh, d, n, splits, rows):
     out = torch.empty_like(q)
     ops.attention_decode(q, kp, vp, out, kv_len, tables, qh, 0.125, 0, splits, po, ml)
     got, want = base.clone(), base.clone()
-    ssq = ops.skinny_gemm_merged(po, ml, splits, qh, d, w, got, bias=bias)
+    ssq = ops.skinny_gemm_merged(po, ml, splits, qh, d, ops.tile_weights_in_chunks(w), got, bias=bias)
     ssq_want = ops.skinny_gemm(out, w, epilogue=ops.SKINNY_RESIDUAL, stream=want, bias=bias)
     assert torch.equal(got, want) and torch.equal(ssq, ssq_want)
     # product and bias rounded once, then their sum with the stream: half of the last of eight bits each, and the 32-bit sums

@@ -8,17 +8,17 @@
 //   S^T [16 keys x 16 columns]   = K [16 keys x d]   * Q^T [d x 16 columns]
 //   O^T [16 dims x 16 columns]  += V^T [16 dims x 16 keys] * P^T [16 keys x 16 columns]
 //
-// with v_mfma_f32_16x16x16_bf16: operand A gives lane l row l%16 and the four k-indices
-// 4*(l/16)..+3; operand B gives lane l column l%16 and the same k-indices; the result gives lane l
-// column l%16 and rows 4*(l/16)..+3. So S^T comes out exactly in the layout that P^T needs as
-// operand B of the second product. A "column" is a query head of the group in the decode kernel
-// and a query position in the prefill kernel.
+// with v_mfma_f32_16x16x32_bf16, keys in pairs of tiles: operand A gives lane l row l%16 and the eight
+// k-indices 8*(l/16)..+7; operand B gives lane l column l%16 and the same k-indices; the result gives lane l
+// column l%16 and rows 4*(l/16)..+3. The 32 keys of a pair are dealt to the two products K Q^T so (8 (row / 4) + row % 4 and four
+// on) that S^T comes out exactly in the layout that P^T needs as operand B of the second product. Heads of 16 take
+// v_mfma_f32_16x16x16_bf16, four k-indices a lane: in prompts a kernel of their own, tile by tile, whose layout is the product's as it
+// is; in decode steps, where heads of 48, 80 and 112 take it for their last sixteen dims as well, for K Q^T. A "column" is
+// a query head of the group in the decode kernel and a query position in the prefill kernels.
 //
 // K pages are [kv_heads][page_size][head_dim] and V pages [kv_heads][head_dim][page_size]: operand
 // A of the first product reads head_dim-contiguous keys, operand A of the second reads
-// key-contiguous dims. The d index of the first product is permuted (lane group g takes the
-// contiguous range [g*d/4, (g+1)*d/4)), identically for K and Q, which leaves the dot product
-// unchanged and makes each lane's K load one contiguous run.
+// key-contiguous dims.
 //
 // Needs page_size % 16 == 0 and head_dim = 16*DCH with DCH <= 8; other shapes take the generic
 // kernel. Scores are scaled by `scale`; exp is taken as exp2 with log2(e) folded into the scale.
@@ -1207,8 +1207,9 @@ static size_t decode_states(int group, int head_dim) {
   return (size_t)4 * (head_dim / 16) * 4 * (group < 16 ? group : 16) * sizeof(float4v);
 }
 
-// Waves of a decode workgroup, `group` query heads a kv head: eight where every workgroup has a compute unit to itself (few keys then
-// need no second run, whose merge costs more than it saves: one_run_keys in parts/attention_kernels.py has the figures), with more workgroups four, of
+// Waves of a decode workgroup, `group` query heads a kv head: eight where every workgroup has a compute unit to itself (few keys of
+// several requests then need no second run, whose merge costs more than it saves: one_run_keys in parts/attention_kernels.py has the
+// figures, runs_for_the_product those of one request whose o projection merges), with more workgroups four, of
 // which several share a unit. The waves' states have to fit 48 KB of LDS: heads of 128 in groups of up to twelve, of 112 up to 13.
 extern "C" int dli_attention_decode_waves(int64_t workgroups, int group, int head_dim, int units) {
   return workgroups <= units && 2 * decode_states(group, head_dim) <= 48 * 1024 ? 8 : 4;

@@ -199,6 +199,9 @@ _SIGNATURES = {
     "dli_conv_prepare_in_runs": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
     "dli_conv_prepare": [_c_ptr, _c_i64, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr,
                          _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
+    "dli_gated_delta_single_takes": [_c_int, _c_int, _c_int, _c_int, _c_int],
+    "dli_gated_delta_single": [_c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr,
+                               _c_ptr, _c_float, _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "dli_gated_delta_scan": [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_int,
                              _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
     "dli_poly_norm": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_float, _c_int, _c_ptr],
@@ -2318,6 +2321,40 @@ def gated_delta_scan(prep: torch.Tensor, state: torch.Tensor, q_start: torch.Ten
         _ptr(prep), prep.stride(0), _ptr(state), state.stride(0), _ptr(q_start), _ptr(positions), _ptr(state_slots),
         _ptr(o), o.stride(0), entries, n, heads, kv_heads, dim, vdim, *cut[:3], *map(_ptr, cut[3:]), _stream()),
         "gated_delta_scan")
+
+
+def gated_delta_single_takes(heads: int, kv_heads: int, dim: int, vdim: int, taps: int) -> bool:
+    """Whether :func:`gated_delta_single` has a kernel for these sizes."""
+    return bool(library().dli_gated_delta_single_takes(heads, kv_heads, dim, vdim, taps))
+
+
+def gated_delta_single(proj: torch.Tensor, b_off: int, a_off: int, g_off: int, conv_w: torch.Tensor, a_log: torch.Tensor,
+                       dt_bias: torch.Tensor, state: torch.Tensor, kept_offset: int, positions: torch.Tensor, state_slots: torch.Tensor,
+                       norm_w: torch.Tensor, eps: float, out: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim: int) -> None:
+    """:func:`conv_prepare`, :func:`gated_delta_scan` and :func:`head_norm_gate` (gate ``silu`` of the columns from ``g_off`` on) of
+    a step of single tokens in one kernel, a row a request; the same bits."""
+    _f32_rows(proj, "proj")
+    _dense(conv_w, "conv_w", torch.float32, 2)
+    channels, taps = conv_w.shape
+    n, hv = proj.shape[0], heads * vdim
+    _require(gated_delta_single_takes(heads, kv_heads, dim, vdim, taps), "gated_delta_single: sizes that its kernel does not take")
+    _require(channels == 2 * kv_heads * dim + hv, "conv_w must hold a row per channel of q, k and v")
+    for name, t, size in (("a_log", a_log, heads), ("dt_bias", dt_bias, heads), ("norm_w", norm_w, hv)):
+        _dense(t, name, torch.float32, 1)
+        _require(t.shape[0] == size, f"{name} must hold {size} values")
+    _rows(out, "out", out.dtype)
+    _require(out.shape == (n, hv), "out must be [n, heads*vdim]")
+    _require(state.is_cuda and state.dtype == torch.float32 and state.dim() == 2 and state.stride(1) == 1 and kept_offset >= hv * dim
+             and state.shape[1] >= kept_offset + (taps - 1) * channels, "state must be float32 [slots, >= state and kept inputs]")
+    for name, t in (("positions", positions), ("state_slots", state_slots)):
+        _dense(t, name, torch.int32, 1)
+        _require(t.shape[0] == n, f"{name}: single tokens, a row an entry")
+    _require(all(channels <= at and at + size <= proj.shape[1] for at, size in ((b_off, heads), (a_off, heads), (g_off, hv))),
+             "beta's, the decay's or the gate's columns lie outside proj")
+    _check(library().dli_gated_delta_single(
+        _ptr(proj), proj.stride(0), int(b_off), int(a_off), int(g_off), _ptr(conv_w), _ptr(a_log), _ptr(dt_bias), _ptr(state),
+        state.stride(0), int(kept_offset), _ptr(positions), _ptr(state_slots), _ptr(norm_w), float(eps), _ptr(out), out.stride(0), n,
+        heads, kv_heads, dim, vdim, taps, _is_bf16(out.dtype), _stream()), "gated_delta_single")
 
 
 HEAD_GATES = {"sigmoid": 0, "silu": 1, "none": 2, "silu_first": 3}

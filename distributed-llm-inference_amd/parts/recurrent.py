@@ -242,6 +242,12 @@ class GatedDelta(Mixer):
             proj = linear_f32(self.rt, as_operand(self.rt, x, ctx), self.w_in)
         g_off = self.channels
         b_off, a_off = g_off + self.hv, g_off + self.hv + H
+        if ctx.num_decode == ctx.num_entries and ops.gated_delta_single_takes(H, self.num_kv_heads, self.head_dim, self.value_dim, self.conv_taps):
+            out = self.rt.empty(n, self.hv)
+            ops.gated_delta_single(proj, b_off, a_off, g_off, self.conv_w, self.a_log, self.dt_bias, state, self.state_floats,
+                                   ctx.positions, ctx.state_slots, self.norm_w, self.norm_eps, out, H, self.num_kv_heads,
+                                   self.head_dim, self.value_dim)
+            return linear_f32(self.rt, out, self.w_o)
         width = self.channels + 2 * H
         prep = torch.empty(n, -(-width // 4) * 4, device=self.rt.device, dtype=torch.float32)[:, :width]   # rows of whole 16 bytes
         ops.conv_prepare(proj, b_off, a_off, self.conv_w, self.a_log, self.dt_bias, state, self.state_floats,

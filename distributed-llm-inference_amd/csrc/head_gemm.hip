@@ -105,7 +105,7 @@ __global__ __launch_bounds__(HEAD_KS * 64) void head_gemm_kernel(
     for (int j = 0; j < 2; ++j) {
       const int tile = min(2 * pair + j, tiles - 1);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) dst[j][q] = *w_at(tile, b, q);
+      for (int q = 0; q < 4; ++q) dst[j][q] = load_streamed(w_at(tile, b, q));
     }
   };
 

@@ -69,7 +69,7 @@ struct MidArgs {
 // few trips to memory, and what bounds them is how many bytes are under way. The NW waves of one
 // kw share that block's activations through LDS; the KW partial tiles of a feature tile meet in
 // LDS at the end and are added in the order of kw. grid (ceil(tiles / NW), splits).
-template <int MT, int NW, int KW, int EPI>
+template <int MT, int NW, int KW, int EPI, bool TILED>
 __global__ __launch_bounds__(NW * KW * 64) void mid_gemm_kernel(MidArgs p) {
   constexpr int NA = EPI == MID_SWIGLU ? 2 : 1;
   constexpr int NG = NW * 64;          // threads that stage one kw's blocks
@@ -114,17 +114,17 @@ __global__ __launch_bounds__(NW * KW * 64) void mid_gemm_kernel(MidArgs p) {
   // issues the same loads, the number of loads on their way is known at every wait, and a step
   // waits for its own block only.
   const int KP = nblk * 128;           // a row of the tile-ordered copy: whole blocks
-  const unsigned w_bytes = (unsigned)((int64_t)p.w_rows * (p.tiled ? KP : K) * 2);
+  const unsigned w_bytes = (unsigned)((int64_t)p.w_rows * (TILED ? KP : K) * 2);
   const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc((void*)p.w, 0, w_bytes, 0x00020000);
   const unsigned x_bytes = (unsigned)(((int64_t)(M - 1) * p.ldx + K) * 2);
   const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, x_bytes, 0x00020000);
   // this lane's first weight fragment (byte offset) and the steps to the next block and product
   unsigned wbase[NA];
-  const int blk_stride = p.tiled ? 4096 : 256, q_stride = p.tiled ? 1024 : 16;
+  constexpr int blk_stride = TILED ? 4096 : 256, q_stride = TILED ? 1024 : 16;
 #pragma unroll
   for (int a = 0; a < NA; ++a) {
     const int tl = min(tile, tiles - 1);
-    if (p.tiled) {
+    if constexpr (TILED) {
       wbase[a] = (unsigned)(((int64_t)(tl + a * (p.up_offset / 16)) * 16 * KP + lane * 8) * 2);
     } else {
       const int n = min(tl * 16 + col, N - 1) + a * p.up_offset;
@@ -138,7 +138,8 @@ __global__ __launch_bounds__(NW * KW * 64) void mid_gemm_kernel(MidArgs p) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const unsigned at = wanted ? wbase[a] + (unsigned)(b * blk_stride + q * q_stride) : w_bytes;
-        dst[a][q] = as_bf16x8(__builtin_amdgcn_raw_buffer_load_b128(wres, (int)at, 0, 0));
+        // (row by row a line's parts are asked for by several loads, which a line that leaves the caches first would not outlive)
+        dst[a][q] = as_bf16x8(__builtin_amdgcn_raw_buffer_load_b128(wres, (int)at, 0, TILED ? STREAMED : 0));
       }
   };
   const bool norm = p.norm_w != nullptr;
@@ -512,7 +513,8 @@ int launch_mid(int nw, int kw, const MidArgs& a, hipStream_t stream) {
   const dim3 grid((tiles + nw - 1) / nw, a.splits);
 #define MID_CASE(NW_, KW_)                                                              \
   if (nw == NW_ && kw == KW_) {                                                         \
-    mid_gemm_kernel<MT, NW_, KW_, EPI><<<grid, NW_ * KW_ * 64, 0, stream>>>(a);         \
+    if (a.tiled) mid_gemm_kernel<MT, NW_, KW_, EPI, true><<<grid, NW_ * KW_ * 64, 0, stream>>>(a);  \
+    else mid_gemm_kernel<MT, NW_, KW_, EPI, false><<<grid, NW_ * KW_ * 64, 0, stream>>>(a);         \
     return dli_launch_status();                                                         \
   }
   if constexpr (EPI == MID_SWIGLU) {

@@ -442,8 +442,13 @@ __global__ __launch_bounds__(256) void expert_few_kernel(ExpertArgs p, const bf1
   exm_bf16x8 held[EXF_AHEAD][6];
   auto fetch = [&](int j, int chunk) {                                           // (past the end: pieces that no product takes)
     const int k0 = min(chunk, chunks - 1) * EXF_K;
+    const auto from = [&](int i) {
+      return reinterpret_cast<const exm_bf16x8*>(src[i] + min(k0 + 8 * (at ^ ((at_row + 8 * i) % 16)), depth - 8));
+    };
 #pragma unroll
-    for (int i = 0; i < 6; ++i) held[j][i] = exm_load(src[i] + min(k0 + 8 * (at ^ ((at_row + 8 * i) % 16)), depth - 8));
+    for (int i = 0; i < 4; ++i) held[j][i] = load_streamed(from(i));   // (a choice between this load and the other would become the other)
+#pragma unroll
+    for (int i = 4; i < 6; ++i) held[j][i] = *from(i);
   };
 #pragma unroll
   for (int j = 0; j < EXF_AHEAD; ++j) fetch(j, j);

@@ -156,7 +156,7 @@ __global__ __launch_bounds__(KS * 64) void skinny4_kernel(
     const bool inside = k < K && c < c1;  // the last chunk may reach past k; K % 8 == 0
     const int kc = k < K ? k : 0;
 #pragma unroll
-    for (int f = 0; f < FQ; ++f) st.wf[f].raw = *reinterpret_cast<const u32x4*>(wrow[f] + kc);
+    for (int f = 0; f < FQ; ++f) st.wf[f].raw = load_streamed(reinterpret_cast<const u32x4*>(wrow[f] + kc));
     if constexpr (!XL) {
       const int k_at = inside ? k * 2 : (int)x_bytes;  // one offset for every case, no branch
 #pragma unroll

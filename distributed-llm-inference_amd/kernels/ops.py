@@ -199,6 +199,10 @@ _SIGNATURES = {
     "dli_conv_prepare_in_runs": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
     "dli_conv_prepare": [_c_ptr, _c_i64, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr,
                          _c_ptr, _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
+    "dli_decode_flow_bytes": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
+    "dli_decode_flow_parts": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
+    "dli_decode_flow": [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int,
+                        _c_int, _c_int, _c_int, _c_float, _c_float, _c_ptr],
     "dli_gated_delta_single_takes": [_c_int, _c_int, _c_int, _c_int, _c_int],
     "dli_gated_delta_single": [_c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr,
                                _c_ptr, _c_float, _c_ptr, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
@@ -1067,6 +1071,48 @@ def gemm_workspace(device: torch.device) -> tuple[torch.Tensor, int]:
     if workspace is None:
         workspace = _gemm_workspaces[index] = torch.empty(_GEMM_WORKSPACE_BYTES, dtype=torch.uint8, device=device)
     return workspace, _GEMM_WORKSPACE_BYTES
+
+
+def decode_flow_bytes(layers: int, hidden: int, q_heads: int, kv_heads: int, head_dim: int, inner: int) -> int:
+    """Bytes of the words that :func:`decode_flow` hands its results on by; 0 where it does not take these sizes."""
+    return int(library().dli_decode_flow_bytes(layers, hidden, q_heads, kv_heads, head_dim, inner))
+
+
+def decode_flow_parts(layers: int, hidden: int, q_heads: int, kv_heads: int, head_dim: int, inner: int) -> int:
+    """Parts of the row's sum of squares that :func:`decode_flow` leaves."""
+    return int(library().dli_decode_flow_parts(layers, hidden, q_heads, kv_heads, head_dim, inner))
+
+
+def decode_flow(table: torch.Tensor, words: torch.Tensor, tickets: torch.Tensor, x: torch.Tensor, ssq_out: torch.Tensor,
+                angles: torch.Tensor, slots: torch.Tensor, kv_len: torch.Tensor, block_tables: torch.Tensor, sizes: Sequence[int],
+                page_size: int, eps: float, scale: float) -> None:
+    """All pre-norm blocks of a decode step of one row on the stream ``x [1, hidden]`` (in place; the row's sum of squares in parts
+    to ``ssq_out [parts, 1]``). ``table``: int64 ``[layers, 8]``, the addresses of each layer's two norm weights (float32), its
+    q/k/v, o, gate/up and down matrices (bfloat16, row by row) and its K and V pages; ``words`` and ``tickets``: zeros when made,
+    then these launches' own, which must not overlap; ``angles`` float32 ``[1, 2, head_dim/2]``; ``sizes``: layers, hidden size,
+    heads, kv heads, head size, inner size of the feed-forward."""
+    layers, hidden, q_heads, kv_heads, head_dim, inner = sizes
+    nbytes = decode_flow_bytes(*sizes)
+    _require(nbytes > 0, "decode_flow: sizes that its kernel does not take")
+    _dense(table, "table", torch.int64, 2)
+    _require(table.shape == (layers, 8), "table must be [layers, 8]")
+    _dense(words, "words", torch.int32, 1)
+    _dense(tickets, "tickets", torch.int64, 1)
+    _require(words.numel() * 4 >= nbytes and words.data_ptr() % 16 == 0 and tickets.numel() >= 1, "words or tickets are too few")
+    _dense(x, "x", torch.bfloat16, 2)
+    _require(x.shape == (1, hidden), "x must be one row")
+    _dense(ssq_out, "ssq_out", torch.float32, 2)
+    _require(ssq_out.shape == (decode_flow_parts(*sizes), 1), "ssq_out must be [parts, 1]")
+    _dense(angles, "angles", torch.float32, 3)
+    _require(angles.shape == (1, 2, head_dim // 2), "angles must be [1, 2, head_dim/2]")
+    _dense(slots, "slots", torch.int32, 1)
+    _dense(kv_len, "kv_len", torch.int32, 1)
+    _dense(block_tables, "block_tables", torch.int32, 2)
+    _require(slots.shape[0] == 1 and kv_len.shape[0] >= 1 and block_tables.shape[0] >= 1, "one row, one request")
+    _check(library().dli_decode_flow(
+        _ptr(table), layers, _ptr(words), _ptr(tickets), _ptr(x), _ptr(ssq_out), _ptr(angles), _ptr(slots), _ptr(kv_len),
+        _ptr(block_tables), block_tables.shape[1], hidden, q_heads, kv_heads, head_dim, inner, int(page_size), float(eps),
+        float(scale), _stream()), "decode_flow")
 
 
 def prenorm_blocks(x: torch.Tensor, blocks, count: int, step) -> bool:

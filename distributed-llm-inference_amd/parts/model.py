@@ -41,6 +41,9 @@ class BoundCaches(list):
 
     derived: Any = None             # NativeBlocks, or False where that route does not apply
     derived_for: int = -1           # the model's ``weights_version`` it was made for
+    flow: Any = None                # DecodeFlow, or False where that route does not apply
+    flow_for: int = -1
+    retired: tuple = ()             # memory of earlier ones, whose addresses recorded steps hold
 
 
 def _walk(part: Part):
@@ -177,7 +180,8 @@ class Model:
 
     def _forward_stream(self, ctx: Any, caches: Sequence[Any]) -> torch.Tensor:
         stream = self.embedding.forward_stream(ctx.token_ids)
-        order = [self.layers[entry.layer] for entry in self.spec.schedule]
+        flow = self._decode_flow(caches) if ctx.num_tokens == 1 else None
+        order = [] if flow is not None and flow.run(stream, ctx) else [self.layers[entry.layer] for entry in self.spec.schedule]
         for i, (layer, cache) in enumerate(zip(order, caches)):
             # the norm that the stream meets next: the following entry's first, or the final one
             after = order[i + 1].block.first_norm(order[i + 1].parts) if i + 1 < len(order) else self.final_norm
@@ -206,6 +210,23 @@ class Model:
             caches.derived = NativeBlocks.build(self, caches) or False
             caches.derived_for = self.weights_version
         return caches.derived or None
+
+    def _decode_flow(self, caches: Sequence[Any]):
+        """All blocks as one launch for steps of one row, made once per bound list of caches and set of weights and kept on that
+        list; ``None`` where that route does not apply, or would have to be made while the stream is being captured (its
+        memory would belong to that graph)."""
+        if not isinstance(caches, BoundCaches) or not self.rt.is_bf16 or not self.native_steps:
+            return None
+        if caches.flow is None or caches.flow_for != self.weights_version:
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            from .decode_flow import DecodeFlow
+
+            if caches.flow:
+                caches.retired += caches.flow.memory()
+            caches.flow = DecodeFlow.build(self, caches) or False
+            caches.flow_for = self.weights_version
+        return caches.flow or None
 
     def forward(self, ctx: Any, caches: Sequence[Any]) -> torch.Tensor:
         """Run the step's tokens through the schedule; float32 logits ``[wanted rows, vocab]``."""

@@ -120,8 +120,9 @@ def runs_of_tiles(key_tiles: np.ndarray, workgroups_per_tile: int, units: int, m
     spare = CUT_BELOW_WORKGROUPS_PER_UNIT * units // max(1, workgroups_per_tile) - key_tiles.size
     if spare <= 0 or key_tiles.size == 0:
         return runs
-    share = lambda i: -(-int(key_tiles[i]) // int(runs[i]))   # the tile's longest run
-    heap = [(-share(i), i) for i in range(key_tiles.size)]
+    # (Python's own numbers: one of an array's takes five times as long)
+    tiles, count = key_tiles.tolist(), [1] * key_tiles.size
+    heap = [(-t, i) for i, t in enumerate(tiles)]        # (the tile's longest run, negative)
     heapq.heapify(heap)
     # What a compute unit has to do in all, in tiles of 32 keys of one workgroup. Under a causal
     # mask from the prompt's start, the short tiles' workgroups leave early and the longest runs end
@@ -133,18 +134,17 @@ def runs_of_tiles(key_tiles: np.ndarray, workgroups_per_tile: int, units: int, m
     per_unit = float(key_tiles.sum()) * workgroups_per_tile / units
     lone_cost = LONE_TILE_COST if float(key_tiles.mean()) < 0.75 * float(key_tiles.max()) else 2 * LONE_TILE_COST
     while spare > 0:
-        longest_run, i = heapq.heappop(heap)
+        longest_run, i = heap[0]
         if -longest_run * lone_cost <= per_unit:
             break   # the launch is as long as its work by now, not as its longest workgroup
-        if runs[i] >= most or int(key_tiles[i]) // (int(runs[i]) + 1) < MIN_RUN_TILES:
+        if count[i] >= most or tiles[i] // (count[i] + 1) < MIN_RUN_TILES:
             break   # the longest workgroup cannot get shorter
-        runs[i] += 1
+        count[i] += 1
         spare -= 1
-        heapq.heappush(heap, (-share(i), i))
-    longest = int(key_tiles.max())
-    if max(share(i) for i in range(key_tiles.size)) * 20 > longest * 17:
-        runs[:] = 1
-    return runs
+        heapq.heapreplace(heap, (-(-(-tiles[i] // count[i])), i))
+    if -heap[0][0] * 20 > max(tiles) * 17:
+        return runs
+    return np.asarray(count, np.int64)
 
 
 def round_about(order: np.ndarray, per_round: int) -> np.ndarray:
@@ -182,12 +182,12 @@ def list_tiles(q_len: np.ndarray, kv_len: np.ndarray, first_entry: int, rows: in
     tile becomes ``workgroups_per_tile`` workgroups, one per group of query heads) is turned round,
     so that a unit that got a long tile in one round gets a short one in the next. A cut tile is
     listed once per run, each time with its share of the keys."""
-    ent, q0s = [], []
-    for e in range(first_entry, q_len.size):
-        for q0 in range(0, int(q_len[e]), rows):
-            ent.append(e)
-            q0s.append(q0)
-    ent_a, q0_a = np.asarray(ent, np.int32), np.asarray(q0s, np.int32)
+    def counted(counts: np.ndarray) -> np.ndarray:   # 0, 1, .. count - 1 of each
+        return np.arange(int(counts.sum())) - np.repeat(np.cumsum(counts) - counts, counts)
+
+    of_entry = np.maximum(-(-q_len[first_entry:].astype(np.int64) // rows), 0)
+    ent_a = np.repeat(np.arange(first_entry, q_len.size, dtype=np.int32), of_entry)
+    q0_a = (counted(of_entry) * rows).astype(np.int32)
     if ent_a.size == 0:
         return ent_a, q0_a, None, 0, 0
     length = q_len[ent_a].astype(np.int64)
@@ -202,7 +202,7 @@ def list_tiles(q_len: np.ndarray, kv_len: np.ndarray, first_entry: int, rows: in
         return ent_a[order], q0_a[order], None, 0, 0
     # the list's entries: a tile once per run, each with its share of the keys
     which = np.repeat(np.arange(ent_a.size), runs)
-    run = np.concatenate([np.arange(r) for r in runs])
+    run = counted(runs)
     place = np.cumsum(cut) - 1                       # the cut tiles numbered in list order
     code = np.where(cut[which], run | runs[which] << 4 | place[which] << 8, -1)
     share = -(-key_tiles[which] // runs[which])
@@ -211,9 +211,10 @@ def list_tiles(q_len: np.ndarray, kv_len: np.ndarray, first_entry: int, rows: in
 
 
 def prefill_tiles(ctx: Any, head_dim: int, q_heads: int, kv_heads: int, first_entry: int, device: torch.device,
-                  window: int = 0) -> PrefillTiles:
+                  window: int = 0, pieces: Optional["ChunkPieces"] = None) -> PrefillTiles:
     """The tile list of the step's portions for :func:`ops.attention_prefill` (made once per step
-    and shape; the buffers of the cut tiles serve every layer of that shape in turn)."""
+    and shape; the buffers of the cut tiles serve every layer of that shape in turn). ``pieces``: of these in place
+    of the entries."""
     rows = ops.attention_prefill_tile_rows(head_dim, q_heads, kv_heads)
     units = ops.compute_units(device)
     cut_floats = ops.attention_prefill_cut_floats(head_dim, q_heads, kv_heads)
@@ -223,9 +224,10 @@ def prefill_tiles(ctx: Any, head_dim: int, q_heads: int, kv_heads: int, first_en
     may_cut = window == 0 and cut_floats > 0
 
     def make() -> PrefillTiles:
-        q_len = (ctx.q_start_host[1:] - ctx.q_start_host[:-1]).astype(np.int64)
-        ent, q0, code, n_cut, room = list_tiles(q_len, np.asarray(ctx.kv_len_host), first_entry, rows, per_tile,
-                                                units, may_cut)
+        q_start, kv_len, first = ((ctx.q_start_host, np.asarray(ctx.kv_len_host), first_entry) if pieces is None
+                                  else (pieces.q_start_host, pieces.kv_len_host, 0))
+        q_len = (q_start[1:] - q_start[:-1]).astype(np.int64)
+        ent, q0, code, n_cut, room = list_tiles(q_len, kv_len, first, rows, per_tile, units, may_cut)
         if code is None:
             return PrefillTiles(*ctx.upload([ent, q0]))
         entry_t, q0_t, code_t = ctx.upload([ent, q0, code])
@@ -233,7 +235,86 @@ def prefill_tiles(ctx: Any, head_dim: int, q_heads: int, kv_heads: int, first_en
                             torch.empty(n_cut * room * cut_floats, device=device, dtype=torch.float32),
                             torch.zeros(n_cut * q_heads, device=device, dtype=torch.int32))
 
-    return ctx.step_lists(("prefill tiles", rows, per_tile, first_entry, may_cut), make)
+    return ctx.step_lists(("prefill tiles", rows, per_tile, first_entry, may_cut, 0 if pieces is None else pieces.chunk), make)
+
+
+def chunk_pieces(q_start: np.ndarray, kv_len: np.ndarray, first_entry: int, chunk: int) -> tuple[np.ndarray, ...]:
+    """The portions ``first_entry..`` of a step under a chunked mask as pieces that are causal by themselves: the rows of an
+    entry that lie in one chunk see that chunk's keys and no others. Returns each piece's entry, its first key's position, where its rows
+    begin (and the last one's end) and how many keys it has."""
+    entry, first_key, begin, keys = [], [], [], []
+    for e in range(first_entry, kv_len.size):
+        row, end, pos = int(q_start[e]), int(q_start[e + 1]), int(kv_len[e]) - int(q_start[e + 1] - q_start[e])
+        while row < end:
+            low = pos // chunk * chunk
+            n = min(end - row, low + chunk - pos)
+            entry.append(e)
+            first_key.append(low)
+            begin.append(row)
+            keys.append(pos + n - low)
+            row, pos = row + n, pos + n
+    begin.append(int(q_start[-1]))
+    return tuple(np.asarray(a, np.int32) for a in (entry, first_key, begin, keys))
+
+
+class ChunkPieces:
+    """:func:`chunk_pieces` of a step on the device, with each piece's pages."""
+
+    def __init__(self, ctx: Any, grp: Any, first_entry: int, chunk: int) -> None:
+        entry, first_key, self.q_start_host, self.kv_len_host = chunk_pieces(ctx.q_start_host, np.asarray(ctx.kv_len_host), first_entry, chunk)
+        self.chunk = chunk
+        width = max(1, -(-int(self.kv_len_host.max()) // ctx.page_size))
+        at = np.minimum(first_key[:, None] // ctx.page_size + np.arange(width, dtype=np.int32), grp.block_tables.shape[1] - 1)
+        self.q_start, self.kv_len, where = ctx.upload([self.q_start_host, self.kv_len_host, entry[:, None] * grp.block_tables.shape[1] + at])
+        self.block_tables = grp.block_tables.view(-1)[where]
+
+
+# Pairs of a query head's row and a key from which a step's portions take that kernel. Below, the lists of its tiles, which the host makes
+# while the step's first kernels wait to be launched, cost as much as it gives. Prompts, all other kernels of the step included, us, the
+# kernel for changed scores and this one (millions of pairs): Miberax 1,024 wide 1 x 1,500 (17) 2,487 2,594, 4 x 1,400 (60) 4,536
+# 4,399; 2,048 wide 1 x 1,600 (39) 3,936 3,803, 1 x 2,048 (64) 5,010 4,508, 1 x 6,000 11,645 10,715; Rurorax 1,024 wide 1 x 2,000 (31) 1,803
+# 1,969, 2 x 1,500 (34) 2,077 2,056, 2 x 2,900 (91) 3,306 3,217; 2,048 wide 1 x 4,096 (256) 6,030 5,740; Betepel 1,024 wide 3 x 700 (11)
+# 2,272 2,458.
+PLAIN_FROM_PAIRS = 36 << 20
+
+
+def plain_portions(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, out: torch.Tensor, ctx: Any, cache: Any,
+                   q_heads: int, scale: float, *, chunk: int = 0, window: int = 0, keep_first: int = 0) -> bool:
+    """The attention of the step's portions by the kernel that shares key tiles through LDS, where a chunked mask or a
+    window is all that changes it: under a mask that no row of the step meets, a window that keeps no first positions, or
+    chunks of whole pages, whose rows are entries by themselves. False (nothing has run) elsewhere. (The kernel for
+    changed scores takes blocks of 64 keys by way of registers, one barrier a block: a prompt of 4,096 tokens in chunks of 2,048, 32
+    heads of 64 on 8, 149 us a layer and 75.)"""
+    def make() -> Optional[tuple]:
+        grp, nd = ctx.groups[cache.group], ctx.num_decode
+        pages, kv_heads, page_size, head_dim = k_pages.shape
+        if (tuple(v_pages.shape) != (pages, kv_heads, head_dim, page_size) or scale <= 0.0
+                or not ops.attention_mfma_supports(head_dim, page_size, k_pages.dtype)):
+            return None
+        new, keys = np.diff(ctx.q_start_host)[nd:].astype(np.int64), np.asarray(ctx.kv_len_host)[nd:].astype(np.int64)
+        seen = np.minimum(keys, max(chunk, window)) if chunk or window else keys   # (by the last row, or one in the middle)
+        if q_heads * int((new * np.minimum(seen, keys - new // 2)).sum()) < PLAIN_FROM_PAIRS:
+            return None
+        longest = int(keys.max())
+        met_chunk, met_window = (n if 0 < n < longest else 0 for n in (chunk, window))
+        if met_window and (keep_first or met_chunk) or met_chunk % page_size:
+            return None
+        if not met_chunk:
+            return ctx.q_start, ctx.kv_len, grp.block_tables, prefill_tiles(ctx, head_dim, q_heads, kv_heads, nd, q.device, met_window), met_window
+        pieces = ctx.step_lists(("chunk pieces", met_chunk, nd, cache.group), lambda: ChunkPieces(ctx, grp, nd, met_chunk))
+        return (pieces.q_start, pieces.kv_len, pieces.block_tables,
+                prefill_tiles(ctx, head_dim, q_heads, kv_heads, nd, q.device, 0, pieces), 0)
+
+    if out.dtype != k_pages.dtype:
+        return False
+    # (asked once a step: a step of few tokens waits for its launches, and layers are alike)
+    plan = ctx.step_lists(("plain portions", q_heads, tuple(k_pages.shape), tuple(v_pages.shape), cache.group, scale, chunk, window, keep_first), make)
+    if plan is None:
+        return False
+    q_start, kv_len, tables, t, met_window = plan
+    ops.attention_prefill(q, k_pages, v_pages, out, q_start, kv_len, tables, t.entry, t.q0, q_heads, scale, met_window, t.cut, t.cut_tiles,
+                          t.cut_room, t.cut_buf, t.cut_count)
+    return True
 
 
 def paged_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, out: torch.Tensor,

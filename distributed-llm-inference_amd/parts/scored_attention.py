@@ -51,6 +51,7 @@ from typing import Any, Mapping, Optional
 import torch
 
 from ..kernels import ops
+from .attention_kernels import plain_portions
 from .base import Mixer, PagedKVSpec, PositionEncoding, Runtime
 from .linear import as_operand, linear_f32, stack_rows
 from .registry import build_part, register_part
@@ -89,6 +90,10 @@ def paged_scored_attention(rt: Runtime, ctx: Any, cache: Any, q: torch.Tensor, o
             ops.attention_scored(q[:nd], cache.k_pages, cache.v_pages, out[:nd], ctx.q_start[:nd + 1], ctx.kv_len[:nd],
                                  grp.block_tables[:nd], None, None, num_heads, scale,
                                  gate=None if gate is None else gate[:nd], **changes)
+        masks = {n: changes.get(n) or 0 for n in ("chunk", "window", "keep_first")}
+        if gate is None and not _changes_beside(masks, changes) and plain_portions(q, cache.k_pages, cache.v_pages, out, ctx, cache, num_heads,
+                                                                                    scale, **masks):
+            return
         if ops.attention_grouped_supports(head_dim, value_dim, ctx.page_size, rt.dtype):
             tiles = ctx.q_tiles(ops.attention_grouped_tile_tokens(num_heads, cache.k_pages.shape[1]), first_entry=nd)
             ops.attention_grouped(q, cache.k_pages, cache.v_pages, out, ctx.q_start, ctx.kv_len, grp.block_tables, tiles[0], tiles[1],
@@ -103,12 +108,15 @@ def paged_scored_attention(rt: Runtime, ctx: Any, cache: Any, q: torch.Tensor, o
                              tiles[0], tiles[1], num_heads, scale, gate=gate, **changes)
 
 
+def _changes_beside(named: Any, changes: Mapping[str, Any]) -> bool:
+    """Whether anything but what is named changes the scores."""
+    return any(bool(v) if not isinstance(v, torch.Tensor) else True for n, v in changes.items() if n not in named and v is not None)
+
+
 def _keyvalue_takes(rt: Runtime, head_dim: int, value_dim: int, out: torch.Tensor, changes: Mapping[str, Any]) -> bool:
     """Whether the matrix-core kernel for values that are keys computes this attention: its sizes, and no change to
     the scores but a window and a sink per head."""
-    others = any(bool(v) if not isinstance(v, torch.Tensor) else True
-                 for n, v in changes.items() if n not in ("window", "sinks") and v is not None)
-    return not others and out.dtype == rt.dtype and ops.attention_keyvalue_supports(head_dim, value_dim, rt.dtype)
+    return not _changes_beside(("window", "sinks"), changes) and out.dtype == rt.dtype and ops.attention_keyvalue_supports(head_dim, value_dim, rt.dtype)
 
 
 @register_part("mixer", "scored_attention")

@@ -1,0 +1,72 @@
+"""Portions whose mask is all that changes their attention: the kernel that shares key tiles against the one for changed scores."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+class _Cache:
+    def __init__(self, k, v):
+        self.group, self.k_pages, self.v_pages = 0, k, v
+
+
+def _context(page, old, new, decode):
+    """A step of `decode` single tokens and then portions, over pages in no order."""
+    from dli_amd.engine.batch import GroupView, StepContext
+
+    kv = np.asarray(old, np.int32) + np.asarray(new, np.int32)
+    q_start = np.concatenate([[0], np.cumsum(new)]).astype(np.int32)
+    width = int(-(-kv.max() // page)) + 1
+    tables = np.random.default_rng(1).permutation(len(new) * width).reshape(len(new), width).astype(np.int32)
+    on = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    empty = torch.zeros(0, dtype=torch.int32, device="cuda")
+    positions = np.concatenate([np.arange(o, o + n) for o, n in zip(old, new)]).astype(np.int32)
+    ctx = StepContext(device=torch.device("cuda"), page_size=page, num_tokens=int(q_start[-1]), num_entries=len(new), num_decode=decode,
+                      token_ids=empty, positions=on(positions), q_start=on(q_start), kv_len=on(kv), state_slots=empty, logit_rows=empty,
+                      groups=[GroupView(empty, on(tables), width)], q_start_host=q_start, kv_len_host=kv)
+    return ctx, len(new) * width
+
+
+# chunks that are met and not, whose edges rows and cached keys lie on and beside, one key a piece; windows met, not met, and not met beside kept
+# positions; heads of all kinds that share tiles; pages of one tile and of several; single tokens in front
+@pytest.mark.parametrize("masks,page", [({"chunk": 64}, 16), ({"chunk": 192}, 32), ({"chunk": 4096}, 16), ({"window": 100}, 16), ({}, 64),
+                                        ({"window": 4096, "keep_first": 4}, 16), ({"chunk": 64, "window": 4096}, 16)])
+@pytest.mark.parametrize("heads,kv,dim", [(4, 1, 64), (8, 8, 64), (6, 2, 128), (3, 3, 48)])
+def test_same_results(monkeypatch, masks, page, heads, kv, dim):
+    from dli_amd.kernels import ops
+    from dli_amd.parts import attention_kernels as A
+
+    monkeypatch.setattr(A, "PLAIN_FROM_PAIRS", 0)
+    old, new = [70, 0, 63, 64, 65, 0, 130], [1, 200, 1, 64, 63, 3, 700]
+    ctx, pages = _context(page, old, new, 1)
+    gen = torch.Generator(device="cuda").manual_seed(heads + page)
+    draw = lambda *s: torch.randn(*s, device="cuda", generator=gen).bfloat16()
+    n = ctx.num_tokens
+    q, k, v = draw(n, heads * dim), draw(pages, kv, page, dim), draw(pages, kv, dim, page)
+    got, want = torch.zeros(n, heads * dim, device="cuda").bfloat16(), torch.zeros(n, heads * dim, device="cuda").bfloat16()
+    assert A.plain_portions(q, k, v, got, ctx, _Cache(k, v), heads, dim ** -0.5, **masks)
+    tiles = ctx.q_tiles(ops.attention_grouped_tile_tokens(heads, kv), first_entry=1)
+    ops.attention_grouped(q, k, v, want, ctx.q_start, ctx.kv_len, ctx.groups[0].block_tables, tiles[0], tiles[1], heads, dim ** -0.5, **masks)
+    # weights are rounded to bfloat16 (2^-9 each at most) against one reference point or another, and the results once more
+    assert (got[1:].float() - want[1:].float()).abs().max() <= 3 * 2.0 ** -9 * want.float().abs().max()
+    assert not got[0].any()   # the single token's row is another kernel's
+
+
+def test_what_stays_with_the_kernel_for_changed_scores(monkeypatch):
+    from dli_amd.parts import attention_kernels as A
+
+    monkeypatch.setattr(A, "PLAIN_FROM_PAIRS", 0)
+
+    def takes(page=16, v_dim=64, out=torch.bfloat16, scale=0.125, **masks):
+        ctx, pages = _context(page, [0], [300], 0)
+        k, v = torch.zeros(pages, 2, page, 64, device="cuda").bfloat16(), torch.zeros(pages, 2, v_dim, page, device="cuda").bfloat16()
+        q = torch.zeros(300, 256, device="cuda").bfloat16()
+        return A.plain_portions(q, k, v, torch.zeros(300, 4 * v_dim, device="cuda", dtype=out), ctx, _Cache(k, v), 4, scale, **masks)
+
+    assert takes() and takes(chunk=64)
+    assert not any([takes(chunk=40), takes(page=8), takes(v_dim=32), takes(out=torch.float32), takes(scale=-0.125), takes(window=64, keep_first=4),
+                    takes(chunk=64, window=100)])
+    monkeypatch.setattr(A, "PLAIN_FROM_PAIRS", 4 * 300 * 151)
+    assert not takes()

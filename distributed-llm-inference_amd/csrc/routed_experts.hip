@@ -416,16 +416,62 @@ __device__ __forceinline__ exm_bf16x8 exm_load(const bf16_t* p) { return *reinte
 // 117 (6.0 TB/s); 8 of 2,048 on 4,096, 1 row (67 MB) 72.5 -> 17.3. Four chunks ahead: the same.
 #define EXF_K 256
 #define EXF_AHEAD 3
-template <bool UP>
-__global__ __launch_bounds__(256) void expert_few_kernel(ExpertArgs p, const bf16_t* __restrict__ x, int64_t x_stride,
+// Up to as many choices as a wave has lanes: every workgroup sorts them for itself, a choice a lane, and no kernel does it before (which
+// took 4.5 us of a step of two rows with eight choices, this 0.7 to 1.3 in each of the two products).
+#define EXF_SLOTS DLI_WAVE
+struct FewChoices {
+  int* ids; TableChoice choice;   // choice.table: looked up, and written to ids with the weights by the first workgroup of the up product
+  int slots, experts;
+};
+// Tile `tile`: its expert, first sorted row and the last's end; -1 where there are not so many. order[sorted row]: the slot (every wave
+// leaves all of it). Inside an expert's run the rows come in the order of their slots.
+__device__ __forceinline__ int few_tile(const FewChoices& f, bool writes, int tile, int* order, int& r0, int& rend) {
+  const int lane = threadIdx.x % DLI_WAVE, slot = min(lane, f.slots - 1);
+  const int chosen = f.choice.table != nullptr ? table_choice(f.choice.table, f.choice.token_ids, f.choice.vocab, f.choice.top, slot) : f.ids[slot];
+  if (writes && (int)threadIdx.x < f.slots) {
+    f.ids[slot] = chosen;
+    f.choice.weights[slot] = 1.f / (float)f.choice.top;
+  }
+  const int e = lane < f.slots && chosen >= 0 && chosen < f.experts ? chosen : f.experts;   // (those without rows behind all others)
+  int before = 0, among = 0;                                    // sorted rows before this one, and of its own expert
+  for (int j = 0; j < f.slots; ++j) {
+    const int other = __builtin_amdgcn_readlane(e, j);
+    before += other < e || (other == e && j < lane) ? 1 : 0;
+    among += other == e && j < lane ? 1 : 0;
+  }
+  const bool live = e < f.experts, first = live && among % EXM_FEW == 0;
+  int tiles = 0;                                                // before this row's
+  for (unsigned long long left = __ballot(first); left != 0; left &= left - 1)
+    tiles += __builtin_amdgcn_readlane(before, __builtin_ctzll(left)) < before ? 1 : 0;
+  if (live) order[before] = lane;
+  const unsigned long long mine = __ballot(first && tiles == tile);
+  if (mine == 0) return -1;
+  const int at = __builtin_ctzll(mine), expert = __builtin_amdgcn_readlane(e, at);
+  r0 = __builtin_amdgcn_readlane(before, at);
+  rend = min(r0 + EXM_FEW, r0 - __builtin_amdgcn_readlane(among, at) + (int)__popcll(__ballot(e == expert)));
+  return expert;
+}
+
+template <bool UP, bool SORTS>
+__global__ __launch_bounds__(256) void expert_few_kernel(ExpertArgs p, FewChoices choices, const bf16_t* __restrict__ x, int64_t x_stride,
                                                          const bf16_t* __restrict__ w0, const bf16_t* __restrict__ w1,
                                                          bf16_t* __restrict__ y, float* __restrict__ z, float limit, float alpha,
                                                          float up_shift) {
   const int tile = blockIdx.x;
-  if (tile >= p.tile_count[0]) return;
   __shared__ __attribute__((aligned(16))) bf16_t sm[2][48][EXF_K];
   __shared__ __attribute__((aligned(16))) float up_sums[64][4];
-  const int e = p.tile_expert[tile], r0 = p.tile_row0[tile], rend = min(p.offsets[e + 1], r0 + 16);
+  __shared__ int sorted[SORTS ? EXF_SLOTS : 1];
+  int e, r0, rend;
+  if constexpr (SORTS) {
+    e = few_tile(choices, UP && choices.choice.table != nullptr && blockIdx.x == 0 && blockIdx.y == 0, tile, sorted, r0, rend);
+    if (e < 0) return;
+  } else {
+    if (tile >= p.tile_count[0]) return;
+    e = p.tile_expert[tile];
+    r0 = p.tile_row0[tile];
+    rend = min(p.offsets[e + 1], r0 + 16);
+  }
+  const auto slot_of = [&](int r) { return SORTS ? sorted[r] : p.order[r]; };
   const int depth = UP ? p.width : p.ff, features = UP ? p.ff : p.width, n0 = blockIdx.y * (UP ? 16 : 32);
   const int at_row = threadIdx.x / 32, at = threadIdx.x % 32;
   const bf16_t* src[6];
@@ -437,7 +483,7 @@ __global__ __launch_bounds__(256) void expert_few_kernel(ExpertArgs p, const bf1
 #pragma unroll
   for (int i = 0; i < 2; ++i) {                                                  // (a row past the end repeats the last)
     const int r = min(r0 + at_row + 8 * i, rend - 1);
-    src[4 + i] = x + (int64_t)(UP ? p.order[r] / p.top : r) * x_stride;
+    src[4 + i] = x + (int64_t)(UP ? slot_of(r) / p.top : r) * x_stride;
   }
   const int lane = threadIdx.x % DLI_WAVE, wave = threadIdx.x / DLI_WAVE, c = lane % 16, g = lane / 16;
   const int chunks = (depth + EXF_K - 1) / EXF_K;
@@ -488,11 +534,11 @@ __global__ __launch_bounds__(256) void expert_few_kernel(ExpertArgs p, const bf1
   const int r = r0 + c, n = n0 + (UP ? 0 : 16 * wave) + 4 * g;
   if (wave >= (UP ? 1 : 2) || r >= rend || n >= features) return;               // (features come in fours)
   if (UP) {
-    const float iw = p.in_weight != nullptr ? p.in_weight[p.order[r]] : 1.f;
+    const float iw = p.in_weight != nullptr ? p.in_weight[slot_of(r)] : 1.f;
     const exm_float4 up = *reinterpret_cast<const exm_float4*>(up_sums[lane]);
     for (int i = 0; i < 4; ++i) y[(int64_t)r * p.ff + n + i] = (bf16_t)clamped_glu(iw * acc[i], iw * up[i], limit, alpha, up_shift);
   } else {
-    const int64_t slot = p.order[r];
+    const int64_t slot = slot_of(r);
     for (int i = 0; i < 4; ++i) z[slot * p.width + n + i] = acc[i];
   }
 }
@@ -976,13 +1022,21 @@ int dli_expert_products(int* ids, const int* table, const int* token_ids, int vo
     if (dli_table_choose(table, token_ids, rows, top, vocab, ids, weights, stream) != DLI_OK) return DLI_ERR_LAUNCH;
     choice.table = nullptr;
   }
+  ExpertArgs p;
+  p.tile_expert = tile_expert; p.tile_row0 = tile_row0; p.tile_count = tile_count; p.offsets = offsets; p.order = order;
+  p.top = top; p.width = width; p.ff = ff; p.in_weight = in_weight;
+  if (mfma && slots <= EXF_SLOTS && !expert_tiled(slots, experts, width, ff, is_bf16) && expert_few(slots, experts, width, ff)) {
+    const FewChoices choices = {ids, choice, (int)slots, experts}, chosen = {ids, {nullptr, nullptr, 0, top, nullptr}, (int)slots, experts};
+    expert_few_kernel<true, true><<<dim3(max_tiles, (ff + 15) / 16), 256, 0, stream>>>(p, choices, (const bf16_t*)h, h_stride, (const bf16_t*)w_gate,
+                                                                                       (const bf16_t*)w_up, (bf16_t*)y, nullptr, limit, alpha, up_shift);
+    expert_few_kernel<false, true><<<dim3(max_tiles, (width + 31) / 32), 256, 0, stream>>>(p, chosen, (const bf16_t*)y, ff, (const bf16_t*)w_down,
+                                                                                           nullptr, nullptr, z, 0.f, 0.f, 0.f);
+    return dli_launch_status();
+  }
   expert_sort_kernel<<<1, 1024, 2 * experts * sizeof(int), stream>>>(ids, choice, (int)slots, experts, offsets, order, tile_expert,
                                                                      tile_row0, tile_count, max_tiles,
                                                                      dli_expert_tile_rows(slots, experts, width, ff, is_bf16));
   if (dli_launch_status() != DLI_OK) return DLI_ERR_LAUNCH;
-  ExpertArgs p;
-  p.tile_expert = tile_expert; p.tile_row0 = tile_row0; p.tile_count = tile_count; p.offsets = offsets; p.order = order;
-  p.top = top; p.width = width; p.ff = ff; p.in_weight = in_weight;
   if (expert_tiled(slots, experts, width, ff, is_bf16)) {
     const unsigned tiles8 = 8 * ((max_tiles + 7) / 8);
     if ((int64_t)tiles8 * (ff / 64 + width / 128) > 0x7fffffff || ((uintptr_t)z % 16)) return DLI_ERR_ARGUMENT;
@@ -993,9 +1047,9 @@ int dli_expert_products(int* ids, const int* table, const int* token_ids, int vo
     return dli_launch_status();
   }
   if (mfma && expert_few(slots, experts, width, ff)) {
-    expert_few_kernel<true><<<dim3(max_tiles, (ff + 15) / 16), 256, 0, stream>>>(p, (const bf16_t*)h, h_stride, (const bf16_t*)w_gate,
+    expert_few_kernel<true, false><<<dim3(max_tiles, (ff + 15) / 16), 256, 0, stream>>>(p, FewChoices(), (const bf16_t*)h, h_stride, (const bf16_t*)w_gate,
                                                                                  (const bf16_t*)w_up, (bf16_t*)y, nullptr, limit, alpha, up_shift);
-    expert_few_kernel<false><<<dim3(max_tiles, (width + 31) / 32), 256, 0, stream>>>(p, (const bf16_t*)y, ff, (const bf16_t*)w_down, nullptr,
+    expert_few_kernel<false, false><<<dim3(max_tiles, (width + 31) / 32), 256, 0, stream>>>(p, FewChoices(), (const bf16_t*)y, ff, (const bf16_t*)w_down, nullptr,
                                                                                      nullptr, z, 0.f, 0.f, 0.f);
     return dli_launch_status();
   }

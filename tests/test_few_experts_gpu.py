@@ -72,3 +72,30 @@ def test_shared_expert(rows, k, ff):
     # gate, up and their product round to 2^-9 of up to three, some the other way (2^-8), summed with weights of ff^-0.5; the
     # identity expert's row is the input, the sums stay 32-bit
     assert (got - want).abs().max() < 2 ** -8 * 3 * 4
+
+
+# choices a wave sorts for itself: one, a token's, as many as there are lanes; an expert with more than a tile's rows, experts without rows,
+# choices that have none (identity experts), nothing but those
+@pytest.mark.parametrize("rows", [1, 3, 16])
+@pytest.mark.parametrize("kind", ["spread", "one", "identity", "none"])
+@pytest.mark.parametrize("table", [False, True])
+def test_choices_sorted_on_the_way(ops, rows, kind, table):
+    experts, top, width, ff, vocab = 8, 4, 96, 64, 40
+    gen = torch.Generator().manual_seed(rows)
+    most = {"spread": experts, "one": 1, "identity": experts + 4, "none": experts}[kind]
+    choices = torch.randint(0, most, (vocab, top), generator=gen, dtype=torch.int32) + (experts if kind == "none" else 0)
+    tokens = torch.randint(0, vocab, (rows + 20,), generator=gen, dtype=torch.int32)
+    w_gate, w_up, w_down = ((torch.randn(experts, *s, generator=gen) * s[1] ** -0.5).bfloat16().cuda() for s in ((ff, width), (ff, width), (width, ff)))
+    h = torch.randn(rows + 20, width, generator=gen).bfloat16().cuda()
+
+    def run(n):
+        ids = choices[tokens[:n].long()].cuda()
+        given = torch.full_like(ids, -7) if table else ids.clone()
+        weights = torch.zeros(n, top, device="cuda")
+        z = ops.expert_products(given, h[:n], w_gate, w_up, w_down, 7.0, 1.702, 1.0,
+                                choose=(choices.cuda(), tokens[:n].cuda(), weights) if table else None)
+        assert torch.equal(given, ids) and (not table or (weights == 1 / top).all())
+        real = (ids < experts).reshape(-1)
+        return z[:rows * top][real[:rows * top]]
+
+    assert torch.equal(run(rows), run(rows + 20))   # (80 choices and more: sorted by a kernel of its own)

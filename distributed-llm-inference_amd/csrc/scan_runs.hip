@@ -4,30 +4,31 @@
 // sums with a bonus, at one instruction every four to five cycles); cut into runs the chip's waves are full. A run's effect
 // on the state before it is linear, S_after = M S_before + E, o_t = o_t(from zero) + S_before^T y_t, so:
 //
-//   walk     every run token by token, from a state of zeros (an entry's first run from the request's own, which makes
-//            its results final): o and E. Where the rule mixes keys (RUNS_DELTA, RUNS_GATED) 64 more columns start from the unit
+//   walk     every run token by token (RUNS_GATED: sixteen at a time, on the matrix cores), from a state of zeros (an entry's
+//            first run from the request's own, which makes its results final): o and E. Where the rule mixes keys (RUNS_DELTA, RUNS_GATED) 64 more columns start from the unit
 //            matrix and take no input: they end as M, and their outputs are y. Where it does not (RUNS_BONUS), M is the
 //            product of the run's decays per key and y_t = r_t times their product before t.
 //   carry    per request and head the states between the runs, one after the other: E_s <- M_s E_(s-1) + E_s on the matrix
 //            cores (v_mfma_f32_16x16x4_f32); the last one is the request's new state.
 //   finish   o_t += E_(s-1)^T y_t on the matrix cores, and in the same pass the per-head norm and gate where the rule has them.
 //
-// walk: a workgroup of four waves takes one (run, head) and 64 columns, values or unit matrix; sixteen lanes (a DPP row) share
-// four columns and hold four keys of each, so that five 16-byte reads of LDS a token serve sixteen columns (with one column
+// walk, token by token: a workgroup of four waves takes one (run, head) and 64 columns, values or unit matrix; sixteen lanes
+// (a DPP row) share four columns and hold four keys of each, so that five 16-byte reads of LDS a token serve sixteen columns (with one column
 // a lane, as token by token, LDS is what bounds it). The vectors of sixteen tokens are staged by the workgroup, the next
 // sixteen are on their way meanwhile. What bounds it: vector instructions, some 75 to 110 a token and wave at four cycles each (110 to 130
 // while a sum over the lanes took each column by itself: the walk of one prompt of 2,048 tokens 133 -> 108 us RUNS_DELTA, 54 -> 49
-// RUNS_BONUS, of four prompts, 2,990 tokens, 168 -> 125 RUNS_GATED, and as far from 64 bits or less).
+// RUNS_BONUS, and as far from 64 bits or less).
 //
 // Measured (one prompt of 2,048 tokens, 32 heads, walk + carry + finish, us): RUNS_DELTA 108 + 15 + 21 against 578 and 17 for
-// the norm, RUNS_BONUS 49 + 8 + 17 against 378 and 17, RUNS_GATED 117 in all against 410. Where the cut lies: ops.scan_runs.
-// Beside 255 single tokens, which keep the kernel of steps of single tokens: 245, 168 and 183 us a layer (5,150, 2,880 and 2,610 token
-// by token; 1,048, 1,301 and 818 with every entry cut and the launch as large as the longest entry times the entries).
+// the norm, RUNS_BONUS 49 + 8 + 17 against 378 and 17, RUNS_GATED 90 in all against 410. Where the cut lies: ops.scan_runs.
+// Beside 255 single tokens, which keep the kernel of steps of single tokens: 245, 168 and (walked token by token then) 183 us a
+// layer (5,150, 2,880 and 2,610 token by token; 1,048, 1,301 and 818 with every entry cut and the launch as large as the longest entry times the entries).
 // Distance from the rules in 64 bits against token by token (2-norm; 300 to 4,096 tokens, 8 to 32 heads, every row of outputs and
-// the state left): 0.99 to 1.00 times as far RUNS_DELTA, 1.01 to 1.03 RUNS_BONUS, 0.97 to 1.04 RUNS_GATED, 4e-8 to 2e-7 either way.
+// the state left): 0.99 to 1.00 times as far RUNS_DELTA, 1.01 to 1.03 RUNS_BONUS, 4e-8 to 2e-7 either way.
 #include "scan_runs.h"
 
 typedef float rf4 __attribute__((ext_vector_type(4)));
+typedef double rd4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float runs_row_sum(float x) {   // over the sixteen lanes of a DPP row
   x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0xB1, 0xF, 0xF, false));
@@ -94,8 +95,7 @@ __device__ __forceinline__ int runs_before(const RunsArgs& p, int entry) {
 template <int RULE>
 __global__ __launch_bounds__(256) void scan_runs_walk_kernel(RunsArgs p) {
   constexpr int D = 64, TB = 16;
-  __shared__ rf4 sk[TB * 16], sr[TB * 16], sv[TB * 16], sw[RULE == RUNS_GATED ? 1 : TB * 16], sc[RULE == RUNS_DELTA ? TB * 16 : 1];
-  __shared__ float sg[RULE == RUNS_GATED ? 2 * TB : 1];
+  __shared__ rf4 sk[TB * 16], sr[TB * 16], sv[TB * 16], sw[TB * 16], sc[RULE == RUNS_DELTA ? TB * 16 : 1];
   const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, vloc = lane / 16, part = lane % 16;
   const RunsPlace place = runs_place(p, blockIdx.y);
   const int entry = place.entry, run = place.run, first = place.first, row0 = place.row0, n = place.n, head = blockIdx.x;
@@ -123,18 +123,12 @@ __global__ __launch_bounds__(256) void scan_runs_walk_kernel(RunsArgs p) {
   // staging: sixteen threads a token, four values each
   const int bt = tid / 16, bc = tid % 16 * 4;
   rf4 fk, fr, fv = {0.f, 0.f, 0.f, 0.f}, fw, fa;
-  float fb = 0.f, fg = 0.f;
   const auto fetch = [&](int t0) {
     const int64_t row = row0 + min(t0 + bt, n - 1);
     fk = *reinterpret_cast<const rf4*>(p.k + row * p.k_stride + qk_col + bc);
     fr = *reinterpret_cast<const rf4*>(p.r + row * p.r_stride + qk_col + bc);
     if (!unit) fv = *reinterpret_cast<const rf4*>(p.v + row * p.v_stride + v_col + bc);
-    if constexpr (RULE == RUNS_GATED) {
-      fb = p.w[row * p.w_stride + head];
-      fg = p.w[row * p.w_stride + p.heads + head];
-    } else {
-      fw = *reinterpret_cast<const rf4*>(p.w + row * p.w_stride + v_col + bc);
-    }
+    fw = *reinterpret_cast<const rf4*>(p.w + row * p.w_stride + v_col + bc);
     if constexpr (RULE == RUNS_DELTA) fa = *reinterpret_cast<const rf4*>(p.a + row * p.a_stride + v_col + bc);
   };
   const int64_t dst_stride = unit ? (int64_t)p.heads * D : p.o_stride;
@@ -167,21 +161,12 @@ __global__ __launch_bounds__(256) void scan_runs_walk_kernel(RunsArgs p) {
         us[c] = fmaf(k[3], s[3][c], fmaf(k[2], s[2][c], fmaf(k[1], s[1][c], k[0] * s[0][c])));
       }
       const float us_own = runs_own_sum(us);
-      if constexpr (RULE == RUNS_DELTA) {
-        const rf4 w = sw[t * 16 + part], a = sc[t * 16 + part], v = runs_to_columns(v_own);
-        us = runs_to_columns(us_own);
+      const rf4 w = sw[t * 16 + part], a = sc[t * 16 + part], v = runs_to_columns(v_own);
+      us = runs_to_columns(us_own);
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
+      for (int c = 0; c < 4; ++c)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) s[i][c] = fmaf(w[i], s[i][c], fmaf(k[i], v[c], -a[i] * us[c]));
-      } else {
-        const float g = sg[2 * t], bg = sg[2 * t + 1];   // g and beta g; v comes times beta
-        const rf4 u = runs_to_columns(fmaf(-bg, us_own, v_own));
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) s[i][c] = fmaf(k[i], u[c], g * s[i][c]);
-      }
+        for (int i = 0; i < 4; ++i) s[i][c] = fmaf(w[i], s[i][c], fmaf(k[i], v[c], -a[i] * us[c]));
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         o[c] = fmaf(r[3], s[3][c], fmaf(r[2], s[2][c], fmaf(r[1], s[1][c], r[0] * s[0][c])));
@@ -199,16 +184,8 @@ __global__ __launch_bounds__(256) void scan_runs_walk_kernel(RunsArgs p) {
     }
     sk[tid] = fk;
     sr[tid] = fr;
-    if constexpr (RULE == RUNS_GATED) {
-      sv[tid] = fv * fb;
-      if (bc == 0) {
-        sg[2 * bt] = fg;
-        sg[2 * bt + 1] = fb * fg;
-      }
-    } else {
-      sv[tid] = fv;
-      sw[tid] = fw;
-    }
+    sv[tid] = fv;
+    sw[tid] = fw;
     if (t0 + TB < n) fetch(t0 + TB);   // on their way while this batch is walked
     __syncthreads();
     const int nb = min(TB, n - t0);
@@ -232,6 +209,209 @@ __global__ __launch_bounds__(256) void scan_runs_walk_kernel(RunsArgs p) {
 #pragma unroll
   for (int c = 0; c < 4; ++c) *reinterpret_cast<rf4*>(end + column[c] * D + part * 4) = rf4{s[0][c], s[1][c], s[2][c], s[3][c]};
   if (RULE == RUNS_BONUS && wave == 0 && vloc == 0) *reinterpret_cast<rf4*>(p.moves + at + part * 4) = decay;
+}
+
+// The walk of RUNS_GATED, sixteen tokens at a time on the matrix cores (v_mfma_f32_16x16x4_f32, 32-bit products and sums). With S the
+// state before the sixteen, G_t the product of their g up to t, D_ts that of g behind s up to t, b beta:
+//
+//   u_t = b_t (v_t - G_t S^T k_t - sum_(s<t) D_ts (k_t . k_s) u_s)      (forward substitution: four tokens at a time, the others' sums
+//   o_t = G_t S^T r_t + sum_(s<=t) D_ts (r_t . k_s) u_s                  go on as a product)
+//   S  <- G_T S + sum_s D_Ts k_s u_s^T
+//
+// The products of g are made as products, never as quotients, and a factor that is left out is left out by choice and not by a
+// product with zero: what is infinite at a token stays out of the tokens before it. A workgroup of four waves takes one (run, head)
+// and 64 columns, a wave sixteen of them: lane (c, g) holds keys 16 kb + 4 g .. + 3 of column c, which are operands and results of the
+// products as they stand. The dot products of the tokens with each other are made a quarter a wave.
+// What bounds it: 63 products of 32 cycles a wave and sixteen tokens, and four meetings of the workgroup. Token by token, as
+// the other rules are walked (their decays are a value a key), the vector units spent some 80 instructions of four cycles a token
+// and wave: walk, carry and sums of 32 heads, us, four prompts of 2,990 tokens 169 -> 120, one of 2,048 111 -> 90 and of 300 37 -> 30,
+// sixteen of 375 148 -> 112, one of 8,192 368 -> 280. As far from 64 bits as token by token or less
+// (2-norm; 300 to 2,048 tokens, 8 to 32 heads, g near 1, from 0.37 on, from 0.0025 on and with zeros among them, keys alike and not:
+// outputs 0.62 to 1.04 times, before 0.86 to 1.21; the state left 0.82 to 1.08, before 0.97 to 1.18).
+template <int SHIFT>
+__device__ __forceinline__ float runs_before_by(float x) {   // the value SHIFT lanes before in the DPP row, 1 before its first
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0x3f800000, __builtin_bit_cast(int, x), 0x110 + SHIFT, 0xF, 0xF, false));
+}
+template <int SHIFT>
+__device__ __forceinline__ float runs_behind_by(float x) {   // SHIFT lanes behind, 1 past its last
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0x3f800000, __builtin_bit_cast(int, x), 0x100 + SHIFT, 0xF, 0xF, false));
+}
+__device__ __forceinline__ float runs_product_behind(float x) {   // of the lanes behind this one in its DPP row
+  x = runs_behind_by<1>(x);
+  x *= runs_behind_by<1>(x);
+  x *= runs_behind_by<2>(x);
+  x *= runs_behind_by<4>(x);
+  return x * runs_behind_by<8>(x);
+}
+__global__ __launch_bounds__(256, 4) void scan_gated_walk_kernel(RunsArgs p) {
+  constexpr int D = 64, TB = 16, WIDE = 84, SQ = 20;   // (rows of LDS: no two of sixteen lanes' 16-byte reads on one bank)
+  __shared__ __attribute__((aligned(16))) float sk[TB * WIDE], sr[TB * WIDE], keep[TB * SQ], give[TB * SQ];
+  __shared__ __attribute__((aligned(16))) float dots[2][4][TB * SQ];
+  __shared__ __attribute__((aligned(16))) float s_g[TB], s_b[TB], s_bg[TB], s_e[TB];
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, c = lane % 16, g = lane / 16, bt = tid / 16;
+  const RunsPlace place = runs_place(p, blockIdx.y);
+  const int run = place.run, row0 = place.row0, n = place.n, head = blockIdx.x;
+  const bool unit = blockIdx.z != 0;   // the columns of the unit matrix
+  if (n <= 0 || (unit && run == 0)) return;
+  const int col = wave * 16 + c;
+  const int64_t qk_col = (int64_t)(head / p.group) * D, v_col = (int64_t)head * D;
+
+  rf4 s[4];   // keys 16 kb + 4 g + i of the column
+  const bool real = run == 0 && p.positions[place.first] != 0;
+  const float* st = p.state + (int64_t)p.state_slots[place.entry] * p.state_stride + (int64_t)head * D * D;   // [value][key]
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) {
+    rf4 old = {0.f, 0.f, 0.f, 0.f};
+    if (real) old = *reinterpret_cast<const rf4*>(st + col * D + 16 * kb + 4 * g);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[kb][i] = unit ? (16 * kb + 4 * g + i == col ? 1.f : 0.f) : old[i];
+  }
+  rf4 fk, fr, fv = {0.f, 0.f, 0.f, 0.f};
+  float fb = 0.f, fg = 1.f;
+  const auto fetch = [&](int t0) {
+    const int64_t row = row0 + min(t0 + bt, n - 1), token = row0 + min(t0 + c, n - 1);
+    fk = *reinterpret_cast<const rf4*>(p.k + row * p.k_stride + qk_col + 4 * c);
+    fr = *reinterpret_cast<const rf4*>(p.r + row * p.r_stride + qk_col + 4 * c);
+    fb = p.w[token * p.w_stride + head];
+    fg = p.w[token * p.w_stride + p.heads + head];
+    if (!unit)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) fv[i] = p.v[(int64_t)(row0 + min(t0 + 4 * g + i, n - 1)) * p.v_stride + v_col + col];
+  };
+  const int64_t dst_stride = unit ? (int64_t)p.heads * D : p.o_stride;
+  float* dst = (unit ? p.y + (row0 - p.row0) * dst_stride : p.o + row0 * dst_stride) + v_col + col;
+
+  fetch(0);
+  for (int t0 = 0; t0 < n; t0 += TB) {
+    const bool there = t0 + bt < n;   // rows past the last: keys and values of zero, g of one, beta of zero
+    __syncthreads();   // the sixteen before have been walked
+    *reinterpret_cast<rf4*>(&sk[bt * WIDE + 4 * c]) = there ? fk : rf4{0.f, 0.f, 0.f, 0.f};
+    *reinterpret_cast<rf4*>(&sr[bt * WIDE + 4 * c]) = fr;
+    const float decay = t0 + c < n ? fg : 1.f, beta = t0 + c < n ? fb : 0.f;   // token c's
+    float upto = decay;
+    upto *= runs_before_by<1>(upto);
+    upto *= runs_before_by<2>(upto);
+    upto *= runs_before_by<4>(upto);
+    upto *= runs_before_by<8>(upto);
+    const float behind = runs_product_behind(c <= bt ? decay : 1.f);   // D of token bt and token c
+    if (tid < TB) {
+      s_g[c] = upto;
+      s_b[c] = beta;
+      s_bg[c] = beta * upto;
+      s_e[c % 4 * 4 + c / 4] = runs_product_behind(decay);
+    }
+    const float all = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, upto), 15));
+    const rf4 v = fv;
+    if (t0 + TB < n) fetch(t0 + TB);   // on their way while these are walked
+    __syncthreads();
+    {
+      const rf4 kw = *reinterpret_cast<const rf4*>(&sk[c * WIDE + 16 * wave + 4 * g]);
+      const rf4 rw = *reinterpret_cast<const rf4*>(&sr[c * WIDE + 16 * wave + 4 * g]);
+      rd4 kk = {0., 0., 0., 0.}, rk = {0., 0., 0., 0.};   // (in 64-bit: each of them counts in as many sums as there are columns)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        kk = __builtin_amdgcn_mfma_f64_16x16x4f64((double)kw[i], (double)kw[i], kk, 0, 0, 0);
+        rk = __builtin_amdgcn_mfma_f64_16x16x4f64((double)rw[i], (double)kw[i], rk, 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {   // (these results lie in rows g, g + 4, ..)
+        dots[0][wave][(4 * i + g) * SQ + c] = (float)kk[i];
+        dots[1][wave][(4 * i + g) * SQ + c] = (float)rk[i];
+      }
+    }
+    rf4 ks[4], rs[4];   // (sixteen keys a sum, and a tree of these: one sum over all 64 is half again as far from 64 bits)
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+      const rf4 ka = *reinterpret_cast<const rf4*>(&sk[c * WIDE + 16 * kb + 4 * g]);
+      const rf4 ra = *reinterpret_cast<const rf4*>(&sr[c * WIDE + 16 * kb + 4 * g]);
+      ks[kb] = rs[kb] = rf4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        ks[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[i], s[kb][i], ks[kb], 0, 0, 0);
+        rs[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[i], s[kb][i], rs[kb], 0, 0, 0);
+      }
+    }
+    const rf4 from_s = (ks[0] + ks[1]) + (ks[2] + ks[3]);
+    rf4 o = (rs[0] + rs[1]) + (rs[2] + rs[3]);
+    __syncthreads();
+    {
+      const int at = bt * SQ + c;
+      const float kk = (dots[0][0][at] + dots[0][1][at]) + (dots[0][2][at] + dots[0][3][at]);
+      const float rk = (dots[1][0][at] + dots[1][1][at]) + (dots[1][2][at] + dots[1][3][at]);
+      float within = -(s_b[bt] * behind) * kk;
+      asm("" : "+v"(within));   // (made by every lane: behind a branch the reads of LDS would wait for each other)
+      keep[bt * SQ + c] = there && c < bt ? within : 0.f;
+      give[bt * SQ + c % 4 * 4 + c / 4] = c <= bt ? behind * rk : 0.f;   // (a lane's four tokens g, g + 4, .. side by side)
+    }
+    __syncthreads();
+    // A lane's own four tokens to all lanes of its column by way of LDS (in registers it is fourteen instructions a value). What is
+    // taken off v is summed first and u rounded once at its own size: taken off term by term it doubles the distance from 64 bits.
+    float* turned = &dots[0][wave][c * SQ];   // (the wave's own, and v behind it)
+    rf4 off;
+    {
+      const rf4 bg4 = *reinterpret_cast<const rf4*>(&s_bg[4 * g]);
+      rf4 vz = v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) off[i] = -bg4[i] * from_s[i];
+      if (t0 + TB > n)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          off[i] = t0 + 4 * g + i < n ? off[i] : 0.f;
+          vz[i] = t0 + 4 * g + i < n ? vz[i] : 0.f;
+        }
+      *reinterpret_cast<rf4*>(turned + 4 * g) = off;
+      *reinterpret_cast<rf4*>(turned + 4 * TB * SQ + 4 * g) = vz;
+      o *= *reinterpret_cast<const rf4*>(&s_g[4 * g]);
+    }
+    rf4 mine;   // u of tokens g, g + 4, g + 8, g + 12
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      __builtin_amdgcn_wave_barrier();
+      rf4 y = *reinterpret_cast<const rf4*>(turned + 4 * q), u;
+      const rf4 vq = *reinterpret_cast<const rf4*>(turned + 4 * TB * SQ + 4 * q), bq = *reinterpret_cast<const rf4*>(&s_b[4 * q]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const rf4 l = *reinterpret_cast<const rf4*>(&keep[(4 * q + i) * SQ + 4 * q]);
+#pragma unroll
+        for (int j = 0; j < i; ++j) y[i] = fmaf(l[j], u[j], y[i]);
+        u[i] = fmaf(bq[i], vq[i], y[i]);
+      }
+      asm("" : "+v"(u[0]), "+v"(u[1]), "+v"(u[2]), "+v"(u[3]));
+      mine[q] = g < 2 ? (g == 0 ? u[0] : u[1]) : (g == 2 ? u[2] : u[3]);
+      if (q < 3) {
+        off = __builtin_amdgcn_mfma_f32_16x16x4f32(keep[c * SQ + 4 * q + g], mine[q], off, 0, 0, 0);
+        __builtin_amdgcn_wave_barrier();
+        *reinterpret_cast<rf4*>(turned + 4 * g) = off;
+      }
+    }
+    const bool finite = __builtin_isfinite(mine[0]) && __builtin_isfinite(mine[1]) && __builtin_isfinite(mine[2]) && __builtin_isfinite(mine[3]);
+    if (__ballot(!finite) == 0) {
+      const rf4 part = *reinterpret_cast<const rf4*>(&give[c * SQ + 4 * g]);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) o = __builtin_amdgcn_mfma_f32_16x16x4f32(part[q], mine[q], o, 0, 0, 0);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        for (int j = 0; j < 4; ++j) {   // token 4 q + j
+          const float u = __shfl(mine[q], 16 * j + c, DLI_WAVE);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i] = 4 * q + j <= 4 * g + i ? fmaf(give[(4 * g + i) * SQ + 4 * j + q], u, o[i]) : o[i];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (t0 + 4 * g + i < n) dst[(t0 + 4 * g + i) * dst_stride] = o[i];
+    mine *= *reinterpret_cast<const rf4*>(&s_e[4 * g]);
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) s[kb] *= all;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) s[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(sk[(4 * q + g) * WIDE + 16 * kb + c], mine[q], s[kb], 0, 0, 0);
+  }
+  float* end = (unit ? p.moves : p.ends) + ((int64_t)blockIdx.y * p.heads + head) * D * D;
+#pragma unroll
+  for (int kb = 0; kb < 4; ++kb) *reinterpret_cast<rf4*>(end + col * D + 16 * kb + 4 * g) = s[kb];
 }
 
 // A workgroup takes sixteen values of one (entry, head) through all its runs. Lane (i, g) of wave w makes keys 16 w + i of
@@ -378,7 +558,7 @@ int scan_runs(const RunsArgs& p, int rule, int finish, int out_is_bf16, hipStrea
     scan_runs_walk_kernel<RUNS_BONUS><<<walk, 256, 0, stream>>>(p);
     scan_runs_carry_kernel<RUNS_BONUS><<<carry, 256, 0, stream>>>(p);
   } else {
-    scan_runs_walk_kernel<RUNS_GATED><<<walk, 256, 0, stream>>>(p);
+    scan_gated_walk_kernel<<<walk, 256, 0, stream>>>(p);
     scan_runs_carry_kernel<RUNS_GATED><<<carry, 256, 0, stream>>>(p);
   }
   const dim3 done(p.heads, slots, (p.run_rows + 63) / 64);

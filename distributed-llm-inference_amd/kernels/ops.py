@@ -2080,11 +2080,11 @@ def recurrent_scan_supports(dim: int) -> bool:
 
 # A step whose longest entry has fewer rows is walked token by token: at 128 rows of one entry both ways take the same (41 to 45 and
 # 36 us a layer, generalized delta rule with 8 to 32 heads; 29 and 32 the bonus rule), at 300 with 32 heads 90 and 48, at 2,048
-# 584 and 150 (bonus rule 388 and 80, gated rule 422 and 137).
+# 584 and 150 (bonus rule 388 and 80, gated rule 410 and 90).
 RUNS_FROM_ROWS = 128
 RUNS_MIN_ROWS = 64      # rows of a run at least
 # Workgroups of the walk that a step is cut for: four a compute unit, one wave of each a SIMD (32 heads, delta / bonus / gated:
-# 2,048 tokens 166 / 77 / 143 us in runs of 64 rows, 150 / 77 / 137 of 128, 157 / 98 / 147 of 256).
+# 2,048 tokens 166 / 77 / 104 us in runs of 64 rows, 150 / 77 / 90 of 128, 157 / 98 / 93 of 256).
 RUNS_WORKGROUPS = 1024
 # From this many heads on that are walked side by side, entries as long as the longest counted, an entry is one run where every
 # further run would walk the unit columns again: 12 prompts of 400 tokens with 16 heads (192) 160 us instead of 169 in runs of 208
@@ -2110,6 +2110,7 @@ def scan_runs(entries: int, rows: int, heads: int, longest: int, unit_columns: b
         # entries 34 and 36), 200 with 64 (4 entries of 16 heads, 192 rows 45 and 47, 256 rows 57 and 49), 380 with 96, 700 with
         # 128 (8 of 16 heads, 200 rows 54 and 73, 700 rows 172 and 180), never with 192 (12 of 16 heads, 400 rows 120 and 139)
         # and 288 (12 of 24 heads 168 and 188). With more, one run an entry is faster (16 of 375 rows with 32 heads 273 and 183).
+        # (Of runs walked token by token; sixteen tokens at a time they take 0.6 to 0.8 of that: 170 rows 24, the last 112.)
         from_rows += 24 + (20 if entries > 1 else 0) + side_by_side ** 3 // 3800
     elif side_by_side <= 64 and (entries > 1 or not unit_columns):
         from_rows += 16   # (2 entries of 128 rows with 32 heads, generalized delta rule: 44.5 and 47.6)

@@ -15,7 +15,7 @@
 // for. (A wait gives up after about a second all the same, and its value is then not a number.)
 //
 // What bounds it: a kind's chain of store, load (0.9 to 1.5 us from one workgroup's store to another's registers), sum over lanes,
-// barrier, reads of LDS, products and their sum, 2.3 us a kind where a kernel of its own takes 3.8. 150 kinds without any work between
+// barrier, reads of LDS, products and their sum, 2.6 us a kind where a kernel of its own takes 3.8. 150 kinds without any work between
 // them took 1.35 us each with 16 workgroups and 1.8 with 96, so pieces are few and large: eight rows a wave and eight waves, not four. One
 // request, a step and seven more, ms, kernel by kernel -> now: 135M sizes, 48 keys 4.63 3.14, 512 4.77 3.43, 8,000 6.04 4.08; 360M sizes
 // 5.98 3.92, 6.26 4.23, 7.18 4.85. (Wider models are refused: their weights do not wait in registers two layers ahead, and 4 KB of

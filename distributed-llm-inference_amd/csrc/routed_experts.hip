@@ -534,7 +534,9 @@ __global__ __launch_bounds__(256) void expert_few_kernel(ExpertArgs p, FewChoice
   const int r = r0 + c, n = n0 + (UP ? 0 : 16 * wave) + 4 * g;
   if (wave >= (UP ? 1 : 2) || r >= rend || n >= features) return;               // (features come in fours)
   if (UP) {
-    const float iw = p.in_weight != nullptr ? p.in_weight[slot_of(r)] : 1.f;
+    // (a table's weights are known: the first workgroup may still be on its way to writing them)
+    const bool table_weight = SORTS && choices.choice.table != nullptr;
+    const float iw = p.in_weight == nullptr ? 1.f : table_weight ? 1.f / (float)choices.choice.top : p.in_weight[slot_of(r)];
     const exm_float4 up = *reinterpret_cast<const exm_float4*>(up_sums[lane]);
     for (int i = 0; i < 4; ++i) y[(int64_t)r * p.ff + n + i] = (bf16_t)clamped_glu(iw * acc[i], iw * up[i], limit, alpha, up_shift);
   } else {
@@ -1025,7 +1027,9 @@ int dli_expert_products(int* ids, const int* table, const int* token_ids, int vo
   ExpertArgs p;
   p.tile_expert = tile_expert; p.tile_row0 = tile_row0; p.tile_count = tile_count; p.offsets = offsets; p.order = order;
   p.top = top; p.width = width; p.ff = ff; p.in_weight = in_weight;
-  if (mfma && slots <= EXF_SLOTS && !expert_tiled(slots, experts, width, ff, is_bf16) && expert_few(slots, experts, width, ff)) {
+  // (with a table the products write its weights themselves, so of weights on the inputs they take none or those)
+  const bool own_weights = choice.table == nullptr || in_weight == nullptr || in_weight == weights;
+  if (mfma && own_weights && slots <= EXF_SLOTS && !expert_tiled(slots, experts, width, ff, is_bf16) && expert_few(slots, experts, width, ff)) {
     const FewChoices choices = {ids, choice, (int)slots, experts}, chosen = {ids, {nullptr, nullptr, 0, top, nullptr}, (int)slots, experts};
     expert_few_kernel<true, true><<<dim3(max_tiles, (ff + 15) / 16), 256, 0, stream>>>(p, choices, (const bf16_t*)h, h_stride, (const bf16_t*)w_gate,
                                                                                        (const bf16_t*)w_up, (bf16_t*)y, nullptr, limit, alpha, up_shift);

@@ -99,3 +99,25 @@ def test_choices_sorted_on_the_way(ops, rows, kind, table):
         return z[:rows * top][real[:rows * top]]
 
     assert torch.equal(run(rows), run(rows + 20))   # (80 choices and more: sorted by a kernel of its own)
+
+
+# weights on the inputs of experts that a table names: the table's own, which the products' launch writes, and others
+@pytest.mark.parametrize("rows", [1, 3, 16])
+@pytest.mark.parametrize("own", [True, False])
+def test_table_with_weights_on_the_inputs(ops, rows, own):
+    experts, top, width, ff, vocab, many = 8, 4, 96, 64, 40, 36
+    gen = torch.Generator().manual_seed(rows)
+    choices = torch.rand(vocab, experts, generator=gen).argsort(1)[:, :top].int().contiguous()
+    tokens = torch.randint(0, vocab, (many,), generator=gen, dtype=torch.int32)
+    w_gate, w_up, w_down = ((torch.randn(experts, *s, generator=gen) * s[1] ** -0.5).bfloat16().cuda() for s in ((ff, width), (ff, width), (width, ff)))
+    h, other = torch.randn(many, width, generator=gen).bfloat16().cuda(), torch.rand(many, top, generator=gen).cuda()
+
+    def run(n):
+        weights = torch.full((n, top), float("nan"), device="cuda")
+        z = ops.expert_products(torch.full((n, top), -7, dtype=torch.int32, device="cuda"), h[:n], w_gate, w_up, w_down, 7.0, 1.702, 1.0,
+                                in_weights=weights if own else other[:n], choose=(choices.cuda(), tokens[:n].cuda(), weights))
+        assert (weights == 1 / top).all()
+        return z[:rows * top]
+
+    got = run(rows)
+    assert got.isfinite().all() and torch.equal(got, run(many))   # (144 choices: the weights are there a launch earlier)

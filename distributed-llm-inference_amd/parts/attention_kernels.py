@@ -223,19 +223,25 @@ def prefill_tiles(ctx: Any, head_dim: int, q_heads: int, kv_heads: int, first_en
     per_tile = q_heads * rows // 128 if cut_floats > 0 else q_heads
     may_cut = window == 0 and cut_floats > 0
 
-    def make() -> PrefillTiles:
+    def make_lists() -> tuple:
         q_start, kv_len, first = ((ctx.q_start_host, np.asarray(ctx.kv_len_host), first_entry) if pieces is None
                                   else (pieces.q_start_host, pieces.kv_len_host, 0))
         q_len = (q_start[1:] - q_start[:-1]).astype(np.int64)
         ent, q0, code, n_cut, room = list_tiles(q_len, kv_len, first, rows, per_tile, units, may_cut)
-        if code is None:
-            return PrefillTiles(*ctx.upload([ent, q0]))
-        entry_t, q0_t, code_t = ctx.upload([ent, q0, code])
+        return (*ctx.upload([ent, q0] if code is None else [ent, q0, code]), *([None] if code is None else []), n_cut, room)
+
+    # (the lists do not depend on the head size, which layers of one step may differ in; a cut tile's buffers do)
+    shape = ("prefill tiles", rows, per_tile, first_entry, may_cut, 0 if pieces is None else pieces.chunk)
+
+    def make() -> PrefillTiles:
+        entry_t, q0_t, code_t, n_cut, room = ctx.step_lists(shape, make_lists)
+        if code_t is None:
+            return PrefillTiles(entry_t, q0_t)
         return PrefillTiles(entry_t, q0_t, code_t, n_cut, room,
                             torch.empty(n_cut * room * cut_floats, device=device, dtype=torch.float32),
                             torch.zeros(n_cut * q_heads, device=device, dtype=torch.int32))
 
-    return ctx.step_lists(("prefill tiles", rows, per_tile, first_entry, may_cut, 0 if pieces is None else pieces.chunk), make)
+    return ctx.step_lists((*shape, q_heads, cut_floats), make)
 
 
 def chunk_pieces(q_start: np.ndarray, kv_len: np.ndarray, first_entry: int, chunk: int) -> tuple[np.ndarray, ...]:

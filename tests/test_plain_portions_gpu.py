@@ -54,6 +54,25 @@ def test_same_results(monkeypatch, masks, page, heads, kv, dim):
     assert not got[0].any()   # the single token's row is another kernel's
 
 
+def test_layers_with_heads_of_two_sizes_in_one_step():
+    """A prompt whose longest tiles have their keys cut, in a step whose layers differ in their head size."""
+    from dli_amd.kernels import ops
+    from dli_amd.parts import attention_kernels as A
+
+    heads, kv, n = 32, 8, 1600
+    ctx, pages = _context(16, [0], [n], 0)
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    draw = lambda *s: torch.randn(*s, device="cuda", generator=gen).bfloat16()
+    for dim in (64, 128, 64):
+        q, k, v = draw(n, heads * dim), draw(pages, kv, 16, dim), draw(pages, kv, dim, 16)
+        got, want = torch.zeros_like(q), torch.zeros_like(q)
+        assert A.plain_portions(q, k, v, got, ctx, _Cache(k, v), heads, dim ** -0.5, chunk=4096)
+        tiles = ctx.q_tiles(ops.attention_grouped_tile_tokens(heads, kv))
+        ops.attention_grouped(q, k, v, want, ctx.q_start, ctx.kv_len, ctx.groups[0].block_tables, tiles[0], tiles[1], heads, dim ** -0.5, chunk=4096)
+        assert (got.float() - want.float()).abs().max() <= 3 * 2.0 ** -9 * want.float().abs().max()   # as above
+    assert A.prefill_tiles(ctx, 64, heads, kv, 0, q.device).cut is not None
+
+
 def test_what_stays_with_the_kernel_for_changed_scores(monkeypatch):
     from dli_amd.parts import attention_kernels as A
 

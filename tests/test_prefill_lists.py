@@ -1,0 +1,37 @@
+"""What a step's layers share of the prompt attention's tile lists, where they differ in their heads."""
+
+import numpy as np
+import pytest
+import torch
+
+
+def _context(monkeypatch, new):
+    from dli_amd.engine import batch
+    from dli_amd.kernels import ops
+
+    monkeypatch.setattr(ops, "compute_units", lambda device: 256)
+    monkeypatch.setattr(batch, "upload", lambda arrays, device: [torch.from_numpy(np.ascontiguousarray(a)) for a in arrays])
+    empty = torch.zeros(0, dtype=torch.int32)
+    q_start = np.concatenate([[0], np.cumsum(new)]).astype(np.int32)
+    return batch.StepContext(device=torch.device("cpu"), page_size=16, num_tokens=int(q_start[-1]), num_entries=len(new), num_decode=0,
+                             token_ids=empty, positions=empty, q_start=empty, kv_len=empty, state_slots=empty, logit_rows=empty, groups=[],
+                             q_start_host=q_start, kv_len_host=np.asarray(new, np.int32))
+
+
+# the smaller heads first and the larger; more heads and fewer on the same tiles; prompts that are cut and one that is not
+@pytest.mark.parametrize("tokens", [300, 1600, 2048])
+@pytest.mark.parametrize("shapes", [[(64, 32, 8), (128, 32, 8), (32, 32, 8)], [(128, 32, 8), (64, 32, 8)], [(64, 16, 4), (64, 32, 8), (112, 16, 4)]])
+def test_every_shape_has_buffers_of_its_own_size(monkeypatch, tokens, shapes):
+    from dli_amd.kernels import ops
+    from dli_amd.parts.attention_kernels import prefill_tiles
+
+    ctx = _context(monkeypatch, [tokens])
+    made = [prefill_tiles(ctx, *shape, 0, ctx.device) for shape in shapes]
+    for (dim, heads, kv), t in zip(shapes, made):
+        assert (t.cut is None) == (tokens == 300)
+        if t.cut is not None:
+            assert t.cut_buf.numel() == t.cut_tiles * t.cut_room * ops.attention_prefill_cut_floats(dim, heads, kv)
+            assert t.cut_count.numel() == t.cut_tiles * heads
+    assert [prefill_tiles(ctx, *shape, 0, ctx.device) for shape in shapes] == made   # one a shape and step
+    alike = [t for (_, heads, kv), t in zip(shapes, made) if (heads, kv) == (32, 8)]
+    assert all(t.entry is alike[0].entry and t.q0 is alike[0].q0 and t.cut is alike[0].cut for t in alike)   # the list is one

@@ -51,6 +51,7 @@ struct FlowArgs {
   float eps, scale_log2e;
   int rows[4], wgs[4];        // q/k/v, o, gate/up, down: rows of weights a workgroup, workgroups a layer
   int splits, layer_wgs;   // splits: the most that a request's keys are cut into
+  int new_token_wait;      // after how many looks the attention gives up on the new token's query, key and value
 };
 
 // Waits until four words carry the tag in their lower half.
@@ -252,9 +253,11 @@ __device__ __forceinline__ void flow_attention(const FlowArgs& p, const FlowLaye
 #pragma unroll
       for (int c = 0; c < DCH; ++c) wrong |= asks_v ? v_new[c] ^ tag : 0u;
       if ((wrong & 0xffffu) == 0) break;
-      if (tries == FLOW_WAIT) {
+      if (tries == p.new_token_wait) {   // (a lane's values belong to its column's heads, its part of the new token's value to all of them)
 #pragma unroll
         for (int c = 0; c < 4 * KC; ++c) w[c] = flow_u4{0x7fc00000u, 0x7fc00000u, 0x7fc00000u, 0x7fc00000u};
+#pragma unroll
+        for (int c = 0; c < DCH; ++c) v_new[c] = 0x7fc00000u;
         break;
       }
     }
@@ -666,15 +669,17 @@ int dli_decode_flow_parts(int layers, int hidden, int q_heads, int kv_heads, int
 
 // x [hidden] bfloat16: the stream, in place; ssq_out float32 [dli_decode_flow_parts]. layers_at: per layer the addresses norm1, norm2, w_qkv,
 // w_o, w_gate_up, w_down, k_pages, v_pages (on the device). tickets: one zero before the first launch, then the launches' own.
-// At most table_width * page_size keys.
+// At most table_width * page_size keys. new_token_wait: after how many looks the attention gives up on the new token's query, key and
+// value (negative: as every other wait).
 int dli_decode_flow(const void* layers_at, int layers, void* words, void* tickets, void* x, float* ssq_out, const float* angles, const int* slots,
                     const int* kv_len, const int* block_table, int table_width, int hidden, int q_heads, int kv_heads, int head_dim, int inner,
-                    int page_size, float eps, float scale, hipStream_t stream) {
+                    int page_size, float eps, float scale, int new_token_wait, hipStream_t stream) {
   FlowArgs a;
   if (!flow_plan(a, layers, hidden, q_heads, kv_heads, head_dim, inner) || page_size < 16 || page_size % 16 || table_width < 1 ||
       (int64_t)table_width * page_size > (int64_t)1 << 30) return DLI_ERR_ARGUMENT;
   a.layers = (const FlowLayer*)layers_at; a.words = words; a.tickets = (unsigned long long*)tickets;
   a.x = (bf16_t*)x; a.ssq_out = ssq_out; a.angles = angles; a.slots = slots; a.kv_len = kv_len; a.block_table = block_table; a.table_width = table_width;
+  a.new_token_wait = new_token_wait < 0 ? FLOW_WAIT : new_token_wait;
   a.splits = flow_splits(table_width * page_size);
   a.layer_wgs += kv_heads * a.splits;
   a.page_size = page_size; a.page_of = page_of_tile(page_size); a.eps = eps; a.scale_log2e = scale * 1.4426950408889634f;

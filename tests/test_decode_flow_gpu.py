@@ -82,6 +82,63 @@ def test_what_it_does_not_take():
     assert not any(ops.decode_flow_bytes(*s) for s in refused)
 
 
+class _Launches:
+    """Launches of the kernel by itself, over weights and pages of its own: one request of 20 keys, in the order of a page table."""
+
+    def __init__(self, sizes, seed):
+        from dli_amd.kernels import ops
+
+        layers, hidden, heads, kv, dim, inner = self.sizes = sizes
+        gen = torch.Generator(device="cuda").manual_seed(seed)
+        draw = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+        matrix = lambda *s: draw(*s).mul_(s[1] ** -0.5).bfloat16()
+        self.held = [[1 + 0.1 * draw(hidden), 1 + 0.1 * draw(hidden), matrix((heads + 2 * kv) * dim, hidden), matrix(hidden, heads * dim),
+                      matrix(2 * inner, hidden), matrix(hidden, inner), draw(3, kv, 16, dim).bfloat16(), draw(3, kv, dim, 16).bfloat16()]
+                     for _ in range(layers)]
+        self.table = torch.tensor([[t.data_ptr() for t in row] for row in self.held], dtype=torch.int64).cuda()
+        self.xs = draw(6, hidden).bfloat16()
+        turn = 19 * 10000.0 ** (-torch.arange(dim // 2, device="cuda") / (dim // 2))
+        self.angles = torch.stack([turn.cos(), turn.sin()])[None].float().contiguous()
+        on = lambda *v: torch.tensor(v, dtype=torch.int32, device="cuda")
+        self.slot, self.keys, self.pages = on(2 * 16 + 3), on(20), on(1, 2)[None].contiguous()
+        self.words_of = lambda: torch.zeros(ops.decode_flow_bytes(*sizes) // 4, dtype=torch.int32, device="cuda")
+        self.ssq = torch.empty(ops.decode_flow_parts(*sizes), 1, device="cuda")
+
+    def run(self, words, launch, x, **more):
+        """The stream behind a launch that is the ``launch``-th of these words (from 0 on), on a row."""
+        from dli_amd.kernels import ops
+
+        dim, stream = self.sizes[4], x[None].clone()
+        ops.decode_flow(self.table, words, torch.tensor([launch << 32], dtype=torch.int64, device="cuda"), stream, self.ssq, self.angles,
+                        self.slot, self.keys, self.pages, self.sizes, 16, 1e-5, dim ** -0.5, **more)
+        return stream[0]
+
+
+def test_numbers_of_launches_go_round():
+    """A word's tag is 16 bits of the launch's number: on both sides of 65,536 launches the results are those of the first ones."""
+    at = _Launches(SIZES[1], 5)
+    early, late = at.words_of(), at.words_of()
+    for i, x in enumerate(at.xs):
+        first, then = at.run(early, i, x), at.run(late, 65533 + i, x)
+        assert first.isfinite().all() and torch.equal(first, then)
+
+
+@pytest.mark.parametrize("sizes", [SIZES[3], (1, 576, 9, 3, 64, 1536), (1, 384, 6, 2, 128, 640)])
+def test_values_that_never_came_are_not_numbers(sizes):
+    """Attention that gives up at its first look, where the query, the key and as many of a value's sixteen as a kv head has heads carry
+    the launch's tag already and the others the one before's: the result is the right one (they came in time) or is not a number."""
+    _, _, heads, kv, dim, _ = sizes
+    at = _Launches(sizes, 6)
+    words, of_second = at.words_of(), at.words_of()
+    at.run(words, 0, at.xs[0])
+    right = at.run(of_second, 1, at.xs[1])
+    there = torch.arange((heads + 2 * kv) * dim, device="cuda")
+    there = there[(there < (heads + kv) * dim) | (there % 16 < heads // kv)]
+    words[there] = of_second[there]
+    got = at.run(words, 1, at.xs[1], new_token_wait=0)
+    assert right.isfinite().all() and (torch.equal(got, right) or got.isnan().all())
+
+
 def test_reloaded_weights_are_used():
     """What a recorded step holds of the route's own memory outlives the weights that it was made for."""
     from dli_amd.engine.core import build_core

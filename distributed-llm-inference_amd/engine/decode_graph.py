@@ -78,6 +78,7 @@ class DecodeGraphs:
         self.n_groups = step_fn.manager.num_groups
         self.captured: dict[tuple, _Captured] = {}
         self._asked: dict[tuple, int] = {}   # decode steps that a shape that is not recorded has been asked for
+        self._weights = step_fn.model.weights_version   # whose addresses the recorded steps hold
         _RECORDERS.add(self)
         self.replays = 0
         self.enabled = self._supported()
@@ -95,6 +96,14 @@ class DecodeGraphs:
         return all(len(e.tokens) == 1 and e.start + steps <= self.max_width * ps for e in entries)
 
     # ------------------------------------------------------------------ capture
+
+    def _forget_older(self) -> None:
+        """Drop the steps that were recorded before the model's weights were loaded anew: they read the tensors of then."""
+        if self._weights != self.step_fn.model.weights_version:
+            torch.cuda.synchronize()
+            self.captured.clear()
+            self._asked.clear()
+            self._weights = self.step_fn.model.weights_version
 
     def _layout(self, b: int, width: int) -> tuple[dict, int]:
         fields = [("token_ids", b), ("positions", b), ("q_start", b + 1), ("kv_len", b), ("state_slots", b),
@@ -228,6 +237,7 @@ class DecodeGraphs:
         two tokens of a live request later. Returns the number of graphs captured by this call."""
         if not self.enabled:
             return 0
+        self._forget_older()
         ps = self.step_fn.manager.page_size
         max_len = min(int(max_len), self.max_width * ps)
         keys = set()
@@ -261,6 +271,7 @@ class DecodeGraphs:
         sampled = sampling is not None
         if steps > 1 and not sampled:
             raise ValueError("several steps in a row need the sampling parameters")
+        self._forget_older()
         key = self._shape_key(n, max(e.start + steps for e in entries), sampled, steps)
         cap = self.captured.get(key)
         if cap is None:

@@ -66,10 +66,6 @@ class DecodeFlow:
             return None
         return DecodeFlow(fields, caches, model.layers[model.spec.schedule[0].layer].parts["mixer"].position, model.rt.device)
 
-    def memory(self) -> tuple:
-        """What a launch holds the addresses of besides weights and pages."""
-        return self.table, self.words, self.tickets
-
     def run(self, stream: DecodeStream, ctx: Any) -> bool:
         """All blocks on a stream of one row; False (and nothing has run) where the step is not the kernel's."""
         grp = ctx.groups[self.group]

@@ -43,7 +43,6 @@ class BoundCaches(list):
     derived_for: int = -1           # the model's ``weights_version`` it was made for
     flow: Any = None                # DecodeFlow, or False where that route does not apply
     flow_for: int = -1
-    retired: tuple = ()             # memory of earlier ones, whose addresses recorded steps hold
 
 
 def _walk(part: Part):
@@ -223,7 +222,7 @@ class Model:
             from .decode_flow import DecodeFlow
 
             if caches.flow:
-                caches.retired += caches.flow.memory()
+                torch.cuda.synchronize()   # its launches may have run on other streams than the one its memory was made on
             caches.flow = DecodeFlow.build(self, caches) or False
             caches.flow_for = self.weights_version
         return caches.flow or None

@@ -139,8 +139,9 @@ def test_values_that_never_came_are_not_numbers(sizes):
     assert right.isfinite().all() and (torch.equal(got, right) or got.isnan().all())
 
 
-def test_reloaded_weights_are_used():
-    """What a recorded step holds of the route's own memory outlives the weights that it was made for."""
+@pytest.mark.parametrize("recorded", [False, True])
+def test_reloaded_weights_are_used(recorded):
+    """Steps recorded on other weights are forgotten with them, and the route's own memory is made anew."""
     from dli_amd.engine.core import build_core
     from dli_amd.trace import TraceSession
     from dli_amd.weights import load_model, write_random_model
@@ -150,6 +151,8 @@ def test_reloaded_weights_are_used():
         _, weights = P.load_folder(folder)
         model = load_model(folder, dtype="bfloat16")
     core = build_core(model, num_pages=8, page_size=16, max_seqs=4, enable_prefix_caching=False, watermark=0.0)
+    if recorded:
+        core.step.enable_decode_graphs(1, 32)
     session = TraceSession(core)
     step = lambda name: session.step([{"id": name, "tokens": [7], "want": [0]}]).clone()
     first, again = step("a"), step("b")
@@ -159,7 +162,6 @@ def test_reloaded_weights_are_used():
     model.load_weights({n: (weights[n].float() * 0.5).to("cuda", kinds[s.role]) for n, s in model.weight_specs().items()})
     second = step("c")
     assert core.step.caches.flow is not before and not torch.equal(first, second)
-    assert any(words is before.words for words in core.step.caches.retired)
-    model.native_steps = False
+    core.step.graphs, model.native_steps = None, False
     by_blocks = step("d")
     assert (second - by_blocks).norm() <= 0.02 * by_blocks.norm()

@@ -416,9 +416,13 @@ __device__ __forceinline__ exm_bf16x8 exm_load(const bf16_t* p) { return *reinte
 // 117 (6.0 TB/s); 8 of 2,048 on 4,096, 1 row (67 MB) 72.5 -> 17.3. Four chunks ahead: the same.
 #define EXF_K 256
 #define EXF_AHEAD 3
-// Up to as many choices as a wave has lanes: every workgroup sorts them for itself, a choice a lane, and no kernel does it before (which
-// took 4.5 us of a step of two rows with eight choices, this 0.7 to 1.3 in each of the two products).
-#define EXF_SLOTS DLI_WAVE
+// A few choices: every workgroup sorts them for itself, a choice a lane, and no kernel does it before. That kernel takes 4.5 us; sorting
+// here takes the longer the more choices there are, in every workgroup of both products. All of it, us, by the kernel and here, at 4, 8,
+// 16, 32 and 64 choices: 4 of 32 experts, 1,024 of 2,048 wide 20.4 17.6, 26.9 24.8, 48 48, 68 78, 80 101; 512 of 1,024 14.2 11.6, 16.6
+// 13.7, 20.4 21.0, 31.7 38, 36.6 46; 8 of 64, 256 of 1,024 (8 on) 14.1 11.7, 17.2 16.5, 21.4 25.3, 33.3 51.8; one of 128, 128 of 512 11.6
+// 9.0, 12.1 9.9, 12.7 11.5, 14.3 15.7, 18.9 30.
+#define EXF_SLOTS 16
+static_assert(EXF_SLOTS <= DLI_WAVE, "a choice a lane");
 struct FewChoices {
   int* ids; TableChoice choice;   // choice.table: looked up, and written to ids with the weights by the first workgroup of the up product
   int slots, experts;

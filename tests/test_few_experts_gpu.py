@@ -102,7 +102,7 @@ def test_choices_sorted_on_the_way(ops, rows, kind, table):
 
 
 # weights on the inputs of experts that a table names: the table's own, which the products' launch writes, and others
-@pytest.mark.parametrize("rows", [1, 3, 16])
+@pytest.mark.parametrize("rows", [1, 3, 4, 16])   # the most choices that the products sort themselves, and more
 @pytest.mark.parametrize("own", [True, False])
 def test_table_with_weights_on_the_inputs(ops, rows, own):
     experts, top, width, ff, vocab, many = 8, 4, 96, 64, 40, 36

@@ -282,6 +282,21 @@ class ChunkPieces:
 # 1,969, 2 x 1,500 (34) 2,077 2,056, 2 x 2,900 (91) 3,306 3,217; 2,048 wide 1 x 4,096 (256) 6,030 5,740; Betepel 1,024 wide 3 x 700 (11)
 # 2,272 2,458.
 PLAIN_FROM_PAIRS = 36 << 20
+# How many times as many where chunks fill no more than half a tile's rows, which are 32, 64 or 128 for groups of a multiple of four, two
+# or one query heads: the rest of a tile is work for nothing, in every chunk, so never. Steps of 41 million pairs, us a layer, by the
+# kernel for changed scores and by this one: 32 heads of 64 on 32, chunks of 32 191 270, 48 157 157, 64 100 100, 80 99 80, 96 78 58; of 48,
+# 64 84 93, 80 92 73; 24 of 64 on 8, 48 151 152, 64 97 88, 80 98 76; 16 of 64 on 8, 32 101 99, 48 130 94; 32 of 128 on 16, 16 412 523, 32 346
+# 288, 48 277 176; 32 of 64 on 8, 16 195 193, 32 168 119. (The host's lists of the pieces, 240 us for 64 tokens each and 480 for 32, aside.)
+SHORT_CHUNKS = 1 << 20
+
+
+def plain_pays(head_dim: int, q_heads: int, kv_heads: int, pairs: int, chunk: int) -> bool:
+    """Whether the kernel that shares key tiles is the one for a step's portions of so many pairs, cut into chunks of ``chunk`` (0: not
+    cut). Heads of 16 have no such kernel: 32 on 8, 2,048 tokens 91 us by the kernel for changed scores, 101 by theirs."""
+    if not ops.attention_prefill_cut_floats(head_dim, q_heads, kv_heads):
+        return False
+    short = 0 < 2 * chunk <= ops.attention_prefill_tile_rows(head_dim, q_heads, kv_heads)
+    return pairs >= PLAIN_FROM_PAIRS * (SHORT_CHUNKS if short else 1)
 
 
 def plain_portions(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, out: torch.Tensor, ctx: Any, cache: Any,
@@ -299,10 +314,10 @@ def plain_portions(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor
             return None
         new, keys = np.diff(ctx.q_start_host)[nd:].astype(np.int64), np.asarray(ctx.kv_len_host)[nd:].astype(np.int64)
         seen = np.minimum(keys, max(chunk, window)) if chunk or window else keys   # (by the last row, or one in the middle)
-        if q_heads * int((new * np.minimum(seen, keys - new // 2)).sum()) < PLAIN_FROM_PAIRS:
-            return None
         longest = int(keys.max())
         met_chunk, met_window = (n if 0 < n < longest else 0 for n in (chunk, window))
+        if not plain_pays(head_dim, q_heads, kv_heads, q_heads * int((new * np.minimum(seen, keys - new // 2)).sum()), met_chunk):
+            return None
         if met_window and (keep_first or met_chunk) or met_chunk % page_size:
             return None
         if not met_chunk:

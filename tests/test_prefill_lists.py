@@ -1,4 +1,4 @@
-"""What a step's layers share of the prompt attention's tile lists, where they differ in their heads."""
+"""What a step's layers share of the prompt attention's tile lists, where they differ in their heads; which masked portions it takes."""
 
 import numpy as np
 import pytest
@@ -35,3 +35,14 @@ def test_every_shape_has_buffers_of_its_own_size(monkeypatch, tokens, shapes):
     assert [prefill_tiles(ctx, *shape, 0, ctx.device) for shape in shapes] == made   # one a shape and step
     alike = [t for (_, heads, kv), t in zip(shapes, made) if (heads, kv) == (32, 8)]
     assert all(t.entry is alike[0].entry and t.q0 is alike[0].q0 and t.cut is alike[0].cut for t in alike)   # the list is one
+
+
+def test_which_portions_share_key_tiles():
+    from dli_amd.parts.attention_kernels import PLAIN_FROM_PAIRS, plain_pays
+
+    many = 40 << 20
+    assert PLAIN_FROM_PAIRS <= many
+    assert all(plain_pays(*s) for s in [(64, 32, 8, many, 0), (64, 32, 8, many, 32), (64, 16, 8, many, 48), (64, 32, 32, many, 80), (48, 24, 8, many, 80),
+                                        (128, 32, 8, many, 2048)])
+    assert not any(plain_pays(*s) for s in [(64, 32, 8, PLAIN_FROM_PAIRS - 1, 0), (64, 32, 8, many, 16), (64, 16, 8, many, 32), (64, 32, 32, many, 64),
+                                            (48, 24, 8, many, 48), (16, 32, 8, many, 0), (16, 32, 8, many, 2048), (64, 32, 32, 16 * many, 64)])

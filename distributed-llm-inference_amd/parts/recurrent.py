@@ -172,6 +172,19 @@ class WKV(_MatrixStateMixer):
         return linear_f32(self.rt, out, self.w_o)
 
 
+def single_kernel_pays(rows: int, heads: int, kv_heads: int, head_dim: int, value_dim: int, taps: int) -> bool:
+    """Whether a step of so many single tokens goes through the one kernel that does all of the gated delta rule. Its workgroups, one a
+    (request, q/k head), are sixteen waves of four value columns each; where the heads on a q/k head have fewer than 64 columns between
+    them most waves idle, and with many such workgroups the three kernels are ahead. Three kernels and one, us: four columns, 512
+    workgroups 8.1 5.0, 2,048 9.9 12.3; 16 columns (keys of 16, 32, 64) 512 8.0 5.1, 8.1 5.1, 8.6 5.6, 2,048 11.7 12.7, 12.1 13.2,
+    13.3 15.3, 8,192 28 42, 30 43, 34 49; 32 columns 2,048 14.2 13.4, 14.9 14.2, 17.3 16.0, 8,192 39 44, 41 45, 44 50. Keys of 128 make
+    a wave's work long enough (16 columns, 2,048 23 20, 8,192 63 63, 32,768 290 276), and so do 64 columns (8,192 57 51, 59 52, 65 59)."""
+    if not ops.gated_delta_single_takes(heads, kv_heads, head_dim, value_dim, taps):
+        return False
+    columns = heads // kv_heads * value_dim
+    return columns >= 64 or head_dim >= 128 or rows * kv_heads <= 64 * max(columns, 16)
+
+
 @register_part("mixer", "gated_delta")
 class GatedDelta(Mixer):
     """The gated delta rule. From the rows ``h``: q and k (``num_kv_heads x head_dim``) and v (``num_heads x
@@ -242,7 +255,7 @@ class GatedDelta(Mixer):
             proj = linear_f32(self.rt, as_operand(self.rt, x, ctx), self.w_in)
         g_off = self.channels
         b_off, a_off = g_off + self.hv, g_off + self.hv + H
-        if ctx.num_decode == ctx.num_entries and ops.gated_delta_single_takes(H, self.num_kv_heads, self.head_dim, self.value_dim, self.conv_taps):
+        if ctx.num_decode == ctx.num_entries and single_kernel_pays(n, H, self.num_kv_heads, self.head_dim, self.value_dim, self.conv_taps):
             out = self.rt.empty(n, self.hv)
             ops.gated_delta_single(proj, b_off, a_off, g_off, self.conv_w, self.a_log, self.dt_bias, state, self.state_floats,
                                    ctx.positions, ctx.state_slots, self.norm_w, self.norm_eps, out, H, self.num_kv_heads,

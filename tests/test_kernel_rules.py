@@ -118,3 +118,21 @@ def test_rotated_rows_that_just_fit(kv, d, dtype):
     shares = lambda heads: ops.rope_kv_shares(4096, d, heads, heads, d, getattr(torch, dtype), 256)
     assert 8 * d * 4 + 8 * kv * d * getattr(torch, dtype).itemsize == 48 * 1024
     assert shares(kv) == 1 and shares(kv - 1) == 1 and shares(kv + 1 + kv % 2) == 0
+
+
+# (rows, heads, q/k heads, key size, value size): us by the three kernels of the gated delta rule's single tokens, and by the one
+GATED_SINGLES = {
+    (4, 32, 8, 64, 64): (8.3, 5.5), (256, 32, 8, 64, 64): (58.0, 52.3), (256, 32, 32, 64, 64): (64.8, 57.0), (256, 128, 128, 16, 64): (199.3, 185.0),
+    (16, 32, 32, 64, 16): (8.6, 5.6), (64, 8, 8, 64, 16): (9.0, 5.6), (256, 8, 8, 16, 16): (12.0, 12.6), (64, 32, 32, 16, 16): (11.7, 12.7),
+    (64, 32, 32, 64, 16): (13.3, 15.3), (256, 32, 32, 32, 16): (30.4, 43.1), (256, 32, 32, 128, 16): (63.3, 63.3), (64, 64, 32, 64, 16): (17.7, 16.1),
+    (64, 8, 8, 16, 4): (8.1, 5.0), (64, 32, 32, 16, 4): (9.9, 12.3),
+    (256, 32, 32, 64, 32): (44.0, 49.5), (256, 64, 32, 16, 16): (40.1, 44.1), (16, 128, 128, 64, 32): (17.3, 15.9), (256, 128, 128, 128, 32): (481.0, 313.0)}
+
+
+def test_single_tokens_of_the_gated_delta_rule():
+    from dli_amd.parts.recurrent import single_kernel_pays
+
+    for sizes, (three, one) in GATED_SINGLES.items():
+        chosen = one if single_kernel_pays(*sizes, 4) else three
+        assert chosen <= 1.03 * min(three, one), sizes
+    assert not single_kernel_pays(4, 32, 8, 48, 64, 4) and not single_kernel_pays(4, 32, 8, 64, 64, 5)   # sizes without such a kernel

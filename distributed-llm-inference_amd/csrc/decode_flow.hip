@@ -51,7 +51,6 @@ struct FlowArgs {
   float eps, scale_log2e;
   int rows[4], wgs[4];        // q/k/v, o, gate/up, down: rows of weights a workgroup, workgroups a layer
   int splits, layer_wgs;   // splits: the most that a request's keys are cut into
-  int new_token_wait;      // after how many looks the attention gives up on the new token's query, key and value
 };
 
 // Waits until four words carry the tag in their lower half.
@@ -182,8 +181,8 @@ __device__ __forceinline__ flow_f4 flow_mfma(flow_u4 a, flow_u4 b, flow_f4 c) {
 }
 
 // One (kv head, run of keys): the arithmetic of the decode attention (attention_mfma.hip). The new token's key and value come by way
-// of their words, as a pair of tiles of which one key counts.
-template <int D, typename Near>
+// of their words, as a pair of tiles of which one key counts; after WAIT looks at them it gives up.
+template <int D, int WAIT, typename Near>
 __device__ __forceinline__ void flow_attention(const FlowArgs& p, const FlowLayer& L, __amdgpu_buffer_rsrc_t words, unsigned layer_at, unsigned tag,
                                                unsigned tag32, int kvh, int split, unsigned char* lds, const Near& near) {
   constexpr int KC = D / 32, DCH = D / 16;
@@ -253,11 +252,9 @@ __device__ __forceinline__ void flow_attention(const FlowArgs& p, const FlowLaye
 #pragma unroll
       for (int c = 0; c < DCH; ++c) wrong |= asks_v ? v_new[c] ^ tag : 0u;
       if ((wrong & 0xffffu) == 0) break;
-      if (tries == p.new_token_wait) {   // (a lane's values belong to its column's heads, its part of the new token's value to all of them)
+      if (tries == WAIT) {   // (of the value, what is not there is told by its word, below)
 #pragma unroll
         for (int c = 0; c < 4 * KC; ++c) w[c] = flow_u4{0x7fc00000u, 0x7fc00000u, 0x7fc00000u, 0x7fc00000u};
-#pragma unroll
-        for (int c = 0; c < DCH; ++c) v_new[c] = 0x7fc00000u;
         break;
       }
     }
@@ -335,8 +332,13 @@ __device__ __forceinline__ void flow_attention(const FlowArgs& p, const FlowLaye
       g.k[0][c] = col == 0 ? k_new[c] : flow_u4{0u, 0u, 0u, 0u};
       g.k[1][c] = flow_u4{0u, 0u, 0u, 0u};
     }
+    // A lane's query is its column's head's alone, its part of the value every head's: a word that never came is not a number here. (Made
+    // so where the wait gives up, the loop's registers moved about: 1.7% of a step of the 135M sizes.)
 #pragma unroll
-    for (int c = 0; c < DCH; ++c) g.v[c] = flow_u4{grp == 0 ? v_new[c] >> 16 : 0u, 0u, 0u, 0u};
+    for (int c = 0; c < DCH; ++c) {
+      const unsigned value = ((v_new[c] ^ tag) & 0xffffu) == 0 ? v_new[c] >> 16 : 0x7fc0u;
+      g.v[c] = flow_u4{grp == 0 ? value : 0u, 0u, 0u, 0u};
+    }
     attend(g, 0, 1);
   }
   l = add_across32(add_across16(l));
@@ -377,7 +379,7 @@ __device__ __forceinline__ void flow_attention(const FlowArgs& p, const FlowLaye
 }
 
 // grid: layers x layer_wgs. Dynamic LDS: the row, or the attention's states.
-template <int D>
+template <int D, int WAIT>
 __global__ __launch_bounds__(FLOW_THREADS) void decode_flow_kernel(FlowArgs p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   __shared__ unsigned long long sh_ticket;
@@ -508,7 +510,7 @@ __global__ __launch_bounds__(FLOW_THREADS) void decode_flow_kernel(FlowArgs p) {
   }
   piece -= p.wgs[0];
   if (piece < p.kv_heads * p.splits) {
-    flow_attention<D>(p, L, words, at_layer, tag, tag32, piece % p.kv_heads, piece / p.kv_heads, lds, [&] {
+    flow_attention<D, WAIT>(p, L, words, at_layer, tag, tag32, piece % p.kv_heads, piece / p.kv_heads, lds, [&] {
       if (layer > 0) near(at_before + p.at_x2, 0xffffu, tag);
     });
     return;
@@ -669,22 +671,22 @@ int dli_decode_flow_parts(int layers, int hidden, int q_heads, int kv_heads, int
 
 // x [hidden] bfloat16: the stream, in place; ssq_out float32 [dli_decode_flow_parts]. layers_at: per layer the addresses norm1, norm2, w_qkv,
 // w_o, w_gate_up, w_down, k_pages, v_pages (on the device). tickets: one zero before the first launch, then the launches' own.
-// At most table_width * page_size keys. new_token_wait: after how many looks the attention gives up on the new token's query, key and
-// value (negative: as every other wait).
+// At most table_width * page_size keys. impatient: the attention gives up on the new token's query, key and value at its first look, so
+// that what it leaves then can be seen (a kernel of its own: the limit as an argument took 0.5% of a step of the 135M sizes).
 int dli_decode_flow(const void* layers_at, int layers, void* words, void* tickets, void* x, float* ssq_out, const float* angles, const int* slots,
                     const int* kv_len, const int* block_table, int table_width, int hidden, int q_heads, int kv_heads, int head_dim, int inner,
-                    int page_size, float eps, float scale, int new_token_wait, hipStream_t stream) {
+                    int page_size, float eps, float scale, int impatient, hipStream_t stream) {
   FlowArgs a;
   if (!flow_plan(a, layers, hidden, q_heads, kv_heads, head_dim, inner) || page_size < 16 || page_size % 16 || table_width < 1 ||
       (int64_t)table_width * page_size > (int64_t)1 << 30) return DLI_ERR_ARGUMENT;
   a.layers = (const FlowLayer*)layers_at; a.words = words; a.tickets = (unsigned long long*)tickets;
   a.x = (bf16_t*)x; a.ssq_out = ssq_out; a.angles = angles; a.slots = slots; a.kv_len = kv_len; a.block_table = block_table; a.table_width = table_width;
-  a.new_token_wait = new_token_wait < 0 ? FLOW_WAIT : new_token_wait;
   a.splits = flow_splits(table_width * page_size);
   a.layer_wgs += kv_heads * a.splits;
   a.page_size = page_size; a.page_of = page_of_tile(page_size); a.eps = eps; a.scale_log2e = scale * 1.4426950408889634f;
   const int rows = 2 * 128 * FLOW_INNER_BLOCKS, states = FLOW_WAVES * ((head_dim / 4) * 16 * 16 + 32 * 4), bytes = rows > states ? rows : states;
-  const auto kernel = head_dim == 64 ? decode_flow_kernel<64> : decode_flow_kernel<128>;
+  const auto kernel = head_dim == 64 ? (impatient ? decode_flow_kernel<64, 0> : decode_flow_kernel<64, FLOW_WAIT>)
+                                     : (impatient ? decode_flow_kernel<128, 0> : decode_flow_kernel<128, FLOW_WAIT>);
   if (bytes > 65536 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) return DLI_ERR_LAUNCH;
   kernel<<<layers * a.layer_wgs, FLOW_THREADS, bytes, stream>>>(a);
   return dli_launch_status();

@@ -1085,13 +1085,13 @@ def decode_flow_parts(layers: int, hidden: int, q_heads: int, kv_heads: int, hea
 
 def decode_flow(table: torch.Tensor, words: torch.Tensor, tickets: torch.Tensor, x: torch.Tensor, ssq_out: torch.Tensor,
                 angles: torch.Tensor, slots: torch.Tensor, kv_len: torch.Tensor, block_tables: torch.Tensor, sizes: Sequence[int],
-                page_size: int, eps: float, scale: float, new_token_wait: int = -1) -> None:
+                page_size: int, eps: float, scale: float, impatient: bool = False) -> None:
     """All pre-norm blocks of a decode step of one row on the stream ``x [1, hidden]`` (in place; the row's sum of squares in parts
     to ``ssq_out [parts, 1]``). ``table``: int64 ``[layers, 8]``, the addresses of each layer's two norm weights (float32), its
     q/k/v, o, gate/up and down matrices (bfloat16, row by row) and its K and V pages; ``words`` and ``tickets``: zeros when made,
     then these launches' own, which must not overlap; ``angles`` float32 ``[1, 2, head_dim/2]``; ``sizes``: layers, hidden size,
-    heads, kv heads, head size, inner size of the feed-forward. A wait that gives up leaves what is not a number; ``new_token_wait``: after
-    how many looks the attention's for the new token's query, key and value does (default: after about a second, as all do)."""
+    heads, kv heads, head size, inner size of the feed-forward. A wait gives up after about a second and
+    leaves what is not a number; ``impatient``: the attention's for the new token does at its first look (for tests)."""
     layers, hidden, q_heads, kv_heads, head_dim, inner = sizes
     nbytes = decode_flow_bytes(*sizes)
     _require(nbytes > 0, "decode_flow: sizes that its kernel does not take")
@@ -1113,7 +1113,7 @@ def decode_flow(table: torch.Tensor, words: torch.Tensor, tickets: torch.Tensor,
     _check(library().dli_decode_flow(
         _ptr(table), layers, _ptr(words), _ptr(tickets), _ptr(x), _ptr(ssq_out), _ptr(angles), _ptr(slots), _ptr(kv_len),
         _ptr(block_tables), block_tables.shape[1], hidden, q_heads, kv_heads, head_dim, inner, int(page_size), float(eps),
-        float(scale), int(new_token_wait), _stream()), "decode_flow")
+        float(scale), int(impatient), _stream()), "decode_flow")
 
 
 def prenorm_blocks(x: torch.Tensor, blocks, count: int, step) -> bool:

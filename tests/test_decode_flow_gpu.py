@@ -135,7 +135,7 @@ def test_values_that_never_came_are_not_numbers(sizes):
     there = torch.arange((heads + 2 * kv) * dim, device="cuda")
     there = there[(there < (heads + kv) * dim) | (there % 16 < heads // kv)]
     words[there] = of_second[there]
-    got = at.run(words, 1, at.xs[1], new_token_wait=0)
+    got = at.run(words, 1, at.xs[1], impatient=True)
     assert right.isfinite().all() and (torch.equal(got, right) or got.isnan().all())
 
 

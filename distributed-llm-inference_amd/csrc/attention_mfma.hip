@@ -675,6 +675,7 @@ __device__ __forceinline__ void tile_barrier() {
 // larger ones: 126 instead of 176 and 196 instead of 276, nothing spilled, no copies between
 // the two register files.)
 #define PREFILL_MAX_CUTS 8  // the most runs that a tile's keys are cut into
+#define LAZY_LOG2 8.f       // how far (log2) a score may exceed the exponentials' reference point before that moves
 
 template <int DCH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DCH <= 4 ? 3 : 2)))
@@ -685,7 +686,7 @@ void attention_prefill_shared_kernel(
     const int* __restrict__ block_tables, int table_stride, const int* __restrict__ tile_entry,
     const int* __restrict__ tile_q0, int q_heads, int kv_heads, int page_size, float scale_log2e,
     int window, int heads_per_wg, const int* __restrict__ tile_cut, int cut_room, float* cut_buf,
-    unsigned* cut_count) {
+    unsigned* cut_count, float slack_log2) {
   constexpr int D = DCH * 16, DK = D / 32;      // DK: k-steps of 32 dims of the first product
   constexpr bool ODD = DCH % 2 != 0;            // sixteen dims more, and K part by part in LDS
   static_assert(DCH >= 2 && DCH <= 8, "heads of 32 to 128");
@@ -748,7 +749,6 @@ void attention_prefill_shared_kernel(
   // beside st[j].m: the value subtracted in the exponent (m, or 0 while m is -inf), and the raw
   // score above which m has to rise
   float m_ref[2], raise_at[2];
-  constexpr float LAZY_LOG2 = 8.f;
   const float inv_scale_log2e = 1.f / scale_log2e;
   int pos[2];
 #pragma unroll
@@ -996,8 +996,11 @@ void attention_prefill_shared_kernel(
       // accumulated rescaled) only when a score of the tile exceeds it by more than 2^LAZY_LOG2,
       // which each lane can tell from its own eight scores. Most tiles then need neither the
       // maximum over the four lanes of a column nor the factor exp2(m_old - m_new); probabilities
-      // lie below 2^LAZY_LOG2 instead of below one, which changes nothing in the quotient O / l
-      // (32-bit sums, and bfloat16 keeps its eight bits at any magnitude).
+      // lie below 2^LAZY_LOG2 instead of below one, where bfloat16 keeps its eight bits as well; but the
+      // weight of a row's largest key is then rounded like the others instead of being one. Against 64 bits
+      // that is 1.04 times the distance for scores of a standard deviation of one, 1.2 for two and more, so
+      // attention that came from kernels with that weight exact asks for no slack (slack_log2 0: 32 heads of
+      // 64 on 8, 2,048 tokens 40.2 -> 46.6 us, 4,096 in chunks of 2,048 63.8 -> 73.7).
       float lane_max[2];
       bool rise = false;
 #pragma unroll
@@ -1018,7 +1021,7 @@ void attention_prefill_shared_kernel(
           for (int c = 0; c < DCH; ++c) st[j].o[c] *= alpha;
           st[j].m = m_new;
           m_ref[j] = m_safe;
-          raise_at[j] = m_new == -INFINITY ? -INFINITY : (m_new + LAZY_LOG2) * inv_scale_log2e;
+          raise_at[j] = m_new == -INFINITY ? -INFINITY : (m_new + slack_log2) * inv_scale_log2e;
         }
       }
 #pragma unroll
@@ -1404,13 +1407,14 @@ extern "C" int dli_attention_prefill_max_cuts() { return PREFILL_MAX_CUTS; }
 // dli_attention_prefill_cut_floats() values; cut_count: one counter per cut tile and workgroup of
 // a tile (cut_tiles * q_heads is enough), zero before the first launch; every launch leaves them
 // zero, and launches that share them or cut_buf must not overlap.
+// top_exact: a row's weights are taken against its largest score so far (heads of 32 and more).
 extern "C" int dli_attention_prefill_bf16(const void* q, int64_t q_stride, const void* k_pages,
                                           const void* v_pages, void* out, int64_t out_stride,
                                           const int* q_start, const int* kv_len,
                                           const int* block_tables, int table_stride,
                                           const int* tile_entry, const int* tile_q0, int tiles,
                                           int q_heads, int kv_heads, int head_dim, int page_size,
-                                          float scale, int window, const int* tile_cut, int cut_tiles,
+                                          float scale, int window, int top_exact, const int* tile_cut, int cut_tiles,
                                           int cut_room, float* cut_buf, unsigned* cut_count, hipStream_t stream) {
   if (tiles <= 0) return DLI_OK;
   if (!dli_attention_mfma_supports(head_dim, page_size) || q_heads <= 0 || kv_heads <= 0 ||
@@ -1430,7 +1434,8 @@ extern "C" int dli_attention_prefill_bf16(const void* q, int64_t q_stride, const
     attention_prefill_shared_kernel<N><<<sgrid, 256, 0, stream>>>(                                \
         (const bf16_t*)q, q_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages, (bf16_t*)out, \
         out_stride, q_start, kv_len, block_tables, table_stride, tile_entry, tile_q0, q_heads,    \
-        kv_heads, page_size, scale * LOG2E, window, hw, tile_cut, cut_room, cut_buf, cut_count);  \
+        kv_heads, page_size, scale * LOG2E, window, hw, tile_cut, cut_room, cut_buf, cut_count,   \
+        top_exact ? 0.f : LAZY_LOG2);                                                             \
     break;
     switch (head_dim / 16) {
       SHARED_CASE(2) SHARED_CASE(3) SHARED_CASE(4) SHARED_CASE(5) SHARED_CASE(6) SHARED_CASE(7) SHARED_CASE(8)

@@ -101,7 +101,7 @@ _SIGNATURES = {
                                          _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_ptr],
     "dli_rope_angles": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
     "dli_attention_prefill_bf16": [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_int,
-                                   _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_ptr,
+                                   _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_ptr,
                                    _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr],
     "dli_attention_prefill_cut_floats": [_c_int, _c_int, _c_int],
     "dli_attention_prefill_max_cuts": [],
@@ -1447,7 +1447,8 @@ def attention_prefill(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Ten
                       q_start: torch.Tensor, kv_len: torch.Tensor, block_tables: torch.Tensor,
                       tile_entry: torch.Tensor, tile_q0: torch.Tensor, q_heads: int, scale: float,
                       window: int = 0, tile_cut: Optional[torch.Tensor] = None, cut_tiles: int = 0, cut_room: int = 0,
-                      cut_buf: Optional[torch.Tensor] = None, cut_count: Optional[torch.Tensor] = None) -> None:
+                      cut_buf: Optional[torch.Tensor] = None, cut_count: Optional[torch.Tensor] = None,
+                      top_exact: bool = False) -> None:
     """Matrix-core attention for portions; operands as :func:`attention_generic`, tiles of
     :func:`attention_prefill_tile_rows` queries (the tile list must be built with that height, in
     any order: every tile has a workgroup of its own and workgroups start in the list's order, so
@@ -1460,7 +1461,10 @@ def attention_prefill(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Ten
     ``cut_tiles`` cut tiles from 0. ``cut_room``: the most runs of any tile; ``cut_buf``: float32,
     ``cut_tiles * cut_room * attention_prefill_cut_floats(...)`` values; ``cut_count``: int32,
     ``cut_tiles * q_heads`` counters, zero before the first launch (every launch leaves them zero;
-    launches that share them must not overlap)."""
+    launches that share them must not overlap).
+
+    ``top_exact`` (heads of 32 and more): a row's weights are taken against its largest score so far, so that the weight of that key is
+    one and not rounded; else against a point that may lie below."""
     kv_heads, page_size, head_dim = _check_paged(q, k_pages, v_pages, out, q_heads)
     for name, t in (("q_start", q_start), ("kv_len", kv_len), ("tile_entry", tile_entry), ("tile_q0", tile_q0)):
         _dense(t, name, torch.int32, 1)
@@ -1483,7 +1487,7 @@ def attention_prefill(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Ten
     _check(library().dli_attention_prefill_bf16(
         _ptr(q), q.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(out), out.stride(0), _ptr(q_start), _ptr(kv_len),
         _ptr(block_tables), block_tables.stride(0), _ptr(tile_entry), _ptr(tile_q0), tile_entry.shape[0], q_heads,
-        kv_heads, head_dim, page_size, float(scale), int(window), _ptr(tile_cut), int(cut_tiles), int(cut_room),
+        kv_heads, head_dim, page_size, float(scale), int(window), int(top_exact), _ptr(tile_cut), int(cut_tiles), int(cut_room),
         _ptr(cut_buf), _ptr(cut_count), _stream()), "attention_prefill")
 
 # ----------------------------------------------------------------------------- sampling

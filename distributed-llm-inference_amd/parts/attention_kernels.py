@@ -334,7 +334,7 @@ def plain_portions(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor
         return False
     q_start, kv_len, tables, t, met_window = plan
     ops.attention_prefill(q, k_pages, v_pages, out, q_start, kv_len, tables, t.entry, t.q0, q_heads, scale, met_window, t.cut, t.cut_tiles,
-                          t.cut_room, t.cut_buf, t.cut_count)
+                          t.cut_room, t.cut_buf, t.cut_count, top_exact=True)
     return True
 
 

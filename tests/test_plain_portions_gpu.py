@@ -54,6 +54,40 @@ def test_same_results(monkeypatch, masks, page, heads, kv, dim):
     assert not got[0].any()   # the single token's row is another kernel's
 
 
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("spread", [1, 2, 4])
+@pytest.mark.parametrize("masks", [{}, {"chunk": 512}, {"window": 300}])
+def test_no_further_from_64_bits(monkeypatch, masks, spread, dim):
+    """Scores of this standard deviation, up to one key for all there is: as far from 64-bit arithmetic as the kernel for changed scores
+    (2-norm over 12,000 rows of a head, whose chance is well below 1%), with 2% for that chance."""
+    from dli_amd.kernels import ops
+    from dli_amd.parts import attention_kernels as A
+
+    monkeypatch.setattr(A, "PLAIN_FROM_PAIRS", 0)
+    heads, kv, n = 8, 2, 1500
+    ctx, pages = _context(16, [0], [n], 0)
+    gen = torch.Generator(device="cuda").manual_seed(spread)
+    draw = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    q, k, v = (draw(n, heads * dim) * spread).bfloat16(), draw(pages, kv, 16, dim).bfloat16(), draw(pages, kv, dim, 16).bfloat16()
+    got, other = torch.zeros_like(q), torch.zeros_like(q)
+    assert A.plain_portions(q, k, v, got, ctx, _Cache(k, v), heads, dim ** -0.5, **masks)
+    tiles = ctx.q_tiles(ops.attention_grouped_tile_tokens(heads, kv))
+    ops.attention_grouped(q, k, v, other, ctx.q_start, ctx.kv_len, ctx.groups[0].block_tables, tiles[0], tiles[1], heads, dim ** -0.5, **masks)
+    table = ctx.groups[0].block_tables[0].long()
+    keys, values = k[table].transpose(1, 2).reshape(-1, kv, dim)[:n], v[table].permute(0, 3, 1, 2).reshape(-1, kv, dim)[:n]
+    keys, values = (t.double().repeat_interleave(heads // kv, 1).transpose(0, 1) for t in (keys, values))
+    scores = torch.matmul(q.view(n, heads, dim).transpose(0, 1).double(), keys.transpose(1, 2).contiguous()) * dim ** -0.5
+    at = torch.arange(n, device="cuda")
+    seen = at[None] <= at[:, None]
+    if "chunk" in masks:
+        seen &= at[None] // 512 == at[:, None] // 512
+    if "window" in masks:
+        seen &= at[None] > at[:, None] - 300
+    want = torch.matmul(scores.masked_fill(~seen, -torch.inf).softmax(-1), values).transpose(0, 1).reshape(n, -1)
+    far, far_other = ((o.double() - want).norm().item() for o in (got, other))
+    assert far <= 1.02 * far_other, far / far_other
+
+
 def test_layers_with_heads_of_two_sizes_in_one_step():
     """A prompt whose longest tiles have their keys cut, in a step whose layers differ in their head size."""
     from dli_amd.kernels import ops

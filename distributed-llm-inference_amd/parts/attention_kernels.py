@@ -276,11 +276,12 @@ class ChunkPieces:
 
 
 # Pairs of a query head's row and a key from which a step's portions take that kernel. Below, the lists of its tiles, which the host makes
-# while the step's first kernels wait to be launched, cost as much as it gives. Prompts, all other kernels of the step included, us, the
-# kernel for changed scores and this one (millions of pairs): Miberax 1,024 wide 1 x 1,500 (17) 2,487 2,594, 4 x 1,400 (60) 4,536
-# 4,399; 2,048 wide 1 x 1,600 (39) 3,936 3,803, 1 x 2,048 (64) 5,010 4,508, 1 x 6,000 11,645 10,715; Rurorax 1,024 wide 1 x 2,000 (31) 1,803
-# 1,969, 2 x 1,500 (34) 2,077 2,056, 2 x 2,900 (91) 3,306 3,217; 2,048 wide 1 x 4,096 (256) 6,030 5,740; Betepel 1,024 wide 3 x 700 (11)
-# 2,272 2,458.
+# while the step's first kernels wait to be launched, cost as much as it gives. In steps whose attention is narrower than 2,048 the device
+# is done sooner and waits for them longer: two thirds more there. Prompts alone, from the call to their logits, us, the kernel for changed
+# scores and this one (millions of pairs): 2,048 wide Miberax 1 x 1,600 (39) 4,147 4,072, 2 x 1,300 (52) 5,611 5,502; Rurorax 1 x 1,600 (39)
+# 3,301 3,224, 1 x 2,200 (74) 4,180 4,054; Betepel 1 x 1,700 (44) 4,679 4,635, 2 x 1,500 (69) 6,534 6,491; 1,024 wide Miberax 1 x 2,300 (36)
+# 3,042 3,096, 4 x 1,150 (40) 4,491 4,554, 4 x 1,400 (60) 4,953 4,958, 3 x 2,000 (92) 5,457 5,351; Rurorax 1 x 2,600 (41) 2,270 2,414, 2 x
+# 1,700 (44) 2,632 2,728, 4 x 1,500 (69) 3,759 3,702; Betepel 3 x 1,300 (39) 4,024 4,006, 2 x 2,500 (78) 5,087 5,039.
 PLAIN_FROM_PAIRS = 36 << 20
 # How many times as many where chunks fill no more than half a tile's rows, which are 32, 64 or 128 for groups of a multiple of four, two
 # or one query heads: the rest of a tile is work for nothing, in every chunk, so never. Steps of 41 million pairs, us a layer, by the
@@ -296,7 +297,8 @@ def plain_pays(head_dim: int, q_heads: int, kv_heads: int, pairs: int, chunk: in
     if not ops.attention_prefill_cut_floats(head_dim, q_heads, kv_heads):
         return False
     short = 0 < 2 * chunk <= ops.attention_prefill_tile_rows(head_dim, q_heads, kv_heads)
-    return pairs >= PLAIN_FROM_PAIRS * (SHORT_CHUNKS if short else 1)
+    narrow = q_heads * head_dim < 2048
+    return pairs >= (PLAIN_FROM_PAIRS * 5 // 3 if narrow else PLAIN_FROM_PAIRS) * (SHORT_CHUNKS if short else 1)
 
 
 def plain_portions(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, out: torch.Tensor, ctx: Any, cache: Any,

@@ -40,9 +40,10 @@ def test_every_shape_has_buffers_of_its_own_size(monkeypatch, tokens, shapes):
 def test_which_portions_share_key_tiles():
     from dli_amd.parts.attention_kernels import PLAIN_FROM_PAIRS, plain_pays
 
-    many = 40 << 20
+    many, more = 40 << 20, 64 << 20
     assert PLAIN_FROM_PAIRS <= many
-    assert all(plain_pays(*s) for s in [(64, 32, 8, many, 0), (64, 32, 8, many, 32), (64, 16, 8, many, 48), (64, 32, 32, many, 80), (48, 24, 8, many, 80),
-                                        (128, 32, 8, many, 2048)])
-    assert not any(plain_pays(*s) for s in [(64, 32, 8, PLAIN_FROM_PAIRS - 1, 0), (64, 32, 8, many, 16), (64, 16, 8, many, 32), (64, 32, 32, many, 64),
-                                            (48, 24, 8, many, 48), (16, 32, 8, many, 0), (16, 32, 8, many, 2048), (64, 32, 32, 16 * many, 64)])
+    assert all(plain_pays(*s) for s in [(64, 32, 8, many, 0), (64, 32, 8, many, 32), (128, 16, 8, many, 48), (64, 32, 32, many, 80), (64, 16, 8, more, 48),
+                                        (48, 24, 8, more, 80), (128, 32, 8, many, 2048), (64, 16, 4, more, 1024)])
+    assert not any(plain_pays(*s) for s in [(64, 32, 8, PLAIN_FROM_PAIRS - 1, 0), (64, 32, 8, many, 16), (128, 16, 8, many, 32), (64, 32, 32, many, 64),
+                                            (48, 24, 8, more, 48), (16, 32, 8, more, 0), (16, 32, 8, more, 2048), (64, 32, 32, 16 * many, 64),
+                                            (64, 16, 4, many, 1024), (64, 16, 4, many, 0)])

@@ -308,20 +308,20 @@ def plain_portions(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor
     chunks of whole pages, whose rows are entries by themselves. False (nothing has run) elsewhere. (The kernel for
     changed scores takes blocks of 64 keys by way of registers, one barrier a block: a prompt of 4,096 tokens in chunks of 2,048, 32
     heads of 64 on 8, 149 us a layer and 75.)"""
-    def make() -> Optional[tuple]:
+    def make() -> tuple:
         grp, nd = ctx.groups[cache.group], ctx.num_decode
         pages, kv_heads, page_size, head_dim = k_pages.shape
         if (tuple(v_pages.shape) != (pages, kv_heads, head_dim, page_size) or scale <= 0.0
                 or not ops.attention_mfma_supports(head_dim, page_size, k_pages.dtype)):
-            return None
+            return ()
         new, keys = np.diff(ctx.q_start_host)[nd:].astype(np.int64), np.asarray(ctx.kv_len_host)[nd:].astype(np.int64)
         seen = np.minimum(keys, max(chunk, window)) if chunk or window else keys   # (by the last row, or one in the middle)
         longest = int(keys.max())
         met_chunk, met_window = (n if 0 < n < longest else 0 for n in (chunk, window))
         if not plain_pays(head_dim, q_heads, kv_heads, q_heads * int((new * np.minimum(seen, keys - new // 2)).sum()), met_chunk):
-            return None
+            return ()
         if met_window and (keep_first or met_chunk) or met_chunk % page_size:
-            return None
+            return ()
         if not met_chunk:
             return ctx.q_start, ctx.kv_len, grp.block_tables, prefill_tiles(ctx, head_dim, q_heads, kv_heads, nd, q.device, met_window), met_window
         pieces = ctx.step_lists(("chunk pieces", met_chunk, nd, cache.group), lambda: ChunkPieces(ctx, grp, nd, met_chunk))
@@ -330,9 +330,9 @@ def plain_portions(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor
 
     if out.dtype != k_pages.dtype:
         return False
-    # (asked once a step: a step of few tokens waits for its launches, and layers are alike)
+    # (asked once a step, also where the answer is no: a step of few tokens waits for its launches, and layers are alike)
     plan = ctx.step_lists(("plain portions", q_heads, tuple(k_pages.shape), tuple(v_pages.shape), cache.group, scale, chunk, window, keep_first), make)
-    if plan is None:
+    if not plan:
         return False
     q_start, kv_len, tables, t, met_window = plan
     ops.attention_prefill(q, k_pages, v_pages, out, q_start, kv_len, tables, t.entry, t.q0, q_heads, scale, met_window, t.cut, t.cut_tiles,

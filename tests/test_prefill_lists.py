@@ -11,10 +11,11 @@ def _context(monkeypatch, new):
 
     monkeypatch.setattr(ops, "compute_units", lambda device: 256)
     monkeypatch.setattr(batch, "upload", lambda arrays, device: [torch.from_numpy(np.ascontiguousarray(a)) for a in arrays])
-    empty = torch.zeros(0, dtype=torch.int32)
+    empty, width = torch.zeros(0, dtype=torch.int32), -(-max(new) // 16)
     q_start = np.concatenate([[0], np.cumsum(new)]).astype(np.int32)
     return batch.StepContext(device=torch.device("cpu"), page_size=16, num_tokens=int(q_start[-1]), num_entries=len(new), num_decode=0,
-                             token_ids=empty, positions=empty, q_start=empty, kv_len=empty, state_slots=empty, logit_rows=empty, groups=[],
+                             token_ids=empty, positions=empty, q_start=empty, kv_len=empty, state_slots=empty, logit_rows=empty,
+                             groups=[batch.GroupView(empty, torch.zeros(len(new), width, dtype=torch.int32), width)],
                              q_start_host=q_start, kv_len_host=np.asarray(new, np.int32))
 
 
@@ -47,3 +48,17 @@ def test_which_portions_share_key_tiles():
     assert not any(plain_pays(*s) for s in [(64, 32, 8, PLAIN_FROM_PAIRS - 1, 0), (64, 32, 8, many, 16), (128, 16, 8, many, 32), (64, 32, 32, many, 64),
                                             (48, 24, 8, more, 48), (16, 32, 8, more, 0), (16, 32, 8, more, 2048), (64, 32, 32, 16 * many, 64),
                                             (64, 16, 4, many, 1024), (64, 16, 4, many, 0)])
+
+
+def test_a_no_is_asked_for_once_a_step(monkeypatch):
+    """Layers of a step whose portions stay with the kernel for changed scores ask for its plan, which is made once all the same."""
+    from types import SimpleNamespace
+
+    from dli_amd.parts import attention_kernels as A
+
+    ctx, asked = _context(monkeypatch, [100]), []
+    monkeypatch.setattr(A, "plain_pays", lambda *a: asked.append(a))
+    q, k, v = torch.zeros(100, 256).bfloat16(), torch.zeros(7, 2, 16, 64).bfloat16(), torch.zeros(7, 2, 64, 16).bfloat16()
+    for _ in range(3):
+        assert not A.plain_portions(q, k, v, torch.zeros_like(q), ctx, SimpleNamespace(group=0), 4, 0.125, chunk=48)
+    assert len(asked) == 1

@@ -473,7 +473,7 @@ __global__ __launch_bounds__(64) void gated_delta_scan_kernel(GdArgs p) {
 
 // A step of single tokens in one kernel: convolution, recurrence, and each head's norm and gate (as conv_prepare, gated_delta_scan and
 // head_norm_gate make them, sums in their order: the same bits). Apart they are three launches whose waves each wait for two or three
-// trips to memory and hand a few kilobytes on: 4.9 + 5.0 + 4.6 us of a step of four requests (32 heads of 64 on 8), now 7.1 together (traced in the step).
+// trips to memory and hand a few kilobytes on: 4.9 + 5.0 + 4.6 us of a step of four requests (32 heads of 64 on 8), 5.9 to 6.4 together (both traced in a step).
 //
 // A workgroup takes a (request, q/k head) with all the value heads that share it, since the q and k channels' kept inputs are moved
 // on by whoever has read them. Its sixteen waves are units first (q, k, then runs of 64 channels of v, the last one the gates), then

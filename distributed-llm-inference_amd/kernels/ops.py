@@ -2115,7 +2115,10 @@ def scan_runs(entries: int, rows: int, heads: int, longest: int, unit_columns: b
         # entries 34 and 36), 200 with 64 (4 entries of 16 heads, 192 rows 45 and 47, 256 rows 57 and 49), 380 with 96, 700 with
         # 128 (8 of 16 heads, 200 rows 54 and 73, 700 rows 172 and 180), never with 192 (12 of 16 heads, 400 rows 120 and 139)
         # and 288 (12 of 24 heads 168 and 188). With more, one run an entry is faster (16 of 375 rows with 32 heads 273 and 183).
-        # (Of runs walked token by token; sixteen tokens at a time they take 0.6 to 0.8 of that: 170 rows 24, the last 112.)
+        # These are of runs walked token by token; the line lies where they put it. Walked sixteen tokens at a time runs are ahead
+        # wherever it cuts, and earlier. Token by token and in runs, us: one entry of 8 heads, 128 rows 27 23, 160 33 23; of 64 heads
+        # 160 36 30, 256 55 33; two of 32 heads 160 36 33, 208 46 35, 256 55 36; 8 of 16 heads 160 44 44, 256 66 52, 400 101 75, 700 171
+        # 106; 12 of 16 (one run an entry) 128 44 33, 400 123 83, 700 208 138; 12 of 24 400 170 111; 16 of 32 128 96 45, 400 289 114.
         from_rows += 24 + (20 if entries > 1 else 0) + side_by_side ** 3 // 3800
     elif side_by_side <= 64 and (entries > 1 or not unit_columns):
         from_rows += 16   # (2 entries of 128 rows with 32 heads, generalized delta rule: 44.5 and 47.6)

@@ -307,7 +307,7 @@ def plain_portions(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor
     window is all that changes it: under a mask that no row of the step meets, a window that keeps no first positions, or
     chunks of whole pages, whose rows are entries by themselves. False (nothing has run) elsewhere. (The kernel for
     changed scores takes blocks of 64 keys by way of registers, one barrier a block: a prompt of 4,096 tokens in chunks of 2,048, 32
-    heads of 64 on 8, 149 us a layer and 75.)"""
+    heads of 64 on 8, 149 us a layer and 74.)"""
     def make() -> tuple:
         grp, nd = ctx.groups[cache.group], ctx.num_decode
         pages, kv_heads, page_size, head_dim = k_pages.shape

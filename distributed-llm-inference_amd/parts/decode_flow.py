@@ -17,8 +17,12 @@ import torch
 from ..kernels import ops
 from .base import DecodeStream
 
-# The kernel takes the longest context that the step's tables can hold at two to eight pairs of tiles a wave; longer ones
-# have their keys cut over more workgroups by the attention's own kernel.
+# Of the longest context that the step's tables can hold. Up to here a wave has one pair of tiles of keys (4,096 keys) or two, all of them
+# on their way at once; longer contexts the attention's own kernel cuts over more workgroups than the sixteen a kv head of this one. Kernel by
+# kernel -> in one launch, a step and seven more, ms, at 8,000, 12,000, 16,000, 33,000 and 66,000 keys: 135M sizes 5.74 4.22, 6.17 4.98,
+# 6.30 5.26, 7.43 7.84, 8.33 11.7; 12 layers of 1,024 with 8 heads of 128 on 2 2.99 2.30, 3.12 2.76, 3.15 2.86, 4.09 4.80, 4.76 7.43; 16 heads
+# of 64 on 16 4.04 2.99, 4.42 3.47, 4.69 3.73, 6.32 5.59, 9.01 8.94. (Tables grow in powers of two: the next one holds 16,384, its tests end
+# here.)
 MOST_KEYS = 8192
 
 

@@ -225,7 +225,10 @@ class Model:
                 torch.cuda.synchronize()   # its launches may have run on other streams than the one its memory was made on
             caches.flow = DecodeFlow.build(self, caches) or False
             caches.flow_for = self.weights_version
-        return caches.flow or None
+        if not caches.flow or any("forward_stream" in own or "fused_params" in own for layer in self.layers
+                                  for own in map(vars, (layer.block, *layer.parts.values()))):
+            return None   # (what an object is given of its own in the place of its class's method runs, block by block)
+        return caches.flow
 
     def forward(self, ctx: Any, caches: Sequence[Any]) -> torch.Tensor:
         """Run the step's tokens through the schedule; float32 logits ``[wanted rows, vocab]``."""

@@ -236,3 +236,25 @@ def test_a_block_of_ones_own_is_told_of_norms_only():
     assert Model._met_with(both, "first_norm") is None and isinstance(Model._met_with(both, "meets"), NormPair)
     assert isinstance(Model._met_with(alone, "first_norm"), Norm) and Model._met_with(alone, "meets") is None
     assert Model._met_with(changed, "first_norm") is None and Model._met_with(changed, "meets") is None
+
+
+@pytest.mark.parametrize("role", [None, "mixer", "feed_forward", "mixer_norm", "feed_forward_norm"])
+def test_one_launch_steps_aside_for_an_object_with_a_form_of_its_own(role):
+    """A block or part whose object, not its class, has another ``forward_stream`` or ``fused_params`` is asked for it in steps of one
+    row too: all layers in one launch would pass it by."""
+    from dli_amd.parts.model import BoundCaches, Model
+    from dli_amd.weights.loader import build_model
+    from tiny_configs import TINY_B
+
+    model, _ = build_model(TINY_B, Runtime(torch.device("cpu"), torch.bfloat16))
+    caches, flow = BoundCaches(), object()
+    caches.flow, caches.flow_for = flow, model.weights_version
+    assert isinstance(model, Model) and model._decode_flow(caches) is flow
+    layer = model.layers[-1]
+    part = layer.block if role is None else layer.parts[role]
+    form = "fused_params" if "norm" in (role or "") else "forward_stream"
+    own = getattr(part, form)
+    setattr(part, form, lambda *a, **kw: own(*a, **kw))
+    assert model._decode_flow(caches) is None
+    delattr(part, form)
+    assert model._decode_flow(caches) is flow
